@@ -45,6 +45,8 @@ constexpr int SUBBINS = 64;     // second level inside the threshold bin: the ne
 constexpr int SUB_RANK_CAP = 128; // ties of one second-level step that are ranked by direct comparison (more: digit by digit)
 constexpr int SEL_CHUNK = 4096; // scores per workgroup of the select kernel
 constexpr int TIE_CAP = 8192;   // capacity of the per-row tie list
+constexpr int INDEXER_ROW_MAX = 32768; // rows up to this length are selected by one kernel (indexer_row_topk_kernel)
+constexpr int SCORE_GROUPS = 512; // workgroups of the paged score kernel below which its spans are made shorter
 
 __device__ __forceinline__ float f16_bits_to_f32(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
 // A scale as it lies in memory (fp16 bits, or fp32 in the fp32-scale variant) and as the fp32 factor it stands for.
@@ -142,8 +144,8 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v)
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// The workgroup's histograms (S1 query tokens, one 2048-key span) go to its own slots, as 16-bit counts (at most 2048
-// each), two per lane.  The span-0 workgroup also clears the select kernel's list counters of its query tokens.  256 lanes.
+// The workgroup's histograms (S1 query tokens, one span of keys) go to its own slots, as 16-bit counts (a span has at
+// most 2048 keys), two per lane.  The span-0 workgroup also clears the select kernel's list counters of its query tokens.  256 lanes.
 template <int S1>
 __device__ __forceinline__ void flush_span_hist(const IndexerArgs& a, const uint32_t (*hist)[SBINS], int row0, int span, int tid)
 {
@@ -252,13 +254,13 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a)
             if (ok && g == 0) {
                 const float sc = sum[0] * (present[j] ? ScaleOf<F32>::f32(ksb[j]) : 0.f);
                 a.scores[(int64_t)(row0 + s) * a.score_stride + tok] = sc;
-                if (tok < eff) atomicAdd(&hist[s][score_bin(score_key(sc))], 1u);
+                if (a.use_hist && tok < eff) atomicAdd(&hist[s][score_bin(score_key(sc))], 1u);
             }
         }
     }
     } // pass
     __syncthreads();
-    flush_span_hist<S1>(a, hist, row0, (int)blockIdx.x, tid);
+    if (a.use_hist) flush_span_hist<S1>(a, hist, row0, (int)blockIdx.x, tid);
 }
 
 // relu(a) * 2^-11 and relu(b) * 2^-11, each rounded once to fp16, packed (a in the low half).  The int32 sums arrive
@@ -284,10 +286,8 @@ __device__ __forceinline__ uint32_t relu_scale_pack(int a, int b)
 // files its results 64 at a time: w_scale sits in every row of the head-sum operand, so every lane group holds the 16
 // scores of a key group and lane group g keeps those of key group g - after four key groups lane l holds the score of
 // key l of the 64, next to that key's scale (loaded with one 128-byte instruction per 64 keys).
-constexpr int PPASSES = 4; // passes (of 512 keys) per workgroup of the paged kernel
-constexpr int SPAN = CHUNK * PPASSES; // keys per workgroup of either score kernel: one histogram slot
-static_assert(SPAN == CHUNK * PASSES, "both score kernels own spans of the same size");
-template <int S1, bool F32>
+// PPASSES: passes (of 512 keys) per workgroup, pick_passes' choice
+template <int S1, bool F32, int PPASSES>
 __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kernel(IndexerArgs a)
 {
     constexpr int NBUF = 2; // half-pass buffers: NBUF-1 halves ahead (deeper prefetch measured no faster)
@@ -298,7 +298,7 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
     const int l16 = lane & 15, g = lane >> 4;
     const int sgrp = blockIdx.z;
     const int bs = a.block_size;
-    // The (sequence, 2048-key span) of this workgroup: by its place in the grid when every sequence fills its spans.
+    // The (sequence, span of 512 PPASSES keys) of this workgroup: by its place in the grid when every sequence fills its spans.
     // With ragged lengths the workgroups that have work should be the first ones of the launch order, so that they
     // spread evenly over the CUs: workgroup w (its place in launch order, sequence-major) takes the w-th span that
     // holds keys.  Every wavefront finds it on its own from the sequence lengths (lane l holds sequences l, l + 64, ..;
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
             const float sc = res[s] * ks;
             s_sc[s][tok - span * (CHUNK * PPASSES)] = sc;
             const int eff = L - (a.s1 - 1 - (sgrp * S1 + s));
-            if (tok < eff) atomicAdd(&hist[s][score_bin(score_key(sc))], 1u);
+            if (a.use_hist && tok < eff) atomicAdd(&hist[s][score_bin(score_key(sc))], 1u);
         }
     };
 
@@ -474,10 +474,11 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
     for (int s = 0; s < S1; ++s) {
         float* dst = a.scores + (int64_t)(row0 + s) * a.score_stride + (int64_t)span * (CHUNK * PPASSES);
 #pragma unroll
-        for (int i = 0; i < CHUNK * PPASSES / 1024; ++i)
-            *reinterpret_cast<f32x4*>(dst + 4 * (tid + 256 * i)) = *reinterpret_cast<const f32x4*>(&s_sc[s][4 * (tid + 256 * i)]);
+        for (int i = 0; i < (CHUNK * PPASSES + 1023) / 1024; ++i)
+            if (4 * (tid + 256 * i) < CHUNK * PPASSES)
+                *reinterpret_cast<f32x4*>(dst + 4 * (tid + 256 * i)) = *reinterpret_cast<const f32x4*>(&s_sc[s][4 * (tid + 256 * i)]);
     }
-    flush_span_hist<S1>(a, hist, row0, span, tid);
+    if (a.use_hist) flush_span_hist<S1>(a, hist, row0, span, tid);
 }
 
 __global__ void indexer_fill_kernel(int32_t* p, int n, int32_t v)
@@ -548,7 +549,7 @@ __global__ __launch_bounds__(256) void indexer_select_kernel(IndexerArgs a)
     const int n = max(len - (a.s1 - 1 - (row - bi * a.s1)), 0);
     // (a workgroup past the row's end leaves further down, behind the first use of what was requested above: an exit
     // here would let the compiler move those requests behind the wait for the length - two round trips instead of one)
-    const int nsp = min((len + SPAN - 1) / SPAN, a.pchunks); // spans whose workgroup ran
+    const int nsp = min((len + a.span - 1) / a.span, a.pchunks); // spans whose workgroup ran
     if (tid == 0) s_bin = 0xffffffffu; // n <= k: no threshold bin, everything is a winner
 
     uint32_t acc[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
@@ -687,105 +688,125 @@ __device__ __forceinline__ void radix_select64(Each&& for_each, Emit&& emit, uin
     }
 }
 
-// cand[0 .. m) holds the selected words in any order (the rest of its 2048 slots is zero): write their indices in
-// descending word order, then -1 up to k.  The words are first grouped by key into at most 2048 equal steps of the
-// selected keys' range, so a counting pass (histogram, suffix scan, scatter) puts every word within a few slots of
-// its place - and then ranked inside their group by direct comparison.  A bin with more than 64 words (heavily tied scores)
-// would make that ranking quadratic; then a bitonic sort of all 2048 words is used instead.
-// Workgroup of 1024 lanes; hist has 2048 words, scratch 8192 words (start | cursor | grouped words), tmp 16.
-__device__ __forceinline__ void order_and_write(uint64_t* cand, uint32_t m, uint32_t* hist, uint32_t* scratch,
-                                                uint32_t* tmp, uint32_t* s_flag, int32_t* out, int k)
+// A word's group for ordering: a non-decreasing function of its key with values 0 .. 2047.  `kind` 0 cuts the scores'
+// range into equal steps (rounding is monotone: neither the difference nor the product turns two scores around), kind 1
+// the range of their ordered keys - steps in proportion to the magnitude.
+__device__ __forceinline__ float key_to_score(uint32_t key) { return __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key); }
+struct KeyGroups {
+    uint32_t kmin, kmax;
+    float fmin, per;
+    int shift;
+    bool linear_ok; // the scores' range is finite and not empty
+    __device__ __forceinline__ KeyGroups(uint32_t lo, uint32_t hi) : kmin(lo), kmax(hi)
+    {
+        fmin = key_to_score(lo);
+        const float span = key_to_score(hi) - fmin;
+        per = 2047.0f / span;
+        shift = max(0, 21 - (int)__builtin_clz((hi - lo) | 1u));
+        linear_ok = span > 0.f && span < __builtin_inff() && per < __builtin_inff();
+    }
+    __device__ __forceinline__ uint32_t of(uint32_t key, int kind) const
+    {
+        return kind == 0 ? min((uint32_t)((key_to_score(key) - fmin) * per), 2047u) : (key - kmin) >> shift;
+    }
+};
+
+// Ordering: word w[h] of a lane is real if tid + 1024 h < m (m <= 1024 PER); calls write(rank, word) for the k first of
+// them in descending word order.  kmin / kmax bound the words' keys.  The words are grouped by KeyGroups, so a counting pass
+// (histogram, suffix scan, scatter) puts every word within a few slots of its place - and then ranked inside their group by
+// direct comparison.  Equal steps of the score come first: bell-shaped scores leave a few words in a step wherever the
+// selection ends.  If those crowd (more than GROUP_CAP words in one), equal steps of the keys; if these do too (heavily tied
+// scores), a bitonic sort.  (Steps of the keys alone crowd near zero, and a row whose selection reaches scores of both signs
+// then paid for the sort: 18 us against 8.)
+// Workgroup of 1024 lanes; buf has 1024 PER words, hist and start 2048, tmp 16.
+constexpr uint32_t GROUP_CAP = 64;
+template <int PER, class Write>
+__device__ __forceinline__ void order_words(const uint64_t (&w)[PER], uint32_t m, uint32_t kmin, uint32_t kmax, uint64_t* buf, uint32_t* hist,
+                                            uint32_t* start, uint32_t* tmp, uint32_t* s_flag, int k, Write&& write)
 {
     const int tid = threadIdx.x;
-    uint32_t* start = scratch;          // [2048] slots taken by the higher bins
-    uint32_t* cursor = scratch + NBINS; // [2048]
-    uint64_t* grouped = reinterpret_cast<uint64_t*>(scratch + 2 * NBINS); // [2048]
-    hist[tid] = 0;
-    hist[tid + 1024] = 0;
-    cursor[tid] = 0;
-    cursor[tid + 1024] = 0;
-    if (tid == 0) {
-        *s_flag = 0;
-        tmp[14] = 0xffffffffu; // smallest selected key
-        tmp[15] = 0u;          // largest selected key
-    }
-    __syncthreads();
-    uint64_t w[2];
-    uint32_t bin[2];
-    bool valid[2];
-    uint32_t kmin = 0xffffffffu, kmax = 0u;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int i = tid + 1024 * h;
-        valid[h] = (uint32_t)i < m;
-        w[h] = cand[i];
-        if (valid[h]) {
-            kmin = min(kmin, (uint32_t)(w[h] >> 32));
-            kmax = max(kmax, (uint32_t)(w[h] >> 32));
-        }
-    }
-    kmin = wave_min(kmin);
-    kmax = wave_max(kmax);
-    if ((tid & 63) == 0) {
-        atomicMin(&tmp[14], kmin);
-        atomicMax(&tmp[15], kmax);
-    }
-    __syncthreads();
-    // bins: the selected keys' range cut into at most 2048 equal steps (the keys are order-preserving images of the
-    // scores, dense enough over the top-k range that a step holds a handful of words)
-    kmin = tmp[14];
-    const uint32_t range = tmp[15] - kmin;
-    const int shift = max(0, 21 - (int)__builtin_clz(range | 1u));
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        bin[h] = ((uint32_t)(w[h] >> 32) - kmin) >> shift;
-        if (valid[h]) atomicAdd(&hist[bin[h]], 1u);
-    }
-    __syncthreads();
-    {
-        const uint32_t h_lo = hist[2 * tid], h_hi = hist[2 * tid + 1]; // lane t owns bins 2t and 2t+1
-        if (h_lo > 64u || h_hi > 64u) *s_flag = 1;
-        const uint32_t incl = block_suffix_sum<16>(h_lo + h_hi, tmp);
-        start[2 * tid + 1] = incl - h_lo - h_hi;
-        start[2 * tid] = incl - h_lo;
-    }
-    __syncthreads();
-    if (*s_flag == 0) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-            if (valid[h]) grouped[start[bin[h]] + atomicAdd(&cursor[bin[h]], 1u)] = w[h];
+    const KeyGroups groups(kmin, kmax);
+    uint32_t bin[PER];
+    for (int kind = groups.linear_ok ? 0 : 1; kind < 2; ++kind) { // (block-uniform)
+        __syncthreads();
+        hist[tid] = 0;
+        hist[tid + 1024] = 0;
+        if (tid == 0) *s_flag = 0;
         __syncthreads();
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-            if (valid[h]) {
-                const uint32_t s0 = start[bin[h]], c = hist[bin[h]];
-                uint32_t rank = 0;
-                for (uint32_t j = 0; j < c; ++j) rank += grouped[s0 + j] > w[h] ? 1u : 0u;
-                if ((int)(s0 + rank) < k) out[s0 + rank] = (int32_t)(0xffffffffu - (uint32_t)(w[h] & 0xffffffffull));
-            }
-        for (int j = (int)m + tid; j < k; j += 1024) out[j] = -1;
-        return;
+        for (int h = 0; h < PER; ++h) {
+            bin[h] = groups.of((uint32_t)(w[h] >> 32), kind);
+            if ((uint32_t)(tid + 1024 * h) < m) atomicAdd(&hist[bin[h]], 1u);
+        }
+        __syncthreads();
+        {
+            const uint32_t h_lo = hist[2 * tid], h_hi = hist[2 * tid + 1]; // lane t owns bins 2t and 2t+1
+            if (h_lo > GROUP_CAP || h_hi > GROUP_CAP) *s_flag = 1;
+            const uint32_t incl = block_suffix_sum<16>(h_lo + h_hi, tmp);
+            start[2 * tid + 1] = incl - h_lo - h_hi; // slots taken by the higher bins
+            start[2 * tid] = incl - h_lo;
+        }
+        __syncthreads();
+        if (*s_flag == 0) {
+#pragma unroll
+            for (int h = 0; h < PER; ++h)
+                if ((uint32_t)(tid + 1024 * h) < m) buf[atomicAdd(&start[bin[h]], 1u)] = w[h]; // (start ends up as the bin's end)
+            __syncthreads();
+#pragma unroll
+            for (int h = 0; h < PER; ++h)
+                if ((uint32_t)(tid + 1024 * h) < m) {
+                    const uint32_t c = hist[bin[h]], s0 = start[bin[h]] - c;
+                    if ((int)s0 >= k) continue;
+                    uint32_t rank = s0;
+                    for (uint32_t j = 0; j < c; ++j) rank += buf[s0 + j] > w[h] ? 1u : 0u;
+                    if ((int)rank < k) write((int)rank, w[h]);
+                }
+            return;
+        }
     }
-    // bitonic sort, descending, 2048 words, two per lane.  A compare-exchange step of stride <= 64 stays inside
+    // bitonic sort, descending, two words per lane and 2048 words.  A compare-exchange step of stride <= 64 stays inside
     // the 128 words owned by one wavefront (lane i of wave w handles the pair (128w + 2i - i%stride, + stride)),
     // so only the steps of stride >= 128 need a workgroup barrier; the others rely on LDS operations of one
     // wavefront completing in order.
-    for (int size = 2; size <= MAX_K; size <<= 1) {
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < PER; ++h) buf[tid + 1024 * h] = (uint32_t)(tid + 1024 * h) < m ? w[h] : 0ull;
+    __syncthreads();
+    for (int size = 2; size <= 1024 * PER; size <<= 1) {
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
             if (stride >= 128) __syncthreads();
-            const int pos = 2 * tid - (tid & (stride - 1)); // lower index of the pair
-            const bool desc = (pos & size) == 0;
-            const uint64_t lo = cand[pos], hi = cand[pos + stride];
-            if ((lo < hi) == desc) {
-                cand[pos] = hi;
-                cand[pos + stride] = lo;
+#pragma unroll
+            for (int q = 0; q < PER / 2; ++q) {
+                const int i = tid + 1024 * q;
+                const int pos = 2 * i - (i & (stride - 1)); // lower index of the pair
+                const bool desc = (pos & size) == 0;
+                const uint64_t lo = buf[pos], hi = buf[pos + stride];
+                if ((lo < hi) == desc) {
+                    buf[pos] = hi;
+                    buf[pos + stride] = lo;
+                }
             }
             if (stride >= 128) __syncthreads();
             else __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         }
     }
     __syncthreads();
-    for (int j = tid; j < k; j += 1024) out[j] = (int32_t)(0xffffffffu - (uint32_t)(cand[j] & 0xffffffffull));
+    for (int j = tid; j < min((int)m, k); j += 1024) write(j, buf[j]);
+}
+__device__ __forceinline__ int word_index(uint64_t w) { return (int)(0xffffffffu - (uint32_t)(w & 0xffffffffull)); }
+
+// smallest and largest key of the block, into (and out of) tmp[14] and tmp[15], which hold ~0 and 0 before; 1024 lanes
+__device__ __forceinline__ void block_key_range(uint32_t& kmin, uint32_t& kmax, uint32_t* tmp)
+{
+    kmin = wave_min(kmin);
+    kmax = wave_max(kmax);
+    if ((threadIdx.x & 63) == 0) {
+        atomicMin(&tmp[14], kmin);
+        atomicMax(&tmp[15], kmax);
+    }
+    __syncthreads();
+    kmin = tmp[14];
+    kmax = tmp[15];
 }
 
 __global__ __launch_bounds__(1024) void indexer_topk_kernel(IndexerArgs a)
@@ -911,17 +932,40 @@ __global__ __launch_bounds__(1024) void indexer_topk_kernel(IndexerArgs a)
     }
     __syncthreads();
 
-    order_and_write(cand, (uint32_t)min(n, k), hist, reinterpret_cast<uint32_t*>(tie), tmp, &s_bin,
-                    a.topk_res + (int64_t)row * k, k);
+    // the indices of the selected words, best first, then -1
+    int32_t* out = a.topk_res + (int64_t)row * k;
+    const uint32_t m = (uint32_t)min(n, k);
+    for (int j = (int)m + tid; j < k; j += 1024) out[j] = -1;
+    uint64_t w[2];
+    uint32_t kmin = 0xffffffffu, kmax = 0u;
+    if (tid == 0) {
+        tmp[14] = 0xffffffffu;
+        tmp[15] = 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        w[h] = cand[tid + 1024 * h];
+        if ((uint32_t)(tid + 1024 * h) < m) {
+            kmin = min(kmin, (uint32_t)(w[h] >> 32));
+            kmax = max(kmax, (uint32_t)(w[h] >> 32));
+        }
+    }
+    block_key_range(kmin, kmax, tmp);
+    order_words<2>(w, m, kmin, kmax, cand, hist, reinterpret_cast<uint32_t*>(tie), tmp, &s_bin, k,
+                   [&](int rank, uint64_t word) { out[rank] = word_index(word); });
 }
 
 // Standalone top-k of fp32 rows (pypto.topk: python/pypto/op/comparison.py:302-344; order of equal values - smaller
 // index first - framework/src/interface/interpreter/calculator/calc_torch.cpp:2481-2494,2734-2749): values and int32
-// indices of the k largest (or smallest) elements of every row, best first.  One workgroup of 1024 lanes per row.  Rows
-// of up to TOPK_SORT_CAP elements are sorted whole in LDS; longer rows (then k <= MAX_K) go through the radix select
-// first.  Words are (key << 32 | ~index) with the order-preserving key of the value (of its negation for the smallest),
+// indices of the k largest (or smallest) elements of every row, best first.  One workgroup of 1024 lanes per row.
+// Words are (key << 32 | ~index) with the order-preserving key of the value (of its negation for the smallest),
 // so descending word order is the rule above; -0 and +0 count as equal.
+// topk_sort_kernel sorts the whole row in LDS: k beyond MAX_K (rows of up to TOPK_SORT_CAP elements), and rows of up to
+// TOPK_SORT_SMALL elements, where its 28 steps are fewer than the fixed steps of the other kernel.
+// topk_select_kernel serves everything else: it finds the k largest words and orders only those.
 constexpr int TOPK_SORT_CAP = 8192;
+constexpr int TOPK_SORT_SMALL = 128;
 
 // bitonic sort of a[0 .. p), p a power of two <= TOPK_SORT_CAP, descending; 1024 lanes
 __device__ __forceinline__ void bitonic_desc(uint64_t* a, int p)
@@ -943,41 +987,252 @@ __device__ __forceinline__ void bitonic_desc(uint64_t* a, int p)
     __syncthreads();
 }
 
-__global__ __launch_bounds__(1024) void topk_rows_kernel(const float* __restrict__ x, float* __restrict__ values,
+__global__ __launch_bounds__(1024) void topk_sort_kernel(const float* __restrict__ x, float* __restrict__ values,
                                                          int32_t* __restrict__ indices, int n, int k, int largest)
 {
     __shared__ uint64_t buf[TOPK_SORT_CAP];
-    __shared__ uint32_t hist[NBINS];
-    __shared__ uint32_t tmp[16];
-    __shared__ uint32_t s_bin, s_krem, s_cnt, s_out;
     const int tid = threadIdx.x;
     const float* row = x + (int64_t)blockIdx.x * n;
-    auto word = [&](int i) { return make_cand(score_key(largest ? row[i] : -row[i]), i); };
-    int p;
-    if (n <= TOPK_SORT_CAP) {
-        p = 2;
-        while (p < n) p <<= 1;
-        for (int i = tid; i < p; i += 1024) buf[i] = i < n ? word(i) : 0ull; // (every real word is > 0: its index part is)
-    } else {
-        p = MAX_K;
-        for (int i = tid; i < MAX_K; i += 1024) buf[i] = 0ull;
-        if (tid == 0) s_out = 0;
-        __syncthreads();
-        auto each = [&](auto&& f) {
-            for (int i = tid; i < n; i += 1024) f(word(i));
-        };
-        auto emit = [&](uint64_t w) {
-            const uint32_t q = atomicAdd(&s_out, 1u);
-            if (q < MAX_K) buf[q] = w;
-        };
-        radix_select64(each, emit, (uint32_t)k, 64, hist, tmp, &s_bin, &s_krem, &s_cnt);
-    }
+    int p = 2;
+    while (p < n) p <<= 1;
+    // (every real word is > 0: its index part is)
+    for (int i = tid; i < p; i += 1024) buf[i] = i < n ? make_cand(score_key(largest ? row[i] : -row[i]), i) : 0ull;
     bitonic_desc(buf, p);
     for (int j = tid; j < k; j += 1024) {
-        const int i = (int)(0xffffffffu - (uint32_t)(buf[j] & 0xffffffffull));
+        const int i = word_index(buf[j]);
         indices[(int64_t)blockIdx.x * k + j] = i;
         values[(int64_t)blockIdx.x * k + j] = row[i];
     }
+}
+
+// The k (<= MAX_K) first words of a row in descending word order, by one workgroup of 1024 lanes in one pass over the row:
+// calls write(rank, word).  Bound by latency, not by bytes: a chain of memory round trips, LDS passes and barriers.
+//   1. ROW_SAMPLES elements, evenly spaced, are counted in equal steps of their scores' range; a suffix scan gives a pivot
+//      that somewhat more than k elements of the row should reach (four standard deviations of the sample count more).
+//   2. The row - requested before anything else - is filtered: the words that reach the pivot go to
+//      LDS, a wavefront's with one counter update per 16 elements of a lane.
+//   3. If at least k and at most ROW_CAP did (else: row_select_exact), they are put in order by order_words, which drops
+//      those behind the k-th.
+// Rows of up to ROW_CAP elements skip 1 and keep everything.  NPT: elements per lane; 0: rows of any length, 32 elements per
+// lane (128 KB) in flight.  `VEC` consecutive elements go to one lane (4: `load4(i)`, 16-byte aligned and readable up to the next
+// multiple of 4096 elements, `cap`), so that the requests are wide.
+constexpr int ROW_CAP = 4096, ROW_SAMPLES = 4096;
+struct RowLds {
+    uint64_t buf[ROW_CAP];
+    uint32_t hist[NBINS];
+    uint32_t start[NBINS];
+    uint32_t tmp[16];
+    uint32_t bin, krem, cnt, out;
+};
+
+// The same selection by counting passes over the row (11 key bits a pass, then the indices of equal keys): for rows whose
+// sampled pivot misjudged - heavy ties, scores sorted by position in step with the samples, far outliers.  Leaves the k
+// selected words in lds.buf.
+template <class Load>
+__device__ __forceinline__ void row_select_exact(RowLds& lds, int n, int k, Load&& load)
+{
+    const int tid = threadIdx.x;
+    auto each = [&](auto&& f) {
+        constexpr int AHEAD = 8; // (a lane's requests in flight)
+        for (int base = tid; base < n; base += 1024 * AHEAD) {
+            float v[AHEAD];
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j) v[j] = load(min(base + 1024 * j, n - 1));
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j)
+                if (base + 1024 * j < n) f(make_cand(score_key(v[j]), base + 1024 * j));
+        }
+    };
+    __syncthreads();
+    if (tid == 0) lds.out = 0u;
+    __syncthreads();
+    radix_select64(each, [&](uint64_t w) {
+        const uint32_t p = atomicAdd(&lds.out, 1u);
+        if (p < MAX_K) lds.buf[p] = w;
+    }, (uint32_t)k, 64, lds.hist, lds.tmp, &lds.bin, &lds.krem, &lds.cnt);
+    __syncthreads();
+}
+
+template <int NPT, int VEC, class Load, class Load4, class Length, class Write>
+__device__ __forceinline__ void select_row(RowLds& lds, int cap, int k, Load&& load, Load4&& load4, Length&& length, Write&& write)
+{
+    constexpr int CH = NPT > 0 ? NPT : 16; // elements per lane filtered together
+    constexpr int AHEAD = NPT > 0 ? 1 : 2; // such groups in flight
+    const int tid = threadIdx.x, lane = tid & 63;
+    // element j of this lane
+    auto index = [&](int j) { return VEC == 4 ? 4 * (tid + 1024 * (j >> 2)) + (j & 3) : tid + 1024 * j; };
+    float v[AHEAD][CH];
+    auto request = [&](int j0, float (&to)[CH]) {
+        if constexpr (VEC == 4) {
+#pragma unroll
+            for (int j = 0; j < CH; j += 4) {
+                const f32x4 q = load4(min(index(j0 + j), cap - 4));
+#pragma unroll
+                for (int c = 0; c < 4; ++c) to[j + c] = q[c];
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < CH; ++j) to[j] = load(min(index(j0 + j), cap - 1));
+        }
+    };
+#pragma unroll
+    for (int g = 0; g < AHEAD; ++g) request(g * CH, v[g]);
+    const int n = length(); // (its loads travel with the row's)
+    if (n <= 0) return;     // block-uniform
+    k = min(k, n);
+    lds.hist[tid] = 0u;
+    lds.hist[tid + 1024] = 0u;
+    if (tid == 0) {
+        lds.out = 0u;
+        lds.bin = 0u;
+        lds.tmp[14] = 0xffffffffu;
+        lds.tmp[15] = 0u;
+    }
+    uint32_t pivot = 0u;
+    if (n > ROW_CAP) { // block-uniform
+        constexpr int PER = ROW_SAMPLES / 1024;
+        uint32_t key[PER], kmin = 0xffffffffu, kmax = 0u;
+        float sv[PER];
+#pragma unroll
+        for (int q = 0; q < PER; ++q) sv[q] = load((int)(((int64_t)(tid + 1024 * q) * n) / ROW_SAMPLES));
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            key[q] = score_key(sv[q]);
+            kmin = min(kmin, key[q]);
+            kmax = max(kmax, key[q]);
+        }
+        __syncthreads();
+        block_key_range(kmin, kmax, lds.tmp);
+        const KeyGroups groups(kmin, kmax);
+        if (groups.linear_ok) {
+#pragma unroll
+            for (int q = 0; q < PER; ++q) atomicAdd(&lds.hist[groups.of(key[q], 0)], 1u);
+            __syncthreads();
+            const float expect = (float)k * ((float)ROW_SAMPLES / (float)n);
+            const uint32_t target = (uint32_t)(expect + 4.f * __builtin_sqrtf(expect)) + 2u;
+            const uint32_t h_lo = lds.hist[2 * tid], h_hi = lds.hist[2 * tid + 1]; // lane t owns bins 2t and 2t+1
+            const uint32_t incl = block_suffix_sum<16>(h_lo + h_hi, lds.tmp);
+            // the highest step that `target` samples reach
+            if (incl >= target && incl - h_lo - h_hi < target) lds.bin = incl - h_lo >= target ? 2 * tid + 1 : 2 * tid;
+            __syncthreads();
+            pivot = f32_to_ordered(groups.fmin + (float)lds.bin / groups.per);
+        }
+        __syncthreads();
+        if (tid == 0) {
+            lds.tmp[14] = 0xffffffffu;
+            lds.tmp[15] = 0u;
+        }
+    }
+    __syncthreads();
+    uint32_t bottom = 0xffffffffu, top = 0u; // smallest and largest key that reached the pivot
+    auto filter = [&](int j0, const float (&from)[CH]) { // elements j0 .. j0 + CH - 1 of the lane
+        uint32_t key[CH], count = 0;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const uint32_t u = max(score_key(from[j]), 1u); // (0: no element; only NaNs have keys that low)
+            key[j] = index(j0 + j) < n && u >= pivot ? u : 0u;
+            top = max(top, key[j]);
+            bottom = min(bottom, key[j] - 1u);
+            count += key[j] != 0u ? 1u : 0u;
+        }
+        const uint32_t incl = wave_prefix_sum(count);
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        if (total == 0u) return; // wave-uniform
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(&lds.out, total);
+        at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) + incl - count;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            if (key[j] != 0u && at < ROW_CAP) lds.buf[at] = make_cand(key[j], index(j0 + j));
+            at += key[j] != 0u ? 1u : 0u;
+        }
+    };
+    if constexpr (NPT > 0) {
+        filter(0, v[0]);
+    } else {
+        for (int j0 = 0; 1024 * j0 < n; j0 += AHEAD * CH) { // block-uniform
+#pragma unroll
+            for (int g = 0; g < AHEAD; ++g) {
+                filter(j0 + g * CH, v[g]);
+                if (1024 * (j0 + (g + AHEAD) * CH) < n) request(j0 + (g + AHEAD) * CH, v[g]);
+                __builtin_amdgcn_sched_barrier(0); // (no further look-ahead: it would cost registers)
+            }
+        }
+    }
+    bottom = wave_min(bottom);
+    top = wave_max(top);
+    if (lane == 0) {
+        atomicMin(&lds.tmp[14], bottom);
+        atomicMax(&lds.tmp[15], top);
+    }
+    __syncthreads();
+    uint32_t m = lds.out, kmin = lds.tmp[14] + 1u, kmax = lds.tmp[15];
+    const bool exact = m < (uint32_t)k || m > ROW_CAP; // block-uniform
+    if (exact) {
+        row_select_exact(lds, n, k, load);
+        m = (uint32_t)k;
+    }
+    uint64_t w[ROW_CAP / 1024];
+#pragma unroll
+    for (int h = 0; h < ROW_CAP / 1024; ++h) w[h] = lds.buf[tid + 1024 * h];
+    if (exact) {
+        if (tid == 0) {
+            lds.tmp[14] = 0xffffffffu;
+            lds.tmp[15] = 0u;
+        }
+        __syncthreads();
+        kmin = 0xffffffffu;
+        kmax = 0u;
+#pragma unroll
+        for (int h = 0; h < ROW_CAP / 1024; ++h)
+            if ((uint32_t)(tid + 1024 * h) < m) {
+                kmin = min(kmin, (uint32_t)(w[h] >> 32));
+                kmax = max(kmax, (uint32_t)(w[h] >> 32));
+            }
+        block_key_range(kmin, kmax, lds.tmp);
+    }
+    order_words<ROW_CAP / 1024>(w, m, kmin, kmax, lds.buf, lds.hist, lds.start, lds.tmp, &lds.cnt, k, write);
+}
+
+// The indexer's selection as one kernel over the score rows, for rows of at most INDEXER_ROW_MAX keys: no histograms, no
+// lists in the workspace, one launch less.  Indices only, -1 behind the last.
+template <int NPT>
+__global__ __launch_bounds__(1024) void indexer_row_topk_kernel(IndexerArgs a)
+{
+    __shared__ RowLds lds;
+    const int tid = threadIdx.x, row = blockIdx.x;
+    const float* x = a.scores + (int64_t)row * a.score_stride;
+    int32_t* out = a.topk_res + (int64_t)row * a.k;
+    auto length = [&]() {
+        const int n = row_length(a.act_seq, row, a.s1, a.max_ctx);
+        for (int j = min(n, a.k) + tid; j < a.k; j += 1024) out[j] = -1;
+        return n;
+    };
+    select_row<NPT, 4>(lds, a.score_stride, a.k, [&](int i) { return x[i]; },
+                       [&](int i) { return *reinterpret_cast<const f32x4*>(x + i); }, length,
+                       [&](int rank, uint64_t w) { out[rank] = word_index(w); });
+}
+
+// 16 rows of 20000, k = 2048: 14.6 us (counting passes that read the row twice per 11 bits, and a bitonic sort of all selected
+// words: 53); 2 rows of 4440, k = 563: 7 us (the row sorted whole: 66).
+template <int NPT>
+__global__ __launch_bounds__(1024) void topk_select_kernel(const float* __restrict__ x, float* __restrict__ values,
+                                                           int32_t* __restrict__ indices, int n, int k, int largest)
+{
+    __shared__ RowLds lds;
+    const float* row = x + (int64_t)blockIdx.x * n;
+    auto load = [&](int i) { return largest ? row[i] : -row[i]; };
+    int32_t* out_i = indices + (int64_t)blockIdx.x * k;
+    float* out_v = values + (int64_t)blockIdx.x * k;
+    select_row<NPT, 1>(lds, n, k, load, [&](int) { return f32x4{}; }, [&]() { return n; }, [&](int rank, uint64_t w) {
+        const int i = word_index(w);
+        float v = key_to_score((uint32_t)(w >> 32));
+        v = largest ? v : -v;
+        // (the key has lost the sign of a zero and may have lost a NaN's bits: those come from the row)
+        if (!(fabsf(v) > 0.f)) v = row[i];
+        out_i[rank] = i;
+        out_v[rank] = v;
+    });
 }
 
 } // namespace
@@ -987,17 +1242,29 @@ bool topk_supported(int64_t n, int64_t k) { return n >= 1 && k >= 1 && k <= n &&
 hipError_t topk_launch(const float* x, float* values, int32_t* indices, int64_t rows, int n, int k, bool largest, hipStream_t stream)
 {
     if (rows == 0) return hipSuccess;
-    hipLaunchKernelGGL(topk_rows_kernel, dim3((unsigned)rows), dim3(1024), 0, stream, x, values, indices, n, k, largest ? 1 : 0);
+    void (*kern)(const float*, float*, int32_t*, int, int, int) =
+        n <= TOPK_SORT_SMALL || k > MAX_K ? topk_sort_kernel : n <= 4096 ? topk_select_kernel<4> :
+        n <= 16384 ? topk_select_kernel<16> : topk_select_kernel<0>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(1024), 0, stream, x, values, indices, n, k, largest ? 1 : 0);
     return hipGetLastError();
 }
 
 // workspace: scores [t, stride] f32 | span_hist [t, spans, 256] u16 | counters [t, 4] u32 | winners [t, 2048] u64 |
-// ties [t, 8192] u64; spans = stride / 2048
+// ties [t, 8192] u64; spans = stride / span
 static uint64_t align256(uint64_t x) { return (x + 255) & ~(uint64_t)255; }
+
+// Passes of 512 keys per workgroup of the paged score kernel: four (the query's set-up is paid once per 2048 keys) where
+// that still leaves every CU its fill of workgroups, fewer where the batch and its contexts are small - a single 4 K
+// context is 2 workgroups of four passes, and took 13.5 us.
+static int pick_passes(int64_t t, int64_t stride)
+{
+    const int64_t groups = t * (stride / CHUNK);
+    return groups >= 4 * SCORE_GROUPS ? 4 : groups >= 2 * SCORE_GROUPS ? 2 : 1;
+}
 
 uint64_t indexer_workspace_bytes(int t, int stride)
 {
-    const uint64_t spans = (uint64_t)stride / SPAN;
+    const uint64_t spans = (uint64_t)stride / (CHUNK * pick_passes(t, stride));
     return align256((uint64_t)t * stride * 4) + align256((uint64_t)t * spans * SBINS * 2) + align256((uint64_t)t * 4 * 4) +
            align256((uint64_t)t * (MAX_K + TIE_CAP) * 8);
 }
@@ -1005,7 +1272,9 @@ uint64_t indexer_workspace_bytes(int t, int stride)
 void indexer_bind_workspace(IndexerArgs& a, void* ws)
 {
     const int t = a.b * a.s1;
-    const uint64_t spans = (uint64_t)a.score_stride / SPAN;
+    // (the unpaged kernel's spans have four passes always)
+    a.span = a.block_size % 128 == 0 ? CHUNK * pick_passes(t, a.score_stride) : CHUNK * PASSES;
+    const uint64_t spans = (uint64_t)a.score_stride / a.span;
     uint8_t* p = static_cast<uint8_t*>(ws);
     a.scores = reinterpret_cast<float*>(p);
     p += align256((uint64_t)t * a.score_stride * 4);
@@ -1018,6 +1287,15 @@ void indexer_bind_workspace(IndexerArgs& a, void* ws)
     a.pchunks = (int32_t)spans;
 }
 
+template <int PPASSES>
+static void launch_score_paged(const IndexerArgs& a, hipStream_t stream)
+{
+    const bool s2 = a.s1 % 2 == 0;
+    auto kern = s2 ? (a.scales_f32 ? indexer_score_paged_kernel<2, true, PPASSES> : indexer_score_paged_kernel<2, false, PPASSES>)
+                   : (a.scales_f32 ? indexer_score_paged_kernel<1, true, PPASSES> : indexer_score_paged_kernel<1, false, PPASSES>);
+    hipLaunchKernelGGL(kern, dim3((a.max_ctx + CHUNK * PPASSES - 1) / (CHUNK * PPASSES), a.b, s2 ? a.s1 / 2 : a.s1), dim3(256), 0, stream, a);
+}
+
 hipError_t indexer_launch(const IndexerArgs& a, hipStream_t stream)
 {
     const int t = a.b * a.s1;
@@ -1028,36 +1306,37 @@ hipError_t indexer_launch(const IndexerArgs& a, hipStream_t stream)
         hipLaunchKernelGGL(indexer_fill_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, a.topk_res, n, -1);
         return hipGetLastError();
     }
-    // one workgroup per 2048-key span the page table can address (a.pchunks slots per query token hold at least as many)
-    const int chunks = (max_ctx + SPAN - 1) / SPAN;
-    const int pchunks = chunks;
+    // one workgroup per span of keys the page table can address (a.pchunks slots per query token hold at least as many)
     IndexerArgs args = a;
     args.max_ctx = max_ctx;
+    args.use_hist = max_ctx > INDEXER_ROW_MAX;
     {
         ScopedKernelTimer tm(KID_INDEXER_SCORE, stream);
-        const bool pow2 = (a.block_size & (a.block_size - 1)) == 0;
-        const bool s2 = a.s1 % 2 == 0, f32 = a.scales_f32;
         if (a.block_size % 128 == 0) {
-            auto kern = s2 ? (f32 ? indexer_score_paged_kernel<2, true> : indexer_score_paged_kernel<2, false>)
-                           : (f32 ? indexer_score_paged_kernel<1, true> : indexer_score_paged_kernel<1, false>);
-            hipLaunchKernelGGL(kern, dim3(pchunks, a.b, s2 ? a.s1 / 2 : a.s1), dim3(256), 0, stream, args);
+            if (a.span == 4 * CHUNK) launch_score_paged<4>(args, stream);
+            else if (a.span == 2 * CHUNK) launch_score_paged<2>(args, stream);
+            else launch_score_paged<1>(args, stream);
         } else {
+            const bool pow2 = (a.block_size & (a.block_size - 1)) == 0;
+            const bool s2 = a.s1 % 2 == 0, f32 = a.scales_f32;
             auto kern = s2 ? (pow2 ? (f32 ? indexer_score_kernel<2, true, true> : indexer_score_kernel<2, true, false>)
                                    : (f32 ? indexer_score_kernel<2, false, true> : indexer_score_kernel<2, false, false>))
                            : (pow2 ? (f32 ? indexer_score_kernel<1, true, true> : indexer_score_kernel<1, true, false>)
                                    : (f32 ? indexer_score_kernel<1, false, true> : indexer_score_kernel<1, false, false>));
-            hipLaunchKernelGGL(kern, dim3(chunks, a.b, s2 ? a.s1 / 2 : a.s1), dim3(256), 0, stream, args);
+            hipLaunchKernelGGL(kern, dim3((max_ctx + a.span - 1) / a.span, a.b, s2 ? a.s1 / 2 : a.s1), dim3(256), 0, stream, args);
         }
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    {
+    if (args.use_hist) {
         ScopedKernelTimer tm(KID_INDEXER_SELECT, stream);
         hipLaunchKernelGGL(indexer_select_kernel, dim3((max_ctx + SEL_CHUNK - 1) / SEL_CHUNK, t), dim3(256), 0, stream, args);
     }
     {
         ScopedKernelTimer tm(KID_INDEXER_TOPK, stream);
-        hipLaunchKernelGGL(indexer_topk_kernel, dim3(t), dim3(1024), 0, stream, args);
+        auto kern = args.use_hist ? indexer_topk_kernel : max_ctx <= 4096 ? indexer_row_topk_kernel<4> :
+                    max_ctx <= 16384 ? indexer_row_topk_kernel<16> : indexer_row_topk_kernel<0>;
+        hipLaunchKernelGGL(kern, dim3(t), dim3(1024), 0, stream, args);
     }
     return hipGetLastError();
 }

@@ -49,7 +49,7 @@ struct IndexerArgs {
     const int32_t* block_table;  // [b, bt_stride]
     int32_t* topk_res;           // [t, k]
     float* scores;               // workspace [t, score_stride]
-    uint16_t* span_hist;         // workspace [t, pchunks, 256]: per 2048-key span, histogram of the score keys (quarter octaves)
+    uint16_t* span_hist;         // workspace [t, pchunks, 256]: per span of keys, histogram of the score keys (quarter octaves)
     uint32_t* counters;          // workspace [t, 4]: winners, ties (cleared by the score kernel)
     uint64_t* winners;           // workspace [t, 2048]
     uint64_t* ties;              // workspace [t, 8192]
@@ -57,7 +57,9 @@ struct IndexerArgs {
     int32_t b, s1, nh, block_size, bt_stride, k, score_stride;
     int32_t max_ctx; // set by indexer_launch: bt_stride * block_size, the longest sequence the page table can address
     bool scales_f32; // q_scale and k_scale are fp32: w_scale = fp16(q_scale * fp32(weight)), k_scale enters the score as it is
-    int32_t pchunks; // set by indexer_bind_workspace: histogram slots (2048-key spans) per query token = score_stride / 2048
+    int32_t span;    // set by indexer_bind_workspace: keys per workgroup of the score kernel
+    int32_t pchunks; // set by indexer_bind_workspace: histogram slots (spans of keys) per query token = score_stride / span
+    bool use_hist;   // set by indexer_launch: the selection needs the score kernel's histograms
 };
 
 uint64_t indexer_workspace_bytes(int t, int score_stride);

@@ -140,6 +140,20 @@ def test_all_scores_equal_keeps_the_first_indices(cuda):
     assert torch.equal(got[0, 0], want) and torch.equal(got[1, 0], want)
 
 
+@pytest.mark.parametrize("act", [[4095, 4096, 300], [4097, 16383, 2049], [16384, 100], [16385, 5000], [32768, 2048], [32769, 4097]])
+def test_row_lengths_at_the_selection_kernels_edges(cuda, act):
+    """The longest context picks the selection kernel (rows of up to 4096, 16384 and 32768 keys by one kernel, longer ones by
+    two); the others are short rows under it.  Then the same lengths with every key alike: the answer is the first indices."""
+    case = oi.make_case(len(act), 1, act, seed=sum(act))
+    check_topk(case, run_indexer(case, cuda))
+    case["key_cache"][:] = case["key_cache"][0, 0]
+    case["k_scale"][:] = case["k_scale"][0, 0]
+    got = run_indexer(case, cuda)
+    for r, n in enumerate(act):
+        m = min(n, 2048)
+        assert torch.equal(got[r, 0, :m], torch.arange(m, dtype=torch.int32)) and (got[r, 0, m:] == -1).all()
+
+
 def test_all_scores_zero(cuda):
     # relu kills every head: scores are +0 / -0, which the ordering must treat as equal
     case = oi.make_case(1, 2, [5000], seed=7)

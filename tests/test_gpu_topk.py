@@ -90,3 +90,20 @@ def test_errors(cuda):
         topk(x[:, :8].contiguous(), 9)
     with pytest.raises(FeError, match="float32"):
         topk(x.half(), 2)
+
+
+@pytest.mark.parametrize("n", [128, 129, 1025, 4095, 4096, 4097, 16384, 16385, 32768, 33000, 70001])
+def test_row_lengths_at_the_kernels_edges(cuda, n):
+    """One element more or less than a lane's, the candidate list's and a request group's capacity; bell-shaped rows (the
+    sampled pivot serves), heavy ties, a row in step with the samples (every 16th element of 65536 is large: the pivot
+    comes out too high), one far outlier, and infinities."""
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn((5, n), generator=g)
+    x[1] = torch.randint(-2, 3, (n,), generator=g).float()
+    x[2, ::max(n // 4096, 2)] += 100.0
+    x[3, n // 3] = 1e30
+    x[4, n // 2] = float("inf")
+    x[4, 0] = float("-inf")
+    for k in (1, min(n, 2048)):
+        check(x, k, None, True, cuda)
+    check(x, min(n, 100), None, False, cuda)
