@@ -79,6 +79,7 @@ struct SelectExpertsArgs {
     int32_t* topk_ids;   // [t, top_k]
     int64_t t;
     int32_t ne, top_k, topk_group, n_group;
+    uint32_t group_magic; // set by select_experts_launch: expert / group size as a multiplication
     float routed_scaling_factor;
     bool renormalize, fill_neg_inf, logits_bf16, bias_bf16;
 };

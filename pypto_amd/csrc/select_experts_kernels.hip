@@ -2,8 +2,8 @@
 // weights.  Reference: models/glm_v4_5/glm_select_experts.py:60-228 (kernel) and :274-313 (golden);
 // python/tests/ut/interpreter/_ops/moe_gating_topk.py:223-287 (groups, -inf fill, scaling factor).
 //
-// The whole problem is a few MB (8192 x 160 logits): what bounds the kernels is vector instruction issue, more than half
-// of it the double-precision sigmoid.  Groups are ranked by counting (rank of g = number of groups that come before g
+// The whole problem is a few MB (8192 x 160 logits): what bounds the kernels is vector instruction issue (many tokens) and
+// the length of one wavefront's instruction chain (few), both mostly the sigmoid and the arg-max rounds.  Groups are ranked by counting (rank of g = number of groups that come before g
 // in the order "value descending, index ascending"), experts by top_k rounds of an arg-max on (ordered score, ~id).
 // select_experts_rows_kernel puts four tokens in a wavefront (the router's shapes); select_experts_kernel, one token per
 // wavefront, takes the shapes with more than 16 groups or 16 selected experts.
@@ -26,6 +26,37 @@ __device__ __forceinline__ float load_as_f32(const uint16_t* p, int64_t i) { ret
 
 // true when (v2, e2) comes before (v, e)
 __device__ __forceinline__ int before(float v2, int e2, float v, int e) { return (v2 > v) || (v2 == v && e2 < e); }
+
+// sigmoid(x) = 1 / (1 + exp(-x)) in double precision, rounded once to fp32: the correctly rounded value but for about one
+// argument in 10^8, whose exact value lies within 1e-15 of the middle between two floats (as with any double-precision
+// exp).  exp by Cody-Waite reduction to |r| <= ln2 / 2 and the Taylor polynomial of degree 12 (remainder below 2e-16), the
+// reciprocal by two Newton steps: 33 instructions where the library's exp and division take about 110.  The argument is
+// clamped where the fp32 result no longer changes (0 and 1 from |x| = 104 and 17 on).
+__device__ __forceinline__ float sigmoid_f32(float x)
+{
+    const double t = -(double)fminf(fmaxf(x, -200.f), 200.f);
+    const double k = __builtin_rint(t * 1.4426950408889634);
+    double r = __builtin_fma(k, -0x1.62e42fefa0000p-1, t);     // ln 2 cut to 36 bits: k times it is exact
+    r = __builtin_fma(k, -0x1.cf79abc9e3b398p-40, r);          // the rest of ln 2
+    double p = 1.0 / 479001600.0;
+    p = __builtin_fma(p, r, 1.0 / 39916800.0);
+    p = __builtin_fma(p, r, 1.0 / 3628800.0);
+    p = __builtin_fma(p, r, 1.0 / 362880.0);
+    p = __builtin_fma(p, r, 1.0 / 40320.0);
+    p = __builtin_fma(p, r, 1.0 / 5040.0);
+    p = __builtin_fma(p, r, 1.0 / 720.0);
+    p = __builtin_fma(p, r, 1.0 / 120.0);
+    p = __builtin_fma(p, r, 1.0 / 24.0);
+    p = __builtin_fma(p, r, 1.0 / 6.0);
+    p = __builtin_fma(p, r, 0.5);
+    p = __builtin_fma(p, r, 1.0);
+    p = __builtin_fma(p, r, 1.0);
+    const double d = 1.0 + __builtin_amdgcn_ldexp(p, (int)k);
+    double y = __builtin_amdgcn_rcp(d);
+    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+    return x == x ? (float)y : x; // (the clamp would lose a NaN)
+}
 
 // Wavefront-wide maximum of a u32, the same value in every lane, in the vector unit's own lane network (DPP row_shr
 // steps inside the rows of 16 lanes, row_bcast15 / row_bcast31 across them).
@@ -84,8 +115,7 @@ __global__ __launch_bounds__(64) void select_experts_kernel(SelectExpertsArgs a)
             own_s[j] = 0.f;
             if (e < ne) {
                 const float x = load_as_f32(logits, tok * ne + e);
-                // sigmoid in double, rounded once: the correctly rounded fp32 value whatever the libm
-                const float sg = (float)(1.0 / (1.0 + exp(-(double)x)));
+                const float sg = sigmoid_f32(x);
                 own_s[j] = sg;
                 own_x[j] = sg + bs[j];
             }
@@ -143,124 +173,223 @@ __global__ __launch_bounds__(64) void select_experts_kernel(SelectExpertsArgs a)
     }
 }
 
-// The same selection with four tokens per wavefront, one per row of 16 lanes: lane c of a row holds experts c, c + 16,
-// ... (NS of them), so no lane idles at 160 experts and every cross-lane step serves four tokens at once.  Reductions run
-// inside the rows - a maximum by four rotations (row_ror 8, 4, 2, 1: every lane of the row ends up with it) - group ranks by
-// rotating the row's group maxima past every lane.  For up to 16 groups and 16 selected experts (the router's shapes).
+// The same selection with four tokens per wavefront, one per row of 16 lanes: lane c of a row holds experts 32 i + 2 c and
+// 32 i + 2 c + 1 (NS in all), so no lane idles at 160 experts, every cross-lane step serves four tokens at once and logits
+// and bias come two to a load.  Reductions run inside the rows - a maximum by four rotations (row_ror 8, 4, 2, 1: every
+// lane of the row ends up with it) - group ranks by rotating the row's group maxima past every lane.  For up to 16 groups
+// and 16 selected experts (the router's shapes).
+//
+// (ordered score, ~id) of an expert are the mantissa of one double (order_word), so a comparison of both is one instruction.
+// Up to eight selected experts (TOP8): every lane sorts its own and keeps eight, and four merges with the lanes 8, 4, 2 and 1
+// places away leave the row's eight in order in all of its lanes - about 300 instructions where eight arg-max rounds over
+// score and id took 800.  More: rounds of an arg-max.  The selected experts' sigmoid values are read back from LDS.
+// 8192 tokens x 160 experts, 8 of 4 of 8 groups: 11.1 us with the library's exp and the rounds, 7.7 now; 8 tokens: 9.2
+// us, 4.8 now (what is left is one wavefront's chain: loads, 33 dependent double-precision steps, the merges).
 template <int N>
 __device__ __forceinline__ uint32_t row_ror(uint32_t v)
 {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x120 + N, 0xf, 0xf, false);
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x120 + N, 0xf, 0xf, true);
 }
-__device__ __forceinline__ uint32_t row_max_u32(uint32_t v)
+template <int N>
+__device__ __forceinline__ double row_ror_max(double v)
 {
-    v = max(v, row_ror<8>(v));
-    v = max(v, row_ror<4>(v));
-    v = max(v, row_ror<2>(v));
-    v = max(v, row_ror<1>(v));
-    return v;
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint64_t o = ((uint64_t)row_ror<N>((uint32_t)(b >> 32)) << 32) | row_ror<N>((uint32_t)b);
+    return __builtin_fmax(v, __builtin_bit_cast(double, o));
 }
-template <int K>
-__device__ __forceinline__ void rank_step(int& rank, float m, int c, int delta, int ng)
+// (ordered value, smaller index first) as one double, exact: 2^52 + value * 256 + (255 - index)
+__device__ __forceinline__ double order_word(uint32_t value, int index)
 {
-    if constexpr (K < 16) {
-        const float m2 = __builtin_bit_cast(float, row_ror<K>(__builtin_bit_cast(uint32_t, m)));
-        const int g2 = (c + K * delta) & 15; // the lane of the row the rotation brought here
-        rank += (g2 < ng) & before(m2, g2, m, c);
-        rank_step<K + 1>(rank, m, c, delta, ng);
+    return __builtin_bit_cast(double, 0x4330000000000000ull | ((uint64_t)value << 8) | (uint32_t)(255 - index));
+}
+__device__ __forceinline__ int order_word_index(double w) { return 255 - (int)(__builtin_bit_cast(uint64_t, w) & 255u); }
+// rank of m among the row's words, by rotating the row past every lane: K = 1 .. LAST rotations (the words of a row that
+// repeat with period 8 are all seen after 7)
+template <int K, int LAST>
+__device__ __forceinline__ void rank_step(int& rank, double m)
+{
+    if constexpr (K <= LAST) {
+        const uint64_t b = __builtin_bit_cast(uint64_t, m);
+        const uint64_t o = ((uint64_t)row_ror<K>((uint32_t)(b >> 32)) << 32) | row_ror<K>((uint32_t)b);
+        rank += __builtin_bit_cast(double, o) > m ? 1 : 0;
+        rank_step<K + 1, LAST>(rank, m);
     }
 }
 
-template <typename LT, typename BT, int NS>
+// a and b in descending order
+__device__ __forceinline__ void order_pair(double& a, double& b)
+{
+    const double hi = __builtin_fmax(a, b), lo = __builtin_fmin(a, b);
+    a = hi;
+    b = lo;
+}
+// k[0 .. N) in descending order: Batcher's odd-even merge sort, N a power of two
+template <int N>
+__device__ __forceinline__ void sort_desc(double* k)
+{
+#pragma unroll
+    for (int p = 1; p < N; p *= 2)
+#pragma unroll
+        for (int q = p; q >= 1; q /= 2)
+#pragma unroll
+            for (int j = q % p; j + q < N; j += 2 * q)
+#pragma unroll
+                for (int i = 0; i < q; ++i)
+                    if (i + j + q < N && (i + j) / (2 * p) == (i + j + q) / (2 * p)) order_pair(k[i + j], k[i + j + q]);
+}
+// k[0 .. 8), a bitonic sequence, in descending order
+__device__ __forceinline__ void merge8_desc(double* k)
+{
+#pragma unroll
+    for (int q = 4; q >= 1; q /= 2)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if ((i & q) == 0) order_pair(k[i], k[i + q]);
+}
+// k: the eight largest words of the lane, descending -> those of the lane and the lane N places round the row
+template <int N>
+__device__ __forceinline__ void merge_lanes(double (&k)[8])
+{
+    double o[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint64_t b = __builtin_bit_cast(uint64_t, k[i]);
+        o[i] = __builtin_bit_cast(double, ((uint64_t)row_ror<N>((uint32_t)(b >> 32)) << 32) | row_ror<N>((uint32_t)b));
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) k[i] = __builtin_fmax(k[i], o[7 - i]);
+    merge8_desc(k);
+}
+// elements e and e + 1 (e even) of a row of n; `pairs`: n is even, so the pair is aligned and inside
+__device__ __forceinline__ void load_pair(const float* p, int64_t row, int e, int n, bool pairs, float& a, float& b)
+{
+    if (pairs) {
+        const float2 v = *reinterpret_cast<const float2*>(p + row * n + e);
+        a = v.x;
+        b = v.y;
+    } else {
+        a = p[row * n + e];
+        b = p[row * n + min(e + 1, n - 1)];
+    }
+}
+__device__ __forceinline__ void load_pair(const uint16_t* p, int64_t row, int e, int n, bool pairs, float& a, float& b)
+{
+    if (pairs) {
+        const uint32_t v = *reinterpret_cast<const uint32_t*>(p + row * n + e);
+        a = __uint_as_float(v << 16);
+        b = __uint_as_float(v & 0xffff0000u);
+    } else {
+        a = load_as_f32(p, row * n + e);
+        b = load_as_f32(p, row * n + min(e + 1, n - 1));
+    }
+}
+
+template <typename LT, typename BT, int NS, bool TOP8>
 __global__ __launch_bounds__(64) void select_experts_rows_kernel(SelectExpertsArgs a)
 {
     __shared__ uint32_t s_gkey[4][16];
+    __shared__ float s_sig[4][16 * NS];
+    __shared__ __align__(16) float s_w[4][16];
 
     const int lane = threadIdx.x, row = lane >> 4, c = lane & 15;
-    const int ne = a.ne, ng = a.n_group, gs = ne / ng;
+    const int ne = a.ne, ng = a.n_group;
     const LT* logits = static_cast<const LT*>(a.logits);
     const BT* bias = static_cast<const BT*>(a.bias);
     const float fill = a.fill_neg_inf ? -__builtin_inff() : 0.0f;
-    // which way row_ror turns, found out once: lane c receives lane (c + delta) & 15
-    const int delta = ((int)row_ror<1>((uint32_t)c) - c) & 15;
-    int grp[NS];
-    float bs[NS];
-#pragma unroll
-    for (int j = 0; j < NS; ++j) {
-        const int e = c + 16 * j;
-        grp[j] = e < ne ? e / gs : 0;
-        bs[j] = e < ne ? load_as_f32(bias, e) : 0.f;
-    }
+    const bool pairs = (ne & 1) == 0;
+    auto expert = [&](int j) { return 32 * (j >> 1) + 2 * c + (j & 1); };
 
+    float bs[NS];
+    bool have_bias = false;
     for (int64_t tok0 = (int64_t)blockIdx.x * 4; tok0 < a.t; tok0 += (int64_t)gridDim.x * 4) {
         const int64_t tok = tok0 + row;
         const bool live = tok < a.t;
         const int64_t tl = live ? tok : a.t - 1; // (rows past the last token work on the last one and store nothing)
-        float own_x[NS], own_s[NS];
-        if (c < ng) s_gkey[row][c] = 0u;
+        float x[NS];
+        // (slots past the last expert load it again and are left out below)
 #pragma unroll
-        for (int j = 0; j < NS; ++j) {
-            const int e = c + 16 * j;
-            own_x[j] = 0.f;
-            own_s[j] = 0.f;
-            if (e < ne) {
-                const float x = load_as_f32(logits, tl * ne + e);
-                // sigmoid in double, rounded once: the correctly rounded fp32 value whatever the libm
-                const float sg = (float)(1.0 / (1.0 + exp(-(double)x)));
-                own_s[j] = sg;
-                own_x[j] = sg + bs[j];
-            }
+        for (int j = 0; j < NS; j += 2) load_pair(logits, tl, min(expert(j), (ne - 1) & ~1), ne, pairs, x[j], x[j + 1]);
+        if (!have_bias) {
+#pragma unroll
+            for (int j = 0; j < NS; j += 2) load_pair(bias, 0, min(expert(j), (ne - 1) & ~1), ne, pairs, bs[j], bs[j + 1]);
+            have_bias = true;
         }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < NS; ++j)
-            if (c + 16 * j < ne) atomicMax(&s_gkey[row][grp[j]], f32_to_ordered(own_x[j]));
-        __syncthreads();
-        // lane g < ng of a row: the maximum of the token's group g and its rank (value descending, index ascending)
-        const float m = ordered_to_f32(s_gkey[row][c < ng ? c : 0]);
-        int rank = 0;
-        rank_step<1>(rank, m, c, delta, ng);
-        const uint64_t keep = __ballot(c < ng && rank < a.topk_group); // bit 16 row + g
-        uint32_t hi[NS], lo[NS];
+        float own_x[NS];
 #pragma unroll
         for (int j = 0; j < NS; ++j) {
-            const int e = c + 16 * j;
-            if (!((keep >> (16 * row + grp[j])) & 1ull)) own_x[j] = fill;
-            hi[j] = e < ne ? f32_to_ordered(own_x[j] + 0.0f) : 0u;
-            lo[j] = e < ne ? (uint32_t)(~e) : 0u;
+            const float sg = sigmoid_f32(x[j]);
+            own_x[j] = sg + bs[j];
+            s_sig[row][expert(j)] = sg;
+        }
+        uint64_t keep = ~0ull; // bit 16 row + g: group g is kept
+        if (ng > 1) { // (uniform) one group is kept whole
+            if (c < ng) s_gkey[row][c] = 0u;
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < NS; ++j)
+                if (expert(j) < ne) atomicMax(&s_gkey[row][__umul24((uint32_t)expert(j), a.group_magic) >> 16], f32_to_ordered(own_x[j]));
+            __syncthreads();
+            // lane g < ng of a row: the maximum of the token's group g and its rank (value descending, index ascending);
+            // up to eight groups are held twice by the row
+            const int g = ng <= 8 ? c & 7 : c;
+            const uint32_t gk = s_gkey[row][g < ng ? g : 0];
+            const double m = g < ng ? order_word(f32_to_ordered(ordered_to_f32(gk) + 0.0f), g) : 0.0;
+            int rank = 0;
+            if (ng <= 8) rank_step<1, 7>(rank, m);
+            else rank_step<1, 15>(rank, m);
+            keep = __ballot(c < ng && rank < a.topk_group);
+        }
+        const uint32_t keep_row = (uint32_t)(keep >> (16 * row));
+        double key[NS];
+#pragma unroll
+        for (int j = 0; j < NS; ++j) {
+            const int e = expert(j);
+            const float v = (keep_row >> (__umul24((uint32_t)e, a.group_magic) >> 16)) & 1u ? own_x[j] : fill;
+            const uint32_t hi = f32_to_ordered(v + 0.0f);
+            key[j] = e < ne ? order_word(hi, e) : 0.0;
         }
         int my_id = 0;
-        float my_w = 0.f, sum = 0.f;
-        for (int r = 0; r < a.top_k; ++r) {
-            uint32_t h = hi[0];
+        if constexpr (TOP8) {
+            // the lane's eight largest, in order; then those of 2, 4, 8 and 16 lanes
+            double top[8];
+            sort_desc<8>(key);
+            sort_desc<NS - 8>(key + 8);
 #pragma unroll
-            for (int j = 1; j < NS; ++j) h = max(h, hi[j]);
-            const uint32_t hmax = row_max_u32(h);
-            uint32_t cand = 0u;
+            for (int i = 0; i < 8; ++i) top[i] = 7 - i < NS - 8 ? __builtin_fmax(key[i], key[15 - i]) : key[i];
+            merge8_desc(top);
+            merge_lanes<8>(top);
+            merge_lanes<4>(top);
+            merge_lanes<2>(top);
+            merge_lanes<1>(top);
 #pragma unroll
-            for (int j = 0; j < NS; ++j) cand = max(cand, hi[j] == hmax ? lo[j] : 0u);
-            const uint32_t lmax = row_max_u32(cand);
-            // the winner's sigmoid value (positive, so its bits order like the value): only its owner offers it
-            uint32_t wb = 0u;
+            for (int i = 0; i < 8; ++i) my_id = c == i ? order_word_index(top[i]) : my_id;
+        } else {
+            for (int r = 0; r < a.top_k; ++r) {
+                double best = key[0];
 #pragma unroll
-            for (int j = 0; j < NS; ++j) {
-                const bool win = hi[j] == hmax && lo[j] == lmax;
-                wb = max(wb, win ? __builtin_bit_cast(uint32_t, own_s[j]) : 0u);
-                hi[j] = win ? 0u : hi[j];
-            }
-            const float w = __builtin_bit_cast(float, row_max_u32(wb));
-            sum += w;
-            if (c == r) {
-                my_id = (int)~lmax;
-                my_w = w;
+                for (int j = 1; j < NS; ++j) best = __builtin_fmax(best, key[j]);
+                best = row_ror_max<8>(best);
+                best = row_ror_max<4>(best);
+                best = row_ror_max<2>(best);
+                best = row_ror_max<1>(best);
+#pragma unroll
+                for (int j = 0; j < NS; ++j) key[j] = key[j] == best ? 0.0 : key[j]; // (words are distinct)
+                my_id = c == r ? order_word_index(best) : my_id;
             }
         }
+        my_id = my_id < ne ? my_id : 0; // (fewer than eight experts in all: the lanes past the last have no word)
+        __syncthreads();
+        const float my_w = s_sig[row][my_id];
+        s_w[row][c] = my_w;
+        __syncthreads();
+        float sum = 0.f;
+        for (int r = 0; r < a.top_k; ++r) sum += s_w[row][r];
         if (live && c < a.top_k) {
             a.topk_ids[tok * a.top_k + c] = my_id;
             const float w = a.renormalize ? my_w / sum : my_w;
             a.topk_weights[tok * a.top_k + c] = w * a.routed_scaling_factor;
         }
-        __syncthreads(); // the group maxima are cleared for the next tokens only after every lane has read them
+        __syncthreads(); // LDS is written for the next tokens only after every lane has read it
     }
 }
 
@@ -278,19 +407,23 @@ static void launch_typed(const SelectExpertsArgs& a, hipStream_t stream)
     if (a.n_group <= 16 && a.top_k <= 16) {
         const int64_t wgs = (a.t + 3) / 4;
         const int grid = (int)(wgs < 16384 ? wgs : 16384);
-        if (a.ne <= 160)
-            hipLaunchKernelGGL((select_experts_rows_kernel<LT, BT, 10>), dim3(grid), dim3(64), 0, stream, a);
-        else
-            hipLaunchKernelGGL((select_experts_rows_kernel<LT, BT, 16>), dim3(grid), dim3(64), 0, stream, a);
+        const bool top8 = a.top_k <= 8;
+        auto kern = a.ne <= 160 ? (top8 ? select_experts_rows_kernel<LT, BT, 10, true> : select_experts_rows_kernel<LT, BT, 10, false>)
+                                : (top8 ? select_experts_rows_kernel<LT, BT, 16, true> : select_experts_rows_kernel<LT, BT, 16, false>);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(64), 0, stream, a);
     } else {
         const int grid = (int)(a.t < 16384 ? a.t : 16384);
         hipLaunchKernelGGL((select_experts_kernel<LT, BT>), dim3(grid), dim3(64), 0, stream, a);
     }
 }
 
-hipError_t select_experts_launch(const SelectExpertsArgs& a, hipStream_t stream)
+hipError_t select_experts_launch(const SelectExpertsArgs& args, hipStream_t stream)
 {
-    if (a.t == 0) return hipSuccess;
+    if (args.t == 0) return hipSuccess;
+    SelectExpertsArgs a = args;
+    // e / group size = e * ceil(2^16 / group size) >> 16 for e < 256: the product is off by less than e / 2^16 < 1 / group size
+    const int gs = a.ne / a.n_group;
+    a.group_magic = (uint32_t)((65536 + gs - 1) / gs);
     ScopedKernelTimer timer(KID_SELECT_EXPERTS, stream);
     if (a.logits_bf16) {
         if (a.bias_bf16) launch_typed<uint16_t, uint16_t>(a, stream);

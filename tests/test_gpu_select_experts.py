@@ -67,6 +67,19 @@ def test_dtypes_sizes_and_flags(cuda):
             check(logits, bias, k, renorm, tg, ng, cuda, scale=1.5, neg=bool(seed % 2))
 
 
+@pytest.mark.parametrize("t,ne,ng,tg,k", [(1, 7, 1, 1, 7), (3, 3, 3, 2, 2), (5, 159, 3, 2, 8), (6, 160, 16, 3, 9), (4, 160, 8, 8, 8),
+                                          (7, 161, 7, 3, 8), (2, 255, 5, 2, 8), (9, 256, 16, 16, 16), (1025, 33, 11, 4, 1)])
+def test_odd_expert_counts_and_both_selection_forms(cuda, t, ne, ng, tg, k):
+    """Odd expert counts (no paired loads), fewer experts than a lane row, up to 8 and more groups, up to 8 and more selected
+    experts, and logits whose sigmoid saturates: the correctly rounded value is 0 or 1 there."""
+    for ld in (torch.float32, torch.bfloat16):
+        logits, bias = ose.make_case(t, ne, t + ne, logits_dtype=ld, bias_dtype=torch.float32)
+        check(logits, bias, k, True, tg, ng, cuda, scale=1.5, neg=True)
+        check(logits, bias, k, False, tg, ng, cuda)
+    logits[:, ::2] = torch.tensor([-120.0, 40.0, -300.0, 3e38])[torch.arange((ne + 1) // 2) % 4].to(logits.dtype)
+    check(logits, bias, k, False, tg, ng, cuda)
+
+
 def test_exact_ties(cuda):
     logits = torch.zeros((3, 160))
     bias = torch.zeros(160, dtype=torch.bfloat16)
