@@ -493,8 +493,9 @@ int plan_gqa(const PtoTensorDesc* ts, uint32_t n, const PtoGqaParams* p, GqaPlan
     a.block_size = (int32_t)bs;
     a.bt_stride = (int32_t)ts[3].shape[1];
     a.softmax_scale = p->softmax_scale;
-    pto::gqa_pick_chunk((int)max_ctx, p->kv_chunk, &a.chunk, &a.nsplit);
-    plan->ws_bytes = pto::gqa_workspace_bytes(t, (int)nq, a.nsplit);
+    a.plan = nullptr;
+    pto::gqa_plan(a, p->kv_chunk);
+    plan->ws_bytes = pto::gqa_workspace_bytes(a);
     return PTO_OK;
 }
 
@@ -878,10 +879,7 @@ static int gqa_decode_launch_async(const PtoTensorDesc* tensors, uint32_t n_tens
         if (workspace == nullptr || workspace_bytes < plan.ws_bytes)
             return fail(PTO_ERR_WORKSPACE, "%s: workspace of %llu bytes required, got %llu", op,
                         (unsigned long long)plan.ws_bytes, (unsigned long long)(workspace ? workspace_bytes : 0));
-        pto::GqaArgs& a = plan.args;
-        const uint64_t rows = (uint64_t)a.b * a.s1 * a.nq;
-        a.part_o = static_cast<float*>(workspace);
-        a.part_ml = a.part_o + rows * a.nsplit * 128;
+        pto::gqa_bind_workspace(plan.args, workspace);
     }
     hipError_t e = pto::gqa_launch(plan.args, static_cast<hipStream_t>(hip_stream));
     if (e != hipSuccess) return fail(PTO_ERR_HIP, "%s: HIP launch failed: %s", op, hipGetErrorString(e));

@@ -5,18 +5,28 @@
 // does 12 flop per byte, so it is bound by HBM bandwidth; the design goal is to keep enough 16-byte loads in flight
 // and to touch every byte once.
 //
-// Grid: (KV chunk, KV head x 16-head sub-group, query token); 256 lanes = 4 wavefronts that free-run (no barrier in
-// the main loop).  A wave owns every fourth 32-token sub-tile of the chunk (so the four waves together walk whole
-// 128-token pages), prefetches the next sub-tile's K and V into registers while it works on the current one, and
-// keeps its own online-softmax state (m, l, O); the four states are merged through LDS at the end and written either
-// as the final bf16 rows (one chunk) or as fp32 partials that gqa_combine_kernel merges.
+// One workgroup per (KV chunk of a sequence, KV head, RT row tiles): a row tile is a query token of the sequence and up to 16
+// of the KV head's query heads.  256 lanes = 4 wavefronts that free-run (no barrier in the main loop).  A wave owns every
+// fourth 32-token sub-tile of the chunk (so the four waves together walk whole 128-token pages), moves it from registers to
+// its own LDS, requests the next one and computes, and keeps its own online-softmax state (m, l, O) per row tile; the four
+// states are merged through LDS at the end and written either as the final bf16 rows (one chunk per sequence) or as fp32
+// partials that gqa_combine_kernel merges.
+//   Loads take whole 256-byte cache rows, four to an instruction.  (K in the operand's layout straight from memory takes half
+// cache lines, twice, from 16 rows: 868 us against 853 at 4.8 GB, and unusable without cache retention.)
+//   Where the batch's keys do not fit the 256 MB last-level cache, they are loaded past it (non-temporal; a plain read
+// stream reaches 6.3 TB/s on this card, a non-temporal one 7.1): 853 -> 800 us.  Where they fit, the caches serve part of it.
+//   The page-table entries of 64 pages are held by a wavefront's lanes: a look-up from memory in front of every sub-tile
+// waited for the sub-tile in flight as well (loads complete in order): 1077 -> 868 us.
+//   Chunks are chosen on the device from the lengths (choose_chunk): as long as they can be while the workgroups fill the
+// chip a whole number of times.  Two row tiles per workgroup (two query tokens of a sequence) share every K and V byte.
+//   64 sequences of 4096 .. 32768 tokens, 96 / 8 heads: 1090 us with fixed chunks of 1024, 796 now (4.8 GB); 8
+// sequences up to 8192, 12 / 1 heads: 21 us, 13.5 now, most of it the chain lengths - page table - keys - merge.
 //
-//   S^T[token, head] = K Q^T : v_mfma_f32_16x16x32_bf16, A = K rows loaded from global memory straight into the
-//       operand layout (lane = token l%16, 8 dims at 8*(l/16) + 32*j), B = Q (resident, heads padded to 16).
-//   O^T[dim, head] += V^T P~^T : A = V^T through a wave-private, XOR-swizzled LDS tile and ds_read_b64_tr_b16,
-//       B = P~ rounded to bf16, which is exactly the register layout S^T comes out in (lane = head l%16, 4 tokens
-//       per 16-token block), so P~ never leaves registers.  The contraction index is visited in the order
-//       {4g..4g+3, 16+4g..16+4g+3} per lane group g on both operands.
+//   S^T[token, head] = K Q^T : v_mfma_f32_16x16x32_bf16, A = K rows (lane = token l%16, 8 dims at 8*(l/16) + 32*j), B = Q
+//       (resident, heads padded to 16).
+//   O^T[dim, head] += V^T P~^T : A = V^T by ds_read_b64_tr_b16, B = P~ rounded to bf16, which is exactly the register layout
+//       S^T comes out in (lane = head l%16, 4 tokens per 16-token block), so P~ never leaves registers.  The contraction
+//       index is visited in the order {4g..4g+3, 16+4g..16+4g+3} per lane group g on both operands.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -32,6 +42,9 @@ constexpr int GSUB = 32;     // tokens per wave sub-tile
 constexpr int GWAVES = 4;
 constexpr int GROW = GD * 2; // bytes per staged V row
 constexpr float LOG2E = 1.4426950408889634f;
+constexpr int GQA_SLOTS = 256;   // one workgroup per CU (two fit; twice as many shorter ones measured 5 to 15 % slower on small batches)
+constexpr int GQA_TARGET = 4096; // tokens a workgroup should have at most, where there are enough
+constexpr int GQA_MAX_SPLIT = 128; // chunks per sequence on average at most (the combine kernel walks them)
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -43,52 +56,173 @@ __device__ __forceinline__ s16x4 lds_read_tr(uint8_t* p) { return __builtin_amdg
 __device__ __forceinline__ int vswz(int t, int c16) { return ((((c16 >> 1) ^ (t & 7)) << 5) | ((c16 & 1) << 4)); }
 
 struct SubTile {
-    u32x4 k[2][4]; // [16-token block][k-step]: 8 dims of this lane's token
-    u32x4 v[8];    // row 4*i + l/16, 16-byte chunk l%16
+    u32x4 k[8], v[8]; // row 4*i + l/16, 16-byte chunk l%16
+    bool mapped;   // the page exists
 };
 
+// wavefront-wide inclusive prefix sum in the lane network
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ int gqa_dpp_add(int v)
+{
+    return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROW_MASK, 0xf, false);
+}
+__device__ __forceinline__ int gqa_prefix_sum(int v)
+{
+    v = gqa_dpp_add<0x111, 0xf>(v);
+    v = gqa_dpp_add<0x112, 0xf>(v);
+    v = gqa_dpp_add<0x114, 0xf>(v);
+    v = gqa_dpp_add<0x118, 0xf>(v);
+    v = gqa_dpp_add<0x142, 0xa>(v); // rows 1 and 3 add the totals of rows 0 and 2
+    return gqa_dpp_add<0x143, 0xc>(v);
+}
+
+// The lengths of up to GQA_SCAN sequences, by one wavefront: lane l holds those of sequences l, l + 64, ..  (cut to the page
+// table's reach; -1 past the last sequence).
+constexpr int GQA_SCAN = 256;
+struct Lengths {
+    int len[GQA_SCAN / 64];
+    __device__ __forceinline__ void fetch(const GqaArgs& a, int lane)
+    {
+        const int reach = a.bt_stride * a.block_size;
+#pragma unroll
+        for (int j = 0; j < GQA_SCAN / 64; ++j) len[j] = 64 * j < a.b ? a.act_seq[min(lane + 64 * j, a.b - 1)] : 0; // (requested together)
+#pragma unroll
+        for (int j = 0; j < GQA_SCAN / 64; ++j) len[j] = lane + 64 * j < a.b ? max(min(len[j], reach), 0) : -1;
+    }
+    // chunks of 128 c tokens of the lane's j-th sequence: an empty sequence has one too (its output rows are zero).  The
+    // quotient by way of fp32 is off by at most one and put right (the counts of 128 tokens are below 2^24: exact).
+    __device__ __forceinline__ int chunks(int j, int c, float inv_c) const
+    {
+        const int n = (len[j] + 127) >> 7;
+        int q = (int)((float)(n + c - 1) * inv_c);
+        const int r = n + c - 1 - q * c;
+        q += r < 0 ? -1 : r >= c ? 1 : 0;
+        return len[j] < 0 ? 0 : max(1, q);
+    }
+    __device__ __forceinline__ int units(const GqaArgs& a, int c) const
+    {
+        const float inv_c = 1.f / (float)c;
+        int n = 0;
+#pragma unroll
+        for (int j = 0; j < GQA_SCAN / 64; ++j)
+            if (64 * j < a.b) n += chunks(j, c, inv_c); // (uniform)
+        return __builtin_amdgcn_readlane(gqa_prefix_sum(n), 63);
+    }
+};
+
+// The batch's chunk length: the smallest multiple of 128 tokens that cuts it into no more units than fill the chip's
+// GQA_SLOTS workgroup slots a whole number of times - as many times as it takes to keep workgroups near GQA_TARGET tokens
+// (fewer, longer ones pay less for starting up and for partials; more even out what the memory system serves unevenly).
+// Depends on the lengths alone, so every wavefront finds the same one; the result never exceeds units_cap units.
+__device__ __forceinline__ int choose_chunk(const GqaArgs& a, const Lengths& ls)
+{
+    int sum = 0, longest = 0;
+#pragma unroll
+    for (int j = 0; j < GQA_SCAN / 64; ++j) {
+        if (64 * j >= a.b) break; // (uniform)
+        sum += (max(ls.len[j], 0) + 127) >> 7;
+        longest = max(longest, ls.len[j]);
+    }
+    sum = __builtin_amdgcn_readlane(gqa_prefix_sum(sum), 63);
+    // rounds of GQA_SLOTS workgroups with GQA_TARGET tokens
+    const int rounds = max((int)ceilf((float)sum * (float)a.columns * (128.f / GQA_SLOTS / GQA_TARGET)), 1);
+    const int target = min(max(rounds * GQA_SLOTS / a.columns, a.b), a.units_cap);
+    int lo = max((sum + target - 1) / target, 1); // (no shorter chunk can do)
+    if (ls.units(a, lo) <= target) return lo * 128;
+    longest = (int)wave_max_f32((float)longest) + 128; // the batch's (as a float it may be off by less than 128)
+    int hi = max((longest + 127) / 128, lo + 1); // one chunk per sequence: at most a.b <= target units
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (ls.units(a, mid) <= target) hi = mid;
+        else lo = mid;
+    }
+    return hi * 128;
+}
+
+// chunk length, and the (sequence, chunk) of unit u with the sequence's first unit; false: no such unit
+__device__ __forceinline__ bool gqa_unit(const GqaArgs& a, int u, int lane, int& chunk, int& bi, int& split)
+{
+    chunk = a.chunk;
+    if (a.b > GQA_SCAN) { // (fixed chunks by the unit's place)
+        bi = u / a.nsplit;
+        split = u - bi * a.nsplit;
+        return bi < a.b;
+    }
+    Lengths ls;
+    ls.fetch(a, lane);
+    if (chunk == 0) chunk = choose_chunk(a, ls);
+    const float inv_c = 1.f / (float)(chunk >> 7);
+    int base = 0;
+    bi = -1;
+#pragma unroll
+    for (int j = 0; j < GQA_SCAN / 64; ++j) {
+        if (64 * j >= a.b || bi >= 0) break; // uniform
+        const int cnt = ls.chunks(j, chunk >> 7, inv_c);
+        const int incl = gqa_prefix_sum(cnt), excl = incl - cnt;
+        const uint64_t hit = __ballot(u >= base + excl && u < base + incl); // at most one lane
+        if (hit != 0ull) {
+            const int l = __builtin_ctzll(hit);
+            bi = 64 * j + l;
+            split = u - base - __builtin_amdgcn_readlane(excl, l);
+        }
+        base += __builtin_amdgcn_readlane(incl, 63);
+    }
+    return bi >= 0;
+}
+
+template <int RT, bool NT>
 __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a)
 {
-    __shared__ __align__(16) uint8_t lds[GWAVES * GSUB * GROW]; // V staging, later the merge buffer (4 x 16 x 128 fp32)
+    // K and V staging, a pair of sub-tiles per wave; later the merge buffer (4 x 16 x 128 fp32)
+    __shared__ __align__(16) uint8_t lds[2 * GWAVES * GSUB * GROW];
     __shared__ float s_ml[GWAVES][16][2];
 
-    const int split = blockIdx.x;
-    const int n2 = blockIdx.y / a.hsub, hs = blockIdx.y % a.hsub;
-    const int tq = blockIdx.z;
-    const int bi = tq / a.s1, si = tq - bi * a.s1;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g4 = lane >> 4;
-
-    int cur = a.act_seq[bi] - (a.s1 - 1 - si);
-    cur = cur < 0 ? 0 : cur;
-    const int reach = a.bt_stride * a.block_size;
-    cur = cur > reach ? reach : cur;
-    const int start = split * a.chunk;
-    const int end = (start + a.chunk < cur) ? start + a.chunk : cur;
-
-    const int g = a.nq / a.nkv;
-    uint16_t* out = static_cast<uint16_t*>(a.out);
-    if (start >= end) {
-        if (a.nsplit == 1) { // nothing to attend: the output rows are zero
-            const int n = tid >> 4, hloc = hs * 16 + n;
-            if (hloc < g) {
-                const u32x4 z = {0u, 0u, 0u, 0u};
-                *reinterpret_cast<u32x4*>(out + ((int64_t)tq * a.nq + n2 * g + hloc) * GD + (tid & 15) * 8) = z;
-            }
-        }
-        return;
+    // Order of the workgroups: eight units side by side, and behind each other those that read the same keys, then the KV
+    // heads, whose rows lie beside each other in the cache.  Workgroups go to the eight dies in turn, so the readers of the
+    // same keys share an L2.
+    const int readers = a.s1 * a.hsub / RT;
+    int u, n2, rd;
+    {
+        const uint32_t lin = blockIdx.x + gridDim.x * blockIdx.y, per = 8u * readers * a.nkv;
+        const uint32_t o = lin / per, in = lin - o * per;
+        u = (int)(o * 8 + (in & 7));
+        rd = (int)((in >> 3) % readers) * RT;
+        n2 = (int)((in >> 3) / readers);
+    }
+    int bi, split, chunk;
+    if (!gqa_unit(a, u, lane, chunk, bi, split)) return;
+    if (a.part_o != nullptr && tid == 0 && rd == 0 && n2 == 0) { // for the combine kernel
+        if (u == 0) a.plan[0] = chunk;
+        if (split == 0) a.plan[1 + bi] = u;
     }
 
-    // Q fragment: B operand, lane = head r16 of this sub-group, dims 8*g4 + 32*j
-    u32x4 qf[4];
-    {
-        const int hloc = hs * 16 + r16;
+    const int g = a.nq / a.nkv;
+    const int len = min(a.act_seq[bi], a.bt_stride * a.block_size);
+    const int start = split * chunk;
+    int tok_q[RT], hs[RT], end_r[RT], end = 0; // row tile r: its query token, head sub-group and end of the chunk
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+        const int si = (rd + r) / a.hsub;
+        hs[r] = rd + r - si * a.hsub;
+        tok_q[r] = bi * a.s1 + si;
+        end_r[r] = min(start + chunk, min(max(a.act_seq[bi] - (a.s1 - 1 - si), 0), max(len, 0)));
+        end = max(end, end_r[r]);
+    }
+    uint16_t* out = static_cast<uint16_t*>(a.out);
+
+    // Q fragments: B operand, lane = head r16 of the row tile, dims 8*g4 + 32*j
+    u32x4 qf[RT][4];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+        const int hloc = hs[r] * 16 + r16;
         const bool ok = hloc < g;
-        const uint16_t* qp = static_cast<const uint16_t*>(a.q) + ((int64_t)tq * a.nq + n2 * g + (ok ? hloc : 0)) * GD;
+        const uint16_t* qp = static_cast<const uint16_t*>(a.q) + ((int64_t)tok_q[r] * a.nq + n2 * g + (ok ? hloc : 0)) * GD;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            qf[j] = *reinterpret_cast<const u32x4*>(qp + 8 * (g4 + 4 * j));
-            if (!ok) qf[j] = u32x4{0u, 0u, 0u, 0u};
+            qf[r][j] = *reinterpret_cast<const u32x4*>(qp + 8 * (g4 + 4 * j));
+            if (!ok) qf[r][j] = u32x4{0u, 0u, 0u, 0u};
         }
     }
 
@@ -96,120 +230,154 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a)
     const uint8_t* vbase = static_cast<const uint8_t*>(a.v) + (int64_t)n2 * GROW;
     const int64_t row_pitch = (int64_t)a.nkv * GROW;
     const int32_t* bt = a.block_table + (int64_t)bi * a.bt_stride;
-    uint8_t* myv = lds + w * (GSUB * GROW);
+    uint8_t* myk = lds + 2 * w * (GSUB * GROW);
+    uint8_t* myv = myk + GSUB * GROW;
 
-    const int nsub = (end - start + GSUB - 1) / GSUB;
+    const int nsub = (max(end - start, 0) + GSUB - 1) / GSUB;
     const float sc = a.softmax_scale * LOG2E;
 
-    f32x4 o[8];
+    f32x4 o[RT][8];
+    float m_run[RT], l_run[RT];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m_run = -INFINITY, l_run = 0.f;
+    for (int r = 0; r < RT; ++r) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[r][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        m_run[r] = -INFINITY;
+        l_run[r] = 0.f;
+    }
 
-    // a sub-tile lies inside one page (block_size is a multiple of 32 and chunks start on multiples of 128)
+    // Page-table entries: lane p holds that of page `window` + p (-1: none).  A sub-tile lies inside one page (block_size is a
+    // multiple of 32 and chunks start on multiples of 128).
+    int window = start / a.block_size;
+    int entry = -1;
+    auto fetch_entries = [&]() {
+        const int e = bt[min(window + lane, a.bt_stride - 1)];
+        entry = e >= 0 && e < a.n_blocks ? e : -1;
+    };
+    if (nsub > 0) fetch_entries();
     auto load = [&](int i, SubTile& t) {
         const int p0 = start + GSUB * i;
         const int page = p0 / a.block_size;
-        int blk = __builtin_amdgcn_readfirstlane(bt[page]);
-        blk = (blk < 0 || blk >= a.n_blocks) ? 0 : blk; // an unmapped page is masked in compute(); keep the loads in bounds
-        const int64_t row0 = (int64_t)blk * a.block_size + (p0 - page * a.block_size);
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                t.k[tb][j] = *reinterpret_cast<const u32x4*>(kbase + (row0 + tb * 16 + r16) * row_pitch + (g4 + 4 * j) * 16);
-#pragma unroll
-        for (int i8 = 0; i8 < 8; ++i8)
-            t.v[i8] = *reinterpret_cast<const u32x4*>(vbase + (row0 + 4 * i8 + g4) * row_pitch + r16 * 16);
-    };
-
-    auto compute = [&](int i, const SubTile& t) {
-        const int p0 = start + GSUB * i;
-        const int page = p0 / a.block_size;
-        const int blk = __builtin_amdgcn_readfirstlane(bt[page]);
-        const bool mapped = blk >= 0 && blk < a.n_blocks;
-        f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, t.k[0][j]),
-                                                         __builtin_bit_cast(bf16x8, qf[j]), s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, t.k[1][j]),
-                                                         __builtin_bit_cast(bf16x8, qf[j]), s1, 0, 0, 0);
+        if (page - window >= 64) { // (uniform; chunks of more than 64 pages)
+            window = page;
+            fetch_entries();
         }
-        // stage V for the transposing reads while the scores are in flight
+        const int blk = __builtin_amdgcn_readlane(entry, page - window);
+        t.mapped = blk >= 0; // an unmapped page is masked in compute(); its loads stay in bounds
+        const int64_t row0 = (int64_t)max(blk, 0) * a.block_size + (p0 - page * a.block_size);
+        auto row = [&](const uint8_t* base, int i8) {
+            const u32x4* p = reinterpret_cast<const u32x4*>(base + (row0 + 4 * i8 + g4) * row_pitch + r16 * 16);
+            return NT ? __builtin_nontemporal_load(p) : *p;
+        };
+#pragma unroll
+        for (int i8 = 0; i8 < 8; ++i8) t.k[i8] = row(kbase, i8);
+#pragma unroll
+        for (int i8 = 0; i8 < 8; ++i8) t.v[i8] = row(vbase, i8);
+    };
+    auto stage = [&](const SubTile& t) {
+#pragma unroll
+        for (int i8 = 0; i8 < 8; ++i8) {
+            const int tv = 4 * i8 + g4;
+            *reinterpret_cast<u32x4*>(myk + tv * GROW + vswz(tv, r16)) = t.k[i8];
+        }
 #pragma unroll
         for (int i8 = 0; i8 < 8; ++i8) {
             const int tv = 4 * i8 + g4;
             *reinterpret_cast<u32x4*>(myv + tv * GROW + vswz(tv, r16)) = t.v[i8];
         }
-        float sv[8];
-        float mt = -INFINITY;
+    };
+
+    auto compute = [&](int i, bool mapped) {
+        const int p0 = start + GSUB * i;
+        f32x4 s0[RT], s1[RT];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const int tok = p0 + (r >> 2) * 16 + 4 * g4 + (r & 3);
-            const float x = (r < 4 ? s0[r & 3] : s1[r & 3]) * sc;
-            sv[r] = (tok < end && mapped) ? x : -INFINITY;
-            mt = fmaxf(mt, sv[r]);
-        }
-        mt = fmaxf(mt, __shfl_xor(mt, 16));
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
-        const float m_new = fmaxf(m_run, mt);
-        const float mref = (m_new == -INFINITY) ? 0.f : m_new;
-        const float alpha = exp2f(m_run - mref);
-        float p[8], psum = 0.f;
+        for (int r = 0; r < RT; ++r) s0[r] = s1[r] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            p[r] = exp2f(sv[r] - mref);
-            psum += p[r];
-        }
-        l_run = l_run * alpha + psum;
-        m_run = m_new;
-        if (__any(alpha != 1.f)) {
+        for (int j = 0; j < 4; ++j) {
+            const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(myk + r16 * GROW + vswz(r16, g4 + 4 * j));
+            const bf16x8 k1 = *reinterpret_cast<const bf16x8*>(myk + (r16 + 16) * GROW + vswz(r16, g4 + 4 * j));
 #pragma unroll
-            for (int db = 0; db < 8; ++db) o[db] *= alpha;
+            for (int r = 0; r < RT; ++r) {
+                s0[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, __builtin_bit_cast(bf16x8, qf[r][j]), s0[r], 0, 0, 0);
+                s1[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, __builtin_bit_cast(bf16x8, qf[r][j]), s1[r], 0, 0, 0);
+            }
         }
-        const u32x4 pf = {pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
-                          pack_bf16x2(p[6], p[7])};
+        u32x4 pf[RT];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            float sv[8];
+            float mt = -INFINITY;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int tok = p0 + (e >> 2) * 16 + 4 * g4 + (e & 3);
+                const float x = (e < 4 ? s0[r][e & 3] : s1[r][e & 3]) * sc;
+                sv[e] = (tok < end_r[r] && mapped) ? x : -INFINITY;
+                mt = fmaxf(mt, sv[e]);
+            }
+            mt = fmaxf(mt, __shfl_xor(mt, 16));
+            mt = fmaxf(mt, __shfl_xor(mt, 32));
+            const float m_new = fmaxf(m_run[r], mt);
+            const float mref = (m_new == -INFINITY) ? 0.f : m_new;
+            const float alpha = exp2f(m_run[r] - mref);
+            float p[8], psum = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                p[e] = exp2f(sv[e] - mref);
+                psum += p[e];
+            }
+            l_run[r] = l_run[r] * alpha + psum;
+            m_run[r] = m_new;
+            if (__any(alpha != 1.f)) {
+#pragma unroll
+                for (int db = 0; db < 8; ++db) o[r][db] *= alpha;
+            }
+            pf[r] = u32x4{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]), pack_bf16x2(p[6], p[7])};
+        }
         const int tok_lo = 4 * g4 + (r16 >> 2);
 #pragma unroll
         for (int db = 0; db < 8; ++db) {
             const s16x4 lo = lds_read_tr(myv + tok_lo * GROW + ((db ^ (tok_lo & 7)) << 5) + (r16 & 3) * 8);
             const s16x4 hi = lds_read_tr(myv + (tok_lo + 16) * GROW + ((db ^ (tok_lo & 7)) << 5) + (r16 & 3) * 8);
             const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-            o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, both),
-                                                            __builtin_bit_cast(bf16x8, pf), o[db], 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+                o[r][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, both),
+                                                                   __builtin_bit_cast(bf16x8, pf[r]), o[r][db], 0, 0, 0);
         }
     };
 
     if (w < nsub) {
-        SubTile cur_t, nxt_t;
+        SubTile t;
         int i = w;
-        load(i, cur_t);
+        load(i, t);
         for (; i + GWAVES < nsub; i += GWAVES) {
-            load(i + GWAVES, nxt_t);
-            compute(i, cur_t);
-            cur_t = nxt_t;
+            const bool mapped = t.mapped;
+            stage(t);
+            load(i + GWAVES, t);
+            compute(i, mapped);
         }
-        compute(i, cur_t);
+        stage(t);
+        compute(i, t.mapped);
     }
-    l_run += __shfl_xor(l_run, 16);
-    l_run += __shfl_xor(l_run, 32);
 
     // merge the four waves
-    __syncthreads();
     float* mo = reinterpret_cast<float*>(lds);
 #pragma unroll
-    for (int db = 0; db < 8; ++db)
-        *reinterpret_cast<f32x4*>(mo + (w * 16 + r16) * GD + 16 * db + 4 * g4) = o[db];
-    if (g4 == 0) {
-        s_ml[w][r16][0] = m_run;
-        s_ml[w][r16][1] = l_run;
-    }
-    __syncthreads();
-    {
+    for (int r = 0; r < RT; ++r) {
+        l_run[r] += __shfl_xor(l_run[r], 16);
+        l_run[r] += __shfl_xor(l_run[r], 32);
+        __syncthreads();
+#pragma unroll
+        for (int db = 0; db < 8; ++db)
+            *reinterpret_cast<f32x4*>(mo + (w * 16 + r16) * GD + 16 * db + 4 * g4) = o[r][db];
+        if (g4 == 0) {
+            s_ml[w][r16][0] = m_run[r];
+            s_ml[w][r16][1] = l_run[r];
+        }
+        __syncthreads();
         const int n = tid >> 4, d0 = (tid & 15) * 8;
-        const int hloc = hs * 16 + n;
-        if (hloc >= g) return;
+        const int hloc = hs[r] * 16 + n;
+        if (hloc >= g) continue;
         float M = -INFINITY;
 #pragma unroll
         for (int ww = 0; ww < GWAVES; ++ww) M = fmaxf(M, s_ml[ww][n][0]);
@@ -228,18 +396,19 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a)
                 }
             }
         }
-        const int64_t head_row = (int64_t)tq * a.nq + n2 * g + hloc;
-        if (a.nsplit == 1) {
+        if (a.part_o == nullptr) {
+            const int64_t head_row = (int64_t)tok_q[r] * a.nq + n2 * g + hloc;
             const float inv = L > 0.f ? 1.f / L : 0.f;
             const u32x4 pk = {pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv),
                               pack_bf16x2(acc[4] * inv, acc[5] * inv), pack_bf16x2(acc[6] * inv, acc[7] * inv)};
             *reinterpret_cast<u32x4*>(out + head_row * GD + d0) = pk;
         } else {
-            float* po = a.part_o + (head_row * a.nsplit + split) * GD + d0;
+            const int64_t slot = ((int64_t)u * a.s1 + (tok_q[r] - bi * a.s1)) * a.nq + n2 * g + hloc;
+            float* po = a.part_o + slot * GD + d0;
             *reinterpret_cast<f32x4*>(po) = f32x4{acc[0], acc[1], acc[2], acc[3]};
             *reinterpret_cast<f32x4*>(po + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
             if ((tid & 15) == 0) {
-                float* pm = a.part_ml + (head_row * a.nsplit + split) * 2;
+                float* pm = a.part_ml + slot * 2;
                 pm[0] = M;
                 pm[1] = L;
             }
@@ -247,11 +416,18 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a)
     }
 }
 
-// One wave quarter (32 lanes x 4 dims) per head row: merges the chunks that hold tokens of this query token.
-__global__ __launch_bounds__(128) void gqa_combine_kernel(GqaArgs a)
+// Merges the chunks that hold tokens of a query token: 32 lanes x 4 dims per head row and group of chunks, GROUPS such
+// groups per row (merged through LDS) where there are many chunks - one group would walk them in too long a chain.
+template <int GROUPS>
+__global__ __launch_bounds__(256) void gqa_combine_kernel(GqaArgs a)
 {
-    const int64_t head_row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 5);
-    if (head_row >= (int64_t)a.b * a.s1 * a.nq) return;
+    constexpr int ROWS = 8 / GROUPS;
+    __shared__ __align__(16) float s_acc[GROUPS > 1 ? 8 : 1][128];
+    __shared__ float s_m[8], s_l[8];
+    const int part = threadIdx.x >> 5, grp = part % GROUPS;
+    const int64_t last_row = (int64_t)a.b * a.s1 * a.nq - 1;
+    const int64_t want = (int64_t)blockIdx.x * ROWS + part / GROUPS;
+    const int64_t head_row = want < last_row ? want : last_row; // (surplus groups redo the last row)
     const int d0 = (threadIdx.x & 31) * 4;
     const int tq = (int)(head_row / a.nq);
     const int bi = tq / a.s1, si = tq - bi * a.s1;
@@ -259,40 +435,63 @@ __global__ __launch_bounds__(128) void gqa_combine_kernel(GqaArgs a)
     cur = cur < 0 ? 0 : cur;
     const int reach = a.bt_stride * a.block_size;
     cur = cur > reach ? reach : cur;
-    const int nvalid = (cur + a.chunk - 1) / a.chunk;
-    const float* pm = a.part_ml + head_row * a.nsplit * 2;
-    const float* po = a.part_o + head_row * a.nsplit * GD + d0;
-    // eight chunks' loads in flight at a time (a chunk past the last valid one re-reads the last and is dropped): the
-    // additions keep the order of the chunks
+    const int chunk = a.plan[0];
+    const int nvalid = (cur + chunk - 1) / chunk;
+    // the unit's partials lie [query token of the sequence, head]
+    const int64_t slot0 = ((int64_t)a.plan[1 + bi] * a.s1 + si) * a.nq + (head_row - (int64_t)tq * a.nq), per = (int64_t)a.s1 * a.nq;
+    const float* pm = a.part_ml + slot0 * 2;
+    const float* po = a.part_o + slot0 * GD + d0;
+    // eight chunks' loads in flight at a time (a chunk past the last valid one re-reads the last and is dropped): an online
+    // merge, chunks grp, grp + GROUPS, .. in order
     constexpr int G = 8;
-    float M = -INFINITY;
-    for (int s0 = 0; s0 < nvalid; s0 += G) {
-        float m[G];
-#pragma unroll
-        for (int j = 0; j < G; ++j) m[j] = pm[2 * min(s0 + j, nvalid - 1)];
-#pragma unroll
-        for (int j = 0; j < G; ++j) M = fmaxf(M, m[j]);
-    }
-    float L = 0.f;
+    float M = -INFINITY, L = 0.f;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    if (M > -INFINITY) {
-        for (int s0 = 0; s0 < nvalid; s0 += G) {
-            f32x4 v[G];
-            float m[G], l[G];
+    for (int s0 = grp; s0 < nvalid; s0 += G * GROUPS) {
+        f32x4 v[G];
+        float m[G], l[G], top = M;
+#pragma unroll
+        for (int j = 0; j < G; ++j) {
+            const int s = min(s0 + j * GROUPS, nvalid - 1);
+            m[j] = pm[2 * per * s];
+            l[j] = pm[2 * per * s + 1];
+            v[j] = *reinterpret_cast<const f32x4*>(po + per * s * GD);
+        }
+#pragma unroll
+        for (int j = 0; j < G; ++j) top = fmaxf(top, m[j]);
+        if (top > -INFINITY) {
+            const float old = exp2f(M - top);
+            L *= old;
+            acc *= old;
+            M = top;
 #pragma unroll
             for (int j = 0; j < G; ++j) {
-                const int s = min(s0 + j, nvalid - 1);
-                m[j] = pm[2 * s];
-                l[j] = pm[2 * s + 1];
-                v[j] = *reinterpret_cast<const f32x4*>(po + (int64_t)s * GD);
-            }
-#pragma unroll
-            for (int j = 0; j < G; ++j) {
-                if (s0 + j < nvalid) {
+                if (s0 + j * GROUPS < nvalid) {
                     const float wgt = exp2f(m[j] - M);
                     L += wgt * l[j];
                     acc += v[j] * wgt;
                 }
+            }
+        }
+    }
+    if constexpr (GROUPS > 1) {
+        *reinterpret_cast<f32x4*>(&s_acc[part][d0]) = acc;
+        if ((threadIdx.x & 31) == 0) {
+            s_m[part] = M;
+            s_l[part] = L;
+        }
+        __syncthreads();
+        if (grp != 0) return;
+        float top = -INFINITY;
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) top = fmaxf(top, s_m[part + g]);
+        L = 0.f;
+        acc = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (top > -INFINITY) {
+#pragma unroll
+            for (int g = 0; g < GROUPS; ++g) {
+                const float wgt = exp2f(s_m[part + g] - top);
+                L += wgt * s_l[part + g];
+                acc += *reinterpret_cast<const f32x4*>(&s_acc[part + g][d0]) * wgt;
             }
         }
     }
@@ -310,21 +509,61 @@ __global__ void gqa_zero_kernel(uint32_t* out, int64_t n_words)
 
 } // namespace
 
-void gqa_pick_chunk(int max_ctx, int forced_chunk, int* chunk, int* nsplit)
+// units_cap: chunks of all sequences together.  One chunk per sequence and no second kernel where the sequences alone give
+// GQA_SLOTS workgroups of at most GQA_TARGET tokens.
+void gqa_plan(GqaArgs& a, int forced_chunk)
 {
-    int c = forced_chunk > 0 ? (forced_chunk + 127) / 128 * 128 : 1024;
-    int n = max_ctx > 0 ? (max_ctx + c - 1) / c : 1;
-    if (forced_chunk <= 0 && n > 64) {
-        c = ((max_ctx + 63) / 64 + 127) / 128 * 128;
-        n = (max_ctx + c - 1) / c;
+    const int64_t t = (int64_t)a.b * a.s1;
+    const int64_t max_ctx = (int64_t)a.bt_stride * a.block_size;
+    if (t == 0) { // (nothing to launch)
+        a.chunk = 128;
+        a.nsplit = a.row_tiles = a.columns = 1;
+        a.units_cap = 0;
+        return;
     }
-    *chunk = c;
-    *nsplit = n < 1 ? 1 : n;
+    a.row_tiles = a.s1 * a.hsub % 2 == 0 ? 2 : 1;
+    a.columns = (int32_t)((int64_t)a.nkv * a.s1 * a.hsub / a.row_tiles);
+    if (forced_chunk > 0) {
+        a.chunk = (forced_chunk + 127) / 128 * 128;
+    } else if (a.b > GQA_SCAN) {
+        a.chunk = GQA_TARGET;
+    } else {
+        const int64_t round = (int64_t)GQA_SLOTS * (GQA_TARGET / 128);
+        const int64_t work = (int64_t)a.b * ((max_ctx + 127) / 128) * a.columns;
+        const int64_t rounds = (work + round - 1) / round;
+        int64_t target = (rounds > 1 ? rounds : 1) * GQA_SLOTS / a.columns;
+        const int64_t most = (int64_t)a.b * (max_ctx > 128 * GQA_MAX_SPLIT ? GQA_MAX_SPLIT : (max_ctx + 127) / 128);
+        if (target > most) target = most;
+        a.chunk = 0; // chosen on the device
+        a.units_cap = (int32_t)(target > a.b ? target : a.b);
+        a.nsplit = a.units_cap > a.b ? 2 : 1;
+        if (a.nsplit == 1) a.chunk = (int32_t)((max_ctx + 127) / 128 * 128);
+    }
+    if (a.chunk > 0) {
+        const int64_t n = (max_ctx + a.chunk - 1) / a.chunk;
+        a.nsplit = n < 1 ? 1 : (int32_t)n;
+        a.units_cap = (int32_t)(a.b * (int64_t)a.nsplit);
+    }
+    a.stream_past_cache = (double)t / (a.s1 > 0 ? a.s1 : 1) * (double)max_ctx * a.nkv * 2 * GROW > 256e6;
 }
 
-uint64_t gqa_workspace_bytes(int64_t t, int nq, int nsplit)
+static uint64_t gqa_align(uint64_t x) { return (x + 255) & ~(uint64_t)255; }
+
+// partials [units_cap, s1, nq, 128] fp32 | (m, l) [units_cap, s1, nq, 2] fp32 | chunk length, first unit of every sequence
+uint64_t gqa_workspace_bytes(const GqaArgs& a)
 {
-    return nsplit > 1 ? (uint64_t)t * nq * nsplit * (GD + 2) * sizeof(float) : 0;
+    if (a.nsplit == 1) return 0;
+    const uint64_t rows = (uint64_t)a.units_cap * a.s1 * a.nq;
+    return gqa_align(rows * GD * 4) + gqa_align(rows * 8) + gqa_align((1 + (uint64_t)a.b) * 4);
+}
+
+void gqa_bind_workspace(GqaArgs& a, void* workspace)
+{
+    const uint64_t rows = (uint64_t)a.units_cap * a.s1 * a.nq;
+    uint8_t* p = static_cast<uint8_t*>(workspace);
+    a.part_o = reinterpret_cast<float*>(p);
+    a.part_ml = reinterpret_cast<float*>(p + gqa_align(rows * GD * 4));
+    a.plan = reinterpret_cast<int32_t*>(p + gqa_align(rows * GD * 4) + gqa_align(rows * 8));
 }
 
 hipError_t gqa_launch(const GqaArgs& a, hipStream_t stream)
@@ -339,14 +578,25 @@ hipError_t gqa_launch(const GqaArgs& a, hipStream_t stream)
     }
     {
         ScopedKernelTimer timer(KID_GQA_DECODE, stream);
-        hipLaunchKernelGGL(gqa_decode_kernel, dim3(a.nsplit, a.nkv * a.hsub, (unsigned)t), dim3(256), 0, stream, a);
+        const int64_t units = ((int64_t)a.units_cap + 7) / 8 * 8;
+        const int64_t groups = units * a.columns;
+        const int64_t gx = groups < (1 << 22) ? groups : (1 << 22);
+        if (groups + gx > 0xffffffffll) return hipErrorInvalidValue;
+        auto kern = a.row_tiles == 2 ? (a.stream_past_cache ? gqa_decode_kernel<2, true> : gqa_decode_kernel<2, false>)
+                                     : (a.stream_past_cache ? gqa_decode_kernel<1, true> : gqa_decode_kernel<1, false>);
+        hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)((groups + gx - 1) / gx)), dim3(256), 0, stream, a);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.nsplit == 1) return e;
     {
         ScopedKernelTimer timer(KID_GQA_COMBINE, stream);
         const int64_t rows = t * a.nq;
-        hipLaunchKernelGGL(gqa_combine_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(128), 0, stream, a);
+        // (eight groups per row for few rows of many chunks: 16 chunks take one group 9 us where rows are few; with many rows the
+        // second step costs more than it saves, 20 us against 6 at 6144 rows)
+        if (a.units_cap > 12 * a.b && rows <= 2048)
+            hipLaunchKernelGGL(gqa_combine_kernel<8>, dim3((unsigned)rows), dim3(256), 0, stream, a);
+        else
+            hipLaunchKernelGGL(gqa_combine_kernel<1>, dim3((unsigned)((rows + 7) / 8)), dim3(256), 0, stream, a);
     }
     return hipGetLastError();
 }

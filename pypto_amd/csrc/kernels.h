@@ -95,15 +95,21 @@ struct GqaArgs {
     const int32_t* block_table; // [b, bt_stride]
     const int32_t* act_seq;     // [b]
     void* out;                  // [t, nq, 128] bf16
-    float* part_o;              // workspace [t*nq, nsplit, 128] fp32 (nsplit > 1)
-    float* part_ml;             // workspace [t*nq, nsplit, 2]: running max (log2 units), sum
+    float* part_o;              // workspace, null if every sequence is one chunk: partials by unit (a chunk of a sequence)
+    float* part_ml;             // workspace: running max (log2 units), sum
+    int32_t* plan;              // workspace: chunk length, first unit of every sequence
     int64_t n_blocks;
-    int32_t b, s1, nq, nkv, hsub, block_size, bt_stride, nsplit, chunk;
+    int32_t b, s1, nq, nkv, hsub, block_size, bt_stride;
+    // set by gqa_plan: chunks per sequence (at most; > 1: the combine kernel runs), chunk length (0: chosen on the device),
+    // 16-row tiles per workgroup, workgroups per unit, units of the batch at most
+    int32_t nsplit, chunk, row_tiles, columns, units_cap;
+    bool stream_past_cache;     // set by gqa_plan
     float softmax_scale;
 };
 
-void gqa_pick_chunk(int max_ctx, int forced_chunk, int* chunk, int* nsplit);
-uint64_t gqa_workspace_bytes(int64_t t, int nq, int nsplit);
+void gqa_plan(GqaArgs& a, int forced_chunk);
+uint64_t gqa_workspace_bytes(const GqaArgs& a);
+void gqa_bind_workspace(GqaArgs& a, void* workspace);
 hipError_t gqa_launch(const GqaArgs& a, hipStream_t stream);
 
 // ---------------------------------------------------------------- lightning indexer prolog

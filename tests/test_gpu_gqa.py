@@ -134,6 +134,29 @@ def test_full_size_config4(cuda):
     check(out[sel].contiguous(), sub_case, "config4 (sampled sequences)")
 
 
+@pytest.mark.parametrize("s1,nq,nkv,act", [(1, 12, 1, [1]), (1, 12, 1, [128, 129, 0, 33]), (2, 12, 1, [4097, 1, 2, 700]), (3, 12, 2, [500, 2, 1300]),
+                                           (1, 40, 2, [900, 31]), (2, 34, 2, [64, 260]), (1, 12, 1, [9000] + [5] * 70),
+                                           (1, 12, 2, [0] * 3 + [1500, 0, 40]), (1, 12, 1, [3, 200] * 150), (1, 96, 8, [300] * 40)])
+def test_chunk_choice_and_row_tiles(cuda, s1, nq, nkv, act):
+    """Chunks chosen from the lengths: single tokens, page edges, empty sequences, one long sequence among many short ones
+    (lengths beyond one wavefront's lanes), more sequences than the device-side choice takes, one chunk per sequence; one and
+    two row tiles per workgroup from query tokens and from head sub-groups."""
+    case = gqa.make_case(len(act), s1, nq, nkv, act, seed=len(act) + nq)
+    check(run(case, cuda), case, f"{s1} {nq} {nkv} {act[:6]}")
+
+
+def test_keys_beyond_the_last_level_cache(cuda):
+    # a page table that reaches far enough for the loads past the caches (over 256 MB of keys and values), short sequences in it
+    case = gqa.make_case(2, 2, 12, 1, [700, 300], seed=77)
+    bt = case["block_table"]
+    wide = torch.full((2, 2100), -1, dtype=bt.dtype)
+    wide[:, :bt.shape[1]] = bt
+    near = run(case, cuda)
+    far = run(dict(case, block_table=wide), cuda)
+    check(far, case, "wide page table")
+    assert torch.equal(near, far)
+
+
 def test_cache_without_pages_gives_zeros(cuda):
     # a page table with columns and positive lengths over a cache that holds no page: zero rows, no read of the cache
     case = gqa.make_case(2, 2, 12, 1, [300, 40], seed=9)
