@@ -16,7 +16,7 @@
 // (v_mfma_f32_16x16x32_f16: row 0 of A holds w_scale, B is the fp16 tile just produced; every product of two
 // fp16 values is exact in fp32, so this is the golden's fp32 sum up to the order of additions).  Scores go to
 // a dense fp32 row per query token, and their order-preserving keys into a 256-bin histogram in LDS (score_bin:
-// quarter octaves).  Every workgroup owns a 2048-key span of its sequence and leaves its histogram in a slot of
+// quarter octaves).  Every workgroup owns a span of its sequence's keys and leaves its histogram in a slot of
 // its own in the workspace (16-bit counts): plain stores, nothing to clear beforehand and no global atomics.
 //
 // indexer_select_kernel: every workgroup adds up the spans' histograms of its query token, finds the bin B that
@@ -145,7 +145,7 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v)
 }
 
 // The workgroup's histograms (S1 query tokens, one span of keys) go to its own slots, as 16-bit counts (a span has at
-// most 2048 keys), two per lane.  The span-0 workgroup also clears the select kernel's list counters of its query tokens.  256 lanes.
+// most 4096 keys), two per lane.  The span-0 workgroup also clears the select kernel's list counters of its query tokens.  256 lanes.
 template <int S1>
 __device__ __forceinline__ void flush_span_hist(const IndexerArgs& a, const uint32_t (*hist)[SBINS], int row0, int span, int tid)
 {
@@ -281,19 +281,23 @@ __device__ __forceinline__ uint32_t relu_scale_pack(int a, int b)
 }
 
 // Score kernel for block sizes that are multiples of 128: a wavefront owns 128 consecutive keys of one page per pass
-// (one page-table entry; the entries of all its passes are fetched up front with one load, lane p holding pass p's),
-// keeps the loads of the next NBUF-1 half passes (64 keys, 8 KB each) in flight while it scores the current one, and
-// files its results 64 at a time: w_scale sits in every row of the head-sum operand, so every lane group holds the 16
-// scores of a key group and lane group g keeps those of key group g - after four key groups lane l holds the score of
-// key l of the 64, next to that key's scale (loaded with one 128-byte instruction per 64 keys).
-// PPASSES: passes (of 512 keys) per workgroup, pick_passes' choice
-template <int S1, bool F32, int PPASSES>
+// (one page-table entry; the entries of all its passes are fetched up front with one load, lane p holding pass p's).  Keys
+// travel 64 at a time (8 KB, eight whole 128-byte rows to an instruction) through registers into the wavefront's own LDS,
+// from where they are read in operand layout while the next 64 are on the way.  Results are filed 64 at a time: w_scale sits
+// in every row of the head-sum operand, so every lane group holds the 16 scores of a key group and lane group g keeps those
+// of key group g - after four key groups lane l holds the score of key l of the 64, next to that key's scale (loaded with one
+// 128-byte instruction per 64 keys).
+// PPASSES: passes (of 512 keys) per workgroup, pick_passes' choice.  NT: loads past the caches' retention, for batches whose
+// keys do not fit the last-level cache - which needs the whole-row loads: taken in operand layout, a row is two loads of
+// half a cache line, and a line that is not kept in between is fetched twice (32 x 64 K keys, 272 MB: 56.8 us in operand
+// layout, 65.0 with non-temporal loads; 57.8 and 52.7 this way).
+template <int S1, bool F32, int PPASSES, bool NT>
 __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kernel(IndexerArgs a)
 {
-    constexpr int NBUF = 2; // half-pass buffers: NBUF-1 halves ahead (deeper prefetch measured no faster)
     constexpr int NHALF = 2 * PPASSES;
     __shared__ __align__(16) uint32_t hist[S1][SBINS];
     __shared__ __align__(16) float s_sc[S1][CHUNK * PPASSES]; // the workgroup's scores, written out in one burst at the end
+    __shared__ __align__(16) uint8_t s_keys[4][64 * D];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, g = lane >> 4;
     const int sgrp = blockIdx.z;
@@ -363,24 +367,29 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
         return (int64_t)(((uint64_t)hi << 32) | lo);
     };
 
-    i32x4 kf[NBUF][4][2];
-    typename ScaleOf<F32>::raw ksc[NBUF][2]; // [buffer][unused for odd halves]: the scales of a pass travel with its first half
-    auto load_half = [&](int hh, int buf) {
+    // 64 keys on the way: load i holds chunk lane % 8 of key 8 i + lane / 8; in LDS the 16-byte chunks of a key are XOR-ed with
+    // the key, so that both the row writes and the operand reads fall on all banks
+    i32x4 raw[8];
+    typename ScaleOf<F32>::raw ksc_next;
+    auto load_half = [&](int hh) {
         const int64_t r = pass_row(hh >> 1);
         const int64_t rb = r < 0 ? 0 : r;
-        const int8_t* kp = a.k_cache + (rb + 64 * (hh & 1) + l16) * D + 16 * g;
+        const int8_t* kp = a.k_cache + (rb + 64 * (hh & 1)) * D + 16 * lane;
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-            kf[buf][jj][0] = *reinterpret_cast<const i32x4*>(kp + jj * 16 * D);
-            kf[buf][jj][1] = *reinterpret_cast<const i32x4*>(kp + jj * 16 * D + 64);
+        for (int i = 0; i < 8; ++i) {
+            const i32x4* p = reinterpret_cast<const i32x4*>(kp + i * 8 * D);
+            raw[i] = NT ? __builtin_nontemporal_load(p) : *p;
         }
-        ksc[buf][0] = static_cast<const typename ScaleOf<F32>::raw*>(a.k_scale)[rb + 64 * (hh & 1) + lane];
+        ksc_next = static_cast<const typename ScaleOf<F32>::raw*>(a.k_scale)[rb + 64 * (hh & 1) + lane];
     };
+    uint8_t* keys = s_keys[wave];
+    uint8_t* key_dst = keys + (lane >> 3) * D + (((lane & 7) ^ (lane >> 3)) << 4);
+    const uint8_t* key_src0 = keys + l16 * D + ((g ^ (l16 & 7)) << 4);
+    const uint8_t* key_src1 = keys + l16 * D + (((g + 4) ^ (l16 & 7)) << 4);
     // The key loads go out first; the query and its scales follow them (memory operations complete in order, and the
     // first MFMA needs all of them).  Every memory operation from here on is unconditional, so that the number in
     // flight is the same on every path into the loop and the waits can count them.
-#pragma unroll
-    for (int u = 0; u < NBUF - 1; ++u) load_half(u, u);
+    load_half(0);
     // int8 A fragments: head hb*16 + l16, bytes 64*ks + 16*g .. +15
     i32x4 qf[S1][4][2];
 #pragma unroll
@@ -419,20 +428,22 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
     for (int i = tid; i < S1 * SBINS; i += 256) (&hist[0][0])[i] = 0;
     __syncthreads();
 
-    auto compute_half = [&](int hh, int buf) {
+    auto compute_half = [&](int hh, typename ScaleOf<F32>::raw ksc) {
         float res[S1];
 #pragma unroll
         for (int s = 0; s < S1; ++s) res[s] = 0.f;
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
+            const i32x4 kf0 = *reinterpret_cast<const i32x4*>(key_src0 + jj * 16 * D);
+            const i32x4 kf1 = *reinterpret_cast<const i32x4*>(key_src1 + jj * 16 * D);
 #pragma unroll
             for (int s = 0; s < S1; ++s) {
                 u32x4 y[2];
 #pragma unroll
                 for (int hb = 0; hb < 4; ++hb) {
                     i32x4 acc = {SCORE_BIAS, SCORE_BIAS, SCORE_BIAS, SCORE_BIAS};
-                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(qf[s][hb][0], kf[buf][jj][0], acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(qf[s][hb][1], kf[buf][jj][1], acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(qf[s][hb][0], kf0, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(qf[s][hb][1], kf1, acc, 0, 0, 0);
                     y[hb >> 1][2 * (hb & 1)] = relu_scale_pack(acc[0], acc[1]);
                     y[hb >> 1][2 * (hb & 1) + 1] = relu_scale_pack(acc[2], acc[3]);
                 }
@@ -443,7 +454,7 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
             }
         }
         const int tok = wtok + (hh >> 1) * CHUNK + 64 * (hh & 1) + lane;
-        const float ks = pass_row(hh >> 1) >= 0 ? ScaleOf<F32>::f32(ksc[buf][0]) : 0.f;
+        const float ks = pass_row(hh >> 1) >= 0 ? ScaleOf<F32>::f32(ksc) : 0.f;
 #pragma unroll
         for (int s = 0; s < S1; ++s) {
             const float sc = res[s] * ks;
@@ -453,19 +464,13 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
         }
     };
 
-    // NBUF halves per trip, so that buffer indices are compile-time constants; past the end the last half is loaded
-    // again (a cache hit whose data is never used) so that the loads stay unconditional
-    static_assert(NHALF % NBUF == 0, "whole trips");
-    for (int base = 0; base < NHALF; base += NBUF) {
+    // (past the end the last half is loaded again, a cache hit whose data is never used, so that the loads stay unconditional)
+    for (int hh = 0; hh < NHALF; ++hh) {
 #pragma unroll
-        for (int u = 0; u < NBUF; ++u) {
-            const int hh = base + u;
-            if (hh < NHALF) {
-                const int nx = hh + NBUF - 1;
-                load_half(nx < NHALF ? nx : NHALF - 1, (u + NBUF - 1) % NBUF);
-                compute_half(hh, u);
-            }
-        }
+        for (int i = 0; i < 8; ++i) *reinterpret_cast<i32x4*>(key_dst + i * 8 * D) = raw[i]; // (8 keys on: the same XOR)
+        const typename ScaleOf<F32>::raw ksc = ksc_next;
+        load_half(hh + 1 < NHALF ? hh + 1 : NHALF - 1);
+        compute_half(hh, ksc);
     }
     __syncthreads();
     // one contiguous 8 KB write per query token (256-byte stores from inside the loop, between the key loads, cost
@@ -1253,18 +1258,22 @@ hipError_t topk_launch(const float* x, float* values, int32_t* indices, int64_t 
 // ties [t, 8192] u64; spans = stride / span
 static uint64_t align256(uint64_t x) { return (x + 255) & ~(uint64_t)255; }
 
-// Passes of 512 keys per workgroup of the paged score kernel: four (the query's set-up is paid once per 2048 keys) where
-// that still leaves every CU its fill of workgroups, fewer where the batch and its contexts are small - a single 4 K
-// context is 2 workgroups of four passes, and took 13.5 us.
-static int pick_passes(int64_t t, int64_t stride)
+// Passes of 512 keys per workgroup of the paged score kernel: as many as leave SCORE_GROUPS workgroups, eight at most.  Where
+// there are keys for that, few long streams serve best (32 x 64 K keys: 50 us with eight passes, 53 with four, 58 with two);
+// a small batch needs short ones to reach every CU (a single 4 K context is 2 workgroups of four passes: 12 us, against 6).
+static int pick_passes(int b, int s1, int64_t stride)
 {
-    const int64_t groups = t * (stride / CHUNK);
-    return groups >= 4 * SCORE_GROUPS ? 4 : groups >= 2 * SCORE_GROUPS ? 2 : 1;
+    const int64_t groups = (int64_t)b * (s1 % 2 == 0 ? s1 / 2 : s1) * (stride / CHUNK); // of one pass
+    int p = 8;
+    while (p > 1 && groups < p * SCORE_GROUPS) p >>= 1;
+    return p;
 }
 
-uint64_t indexer_workspace_bytes(int t, int stride)
+uint64_t indexer_workspace_bytes(int b, int s1, int stride)
 {
-    const uint64_t spans = (uint64_t)stride / (CHUNK * pick_passes(t, stride));
+    const int t = b * s1;
+    const int passes = pick_passes(b, s1, stride);
+    const uint64_t spans = (uint64_t)stride / (CHUNK * (passes < PASSES ? passes : PASSES)); // (the unpaged kernel's spans: PASSES)
     return align256((uint64_t)t * stride * 4) + align256((uint64_t)t * spans * SBINS * 2) + align256((uint64_t)t * 4 * 4) +
            align256((uint64_t)t * (MAX_K + TIE_CAP) * 8);
 }
@@ -1272,8 +1281,7 @@ uint64_t indexer_workspace_bytes(int t, int stride)
 void indexer_bind_workspace(IndexerArgs& a, void* ws)
 {
     const int t = a.b * a.s1;
-    // (the unpaged kernel's spans have four passes always)
-    a.span = a.block_size % 128 == 0 ? CHUNK * pick_passes(t, a.score_stride) : CHUNK * PASSES;
+    a.span = a.block_size % 128 == 0 ? CHUNK * pick_passes(a.b, a.s1, a.score_stride) : CHUNK * PASSES;
     const uint64_t spans = (uint64_t)a.score_stride / a.span;
     uint8_t* p = static_cast<uint8_t*>(ws);
     a.scores = reinterpret_cast<float*>(p);
@@ -1290,9 +1298,15 @@ void indexer_bind_workspace(IndexerArgs& a, void* ws)
 template <int PPASSES>
 static void launch_score_paged(const IndexerArgs& a, hipStream_t stream)
 {
-    const bool s2 = a.s1 % 2 == 0;
-    auto kern = s2 ? (a.scales_f32 ? indexer_score_paged_kernel<2, true, PPASSES> : indexer_score_paged_kernel<2, false, PPASSES>)
-                   : (a.scales_f32 ? indexer_score_paged_kernel<1, true, PPASSES> : indexer_score_paged_kernel<1, false, PPASSES>);
+    const bool s2 = a.s1 % 2 == 0, f32 = a.scales_f32;
+    // non-temporal where one call's keys (if they fill the page table) would take the last-level cache's better part (109 MB:
+    // 26.2 -> 24.8 us, 272 MB: 57.8 -> 52.7; 68 MB, found there from one call to the next: 15.0 -> 16.4) and not more than
+    // two workgroups read them
+    const bool nt = (double)a.b * a.max_ctx * D > 96e6 && a.s1 <= 2;
+    auto kern = s2 ? (f32 ? (nt ? indexer_score_paged_kernel<2, true, PPASSES, true> : indexer_score_paged_kernel<2, true, PPASSES, false>)
+                          : (nt ? indexer_score_paged_kernel<2, false, PPASSES, true> : indexer_score_paged_kernel<2, false, PPASSES, false>))
+                   : (f32 ? (nt ? indexer_score_paged_kernel<1, true, PPASSES, true> : indexer_score_paged_kernel<1, true, PPASSES, false>)
+                          : (nt ? indexer_score_paged_kernel<1, false, PPASSES, true> : indexer_score_paged_kernel<1, false, PPASSES, false>));
     hipLaunchKernelGGL(kern, dim3((a.max_ctx + CHUNK * PPASSES - 1) / (CHUNK * PPASSES), a.b, s2 ? a.s1 / 2 : a.s1), dim3(256), 0, stream, a);
 }
 
@@ -1313,7 +1327,8 @@ hipError_t indexer_launch(const IndexerArgs& a, hipStream_t stream)
     {
         ScopedKernelTimer tm(KID_INDEXER_SCORE, stream);
         if (a.block_size % 128 == 0) {
-            if (a.span == 4 * CHUNK) launch_score_paged<4>(args, stream);
+            if (a.span == 8 * CHUNK) launch_score_paged<8>(args, stream);
+            else if (a.span == 4 * CHUNK) launch_score_paged<4>(args, stream);
             else if (a.span == 2 * CHUNK) launch_score_paged<2>(args, stream);
             else launch_score_paged<1>(args, stream);
         } else {

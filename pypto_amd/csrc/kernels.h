@@ -62,7 +62,7 @@ struct IndexerArgs {
     bool use_hist;   // set by indexer_launch: the selection needs the score kernel's histograms
 };
 
-uint64_t indexer_workspace_bytes(int t, int score_stride);
+uint64_t indexer_workspace_bytes(int b, int s1, int score_stride);
 void indexer_bind_workspace(IndexerArgs& a, void* workspace);
 hipError_t indexer_launch(const IndexerArgs& a, hipStream_t stream);
 

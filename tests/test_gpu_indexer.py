@@ -247,6 +247,22 @@ def test_wide_page_table_many_sequences(cuda):
     assert torch.equal(run_indexer(wide, cuda), narrow)
 
 
+@pytest.mark.parametrize("bs,cols,s1", [(48, 700, 1), (48, 700, 2), (128, 270, 1), (128, 270, 2), (128, 70, 4)])
+def test_span_lengths_follow_the_page_tables_reach(cuda, bs, cols, s1):
+    """Short sequences under wide page tables: the reach, not the lengths, picks the passes per workgroup (1 to 8) and whether
+    keys are loaded past the caches, in the paged and in the plain score kernel; the selection is that of a narrow table."""
+    g = torch.Generator().manual_seed(cols + s1)
+    act = torch.randint(1, 900, (64,), generator=g).tolist()
+    case = oi.make_case(64, s1, act, seed=43, selected_count=128, block_size=bs)
+    gold_scores = indexer_scores(case, exact=True)
+    narrow = run_indexer(case, cuda)
+    check_topk(case, narrow, exact=gold_scores)
+    bt = case["block_table"]
+    wide = dict(case)
+    wide["block_table"] = torch.cat([bt, torch.full((bt.shape[0], cols - bt.shape[1]), -1, dtype=bt.dtype)], dim=1).contiguous()
+    assert torch.equal(run_indexer(wide, cuda), narrow)
+
+
 def test_other_selection_sizes_and_block_sizes(cuda):
     case = oi.make_case(2, 1, [1000, 70], seed=8, selected_count=64)
     check_topk(case, run_indexer(case, cuda))
