@@ -18,13 +18,14 @@
 //                     dimension contiguous in memory) is loaded in one go, parked in LDS and read back with 8-bit
 //                     transposing reads as the A operand of the int8 MFMA; int32 partial sums to the workspace (exact,
 //                     so the split over the contraction changes nothing)
-//   apq_head_kernel   one workgroup per (head, token): sum of the partials, bias, dequantisation, head norm, rotary
+//   apq_head_kernel   one wavefront per (head, token): sum of the partials, bias, dequantisation, head norm, rotary
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <algorithm>
 
 #include "common.h"
+#include "gemm_tile.h"
 #include "kernels.h"
 #include "prolog_common.h"
 #include "timing.h"
@@ -194,129 +195,231 @@ __global__ __launch_bounds__(256) void apq_gemm_kernel(AttnPreArgs a)
     }
 }
 
-// The projection at prefill sizes (128 tokens and more): a workgroup owns 128 tokens x 128 outputs over one split of
-// the contraction and walks it in stages of 128 rows, both operands staged through LDS with the next stage's global
-// loads in flight while the current stage is multiplied.  Wave (wr, wc) owns tokens [64 wr, +64) x outputs [64 wc, +64):
-// every operand fragment read from LDS feeds four MFMAs, and the weights are read once per 128 tokens instead of once
-// per 32.  Same int32 partial sums as apq_gemm_kernel (exact, so neither the tiling nor the split shows).
-// grid (n_out / 128, splits, token tiles of 128), 256 lanes.
-constexpr int BTOK = 128, BK = 128;
-constexpr int BQROW = BK + 16; // bytes per LDS row of the [token][k] int8 tile (padded against bank conflicts)
-__global__ __launch_bounds__(256, 3) void apq_gemm_big_kernel(AttnPreArgs a, int per)
+// The projection at prefill sizes (128 tokens and more): a workgroup owns 32 TB tokens x 256 outputs - two heads - over one
+// split of the contraction (gemm_tile.h; an odd last head is taken twice and dropped).  An XCD takes neighbouring heads.  Where one split covers the whole contraction the head's epilogue runs on the
+// tile: the sums never go to memory (777 tokens x 112 heads: 45 MB written and read again, and a kernel of 87 K small
+// workgroups).  Same operations in the same order as apq_head_kernel, so the same bits: its sum over the 128 squares is a
+// butterfly over dims 32, 16, .. 1 apart, which here are register, lane and register exchanges.
+// grid (heads / 2 rounded up, splits, token tiles), 512 lanes.
+template <int TB, bool WHOLE>
+__global__ __launch_bounds__(GT_LANES, 2) void apq_gemm_big_kernel(AttnPreArgs a, int per)
 {
-    __shared__ __align__(16) uint8_t wl[BK * AROW];
-    __shared__ __align__(16) uint8_t ql[BTOK * BQROW];
+#pragma clang fp contract(off)
+    using T = GtTile<TB>;
+    constexpr int OROW = AD * 2 + 16; // bytes per LDS row of a head's bf16 output tile (padded against bank conflicts)
+    constexpr int EPI = 2 * T::TOK * OROW + 4 * T::TOK * 4; // two heads' output tiles, sums of squares of [wc][tokens]
+    __shared__ __align__(16) uint8_t lds[WHOLE && EPI > T::LDS ? EPI : T::LDS];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int l16 = lane & 15, g = lane >> 4, wr = wave >> 1, wc = wave & 1;
-    const int col0 = blockIdx.x * AD, split = blockIdx.y, tok0 = blockIdx.z * BTOK;
-    const int st0 = split * per, stages = min(a.h / BK, st0 + per) - st0; // this split's stages of 128 rows
-    // 128 rows x 128 bytes of either operand per stage = 4 pieces of 16 bytes per lane (rows tid / 8 + 32 i, piece tid % 8)
-    const int srow = tid >> 3, spc = tid & 7;
-    const int8_t* wp = a.w + ((int64_t)st0 * BK + srow) * a.n_out + col0 + 16 * spc;
-    const int8_t* qp[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) qp[i] = a.x_q + (int64_t)min(tok0 + srow + 32 * i, a.t - 1) * a.h + (int64_t)st0 * BK + 16 * spc;
-    u32x4 wst[4], qst[4];
-    auto load = [&](int st) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) qst[i] = *reinterpret_cast<const u32x4*>(qp[i] + st * BK);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) wst[i] = *reinterpret_cast<const u32x4*>(wp + ((int64_t)st * BK + 32 * i) * a.n_out);
-    };
-    i32x4 acc[4][4]; // [db][tb]
+    const int l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
+    const int tile = gridDim.x % 8 == 0 ? (int)(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8) : (int)blockIdx.x;
+    const int heads = a.q_heads + 2 * a.kv_heads, head0 = 2 * tile, head = head0 + (wc >> 1); // of the tile, of this wave
+    const int split = blockIdx.y, tok0 = blockIdx.z * T::TOK;
+    const int st0 = split * per, stages = min(a.h / GT_KI8, st0 + per) - st0; // this split's stages
+    i32x4 acc[4][TB]; // [db][tb]
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
-        for (int tb = 0; tb < 4; ++tb) acc[db][tb] = i32x4{0, 0, 0, 0};
-    load(0);
-    for (int st = 0; st < stages; ++st) {
-        __syncthreads(); // everyone is done with the previous stage's tiles
+        for (int tb = 0; tb < TB; ++tb) acc[db][tb] = i32x4{0, 0, 0, 0};
+    const int8_t* w = a.w + (int64_t)st0 * GT_KI8 * a.n_out;
+    gt_product_i8<TB>(acc, w + head0 * AD, w + min(head0 + 1, heads - 1) * AD, a.n_out, a.x_q + (int64_t)st0 * GT_KI8, a.h, tok0, a.t,
+                      stages, lds);
+    const bool live = head < heads;
+    const int hw = 64 * (wc & 1), col0 = min(head, heads - 1) * AD; // this wave's half of its head; the head's columns
+    // register e of acc[db][tb]: dim hw + 16 db + 4 g + e of the head, token 16 TB wr + 16 tb + l16
+    if constexpr (!WHOLE) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            u32x2* d = reinterpret_cast<u32x2*>(wl + (srow + 32 * i) * AROW + 16 * spc);
-            d[0] = u32x2{wst[i][0], wst[i][1]};
-            d[1] = u32x2{wst[i][2], wst[i][3]};
-            *reinterpret_cast<u32x4*>(ql + (srow + 32 * i) * BQROW + 16 * spc) = qst[i];
+        for (int tb = 0; tb < TB; ++tb) {
+            const int tok = tok0 + 16 * TB * wr + 16 * tb + l16;
+            if (tok >= a.t || !live) continue;
+            int32_t* dst = a.part + ((int64_t)split * a.t + tok) * a.n_out + col0 + hw + 4 * g;
+#pragma unroll
+            for (int db = 0; db < 4; ++db) *reinterpret_cast<i32x4*>(dst + 16 * db) = acc[db][tb];
         }
-        __syncthreads();
-        load(min(st + 1, stages - 1)); // (unconditional: past the end the last stage is fetched again and dropped)
+        return;
+    }
+    float* sums = reinterpret_cast<float*>(lds + 2 * T::TOK * OROW); // [wc][tokens]
+    const bool is_q = head < a.q_heads, is_v = head >= a.q_heads + a.kv_heads; // uniform over the wave
+    const uint16_t* gp = is_q ? a.q_gamma : a.k_gamma;
+    const uint16_t* bp = is_q ? a.q_bias : a.k_bias;
+    float y[4][TB][4]; // [db][tb][e]
 #pragma unroll
-        for (int ks = 0; ks < BK / 64; ++ks) {
-            i32x4 qf[4], wf[4];
+    for (int db = 0; db < 4; ++db) {
+        const int dim = hw + 16 * db + 4 * g;
+        const f32x4 deq = *reinterpret_cast<const f32x4*>(a.deq + col0 + dim);
+        const i32x4 qb = *reinterpret_cast<const i32x4*>(a.qbias + col0 + dim);
 #pragma unroll
-            for (int tb = 0; tb < 4; ++tb)
-                qf[tb] = *reinterpret_cast<const i32x4*>(ql + (64 * wr + 16 * tb + l16) * BQROW + ks * 64 + 16 * g);
-            // (the byte-transposing read: see apq_gemm_kernel)
+        for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
-            for (int db = 0; db < 4; ++db) {
-                const uint8_t* p = wl + (ks * 64 + 16 * g + (l16 >> 1)) * AROW + 64 * wc + 16 * db + 8 * (l16 & 1);
-                const v2i lo = lds_read_tr8(p), hi = lds_read_tr8(p + 8 * AROW);
-                wf[db] = i32x4{lo[0], lo[1], hi[0], hi[1]};
+            for (int e = 0; e < 4; ++e) y[db][tb][e] = round_bf16((float)(acc[db][tb][e] + qb[e]) * deq[e]);
+    }
+    __syncthreads(); // the operand tiles are free
+    if (!is_v) {
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {
+            float m[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float sq[4];
+#pragma unroll
+                for (int db = 0; db < 4; ++db) sq[db] = (y[db][tb][e] * y[db][tb][e]) * (1.0f / AD);
+                m[e] = (sq[0] + sq[2]) + (sq[1] + sq[3]); // dims 32, then 16 apart
+                m[e] += __shfl_xor(m[e], 32, 64);         // 8
+                m[e] += __shfl_xor(m[e], 16, 64);         // 4
             }
-#pragma unroll
-            for (int db = 0; db < 4; ++db)
-#pragma unroll
-                for (int tb = 0; tb < 4; ++tb)
-                    acc[db][tb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[db], qf[tb], acc[db][tb], 0, 0, 0);
+            const float s = (m[0] + m[2]) + (m[1] + m[3]); // 2, 1
+            if (g == 0) sums[wc * T::TOK + 16 * TB * wr + 16 * tb + l16] = s;
         }
     }
-    // register e of acc[db][tb]: output 64 wc + 16 db + 4 g + e, token 64 wr + 16 tb + l16
+    __syncthreads();
+    if (!is_v) {
 #pragma unroll
-    for (int tb = 0; tb < 4; ++tb) {
-        const int tok = tok0 + 64 * wr + 16 * tb + l16;
-        if (tok >= a.t) continue;
-        int32_t* dst = a.part + ((int64_t)split * a.t + tok) * a.n_out + col0 + 64 * wc + 4 * g;
+        for (int tb = 0; tb < TB; ++tb) {
+            const int tl = 16 * TB * wr + 16 * tb + l16;
+            const float denom = sqrtf((sums[(wc & 2) * T::TOK + tl] + sums[(wc | 1) * T::TOK + tl]) + a.eps);
 #pragma unroll
-        for (int db = 0; db < 4; ++db) *reinterpret_cast<i32x4*>(dst + 16 * db) = acc[db][tb];
+            for (int db = 0; db < 4; ++db) {
+                const int dim = hw + 16 * db + 4 * g;
+                const u32x2 gr = *reinterpret_cast<const u32x2*>(gp + dim), br = *reinterpret_cast<const u32x2*>(bp + dim);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int sh = (e & 1) * 16;
+                    y[db][tb][e] = (y[db][tb][e] / denom) * bf16_bits_to_f32((gr[e >> 1] >> sh) & 0xffffu) +
+                                   bf16_bits_to_f32((br[e >> 1] >> sh) & 0xffffu);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+            *reinterpret_cast<u32x2*>(lds + ((wc >> 1) * T::TOK + 16 * TB * wr + 16 * tb + l16) * OROW + (hw + 16 * db + 4 * g) * 2) =
+                u32x2{pack_bf16x2(y[db][tb][0], y[db][tb][1]), pack_bf16x2(y[db][tb][2], y[db][tb][3])};
+    __syncthreads();
+    // tokens x 16 pieces of 8 dims, a head to four waves; a piece's rotary partners are half dims further on or back
+    const int ohead = head0 + (tid >> 8), otid = tid & 255;
+    if (ohead >= heads) return;
+    const bool oq = ohead < a.q_heads, ov = ohead >= a.q_heads + a.kv_heads;
+    const int d0 = 8 * (otid & 15), half = a.half;
+    uint16_t* dst = ov   ? a.v + (int64_t)(ohead - a.q_heads - a.kv_heads) * AD
+                    : oq ? a.q + (int64_t)ohead * AD
+                         : a.k + (int64_t)(ohead - a.q_heads) * AD;
+    const int64_t pitch = (int64_t)(oq ? a.q_heads : a.kv_heads) * AD;
+#pragma unroll 2
+    for (int i = 0; i < T::TOK / 16; ++i) {
+        const int tl = (otid >> 4) + 16 * i, tok = tok0 + tl;
+        if (tok >= a.t) break;
+        const uint16_t* row = reinterpret_cast<const uint16_t*>(lds + ((tid >> 8) * T::TOK + tl) * OROW);
+        u32x4 o = *reinterpret_cast<const u32x4*>(row + d0);
+        if (!ov && d0 < 2 * half) {
+            const uint16_t* cp = a.cos + (int64_t)tok * half;
+            const uint16_t* sp = a.sin + (int64_t)tok * half;
+            if (half % 8 == 0) { // whole pieces on either side
+                const bool first = d0 < half;
+                const int ci = first ? d0 : d0 - half;
+                const u32x4 x = *reinterpret_cast<const u32x4*>(row + (first ? d0 + half : d0 - half));
+                const u32x4 cv = *reinterpret_cast<const u32x4*>(cp + ci), sv = *reinterpret_cast<const u32x4*>(sp + ci);
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    float r[2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const int sh = 16 * e;
+                        const float yn = bf16_bits_to_f32((o[w] >> sh) & 0xffffu), xp = bf16_bits_to_f32((x[w] >> sh) & 0xffffu);
+                        const float cs = bf16_bits_to_f32((cv[w] >> sh) & 0xffffu), sn = bf16_bits_to_f32((sv[w] >> sh) & 0xffffu);
+                        const float p0 = yn * cs, p1 = xp * sn;
+                        r[e] = first ? p0 - p1 : p0 + p1;
+                    }
+                    o[w] = pack_bf16x2(r[0], r[1]);
+                }
+            } else {
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    float r[2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const int dim = d0 + 2 * w + e;
+                        r[e] = bf16_to_f32(row[dim]);
+                        if (dim < half)
+                            r[e] = r[e] * bf16_to_f32(cp[dim]) - bf16_to_f32(row[dim + half]) * bf16_to_f32(sp[dim]);
+                        else if (dim < 2 * half)
+                            r[e] = r[e] * bf16_to_f32(cp[dim - half]) + bf16_to_f32(row[dim - half]) * bf16_to_f32(sp[dim - half]);
+                    }
+                    o[w] = pack_bf16x2(r[0], r[1]);
+                }
+            }
+        }
+        *reinterpret_cast<u32x4*>(dst + (int64_t)tok * pitch + d0) = o;
     }
 }
 
 // ------------------------------------------------------------------------------------------------ heads
-// grid (q_heads + 2 kv_heads, tokens), 128 lanes: lane = dim of the head
-__global__ __launch_bounds__(128) void apq_head_kernel(AttnPreArgs a)
+// grid (q_heads + 2 kv_heads, tokens / 4 rounded up), 256 lanes: a wave owns a head of a token, a lane its dims l and 64 + l.
+// Latency-bound: one trip for the partial sums, the rest in registers (the sum over the dims adds in the order of 64-lane
+// halves, 32, 16, .. 1 apart, then the halves).
+__global__ __launch_bounds__(256) void apq_head_kernel(AttnPreArgs a)
 {
 #pragma clang fp contract(off)
-    __shared__ float red[2];
-    __shared__ float ys[AD];
-    const int head = blockIdx.x, tok = blockIdx.y, dim = threadIdx.x;
-    const int col = head * AD + dim;
+    const int head = blockIdx.x, tok = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (tok >= a.t) return;
     const bool is_q = head < a.q_heads, is_v = head >= a.q_heads + a.kv_heads;
     // what the epilogue reads goes out first
-    const float deq = a.deq[col];
-    const int32_t qb = a.qbias[col];
     const uint16_t* gp = is_q ? a.q_gamma : a.k_gamma;
     const uint16_t* bp = is_q ? a.q_bias : a.k_bias;
-    const float gam = bf16_to_f32(gp[dim]), bia = bf16_to_f32(bp[dim]);
     const int rot = 2 * a.half;
-    const int ci = dim < a.half ? dim : (dim < rot ? dim - a.half : 0);
-    const float cs = bf16_to_f32(a.cos[(int64_t)tok * a.half + ci]), sn = bf16_to_f32(a.sin[(int64_t)tok * a.half + ci]);
-    int32_t sum = 0;
-    const int32_t* pp = a.part + (int64_t)tok * a.n_out + col;
+    float deq[2], gam[2], bia[2], cs[2], sn[2];
+    int32_t qb[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int dim = 64 * j + lane;
+        deq[j] = a.deq[head * AD + dim];
+        qb[j] = a.qbias[head * AD + dim];
+        gam[j] = bf16_to_f32(gp[dim]);
+        bia[j] = bf16_to_f32(bp[dim]);
+        const int ci = dim < a.half ? dim : (dim < rot ? dim - a.half : 0);
+        cs[j] = bf16_to_f32(a.cos[(int64_t)tok * a.half + ci]);
+        sn[j] = bf16_to_f32(a.sin[(int64_t)tok * a.half + ci]);
+    }
+    int32_t sum[2] = {0, 0};
+    const int32_t* pp = a.part + (int64_t)tok * a.n_out + head * AD + lane;
     const int64_t pstride = (int64_t)a.t * a.n_out;
 #pragma unroll 8
-    for (int sidx = 0; sidx < a.ksplits; ++sidx) sum += pp[sidx * pstride];
-    const float y = round_bf16((float)(sum + qb) * deq);
+    for (int sidx = 0; sidx < a.ksplits; ++sidx) {
+        sum[0] += pp[sidx * pstride];
+        sum[1] += pp[sidx * pstride + 64];
+    }
+    float y[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) y[j] = round_bf16((float)(sum[j] + qb[j]) * deq[j]);
     if (is_v) {
-        a.v[(int64_t)tok * a.kv_heads * AD + (head - a.q_heads - a.kv_heads) * AD + dim] = f32_to_bf16(y);
+        uint16_t* dst = a.v + ((int64_t)tok * a.kv_heads + head - a.q_heads - a.kv_heads) * AD + lane;
+        dst[0] = f32_to_bf16(y[0]);
+        dst[64] = f32_to_bf16(y[1]);
         return;
     }
-    float m = (y * y) * (1.0f / AD);
+    float m[2] = {(y[0] * y[0]) * (1.0f / AD), (y[1] * y[1]) * (1.0f / AD)};
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m += __shfl_xor(m, o, 64);
-    if ((dim & 63) == 0) red[dim >> 6] = m;
-    __syncthreads();
-    const float denom = sqrtf((red[0] + red[1]) + a.eps);
-    const float yn = round_bf16((y / denom) * gam + bia);
-    ys[dim] = yn;
-    __syncthreads();
-    float o = yn;
-    if (dim < a.half) {
-        o = yn * cs - ys[dim + a.half] * sn;
-    } else if (dim < rot) {
-        o = yn * cs + ys[dim - a.half] * sn;
+    for (int o = 32; o > 0; o >>= 1) {
+        m[0] += __shfl_xor(m[0], o, 64);
+        m[1] += __shfl_xor(m[1], o, 64);
     }
+    const float denom = sqrtf((m[0] + m[1]) + a.eps);
+    float yn[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) yn[j] = round_bf16((y[j] / denom) * gam[j] + bia[j]);
     uint16_t* dst = is_q ? a.q + ((int64_t)tok * a.q_heads + head) * AD : a.k + ((int64_t)tok * a.kv_heads + head - a.q_heads) * AD;
-    dst[dim] = f32_to_bf16(o);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int dim = 64 * j + lane;
+        const int from = dim < a.half ? dim + a.half : dim - a.half; // the rotary partner, if the dim has one
+        const float x0 = __shfl(yn[0], from & 63, 64), x1 = __shfl(yn[1], from & 63, 64), x = from & 64 ? x1 : x0;
+        float o = yn[j];
+        if (dim < a.half)
+            o = yn[j] * cs[j] - x * sn[j];
+        else if (dim < rot)
+            o = yn[j] * cs[j] + x * sn[j];
+        dst[dim] = f32_to_bf16(o);
+    }
 }
 
 } // namespace
@@ -335,28 +438,45 @@ static int stages_per_split(int64_t t, int64_t h, int64_t n_out)
     return wgs >= 8 * 448 ? 4 : wgs >= 2 * 448 ? 2 : 1;
 }
 
-// prefill sizes: stages of 128 rows per workgroup of apq_gemm_big_kernel - all of them while that still leaves
-// 256 workgroups, otherwise as many as do
+// Prefill sizes: token blocks of the tile and stages of 128 rows per workgroup of apq_gemm_big_kernel, by the time they should
+// take in ns.  The grid runs in rounds of one workgroup to each of the 256 CUs; a stage costs its matrix instructions, as the
+// token blocks, and the weights' copies, like about two of them; a round has its ends; the copies together have 26 TB/s; partial sums are written, read again at
+// 8 TB/s (the caches hold them) and cost the head kernel.
 constexpr int BIG_T = 128;
-static int big_stages_per_split(int64_t t, int64_t h, int64_t n_out)
+struct BigPlan { int tb, per; };
+static BigPlan big_plan(int64_t t, int64_t h, int64_t n_out)
 {
-    const int64_t tiles = (n_out / AD) * ((t + BTOK - 1) / BTOK), stages = h / BK;
-    const int64_t splits = std::min<int64_t>(stages, std::max<int64_t>(1, (256 + tiles - 1) / tiles));
-    return (int)((stages + splits - 1) / splits);
+    const int64_t cols = (n_out / AD + 1) / 2, stages = h / GT_KI8;
+    BigPlan best = {8, (int)stages};
+    int64_t best_ns = INT64_MAX;
+    for (const int64_t want : {1, 2, 3, 4, 5, 6, 8, 10}) {
+        const int64_t per = (stages + want - 1) / want, splits = (stages + per - 1) / per;
+        const int64_t sums = splits > 1 ? 4000 + t * n_out * 8 * splits / 8000 : 0;
+        for (int tb = 4; tb <= 8; ++tb) {
+            const int64_t wgs = cols * splits * ((t + 32 * tb - 1) / (32 * tb)), rounds = (wgs + 255) / 256;
+            const int64_t ns = rounds * (per * (tb + 2) * 160 + 12000) + wgs * per * (tb + 8) * 4096 / 26000 + sums;
+            if (ns < best_ns) best = {tb, (int)per}, best_ns = ns;
+        }
+    }
+    return best;
 }
 
 int attention_pre_ksplits(int64_t t, int64_t h, int64_t n_out)
 {
     if (t >= BIG_T) {
-        const int per = big_stages_per_split(t, h, n_out);
-        return (int)((h / BK + per - 1) / per);
+        const int per = big_plan(t, h, n_out).per;
+        return (int)((h / GT_KI8 + per - 1) / per);
     }
     const int per = stages_per_split(t, h, n_out);
     return (int)((h / AK + per - 1) / per);
 }
 
+// one split at prefill sizes: the projection's workgroups finish their heads themselves, no sums go through memory
+static bool attention_pre_whole(int64_t t, int ksplits) { return t >= BIG_T && ksplits == 1; }
+
 uint64_t attention_pre_workspace_bytes(int64_t t, int64_t h, int64_t n_out)
 {
+    if (attention_pre_whole(t, attention_pre_ksplits(t, h, n_out))) return align256((uint64_t)t * h);
     return align256((uint64_t)t * h) + (uint64_t)attention_pre_ksplits(t, h, n_out) * t * n_out * sizeof(int32_t);
 }
 
@@ -369,6 +489,7 @@ void attention_pre_bind_workspace(AttnPreArgs& a, void* ws)
 hipError_t attention_pre_launch(const AttnPreArgs& a, hipStream_t stream)
 {
     if (a.t == 0) return hipSuccess;
+    const bool whole = attention_pre_whole(a.t, a.ksplits);
     hipError_t e;
     {
         ScopedKernelTimer tm(KID_APQ_NORM, stream);
@@ -383,9 +504,14 @@ hipError_t attention_pre_launch(const AttnPreArgs& a, hipStream_t stream)
         const dim3 grid(a.n_out / AD, a.ksplits, (a.t + ATOK - 1) / ATOK);
         const int per = stages_per_split(a.t, a.h, a.n_out);
         if (a.ksplits != attention_pre_ksplits(a.t, a.h, a.n_out)) return hipErrorInvalidValue;
+        const BigPlan big = a.t >= BIG_T ? big_plan(a.t, a.h, a.n_out) : BigPlan{};
         if (a.t >= BIG_T)
-            hipLaunchKernelGGL(apq_gemm_big_kernel, dim3(a.n_out / AD, a.ksplits, (a.t + BTOK - 1) / BTOK), dim3(256), 0, stream, a,
-                               big_stages_per_split(a.t, a.h, a.n_out));
+            gt_dispatch(big.tb, [&](auto tb) {
+                constexpr int TB = decltype(tb)::value;
+                hipLaunchKernelGGL((whole ? apq_gemm_big_kernel<TB, true> : apq_gemm_big_kernel<TB, false>),
+                                   dim3((a.n_out / AD + 1) / 2, a.ksplits, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream, a,
+                                   big.per);
+            });
         else if (per == 4)
             hipLaunchKernelGGL(apq_gemm_kernel<4>, grid, dim3(256), 0, stream, a);
         else if (per == 2)
@@ -393,10 +519,10 @@ hipError_t attention_pre_launch(const AttnPreArgs& a, hipStream_t stream)
         else
             hipLaunchKernelGGL(apq_gemm_kernel<1>, grid, dim3(256), 0, stream, a);
     }
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = hipGetLastError()) != hipSuccess || whole) return e;
     {
         ScopedKernelTimer tm(KID_APQ_HEAD, stream);
-        hipLaunchKernelGGL(apq_head_kernel, dim3(a.q_heads + 2 * a.kv_heads, a.t), dim3(128), 0, stream, a);
+        hipLaunchKernelGGL(apq_head_kernel, dim3(a.q_heads + 2 * a.kv_heads, (a.t + 3) / 4), dim3(256), 0, stream, a);
     }
     return hipGetLastError();
 }

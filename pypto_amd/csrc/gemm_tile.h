@@ -1,0 +1,134 @@
+// Main loop of the products at prefill sizes: a workgroup of 512 lanes owns 32 TB tokens (128 to 256) x 256 outputs.
+//
+// What bounds these products at prefill sizes is what the CUs draw from the L2: with the matrix instructions taken out, the
+// copies of 128 x 128 tiles alone (1.03 GB for 777 tokens x 5120 x 14336) take 77 of the product's 87 us, 13 TB/s, wherever the
+// tiles lie, and staging through registers under two barriers a stage took 99 us.  So the tile is as large as LDS and registers
+// hold (537 MB and 74 us there, of which the copies hide 14 us less than all; a ring of five half stages with the fragments read
+// a stage ahead is no faster), and
+//  - a stage's operands are copied to LDS by the memory pipe itself (global_load_lds_dwordx4: no registers, no LDS store
+//    instructions), into the buffer that is not being read, so that a stage has one barrier;
+//  - rows of 128 bytes are kept unpadded (a copy writes 64 lanes x 16 bytes in a row) and spread over the banks by
+//    exchanging their 16-byte pieces, piece c of row r at position c ^ f(r): the copy takes the exchange on its global
+//    side, where the 8 lanes of a row cover the same 128 bytes in another order.
+// Wave (wr, wc) owns tokens [16 TB wr, +16 TB) x outputs [64 wc, +64).  Contraction lengths are multiples of a stage; rows past
+// the last token re-read it and are dropped by the epilogue.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "common.h"
+#include "prolog_common.h"
+
+namespace pto {
+namespace {
+
+constexpr int GT_OUT = 256;                  // outputs of a workgroup's tile: two halves of 128
+constexpr int GT_LANES = 512;
+constexpr int GT_KI8 = 128;                  // contraction rows per stage
+template <int TB>
+struct GtTile {
+    static constexpr int TOK = 32 * TB;             // tokens of the tile
+    static constexpr int QBYTES = TOK * 128;        // a stage in LDS: token rows | [2] weight rows, 128 bytes each
+    static constexpr int STAGE = QBYTES + 2 * 128 * 128;
+    static constexpr int LDS = 2 * STAGE;           // double-buffered: 96 to 128 KB, one workgroup to a CU
+};
+
+typedef __attribute__((address_space(3))) uint8_t gt_lds;
+
+// 64 lanes x 16 bytes from base + each lane's offset to 1 KB of LDS at d, in lane order; base and d are wave-uniform.  Written
+// out because the compiler, which cannot tell the buffers apart, waits for every copy in flight before the next LDS read; the
+// copies are waited for in gt_landed alone.  (One wait state between writing M0 and the copy that uses it; M0 is no register
+// that the compiler keeps values in, and nothing else in these kernels reads it.)
+__device__ __forceinline__ void gt_copy(const void* base, uint32_t offset, uint8_t* d)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"((gt_lds*)d), "v"(offset), "s"(base)
+                 : "memory");
+}
+
+// this wave's copies have landed, and with the barrier everybody's
+__device__ __forceinline__ void gt_landed()
+{
+    __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0)
+    __syncthreads();
+}
+
+// acc[nb][tb] += w[k, col0 + ..]^T . q[token, k], int8.  w0, w1: first contraction row of the two halves' columns, ldw bytes a
+// row; q: [t, ldq], column of the first contraction row.  Register e of acc[nb][tb]: output 64 wc + 16 nb + 4 g + e, token
+// 16 TB wr + 16 tb + l16.  The caller puts a barrier in front of using lds again.
+template <int TB>
+__device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t* w0, const int8_t* w1, int64_t ldw, const int8_t* q,
+                                              int64_t ldq, int tok0, int t, int stages, uint8_t* lds)
+{
+    using T = GtTile<TB>;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
+    // copy i of a wave: rows 64 i + 8 wave + lane / 8 of either operand
+    const int row = 8 * wave + (lane >> 3), pos = lane & 7;
+    const int8_t* qb = q + (int64_t)tok0 * ldq;
+    uint32_t qo[(TB + 1) / 2], wo[2];
+#pragma unroll
+    for (int i = 0; i < (TB + 1) / 2; ++i)
+        qo[i] = (uint32_t)(min(row + 64 * i, t - 1 - tok0) * (int)ldq + 16 * (pos ^ ((row >> 1) & 7)));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) wo[i] = (uint32_t)((row + 64 * i) * (int)ldw + 16 * (pos ^ (((row >> 1) & 3) | ((row >> 2) & 4))));
+    auto copy = [&](int st) {
+        uint8_t* d = lds + (st & 1) * T::STAGE + 1024 * wave;
+#pragma unroll
+        for (int i = 0; i < (TB + 1) / 2; ++i)
+            if (8 * i + wave < 4 * TB) gt_copy(qb + st * GT_KI8, qo[i], d + 8192 * i); // (uniform over the wave)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gt_copy((i < 2 ? w0 : w1) + (int64_t)st * GT_KI8 * ldw, wo[i & 1], d + T::QBYTES + 8192 * i);
+    };
+    // token fragments: row 16 TB wr + 16 tb + l16, piece 4 ks + g.  Weight fragments by the byte-transposing read, which hands
+    // lane i of a 16-lane group byte i % 8 of the chunks addressed by lanes i / 8, i / 8 + 2, ...: lane i points at row i / 2
+    // (+ 8 for the second read), half i % 2 of the 16-column piece 4 (wc & 1) + nb, and gets column i over rows 0 .. 7
+    const uint8_t* qr = lds + (16 * TB * wr + l16) * 128;
+    const int qpos = 16 * (g ^ ((l16 >> 1) & 7));
+    const uint8_t* wrow = lds + T::QBYTES + (wc >> 1) * 16384 + (16 * g + (l16 >> 1)) * 128 + 8 * (l16 & 1);
+    int wpos[4];
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) wpos[nb] = 16 * ((4 * (wc & 1) + nb) ^ (((l16 >> 2) & 3) | ((g & 1) << 2)));
+    copy(0);
+    for (int st = 0; st < stages; ++st) {
+        gt_landed(); // stage st is there, and everyone is done with the other buffer
+        if (st + 1 < stages) copy(st + 1);
+        const int b = (st & 1) * T::STAGE;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            i32x4 qf[TB], wf[4];
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) {
+                const uint8_t* p = wrow + b + 8192 * ks + wpos[nb];
+                const v2i lo = lds_read_tr8(p), hi = lds_read_tr8(p + 1024);
+                wf[nb] = i32x4{lo[0], lo[1], hi[0], hi[1]};
+            }
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb) qf[tb] = *reinterpret_cast<const i32x4*>(qr + b + 2048 * tb + (qpos ^ (64 * ks)));
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+                for (int nb = 0; nb < 4; ++nb)
+                    acc[nb][tb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[nb], qf[tb], acc[nb][tb], 0, 0, 0);
+        }
+    }
+}
+
+// f(integral constant TB) for the run-time value tb
+template <class F>
+inline void gt_dispatch(int tb, F&& f)
+{
+    switch (tb) {
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 5: f(std::integral_constant<int, 5>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    case 7: f(std::integral_constant<int, 7>{}); break;
+    default: f(std::integral_constant<int, 8>{}); break;
+    }
+}
+
+} // namespace
+} // namespace pto

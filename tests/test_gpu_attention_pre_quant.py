@@ -154,6 +154,15 @@ def test_whole_model_heads(cuda):
     check(case, run(case, cuda))
 
 
+@pytest.mark.parametrize("t,q_heads,kv_heads,half", [(128, 3, 1, 20), (129, 2, 1, 64), (1300, 48, 2, 32), (1500, 48, 2, 8), (1800, 48, 2, 1),
+                                                     (2100, 47, 2, 32)])
+def test_prefill_in_one_split(cuda, t, q_heads, kv_heads, half):
+    """One split over the contraction (short here): the projection's workgroups finish their heads themselves.  Tiles of 128,
+    160, 192, 224 and 256 tokens with a remainder, an odd number of heads, rotary halves of whole and of broken pieces."""
+    case = op.make_case(t, h=256, q_heads=q_heads, kv_heads=kv_heads, half=half, seed=40 + t)
+    check(case, run(case, cuda))
+
+
 @pytest.mark.parametrize("h,half", [(256, 64), (6144, 16), (6400, 1), (16384, 32)])
 def test_hidden_sizes_and_rotary_widths(cuda, h, half):
     """The narrowest and the widest hidden size, both sides of the switch between the two norm kernels, full and
