@@ -252,7 +252,6 @@ __global__ __launch_bounds__(GT_LANES, 2) void apq_gemm_big_kernel(AttnPreArgs a
 #pragma unroll
             for (int e = 0; e < 4; ++e) y[db][tb][e] = round_bf16((float)(acc[db][tb][e] + qb[e]) * deq[e]);
     }
-    __syncthreads(); // the operand tiles are free
     if (!is_v) {
 #pragma unroll
         for (int tb = 0; tb < TB; ++tb) {

@@ -32,7 +32,8 @@ struct GtTile {
     static constexpr int TOK = 32 * TB;             // tokens of the tile
     static constexpr int QBYTES = TOK * 128;        // a stage in LDS: token rows | [2] weight rows, 128 bytes each
     static constexpr int STAGE = QBYTES + 2 * 128 * 128;
-    static constexpr int LDS = 2 * STAGE;           // double-buffered: 96 to 128 KB, one workgroup to a CU
+    static constexpr int RING = 3 * STAGE <= 160 * 1024 ? 3 : 2; // stages in LDS, one workgroup to a CU: up to 160 tokens two in flight
+    static constexpr int LDS = RING * STAGE;
 };
 
 typedef __attribute__((address_space(3))) uint8_t gt_lds;
@@ -49,16 +50,37 @@ __device__ __forceinline__ void gt_copy(const void* base, uint32_t offset, uint8
                  : "memory");
 }
 
-// this wave's copies have landed, and with the barrier everybody's
+// all but the last N of this wave's copies have landed, and with the barrier everybody's
+template <int N>
 __device__ __forceinline__ void gt_landed()
 {
-    __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0)
+    static_assert(N < 16, "the counter's low bits");
+    __builtin_amdgcn_s_waitcnt(0x0f70 | N); // vmcnt(N)
     __syncthreads();
+}
+
+// copy(stage, byte offset of the buffer) and multiply(byte offset) over the stages, RING - 1 of them ahead; COPIES: what copy
+// issues per wave.  Past the end the last stage is copied again (the landings stay countable) and dropped.  On return nothing
+// is in flight and LDS is the caller's again.
+template <int RING, int STAGE, int COPIES, class Copy, class Multiply>
+__device__ __forceinline__ void gt_stages(int stages, Copy&& copy, Multiply&& multiply)
+{
+#pragma unroll
+    for (int s = 0; s < RING - 1; ++s) copy(min(s, stages - 1), s * STAGE);
+    int in = (RING - 1) * STAGE, out = 0;
+    for (int st = 0; st < stages; ++st) {
+        gt_landed<(RING - 2) * COPIES>(); // stage st is there, and everyone is done with the buffer of the stage before
+        copy(min(st + RING - 1, stages - 1), in);
+        multiply(st, out);
+        in = in == (RING - 1) * STAGE ? 0 : in + STAGE;
+        out = out == (RING - 1) * STAGE ? 0 : out + STAGE;
+    }
+    gt_landed<0>();
 }
 
 // acc[nb][tb] += w[k, col0 + ..]^T . q[token, k], int8.  w0, w1: first contraction row of the two halves' columns, ldw bytes a
 // row; q: [t, ldq], column of the first contraction row.  Register e of acc[nb][tb]: output 64 wc + 16 nb + 4 g + e, token
-// 16 TB wr + 16 tb + l16.  The caller puts a barrier in front of using lds again.
+// 16 TB wr + 16 tb + l16.
 template <int TB>
 __device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t* w0, const int8_t* w1, int64_t ldw, const int8_t* q,
                                               int64_t ldq, int tok0, int t, int stages, uint8_t* lds)
@@ -68,20 +90,24 @@ __device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t*
     const int l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
     // copy i of a wave: rows 64 i + 8 wave + lane / 8 of either operand
     const int row = 8 * wave + (lane >> 3), pos = lane & 7;
+    constexpr int QC = (TB + 1) / 2; // (the last rows again where eight waves have more hands than rows)
     const int8_t* qb = q + (int64_t)tok0 * ldq;
-    uint32_t qo[(TB + 1) / 2], wo[2];
+    uint32_t qo[QC], wo[2];
+    int qd[QC];
 #pragma unroll
-    for (int i = 0; i < (TB + 1) / 2; ++i)
-        qo[i] = (uint32_t)(min(row + 64 * i, t - 1 - tok0) * (int)ldq + 16 * (pos ^ ((row >> 1) & 7)));
+    for (int i = 0; i < QC; ++i) {
+        const int c = min(8 * i + wave, 4 * TB - 1), qrow = 8 * c + (lane >> 3);
+        qd[i] = 1024 * c;
+        qo[i] = (uint32_t)(min(qrow, t - 1 - tok0) * (int)ldq + 16 * (pos ^ ((qrow >> 1) & 7)));
+    }
 #pragma unroll
     for (int i = 0; i < 2; ++i) wo[i] = (uint32_t)((row + 64 * i) * (int)ldw + 16 * (pos ^ (((row >> 1) & 3) | ((row >> 2) & 4))));
-    auto copy = [&](int st) {
-        uint8_t* d = lds + (st & 1) * T::STAGE + 1024 * wave;
+    auto copy = [&](int st, int b) {
 #pragma unroll
-        for (int i = 0; i < (TB + 1) / 2; ++i)
-            if (8 * i + wave < 4 * TB) gt_copy(qb + st * GT_KI8, qo[i], d + 8192 * i); // (uniform over the wave)
+        for (int i = 0; i < QC; ++i) gt_copy(qb + st * GT_KI8, qo[i], lds + b + qd[i]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) gt_copy((i < 2 ? w0 : w1) + (int64_t)st * GT_KI8 * ldw, wo[i & 1], d + T::QBYTES + 8192 * i);
+        for (int i = 0; i < 4; ++i)
+            gt_copy((i < 2 ? w0 : w1) + (int64_t)st * GT_KI8 * ldw, wo[i & 1], lds + b + T::QBYTES + 8192 * i + 1024 * wave);
     };
     // token fragments: row 16 TB wr + 16 tb + l16, piece 4 ks + g.  Weight fragments by the byte-transposing read, which hands
     // lane i of a 16-lane group byte i % 8 of the chunks addressed by lanes i / 8, i / 8 + 2, ...: lane i points at row i / 2
@@ -92,11 +118,7 @@ __device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t*
     int wpos[4];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) wpos[nb] = 16 * ((4 * (wc & 1) + nb) ^ (((l16 >> 2) & 3) | ((g & 1) << 2)));
-    copy(0);
-    for (int st = 0; st < stages; ++st) {
-        gt_landed(); // stage st is there, and everyone is done with the other buffer
-        if (st + 1 < stages) copy(st + 1);
-        const int b = (st & 1) * T::STAGE;
+    gt_stages<T::RING, T::STAGE, QC + 4>(stages, copy, [&](int, int b) {
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
             i32x4 qf[TB], wf[4];
@@ -114,7 +136,79 @@ __device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t*
                 for (int nb = 0; nb < 4; ++nb)
                     acc[nb][tb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[nb], qf[tb], acc[nb][tb], 0, 0, 0);
         }
-    }
+    });
+}
+
+// The same loop in bf16 for 128 tokens x 256 outputs, the outputs in four blocks of 64 columns at src[i], ld[i] values a row;
+// x: [t, ldx], column of the first contraction row.  Wave (wr, wc) owns tokens [64 wr, +64) x block wc.  Register e of
+// sum[tb][nb]: token 64 wr + 32 tb + 8 (e / 4) + 4 hl + e % 4, column 32 nb + lane % 32 of the block.  Sums are chains of at most
+// CHAIN contraction rows, added up in order.
+constexpr int GT_KBF = 64; // contraction rows per stage
+template <int CHAIN>
+__device__ __forceinline__ void gt_product_bf16(f32x16 (&sum)[2][2], const uint16_t* const (&src)[4], const int (&ld)[4], const uint16_t* x,
+                                                int64_t ldx, int tok0, int t, int stages, uint8_t* lds)
+{
+    using T = GtTile<4>;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, hl = lane >> 5, jj = lane & 15, mh = (lane >> 4) & 1, wr = wave >> 2, wc = wave & 3;
+    const int row = 8 * wave + (lane >> 3), pos = lane & 7;
+    const uint16_t* xb = x + (int64_t)tok0 * ldx;
+    uint32_t xo[2], wo[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        xo[i] = (uint32_t)(min(row + 64 * i, t - 1 - tok0) * (int)ldx * 2 + 16 * (pos ^ ((row >> 1) & 7)));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wo[i] = (uint32_t)(row * ld[i] * 2 + 16 * (pos ^ ((row << 1) & 4)));
+    auto copy = [&](int st, int b) {
+        uint8_t* d = lds + b + 1024 * wave;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) gt_copy(xb + st * GT_KBF, xo[i], d + 8192 * i);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gt_copy(src[i] + (int64_t)st * GT_KBF * ld[i], wo[i], d + T::QBYTES + 8192 * i);
+    };
+    // token fragments: row 64 wr + 32 tb + l32, piece 2 ks + hl.  Weight fragments by 16-bit transposing reads: lane jj of a
+    // 16-lane group points at row 8 hl + jj / 4 (+ 4 for the second read) of the step, columns 16 mh + 4 (jj & 3), and gets
+    // column 16 mh + jj over those rows
+    const uint8_t* xr = lds + (64 * wr + l32) * 128;
+    const int xf = (l32 >> 1) & 7;
+    const uint8_t* wrow = lds + T::QBYTES + wc * 8192 + (8 * hl + (jj >> 2)) * 128 + 8 * (jj & 1);
+    const int wpos = 16 * ((2 * mh + ((jj >> 1) & 1)) ^ ((jj >> 1) & 4));
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[tb][nb][e] = sum[tb][nb][e] = 0.f;
+    gt_stages<T::RING, T::STAGE, 6>(stages, copy, [&](int st, int b) {
+#pragma unroll
+        for (int ks = 0; ks < GT_KBF / 16; ++ks) {
+            bf16x8 xv[2], wv[2];
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                const uint8_t* p = wrow + b + 2048 * ks + (wpos ^ (64 * nb));
+                const s16x4 lo = lds_read_tr(p), hi = lds_read_tr(p + 512);
+                wv[nb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            }
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) xv[tb] = *reinterpret_cast<const bf16x8*>(xr + b + 4096 * tb + 16 * ((2 * ks + hl) ^ xf));
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) acc[tb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv[tb], wv[nb], acc[tb][nb], 0, 0, 0);
+        }
+        if ((st + 1) % (CHAIN / GT_KBF) == 0 || st + 1 == stages) {
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        sum[tb][nb][e] += acc[tb][nb][e];
+                        acc[tb][nb][e] = 0.f;
+                    }
+        }
+    });
 }
 
 // f(integral constant TB) for the run-time value tb

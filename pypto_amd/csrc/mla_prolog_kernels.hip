@@ -29,6 +29,7 @@
 #include <stdint.h>
 
 #include "common.h"
+#include "gemm_tile.h"
 #include "kernels.h"
 #include "prolog_common.h"
 #include "prolog_device.h"
@@ -51,10 +52,7 @@ constexpr int QB_MAXS = MAX_R / QB_K / QB_GROUPS; // stages per group at the lar
 constexpr int QB_QP = MTOK * (MAX_R / 16) / 1024; // 16-byte pieces of the q_norm tile per lane at the largest q_lora_rank
 constexpr int BIG_T = 128;        // token count from which the kernels that own an output tile take over
 constexpr int BIG_T2 = 256;       // token count above which their tiles are 256 tokens tall
-#ifndef XA_BIG2_DEPTH
-#define XA_BIG2_DEPTH 2
-#endif
-
+constexpr int QB16_WIDE_T = 33;   // token count from which the bf16 form's q_b product runs per 128 tokens
 
 // 32 outputs x 32 tokens += W[KSTEPS steps of 16 rows, outputs]^T . X[tokens, k]: A by transposing reads of the [k][n]
 // tile in LDS, rows of ROWB bytes.  Lane jj of a 16-lane group points at row 8 hl + jj / 4 (+ 4 for the second read) of
@@ -265,6 +263,50 @@ __global__ __launch_bounds__(256, TB == 1 ? 3 : 2) void mla_xa_big_kernel(MlaPro
         }
 }
 
+// Above 256 tokens the workgroup owns 128 tokens x 256 outputs (gemm_tile.h) over one split of the contraction, a multiple of
+// 256 rows chosen so that the workgroups fill the CUs once: few splits, so few partial sums.  Seven splits of 1024 rows
+// with 256 x 64 tiles wrote 97 MB of partial sums at 1501 tokens, which the norm kernel read again.  An XCD takes neighbouring
+// workgroups in the order token tile, output tile, split.  grid (workgroups rounded up to a multiple of 8), 512 lanes.
+__global__ __launch_bounds__(GT_LANES, 2) void mla_xa_wide_kernel(MlaPrologArgs a, int ttiles, int ntiles, int rows)
+{
+    using T = GtTile<4>;
+    __shared__ __align__(16) uint8_t lds[T::LDS];
+    const int id = (int)(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8);
+    const int tok0 = id % ttiles * T::TOK, nt = id / ttiles % ntiles, split = id / ttiles / ntiles;
+    if (split >= a.ksplits) return; // uniform over the workgroup
+    const int kbeg = split * rows, stages = (min(a.h, kbeg + rows) - kbeg) / GT_KBF;
+    const uint16_t* src[4];
+    int ld[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { // (blocks past the last one: that one again, dropped below)
+        src[i] = xa_source(a, min(4 * nt + i, a.ncols / 64 - 1), ld[i]);
+        src[i] += (int64_t)kbeg * ld[i];
+    }
+    f32x16 acc[2][2];
+    gt_product_bf16<XA_SPLIT>(acc, src, ld, a.x + kbeg, a.h, tok0, a.t, stages, lds);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, hl = lane >> 5, wr = wave >> 2, wc = wave & 3;
+    const int col0 = (4 * nt + wc) * 64;
+    if (col0 >= a.ncols) return;
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int gt = tok0 + 64 * wr + 32 * tb + 8 * (e >> 2) + 4 * hl + (e & 3);
+            if (gt >= a.t) continue;
+            float* out = a.xa_part + ((int64_t)split * a.t + gt) * a.ncols + col0 + l32;
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) out[32 * nb] = acc[tb][nb][e];
+        }
+}
+// its contraction rows per split: as many splits of at least 256 rows as there are CUs for, and no more than the workspace
+// holds.  The same with and without the indexer's columns (counted in), so that the fused operator's sums are the others'.
+static int xa_wide_rows(int64_t t, int64_t h, int64_t r)
+{
+    const int64_t tiles = ((t + 127) / 128) * ((r + MKV + PD + 64 + 255) / 256), most = (h + XA_SPLIT - 1) / XA_SPLIT;
+    const int64_t splits = std::max<int64_t>(1, std::min<int64_t>(most, 256 / tiles));
+    return (int)((h / XA_K + splits - 1) / splits) * XA_K;
+}
+
 // bf16 form of the operator: q_b = q_norm (bf16 [t, r]) @ w_uq_qr (bf16 [r, n * 192]) with the same kernel body;
 // grid (ceil(r / 1024), n * 192 / 64, token tiles of 32); partial sums to qb_part
 __global__ __launch_bounds__(1024) void mla_qb16_kernel(MlaPrologArgs a)
@@ -304,6 +346,84 @@ __global__ __launch_bounds__(256) void mla_qb16_epilogue_kernel(MlaPrologArgs a)
             const float o2 = xo * bf16_to_f32(cp[i + 32]) + xe * bf16_to_f32(snp[i + 32]);
             out[i] = f32_to_bf16(o1);
             out[i + 32] = f32_to_bf16(o2);
+        }
+    }
+}
+
+// The bf16 form at more tokens: 128 tokens x 256 outputs per workgroup over the whole contraction (gemm_tile.h), the epilogue
+// on the tile.  The pair above reads the weights once per 32 tokens and hands fp32 partial sums through memory: 811 us at
+// 1000 tokens.  A block of 64 outputs is half of a head's 128 first dims or its rotary dims; the tile goes through LDS so that
+// it leaves in 16-byte pieces.  grid (n * 192 / 256 rounded up, token tiles of 128), 512 lanes.
+__global__ __launch_bounds__(GT_LANES, 2) void mla_qb16_wide_kernel(MlaPrologArgs a)
+{
+#pragma clang fp contract(off)
+    using T = GtTile<4>;
+    constexpr int OROW = 64 * 2 + 16; // bytes per LDS row of a block's output tile (padded against bank conflicts)
+    static_assert(4 * T::TOK * OROW <= T::LDS, "the output tile takes the operand tiles' place");
+    __shared__ __align__(16) uint8_t lds[T::LDS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hl = lane >> 5, wr = wave >> 2, wc = wave & 3;
+    const int blocks = a.n * MQH / 64, block0 = 4 * blockIdx.x, tok0 = blockIdx.y * T::TOK;
+    const uint16_t* src[4];
+    int ld[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { // (blocks past the last one: that one again, dropped below)
+        src[i] = static_cast<const uint16_t*>(a.w_uq_qr) + min(block0 + i, blocks - 1) * 64;
+        ld[i] = a.n * MQH;
+    }
+    f32x16 acc[2][2];
+    gt_product_bf16<256>(acc, src, ld, reinterpret_cast<const uint16_t*>(a.q_norm), a.r, tok0, a.t, a.r / GT_KBF, lds);
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int tl = 64 * wr + 32 * tb + 8 * (e >> 2) + 4 * hl + (e & 3);
+            uint16_t* row = reinterpret_cast<uint16_t*>(lds + (wc * T::TOK + tl) * OROW) + l32;
+            row[0] = f32_to_bf16(acc[tb][0][e]);
+            row[32] = f32_to_bf16(acc[tb][1][e]);
+        }
+    __syncthreads();
+    const int bl = tid >> 7, block = block0 + bl, head = block / 3; // two waves to a block
+    if (block >= blocks) return;
+    const uint8_t* tile = lds + bl * T::TOK * OROW;
+    if (block % 3 < 2) { // 8 pieces of 8 dims
+        uint16_t* dst = a.qb_nope + head * MNOPE + block % 3 * 64 + 8 * (tid & 7);
+#pragma unroll
+        for (int i = 0; i < T::TOK / 16; ++i) {
+            const int tl = ((tid >> 3) & 15) + 16 * i;
+            if (tok0 + tl < a.t)
+                *reinterpret_cast<u32x4*>(dst + (int64_t)(tok0 + tl) * a.n * MNOPE) =
+                    *reinterpret_cast<const u32x4*>(tile + tl * OROW + 16 * (tid & 7));
+        }
+    } else { // 4 times 8 pairs, rotated into the two halves
+        const int i0 = 8 * (tid & 3);
+#pragma unroll
+        for (int i = 0; i < T::TOK / 32; ++i) {
+            const int tl = ((tid >> 2) & 31) + 32 * i, gt = tok0 + tl;
+            if (gt >= a.t) continue;
+            const u32x4* x = reinterpret_cast<const u32x4*>(tile + tl * OROW + 4 * i0);
+            const uint16_t* cp = a.cos + (int64_t)gt * MROPE + i0;
+            const uint16_t* sp = a.sin + (int64_t)gt * MROPE + i0;
+            const u32x4 xa = x[0], xb = x[1];
+            const u32x4 c1 = *reinterpret_cast<const u32x4*>(cp), c2 = *reinterpret_cast<const u32x4*>(cp + 32);
+            const u32x4 s1 = *reinterpret_cast<const u32x4*>(sp), s2 = *reinterpret_cast<const u32x4*>(sp + 32);
+            u32x4 o1, o2;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                float r1[2], r2[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const uint32_t pair = w < 2 ? xa[2 * w + e] : xb[2 * w + e - 4];
+                    const int sh = 16 * e;
+                    const float xe = bf16_bits_to_f32(pair & 0xffffu), xo = bf16_bits_to_f32(pair >> 16);
+                    r1[e] = xe * bf16_bits_to_f32((c1[w] >> sh) & 0xffffu) + (-xo) * bf16_bits_to_f32((s1[w] >> sh) & 0xffffu);
+                    r2[e] = xo * bf16_bits_to_f32((c2[w] >> sh) & 0xffffu) + xe * bf16_bits_to_f32((s2[w] >> sh) & 0xffffu);
+                }
+                o1[w] = pack_bf16x2(r1[0], r1[1]);
+                o2[w] = pack_bf16x2(r2[0], r2[1]);
+            }
+            uint16_t* out = a.q_rope + ((int64_t)gt * a.n + head) * MROPE + i0;
+            *reinterpret_cast<u32x4*>(out) = o1;
+            *reinterpret_cast<u32x4*>(out + 32) = o2;
         }
     }
 }
@@ -914,12 +1034,16 @@ uint64_t mla_prolog_workspace_bytes(int64_t t, int64_t h, int64_t r, int64_t n, 
 {
     // bf16 form: also the partial sums of q_norm @ w_uq_qr
     return xa_part_bytes(t, h, r + MKV + (n_idx ? PD + n_idx : 0)) + up256((uint64_t)t * n * MNOPE * 2) +
-           (quant ? 0 : xa_part_bytes(t, r, n * MQH));
+           (quant || t >= QB16_WIDE_T ? 0 : xa_part_bytes(t, r, n * MQH));
 }
 
 void mla_prolog_bind_workspace(MlaPrologArgs& a, void* ws)
 {
     uint8_t* p = static_cast<uint8_t*>(ws);
+    if (a.t > BIG_T2) {
+        const int rows = xa_wide_rows(a.t, a.h, a.r);
+        a.ksplits = (a.h + rows - 1) / rows;
+    }
     a.xa_part = reinterpret_cast<float*>(p);
     p += xa_part_bytes(a.t, a.h, a.ncols);
     a.qb_nope = reinterpret_cast<uint16_t*>(p);
@@ -974,8 +1098,12 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         if (big)
             if (a.t <= BIG_T2)
                 hipLaunchKernelGGL((mla_xa_big_kernel<1, 4>), dim3(a.ksplits, a.ncols / 64, (a.t + 127) / 128), dim3(256), 0, stream, a);
-            else
-                hipLaunchKernelGGL((mla_xa_big_kernel<2, XA_BIG2_DEPTH>), dim3(a.ksplits, a.ncols / 64, (a.t + 255) / 256), dim3(256), 0, stream, a);
+            else {
+                const int xtiles = (a.t + 127) / 128, ntiles = (a.ncols + 255) / 256, rows = xa_wide_rows(a.t, a.h, a.r);
+                if (a.ksplits != (a.h + rows - 1) / rows) return hipErrorInvalidValue;
+                hipLaunchKernelGGL(mla_xa_wide_kernel, dim3((xtiles * ntiles * a.ksplits + 7) / 8 * 8), dim3(GT_LANES), 0, stream, a, xtiles,
+                                   ntiles, rows);
+            }
         else
             hipLaunchKernelGGL(mla_xa_kernel, dim3(a.ksplits, a.ncols / 64, ttiles), dim3(1024), 4 * XA_K * XROW2, stream, a);
     }
@@ -990,7 +1118,9 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
     if ((e = hipGetLastError()) != hipSuccess) return e;
     {
         ScopedKernelTimer tm(KID_MLA_QB, stream);
-        if (!a.quant) {
+        if (!a.quant && a.t >= QB16_WIDE_T) {
+            hipLaunchKernelGGL(mla_qb16_wide_kernel, dim3((a.n * MQH + 255) / 256, (a.t + 127) / 128), dim3(GT_LANES), 0, stream, a);
+        } else if (!a.quant) {
             const int nq = a.n * MQH;
             hipLaunchKernelGGL(mla_qb16_kernel, dim3((a.r + XA_SPLIT - 1) / XA_SPLIT, nq / 64, ttiles), dim3(1024),
                                4 * XA_K * XROW2, stream, a);
