@@ -438,9 +438,7 @@ static int stages_per_split(int64_t t, int64_t h, int64_t n_out)
 }
 
 // Prefill sizes: token blocks of the tile and stages of 128 rows per workgroup of apq_gemm_big_kernel, by the time they should
-// take in ns.  The grid runs in rounds of one workgroup to each of the 256 CUs; a stage costs its matrix instructions, as the
-// token blocks, and the weights' copies, like about two of them; a round has its ends; the copies together have 26 TB/s; partial sums are written, read again at
-// 8 TB/s (the caches hold them) and cost the head kernel.
+// take in ns (gt_time_ns); partial sums are written, read again at 8 TB/s (the caches hold them) and cost the head kernel.
 constexpr int BIG_T = 128;
 struct BigPlan { int tb, per; };
 static BigPlan big_plan(int64_t t, int64_t h, int64_t n_out)
@@ -452,8 +450,7 @@ static BigPlan big_plan(int64_t t, int64_t h, int64_t n_out)
         const int64_t per = (stages + want - 1) / want, splits = (stages + per - 1) / per;
         const int64_t sums = splits > 1 ? 4000 + t * n_out * 8 * splits / 8000 : 0;
         for (int tb = 4; tb <= 8; ++tb) {
-            const int64_t wgs = cols * splits * ((t + 32 * tb - 1) / (32 * tb)), rounds = (wgs + 255) / 256;
-            const int64_t ns = rounds * (per * (tb + 2) * 160 + 12000) + wgs * per * (tb + 8) * 4096 / 26000 + sums;
+            const int64_t ns = gt_time_ns(cols * splits * ((t + 32 * tb - 1) / (32 * tb)), per, tb) + sums;
             if (ns < best_ns) best = {tb, (int)per}, best_ns = ns;
         }
     }

@@ -211,6 +211,24 @@ __device__ __forceinline__ void gt_product_bf16(f32x16 (&sum)[2][2], const uint1
     });
 }
 
+// Token blocks TB (4 .. most) of an int8 product's tile, by the time it should take in ns: the grid runs in rounds of one
+// workgroup to each of the 256 CUs; a stage costs its matrix instructions, as the token blocks, and the weights' copies, like
+// about two of them; a round has its ends; the copies together have 26 TB/s.
+inline int64_t gt_time_ns(int64_t wgs, int64_t stages, int tb)
+{
+    return (wgs + 255) / 256 * (stages * (tb + 2) * 160 + 12000) + wgs * stages * (tb + 8) * 4096 / 26000;
+}
+inline int gt_token_blocks(int64_t t, int64_t cols, int64_t stages, int most)
+{
+    int best = 4;
+    int64_t best_ns = INT64_MAX;
+    for (int tb = 4; tb <= most; ++tb) {
+        const int64_t ns = gt_time_ns(cols * ((t + 32 * tb - 1) / (32 * tb)), stages, tb);
+        if (ns < best_ns) best = tb, best_ns = ns;
+    }
+    return best;
+}
+
 // f(integral constant TB) for the run-time value tb
 template <class F>
 inline void gt_dispatch(int tb, F&& f)

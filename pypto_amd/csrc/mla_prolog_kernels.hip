@@ -350,57 +350,34 @@ __global__ __launch_bounds__(256) void mla_qb16_epilogue_kernel(MlaPrologArgs a)
     }
 }
 
-// The bf16 form at more tokens: 128 tokens x 256 outputs per workgroup over the whole contraction (gemm_tile.h), the epilogue
-// on the tile.  The pair above reads the weights once per 32 tokens and hands fp32 partial sums through memory: 811 us at
-// 1000 tokens.  A block of 64 outputs is half of a head's 128 first dims or its rotary dims; the tile goes through LDS so that
-// it leaves in 16-byte pieces.  grid (n * 192 / 256 rounded up, token tiles of 128), 512 lanes.
-__global__ __launch_bounds__(GT_LANES, 2) void mla_qb16_wide_kernel(MlaPrologArgs a)
+// Four blocks of 64 outputs of q_b, TOK tokens each, from LDS rows of QBS_ROW bytes (padded against bank conflicts) to memory in
+// 16-byte pieces: a block is half of a head's 128 first dims, or its rotary dims, rotated on the way.  512 lanes, two waves to a
+// block.
+constexpr int QBS_ROW = 64 * 2 + 16;
+template <int TOK>
+__device__ __forceinline__ void qb_store_blocks(const MlaPrologArgs& a, const uint8_t* lds, int block0, int tok0)
 {
 #pragma clang fp contract(off)
-    using T = GtTile<4>;
-    constexpr int OROW = 64 * 2 + 16; // bytes per LDS row of a block's output tile (padded against bank conflicts)
-    static_assert(4 * T::TOK * OROW <= T::LDS, "the output tile takes the operand tiles' place");
-    __shared__ __align__(16) uint8_t lds[T::LDS];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hl = lane >> 5, wr = wave >> 2, wc = wave & 3;
-    const int blocks = a.n * MQH / 64, block0 = 4 * blockIdx.x, tok0 = blockIdx.y * T::TOK;
-    const uint16_t* src[4];
-    int ld[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { // (blocks past the last one: that one again, dropped below)
-        src[i] = static_cast<const uint16_t*>(a.w_uq_qr) + min(block0 + i, blocks - 1) * 64;
-        ld[i] = a.n * MQH;
-    }
-    f32x16 acc[2][2];
-    gt_product_bf16<256>(acc, src, ld, reinterpret_cast<const uint16_t*>(a.q_norm), a.r, tok0, a.t, a.r / GT_KBF, lds);
-#pragma unroll
-    for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int tl = 64 * wr + 32 * tb + 8 * (e >> 2) + 4 * hl + (e & 3);
-            uint16_t* row = reinterpret_cast<uint16_t*>(lds + (wc * T::TOK + tl) * OROW) + l32;
-            row[0] = f32_to_bf16(acc[tb][0][e]);
-            row[32] = f32_to_bf16(acc[tb][1][e]);
-        }
-    __syncthreads();
+    const int tid = threadIdx.x, blocks = a.n * MQH / 64;
     const int bl = tid >> 7, block = block0 + bl, head = block / 3; // two waves to a block
     if (block >= blocks) return;
-    const uint8_t* tile = lds + bl * T::TOK * OROW;
+    const uint8_t* tile = lds + bl * TOK * QBS_ROW;
     if (block % 3 < 2) { // 8 pieces of 8 dims
         uint16_t* dst = a.qb_nope + head * MNOPE + block % 3 * 64 + 8 * (tid & 7);
 #pragma unroll
-        for (int i = 0; i < T::TOK / 16; ++i) {
+        for (int i = 0; i < TOK / 16; ++i) {
             const int tl = ((tid >> 3) & 15) + 16 * i;
             if (tok0 + tl < a.t)
                 *reinterpret_cast<u32x4*>(dst + (int64_t)(tok0 + tl) * a.n * MNOPE) =
-                    *reinterpret_cast<const u32x4*>(tile + tl * OROW + 16 * (tid & 7));
+                    *reinterpret_cast<const u32x4*>(tile + tl * QBS_ROW + 16 * (tid & 7));
         }
     } else { // 4 times 8 pairs, rotated into the two halves
         const int i0 = 8 * (tid & 3);
 #pragma unroll
-        for (int i = 0; i < T::TOK / 32; ++i) {
+        for (int i = 0; i < TOK / 32; ++i) {
             const int tl = ((tid >> 2) & 31) + 32 * i, gt = tok0 + tl;
             if (gt >= a.t) continue;
-            const u32x4* x = reinterpret_cast<const u32x4*>(tile + tl * OROW + 4 * i0);
+            const u32x4* x = reinterpret_cast<const u32x4*>(tile + tl * QBS_ROW + 4 * i0);
             const uint16_t* cp = a.cos + (int64_t)gt * MROPE + i0;
             const uint16_t* sp = a.sin + (int64_t)gt * MROPE + i0;
             const u32x4 xa = x[0], xb = x[1];
@@ -426,6 +403,39 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb16_wide_kernel(MlaPrologArg
             *reinterpret_cast<u32x4*>(out + 32) = o2;
         }
     }
+}
+
+// The bf16 form at more tokens: 128 tokens x 256 outputs per workgroup over the whole contraction (gemm_tile.h), the epilogue
+// on the tile.  The pair above reads the weights once per 32 tokens and hands fp32 partial sums through memory: 811 us at
+// 1000 tokens.  grid (n * 192 / 256 rounded up, token tiles of 128), 512 lanes.
+__global__ __launch_bounds__(GT_LANES, 2) void mla_qb16_wide_kernel(MlaPrologArgs a)
+{
+#pragma clang fp contract(off)
+    using T = GtTile<4>;
+    static_assert(4 * T::TOK * QBS_ROW <= T::LDS, "the output tile takes the operand tiles' place");
+    __shared__ __align__(16) uint8_t lds[T::LDS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hl = lane >> 5, wr = wave >> 2, wc = wave & 3;
+    const int blocks = a.n * MQH / 64, block0 = 4 * blockIdx.x, tok0 = blockIdx.y * T::TOK;
+    const uint16_t* src[4];
+    int ld[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { // (blocks past the last one: that one again, dropped below)
+        src[i] = static_cast<const uint16_t*>(a.w_uq_qr) + min(block0 + i, blocks - 1) * 64;
+        ld[i] = a.n * MQH;
+    }
+    f32x16 acc[2][2];
+    gt_product_bf16<256>(acc, src, ld, reinterpret_cast<const uint16_t*>(a.q_norm), a.r, tok0, a.t, a.r / GT_KBF, lds);
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int tl = 64 * wr + 32 * tb + 8 * (e >> 2) + 4 * hl + (e & 3);
+            uint16_t* row = reinterpret_cast<uint16_t*>(lds + (wc * T::TOK + tl) * QBS_ROW) + l32;
+            row[0] = f32_to_bf16(acc[tb][0][e]);
+            row[32] = f32_to_bf16(acc[tb][1][e]);
+        }
+    __syncthreads();
+    qb_store_blocks<T::TOK>(a, lds, block0, tok0);
 }
 
 // ------------------------------------------------------------------------------------------------ norms, quantisation, cache
@@ -878,6 +888,45 @@ __global__ __launch_bounds__(256, DEPTH == 1 ? 3 : 2) void mla_qb_big_kernel(Mla
     mla_qb_big_body<DEPTH>(a, blockIdx.x * 128, blockIdx.y * QG_TOK, stage_lds);
 }
 
+// Above 256 tokens: 32 TB tokens x 256 outputs per workgroup (gemm_tile.h), the same exact sums and the same operations behind
+// them.  128 x 128 tiles through registers took 109 us at 1501 tokens, bound by the operands' way into LDS.
+// grid (n * 192 / 256 rounded up, token tiles), 512 lanes.
+template <int TB>
+__global__ __launch_bounds__(GT_LANES, 2) void mla_qb_wide_kernel(MlaPrologArgs a)
+{
+#pragma clang fp contract(off)
+    using T = GtTile<TB>;
+    constexpr int EPI = 4 * T::TOK * QBS_ROW;
+    __shared__ __align__(16) uint8_t lds[EPI > T::LDS ? EPI : T::LDS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
+    const int nq = a.n * MQH, col0 = 256 * blockIdx.x, tok0 = blockIdx.y * T::TOK; // (nq is a multiple of 128)
+    i32x4 acc[4][TB]; // [nb][tb]
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
+    const int8_t* w = static_cast<const int8_t*>(a.w_uq_qr);
+    gt_product_i8<TB>(acc, w + col0, w + min(col0 + 128, nq - 128), nq, a.q_norm, a.r, tok0, a.t, a.r / GT_KI8, lds);
+    // register e of acc[nb][tb]: output 64 wc + 16 nb + 4 g + e, token 16 TB wr + 16 tb + l16
+    f32x4 ws[4];
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + min(col0 + 64 * wc, nq - 64) + 16 * nb + 4 * g);
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) {
+        const int tl = 16 * TB * wr + 16 * tb + l16;
+        const float qs = a.q_norm_scale[min(tok0 + tl, a.t - 1)];
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs) * ws[nb][e];
+            *reinterpret_cast<u32x2*>(lds + (wc * T::TOK + tl) * QBS_ROW + 32 * nb + 8 * g) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        }
+    }
+    __syncthreads();
+    qb_store_blocks<T::TOK>(a, lds, 4 * blockIdx.x, tok0);
+}
+
 // ------------------------------------------------------------------------------------------------ fused with the indexer prolog
 // The fused operator runs the two prologs' per-token kernels side by side in one launch, and likewise the two int8
 // GEMMs on q_norm (192 + 64 workgroups at model sizes: one per compute unit); the indexer's x @ [w_k | w_proj] rides along
@@ -918,13 +967,13 @@ __global__ __launch_bounds__(256, 2) void fused_qb_big_kernel(MlaPrologArgs m, P
         prolog_q_big_body<QB_DEPTH>(p, blockIdx.x - nqb, blockIdx.y * QB_TOK, lds);
 }
 
-// Above 256 tokens the two products are launches of their own again: the MLA product then fills the chip at three
-// workgroups to a CU (one stage of loads in flight, 36 KB of LDS), which the shared launch's 68 KB would not allow.
-// grid (index heads, token tiles of 128), 256 lanes
-__global__ __launch_bounds__(256, 2) void fused_q_big_kernel(PrologArgs p)
+// Above 256 tokens the two products are launches of their own again, with tiles of their own sizes.
+// grid (index heads / 2 rounded up, token tiles), 512 lanes
+template <int TB>
+__global__ __launch_bounds__(GT_LANES, 2) void fused_q_wide_kernel(PrologArgs p)
 {
-    __shared__ __align__(16) uint8_t lds[QB_LDS_BYTES];
-    prolog_q_big_body<QB_DEPTH>(p, blockIdx.x, blockIdx.y * QB_TOK, lds);
+    __shared__ __align__(16) uint8_t lds[prolog_q_wide_lds(TB)];
+    prolog_q_wide_body<TB>(p, 2 * blockIdx.x, blockIdx.y * 32 * TB, lds);
 }
 
 // ------------------------------------------------------------------------------------------------ q_b[:, head, :128] @ w_uk[head]
@@ -1130,11 +1179,22 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
             if (p && a.t <= BIG_T2) {
                 hipLaunchKernelGGL(fused_qb_big_kernel, dim3(qgrid.x + p->n, qgrid.y), dim3(256), 0, stream, a, *p);
             } else {
-                if (a.t <= BIG_T2)
-                    hipLaunchKernelGGL(mla_qb_big_kernel<3>, qgrid, dim3(256), 0, stream, a);
-                else
-                    hipLaunchKernelGGL(mla_qb_big_kernel<1>, qgrid, dim3(256), 0, stream, a);
-                if (p) hipLaunchKernelGGL(fused_q_big_kernel, dim3(p->n, qgrid.y), dim3(256), 0, stream, *p);
+                if (a.t <= BIG_T2) {
+                    hipLaunchKernelGGL(mla_qb_big_kernel<QB_DEPTH>, qgrid, dim3(256), 0, stream, a);
+                } else {
+                    const int cols = (a.n * MQH + 255) / 256;
+                    gt_dispatch(gt_token_blocks(a.t, cols, a.r / GT_KI8, 8), [&](auto tb) {
+                        constexpr int TB = decltype(tb)::value;
+                        hipLaunchKernelGGL(mla_qb_wide_kernel<TB>, dim3(cols, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream, a);
+                    });
+                }
+                if (p) {
+                    const int cols = (p->n + 1) / 2;
+                    gt_dispatch(gt_token_blocks(a.t, cols, a.r / GT_KI8, 7), [&](auto tb) {
+                        constexpr int TB = decltype(tb)::value < 7 ? decltype(tb)::value : 7;
+                        hipLaunchKernelGGL(fused_q_wide_kernel<TB>, dim3(cols, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream, *p);
+                    });
+                }
             }
         } else if (p) {
             const int smem = mla_qb_lds_bytes(a.r) > prolog_q_lds_bytes(a.r) ? mla_qb_lds_bytes(a.r) : prolog_q_lds_bytes(a.r);

@@ -1,6 +1,7 @@
 // Lightning-indexer prolog: device bodies of the query and the key kernels, shared by the operator's own kernels
 // (prolog_kernels.hip) and by the fused MLA + indexer prolog (mla_prolog_kernels.hip).
 #pragma once
+#include "gemm_tile.h"
 #include "kernels.h"
 #include "prolog_common.h"
 
@@ -431,6 +432,134 @@ __device__ __forceinline__ void prolog_q_big_body(const PrologArgs& a, int head,
                 *reinterpret_cast<uint32_t*>(qo + 8 * e4) = pk;
             }
             if (wave == 0 && hl == 0) a.q_scale[(int64_t)gt * a.n + head] = __builtin_bit_cast(uint16_t, (_Float16)(1.0f / sq));
+        }
+    }
+}
+// Above 256 tokens: 32 TB tokens x two heads per workgroup (gemm_tile.h), four waves to a head behind the product; the
+// operations are prolog_q_big_body's, so are the bits (51 us at 1501 tokens there).  512 lanes; an odd last head is taken twice
+// and dropped.
+constexpr int prolog_q_wide_lds(int tb) // the product's stages, or hadamard_q | [2] bf16 tiles | [2] per-wave maxima
+{
+    const int tok = 32 * tb, stage = tok * 128 + 2 * 128 * 128, ring = (3 * stage <= 160 * 1024 ? 3 : 2) * stage;
+    const int epi = PD * PD * 2 + 2 * tok * XROW + 2 * 4 * tok * 4;
+    return epi > ring ? epi : ring;
+}
+template <int TB>
+__device__ __forceinline__ void prolog_q_wide_body(const PrologArgs& a, int head0, int tok0, uint8_t* lds)
+{
+#pragma clang fp contract(off)
+    constexpr int TOK = 32 * TB;
+    static_assert(prolog_q_wide_lds(TB) <= 160 * 1024 && prolog_q_wide_lds(TB) >= GtTile<TB>::LDS, "LDS");
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int l16 = lane & 15, g = lane >> 4, l32 = lane & 31, hl = lane >> 5, wr = wave >> 2, wc = wave & 3;
+    const int64_t nd = (int64_t)a.n * PD;
+    i32x4 acc[4][TB]; // [nb][tb]
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
+    gt_product_i8<TB>(acc, a.w_qb + head0 * PD, a.w_qb + min(head0 + 1, a.n - 1) * PD, nd, a.q_norm, a.r, tok0, a.t, a.r / GT_KI8, lds);
+    uint8_t* had = lds;
+#pragma unroll
+    for (int i = 0; i < PD * PD * 2 / 16 / 512; ++i) reinterpret_cast<u32x4*>(had)[tid + 512 * i] = reinterpret_cast<const u32x4*>(a.had_q)[tid + 512 * i];
+    // register e of acc[nb][tb]: dim 64 (wc & 1) + 16 nb + 4 g + e of head wc / 2, token 16 TB wr + 16 tb + l16
+    {
+        uint8_t* xt = lds + PD * PD * 2 + (wc >> 1) * TOK * XROW;
+        f32x4 ws[4];
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb)
+            ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + (int64_t)min(head0 + (wc >> 1), a.n - 1) * PD + 64 * (wc & 1) + 16 * nb + 4 * g);
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {
+            const int tl = 16 * TB * wr + 16 * tb + l16;
+            const float qs = a.q_norm_scale[min(tok0 + tl, a.t - 1)];
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) {
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs) * ws[nb][e];
+                *reinterpret_cast<u32x2*>(xt + tl * XROW + (64 * (wc & 1) + 16 * nb + 4 * g) * 2) =
+                    u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+            }
+        }
+    }
+    __syncthreads();
+    const int hs = tid >> 8, ht = tid & 255, hwave = wave & 3, head = head0 + hs; // from here on four waves to a head
+    uint8_t* xt = lds + PD * PD * 2 + hs * TOK * XROW;
+    float(*smax)[TOK] = reinterpret_cast<float(*)[TOK]>(lds + PD * PD * 2 + 2 * TOK * XROW + hs * 4 * TOK * 4);
+    // rotary on the first 64 dims: 32 pairs a token (the arithmetic of rope_tile)
+#pragma unroll 4
+    for (int it = 0; it < TOK * 32 / 256; ++it) {
+        const int item = ht + 256 * it;
+        const int tok = item >> 5, i = item & 31;
+        uint16_t* row = reinterpret_cast<uint16_t*>(xt + tok * XROW);
+        const int64_t gtc = (int64_t)min(tok0 + tok, a.t - 1) * PROPE;
+        const uint16_t* cosp = a.cos + gtc;
+        const uint16_t* sinp = a.sin + gtc;
+        const float x1 = bf16_to_f32(row[i]), x2 = bf16_to_f32(row[i + 32]);
+        const float c1 = bf16_to_f32(cosp[i]), c2 = bf16_to_f32(cosp[i + 32]);
+        const float s1 = bf16_to_f32(sinp[i]), s2 = bf16_to_f32(sinp[i + 32]);
+        const float o1 = x1 * c1 + (-x2) * s1;
+        const float o2 = x2 * c2 + x1 * s2;
+        row[i] = f32_to_bf16(o1);
+        row[i + 32] = f32_to_bf16(o2);
+    }
+    __syncthreads();
+    // Y^T[n, token] = H^T[n, k] . X^T[k, token]: wave w of a head owns n in [32 w, 32 w + 32) for the blocks of 32 tokens
+    // (operand addressing as in prolog_q_body)
+    f32x16 y[TB];
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) y[tb][e] = 0.f;
+    {
+        const int jj = lane & 15, mh = (lane >> 4) & 1;
+        const uint8_t* hp = had + (4 * hl + (jj >> 2)) * (PD * 2) + (32 * hwave + 16 * mh + 4 * (jj & 3)) * 2;
+        const uint8_t* xp = xt + l32 * XROW + hl * 8;
+#pragma unroll
+        for (int ks = 0; ks < PD / 16; ++ks) {
+            const s16x4 lo = lds_read_tr(hp + ks * 16 * (PD * 2));
+            const s16x4 hi = lds_read_tr(hp + (ks * 16 + 8) * (PD * 2));
+            const bf16x8 av = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb) {
+                const u32x2 b0 = *reinterpret_cast<const u32x2*>(xp + 32 * tb * XROW + ks * 32);
+                const u32x2 b1 = *reinterpret_cast<const u32x2*>(xp + 32 * tb * XROW + ks * 32 + 16);
+                const bf16x8 bv = __builtin_bit_cast(bf16x8, u32x4{b0[0], b0[1], b1[0], b1[1]});
+                y[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, y[tb], 0, 0, 0);
+            }
+        }
+    }
+    // register e of y[tb]: n = 32 w + 8 (e/4) + 4 hl + e%4, token 32 tb + l32.  Round to bf16, per-token absmax over the 128 n
+    float mx[TB];
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) {
+        mx[tb] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            y[tb][e] = bf16_to_f32(f32_to_bf16(y[tb][e]));
+            mx[tb] = fmaxf(mx[tb], fabsf(y[tb][e]));
+        }
+        mx[tb] = fmaxf(mx[tb], __shfl_xor(mx[tb], 32));
+        if (hl == 0) smax[hwave][32 * tb + l32] = mx[tb];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) {
+        const int tl = 32 * tb + l32;
+        const float m = fmaxf(fmaxf(smax[0][tl], smax[1][tl]), fmaxf(smax[2][tl], smax[3][tl]));
+        const float sq = quant_scale(m);
+        const int gt = tok0 + tl;
+        if (gt < a.t && head < a.n) {
+            int8_t* qo = a.q_int8 + ((int64_t)gt * a.n + head) * PD + 32 * hwave + 4 * hl;
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) {
+                uint32_t pk = 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(y[tb][4 * e4 + e] * sq) & 0xffu) << (8 * e);
+                *reinterpret_cast<uint32_t*>(qo + 8 * e4) = pk;
+            }
+            if (hwave == 0 && hl == 0) a.q_scale[(int64_t)gt * a.n + head] = __builtin_bit_cast(uint16_t, (_Float16)(1.0f / sq));
         }
     }
 }

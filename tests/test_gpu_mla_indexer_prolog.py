@@ -154,6 +154,16 @@ def test_prefill_sizes_fused_equals_separate_and_oracle(cuda):
         check_against_oracle(mla_case, idx_case, fused)
 
 
+@pytest.mark.parametrize("t,n,r,h", [(1100, 2, 128, 512), (1290, 4, 256, 256), (1540, 2, 128, 256), (300, 6, 384, 2304)])
+def test_prefill_index_query_tiles(cuda, t, n, r, h):
+    """Index query tiles of 160, 192, 224 and 128 tokens: the product is exact and the rest the same operations, so the bits of
+    the separate call's 128-token tiles; the last also a contraction of three splits, the latent rank no multiple of 256."""
+    mla_case, idx_case = op.make_fused_case(t, 1, 64, seed=50 + n, n_idx=64, h=h, q_lora_rank=r, n=n)
+    fused = run_fused(mla_case, idx_case, cuda, entry="mla_indexer_prolog_quant_p")
+    same_as_separate(fused, run_separate(mla_case, idx_case, cuda), idx_case)
+    check_against_oracle(mla_case, idx_case, fused)
+
+
 def test_index_head_counts_without_the_side_by_side_kernels(cuda):
     # 32 index heads: x @ w_proj is half an output tile wide, so the fused entry runs the two operators back to back
     mla_case, idx_case = op.make_fused_case(5, 1, 300, seed=23, n_idx=32, h=512, q_lora_rank=256, n=4)

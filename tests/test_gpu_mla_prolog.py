@@ -226,6 +226,20 @@ def check_bf16_form(case, got, eps=EPS, outliers=0.0):
     assert torch.equal(got["q_norm_scale"], torch.zeros_like(got["q_norm_scale"]))
 
 
+@pytest.mark.parametrize("t,n", [(257, 2), (300, 128), (330, 128), (400, 128), (500, 128)])
+def test_prefill_query_tiles(cuda, t, n):
+    # tiles of 128, 160, 192, 224 and 256 tokens of the query product, each with a remainder; two heads: half a tile of outputs
+    case = op.make_case(t, 1, 64, seed=60 + t, h=256, q_lora_rank=128, n=n)
+    check(case, run(case, cuda, entry="mla_prolog_quant_p"))
+
+
+@pytest.mark.parametrize("t,n", [(33, 2), (128, 6), (129, 4), (300, 2)])
+def test_bf16_form_prefill_tiles(cuda, t, n):
+    # from 33 tokens on the query product owns 128 tokens x 256 outputs: remainders of both, chains of 256 rows
+    case = op.make_case(t, 1, 64, seed=70 + t, h=512, q_lora_rank=512, n=n, quant_b=False)
+    check_bf16_form(case, run(case, cuda))
+
+
 def test_bf16_form_reference_case_b4_s2(cuda):
     # the reference's test_b4_s64k2_pa_nd_bf16_d: no quantisation anywhere (empty dequant_scale, bf16 w_uq_qr and cache)
     case = op.make_case(4, 2, 1024, seed=18, quant_b=False)
