@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256) void apq_gemm_kernel(AttnPreArgs a)
     }
 }
 
-// The projection at prefill sizes (128 tokens and more): a workgroup owns 32 TB tokens x 256 outputs - two heads - over one
+// The projection at prefill sizes and larger decode batches (attention_pre_big): a workgroup owns 32 TB tokens x 256 outputs - two heads - over one
 // split of the contraction (gemm_tile.h; an odd last head is taken twice and dropped).  An XCD takes neighbouring heads.  Where one split covers the whole contraction the head's epilogue runs on the
 // tile: the sums never go to memory (777 tokens x 112 heads: 45 MB written and read again, and a kernel of 87 K small
 // workgroups).  Same operations in the same order as apq_head_kernel, so the same bits: its sum over the 128 squares is a
@@ -439,7 +439,10 @@ static int stages_per_split(int64_t t, int64_t h, int64_t n_out)
 
 // Prefill sizes: token blocks of the tile and stages of 128 rows per workgroup of apq_gemm_big_kernel, by the time they should
 // take in ns (gt_time_ns); partial sums are written, read again at 8 TB/s (the caches hold them) and cost the head kernel.
-constexpr int BIG_T = 128;
+// From 33 tokens on (a second token tile of apq_gemm_kernel: 14 heads 16.3 against 15.7 us a call, 64 tokens 19.5 / 18.1), and
+// from 9 where the weights are large (112 heads: 12 tokens 24.8 against 22.2 us, 24: 29.6 / 24.3, 100: 77 / 32; 28 heads and 12
+// tokens are the same, 14 heads 13.1 / 14.3).
+static bool attention_pre_big(int64_t t, int64_t n_out) { return t >= 33 || (t >= 9 && n_out >= 8192); }
 struct BigPlan { int tb, per; };
 static BigPlan big_plan(int64_t t, int64_t h, int64_t n_out)
 {
@@ -459,7 +462,7 @@ static BigPlan big_plan(int64_t t, int64_t h, int64_t n_out)
 
 int attention_pre_ksplits(int64_t t, int64_t h, int64_t n_out)
 {
-    if (t >= BIG_T) {
+    if (attention_pre_big(t, n_out)) {
         const int per = big_plan(t, h, n_out).per;
         return (int)((h / GT_KI8 + per - 1) / per);
     }
@@ -468,11 +471,11 @@ int attention_pre_ksplits(int64_t t, int64_t h, int64_t n_out)
 }
 
 // one split at prefill sizes: the projection's workgroups finish their heads themselves, no sums go through memory
-static bool attention_pre_whole(int64_t t, int ksplits) { return t >= BIG_T && ksplits == 1; }
+static bool attention_pre_whole(int64_t t, int64_t n_out, int ksplits) { return attention_pre_big(t, n_out) && ksplits == 1; }
 
 uint64_t attention_pre_workspace_bytes(int64_t t, int64_t h, int64_t n_out)
 {
-    if (attention_pre_whole(t, attention_pre_ksplits(t, h, n_out))) return align256((uint64_t)t * h);
+    if (attention_pre_whole(t, n_out, attention_pre_ksplits(t, h, n_out))) return align256((uint64_t)t * h);
     return align256((uint64_t)t * h) + (uint64_t)attention_pre_ksplits(t, h, n_out) * t * n_out * sizeof(int32_t);
 }
 
@@ -485,7 +488,7 @@ void attention_pre_bind_workspace(AttnPreArgs& a, void* ws)
 hipError_t attention_pre_launch(const AttnPreArgs& a, hipStream_t stream)
 {
     if (a.t == 0) return hipSuccess;
-    const bool whole = attention_pre_whole(a.t, a.ksplits);
+    const bool whole = attention_pre_whole(a.t, a.n_out, a.ksplits);
     hipError_t e;
     {
         ScopedKernelTimer tm(KID_APQ_NORM, stream);
@@ -500,8 +503,9 @@ hipError_t attention_pre_launch(const AttnPreArgs& a, hipStream_t stream)
         const dim3 grid(a.n_out / AD, a.ksplits, (a.t + ATOK - 1) / ATOK);
         const int per = stages_per_split(a.t, a.h, a.n_out);
         if (a.ksplits != attention_pre_ksplits(a.t, a.h, a.n_out)) return hipErrorInvalidValue;
-        const BigPlan big = a.t >= BIG_T ? big_plan(a.t, a.h, a.n_out) : BigPlan{};
-        if (a.t >= BIG_T)
+        const bool tiles = attention_pre_big(a.t, a.n_out);
+        const BigPlan big = tiles ? big_plan(a.t, a.h, a.n_out) : BigPlan{};
+        if (tiles)
             gt_dispatch(big.tb, [&](auto tb) {
                 constexpr int TB = decltype(tb)::value;
                 hipLaunchKernelGGL((whole ? apq_gemm_big_kernel<TB, true> : apq_gemm_big_kernel<TB, false>),

@@ -50,9 +50,11 @@ constexpr int MQROW = 136;         // bytes per LDS row of a [k][128] int8 weigh
 constexpr int QB_GROUPS = 4;      // wavefront quads of mla_qb_kernel, each with its own stages in flight
 constexpr int QB_MAXS = MAX_R / QB_K / QB_GROUPS; // stages per group at the largest q_lora_rank
 constexpr int QB_QP = MTOK * (MAX_R / 16) / 1024; // 16-byte pieces of the q_norm tile per lane at the largest q_lora_rank
-constexpr int BIG_T = 128;        // token count from which the kernels that own an output tile take over
-constexpr int BIG_T2 = 256;       // token count above which their tiles are 256 tokens tall
-constexpr int QB16_WIDE_T = 33;   // token count from which the bf16 form's q_b product runs per 128 tokens
+constexpr int BIG_T = 33;         // token count from which the kernels that own an output tile take over: the others read the
+                                  // weights once per 32 tokens (fused prolog, 33 tokens: 63.6 against 47.2 us, 96: 87 / 55, 127:
+                                  // 108 / 59; 24 tokens: 43.6 / 46.8)
+constexpr int BIG_T2 = 256;       // token count above which the tiles are 256 outputs wide (127 tokens: 59 against 87 us, 256: 83 /
+                                  // 94, 257: 106 / 94)
 
 // 32 outputs x 32 tokens += W[KSTEPS steps of 16 rows, outputs]^T . X[tokens, k]: A by transposing reads of the [k][n]
 // tile in LDS, rows of ROWB bytes.  Lane jj of a 16-lane group points at row 8 hl + jj / 4 (+ 4 for the second read) of
@@ -169,7 +171,7 @@ __global__ __launch_bounds__(1024) void mla_xa_kernel(MlaPrologArgs a)
     xa_body(a.x, a.h, a.h, src, ld, a.xa_part, a.ncols, blockIdx.y * 64, blockIdx.x, blockIdx.z * MTOK, a.t, xa_lds);
 }
 
-// The same product at prefill sizes (128 tokens and more): a workgroup owns an output tile of 128 tokens x 64 columns
+// The same product at 33 to 256 tokens: a workgroup owns an output tile of 128 tokens x 64 columns
 // over one 1024-row split of the contraction and walks it in stages of 64 rows, both operands staged through LDS, so
 // that the weights are read once per 128 tokens instead of once per 32 and a token row's piece is fetched by 8
 // neighbouring lanes as one 128-byte run.  The global loads of BG_DEPTH stages are in flight at any time (register
@@ -181,13 +183,11 @@ __global__ __launch_bounds__(1024) void mla_xa_kernel(MlaPrologArgs a)
 // as 128-byte runs.  grid (splits, output tiles of 64, token tiles), 256 lanes.
 constexpr int BG_KS = 64;               // contraction rows per stage
 constexpr int BG_XROW = BG_KS * 2 + 16; // bytes per LDS row of the [token][k] tile (padded against bank conflicts)
-// TB: blocks of 32 tokens per wave (the workgroup's tile is 128 TB tokens x 64 columns; with TB = 2 a weight fragment read
-// from LDS feeds two MFMAs and the weights are read half as often, which is what counts once the token count is large
-// enough for the kernel to be bound by what the CUs draw from the L2); DEPTH: stages whose loads are in flight.
-template <int TB, int DEPTH>
-__global__ __launch_bounds__(256, TB == 1 ? 3 : 2) void mla_xa_big_kernel(MlaPrologArgs a)
+// DEPTH: stages whose loads are in flight.  (Two workgroups to a CU: the grid has no more, and three leave too few registers.)
+template <int DEPTH>
+__global__ __launch_bounds__(256, 2) void mla_xa_big_kernel(MlaPrologArgs a)
 {
-    constexpr int TOK = 128 * TB;
+    constexpr int TOK = 128;
     static_assert((XA_SPLIT / BG_KS) % DEPTH == 0 && XA_K % (BG_KS * DEPTH) == 0, "whole rounds of stages in every split");
     __shared__ __align__(16) uint8_t wt[BG_KS * XROW2];
     __shared__ __align__(16) uint8_t xt[TOK * BG_XROW];
@@ -199,25 +199,23 @@ __global__ __launch_bounds__(256, TB == 1 ? 3 : 2) void mla_xa_big_kernel(MlaPro
     const int kbeg = split * XA_SPLIT;
     const int stages = (min(a.h, kbeg + XA_SPLIT) - kbeg) / BG_KS; // a multiple of DEPTH (h is one of 256)
     const int srow = tid >> 3, spc = tid & 7;
-    const uint16_t* xp[4 * TB];
+    const uint16_t* xp[4];
 #pragma unroll
-    for (int i = 0; i < 4 * TB; ++i) xp[i] = a.x + (int64_t)min(tok0 + srow + 32 * i, a.t - 1) * a.h + kbeg + 8 * spc;
+    for (int i = 0; i < 4; ++i) xp[i] = a.x + (int64_t)min(tok0 + srow + 32 * i, a.t - 1) * a.h + kbeg + 8 * spc;
     const uint16_t* wp = src + (int64_t)(kbeg + srow) * ld + 8 * spc;
-    u32x4 xs[DEPTH][4 * TB], ws[DEPTH][2];
+    u32x4 xs[DEPTH][4], ws[DEPTH][2];
     auto load = [&](int st, int u) {
 #pragma unroll
-        for (int i = 0; i < 4 * TB; ++i) xs[u][i] = *reinterpret_cast<const u32x4*>(xp[i] + st * BG_KS);
+        for (int i = 0; i < 4; ++i) xs[u][i] = *reinterpret_cast<const u32x4*>(xp[i] + st * BG_KS);
 #pragma unroll
         for (int i = 0; i < 2; ++i) ws[u][i] = *reinterpret_cast<const u32x4*>(wp + (int64_t)(st * BG_KS + 32 * i) * ld);
     };
-    f32x16 acc[TB][2];
+    f32x16 acc[2], sum[2]; // sums are chains of DEPTH stages, added up in order
 #pragma unroll
-    for (int tb = 0; tb < TB; ++tb)
+    for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[tb][nb][e] = 0.f;
-    const uint8_t* xr = xt + (32 * TB * wave + l32) * BG_XROW + 16 * hl;
+        for (int e = 0; e < 16; ++e) acc[nb][e] = sum[nb][e] = 0.f;
+    const uint8_t* xr = xt + (32 * wave + l32) * BG_XROW + 16 * hl;
     const uint8_t* hp = wt + (8 * hl + (jj >> 2)) * XROW2 + (16 * mh + 4 * (jj & 3)) * 2;
 #pragma unroll
     for (int u = 0; u < DEPTH; ++u) load(u, u);
@@ -226,16 +224,15 @@ __global__ __launch_bounds__(256, TB == 1 ? 3 : 2) void mla_xa_big_kernel(MlaPro
         for (int u = 0; u < DEPTH; ++u) {
             __syncthreads(); // everyone is done with the previous stage's tiles
 #pragma unroll
-            for (int i = 0; i < 4 * TB; ++i) *reinterpret_cast<u32x4*>(xt + (srow + 32 * i) * BG_XROW + 16 * spc) = xs[u][i];
+            for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(xt + (srow + 32 * i) * BG_XROW + 16 * spc) = xs[u][i];
 #pragma unroll
             for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(wt + (srow + 32 * i) * XROW2 + 16 * spc) = ws[u][i];
             __syncthreads();
             load(min(st0 + u + DEPTH, stages - 1), u); // (unconditional: past the end the last stage is fetched again and dropped)
 #pragma unroll
             for (int ks = 0; ks < BG_KS / 16; ++ks) {
-                bf16x8 xf[TB], wf[2];
-#pragma unroll
-                for (int tb = 0; tb < TB; ++tb) xf[tb] = *reinterpret_cast<const bf16x8*>(xr + 32 * tb * BG_XROW + ks * 32);
+                bf16x8 wf[2];
+                const bf16x8 xf = *reinterpret_cast<const bf16x8*>(xr + ks * 32);
 #pragma unroll
                 for (int nb = 0; nb < 2; ++nb) {
                     const s16x4 lo = lds_read_tr(hp + 64 * nb + ks * 16 * XROW2);
@@ -243,24 +240,26 @@ __global__ __launch_bounds__(256, TB == 1 ? 3 : 2) void mla_xa_big_kernel(MlaPro
                     wf[nb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
                 }
 #pragma unroll
-                for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-                    for (int nb = 0; nb < 2; ++nb)
-                        acc[tb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[tb], wf[nb], acc[tb][nb], 0, 0, 0);
+                for (int nb = 0; nb < 2; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, wf[nb], acc[nb], 0, 0, 0);
             }
         }
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                sum[nb][e] += acc[nb][e];
+                acc[nb][e] = 0.f;
+            }
     }
-    // register e of acc[tb][nb]: token 32 TB w + 32 tb + 8 (e / 4) + 4 hl + e % 4, column 32 nb + lane % 32
+    // register e of sum[nb]: token 32 w + 8 (e / 4) + 4 hl + e % 4, column 32 nb + lane % 32
 #pragma unroll
-    for (int tb = 0; tb < TB; ++tb)
+    for (int e = 0; e < 16; ++e) {
+        const int gt = tok0 + 32 * wave + 8 * (e >> 2) + 4 * hl + (e & 3);
+        if (gt >= a.t) continue;
+        float* out = a.xa_part + ((int64_t)split * a.t + gt) * a.ncols + col0 + l32;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int gt = tok0 + 32 * TB * wave + 32 * tb + 8 * (e >> 2) + 4 * hl + (e & 3);
-            if (gt >= a.t) continue;
-            float* out = a.xa_part + ((int64_t)split * a.t + gt) * a.ncols + col0 + l32;
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb) out[32 * nb] = acc[tb][nb][e];
-        }
+        for (int nb = 0; nb < 2; ++nb) out[32 * nb] = sum[nb][e];
+    }
 }
 
 // Above 256 tokens the workgroup owns 128 tokens x 256 outputs (gemm_tile.h) over one split of the contraction, a multiple of
@@ -1083,7 +1082,7 @@ uint64_t mla_prolog_workspace_bytes(int64_t t, int64_t h, int64_t r, int64_t n, 
 {
     // bf16 form: also the partial sums of q_norm @ w_uq_qr
     return xa_part_bytes(t, h, r + MKV + (n_idx ? PD + n_idx : 0)) + up256((uint64_t)t * n * MNOPE * 2) +
-           (quant || t >= QB16_WIDE_T ? 0 : xa_part_bytes(t, r, n * MQH));
+           (quant || t >= BIG_T ? 0 : xa_part_bytes(t, r, n * MQH));
 }
 
 void mla_prolog_bind_workspace(MlaPrologArgs& a, void* ws)
@@ -1146,7 +1145,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         ScopedKernelTimer tm(KID_MLA_XA, stream);
         if (big)
             if (a.t <= BIG_T2)
-                hipLaunchKernelGGL((mla_xa_big_kernel<1, 4>), dim3(a.ksplits, a.ncols / 64, (a.t + 127) / 128), dim3(256), 0, stream, a);
+                hipLaunchKernelGGL(mla_xa_big_kernel<4>, dim3(a.ksplits, a.ncols / 64, (a.t + 127) / 128), dim3(256), 0, stream, a);
             else {
                 const int xtiles = (a.t + 127) / 128, ntiles = (a.ncols + 255) / 256, rows = xa_wide_rows(a.t, a.h, a.r);
                 if (a.ksplits != (a.h + rows - 1) / rows) return hipErrorInvalidValue;
@@ -1167,7 +1166,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
     if ((e = hipGetLastError()) != hipSuccess) return e;
     {
         ScopedKernelTimer tm(KID_MLA_QB, stream);
-        if (!a.quant && a.t >= QB16_WIDE_T) {
+        if (!a.quant && big) {
             hipLaunchKernelGGL(mla_qb16_wide_kernel, dim3((a.n * MQH + 255) / 256, (a.t + 127) / 128), dim3(GT_LANES), 0, stream, a);
         } else if (!a.quant) {
             const int nq = a.n * MQH;

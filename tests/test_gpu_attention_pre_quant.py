@@ -155,7 +155,7 @@ def test_whole_model_heads(cuda):
 
 
 @pytest.mark.parametrize("t,q_heads,kv_heads,half", [(128, 3, 1, 20), (129, 2, 1, 64), (1300, 48, 2, 32), (1500, 48, 2, 8), (1800, 48, 2, 1),
-                                                     (2100, 47, 2, 32)])
+                                                     (2100, 47, 2, 32), (9, 62, 1, 32), (31, 60, 3, 32)])
 def test_prefill_in_one_split(cuda, t, q_heads, kv_heads, half):
     """One split over the contraction (short here): the projection's workgroups finish their heads themselves.  Tiles of 128,
     160, 192, 224 and 256 tokens with a remainder, an odd number of heads, rotary halves of whole and of broken pieces."""
