@@ -183,9 +183,12 @@ __global__ __launch_bounds__(1024) void mla_xa_kernel(MlaPrologArgs a)
 // as 128-byte runs.  grid (splits, output tiles of 64, token tiles), 256 lanes.
 constexpr int BG_KS = 64;               // contraction rows per stage
 constexpr int BG_XROW = BG_KS * 2 + 16; // bytes per LDS row of the [token][k] tile (padded against bank conflicts)
-// DEPTH: stages whose loads are in flight.  (Two workgroups to a CU: the grid has no more, and three leave too few registers.)
-template <int DEPTH>
-__global__ __launch_bounds__(256, 2) void mla_xa_big_kernel(MlaPrologArgs a)
+// DEPTH: stages whose loads are in flight.  CHAINS: sums are chains of 128 rows added up in order, which are mla_xa_kernel's
+// sums bit for bit (a decode step's selection can hang on the last bit of a score, so batches that cross the kernels' border
+// see the same numbers); otherwise one chain of a split's rows.  (With chains two workgroups to a CU: the grid has no more
+// below 128 tokens, and three leave too few registers.)
+template <int DEPTH, bool CHAINS>
+__global__ __launch_bounds__(256, CHAINS ? 2 : 3) void mla_xa_big_kernel(MlaPrologArgs a)
 {
     constexpr int TOK = 128;
     static_assert((XA_SPLIT / BG_KS) % DEPTH == 0 && XA_K % (BG_KS * DEPTH) == 0, "whole rounds of stages in every split");
@@ -210,7 +213,7 @@ __global__ __launch_bounds__(256, 2) void mla_xa_big_kernel(MlaPrologArgs a)
 #pragma unroll
         for (int i = 0; i < 2; ++i) ws[u][i] = *reinterpret_cast<const u32x4*>(wp + (int64_t)(st * BG_KS + 32 * i) * ld);
     };
-    f32x16 acc[2], sum[2]; // sums are chains of DEPTH stages, added up in order
+    f32x16 acc[2], sum[2];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
@@ -242,15 +245,20 @@ __global__ __launch_bounds__(256, 2) void mla_xa_big_kernel(MlaPrologArgs a)
 #pragma unroll
                 for (int nb = 0; nb < 2; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, wf[nb], acc[nb], 0, 0, 0);
             }
-        }
+            if constexpr (CHAINS) {
+                if (u % (128 / BG_KS) == 128 / BG_KS - 1) {
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
+                    for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                sum[nb][e] += acc[nb][e];
-                acc[nb][e] = 0.f;
+                        for (int e = 0; e < 16; ++e) {
+                            sum[nb][e] += acc[nb][e];
+                            acc[nb][e] = 0.f;
+                        }
+                }
             }
+        }
     }
+    if constexpr (!CHAINS) sum[0] = acc[0], sum[1] = acc[1];
     // register e of sum[nb]: token 32 w + 8 (e / 4) + 4 hl + e % 4, column 32 nb + lane % 32
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
@@ -1145,7 +1153,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         ScopedKernelTimer tm(KID_MLA_XA, stream);
         if (big)
             if (a.t <= BIG_T2)
-                hipLaunchKernelGGL(mla_xa_big_kernel<4>, dim3(a.ksplits, a.ncols / 64, (a.t + 127) / 128), dim3(256), 0, stream, a);
+                hipLaunchKernelGGL((a.t < 128 ? mla_xa_big_kernel<4, true> : mla_xa_big_kernel<4, false>), dim3(a.ksplits, a.ncols / 64, (a.t + 127) / 128), dim3(256), 0, stream, a);
             else {
                 const int xtiles = (a.t + 127) / 128, ntiles = (a.ncols + 255) / 256, rows = xa_wide_rows(a.t, a.h, a.r);
                 if (a.ksplits != (a.h + rows - 1) / rows) return hipErrorInvalidValue;
