@@ -630,7 +630,6 @@ int plan_mla_prolog(const PtoTensorDesc* ts, uint32_t n, const PtoMlaPrologParam
     a.w_dq = static_cast<const uint16_t*>(ts[1].addr);
     a.w_uq_qr = ts[2].addr;
     a.quant = quant;
-    a.qb_part = nullptr;
     a.w_qb_scale = static_cast<const float*>(ts[3].addr);
     a.w_uk = static_cast<const uint16_t*>(ts[4].addr);
     a.w_dkv_kr = static_cast<const uint16_t*>(ts[5].addr);
@@ -660,7 +659,7 @@ int plan_mla_prolog(const PtoTensorDesc* ts, uint32_t n, const PtoMlaPrologParam
     a.ksplits = (int32_t)((h + 1023) / 1024);
     a.eps_cq = p->epsilon_cq;
     a.eps_ckv = p->epsilon_ckv;
-    plan->ws_bytes = pto::mla_prolog_workspace_bytes(t, h, r, nh, 0, quant);
+    plan->ws_bytes = pto::mla_prolog_workspace_bytes(t, h, r, nh, 0);
     return PTO_OK;
 }
 
@@ -723,7 +722,7 @@ int plan_fused_prolog(const PtoTensorDesc* ts, uint32_t n, const PtoMlaIndexerPr
     if (rc) return rc;
     plan->fused = pto::fused_prolog_supported(plan->ip.args.n);
     if (plan->fused) { // the indexer's partial sums live inside the MLA prolog's: no workspace of its own
-        plan->mla.ws_bytes = pto::mla_prolog_workspace_bytes(t, plan->mla.args.h, r, plan->mla.args.n, plan->ip.args.n, true);
+        plan->mla.ws_bytes = pto::mla_prolog_workspace_bytes(t, plan->mla.args.h, r, plan->mla.args.n, plan->ip.args.n);
         plan->ip.ws_bytes = 0;
     }
     plan->off_ip_ws = up256(plan->mla.ws_bytes);

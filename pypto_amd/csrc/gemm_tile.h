@@ -54,8 +54,8 @@ __device__ __forceinline__ void gt_copy(const void* base, uint32_t offset, uint8
 template <int N>
 __device__ __forceinline__ void gt_landed()
 {
-    static_assert(N < 16, "the counter's low bits");
-    __builtin_amdgcn_s_waitcnt(0x0f70 | N); // vmcnt(N)
+    static_assert(N < 64, "the counter's six bits");
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | (N >> 4 << 14)); // vmcnt(N)
     __syncthreads();
 }
 

@@ -170,7 +170,6 @@ struct MlaPrologArgs {
     const uint16_t* w_proj;     // products with x ride along in the first kernel
     float* xa_part;             // workspace [ksplits, t, ncols]
     uint16_t* qb_nope;          // workspace [t, n, 128] bf16
-    float* qb_part;             // workspace, bf16 form only: [ceil(r / 1024), t, n*192] partial sums of q_norm @ w_uq_qr
     int64_t cache_rows;
     int32_t t, h, r, n, ksplits;
     int32_t n_idx, ncols;       // index heads (0: not fused); columns of a partial-sum row: r + 576 (+ 128 + n_idx)
@@ -179,7 +178,7 @@ struct MlaPrologArgs {
 };
 
 bool mla_prolog_supported(int64_t h, int64_t r, int64_t n, int64_t d_nope, int64_t d_rope, int64_t c);
-uint64_t mla_prolog_workspace_bytes(int64_t t, int64_t h, int64_t r, int64_t n, int64_t n_idx, bool quant);
+uint64_t mla_prolog_workspace_bytes(int64_t t, int64_t h, int64_t r, int64_t n, int64_t n_idx);
 void mla_prolog_bind_workspace(MlaPrologArgs& a, void* workspace);
 hipError_t mla_prolog_launch(const MlaPrologArgs& a, hipStream_t stream);
 // The fused MLA + indexer prolog as four launches (needs n_idx a multiple of 64); fused_prolog_bind points the indexer's

@@ -314,52 +314,9 @@ static int xa_wide_rows(int64_t t, int64_t h, int64_t r)
     return (int)((h / XA_K + splits - 1) / splits) * XA_K;
 }
 
-// bf16 form of the operator: q_b = q_norm (bf16 [t, r]) @ w_uq_qr (bf16 [r, n * 192]) with the same kernel body;
-// grid (ceil(r / 1024), n * 192 / 64, token tiles of 32); partial sums to qb_part
-__global__ __launch_bounds__(1024) void mla_qb16_kernel(MlaPrologArgs a)
-{
-    extern __shared__ __align__(16) uint8_t xa_lds[];
-    const int nq = a.n * MQH;
-    xa_body(reinterpret_cast<const uint16_t*>(a.q_norm), a.r, a.r, reinterpret_cast<const uint16_t*>(a.w_uq_qr) + blockIdx.y * 64,
-            nq, a.qb_part, nq, blockIdx.y * 64, blockIdx.x, blockIdx.z * MTOK, a.t, xa_lds);
-}
-
-// bf16 form: q_b = bf16(sum of the partial sums); its first 128 dims of a head to qb_nope, the last 64 through the rotary
-// embedding to q_rope.  grid (tokens, n * 192 / 1024 rounded up), 256 lanes: four columns (two pairs) per lane
-__global__ __launch_bounds__(256) void mla_qb16_epilogue_kernel(MlaPrologArgs a)
-{
-#pragma clang fp contract(off)
-    const int tok = blockIdx.x, col = (blockIdx.y * 256 + threadIdx.x) * 4;
-    const int nq = a.n * MQH, splits = (a.r + XA_SPLIT - 1) / XA_SPLIT;
-    if (col >= nq) return;
-    f32x4 acc = *reinterpret_cast<const f32x4*>(a.qb_part + (int64_t)tok * nq + col);
-    for (int sp = 1; sp < splits; ++sp) acc += *reinterpret_cast<const f32x4*>(a.qb_part + ((int64_t)sp * a.t + tok) * nq + col);
-    uint16_t vb[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) vb[e] = f32_to_bf16(acc[e]);
-    const int head = col / MQH, d = col % MQH;
-    if (d < MNOPE) {
-        const u32x2 pk = {(uint32_t)vb[0] | ((uint32_t)vb[1] << 16), (uint32_t)vb[2] | ((uint32_t)vb[3] << 16)};
-        *reinterpret_cast<u32x2*>(a.qb_nope + ((int64_t)tok * a.n + head) * MNOPE + d) = pk;
-    } else {
-        const uint16_t* cp = a.cos + (int64_t)tok * MROPE;
-        const uint16_t* snp = a.sin + (int64_t)tok * MROPE;
-        uint16_t* out = a.q_rope + ((int64_t)tok * a.n + head) * MROPE;
-#pragma unroll
-        for (int pr = 0; pr < 2; ++pr) {
-            const int i = (d - MNOPE) / 2 + pr;
-            const float xe = bf16_to_f32(vb[2 * pr]), xo = bf16_to_f32(vb[2 * pr + 1]);
-            const float o1 = xe * bf16_to_f32(cp[i]) + (-xo) * bf16_to_f32(snp[i]);
-            const float o2 = xo * bf16_to_f32(cp[i + 32]) + xe * bf16_to_f32(snp[i + 32]);
-            out[i] = f32_to_bf16(o1);
-            out[i + 32] = f32_to_bf16(o2);
-        }
-    }
-}
-
 // Four blocks of 64 outputs of q_b, TOK tokens each, from LDS rows of QBS_ROW bytes (padded against bank conflicts) to memory in
-// 16-byte pieces: a block is half of a head's 128 first dims, or its rotary dims, rotated on the way.  512 lanes, two waves to a
-// block.
+// 16-byte pieces: a block is half of a head's 128 first dims, or its rotary dims, rotated on the way.  Two waves to a block (two
+// blocks: 256 lanes).
 constexpr int QBS_ROW = 64 * 2 + 16;
 template <int TOK>
 __device__ __forceinline__ void qb_store_blocks(const MlaPrologArgs& a, const uint8_t* lds, int block0, int tok0)
@@ -412,9 +369,77 @@ __device__ __forceinline__ void qb_store_blocks(const MlaPrologArgs& a, const ui
     }
 }
 
+// bf16 form of the operator, up to 32 tokens: q_b = q_norm (bf16 [t, r]) @ w_uq_qr (bf16 [r, n * 192]), a stream of 75 MB of
+// weights.  A workgroup owns 128 outputs (192 of them at model sizes) and keeps six stages of 64 rows x 256 bytes in flight
+// straight to LDS.  Splits of 1024 rows loaded in one go through registers, their fp32 partial sums through memory and a kernel
+// behind them took 24.4 + 4.8 us at 24 tokens.  The sums: chains of 128 rows added up in order, then splits of 1024 rows.
+// grid (n * 192 / 128 rounded up), 256 lanes: wave w owns outputs [32 w, +32).
+__global__ __launch_bounds__(256) void mla_qb16_kernel(MlaPrologArgs a)
+{
+#pragma clang fp contract(off)
+    constexpr int XB = MTOK * 128, STAGE = XB + 2 * 64 * 128, RING = 7; // a stage: token rows | [2] weight rows of 128 bytes
+    static_assert(2 * MTOK * QBS_ROW <= RING * STAGE, "the output tile takes the stages' place");
+    __shared__ __align__(16) uint8_t lds[RING * STAGE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, hl = lane >> 5, jj = lane & 15, mh = (lane >> 4) & 1;
+    const int nq = a.n * MQH, block0 = 2 * blockIdx.x;
+    const uint16_t* x = reinterpret_cast<const uint16_t*>(a.q_norm);
+    const uint16_t* src[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) // (a block past the last one: that one again, dropped below)
+        src[i] = static_cast<const uint16_t*>(a.w_uq_qr) + min(block0 + i, nq / 64 - 1) * 64;
+    // copies of a wave (layout and exchange of the pieces: gemm_tile.h): token rows 8 w + lane / 8, weight rows 32 i + that
+    const int row = 8 * wave + (lane >> 3), pos = lane & 7;
+    const uint32_t xo = (uint32_t)(min(row, a.t - 1) * a.r * 2 + 16 * (pos ^ ((row >> 1) & 7)));
+    uint32_t wo[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) wo[i] = (uint32_t)((row + 32 * i) * nq * 2 + 16 * (pos ^ ((row << 1) & 4)));
+    const uint8_t* xr = lds + l32 * 128;
+    const int xf = (l32 >> 1) & 7;
+    const uint8_t* wrow = lds + XB + (wave >> 1) * 8192 + (8 * hl + (jj >> 2)) * 128 + 8 * (jj & 1);
+    const int wpos = 16 * ((4 * (wave & 1) + 2 * mh + ((jj >> 1) & 1)) ^ ((jj >> 1) & 4));
+    f32x16 acc, part, sum;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = part[e] = sum[e] = 0.f;
+    const int stages = a.r / 64;
+    gt_stages<RING, STAGE, 5>(
+        stages,
+        [&](int st, int b) {
+            uint8_t* d = lds + b + 1024 * wave;
+            gt_copy(x + st * 64, xo, d);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) gt_copy(src[i >> 1] + (int64_t)st * 64 * nq, wo[i & 1], d + XB + 4096 * i);
+        },
+        [&](int st, int b) {
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                const uint8_t* p = wrow + b + 2048 * ks + wpos;
+                const s16x4 lo = lds_read_tr(p), hi = lds_read_tr(p + 512);
+                const bf16x8 wv = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                const bf16x8 xv = *reinterpret_cast<const bf16x8*>(xr + b + 16 * ((2 * ks + hl) ^ xf));
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv, xv, acc, 0, 0, 0);
+            }
+            const bool last = st + 1 == stages;
+            if (st % 2 == 1 || last) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) part[e] += acc[e], acc[e] = 0.f;
+            }
+            if ((st + 1) % (XA_SPLIT / 64) == 0 || last) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) sum[e] += part[e], part[e] = 0.f;
+            }
+        });
+    // register e: output 32 w + 8 (e / 4) + 4 hl + e % 4, token lane % 32
+#pragma unroll
+    for (int e4 = 0; e4 < 4; ++e4)
+        *reinterpret_cast<u32x2*>(lds + ((wave >> 1) * MTOK + l32) * QBS_ROW + (32 * (wave & 1) + 8 * e4 + 4 * hl) * 2) =
+            u32x2{pack_bf16x2(sum[4 * e4], sum[4 * e4 + 1]), pack_bf16x2(sum[4 * e4 + 2], sum[4 * e4 + 3])};
+    __syncthreads();
+    qb_store_blocks<MTOK>(a, lds, block0, 0);
+}
+
 // The bf16 form at more tokens: 128 tokens x 256 outputs per workgroup over the whole contraction (gemm_tile.h), the epilogue
-// on the tile.  The pair above reads the weights once per 32 tokens and hands fp32 partial sums through memory: 811 us at
-// 1000 tokens.  grid (n * 192 / 256 rounded up, token tiles of 128), 512 lanes.
+// on the tile: 86 us at 1024 tokens, where a kernel that read the weights once per 32 tokens took 811.  grid (n * 192 / 256 rounded up, token tiles of 128), 512 lanes.
 __global__ __launch_bounds__(GT_LANES, 2) void mla_qb16_wide_kernel(MlaPrologArgs a)
 {
 #pragma clang fp contract(off)
@@ -1086,11 +1111,9 @@ static uint64_t xa_part_bytes(int64_t t, int64_t h, int64_t ncols)
     return up256((uint64_t)((h + XA_SPLIT - 1) / XA_SPLIT) * t * ncols * sizeof(float));
 }
 
-uint64_t mla_prolog_workspace_bytes(int64_t t, int64_t h, int64_t r, int64_t n, int64_t n_idx, bool quant)
+uint64_t mla_prolog_workspace_bytes(int64_t t, int64_t h, int64_t r, int64_t n, int64_t n_idx)
 {
-    // bf16 form: also the partial sums of q_norm @ w_uq_qr
-    return xa_part_bytes(t, h, r + MKV + (n_idx ? PD + n_idx : 0)) + up256((uint64_t)t * n * MNOPE * 2) +
-           (quant || t >= BIG_T ? 0 : xa_part_bytes(t, r, n * MQH));
+    return xa_part_bytes(t, h, r + MKV + (n_idx ? PD + n_idx : 0)) + up256((uint64_t)t * n * MNOPE * 2);
 }
 
 void mla_prolog_bind_workspace(MlaPrologArgs& a, void* ws)
@@ -1103,8 +1126,6 @@ void mla_prolog_bind_workspace(MlaPrologArgs& a, void* ws)
     a.xa_part = reinterpret_cast<float*>(p);
     p += xa_part_bytes(a.t, a.h, a.ncols);
     a.qb_nope = reinterpret_cast<uint16_t*>(p);
-    p += up256((uint64_t)a.t * a.n * MNOPE * 2);
-    a.qb_part = reinterpret_cast<float*>(p);
 }
 
 bool fused_prolog_supported(int64_t n_idx) { return n_idx % 64 == 0; }
@@ -1131,9 +1152,6 @@ static hipError_t set_lds_limits()
         if (e != hipSuccess) return e;
         e = hipFuncSetAttribute(reinterpret_cast<const void*>(mla_qb_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 mla_qb_lds_bytes(MAX_R));
-        if (e != hipSuccess) return e;
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(mla_qb16_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                4 * XA_K * XROW2);
         if (e != hipSuccess) return e;
         e = hipFuncSetAttribute(reinterpret_cast<const void*>(fused_qb_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 mla_qb_lds_bytes(MAX_R) > prolog_q_lds_bytes(QMAX_R) ? mla_qb_lds_bytes(MAX_R) : prolog_q_lds_bytes(QMAX_R));
@@ -1177,10 +1195,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         if (!a.quant && big) {
             hipLaunchKernelGGL(mla_qb16_wide_kernel, dim3((a.n * MQH + 255) / 256, (a.t + 127) / 128), dim3(GT_LANES), 0, stream, a);
         } else if (!a.quant) {
-            const int nq = a.n * MQH;
-            hipLaunchKernelGGL(mla_qb16_kernel, dim3((a.r + XA_SPLIT - 1) / XA_SPLIT, nq / 64, ttiles), dim3(1024),
-                               4 * XA_K * XROW2, stream, a);
-            hipLaunchKernelGGL(mla_qb16_epilogue_kernel, dim3(a.t, (nq / 4 + 255) / 256), dim3(256), 0, stream, a);
+            hipLaunchKernelGGL(mla_qb16_kernel, dim3((a.n * MQH + 127) / 128), dim3(256), 0, stream, a);
         } else if (big) {
             const dim3 qgrid(a.n * MQH / 128, (a.t + QG_TOK - 1) / QG_TOK);
             if (p && a.t <= BIG_T2) {
