@@ -139,6 +139,56 @@ __device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t*
     });
 }
 
+// Up to 32 tokens x 128 outputs, 256 lanes: a stream of weights, five stages of 128 rows in flight straight to LDS.  Wave w owns
+// outputs [32 w, +32).  Register e of acc[nb][tb]: output 32 w + 16 nb + 4 g + e, token 16 tb + l16.
+struct GtStream {
+    static constexpr int TOK = 32, QBYTES = TOK * 128, STAGE = QBYTES + 128 * 128, RING = 6, LDS = RING * STAGE;
+};
+__device__ __forceinline__ void gt_stream_i8(i32x4 (&acc)[2][2], const int8_t* w, int64_t ldw, const int8_t* q, int64_t ldq, int t,
+                                             int stages, uint8_t* lds)
+{
+    using T = GtStream;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, g = lane >> 4;
+    // copies of a wave: token rows 8 w + lane / 8; weight rows 32 i + that
+    const int row = 8 * wave + (lane >> 3), pos = lane & 7;
+    const uint32_t qo = (uint32_t)(min(row, t - 1) * (int)ldq + 16 * (pos ^ ((row >> 1) & 7)));
+    uint32_t wo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wo[i] = (uint32_t)((row + 32 * i) * (int)ldw + 16 * (pos ^ (((row >> 1) & 3) | ((row >> 2) & 4))));
+    const uint8_t* qr = lds + l16 * 128;
+    const int qpos = 16 * (g ^ ((l16 >> 1) & 7));
+    const uint8_t* wrow = lds + T::QBYTES + (16 * g + (l16 >> 1)) * 128 + 8 * (l16 & 1);
+    const int wf0 = ((l16 >> 2) & 3) | ((g & 1) << 2); // (transposing reads: see gt_product_i8)
+    gt_stages<T::RING, T::STAGE, 5>(
+        stages,
+        [&](int st, int b) {
+            uint8_t* d = lds + b + 1024 * wave;
+            gt_copy(q + st * GT_KI8, qo, d);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) gt_copy(w + (int64_t)st * GT_KI8 * ldw, wo[i], d + T::QBYTES + 4096 * i);
+        },
+        [&](int, int b) {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                i32x4 qf[2], wf[2];
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) qf[tb] = *reinterpret_cast<const i32x4*>(qr + b + 2048 * tb + (qpos ^ (64 * ks)));
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) {
+                    const uint8_t* p = wrow + b + 8192 * ks + 16 * ((2 * wave + nb) ^ wf0);
+                    const v2i lo = lds_read_tr8(p), hi = lds_read_tr8(p + 1024);
+                    wf[nb] = i32x4{lo[0], lo[1], hi[0], hi[1]};
+                }
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                    for (int tb = 0; tb < 2; ++tb)
+                        acc[nb][tb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[nb], qf[tb], acc[nb][tb], 0, 0, 0);
+            }
+        });
+}
+
 // The same loop in bf16 for 128 tokens x 256 outputs, the outputs in four blocks of 64 columns at src[i], ld[i] values a row;
 // x: [t, ldx], column of the first contraction row.  Wave (wr, wc) owns tokens [64 wr, +64) x block wc.  Register e of
 // sum[tb][nb]: token 64 wr + 32 tb + 8 (e / 4) + 4 hl + e % 4, column 32 nb + lane % 32 of the block.  Sums are chains of at most

@@ -20,8 +20,8 @@
 //   mla_xa_kernel    x @ [w_dq | w_dkv_kr], 256 contraction rows x 128 outputs per workgroup, fp32 partials
 //   mla_norm_kernel  one workgroup per token: fixed-order sum of the partials, both RmsNorms, the quantisations, the
 //                    key's rotary embedding, the three cache writes, q_norm / q_norm_scale
-//   mla_qb_kernel    int8 MFMA GEMM q_norm @ w_uq_qr, 128 outputs x 32 tokens per workgroup, weights double-buffered
-//                    through LDS; dequantisation and the query's rotary embedding in registers
+//   mla_qb_kernel    int8 MFMA GEMM q_norm @ w_uq_qr, 128 outputs x 32 tokens per workgroup, weights streamed to LDS
+//                    (gemm_tile.h); dequantisation and the query's rotary embedding on the tile
 //   mla_wuk_kernel   per (head, 128 outputs): q_b[:, head, :128] @ w_uk[head]
 #include <hip/hip_runtime.h>
 
@@ -40,16 +40,12 @@ namespace {
 
 constexpr int MTOK = 32;          // tokens per workgroup tile
 constexpr int MNOPE = 128, MROPE = 64, MQH = MNOPE + MROPE, MC = 512, MKV = MC + MROPE;
-constexpr int MAX_R = 2048;       // largest q_lora_rank (LDS of mla_norm_kernel, registers of mla_qb_kernel)
+constexpr int MAX_R = 2048;       // largest q_lora_rank (LDS of mla_norm_kernel)
 constexpr int XA_K = 256;         // contraction rows per stage of mla_xa_kernel
 constexpr int XA_SPLIT = 1024;    // contraction rows per workgroup of mla_xa_kernel (one fp32 partial sum each)
 constexpr int XROW2 = 64 * 2 + 16; // bytes per LDS row of a [k][64] bf16 weight tile (padded against bank conflicts)
 constexpr int TROW = 128 * 2 + 32; // bytes per LDS row of a [k][128] bf16 weight tile (padded against bank conflicts)
-constexpr int QB_K = 128;         // contraction rows per stage of mla_qb_kernel
 constexpr int MQROW = 136;         // bytes per LDS row of a [k][128] int8 weight tile (padded, 8-byte aligned)
-constexpr int QB_GROUPS = 4;      // wavefront quads of mla_qb_kernel, each with its own stages in flight
-constexpr int QB_MAXS = MAX_R / QB_K / QB_GROUPS; // stages per group at the largest q_lora_rank
-constexpr int QB_QP = MTOK * (MAX_R / 16) / 1024; // 16-byte pieces of the q_norm tile per lane at the largest q_lora_rank
 constexpr int BIG_T = 33;         // token count from which the kernels that own an output tile take over: the others read the
                                   // weights once per 32 tokens (fused prolog, 33 tokens: 63.6 against 47.2 us, 96: 87 / 55, 127:
                                   // 108 / 59; 24 tokens: 43.6 / 46.8)
@@ -610,172 +606,49 @@ __device__ __forceinline__ void mla_norm_body(const MlaPrologArgs& a, int tok)
 }
 
 // ------------------------------------------------------------------------------------------------ q_norm @ w_uq_qr
-// grid (n * 192 / 128, token tiles of 32), 1024 lanes = 4 groups of 4 wavefronts.  Group g takes the contraction stages
-// g, g + 4, ... (128 rows x 128 outputs each) and issues the loads of all of them at once (registers), so that the
-// whole tile of weights is in flight together; a stage then goes through the group's LDS buffer to be read back byte-
-// transposed.  The token tile of q_norm sits in LDS (loaded ahead of the weights: memory operations complete in
-// order).  Within a group wave w owns outputs [32 w, 32 w + 32) of the tile.  The groups' int32 sums are added through LDS
-// at the end (exact, so the result does not depend on the split).
-__host__ __device__ constexpr int mla_qb_lds_bytes(int r)
-{
-    return QB_GROUPS * QB_K * MQROW + MTOK * (r + 16) + 2 * MTOK * MROPE * 2;
-}
-// qb_lds: [QB_GROUPS][QB_K * MQROW] weights | [32][r + 16] q_norm | [2][32][64] cos, sin
-__device__ __forceinline__ void mla_qb_body(const MlaPrologArgs& a, int col0, int tok0, uint8_t* qb_lds)
+// Up to 32 tokens: 128 outputs per workgroup of 256 lanes behind the streamed product (gemm_tile.h); dequantisation and the
+// query's rotary embedding on the tile.  The int32 sums are exact.
+__device__ __forceinline__ void mla_qb_body(const MlaPrologArgs& a, int tile, uint8_t* lds)
 {
 #pragma clang fp contract(off)
-    const int tid = threadIdx.x & 255, grp = threadIdx.x >> 8, lane = tid & 63, wave = tid >> 6;
-    const int l16 = lane & 15, g = lane >> 4;
-    const int r = a.r, qrowb = r + 16; // padded against bank conflicts (r is a multiple of 128)
-    const int64_t nq = (int64_t)a.n * MQH;
-    uint8_t* wl = qb_lds + grp * (QB_K * MQROW);
-    uint8_t* ql = qb_lds + QB_GROUPS * (QB_K * MQROW);
-    uint16_t* csl = reinterpret_cast<uint16_t*>(ql + MTOK * qrowb); // [2][32][64]: the token tile's cos and sin rows
-
-    // q_norm tile: 32 rows of r bytes, 16-byte pieces over the 1024 lanes (at most QB_QP per lane)
-    const int qpieces = MTOK * (r / 16);
-    u32x4 qst[QB_QP];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4, col0 = 128 * tile;
+    float qs[2];
+    f32x4 ws[2];
 #pragma unroll
-    for (int i = 0; i < QB_QP; ++i) {
-        const int pc = min((int)threadIdx.x + 1024 * i, qpieces - 1);
-        const int row = pc / (r / 16), c = pc % (r / 16);
-        qst[i] = *reinterpret_cast<const u32x4*>(a.q_norm + (int64_t)min(tok0 + row, a.t - 1) * r + 16 * c);
-    }
-    // the token tile's cos / sin rows and scales for the epilogue: loaded now, so that the epilogue waits for nothing
-    u32x4 cst = {0u, 0u, 0u, 0u};
-    if (threadIdx.x < 512) {
-        const int which = threadIdx.x >> 8, row = (threadIdx.x & 255) >> 3, c = threadIdx.x & 7;
-        cst = *reinterpret_cast<const u32x4*>((which ? a.sin : a.cos) + (int64_t)min(tok0 + row, a.t - 1) * MROPE + 8 * c);
-    }
-    float qs_pre[2];
-    f32x4 ws_pre[2];
+    for (int tb = 0; tb < 2; ++tb) qs[tb] = a.q_norm_scale[min(16 * tb + l16, a.t - 1)];
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb) qs_pre[tb] = a.q_norm_scale[min(tok0 + 16 * tb + l16, a.t - 1)];
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb) ws_pre[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + col0 + 32 * wave + 16 * nb + 4 * g);
-    // weights: every stage of this group, 128 rows x 128 bytes = 4 pieces of 16 bytes per lane (rows tid/8 + 32 i, piece
-    // tid%8); stages past the end re-read the last one and are dropped
-    const int stages = r / QB_K;
-    const int srow = tid >> 3, spc = tid & 7;
-    const int8_t* sp = static_cast<const int8_t*>(a.w_uq_qr) + (int64_t)srow * nq + col0 + 16 * spc;
-    u32x4 stg[QB_MAXS][4];
-#pragma unroll
-    for (int j = 0; j < QB_MAXS; ++j) {
-        const int s = min(grp + QB_GROUPS * j, stages - 1);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) stg[j][i] = *reinterpret_cast<const u32x4*>(sp + ((int64_t)s * QB_K + 32 * i) * nq);
-    }
-#pragma unroll
-    for (int i = 0; i < QB_QP; ++i) {
-        const int pc = (int)threadIdx.x + 1024 * i;
-        if (pc < qpieces) *reinterpret_cast<u32x4*>(ql + (pc / (r / 16)) * qrowb + 16 * (pc % (r / 16))) = qst[i];
-    }
-    if (threadIdx.x < 512) reinterpret_cast<u32x4*>(csl)[threadIdx.x] = cst;
+    for (int nb = 0; nb < 2; ++nb) ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + col0 + 32 * wave + 16 * nb + 4 * g);
     i32x4 acc[2][2];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
         for (int tb = 0; tb < 2; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
+    gt_stream_i8(acc, static_cast<const int8_t*>(a.w_uq_qr) + col0, (int64_t)a.n * MQH, a.q_norm, a.r, a.t, a.r / GT_KI8, lds);
 #pragma unroll
-    for (int j = 0; j < QB_MAXS; ++j) {
-        const int s = grp + QB_GROUPS * j;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            u32x2* d = reinterpret_cast<u32x2*>(wl + (srow + 32 * i) * MQROW + 16 * spc);
-            d[0] = u32x2{stg[j][i][0], stg[j][i][1]};
-            d[1] = u32x2{stg[j][i][2], stg[j][i][3]};
-        }
-        __syncthreads();
-        if (s < stages) {
-#pragma unroll
-            for (int ks = 0; ks < QB_K / 64; ++ks) {
-                i32x4 qf[2], wf[2];
-#pragma unroll
-                for (int tb = 0; tb < 2; ++tb)
-                    qf[tb] = *reinterpret_cast<const i32x4*>(ql + (16 * tb + l16) * qrowb + s * QB_K + ks * 64 + 16 * g);
-                // A operand: output 32 w + 16 nb + l16, contraction bytes 16 g .. 16 g + 15 of the step.  An 8-bit
-                // transposing read hands lane i of a 16-lane group byte i % 8 of the chunks addressed by lanes
-                // i / 8, i / 8 + 2, ..., i / 8 + 14: with lane i pointing at row i / 2, column half i % 2, lane i gets
-                // output column i over rows 0 .. 7 - eight of its sixteen contraction bytes per read
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb) {
-                    const uint8_t* p = wl + (ks * 64 + 16 * g + (l16 >> 1)) * MQROW + 32 * wave + 16 * nb + 8 * (l16 & 1);
-                    const v2i lo = lds_read_tr8(p), hi = lds_read_tr8(p + 8 * MQROW);
-                    wf[nb] = i32x4{lo[0], lo[1], hi[0], hi[1]};
-                }
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-                    for (int tb = 0; tb < 2; ++tb)
-                        acc[nb][tb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[nb], qf[tb], acc[nb][tb], 0, 0, 0);
-            }
-        }
-        __syncthreads();
-    }
-    // add the groups' sums: groups 1.. leave theirs in their own (now idle) first buffer, group 0 collects
-    if (grp > 0) {
-        i32x4* red = reinterpret_cast<i32x4*>(wl);
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) red[(2 * nb + tb) * 256 + tid] = acc[nb][tb];
-    }
-    __syncthreads();
-    if (grp > 0) return;
-#pragma unroll
-    for (int og = 1; og < QB_GROUPS; ++og) {
-        const i32x4* red = reinterpret_cast<const i32x4*>(qb_lds + og * (QB_K * MQROW));
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) acc[nb][tb] += red[(2 * nb + tb) * 256 + tid];
-    }
-    // register e of acc[nb][tb]: output col0 + 32 w + 16 nb + 4 g + e, token 16 tb + l16
-#pragma unroll
-    for (int tb = 0; tb < 2; ++tb) {
-        const int gt = tok0 + 16 * tb + l16;
-        if (gt >= a.t) continue;
-        const float qs = qs_pre[tb];
+    for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
-            const int col = col0 + 32 * wave + 16 * nb + 4 * g;
-            const int head = col / MQH, d = col % MQH;
-            const f32x4 ws = ws_pre[nb];
-            uint16_t vb[4];
+            float v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) vb[e] = f32_to_bf16(((float)acc[nb][tb][e] * qs) * ws[e]);
-            if (d < MNOPE) {
-                const u32x2 pk = {(uint32_t)vb[0] | ((uint32_t)vb[1] << 16), (uint32_t)vb[2] | ((uint32_t)vb[3] << 16)};
-                *reinterpret_cast<u32x2*>(a.qb_nope + ((int64_t)gt * a.n + head) * MNOPE + d) = pk;
-            } else {
-                const uint16_t* cp = csl + (16 * tb + l16) * MROPE;
-                const uint16_t* snp = csl + (MTOK + 16 * tb + l16) * MROPE;
-                uint16_t* out = a.q_rope + ((int64_t)gt * a.n + head) * MROPE;
-#pragma unroll
-                for (int pr = 0; pr < 2; ++pr) {
-                    const int i = (d - MNOPE) / 2 + pr;
-                    const float xe = bf16_to_f32(vb[2 * pr]), xo = bf16_to_f32(vb[2 * pr + 1]);
-                    const float o1 = xe * bf16_to_f32(cp[i]) + (-xo) * bf16_to_f32(snp[i]);
-                    const float o2 = xo * bf16_to_f32(cp[i + 32]) + xe * bf16_to_f32(snp[i + 32]);
-                    out[i] = f32_to_bf16(o1);
-                    out[i + 32] = f32_to_bf16(o2);
-                }
-            }
+            for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs[tb]) * ws[nb][e];
+            *reinterpret_cast<u32x2*>(lds + ((wave >> 1) * MTOK + 16 * tb + l16) * QBS_ROW + (32 * (wave & 1) + 16 * nb + 4 * g) * 2) =
+                u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
         }
-    }
+    __syncthreads();
+    qb_store_blocks<MTOK>(a, lds, 2 * tile, 0);
 }
 
 // grid (tokens), 256 lanes
 __global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a) { mla_norm_body(a, blockIdx.x); }
 
-// grid (n * 192 / 128, token tiles of 32), 1024 lanes
-__global__ __launch_bounds__(1024) void mla_qb_kernel(MlaPrologArgs a)
+// grid (n * 192 / 128), 256 lanes
+__global__ __launch_bounds__(256) void mla_qb_kernel(MlaPrologArgs a)
 {
-    extern __shared__ __align__(16) uint8_t qb_lds[];
-    mla_qb_body(a, blockIdx.x * 128, blockIdx.y * MTOK, qb_lds);
+    __shared__ __align__(16) uint8_t lds[GtStream::LDS];
+    mla_qb_body(a, blockIdx.x, lds);
 }
 
-// The same product at prefill sizes (128 tokens and more): a workgroup owns 128 tokens x 128 outputs and walks the
+// The same product at 33 to 256 tokens: a workgroup owns 128 tokens x 128 outputs and walks the
 // contraction in stages of 128 rows, both operands staged through LDS with the next stage's global loads in flight.  Wave
 // (wr, wc) owns tokens [64 wr, +64) x outputs [64 wc, +64): every operand fragment read from LDS feeds four MFMAs.  The
 // int32 sums are exact, so the results are the bits of mla_qb_kernel's.  The outputs go through LDS (in place of the
@@ -849,7 +722,7 @@ __device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0
     #pragma unroll
                     for (int tb = 0; tb < 4; ++tb)
                         qf[tb] = *reinterpret_cast<const i32x4*>(ql + (64 * wr + 16 * tb + l16) * QG_QROW + ks * 64 + 16 * g);
-                    // (the byte-transposing read: see mla_qb_body)
+                    // (the byte-transposing read: see gt_product_i8)
     #pragma unroll
                     for (int nb = 0; nb < 4; ++nb) {
                         const uint8_t* p = wl + (ks * 64 + 16 * g + (l16 >> 1)) * MQROW + 64 * wc + 16 * nb + 8 * (l16 & 1);
@@ -974,15 +847,16 @@ __global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, Prolog
     }
 }
 
-// grid (n * 192 / 128 + index heads, token tiles of 32), 1024 lanes
-__global__ __launch_bounds__(1024) void fused_qb_kernel(MlaPrologArgs m, PrologArgs p)
+// Up to 32 tokens, grid (n * 192 / 128 + index heads), 256 lanes.  With a workgroup of 1024 lanes per tile that loaded all its
+// weights into registers at once and took them through LDS: 15.7 us at one token, 3.2 TB/s.
+__global__ __launch_bounds__(256) void fused_qb_kernel(MlaPrologArgs m, PrologArgs p)
 {
-    extern __shared__ __align__(16) uint8_t fq_lds[];
+    __shared__ __align__(16) uint8_t lds[PROLOG_STREAM_LDS];
     const int nqb = m.n * MQH / 128;
     if ((int)blockIdx.x < nqb)
-        mla_qb_body(m, blockIdx.x * 128, blockIdx.y * MTOK, fq_lds);
+        mla_qb_body(m, blockIdx.x, lds);
     else
-        prolog_q_body(p, blockIdx.x - nqb, blockIdx.y * PTOK, fq_lds);
+        prolog_q_stream_body(p, blockIdx.x - nqb, lds);
 }
 
 // The same pair at prefill sizes: both products per 128 tokens, side by side.  The indexer's epilogue sets the LDS (68 KB:
@@ -1147,15 +1021,8 @@ static hipError_t set_lds_limits()
 {
     static DeviceOnce once;
     return once.run([] {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(mla_xa_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           4 * XA_K * XROW2);
-        if (e != hipSuccess) return e;
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(mla_qb_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                mla_qb_lds_bytes(MAX_R));
-        if (e != hipSuccess) return e;
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(fused_qb_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                mla_qb_lds_bytes(MAX_R) > prolog_q_lds_bytes(QMAX_R) ? mla_qb_lds_bytes(MAX_R) : prolog_q_lds_bytes(QMAX_R));
-        return e;
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(mla_xa_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   4 * XA_K * XROW2);
     });
 }
 
@@ -1219,10 +1086,9 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
                 }
             }
         } else if (p) {
-            const int smem = mla_qb_lds_bytes(a.r) > prolog_q_lds_bytes(a.r) ? mla_qb_lds_bytes(a.r) : prolog_q_lds_bytes(a.r);
-            hipLaunchKernelGGL(fused_qb_kernel, dim3(a.n * MQH / 128 + p->n, ttiles), dim3(1024), smem, stream, a, *p);
+            hipLaunchKernelGGL(fused_qb_kernel, dim3(a.n * MQH / 128 + p->n), dim3(256), 0, stream, a, *p);
         } else {
-            hipLaunchKernelGGL(mla_qb_kernel, dim3(a.n * MQH / 128, ttiles), dim3(1024), mla_qb_lds_bytes(a.r), stream, a);
+            hipLaunchKernelGGL(mla_qb_kernel, dim3(a.n * MQH / 128), dim3(256), 0, stream, a);
         }
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;

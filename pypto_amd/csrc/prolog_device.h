@@ -435,58 +435,16 @@ __device__ __forceinline__ void prolog_q_big_body(const PrologArgs& a, int head,
         }
     }
 }
-// Above 256 tokens: 32 TB tokens x two heads per workgroup (gemm_tile.h), four waves to a head behind the product; the
-// operations are prolog_q_big_body's, so are the bits (51 us at 1501 tokens there).  512 lanes; an odd last head is taken twice
-// and dropped.
-constexpr int prolog_q_wide_lds(int tb) // the product's stages, or hadamard_q | [2] bf16 tiles | [2] per-wave maxima
-{
-    const int tok = 32 * tb, stage = tok * 128 + 2 * 128 * 128, ring = (3 * stage <= 160 * 1024 ? 3 : 2) * stage;
-    const int epi = PD * PD * 2 + 2 * tok * XROW + 2 * 4 * tok * 4;
-    return epi > ring ? epi : ring;
-}
+// What follows the product for one head and TOK = 32 TB tokens, 256 lanes (ht): rotary, Hadamard, quantisation of the bf16 tile
+// xt [TOK][XROW]; had: hadamard_q, smax: per-wave maxima.  Every lane of the workgroup passes its barriers; heads past the last
+// one are dropped.
 template <int TB>
-__device__ __forceinline__ void prolog_q_wide_body(const PrologArgs& a, int head0, int tok0, uint8_t* lds)
+__device__ __forceinline__ void prolog_q_finish(const PrologArgs& a, int head, int tok0, int ht, const uint8_t* had, uint8_t* xt,
+                                                float (*smax)[32 * TB])
 {
 #pragma clang fp contract(off)
     constexpr int TOK = 32 * TB;
-    static_assert(prolog_q_wide_lds(TB) <= 160 * 1024 && prolog_q_wide_lds(TB) >= GtTile<TB>::LDS, "LDS");
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int l16 = lane & 15, g = lane >> 4, l32 = lane & 31, hl = lane >> 5, wr = wave >> 2, wc = wave & 3;
-    const int64_t nd = (int64_t)a.n * PD;
-    i32x4 acc[4][TB]; // [nb][tb]
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb)
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
-    gt_product_i8<TB>(acc, a.w_qb + head0 * PD, a.w_qb + min(head0 + 1, a.n - 1) * PD, nd, a.q_norm, a.r, tok0, a.t, a.r / GT_KI8, lds);
-    uint8_t* had = lds;
-#pragma unroll
-    for (int i = 0; i < PD * PD * 2 / 16 / 512; ++i) reinterpret_cast<u32x4*>(had)[tid + 512 * i] = reinterpret_cast<const u32x4*>(a.had_q)[tid + 512 * i];
-    // register e of acc[nb][tb]: dim 64 (wc & 1) + 16 nb + 4 g + e of head wc / 2, token 16 TB wr + 16 tb + l16
-    {
-        uint8_t* xt = lds + PD * PD * 2 + (wc >> 1) * TOK * XROW;
-        f32x4 ws[4];
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb)
-            ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + (int64_t)min(head0 + (wc >> 1), a.n - 1) * PD + 64 * (wc & 1) + 16 * nb + 4 * g);
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb) {
-            const int tl = 16 * TB * wr + 16 * tb + l16;
-            const float qs = a.q_norm_scale[min(tok0 + tl, a.t - 1)];
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs) * ws[nb][e];
-                *reinterpret_cast<u32x2*>(xt + tl * XROW + (64 * (wc & 1) + 16 * nb + 4 * g) * 2) =
-                    u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-            }
-        }
-    }
-    __syncthreads();
-    const int hs = tid >> 8, ht = tid & 255, hwave = wave & 3, head = head0 + hs; // from here on four waves to a head
-    uint8_t* xt = lds + PD * PD * 2 + hs * TOK * XROW;
-    float(*smax)[TOK] = reinterpret_cast<float(*)[TOK]>(lds + PD * PD * 2 + 2 * TOK * XROW + hs * 4 * TOK * 4);
+    const int lane = ht & 63, hwave = ht >> 6, l32 = lane & 31, hl = lane >> 5;
     // rotary on the first 64 dims: 32 pairs a token (the arithmetic of rope_tile)
 #pragma unroll 4
     for (int it = 0; it < TOK * 32 / 256; ++it) {
@@ -562,6 +520,99 @@ __device__ __forceinline__ void prolog_q_wide_body(const PrologArgs& a, int head
             if (hwave == 0 && hl == 0) a.q_scale[(int64_t)gt * a.n + head] = __builtin_bit_cast(uint16_t, (_Float16)(1.0f / sq));
         }
     }
+}
+
+// Above 256 tokens: 32 TB tokens x two heads per workgroup (gemm_tile.h), four waves to a head behind the product; the
+// operations are prolog_q_big_body's, so are the bits (51 us at 1501 tokens there).  512 lanes; an odd last head is taken twice
+// and dropped.
+constexpr int prolog_q_wide_lds(int tb) // the product's stages, or hadamard_q | [2] bf16 tiles | [2] per-wave maxima
+{
+    const int tok = 32 * tb, stage = tok * 128 + 2 * 128 * 128, ring = (3 * stage <= 160 * 1024 ? 3 : 2) * stage;
+    const int epi = PD * PD * 2 + 2 * tok * XROW + 2 * 4 * tok * 4;
+    return epi > ring ? epi : ring;
+}
+template <int TB>
+__device__ __forceinline__ void prolog_q_wide_body(const PrologArgs& a, int head0, int tok0, uint8_t* lds)
+{
+#pragma clang fp contract(off)
+    constexpr int TOK = 32 * TB;
+    static_assert(prolog_q_wide_lds(TB) <= 160 * 1024 && prolog_q_wide_lds(TB) >= GtTile<TB>::LDS, "LDS");
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
+    const int64_t nd = (int64_t)a.n * PD;
+    i32x4 acc[4][TB]; // [nb][tb]
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
+    gt_product_i8<TB>(acc, a.w_qb + head0 * PD, a.w_qb + min(head0 + 1, a.n - 1) * PD, nd, a.q_norm, a.r, tok0, a.t, a.r / GT_KI8, lds);
+    uint8_t* had = lds;
+#pragma unroll
+    for (int i = 0; i < PD * PD * 2 / 16 / 512; ++i) reinterpret_cast<u32x4*>(had)[tid + 512 * i] = reinterpret_cast<const u32x4*>(a.had_q)[tid + 512 * i];
+    // register e of acc[nb][tb]: dim 64 (wc & 1) + 16 nb + 4 g + e of head wc / 2, token 16 TB wr + 16 tb + l16
+    {
+        uint8_t* xt = lds + PD * PD * 2 + (wc >> 1) * TOK * XROW;
+        f32x4 ws[4];
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb)
+            ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + (int64_t)min(head0 + (wc >> 1), a.n - 1) * PD + 64 * (wc & 1) + 16 * nb + 4 * g);
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {
+            const int tl = 16 * TB * wr + 16 * tb + l16;
+            const float qs = a.q_norm_scale[min(tok0 + tl, a.t - 1)];
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) {
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs) * ws[nb][e];
+                *reinterpret_cast<u32x2*>(xt + tl * XROW + (64 * (wc & 1) + 16 * nb + 4 * g) * 2) =
+                    u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+            }
+        }
+    }
+    __syncthreads();
+    const int hs = tid >> 8, ht = tid & 255, head = head0 + hs; // from here on four waves to a head
+    uint8_t* xt = lds + PD * PD * 2 + hs * TOK * XROW;
+    float(*smax)[TOK] = reinterpret_cast<float(*)[TOK]>(lds + PD * PD * 2 + 2 * TOK * XROW + hs * 4 * TOK * 4);
+    prolog_q_finish<TB>(a, head, tok0, ht, lds, xt, smax);
+}
+
+// Up to 32 tokens: one head per workgroup of 256 lanes behind the streamed product; the bits of prolog_q_body.
+// lds: the stages, afterwards the bf16 tile and the per-wave maxima | hadamard_q, copied along with the first stages
+constexpr int PROLOG_STREAM_LDS = GtStream::LDS + PD * PD * 2;
+static_assert(PTOK * XROW + 4 * PTOK * 4 <= GtStream::LDS && PTOK == GtStream::TOK, "tile and maxima take the stages' place");
+__device__ __forceinline__ void prolog_q_stream_body(const PrologArgs& a, int head, uint8_t* lds)
+{
+#pragma clang fp contract(off)
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
+    uint8_t* had = lds + GtStream::LDS;
+    float qs[2];
+    f32x4 ws[2];
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) qs[tb] = a.q_norm_scale[min(16 * tb + l16, a.t - 1)];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + (int64_t)head * PD + 32 * wave + 16 * nb + 4 * g);
+#pragma unroll
+    for (int i = 0; i < PD * PD * 2 / 4096; ++i) gt_copy(a.had_q, (uint32_t)(4096 * i + 16 * tid), had + 4096 * i + 1024 * wave);
+    i32x4 acc[2][2];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
+    gt_stream_i8(acc, a.w_qb + head * PD, (int64_t)a.n * PD, a.q_norm, a.r, a.t, a.r / GT_KI8, lds);
+    uint8_t* xt = lds;
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs[tb]) * ws[nb][e];
+            *reinterpret_cast<u32x2*>(xt + (16 * tb + l16) * XROW + (32 * wave + 16 * nb + 4 * g) * 2) =
+                u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        }
+    __syncthreads();
+    prolog_q_finish<1>(a, head, 0, tid, had, xt, reinterpret_cast<float(*)[PTOK]>(lds + PTOK * XROW));
 }
 constexpr int PROLOG_BIG_T = 128;   // token count from which the query product runs per 128 tokens
 
