@@ -470,7 +470,8 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb16_wide_kernel(MlaPrologArg
 __device__ __forceinline__ float wave_sum(float v) { return wave_sum_butterfly(v); }
 __device__ __forceinline__ float wave_max(float v) { return wave_max_f32(v); }
 
-// one workgroup of 256 lanes per token
+// one workgroup of 256 lanes per token; S: splits whose partial sums are in flight together
+template <int S>
 __device__ __forceinline__ void mla_norm_body(const MlaPrologArgs& a, int tok)
 {
 #pragma clang fp contract(off)
@@ -502,17 +503,17 @@ __device__ __forceinline__ void mla_norm_body(const MlaPrologArgs& a, int tok)
             cj[j] = min(256 * j + tid, ncols - 1);
             sum[j] = 0.f;
         }
-        // four splits' loads in flight together (a split past the end re-reads the last one and adds zero)
-        for (int s0 = 0; s0 < a.ksplits; s0 += 4) {
-            float v[4][NJ];
+        // (a split past the end re-reads the last one and adds zero)
+        for (int s0 = 0; s0 < a.ksplits; s0 += S) {
+            float v[S][NJ];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < S; ++i) {
                 const float* p = a.xa_part + ((int64_t)min(s0 + i, a.ksplits - 1) * a.t + tok) * a.ncols;
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) v[i][j] = p[cj[j]];
             }
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < S; ++i)
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) sum[j] += s0 + i < a.ksplits ? v[i][j] : 0.f;
         }
@@ -639,7 +640,11 @@ __device__ __forceinline__ void mla_qb_body(const MlaPrologArgs& a, int tile, ui
 }
 
 // grid (tokens), 256 lanes
-__global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a) { mla_norm_body(a, blockIdx.x); }
+template <int S>
+__global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a)
+{
+    mla_norm_body<S>(a, blockIdx.x);
+}
 
 // grid (n * 192 / 128), 256 lanes
 __global__ __launch_bounds__(256) void mla_qb_kernel(MlaPrologArgs a)
@@ -837,13 +842,14 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb_wide_kernel(MlaPrologArgs 
 // GEMMs on q_norm (192 + 64 workgroups at model sizes: one per compute unit); the indexer's x @ [w_k | w_proj] rides along
 // in mla_xa_kernel as three more output tiles.
 // grid (tokens, 2), 256 lanes: y = 0 the MLA norms and cache rows, y = 1 the indexer's key path and weights (128 lanes)
+template <int S>
 __global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, PrologArgs p)
 {
     if (blockIdx.y == 0) {
-        mla_norm_body(m, blockIdx.x);
+        mla_norm_body<S>(m, blockIdx.x);
     } else {
         if (threadIdx.x >= 128) return; // the barriers inside are among the two remaining waves
-        prolog_k_body(p, blockIdx.x);
+        prolog_k_body<S>(p, blockIdx.x);
     }
 }
 
@@ -1051,10 +1057,14 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
     if ((e = hipGetLastError()) != hipSuccess) return e;
     {
         ScopedKernelTimer tm(KID_MLA_NORM, stream);
+        // all partial sums of an output in flight at once for the usual seven splits and fewer, none of them twice for one or two
+        const int in_flight = a.ksplits <= 2 ? 2 : a.ksplits <= 4 ? 4 : 8;
         if (p)
-            hipLaunchKernelGGL(fused_norm_kernel, dim3(a.t, 2), dim3(256), 0, stream, a, *p);
+            hipLaunchKernelGGL((in_flight == 2 ? fused_norm_kernel<2> : in_flight == 4 ? fused_norm_kernel<4> : fused_norm_kernel<8>),
+                               dim3(a.t, 2), dim3(256), 0, stream, a, *p);
         else
-            hipLaunchKernelGGL(mla_norm_kernel, dim3(a.t), dim3(256), 0, stream, a);
+            hipLaunchKernelGGL((in_flight == 2 ? mla_norm_kernel<2> : in_flight == 4 ? mla_norm_kernel<4> : mla_norm_kernel<8>),
+                               dim3(a.t), dim3(256), 0, stream, a);
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
     {
