@@ -3,8 +3,8 @@
 // What bounds these products at prefill sizes is what the CUs draw from the L2: with the matrix instructions taken out, the
 // copies of 128 x 128 tiles alone (1.03 GB for 777 tokens x 5120 x 14336) take 77 of the product's 87 us, 13 TB/s, wherever the
 // tiles lie, and staging through registers under two barriers a stage took 99 us.  So the tile is as large as LDS and registers
-// hold (537 MB and 74 us there, of which the copies hide 14 us less than all; a ring of five half stages with the fragments read
-// a stage ahead is no faster), and
+// hold: 537 MB and 74 us there, where the copies alone take 72 (a round trip per stage) and the rest alone 59; a ring of five
+// half stages with the fragments read a stage ahead is no faster.  And
 //  - a stage's operands are copied to LDS by the memory pipe itself (global_load_lds_dwordx4: no registers, no LDS store
 //    instructions), into the buffer that is not being read, so that a stage has one barrier;
 //  - rows of 128 bytes are kept unpadded (a copy writes 64 lanes x 16 bytes in a row) and spread over the banks by
@@ -24,7 +24,6 @@
 namespace pto {
 namespace {
 
-constexpr int GT_OUT = 256;                  // outputs of a workgroup's tile: two halves of 128
 constexpr int GT_LANES = 512;
 constexpr int GT_KI8 = 128;                  // contraction rows per stage
 template <int TB>

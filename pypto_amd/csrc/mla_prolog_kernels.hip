@@ -665,9 +665,8 @@ constexpr int QG_QROW = QG_K + 16;       // bytes per LDS row of the [token][k] 
 constexpr int QG_OROW = 128 * 2 + 16;    // bytes per LDS row of the [token][128 outputs] bf16 tile
 constexpr int QG_STAGE_BYTES = QG_K * MQROW + QG_TOK * QG_QROW;
 static_assert(QG_TOK * QG_OROW <= QG_STAGE_BYTES, "the output tile takes the operand tiles' place");
-// DEPTH: stages whose loads are in flight (register sets used round-robin).  One keeps the kernel at 158 registers, three
-// workgroups to a CU - what the 768 workgroups of 512 tokens want; at 256 tokens and fewer the grid leaves at most two
-// workgroups to a CU anyway, and the twelve stages of a tile are otherwise twelve memory latencies in a row.
+// DEPTH: stages whose loads are in flight (register sets used round-robin): the grid leaves at most two workgroups to a CU at
+// these sizes, and the twelve stages of a tile are otherwise twelve memory latencies in a row.
 template <int DEPTH>
 __device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0, int tok0, uint8_t* stage_lds)
 {
@@ -792,7 +791,7 @@ __device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0
 }
 
 template <int DEPTH>
-__global__ __launch_bounds__(256, DEPTH == 1 ? 3 : 2) void mla_qb_big_kernel(MlaPrologArgs a)
+__global__ __launch_bounds__(256, 2) void mla_qb_big_kernel(MlaPrologArgs a)
 {
     __shared__ __align__(16) uint8_t stage_lds[QG_STAGE_BYTES];
     mla_qb_big_body<DEPTH>(a, blockIdx.x * 128, blockIdx.y * QG_TOK, stage_lds);
@@ -865,7 +864,7 @@ __global__ __launch_bounds__(256) void fused_qb_kernel(MlaPrologArgs m, PrologAr
         prolog_q_stream_body(p, blockIdx.x - nqb, lds);
 }
 
-// The same pair at prefill sizes: both products per 128 tokens, side by side.  The indexer's epilogue sets the LDS (68 KB:
+// The same pair at 33 to 256 tokens: both products per 128 tokens, side by side.  The indexer's epilogue sets the LDS (68 KB:
 // two workgroups to a CU), so both run with three stages of loads in flight.
 // grid (n * 192 / 128 + index heads, token tiles of 128), 256 lanes
 __global__ __launch_bounds__(256, 2) void fused_qb_big_kernel(MlaPrologArgs m, PrologArgs p)
@@ -1039,7 +1038,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
     const int ttiles = (a.t + MTOK - 1) / MTOK;
     hipError_t e = set_lds_limits();
     if (e != hipSuccess) return e;
-    const bool big = a.t >= BIG_T; // prefill sizes: the kernels that own an output tile
+    const bool big = a.t >= BIG_T; // the kernels that own an output tile
     {
         ScopedKernelTimer tm(KID_MLA_XA, stream);
         if (big)
