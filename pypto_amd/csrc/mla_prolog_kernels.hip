@@ -799,16 +799,19 @@ __global__ __launch_bounds__(256, 2) void mla_qb_big_kernel(MlaPrologArgs a)
 
 // Above 256 tokens: 32 TB tokens x 256 outputs per workgroup (gemm_tile.h), the same exact sums and the same operations behind
 // them.  128 x 128 tiles through registers took 109 us at 1501 tokens, bound by the operands' way into LDS.
-// grid (n * 192 / 256 rounded up, token tiles), 512 lanes.
+constexpr int mla_qb_wide_lds(int tb) // the product's stages, or four blocks of the output tile
+{
+    const int tok = 32 * tb, stage = tok * 128 + 2 * 128 * 128, ring = (3 * stage <= 160 * 1024 ? 3 : 2) * stage;
+    return 4 * tok * QBS_ROW > ring ? 4 * tok * QBS_ROW : ring;
+}
 template <int TB>
-__global__ __launch_bounds__(GT_LANES, 2) void mla_qb_wide_kernel(MlaPrologArgs a)
+__device__ __forceinline__ void mla_qb_wide_body(const MlaPrologArgs& a, int tile, int tok0, uint8_t* lds)
 {
 #pragma clang fp contract(off)
     using T = GtTile<TB>;
-    constexpr int EPI = 4 * T::TOK * QBS_ROW;
-    __shared__ __align__(16) uint8_t lds[EPI > T::LDS ? EPI : T::LDS];
+    static_assert(mla_qb_wide_lds(TB) >= T::LDS, "LDS");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
-    const int nq = a.n * MQH, col0 = 256 * blockIdx.x, tok0 = blockIdx.y * T::TOK; // (nq is a multiple of 128)
+    const int nq = a.n * MQH, col0 = 256 * tile; // (nq is a multiple of 128)
     i32x4 acc[4][TB]; // [nb][tb]
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb)
@@ -833,7 +836,14 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb_wide_kernel(MlaPrologArgs 
         }
     }
     __syncthreads();
-    qb_store_blocks<T::TOK>(a, lds, 4 * blockIdx.x, tok0);
+    qb_store_blocks<T::TOK>(a, lds, 4 * tile, tok0);
+}
+// grid (n * 192 / 256 rounded up, token tiles), 512 lanes
+template <int TB>
+__global__ __launch_bounds__(GT_LANES, 2) void mla_qb_wide_kernel(MlaPrologArgs a)
+{
+    __shared__ __align__(16) uint8_t lds[mla_qb_wide_lds(TB)];
+    mla_qb_wide_body<TB>(a, blockIdx.x, blockIdx.y * 32 * TB, lds);
 }
 
 // ------------------------------------------------------------------------------------------------ fused with the indexer prolog
@@ -878,13 +888,18 @@ __global__ __launch_bounds__(256, 2) void fused_qb_big_kernel(MlaPrologArgs m, P
         prolog_q_big_body<QB_DEPTH>(p, blockIdx.x - nqb, blockIdx.y * QB_TOK, lds);
 }
 
-// Above 256 tokens the two products are launches of their own again, with tiles of their own sizes.
-// grid (index heads / 2 rounded up, token tiles), 512 lanes
+// Above 256 tokens the two products in one launch of gemm_tile.h's tiles: the index heads' part alone is half a round of
+// workgroups up to 512 tokens (call of 257 tokens 94 -> 80 us, 512: 124 -> 104, 1501: the same).  grid (index heads / 2 rounded up + n * 192 / 256 rounded up, token tiles), 512 lanes
 template <int TB>
-__global__ __launch_bounds__(GT_LANES, 2) void fused_q_wide_kernel(PrologArgs p)
+__global__ __launch_bounds__(GT_LANES, 2) void fused_qb_wide_kernel(MlaPrologArgs m, PrologArgs p)
 {
-    __shared__ __align__(16) uint8_t lds[prolog_q_wide_lds(TB)];
-    prolog_q_wide_body<TB>(p, 2 * blockIdx.x, blockIdx.y * 32 * TB, lds);
+    constexpr int A = mla_qb_wide_lds(TB), B = prolog_q_wide_lds(TB);
+    __shared__ __align__(16) uint8_t lds[A > B ? A : B];
+    const int nqt = (p.n + 1) / 2, tok0 = blockIdx.y * 32 * TB;
+    if ((int)blockIdx.x < nqt)
+        prolog_q_wide_body<TB>(p, 2 * blockIdx.x, tok0, lds);
+    else
+        mla_qb_wide_body<TB>(m, blockIdx.x - nqt, tok0, lds);
 }
 
 // ------------------------------------------------------------------------------------------------ q_b[:, head, :128] @ w_uk[head]
@@ -1077,22 +1092,20 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
             if (p && a.t <= BIG_T2) {
                 hipLaunchKernelGGL(fused_qb_big_kernel, dim3(qgrid.x + p->n, qgrid.y), dim3(256), 0, stream, a, *p);
             } else {
-                if (a.t <= BIG_T2) {
+                const int cols = (a.n * MQH + 255) / 256, qcols = p ? (p->n + 1) / 2 : 0;
+                if (a.t <= BIG_T2)
                     hipLaunchKernelGGL(mla_qb_big_kernel<QB_DEPTH>, qgrid, dim3(256), 0, stream, a);
-                } else {
-                    const int cols = (a.n * MQH + 255) / 256;
+                else if (p)
+                    gt_dispatch(gt_token_blocks(a.t, cols + qcols, a.r / GT_KI8, 7), [&](auto tb) {
+                        constexpr int TB = decltype(tb)::value < 7 ? decltype(tb)::value : 7;
+                        hipLaunchKernelGGL(fused_qb_wide_kernel<TB>, dim3(qcols + cols, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream,
+                                           a, *p);
+                    });
+                else
                     gt_dispatch(gt_token_blocks(a.t, cols, a.r / GT_KI8, 8), [&](auto tb) {
                         constexpr int TB = decltype(tb)::value;
                         hipLaunchKernelGGL(mla_qb_wide_kernel<TB>, dim3(cols, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream, a);
                     });
-                }
-                if (p) {
-                    const int cols = (p->n + 1) / 2;
-                    gt_dispatch(gt_token_blocks(a.t, cols, a.r / GT_KI8, 7), [&](auto tb) {
-                        constexpr int TB = decltype(tb)::value < 7 ? decltype(tb)::value : 7;
-                        hipLaunchKernelGGL(fused_q_wide_kernel<TB>, dim3(cols, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream, *p);
-                    });
-                }
             }
         } else if (p) {
             hipLaunchKernelGGL(fused_qb_kernel, dim3(a.n * MQH / 128 + p->n), dim3(256), 0, stream, a, *p);
