@@ -99,14 +99,15 @@ struct Lengths {
         q += r < 0 ? -1 : r >= c ? 1 : 0;
         return len[j] < 0 ? 0 : max(1, q);
     }
-    __device__ __forceinline__ int units(const GqaArgs& a, int c) const
+    // of all sequences (256 sequences of 2^30 tokens have 2^31 chunks of 128: unsigned)
+    __device__ __forceinline__ uint32_t units(const GqaArgs& a, int c) const
     {
         const float inv_c = 1.f / (float)c;
         int n = 0;
 #pragma unroll
         for (int j = 0; j < GQA_SCAN / 64; ++j)
             if (64 * j < a.b) n += chunks(j, c, inv_c); // (uniform)
-        return __builtin_amdgcn_readlane(gqa_prefix_sum(n), 63);
+        return (uint32_t)__builtin_amdgcn_readlane(gqa_prefix_sum(n), 63);
     }
 };
 
@@ -116,18 +117,18 @@ struct Lengths {
 // Depends on the lengths alone, so every wavefront finds the same one; the result never exceeds units_cap units.
 __device__ __forceinline__ int choose_chunk(const GqaArgs& a, const Lengths& ls)
 {
-    int sum = 0, longest = 0;
+    int mine = 0, longest = 0;
 #pragma unroll
     for (int j = 0; j < GQA_SCAN / 64; ++j) {
         if (64 * j >= a.b) break; // (uniform)
-        sum += (max(ls.len[j], 0) + 127) >> 7;
+        mine += (max(ls.len[j], 0) + 127) >> 7;
         longest = max(longest, ls.len[j]);
     }
-    sum = __builtin_amdgcn_readlane(gqa_prefix_sum(sum), 63);
-    // rounds of GQA_SLOTS workgroups with GQA_TARGET tokens
-    const int rounds = max((int)ceilf((float)sum * (float)a.columns * (128.f / GQA_SLOTS / GQA_TARGET)), 1);
-    const int target = min(max(rounds * GQA_SLOTS / a.columns, a.b), a.units_cap);
-    int lo = max((sum + target - 1) / target, 1); // (no shorter chunk can do)
+    const uint32_t sum = (uint32_t)__builtin_amdgcn_readlane(gqa_prefix_sum(mine), 63);
+    // rounds of GQA_SLOTS workgroups with GQA_TARGET tokens (of at most 2^22, so that their slots fit 32 bits)
+    const int rounds = (int)fminf(fmaxf(ceilf((float)sum * (float)a.columns * (128.f / GQA_SLOTS / GQA_TARGET)), 1.f), 0x1p22f);
+    const uint32_t target = (uint32_t)min(max(rounds * GQA_SLOTS / a.columns, a.b), (int)a.units_cap);
+    int lo = max((int)((sum + target - 1) / target), 1); // (no shorter chunk can do)
     if (ls.units(a, lo) <= target) return lo * 128;
     longest = (int)wave_max_f32((float)longest) + 128; // the batch's (as a float it may be off by less than 128)
     int hi = max((longest + 127) / 128, lo + 1); // one chunk per sequence: at most a.b <= target units
@@ -140,14 +141,16 @@ __device__ __forceinline__ int choose_chunk(const GqaArgs& a, const Lengths& ls)
 }
 
 // chunk length, and the (sequence, chunk) of unit u with the sequence's first unit; false: no such unit
-__device__ __forceinline__ bool gqa_unit(const GqaArgs& a, int u, int lane, int& chunk, int& bi, int& split)
+__device__ __forceinline__ bool gqa_unit(const GqaArgs& a, uint32_t unit, int lane, int& chunk, int& bi, int& split)
 {
     chunk = a.chunk;
     if (a.b > GQA_SCAN) { // (fixed chunks by the unit's place)
-        bi = u / a.nsplit;
-        split = u - bi * a.nsplit;
-        return bi < a.b;
+        const uint32_t seq = unit / (uint32_t)a.nsplit;
+        bi = (int)seq;
+        split = (int)(unit - seq * (uint32_t)a.nsplit);
+        return seq < (uint32_t)a.b;
     }
+    const int u = (int)unit;
     Lengths ls;
     ls.fetch(a, lane);
     if (chunk == 0) chunk = choose_chunk(a, ls);
@@ -183,11 +186,12 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a)
     // heads, whose rows lie beside each other in the cache.  Workgroups go to the eight dies in turn, so the readers of the
     // same keys share an L2.
     const int readers = a.s1 * a.hsub / RT;
-    int u, n2, rd;
+    uint32_t u; // (the grid has fewer than 2^32 workgroups)
+    int n2, rd;
     {
         const uint32_t lin = blockIdx.x + gridDim.x * blockIdx.y, per = 8u * readers * a.nkv;
         const uint32_t o = lin / per, in = lin - o * per;
-        u = (int)(o * 8 + (in & 7));
+        u = o * 8 + (in & 7);
         rd = (int)((in >> 3) % readers) * RT;
         n2 = (int)((in >> 3) / readers);
     }
@@ -195,7 +199,7 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a)
     if (!gqa_unit(a, u, lane, chunk, bi, split)) return;
     if (a.part_o != nullptr && tid == 0 && rd == 0 && n2 == 0) { // for the combine kernel
         if (u == 0) a.plan[0] = chunk;
-        if (split == 0) a.plan[1 + bi] = u;
+        if (split == 0) a.plan[1 + bi] = (int32_t)u; // (read for up to GQA_SCAN sequences)
     }
 
     const int g = a.nq / a.nkv;
@@ -438,7 +442,9 @@ __global__ __launch_bounds__(256) void gqa_combine_kernel(GqaArgs a)
     const int chunk = a.plan[0];
     const int nvalid = (cur + chunk - 1) / chunk;
     // the unit's partials lie [query token of the sequence, head]
-    const int64_t slot0 = ((int64_t)a.plan[1 + bi] * a.s1 + si) * a.nq + (head_row - (int64_t)tq * a.nq), per = (int64_t)a.s1 * a.nq;
+    int64_t unit0 = a.plan[1 + bi];
+    if (a.b > GQA_SCAN) unit0 = (int64_t)bi * a.nsplit; // (may leave 32 bits)
+    const int64_t slot0 = (unit0 * a.s1 + si) * a.nq + (head_row - (int64_t)tq * a.nq), per = (int64_t)a.s1 * a.nq;
     const float* pm = a.part_ml + slot0 * 2;
     const float* po = a.part_o + slot0 * GD + d0;
     // eight chunks' loads in flight at a time (a chunk past the last valid one re-reads the last and is dropped): an online
@@ -535,14 +541,14 @@ void gqa_plan(GqaArgs& a, int forced_chunk)
         const int64_t most = (int64_t)a.b * (max_ctx > 128 * GQA_MAX_SPLIT ? GQA_MAX_SPLIT : (max_ctx + 127) / 128);
         if (target > most) target = most;
         a.chunk = 0; // chosen on the device
-        a.units_cap = (int32_t)(target > a.b ? target : a.b);
+        a.units_cap = target > a.b ? target : a.b;
         a.nsplit = a.units_cap > a.b ? 2 : 1;
         if (a.nsplit == 1) a.chunk = (int32_t)((max_ctx + 127) / 128 * 128);
     }
     if (a.chunk > 0) {
         const int64_t n = (max_ctx + a.chunk - 1) / a.chunk;
         a.nsplit = n < 1 ? 1 : (int32_t)n;
-        a.units_cap = (int32_t)(a.b * (int64_t)a.nsplit);
+        a.units_cap = a.b * (int64_t)a.nsplit;
     }
     a.stream_past_cache = (double)t / (a.s1 > 0 ? a.s1 : 1) * (double)max_ctx * a.nkv * 2 * GROW > 256e6;
 }
@@ -578,10 +584,10 @@ hipError_t gqa_launch(const GqaArgs& a, hipStream_t stream)
     }
     {
         ScopedKernelTimer timer(KID_GQA_DECODE, stream);
-        const int64_t units = ((int64_t)a.units_cap + 7) / 8 * 8;
+        const int64_t units = (a.units_cap + 7) / 8 * 8;
         const int64_t groups = units * a.columns;
         const int64_t gx = groups < (1 << 22) ? groups : (1 << 22);
-        if (groups + gx > 0xffffffffll) return hipErrorInvalidValue;
+        if (groups + gx > 0xffffffffll) return hipErrorInvalidValue; // (partials of over 2 TB)
         auto kern = a.row_tiles == 2 ? (a.stream_past_cache ? gqa_decode_kernel<2, true> : gqa_decode_kernel<2, false>)
                                      : (a.stream_past_cache ? gqa_decode_kernel<1, true> : gqa_decode_kernel<1, false>);
         hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)((groups + gx - 1) / gx)), dim3(256), 0, stream, a);
@@ -593,7 +599,7 @@ hipError_t gqa_launch(const GqaArgs& a, hipStream_t stream)
         const int64_t rows = t * a.nq;
         // (eight groups per row for few rows of many chunks: 16 chunks take one group 9 us where rows are few; with many rows the
         // second step costs more than it saves, 20 us against 6 at 6144 rows)
-        if (a.units_cap > 12 * a.b && rows <= 2048)
+        if (a.units_cap > 12 * (int64_t)a.b && rows <= 2048)
             hipLaunchKernelGGL(gqa_combine_kernel<8>, dim3((unsigned)rows), dim3(256), 0, stream, a);
         else
             hipLaunchKernelGGL(gqa_combine_kernel<1>, dim3((unsigned)((rows + 7) / 8)), dim3(256), 0, stream, a);

@@ -101,8 +101,9 @@ struct GqaArgs {
     int64_t n_blocks;
     int32_t b, s1, nq, nkv, hsub, block_size, bt_stride;
     // set by gqa_plan: chunks per sequence (at most; > 1: the combine kernel runs), chunk length (0: chosen on the device),
-    // 16-row tiles per workgroup, workgroups per unit, units of the batch at most
-    int32_t nsplit, chunk, row_tiles, columns, units_cap;
+    // 16-row tiles per workgroup, workgroups per unit
+    int32_t nsplit, chunk, row_tiles, columns;
+    int64_t units_cap; // set by gqa_plan: units of the batch at most (beyond 32 bits with short forced chunks under a wide page table)
     bool stream_past_cache;     // set by gqa_plan
     float softmax_scale;
 };

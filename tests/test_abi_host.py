@@ -276,3 +276,24 @@ def test_paged_gather_validation(lib):
     assert rc == -3 and "status must hold one word" in msg
     # nothing to gather: accepted, nothing launched
     assert launch_rc(lib, "paged_gather", specs(idx=(INT32, (2, 0)), out=(INT8, (0, 656))), p)[0] == 0
+
+
+def gqa_specs(b, s1, nq, nkv, cols, page, pages=1):
+    cache = (BF16, (pages, page, nkv, 128))
+    return [(BF16, (b * s1, nq, 128)), cache, cache, (INT32, (b, cols)), (INT32, (b,)), (BF16, (b * s1, nq, 128))]
+
+
+def gqa_workspace(lib, specs, chunk=0):
+    p = _runtime.GqaParams(0.1, chunk)
+    lib.pto_gqa_decode_workspace.restype = ctypes.c_uint64
+    return lib.pto_gqa_decode_workspace(descs(specs), 6, ctypes.byref(p))
+
+
+@pytest.mark.parametrize("chunk", [0, 4096])
+def test_gqa_workspace_grows_with_the_batch_beyond_32_bits_of_chunks(lib, chunk):
+    """Chunks of the whole batch are counted in 64 bits: with the chunk lengths of one sequence the workspace is proportional
+    to the number of sequences, also where 1023 pages of 2^20 tokens times 16 401 sequences have over 2^32 chunks."""
+    few = gqa_workspace(lib, gqa_specs(512, 1, 1, 1, 1023, 1 << 20), chunk)
+    for b in (16384, 16401, 65535):
+        many = gqa_workspace(lib, gqa_specs(b, 1, 1, 1, 1023, 1 << 20), chunk)
+        assert abs(many / few - b / 512) < 1e-3 * b / 512, (b, many, few)

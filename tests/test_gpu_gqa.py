@@ -136,10 +136,11 @@ def test_full_size_config4(cuda):
 
 @pytest.mark.parametrize("s1,nq,nkv,act", [(1, 12, 1, [1]), (1, 12, 1, [128, 129, 0, 33]), (2, 12, 1, [4097, 1, 2, 700]), (3, 12, 2, [500, 2, 1300]),
                                            (1, 40, 2, [900, 31]), (2, 34, 2, [64, 260]), (1, 12, 1, [9000] + [5] * 70),
-                                           (1, 12, 2, [0] * 3 + [1500, 0, 40]), (1, 12, 1, [3, 200] * 150), (1, 96, 8, [300] * 40)])
+                                           (1, 12, 2, [0] * 3 + [1500, 0, 40]), (1, 12, 1, [3, 200] * 150), (1, 12, 1, [3, 200] * 150 + [9000]),
+                                           (1, 96, 8, [300] * 40)])
 def test_chunk_choice_and_row_tiles(cuda, s1, nq, nkv, act):
     """Chunks chosen from the lengths: single tokens, page edges, empty sequences, one long sequence among many short ones
-    (lengths beyond one wavefront's lanes), more sequences than the device-side choice takes, one chunk per sequence; one and
+    (lengths beyond one wavefront's lanes), more sequences than the device-side choice takes (of one and of several chunks), one chunk per sequence; one and
     two row tiles per workgroup from query tokens and from head sub-groups."""
     case = gqa.make_case(len(act), s1, nq, nkv, act, seed=len(act) + nq)
     check(run(case, cuda), case, f"{s1} {nq} {nkv} {act[:6]}")
