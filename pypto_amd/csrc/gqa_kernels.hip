@@ -28,6 +28,7 @@
 //       S^T comes out in (lane = head l%16, 4 tokens per 16-token block), so P~ never leaves registers.  The contraction
 //       index is visited in the order {4g..4g+3, 16+4g..16+4g+3} per lane group g on both operands.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <stdint.h>
 
 #include "common.h"
@@ -44,7 +45,8 @@ constexpr int GROW = GD * 2; // bytes per staged V row
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr int GQA_SLOTS = 256;   // one workgroup per CU (two fit; twice as many shorter ones measured 5 to 15 % slower on small batches)
 constexpr int GQA_TARGET = 4096; // tokens a workgroup should have at most, where there are enough
-constexpr int GQA_MAX_SPLIT = 128; // chunks per sequence on average at most (the combine kernel walks them)
+constexpr int GQA_MAX_SPLIT = 64; // chunks per sequence on average at most, beyond one round of GQA_SLOTS workgroups: the partials
+                                  // take memory by the page table's reach (512 sequences, 96 / 8 heads, 1 M tokens: 1.6 GB)
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -532,14 +534,16 @@ void gqa_plan(GqaArgs& a, int forced_chunk)
     if (forced_chunk > 0) {
         a.chunk = (forced_chunk + 127) / 128 * 128;
     } else if (a.b > GQA_SCAN) {
-        a.chunk = GQA_TARGET;
+        const int64_t least = (max_ctx + GQA_MAX_SPLIT - 1) / GQA_MAX_SPLIT;
+        a.chunk = least > GQA_TARGET ? (int32_t)((least + 127) / 128 * 128) : GQA_TARGET;
     } else {
         const int64_t round = (int64_t)GQA_SLOTS * (GQA_TARGET / 128);
         const int64_t work = (int64_t)a.b * ((max_ctx + 127) / 128) * a.columns;
         const int64_t rounds = (work + round - 1) / round;
         int64_t target = (rounds > 1 ? rounds : 1) * GQA_SLOTS / a.columns;
-        const int64_t most = (int64_t)a.b * (max_ctx > 128 * GQA_MAX_SPLIT ? GQA_MAX_SPLIT : (max_ctx + 127) / 128);
-        if (target > most) target = most;
+        const int64_t pages = (int64_t)a.b * ((max_ctx + 127) / 128);
+        const int64_t one_round = std::min<int64_t>(GQA_SLOTS / a.columns, 2 * GQA_MAX_SPLIT * (int64_t)a.b);
+        target = std::min(std::min(target, std::max(one_round, GQA_MAX_SPLIT * (int64_t)a.b)), pages);
         a.chunk = 0; // chosen on the device
         a.units_cap = target > a.b ? target : a.b;
         a.nsplit = a.units_cap > a.b ? 2 : 1;

@@ -297,3 +297,12 @@ def test_gqa_workspace_grows_with_the_batch_beyond_32_bits_of_chunks(lib, chunk)
     for b in (16384, 16401, 65535):
         many = gqa_workspace(lib, gqa_specs(b, 1, 1, 1, 1023, 1 << 20), chunk)
         assert abs(many / few - b / 512) < 1e-3 * b / 512, (b, many, few)
+
+
+@pytest.mark.parametrize("b", [4, 64, 256, 257, 512, 2048])
+@pytest.mark.parametrize("cols", [512, 8192, 32768])
+def test_gqa_workspace_is_bounded_by_64_chunks_per_sequence(lib, b, cols):
+    # 96 / 8 heads, pages of 128: however far the page table reaches, the partials (130 fp32 values per head, query token and
+    # chunk) are those of 64 chunks per sequence at most (and the batch's plan and its alignment)
+    size = gqa_workspace(lib, gqa_specs(b, 1, 96, 8, cols, 128))
+    assert 0 < size <= b * 96 * 64 * 130 * 4 + 4 * b + 1024, size

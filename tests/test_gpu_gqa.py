@@ -158,6 +158,17 @@ def test_keys_beyond_the_last_level_cache(cuda):
     assert torch.equal(near, far)
 
 
+@pytest.mark.parametrize("s1,nq,nkv,act,cols", [(1, 12, 1, [3, 200] * 150 + [9000], 2100), (2, 12, 1, [3, 200] * 150 + [9000], 700),
+                                                (1, 12, 1, [5, 300, 0, 129] * 10, 3000), (2, 24, 2, [700, 4097], 8192), (1, 96, 8, [300] * 40, 1024)])
+def test_page_tables_wider_than_the_contexts(cuda, s1, nq, nkv, act, cols):
+    # a serving loop's page tables, as wide as its longest context may get, over short contexts
+    case = gqa.make_case(len(act), s1, nq, nkv, act, seed=len(act) + cols)
+    bt = case["block_table"]
+    wide = torch.full((len(act), cols), -1, dtype=bt.dtype)
+    wide[:, :bt.shape[1]] = bt
+    check(run(dict(case, block_table=wide), cuda), case, f"{cols} columns, {act[:4]}")
+
+
 def test_cache_without_pages_gives_zeros(cuda):
     # a page table with columns and positive lengths over a cache that holds no page: zero rows, no read of the cache
     case = gqa.make_case(2, 2, 12, 1, [300, 40], seed=9)
