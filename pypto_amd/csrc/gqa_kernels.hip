@@ -29,6 +29,7 @@
 //       index is visited in the order {4g..4g+3, 16+4g..16+4g+3} per lane group g on both operands.
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <type_traits>
 #include <stdint.h>
 
 #include "common.h"
@@ -45,6 +46,11 @@ constexpr int GROW = GD * 2; // bytes per staged V row
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr int GQA_SLOTS = 256;   // one workgroup per CU (two fit; twice as many shorter ones measured 5 to 15 % slower on small batches)
 constexpr int GQA_TARGET = 4096; // tokens a workgroup should have at most, where there are enough
+// Workgroups of a launch at most (or one per KV head, query token and head group): the page tables may reach much further than
+// the contexts do, and a workgroup for every unit they have room for costs 1 us on a CU only to find that it has none.  Then
+// workgroups walk the units (64 sequences of 4096 tokens, 96 / 8 heads, 8192 columns: 234 us with a workgroup per unit, 179 so,
+// 172 under tables of 32 columns; 300 sequences, 12 / 1 heads: 1434, 125 and 119).
+constexpr int GQA_GRID = 2048;
 constexpr int GQA_MAX_SPLIT = 64; // chunks per sequence on average at most, beyond one round of GQA_SLOTS workgroups: the partials
                                   // take memory by the page table's reach (512 sequences, 96 / 8 heads, 1 M tokens: 1.6 GB)
 
@@ -142,17 +148,10 @@ __device__ __forceinline__ int choose_chunk(const GqaArgs& a, const Lengths& ls)
     return hi * 128;
 }
 
-// chunk length, and the (sequence, chunk) of unit u with the sequence's first unit; false: no such unit
-__device__ __forceinline__ bool gqa_unit(const GqaArgs& a, uint32_t unit, int lane, int& chunk, int& bi, int& split)
+// Up to GQA_SCAN sequences: the (sequence, chunk) of unit u, and how many units there are; false: no such unit.  chunk: the
+// chunk length, chosen if it is 0.
+__device__ __forceinline__ bool gqa_unit(const GqaArgs& a, int u, int lane, int& chunk, int& bi, int& split, int64_t& total)
 {
-    chunk = a.chunk;
-    if (a.b > GQA_SCAN) { // (fixed chunks by the unit's place)
-        const uint32_t seq = unit / (uint32_t)a.nsplit;
-        bi = (int)seq;
-        split = (int)(unit - seq * (uint32_t)a.nsplit);
-        return seq < (uint32_t)a.b;
-    }
-    const int u = (int)unit;
     Lengths ls;
     ls.fetch(a, lane);
     if (chunk == 0) chunk = choose_chunk(a, ls);
@@ -161,7 +160,7 @@ __device__ __forceinline__ bool gqa_unit(const GqaArgs& a, uint32_t unit, int la
     bi = -1;
 #pragma unroll
     for (int j = 0; j < GQA_SCAN / 64; ++j) {
-        if (64 * j >= a.b || bi >= 0) break; // uniform
+        if (64 * j >= a.b) break; // uniform
         const int cnt = ls.chunks(j, chunk >> 7, inv_c);
         const int incl = gqa_prefix_sum(cnt), excl = incl - cnt;
         const uint64_t hit = __ballot(u >= base + excl && u < base + incl); // at most one lane
@@ -172,39 +171,78 @@ __device__ __forceinline__ bool gqa_unit(const GqaArgs& a, uint32_t unit, int la
         }
         base += __builtin_amdgcn_readlane(incl, 63);
     }
+    total = (uint32_t)base;
     return bi >= 0;
 }
 
-template <int RT, bool NT>
-__global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a)
+// More sequences: chunks of a fixed length, all sequences' first ones, then their second ones, .. (a walk in steps of a multiple of
+// a sequence's chunks would meet the same chunk of every sequence).  Of the 64 units u, u + stride,
+// .. those that have work, as a bit mask over the lanes: they lie inside their sequence, or are its first.
+__device__ __forceinline__ uint64_t gqa_live_units(const GqaArgs& a, int64_t u, int64_t stride, int lane)
+{
+    const int64_t mine = u + lane * stride;
+    const bool in = mine < a.units_cap;
+    const int64_t split = in ? mine / a.b : 0;
+    const int len = a.act_seq[in ? mine - split * a.b : 0];
+    return __ballot(in && (split == 0 || split * a.chunk < len));
+}
+
+// grid: `stride` units x columns.  WALK: fewer units than there may be; a workgroup takes every stride-th, until there is none.
+template <int RT, bool NT, bool WALK>
+__global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int stride)
 {
     // K and V staging, a pair of sub-tiles per wave; later the merge buffer (4 x 16 x 128 fp32)
     __shared__ __align__(16) uint8_t lds[2 * GWAVES * GSUB * GROW];
     __shared__ float s_ml[GWAVES][16][2];
 
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r16 = lane & 15, g4 = lane >> 4;
-    // Order of the workgroups: eight units side by side, and behind each other those that read the same keys, then the KV
-    // heads, whose rows lie beside each other in the cache.  Workgroups go to the eight dies in turn, so the readers of the
-    // same keys share an L2.
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // Order of the workgroups: eight units (or stride, a power of two, if that is less) side by side, and behind each other
+    // those that read the same keys, then the KV heads, whose rows lie beside each other in the cache.  Workgroups go to the
+    // eight dies in turn, so the readers of the same keys share an L2.
     const int readers = a.s1 * a.hsub / RT;
-    uint32_t u; // (the grid has fewer than 2^32 workgroups)
+    uint32_t first;
     int n2, rd;
     {
-        const uint32_t lin = blockIdx.x + gridDim.x * blockIdx.y, per = 8u * readers * a.nkv;
+        const int sh = stride < 8 ? __builtin_ctz(stride) : 3;
+        const uint32_t lin = blockIdx.x + gridDim.x * blockIdx.y, per = (uint32_t)(readers * a.nkv) << sh;
         const uint32_t o = lin / per, in = lin - o * per;
-        u = o * 8 + (in & 7);
-        rd = (int)((in >> 3) % readers) * RT;
-        n2 = (int)((in >> 3) / readers);
+        first = (o << sh) + (in & ((1u << sh) - 1u));
+        rd = (int)((in >> sh) % readers) * RT;
+        n2 = (int)((in >> sh) / readers);
     }
-    int bi, split, chunk;
-    if (!gqa_unit(a, u, lane, chunk, bi, split)) return;
+    if (first >= (uint32_t)stride) return;
+    const int g = a.nq / a.nkv;
+    int chunk = a.chunk;
+    int64_t at = first, total = a.units_cap; // the next unit to look at; units there are (at most)
+    uint64_t live = 0; // beyond GQA_SCAN sequences: units at - 64 stride + l stride that have work
+    for (bool again = false;; again = true) {
+    int tid = threadIdx.x;
+    if constexpr (WALK) asm volatile("" : "+v"(tid)); // (so that nothing derived from it is kept in registers from one unit to the next)
+    const int lane = tid & 63, r16 = lane & 15, g4 = lane >> 4;
+    int bi, split;
+    int64_t u; // the unit's place in the workspace
+    if (a.b > GQA_SCAN) {
+        while (live == 0) {
+            if (at >= total) return;
+            live = gqa_live_units(a, at, stride, lane);
+            at += 64 * (int64_t)stride;
+        }
+        u = at + (__builtin_ctzll(live) - 64) * (int64_t)stride;
+        live &= live - 1;
+        split = (int)(u / a.b);
+        bi = (int)(u - (int64_t)split * a.b);
+        u = (int64_t)bi * a.nsplit + split;
+    } else {
+        u = at;
+        if (at >= total || !gqa_unit(a, (int)at, lane, chunk, bi, split, total)) return;
+        at += stride;
+    }
+    if (again) __syncthreads(); // (everyone is done with the last unit's merge buffer)
     if (a.part_o != nullptr && tid == 0 && rd == 0 && n2 == 0) { // for the combine kernel
-        if (u == 0) a.plan[0] = chunk;
+        if (bi == 0 && split == 0) a.plan[0] = chunk;
         if (split == 0) a.plan[1 + bi] = (int32_t)u; // (read for up to GQA_SCAN sequences)
     }
 
-    const int g = a.nq / a.nkv;
     const int len = min(a.act_seq[bi], a.bt_stride * a.block_size);
     const int start = split * chunk;
     int tok_q[RT], hs[RT], end_r[RT], end = 0; // row tile r: its query token, head sub-group and end of the chunk
@@ -409,7 +447,7 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a)
                               pack_bf16x2(acc[4] * inv, acc[5] * inv), pack_bf16x2(acc[6] * inv, acc[7] * inv)};
             *reinterpret_cast<u32x4*>(out + head_row * GD + d0) = pk;
         } else {
-            const int64_t slot = ((int64_t)u * a.s1 + (tok_q[r] - bi * a.s1)) * a.nq + n2 * g + hloc;
+            const int64_t slot = (u * a.s1 + (tok_q[r] - bi * a.s1)) * a.nq + n2 * g + hloc;
             float* po = a.part_o + slot * GD + d0;
             *reinterpret_cast<f32x4*>(po) = f32x4{acc[0], acc[1], acc[2], acc[3]};
             *reinterpret_cast<f32x4*>(po + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
@@ -420,6 +458,8 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a)
             }
         }
     }
+    if constexpr (!WALK) break;
+    } // units
 }
 
 // Merges the chunks that hold tokens of a query token: 32 lanes x 4 dims per head row and group of chunks, GROUPS such
@@ -588,13 +628,21 @@ hipError_t gqa_launch(const GqaArgs& a, hipStream_t stream)
     }
     {
         ScopedKernelTimer timer(KID_GQA_DECODE, stream);
-        const int64_t units = (a.units_cap + 7) / 8 * 8;
-        const int64_t groups = units * a.columns;
+        // as many units side by side as there can be, but no more than GQA_GRID workgroups
+        int64_t stride = (a.units_cap + 7) / 8 * 8;
+        if (stride * a.columns > GQA_GRID) {
+            stride = std::max(GQA_GRID / a.columns, 1);
+            stride = stride >= 8 ? stride / 8 * 8 : stride >= 4 ? 4 : stride >= 2 ? 2 : 1;
+        }
+        const int64_t groups = stride * a.columns;
         const int64_t gx = groups < (1 << 22) ? groups : (1 << 22);
-        if (groups + gx > 0xffffffffll) return hipErrorInvalidValue; // (partials of over 2 TB)
-        auto kern = a.row_tiles == 2 ? (a.stream_past_cache ? gqa_decode_kernel<2, true> : gqa_decode_kernel<2, false>)
-                                     : (a.stream_past_cache ? gqa_decode_kernel<1, true> : gqa_decode_kernel<1, false>);
-        hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)((groups + gx - 1) / gx)), dim3(256), 0, stream, a);
+        auto kern = [&](auto walk) {
+            constexpr bool W = decltype(walk)::value;
+            return a.row_tiles == 2 ? (a.stream_past_cache ? gqa_decode_kernel<2, true, W> : gqa_decode_kernel<2, false, W>)
+                                    : (a.stream_past_cache ? gqa_decode_kernel<1, true, W> : gqa_decode_kernel<1, false, W>);
+        };
+        hipLaunchKernelGGL((stride < a.units_cap ? kern(std::true_type{}) : kern(std::false_type{})),
+                           dim3((unsigned)gx, (unsigned)((groups + gx - 1) / gx)), dim3(256), 0, stream, a, (int)stride);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.nsplit == 1) return e;

@@ -169,6 +169,35 @@ def test_page_tables_wider_than_the_contexts(cuda, s1, nq, nkv, act, cols):
     check(run(dict(case, block_table=wide), cuda), case, f"{cols} columns, {act[:4]}")
 
 
+def test_wide_page_tables_do_not_cost_workgroups(cuda):
+    """300 sequences of 1024 tokens: tables of 8192 columns may cost a little over tables of 8, not a workgroup for each of the
+    77 K chunks they have room for (which took over ten times the narrow tables' time)."""
+    from pypto_amd.glm_v4_5 import glm_attention as impl
+    b, pages = 300, 8
+    g = torch.Generator(device="cuda").manual_seed(1)
+    k, v = (torch.randn(b * pages, 128, 1, 128, generator=g, device=cuda).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(b, 12, 128, generator=g, device=cuda).to(torch.bfloat16)
+    act = torch.full((b,), 128 * pages, dtype=torch.int32, device=cuda)
+    narrow = torch.arange(b * pages, dtype=torch.int32, device=cuda).view(b, pages)
+    wide = torch.full((b, 8192), -1, dtype=torch.int32, device=cuda)
+    wide[:, :pages] = narrow
+
+    def time(table):
+        out, cfg = torch.empty_like(q), impl.IfaTileShapeConfig()
+        best = math.inf
+        for _ in range(5):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(5):
+                impl.attention(q, k, v, table, act, out, 128 ** -0.5, cfg)
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, start.elapsed_time(end))
+        return best
+
+    assert time(wide) < 3 * time(narrow)
+
+
 def test_cache_without_pages_gives_zeros(cuda):
     # a page table with columns and positive lengths over a cache that holds no page: zero rows, no read of the cache
     case = gqa.make_case(2, 2, 12, 1, [300, 40], seed=9)
