@@ -14,7 +14,9 @@
 //   Loads take whole 256-byte cache rows, four to an instruction.  (K in the operand's layout straight from memory takes half
 // cache lines, twice, from 16 rows: 868 us against 853 at 4.8 GB, and unusable without cache retention.)
 //   Where the batch's keys do not fit the 256 MB last-level cache, they are loaded past it (non-temporal; a plain read
-// stream reaches 6.3 TB/s on this card, a non-temporal one 7.1): 853 -> 800 us.  Where they fit, the caches serve part of it.
+// stream reaches 6.3 TB/s on this card, a non-temporal one 7.1): 853 -> 800 us.  Where they fit, the caches serve part of it
+// (197 MB, two query tokens a sequence: 42 us through the caches, 47 past them).  The lengths decide, not the page tables'
+// reach; the whole sweep exists twice, since a choice at every sub-tile's loads costs 0.5 us at 33 MB (13.4 -> 14.0).
 //   The page-table entries of 64 pages are held by a wavefront's lanes: a look-up from memory in front of every sub-tile
 // waited for the sub-tile in flight as well (loads complete in order): 1077 -> 868 us.
 //   Chunks are chosen on the device from the lengths (choose_chunk): as long as they can be while the workgroups fill the
@@ -44,6 +46,7 @@ constexpr int GSUB = 32;     // tokens per wave sub-tile
 constexpr int GWAVES = 4;
 constexpr int GROW = GD * 2; // bytes per staged V row
 constexpr float LOG2E = 1.4426950408889634f;
+constexpr float GQA_CACHED = 256e6f; // bytes of keys and values that the last-level cache holds
 constexpr int GQA_SLOTS = 256;   // one workgroup per CU (two fit; twice as many shorter ones measured 5 to 15 % slower on small batches)
 constexpr int GQA_TARGET = 4096; // tokens a workgroup should have at most, where there are enough
 // Workgroups of a launch at most (or one per KV head, query token and head group): the page tables may reach much further than
@@ -85,7 +88,7 @@ __device__ __forceinline__ int gqa_prefix_sum(int v)
 }
 
 // The lengths of up to GQA_SCAN sequences, by one wavefront: lane l holds those of sequences l, l + 64, ..  (cut to the page
-// table's reach; -1 past the last sequence).
+// table's reach; -1 past the last sequence); of more, those of GQA_SCAN evenly spaced ones.
 constexpr int GQA_SCAN = 256;
 struct Lengths {
     int len[GQA_SCAN / 64];
@@ -93,7 +96,10 @@ struct Lengths {
     {
         const int reach = a.bt_stride * a.block_size;
 #pragma unroll
-        for (int j = 0; j < GQA_SCAN / 64; ++j) len[j] = 64 * j < a.b ? a.act_seq[min(lane + 64 * j, a.b - 1)] : 0; // (requested together)
+        for (int j = 0; j < GQA_SCAN / 64; ++j) { // (requested together)
+            const int i = lane + 64 * j;
+            len[j] = 64 * j < a.b ? a.act_seq[a.b > GQA_SCAN ? (int)((int64_t)i * a.b / GQA_SCAN) : min(i, a.b - 1)] : 0;
+        }
 #pragma unroll
         for (int j = 0; j < GQA_SCAN / 64; ++j) len[j] = lane + 64 * j < a.b ? max(min(len[j], reach), 0) : -1;
     }
@@ -107,7 +113,21 @@ struct Lengths {
         q += r < 0 ? -1 : r >= c ? 1 : 0;
         return len[j] < 0 ? 0 : max(1, q);
     }
-    // of all sequences (256 sequences of 2^30 tokens have 2^31 chunks of 128: unsigned)
+    // tokens, in units of 128 (256 sequences of 2^30 have 2^31: unsigned)
+    __device__ __forceinline__ uint32_t sum() const
+    {
+        int n = 0;
+#pragma unroll
+        for (int j = 0; j < GQA_SCAN / 64; ++j) n += (max(len[j], 0) + 127) >> 7;
+        return (uint32_t)__builtin_amdgcn_readlane(gqa_prefix_sum(n), 63);
+    }
+    // whether the batch's keys and values are to be loaded past the caches
+    __device__ __forceinline__ bool past_caches(const GqaArgs& a) const
+    {
+        const float seqs = a.b > GQA_SCAN ? (float)a.b / GQA_SCAN : 1.f;
+        return (float)sum() * seqs * (float)a.nkv * (128.f * 2 * GROW) > GQA_CACHED;
+    }
+    // chunks of all sequences
     __device__ __forceinline__ uint32_t units(const GqaArgs& a, int c) const
     {
         const float inv_c = 1.f / (float)c;
@@ -125,14 +145,13 @@ struct Lengths {
 // Depends on the lengths alone, so every wavefront finds the same one; the result never exceeds units_cap units.
 __device__ __forceinline__ int choose_chunk(const GqaArgs& a, const Lengths& ls)
 {
-    int mine = 0, longest = 0;
+    int longest = 0;
 #pragma unroll
     for (int j = 0; j < GQA_SCAN / 64; ++j) {
         if (64 * j >= a.b) break; // (uniform)
-        mine += (max(ls.len[j], 0) + 127) >> 7;
         longest = max(longest, ls.len[j]);
     }
-    const uint32_t sum = (uint32_t)__builtin_amdgcn_readlane(gqa_prefix_sum(mine), 63);
+    const uint32_t sum = ls.sum();
     // rounds of GQA_SLOTS workgroups with GQA_TARGET tokens (of at most 2^22, so that their slots fit 32 bits)
     const int rounds = (int)fminf(fmaxf(ceilf((float)sum * (float)a.columns * (128.f / GQA_SLOTS / GQA_TARGET)), 1.f), 0x1p22f);
     const uint32_t target = (uint32_t)min(max(rounds * GQA_SLOTS / a.columns, a.b), (int)a.units_cap);
@@ -150,10 +169,8 @@ __device__ __forceinline__ int choose_chunk(const GqaArgs& a, const Lengths& ls)
 
 // Up to GQA_SCAN sequences: the (sequence, chunk) of unit u, and how many units there are; false: no such unit.  chunk: the
 // chunk length, chosen if it is 0.
-__device__ __forceinline__ bool gqa_unit(const GqaArgs& a, int u, int lane, int& chunk, int& bi, int& split, int64_t& total)
+__device__ __forceinline__ bool gqa_unit(const GqaArgs& a, const Lengths& ls, int u, int& chunk, int& bi, int& split, int64_t& total)
 {
-    Lengths ls;
-    ls.fetch(a, lane);
     if (chunk == 0) chunk = choose_chunk(a, ls);
     const float inv_c = 1.f / (float)(chunk >> 7);
     int base = 0;
@@ -187,8 +204,8 @@ __device__ __forceinline__ uint64_t gqa_live_units(const GqaArgs& a, int64_t u, 
     return __ballot(in && (split == 0 || split * a.chunk < len));
 }
 
-// grid: `stride` units x columns.  WALK: fewer units than there may be; a workgroup takes every stride-th, until there is none.
-template <int RT, bool NT, bool WALK>
+// grid: `stride` units x columns.  MAY: a batch that fills its page tables is loaded past the caches.  WALK: fewer units than there may be; a workgroup takes every stride-th, until there is none.
+template <int RT, bool WALK, bool MAY>
 __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int stride)
 {
     // K and V staging, a pair of sub-tiles per wave; later the merge buffer (4 x 16 x 128 fp32)
@@ -219,6 +236,8 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
     int tid = threadIdx.x;
     if constexpr (WALK) asm volatile("" : "+v"(tid)); // (so that nothing derived from it is kept in registers from one unit to the next)
     const int lane = tid & 63, r16 = lane & 15, g4 = lane >> 4;
+    Lengths ls;
+    ls.fetch(a, lane);
     int bi, split;
     int64_t u; // the unit's place in the workspace
     if (a.b > GQA_SCAN) {
@@ -234,9 +253,10 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
         u = (int64_t)bi * a.nsplit + split;
     } else {
         u = at;
-        if (at >= total || !gqa_unit(a, (int)at, lane, chunk, bi, split, total)) return;
+        if (at >= total || !gqa_unit(a, ls, (int)at, chunk, bi, split, total)) return;
         at += stride;
     }
+    const bool past_caches = MAY && ls.past_caches(a); // uniform
     if (again) __syncthreads(); // (everyone is done with the last unit's merge buffer)
     if (a.part_o != nullptr && tid == 0 && rd == 0 && n2 == 0) { // for the combine kernel
         if (bi == 0 && split == 0) a.plan[0] = chunk;
@@ -299,7 +319,7 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
         entry = e >= 0 && e < a.n_blocks ? e : -1;
     };
     if (nsub > 0) fetch_entries();
-    auto load = [&](int i, SubTile& t) {
+    auto load = [&](int i, SubTile& t, auto past) {
         const int p0 = start + GSUB * i;
         const int page = p0 / a.block_size;
         if (page - window >= 64) { // (uniform; chunks of more than 64 pages)
@@ -311,7 +331,7 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
         const int64_t row0 = (int64_t)max(blk, 0) * a.block_size + (p0 - page * a.block_size);
         auto row = [&](const uint8_t* base, int i8) {
             const u32x4* p = reinterpret_cast<const u32x4*>(base + (row0 + 4 * i8 + g4) * row_pitch + r16 * 16);
-            return NT ? __builtin_nontemporal_load(p) : *p;
+            return decltype(past)::value ? __builtin_nontemporal_load(p) : *p;
         };
 #pragma unroll
         for (int i8 = 0; i8 < 8; ++i8) t.k[i8] = row(kbase, i8);
@@ -390,18 +410,22 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
         }
     };
 
-    if (w < nsub) {
+    auto sweep = [&](auto past) { // past: loads past the caches
         SubTile t;
         int i = w;
-        load(i, t);
+        load(i, t, past);
         for (; i + GWAVES < nsub; i += GWAVES) {
             const bool mapped = t.mapped;
             stage(t);
-            load(i + GWAVES, t);
+            load(i + GWAVES, t, past);
             compute(i, mapped);
         }
         stage(t);
         compute(i, t.mapped);
+    };
+    if (w < nsub) {
+        if (past_caches) sweep(std::true_type{});
+        else sweep(std::false_type{});
     }
 
     // merge the four waves
@@ -594,7 +618,7 @@ void gqa_plan(GqaArgs& a, int forced_chunk)
         a.nsplit = n < 1 ? 1 : (int32_t)n;
         a.units_cap = a.b * (int64_t)a.nsplit;
     }
-    a.stream_past_cache = (double)t / (a.s1 > 0 ? a.s1 : 1) * (double)max_ctx * a.nkv * 2 * GROW > 256e6;
+    a.past_caches = (double)a.b * (double)max_ctx * a.nkv * 2 * GROW > GQA_CACHED;
 }
 
 static uint64_t gqa_align(uint64_t x) { return (x + 255) & ~(uint64_t)255; }
@@ -638,8 +662,8 @@ hipError_t gqa_launch(const GqaArgs& a, hipStream_t stream)
         const int64_t gx = groups < (1 << 22) ? groups : (1 << 22);
         auto kern = [&](auto walk) {
             constexpr bool W = decltype(walk)::value;
-            return a.row_tiles == 2 ? (a.stream_past_cache ? gqa_decode_kernel<2, true, W> : gqa_decode_kernel<2, false, W>)
-                                    : (a.stream_past_cache ? gqa_decode_kernel<1, true, W> : gqa_decode_kernel<1, false, W>);
+            return a.row_tiles == 2 ? (a.past_caches ? gqa_decode_kernel<2, W, true> : gqa_decode_kernel<2, W, false>)
+                                    : (a.past_caches ? gqa_decode_kernel<1, W, true> : gqa_decode_kernel<1, W, false>);
         };
         hipLaunchKernelGGL((stride < a.units_cap ? kern(std::true_type{}) : kern(std::false_type{})),
                            dim3((unsigned)gx, (unsigned)((groups + gx - 1) / gx)), dim3(256), 0, stream, a, (int)stride);

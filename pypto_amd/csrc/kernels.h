@@ -104,7 +104,7 @@ struct GqaArgs {
     // 16-row tiles per workgroup, workgroups per unit
     int32_t nsplit, chunk, row_tiles, columns;
     int64_t units_cap; // set by gqa_plan: units of the batch at most (beyond 32 bits with short forced chunks under a wide page table)
-    bool stream_past_cache;     // set by gqa_plan
+    bool past_caches;           // set by gqa_plan: a batch that fills its page tables is loaded past the caches
     float softmax_scale;
 };
 
