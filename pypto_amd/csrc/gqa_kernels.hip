@@ -49,11 +49,15 @@ constexpr float LOG2E = 1.4426950408889634f;
 constexpr float GQA_CACHED = 256e6f; // bytes of keys and values that the last-level cache holds
 constexpr int GQA_SLOTS = 256;   // one workgroup per CU (two fit; twice as many shorter ones measured 5 to 15 % slower on small batches)
 constexpr int GQA_TARGET = 4096; // tokens a workgroup should have at most, where there are enough
+constexpr int GQA_TARGET2 = 1024; // and with two row tiles (more only where that would be over GQA_MAX_SPLIT chunks): a wavefront's
+                                  // running sums span 256 tokens, and there are no registers for PIECES (4096: 4 to 10 % faster)
 // Workgroups of a launch at most (or one per KV head, query token and head group): the page tables may reach much further than
 // the contexts do, and a workgroup for every unit they have room for costs 1 us on a CU only to find that it has none.  Then
 // workgroups walk the units (64 sequences of 4096 tokens, 96 / 8 heads, 8192 columns: 234 us with a workgroup per unit, 179 so,
 // 172 under tables of 32 columns; 300 sequences, 12 / 1 heads: 1434, 125 and 119).
-constexpr int GQA_GRID = 2048;
+// With two row tiles the chunks are shorter and a workgroup to each is the better way up to 8192 of them (32 sequences of 16000
+// tokens, two query tokens, 96 / 8 heads, 4096 chunks: 400 us, 415 by a walk).
+constexpr int GQA_GRID = 2048, GQA_GRID2 = 8192;
 constexpr int GQA_MAX_SPLIT = 64; // chunks per sequence on average at most, beyond one round of GQA_SLOTS workgroups: the partials
                                   // take memory by the page table's reach (512 sequences, 96 / 8 heads, 1 M tokens: 1.6 GB)
 
@@ -153,7 +157,8 @@ __device__ __forceinline__ int choose_chunk(const GqaArgs& a, const Lengths& ls)
     }
     const uint32_t sum = ls.sum();
     // rounds of GQA_SLOTS workgroups with GQA_TARGET tokens (of at most 2^22, so that their slots fit 32 bits)
-    const int rounds = (int)fminf(fmaxf(ceilf((float)sum * (float)a.columns * (128.f / GQA_SLOTS / GQA_TARGET)), 1.f), 0x1p22f);
+    const float slot = (float)min(a.longest, GQA_TARGET) * (GQA_SLOTS / 128.f);
+    const int rounds = (int)fminf(fmaxf(ceilf((float)sum * (float)a.columns / slot), 1.f), 0x1p22f);
     const uint32_t target = (uint32_t)min(max(rounds * GQA_SLOTS / a.columns, a.b), (int)a.units_cap);
     int lo = max((int)((sum + target - 1) / target), 1); // (no shorter chunk can do)
     if (ls.units(a, lo) <= target) return lo * 128;
@@ -171,7 +176,7 @@ __device__ __forceinline__ int choose_chunk(const GqaArgs& a, const Lengths& ls)
 // chunk length, chosen if it is 0.
 __device__ __forceinline__ bool gqa_unit(const GqaArgs& a, const Lengths& ls, int u, int& chunk, int& bi, int& split, int64_t& total)
 {
-    if (chunk == 0) chunk = choose_chunk(a, ls);
+    if (chunk == 0) chunk = min(choose_chunk(a, ls), a.longest);
     const float inv_c = 1.f / (float)(chunk >> 7);
     int base = 0;
     bi = -1;
@@ -293,6 +298,7 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
     const uint8_t* kbase = static_cast<const uint8_t*>(a.k) + (int64_t)n2 * GROW;
     const uint8_t* vbase = static_cast<const uint8_t*>(a.v) + (int64_t)n2 * GROW;
     const int64_t row_pitch = (int64_t)a.nkv * GROW;
+    const uint32_t lane_at = (uint32_t)(g4 * (int)row_pitch + r16 * 16); // (nkv is below 2^15)
     const int32_t* bt = a.block_table + (int64_t)bi * a.bt_stride;
     uint8_t* myk = lds + 2 * w * (GSUB * GROW);
     uint8_t* myv = myk + GSUB * GROW;
@@ -300,8 +306,17 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
     const int nsub = (max(end - start, 0) + GSUB - 1) / GSUB;
     const float sc = a.softmax_scale * LOG2E;
 
-    f32x4 o[RT][8];
-    float m_run[RT], l_run[RT];
+    // Sums of the last sub-tiles, up to PIECE of them, and of those before: a chain of the 32 sub-tiles that a wavefront has in
+    // a chunk of 4096 tokens was 25 % further off in fp32 (times are the same).
+    constexpr bool PIECES = RT == 1;
+    constexpr int PIECE = 8;
+    f32x4 o[RT][8], o_before[PIECES ? 8 : 1];
+    float m_run[RT], l_run[RT], l_before = 0.f;
+    int in_piece = 0;
+    if constexpr (PIECES) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o_before[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
 #pragma unroll
@@ -319,7 +334,7 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
         entry = e >= 0 && e < a.n_blocks ? e : -1;
     };
     if (nsub > 0) fetch_entries();
-    auto load = [&](int i, SubTile& t, auto past) {
+    auto load = [&](int i, SubTile& t, auto past) __attribute__((always_inline)) {
         const int p0 = start + GSUB * i;
         const int page = p0 / a.block_size;
         if (page - window >= 64) { // (uniform; chunks of more than 64 pages)
@@ -328,9 +343,9 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
         }
         const int blk = __builtin_amdgcn_readlane(entry, page - window);
         t.mapped = blk >= 0; // an unmapped page is masked in compute(); its loads stay in bounds
-        const int64_t row0 = (int64_t)max(blk, 0) * a.block_size + (p0 - page * a.block_size);
+        const int64_t at0 = ((int64_t)max(blk, 0) * a.block_size + (p0 - page * a.block_size)) * row_pitch; // uniform
         auto row = [&](const uint8_t* base, int i8) {
-            const u32x4* p = reinterpret_cast<const u32x4*>(base + (row0 + 4 * i8 + g4) * row_pitch + r16 * 16);
+            const u32x4* p = reinterpret_cast<const u32x4*>(base + at0 + 4 * i8 * row_pitch + lane_at);
             return decltype(past)::value ? __builtin_nontemporal_load(p) : *p;
         };
 #pragma unroll
@@ -338,7 +353,7 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
 #pragma unroll
         for (int i8 = 0; i8 < 8; ++i8) t.v[i8] = row(vbase, i8);
     };
-    auto stage = [&](const SubTile& t) {
+    auto stage = [&](const SubTile& t) __attribute__((always_inline)) {
 #pragma unroll
         for (int i8 = 0; i8 < 8; ++i8) {
             const int tv = 4 * i8 + g4;
@@ -351,21 +366,24 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
         }
     };
 
-    auto compute = [&](int i, bool mapped) {
+    auto compute = [&](int i, bool mapped) __attribute__((always_inline)) {
         const int p0 = start + GSUB * i;
+        int krow = r16;
+        if constexpr (RT > 1) asm volatile("" : "+v"(krow)); // (the reads' addresses anew for every sub-tile, not in registers)
         f32x4 s0[RT], s1[RT];
 #pragma unroll
         for (int r = 0; r < RT; ++r) s0[r] = s1[r] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(myk + r16 * GROW + vswz(r16, g4 + 4 * j));
-            const bf16x8 k1 = *reinterpret_cast<const bf16x8*>(myk + (r16 + 16) * GROW + vswz(r16, g4 + 4 * j));
+            const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(myk + krow * GROW + vswz(krow, g4 + 4 * j));
+            const bf16x8 k1 = *reinterpret_cast<const bf16x8*>(myk + (krow + 16) * GROW + vswz(krow, g4 + 4 * j));
 #pragma unroll
             for (int r = 0; r < RT; ++r) {
                 s0[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, __builtin_bit_cast(bf16x8, qf[r][j]), s0[r], 0, 0, 0);
                 s1[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, __builtin_bit_cast(bf16x8, qf[r][j]), s1[r], 0, 0, 0);
             }
         }
+        if constexpr (RT > 1) __builtin_amdgcn_sched_barrier(0);
         u32x4 pf[RT];
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
@@ -391,13 +409,19 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
             }
             l_run[r] = l_run[r] * alpha + psum;
             m_run[r] = m_new;
+            if constexpr (PIECES) l_before *= alpha;
             if (__any(alpha != 1.f)) {
 #pragma unroll
-                for (int db = 0; db < 8; ++db) o[r][db] *= alpha;
+                for (int db = 0; db < 8; ++db) {
+                    o[r][db] *= alpha;
+                    if constexpr (PIECES) o_before[db] *= alpha;
+                }
             }
             pf[r] = u32x4{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]), pack_bf16x2(p[6], p[7])};
         }
-        const int tok_lo = 4 * g4 + (r16 >> 2);
+        if constexpr (RT > 1) __builtin_amdgcn_sched_barrier(0);
+        int tok_lo = 4 * g4 + (r16 >> 2);
+        if constexpr (RT > 1) asm volatile("" : "+v"(tok_lo)); // (likewise)
 #pragma unroll
         for (int db = 0; db < 8; ++db) {
             const s16x4 lo = lds_read_tr(myv + tok_lo * GROW + ((db ^ (tok_lo & 7)) << 5) + (r16 & 3) * 8);
@@ -408,9 +432,21 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
                 o[r][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, both),
                                                                    __builtin_bit_cast(bf16x8, pf[r]), o[r][db], 0, 0, 0);
         }
+        if constexpr (PIECES) {
+            if (++in_piece == PIECE) { // uniform
+                in_piece = 0;
+#pragma unroll
+                for (int db = 0; db < 8; ++db) {
+                    o_before[db] += o[0][db];
+                    o[0][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+                l_before += l_run[0];
+                l_run[0] = 0.f;
+            }
+        }
     };
 
-    auto sweep = [&](auto past) { // past: loads past the caches
+    auto sweep = [&](auto past) __attribute__((always_inline)) { // past: loads past the caches
         SubTile t;
         int i = w;
         load(i, t, past);
@@ -428,6 +464,11 @@ __global__ __launch_bounds__(256, 2) void gqa_decode_kernel(GqaArgs a, int strid
         else sweep(std::false_type{});
     }
 
+    if constexpr (PIECES) {
+#pragma unroll
+        for (int db = 0; db < 8; ++db) o[0][db] += o_before[db];
+        l_run[0] += l_before;
+    }
     // merge the four waves
     float* mo = reinterpret_cast<float*>(lds);
 #pragma unroll
@@ -595,13 +636,14 @@ void gqa_plan(GqaArgs& a, int forced_chunk)
     }
     a.row_tiles = a.s1 * a.hsub % 2 == 0 ? 2 : 1;
     a.columns = (int32_t)((int64_t)a.nkv * a.s1 * a.hsub / a.row_tiles);
+    const int64_t least = ((max_ctx + GQA_MAX_SPLIT - 1) / GQA_MAX_SPLIT + 127) / 128 * 128;
+    a.longest = a.row_tiles == 1 ? INT32_MAX : (int32_t)std::max<int64_t>(GQA_TARGET2, least);
     if (forced_chunk > 0) {
         a.chunk = (forced_chunk + 127) / 128 * 128;
     } else if (a.b > GQA_SCAN) {
-        const int64_t least = (max_ctx + GQA_MAX_SPLIT - 1) / GQA_MAX_SPLIT;
-        a.chunk = least > GQA_TARGET ? (int32_t)((least + 127) / 128 * 128) : GQA_TARGET;
+        a.chunk = a.row_tiles == 1 ? (int32_t)std::max<int64_t>(GQA_TARGET, least) : a.longest;
     } else {
-        const int64_t round = (int64_t)GQA_SLOTS * (GQA_TARGET / 128);
+        const int64_t round = (int64_t)GQA_SLOTS * (std::min(a.longest, GQA_TARGET) / 128);
         const int64_t work = (int64_t)a.b * ((max_ctx + 127) / 128) * a.columns;
         const int64_t rounds = (work + round - 1) / round;
         int64_t target = (rounds > 1 ? rounds : 1) * GQA_SLOTS / a.columns;
@@ -609,7 +651,7 @@ void gqa_plan(GqaArgs& a, int forced_chunk)
         const int64_t one_round = std::min<int64_t>(GQA_SLOTS / a.columns, 2 * GQA_MAX_SPLIT * (int64_t)a.b);
         target = std::min(std::min(target, std::max(one_round, GQA_MAX_SPLIT * (int64_t)a.b)), pages);
         a.chunk = 0; // chosen on the device
-        a.units_cap = target > a.b ? target : a.b;
+        a.units_cap = std::max(target, a.b * std::max<int64_t>(1, (max_ctx + a.longest - 1) / a.longest));
         a.nsplit = a.units_cap > a.b ? 2 : 1;
         if (a.nsplit == 1) a.chunk = (int32_t)((max_ctx + 127) / 128 * 128);
     }
@@ -654,8 +696,9 @@ hipError_t gqa_launch(const GqaArgs& a, hipStream_t stream)
         ScopedKernelTimer timer(KID_GQA_DECODE, stream);
         // as many units side by side as there can be, but no more than GQA_GRID workgroups
         int64_t stride = (a.units_cap + 7) / 8 * 8;
-        if (stride * a.columns > GQA_GRID) {
-            stride = std::max(GQA_GRID / a.columns, 1);
+        const int64_t most = a.row_tiles == 1 ? GQA_GRID : GQA_GRID2;
+        if (stride * a.columns > most) {
+            stride = std::max<int64_t>(most / a.columns, 1);
             stride = stride >= 8 ? stride / 8 * 8 : stride >= 4 ? 4 : stride >= 2 ? 2 : 1;
         }
         const int64_t groups = stride * a.columns;

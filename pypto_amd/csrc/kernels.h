@@ -103,6 +103,7 @@ struct GqaArgs {
     // set by gqa_plan: chunks per sequence (at most; > 1: the combine kernel runs), chunk length (0: chosen on the device),
     // 16-row tiles per workgroup, workgroups per unit
     int32_t nsplit, chunk, row_tiles, columns;
+    int32_t longest; // set by gqa_plan: the longest chunk that may be chosen
     int64_t units_cap; // set by gqa_plan: units of the batch at most (beyond 32 bits with short forced chunks under a wide page table)
     bool past_caches;           // set by gqa_plan: a batch that fills its page tables is loaded past the caches
     float softmax_scale;

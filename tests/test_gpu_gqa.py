@@ -169,6 +169,40 @@ def test_page_tables_wider_than_the_contexts(cuda, s1, nq, nkv, act, cols):
     check(run(dict(case, block_table=wide), cuda), case, f"{cols} columns, {act[:4]}")
 
 
+@pytest.mark.parametrize("s1,b", [(1, 64), (2, 60)])
+def test_running_sums_span_256_tokens(cuda, s1, b):
+    """The weighted sums of long chunks are added up in pieces.  With equal weights and values that come in pairs v, -v the
+    exact result is 0, so the output is the rounding error alone.  Modelled on the CPU: four wavefronts take every fourth of
+    128 32-token tiles, exact within a tile, rounded to fp32 once at each addition, in one chain of 32.  Pieces of eight
+    tiles stay some 10 % below that although the matrix instructions round more often; one chain is 6 to 14 % above it."""
+    from pypto_amd.glm_v4_5 import glm_attention as impl
+    n, nkv, pages = 4096, 4, 32
+    g = torch.Generator().manual_seed(7)
+
+    def values(cols):
+        v = torch.randn(n // 2, cols, generator=g).to(torch.bfloat16)
+        return torch.cat([v, -v])[torch.randperm(n, generator=g)]
+
+    merged = torch.zeros(4096)
+    tiles = values(4096).double().view(n // 32, 32, 4096).sum(1)
+    for w in range(4):
+        run = torch.zeros(4096)
+        for t in tiles[w::4]:
+            run = (run.double() + t).float()
+        merged = merged + run
+    model = float(merged.double().pow(2).mean().sqrt())
+
+    v = values(nkv * 128).view(pages, 128, nkv, 128).to(cuda)
+    k = torch.randn(pages, 128, nkv, 128, generator=g).to(torch.bfloat16).to(cuda)
+    q = torch.zeros(b * s1, nkv, 128, dtype=torch.bfloat16, device=cuda)
+    order = torch.stack([torch.randperm(pages, generator=g) for _ in range(b)]).to(torch.int32)
+    table = torch.cat([order, order[:, :s1 - 1]], dim=1).contiguous().to(cuda)   # (the tokens after the first query's)
+    out = torch.empty_like(q)
+    impl.attention(q, k, v, table, torch.full((b,), n + s1 - 1, dtype=torch.int32, device=cuda), out, 0.1, impl.IfaTileShapeConfig())
+    err = float((out.view(b, s1, nkv, 128)[:, 0].double() * n).pow(2).mean().sqrt())
+    assert 0 < err <= model, (err, model)
+
+
 def test_wide_page_tables_do_not_cost_workgroups(cuda):
     """300 sequences of 1024 tokens: tables of 8192 columns may cost a little over tables of 8, not a workgroup for each of the
     77 K chunks they have room for (which took over ten times the narrow tables' time)."""
