@@ -28,6 +28,9 @@
 // the tie list by radix-selecting on the 64-bit words (key << 32 | ~index) (so equal keys resolve to the
 // smaller index), and bitonic-sorts the k words.  A tie list that overflowed its capacity (e.g. all scores
 // equal) falls back to radix-selecting over the whole score row.
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
 #include "timing.h"
@@ -47,6 +50,9 @@ constexpr int SEL_CHUNK = 4096; // scores per workgroup of the select kernel
 constexpr int TIE_CAP = 8192;   // capacity of the per-row tie list
 constexpr int INDEXER_ROW_MAX = 32768; // rows up to this length are selected by one kernel (indexer_row_topk_kernel)
 constexpr int SCORE_GROUPS = 512; // workgroups of the paged score kernel below which its spans are made shorter
+constexpr int SCORE_GROUPS_MIN = 384; // and below which they are made shorter because the contexts are (96 sequences of 1500 .. 16000 keys: 422
+                                      // workgroups of four passes 33.6 us, 900 of two, more than fit the CUs at once, 39.4)
+constexpr float SCORE_CACHED = 96e6f; // bytes of a batch's keys from which they are loaded past the last-level cache
 
 __device__ __forceinline__ float f16_bits_to_f32(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
 // A scale as it lies in memory (fp16 bits, or fp32 in the fp32-scale variant) and as the fp32 factor it stands for.
@@ -145,9 +151,10 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v)
 }
 
 // The workgroup's histograms (S1 query tokens, one span of keys) go to its own slots, as 16-bit counts (a span has at
-// most 4096 keys), two per lane.  The span-0 workgroup also clears the select kernel's list counters of its query tokens.  256 lanes.
+// most 4096 keys), two per lane.  The span-0 workgroup also clears the select kernel's list counters of its query tokens and
+// leaves it the (logarithm of the) passes of a span.  256 lanes.
 template <int S1>
-__device__ __forceinline__ void flush_span_hist(const IndexerArgs& a, const uint32_t (*hist)[SBINS], int row0, int span, int tid)
+__device__ __forceinline__ void flush_span_hist(const IndexerArgs& a, const uint32_t (*hist)[SBINS], int row0, int span, int passes_log2, int tid)
 {
     if (tid < SBINS / 2) {
 #pragma unroll
@@ -157,6 +164,7 @@ __device__ __forceinline__ void flush_span_hist(const IndexerArgs& a, const uint
         }
     }
     if (span == 0 && tid < 4 * S1) a.counters[(int64_t)row0 * 4 + tid] = 0u;
+    if (span == 0 && tid == 0) *a.passes_log2 = (uint32_t)passes_log2; // (every sequence's workgroup writes the same)
 }
 
 // S1 query tokens of one sequence share every key fragment.
@@ -260,7 +268,7 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a)
     }
     } // pass
     __syncthreads();
-    if (a.use_hist) flush_span_hist<S1>(a, hist, row0, (int)blockIdx.x, tid);
+    if (a.use_hist) flush_span_hist<S1>(a, hist, row0, (int)blockIdx.x, __builtin_ctz(PASSES), tid);
 }
 
 // relu(a) * 2^-11 and relu(b) * 2^-11, each rounded once to fp16, packed (a in the low half).  The int32 sums arrive
@@ -287,14 +295,17 @@ __device__ __forceinline__ uint32_t relu_scale_pack(int a, int b)
 // in every row of the head-sum operand, so every lane group holds the 16 scores of a key group and lane group g keeps those
 // of key group g - after four key groups lane l holds the score of key l of the 64, next to that key's scale (loaded with one
 // 128-byte instruction per 64 keys).
-// PPASSES: passes (of 512 keys) per workgroup, pick_passes' choice.  NT: loads past the caches' retention, for batches whose
-// keys do not fit the last-level cache - which needs the whole-row loads: taken in operand layout, a row is two loads of
-// half a cache line, and a line that is not kept in between is fetched twice (32 x 64 K keys, 272 MB: 56.8 us in operand
-// layout, 65.0 with non-temporal loads; 57.8 and 52.7 this way).
-template <int S1, bool F32, int PPASSES, bool NT>
+// A workgroup takes `passes` passes of 512 keys, as score_passes has it for the batch's lengths: PPASSES, what it has for full
+// page tables, or fewer (where the selection needs the spans' histograms, no fewer than there are slots for).  Short contexts under
+// wide tables would otherwise be few long workgroups (32 sequences of 8192 keys under 1024 columns: 24.7 us with spans of
+// 4096 keys).
+// MAY: loads past the caches' retention, where the batch's keys do not fit the last-level cache - which needs the whole-row
+// loads: taken in operand layout, a row is two loads of half a cache line, and a line that is not kept in between is fetched
+// twice (32 x 64 K keys, 272 MB: 56.8 us in operand layout, 65.0 with non-temporal loads; 57.8 and 52.7 this way).
+constexpr int SCAN_SEQS = 256; // sequences whose lengths a wavefront looks at
+template <int S1, bool F32, int PPASSES, bool MAY>
 __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kernel(IndexerArgs a)
 {
-    constexpr int NHALF = 2 * PPASSES;
     __shared__ __align__(16) uint32_t hist[S1][SBINS];
     __shared__ __align__(16) float s_sc[S1][CHUNK * PPASSES]; // the workgroup's scores, written out in one burst at the end
     __shared__ __align__(16) uint8_t s_keys[4][64 * D];
@@ -302,40 +313,61 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
     const int l16 = lane & 15, g = lane >> 4;
     const int sgrp = blockIdx.z;
     const int bs = a.block_size;
-    // The (sequence, span of 512 PPASSES keys) of this workgroup: by its place in the grid when every sequence fills its spans.
-    // With ragged lengths the workgroups that have work should be the first ones of the launch order, so that they
-    // spread evenly over the CUs: workgroup w (its place in launch order, sequence-major) takes the w-th span that
-    // holds keys.  Every wavefront finds it on its own from the sequence lengths (lane l holds sequences l, l + 64, ..;
-    // a wavefront prefix sum of the spans per sequence), which are fetched together with the page-table entries of the
-    // grid place; only if the span is another one (ragged lengths) are those fetched again.  Batches beyond
-    // SCAN_SEQS sequences keep the grid place.
+    // The (sequence, span of 512 passes keys) of this workgroup.  The workgroups that have work should be the first ones of the
+    // launch order, so that they spread evenly over the CUs: workgroup w (its place in launch order, sequence-major) takes the
+    // w-th span that holds keys.  Every wavefront finds it on its own from the sequence lengths (lane l holds sequences l, l +
+    // 64, ..; a wavefront prefix sum of the spans per sequence), which are fetched together with the page-table entries of the
+    // grid place; only if the span is another one (ragged lengths, other passes) are those fetched again.  Batches beyond
+    // SCAN_SEQS sequences keep the grid place, the spans of a sequence turned by its number: workgroups go to the eight
+    // dies in turn, and the first spans of all sequences, often the only ones with keys, would all meet on the same few (300
+    // sequences of 3000 .. 9000 keys under 1024 columns: 426 us).
     // Lane p takes the page-table entry of pass p and the sequence's first entry, and picks once the length is known:
     // it then holds the first cache row of pass p (-1: unmapped page); a pass past the end re-reads the sequence's
     // first page and is discarded.
-    int bi = blockIdx.y, span = blockIdx.x;
-    const uint32_t w = blockIdx.x + gridDim.x * blockIdx.y;
-    constexpr int SCAN_SEQS = 256;
     const bool balanced = a.b <= SCAN_SEQS;
+    const uint32_t w = blockIdx.x + gridDim.x * blockIdx.y;
+    int bi = min((int)blockIdx.y, a.b - 1), span = balanced ? (int)blockIdx.x : (int)((blockIdx.x + blockIdx.y) % gridDim.x);
+    int passes = PPASSES, passes_log2 = __builtin_ctz(PPASSES);
     int lens[SCAN_SEQS / 64];
-    // (unconditional loads, so that they travel with the ones below)
+    // (unconditional loads, so that they travel with the ones below; of more sequences SCAN_SEQS evenly spaced ones)
 #pragma unroll
-    for (int j = 0; j < SCAN_SEQS / 64; ++j) lens[j] = a.act_seq[min(lane + 64 * j, a.b - 1)];
+    for (int j = 0; j < SCAN_SEQS / 64; ++j) {
+        const int i = lane + 64 * j;
+        lens[j] = a.act_seq[balanced ? min(i, a.b - 1) : (int)((int64_t)i * a.b / SCAN_SEQS)];
+    }
     int pg_mine, pg_first, L, mytok;
     auto fetch = [&]() {
-        mytok = span * (CHUNK * PPASSES) + wave * 128 + (lane < PPASSES ? lane : 0) * CHUNK;
+        mytok = span * (CHUNK * passes) + wave * 128 + (lane < passes ? lane : 0) * CHUNK;
         const int32_t* bt = a.block_table + (int64_t)bi * a.bt_stride;
         pg_mine = bt[min(mytok / bs, a.bt_stride - 1)];
         pg_first = bt[0];
         L = min(a.act_seq[bi], a.max_ctx); // keys past the page table's reach do not exist
     };
     fetch();
+    bool past_caches = false;
+    if constexpr (PPASSES > 1 || MAY) {
+        uint32_t groups = 0; // of one pass
+#pragma unroll
+        for (int j = 0; j < SCAN_SEQS / 64; ++j) {
+            lens[j] = lane + 64 * j < a.b ? max(min(lens[j], a.max_ctx), 0) : 0;
+            groups += (uint32_t)((lens[j] + CHUNK - 1) / CHUNK);
+        }
+        groups = (uint32_t)__builtin_amdgcn_readlane((int)wave_prefix_sum(groups), 63);
+        if (balanced && PPASSES > 1) {
+            while (passes > a.min_passes && (uint64_t)groups * (uint32_t)(a.s1 / S1) < (uint32_t)passes * SCORE_GROUPS_MIN) {
+                passes >>= 1;
+                --passes_log2;
+            }
+        }
+        if constexpr (MAY) past_caches = (float)groups * (balanced ? 1.f : (float)a.b / SCAN_SEQS) * (CHUNK * D) > SCORE_CACHED;
+    }
     if (balanced) {
         uint32_t base = 0;
         int fseq = -1, fspan = 0;
 #pragma unroll
         for (int j = 0; j < SCAN_SEQS / 64; ++j) {
             const int len = min(lens[j], a.max_ctx);
-            const uint32_t cnt = (lane + 64 * j < a.b && len > 0) ? (uint32_t)((len + CHUNK * PPASSES - 1) / (CHUNK * PPASSES)) : 0u;
+            const uint32_t cnt = (lane + 64 * j < a.b && len > 0) ? ((uint32_t)((len - 1) / CHUNK) >> passes_log2) + 1u : 0u;
             const uint32_t incl = wave_prefix_sum(cnt), excl = incl - cnt;
             const uint64_t hit = __ballot(w >= base + excl && w < base + incl); // at most one lane, in one round
             if (hit != 0ull && fseq < 0) {
@@ -346,15 +378,16 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
             base += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
         }
         if (fseq < 0) return; // more workgroups than spans with keys
-        if (fseq != bi || fspan != span) {
+        if (fseq != bi || fspan != span || passes != PPASSES) {
             bi = fseq;
             span = fspan;
             fetch();
         }
     }
-    if (span * (CHUNK * PPASSES) >= L) return;
+    const int span_keys = CHUNK * passes;
+    if (span * span_keys >= L) return;
     const int row0 = bi * a.s1 + sgrp * S1;
-    const int wtok = span * (CHUNK * PPASSES) + wave * 128; // first key of this wave's pass 0
+    const int wtok = span * span_keys + wave * 128; // first key of this wave's pass 0
     int64_t myrow;
     {
         const int tc = mytok < L ? mytok : 0;
@@ -367,6 +400,8 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
         return (int64_t)(((uint64_t)hi << 32) | lo);
     };
 
+    // past: loads past the caches; halves: passes of 64 keys per wavefront (known to the compiler for PPASSES: 2 to 6 % faster)
+    auto score = [&](auto past, auto halves) __attribute__((always_inline)) {
     // 64 keys on the way: load i holds chunk lane % 8 of key 8 i + lane / 8; in LDS the 16-byte chunks of a key are XOR-ed with
     // the key, so that both the row writes and the operand reads fall on all banks
     i32x4 raw[8];
@@ -378,7 +413,7 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const i32x4* p = reinterpret_cast<const i32x4*>(kp + i * 8 * D);
-            raw[i] = NT ? __builtin_nontemporal_load(p) : *p;
+            raw[i] = decltype(past)::value ? __builtin_nontemporal_load(p) : *p;
         }
         ksc_next = static_cast<const typename ScaleOf<F32>::raw*>(a.k_scale)[rb + 64 * (hh & 1) + lane];
     };
@@ -458,32 +493,41 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
 #pragma unroll
         for (int s = 0; s < S1; ++s) {
             const float sc = res[s] * ks;
-            s_sc[s][tok - span * (CHUNK * PPASSES)] = sc;
+            s_sc[s][tok - span * span_keys] = sc;
             const int eff = L - (a.s1 - 1 - (sgrp * S1 + s));
             if (a.use_hist && tok < eff) atomicAdd(&hist[s][score_bin(score_key(sc))], 1u);
         }
     };
 
     // (past the end the last half is loaded again, a cache hit whose data is never used, so that the loads stay unconditional)
-    for (int hh = 0; hh < NHALF; ++hh) {
+    for (int hh = 0; hh < halves; ++hh) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) *reinterpret_cast<i32x4*>(key_dst + i * 8 * D) = raw[i]; // (8 keys on: the same XOR)
         const typename ScaleOf<F32>::raw ksc = ksc_next;
-        load_half(hh + 1 < NHALF ? hh + 1 : NHALF - 1);
+        load_half(hh + 1 < halves ? hh + 1 : halves - 1);
         compute_half(hh, ksc);
+    }
+    };
+    if (__builtin_expect(passes != PPASSES, 0)) {
+        score(std::false_type{}, 2 * passes);
+    } else if (past_caches) {
+        asm volatile("; past the caches"); // (else the compiler merges the two sides' first loads, into plain ones)
+        score(std::true_type{}, std::integral_constant<int, 2 * PPASSES>{});
+    } else {
+        score(std::false_type{}, std::integral_constant<int, 2 * PPASSES>{});
     }
     __syncthreads();
     // one contiguous 8 KB write per query token (256-byte stores from inside the loop, between the key loads, cost
     // 2 us more); score rows are padded to whole workgroup spans, so no bounds check
 #pragma unroll
     for (int s = 0; s < S1; ++s) {
-        float* dst = a.scores + (int64_t)(row0 + s) * a.score_stride + (int64_t)span * (CHUNK * PPASSES);
+        float* dst = a.scores + (int64_t)(row0 + s) * a.score_stride + (int64_t)span * span_keys;
 #pragma unroll
         for (int i = 0; i < (CHUNK * PPASSES + 1023) / 1024; ++i)
-            if (4 * (tid + 256 * i) < CHUNK * PPASSES)
+            if (4 * (tid + 256 * i) < span_keys)
                 *reinterpret_cast<f32x4*>(dst + 4 * (tid + 256 * i)) = *reinterpret_cast<const f32x4*>(&s_sc[s][4 * (tid + 256 * i)]);
     }
-    if (a.use_hist) flush_span_hist<S1>(a, hist, row0, span, tid);
+    if (a.use_hist) flush_span_hist<S1>(a, hist, row0, span, passes_log2, tid);
 }
 
 __global__ void indexer_fill_kernel(int32_t* p, int n, int32_t v)
@@ -542,6 +586,7 @@ __global__ __launch_bounds__(256) void indexer_select_kernel(IndexerArgs a)
     constexpr int GROUP = 32;
     const int sg = tid >> 5, oct = tid & 31;
     const uint16_t* sh = a.span_hist + (int64_t)row * a.pchunks * SBINS + 8 * oct;
+    const int shift = __builtin_ctz(CHUNK) + (int)(*a.passes_log2 & 15u); // (not written, and not used, if no sequence has keys)
     u32x4 cv[GROUP / 8];
 #pragma unroll
     for (int j = 0; j < GROUP / 8; ++j) cv[j] = *reinterpret_cast<const u32x4*>(sh + (int64_t)min(sg + 8 * j, a.pchunks - 1) * SBINS);
@@ -554,7 +599,7 @@ __global__ __launch_bounds__(256) void indexer_select_kernel(IndexerArgs a)
     const int n = max(len - (a.s1 - 1 - (row - bi * a.s1)), 0);
     // (a workgroup past the row's end leaves further down, behind the first use of what was requested above: an exit
     // here would let the compiler move those requests behind the wait for the length - two round trips instead of one)
-    const int nsp = min((len + a.span - 1) / a.span, a.pchunks); // spans whose workgroup ran
+    const int nsp = n > 0 ? min(((len - 1) >> shift) + 1, a.pchunks) : 0; // spans whose workgroup ran
     if (tid == 0) s_bin = 0xffffffffu; // n <= k: no threshold bin, everything is a winner
 
     uint32_t acc[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
@@ -1255,12 +1300,13 @@ hipError_t topk_launch(const float* x, float* values, int32_t* indices, int64_t 
 }
 
 // workspace: scores [t, stride] f32 | span_hist [t, spans, 256] u16 | counters [t, 4] u32 | winners [t, 2048] u64 |
-// ties [t, 8192] u64; spans = stride / span
+// ties [t, 8192] u64 | passes_log2 u32; spans = stride / span
 static uint64_t align256(uint64_t x) { return (x + 255) & ~(uint64_t)255; }
 
 // Passes of 512 keys per workgroup of the paged score kernel: as many as leave SCORE_GROUPS workgroups, eight at most.  Where
 // there are keys for that, few long streams serve best (32 x 64 K keys: 50 us with eight passes, 53 with four, 58 with two);
 // a small batch needs short ones to reach every CU (a single 4 K context is 2 workgroups of four passes: 12 us, against 6).
+// The kernel takes fewer where the contexts are shorter than the page tables.
 static int pick_passes(int b, int s1, int64_t stride)
 {
     const int64_t groups = (int64_t)b * (s1 % 2 == 0 ? s1 / 2 : s1) * (stride / CHUNK); // of one pass
@@ -1273,16 +1319,16 @@ uint64_t indexer_workspace_bytes(int b, int s1, int stride)
 {
     const int t = b * s1;
     const int passes = pick_passes(b, s1, stride);
-    const uint64_t spans = (uint64_t)stride / (CHUNK * (passes < PASSES ? passes : PASSES)); // (the unpaged kernel's spans: PASSES)
+    const uint64_t spans = (uint64_t)stride / (CHUNK * std::min(passes, PASSES)); // (the unpaged kernel's spans: PASSES)
     return align256((uint64_t)t * stride * 4) + align256((uint64_t)t * spans * SBINS * 2) + align256((uint64_t)t * 4 * 4) +
-           align256((uint64_t)t * (MAX_K + TIE_CAP) * 8);
+           align256((uint64_t)t * (MAX_K + TIE_CAP) * 8) + 256;
 }
 
 void indexer_bind_workspace(IndexerArgs& a, void* ws)
 {
     const int t = a.b * a.s1;
     a.span = a.block_size % 128 == 0 ? CHUNK * pick_passes(a.b, a.s1, a.score_stride) : CHUNK * PASSES;
-    const uint64_t spans = (uint64_t)a.score_stride / a.span;
+    const uint64_t spans = (uint64_t)a.score_stride / std::min(a.span, CHUNK * PASSES);
     uint8_t* p = static_cast<uint8_t*>(ws);
     a.scores = reinterpret_cast<float*>(p);
     p += align256((uint64_t)t * a.score_stride * 4);
@@ -1292,6 +1338,8 @@ void indexer_bind_workspace(IndexerArgs& a, void* ws)
     p += align256((uint64_t)t * 4 * 4);
     a.winners = reinterpret_cast<uint64_t*>(p);
     a.ties = a.winners + (uint64_t)t * MAX_K;
+    p += align256((uint64_t)t * (MAX_K + TIE_CAP) * 8);
+    a.passes_log2 = reinterpret_cast<uint32_t*>(p);
     a.pchunks = (int32_t)spans;
 }
 
@@ -1299,15 +1347,18 @@ template <int PPASSES>
 static void launch_score_paged(const IndexerArgs& a, hipStream_t stream)
 {
     const bool s2 = a.s1 % 2 == 0, f32 = a.scales_f32;
-    // non-temporal where one call's keys (if they fill the page table) would take the last-level cache's better part (109 MB:
-    // 26.2 -> 24.8 us, 272 MB: 57.8 -> 52.7; 68 MB, found there from one call to the next: 15.0 -> 16.4) and not more than
-    // two workgroups read them
-    const bool nt = (double)a.b * a.max_ctx * D > 96e6 && a.s1 <= 2;
+    // non-temporal where one call's keys take the last-level cache's better part (109 MB: 26.2 -> 24.8 us, 272 MB: 57.8 ->
+    // 52.7; 68 MB, found there from one call to the next: 15.0 -> 16.4) and not more than two workgroups read them
+    const bool nt = (double)a.b * a.max_ctx * D > SCORE_CACHED && a.s1 <= 2;
     auto kern = s2 ? (f32 ? (nt ? indexer_score_paged_kernel<2, true, PPASSES, true> : indexer_score_paged_kernel<2, true, PPASSES, false>)
                           : (nt ? indexer_score_paged_kernel<2, false, PPASSES, true> : indexer_score_paged_kernel<2, false, PPASSES, false>))
                    : (f32 ? (nt ? indexer_score_paged_kernel<1, true, PPASSES, true> : indexer_score_paged_kernel<1, true, PPASSES, false>)
                           : (nt ? indexer_score_paged_kernel<1, false, PPASSES, true> : indexer_score_paged_kernel<1, false, PPASSES, false>));
-    hipLaunchKernelGGL(kern, dim3((a.max_ctx + CHUNK * PPASSES - 1) / (CHUNK * PPASSES), a.b, s2 ? a.s1 / 2 : a.s1), dim3(256), 0, stream, a);
+    // a workgroup for every span of the page tables' reach; fewer passes are taken with fewer than 2 SCORE_GROUPS workgroups
+    // (in all query token groups) full and one more in every sequence
+    const int64_t z = s2 ? a.s1 / 2 : a.s1, gx = (a.max_ctx + CHUNK * PPASSES - 1) / (CHUNK * PPASSES);
+    const int64_t rows = a.b <= SCAN_SEQS && PPASSES > a.min_passes ? std::max<int64_t>(a.b, ((2 * SCORE_GROUPS + z - 1) / z + a.b + gx - 1) / gx) : a.b;
+    hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)rows, (unsigned)z), dim3(256), 0, stream, a);
 }
 
 hipError_t indexer_launch(const IndexerArgs& a, hipStream_t stream)
@@ -1324,6 +1375,7 @@ hipError_t indexer_launch(const IndexerArgs& a, hipStream_t stream)
     IndexerArgs args = a;
     args.max_ctx = max_ctx;
     args.use_hist = max_ctx > INDEXER_ROW_MAX;
+    args.min_passes = args.use_hist ? a.score_stride / a.pchunks / CHUNK : 1; // (no more spans than slots)
     {
         ScopedKernelTimer tm(KID_INDEXER_SCORE, stream);
         if (a.block_size % 128 == 0) {

@@ -249,8 +249,8 @@ def test_wide_page_table_many_sequences(cuda):
 
 @pytest.mark.parametrize("bs,cols,s1", [(48, 700, 1), (48, 700, 2), (128, 270, 1), (128, 270, 2), (128, 70, 4)])
 def test_span_lengths_follow_the_page_tables_reach(cuda, bs, cols, s1):
-    """Short sequences under wide page tables: the reach, not the lengths, picks the passes per workgroup (1 to 8) and whether
-    keys are loaded past the caches, in the paged and in the plain score kernel; the selection is that of a narrow table."""
+    """Short sequences under wide page tables, in the paged and in the plain score kernel: the reach picks the most passes per
+    workgroup (1 to 8) and whether the selection uses histograms; the selection is that of a narrow table."""
     g = torch.Generator().manual_seed(cols + s1)
     act = torch.randint(1, 900, (64,), generator=g).tolist()
     case = oi.make_case(64, s1, act, seed=43, selected_count=128, block_size=bs)
@@ -261,6 +261,51 @@ def test_span_lengths_follow_the_page_tables_reach(cuda, bs, cols, s1):
     wide = dict(case)
     wide["block_table"] = torch.cat([bt, torch.full((bt.shape[0], cols - bt.shape[1]), -1, dtype=bt.dtype)], dim=1).contiguous()
     assert torch.equal(run_indexer(wide, cuda), narrow)
+
+
+@pytest.mark.parametrize("b,lo,hi,cols,s1", [(40, 1, 3000, 256, 1), (30, 8000, 20000, 256, 1), (20, 100, 9000, 1024, 1), (20, 100, 9000, 1024, 2),
+                                             (130, 1, 4000, 1024, 1), (270, 1, 1500, 300, 1), (270, 1, 1500, 40, 2)])
+def test_spans_follow_the_lengths(cuda, b, lo, hi, cols, s1):
+    """Fewer passes per workgroup than full page tables would get: down to one without histograms, to the histograms' slots with
+    them, and more sequences than the choice looks at (spans turned by the sequence); the selection is that of a narrow table."""
+    g = torch.Generator().manual_seed(b + cols)
+    act = torch.randint(lo, hi, (b,), generator=g).tolist()
+    case = oi.make_case(b, s1, act, seed=b, selected_count=512)
+    bt = case["block_table"]
+    wide = dict(case, block_table=torch.cat([bt, torch.full((b, cols - bt.shape[1]), -1, dtype=bt.dtype)], dim=1).contiguous())
+    got = run_indexer(wide, cuda)
+    check_topk(case, got)
+    assert torch.equal(run_indexer(case, cuda), got)
+
+
+def test_wide_page_tables_of_many_sequences_keep_all_dies_busy(cuda):
+    """300 sequences of 2048 keys: tables of 1024 columns cost the selection's empty workgroups, not six times the narrow
+    tables' time (which the score kernel alone took with the first spans of all sequences on one of eight dies)."""
+    from pypto_amd.deepseek_v32_exp import lightning_indexer_quant_impl as li
+    b, pages = 300, 16
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q = torch.randint(-127, 128, (b, 64, 128), generator=g, device=cuda, dtype=torch.int8)
+    k = torch.randint(-127, 128, (b * pages, 128, 1, 128), generator=g, device=cuda, dtype=torch.int8)
+    qs, ks = torch.rand(b, 64, device=cuda).to(torch.float16), torch.rand(b * pages, 128, 1, device=cuda).to(torch.float16)
+    w = torch.rand(b, 64, device=cuda).to(torch.float16)
+    act = torch.full((b,), 128 * pages, dtype=torch.int32, device=cuda)
+    narrow = torch.arange(b * pages, dtype=torch.int32, device=cuda).view(b, pages)
+    wide = torch.full((b, 1024), -1, dtype=torch.int32, device=cuda)
+    wide[:, :pages] = narrow
+
+    def time(table):
+        out, best = torch.zeros(b, 1, 512, dtype=torch.int32, device=cuda), float("inf")
+        for _ in range(5):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(5):
+                li.lightning_indexer_decode(q, qs, k, ks, w, act, table, out, [1], li.LightningIndexerConfigs(), 512)
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, start.elapsed_time(end))
+        return best
+
+    assert time(wide) < 6 * time(narrow)
 
 
 def test_other_selection_sizes_and_block_sizes(cuda):
