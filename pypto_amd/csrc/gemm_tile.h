@@ -191,9 +191,9 @@ __device__ __forceinline__ void gt_stream_i8(i32x4 (&acc)[2][2], const int8_t* w
 // The same loop in bf16 for 128 tokens x 256 outputs, the outputs in four blocks of 64 columns at src[i], ld[i] values a row;
 // x: [t, ldx], column of the first contraction row.  Wave (wr, wc) owns tokens [64 wr, +64) x block wc.  Register e of
 // sum[tb][nb]: token 64 wr + 32 tb + 8 (e / 4) + 4 hl + e % 4, column 32 nb + lane % 32 of the block.  Sums are chains of at most
-// CHAIN contraction rows, added up in order.
+// CHAIN contraction rows, added up in order within GROUP rows, and those sums in order.
 constexpr int GT_KBF = 64; // contraction rows per stage
-template <int CHAIN>
+template <int CHAIN, int GROUP>
 __device__ __forceinline__ void gt_product_bf16(f32x16 (&sum)[2][2], const uint16_t* const (&src)[4], const int (&ld)[4], const uint16_t* x,
                                                 int64_t ldx, int tok0, int t, int stages, uint8_t* lds)
 {
@@ -222,13 +222,29 @@ __device__ __forceinline__ void gt_product_bf16(f32x16 (&sum)[2][2], const uint1
     const int xf = (l32 >> 1) & 7;
     const uint8_t* wrow = lds + T::QBYTES + wc * 8192 + (8 * hl + (jj >> 2)) * 128 + 8 * (jj & 1);
     const int wpos = 16 * ((2 * mh + ((jj >> 1) & 1)) ^ ((jj >> 1) & 4));
-    f32x16 acc[2][2];
+    static_assert(GROUP % CHAIN == 0 && CHAIN % GT_KBF == 0, "whole chains");
+    constexpr bool TWO = GROUP > CHAIN; // (else a chain goes straight to the sums)
+    f32x16 acc[2][2], part[TWO ? 2 : 1][TWO ? 2 : 1];
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[tb][nb][e] = sum[tb][nb][e] = 0.f;
+            for (int e = 0; e < 16; ++e) {
+                acc[tb][nb][e] = sum[tb][nb][e] = 0.f;
+                if constexpr (TWO) part[tb][nb][e] = 0.f;
+            }
+    auto add = [&](auto& to, auto& from) { // from is empty again
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    to[tb][nb][e] += from[tb][nb][e];
+                    from[tb][nb][e] = 0.f;
+                }
+    };
     gt_stages<T::RING, T::STAGE, 6>(stages, copy, [&](int st, int b) {
 #pragma unroll
         for (int ks = 0; ks < GT_KBF / 16; ++ks) {
@@ -246,16 +262,12 @@ __device__ __forceinline__ void gt_product_bf16(f32x16 (&sum)[2][2], const uint1
 #pragma unroll
                 for (int nb = 0; nb < 2; ++nb) acc[tb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv[tb], wv[nb], acc[tb][nb], 0, 0, 0);
         }
-        if ((st + 1) % (CHAIN / GT_KBF) == 0 || st + 1 == stages) {
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        sum[tb][nb][e] += acc[tb][nb][e];
-                        acc[tb][nb][e] = 0.f;
-                    }
+        const bool last = st + 1 == stages;
+        if constexpr (TWO) {
+            if ((st + 1) % (CHAIN / GT_KBF) == 0 || last) add(part, acc);
+            if ((st + 1) % (GROUP / GT_KBF) == 0 || last) add(sum, part);
+        } else {
+            if ((st + 1) % (CHAIN / GT_KBF) == 0 || last) add(sum, acc);
         }
     });
 }

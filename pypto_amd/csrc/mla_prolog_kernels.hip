@@ -286,7 +286,7 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_xa_wide_kernel(MlaPrologArgs 
         src[i] += (int64_t)kbeg * ld[i];
     }
     f32x16 acc[2][2];
-    gt_product_bf16<XA_SPLIT>(acc, src, ld, a.x + kbeg, a.h, tok0, a.t, stages, lds);
+    gt_product_bf16<XA_SPLIT, XA_SPLIT>(acc, src, ld, a.x + kbeg, a.h, tok0, a.t, stages, lds);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, hl = lane >> 5, wr = wave >> 2, wc = wave & 3;
     const int col0 = (4 * nt + wc) * 64;
     if (col0 >= a.ncols) return;
@@ -435,7 +435,9 @@ __global__ __launch_bounds__(256) void mla_qb16_kernel(MlaPrologArgs a)
 }
 
 // The bf16 form at more tokens: 128 tokens x 256 outputs per workgroup over the whole contraction (gemm_tile.h), the epilogue
-// on the tile: 86 us at 1024 tokens, where a kernel that read the weights once per 32 tokens took 811.  grid (n * 192 / 256 rounded up, token tiles of 128), 512 lanes.
+// on the tile: 91 us at 1024 tokens, where a kernel that read the weights once per 32 tokens took 811.  The sums are
+// mla_qb16_kernel's bit for bit (in chains of 256 rows, added up in order, they took 5 us less there and 2 at 33 tokens, and were 10 %
+// further off).  grid (n * 192 / 256 rounded up, token tiles of 128), 512 lanes.
 __global__ __launch_bounds__(GT_LANES, 2) void mla_qb16_wide_kernel(MlaPrologArgs a)
 {
 #pragma clang fp contract(off)
@@ -452,7 +454,7 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb16_wide_kernel(MlaPrologArg
         ld[i] = a.n * MQH;
     }
     f32x16 acc[2][2];
-    gt_product_bf16<256>(acc, src, ld, reinterpret_cast<const uint16_t*>(a.q_norm), a.r, tok0, a.t, a.r / GT_KBF, lds);
+    gt_product_bf16<128, XA_SPLIT>(acc, src, ld, reinterpret_cast<const uint16_t*>(a.q_norm), a.r, tok0, a.t, a.r / GT_KBF, lds);
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb)
 #pragma unroll

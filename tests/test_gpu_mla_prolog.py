@@ -235,9 +235,21 @@ def test_prefill_query_tiles(cuda, t, n):
 
 @pytest.mark.parametrize("t,n", [(33, 2), (128, 6), (129, 4), (300, 2)])
 def test_bf16_form_prefill_tiles(cuda, t, n):
-    # from 33 tokens on the query product owns 128 tokens x 256 outputs: remainders of both, chains of 256 rows
+    # from 33 tokens on the query product owns 128 tokens x 256 outputs: remainders of both, chains of 128 rows
     case = op.make_case(t, 1, 64, seed=70 + t, h=512, q_lora_rank=512, n=n, quant_b=False)
     check_bf16_form(case, run(case, cuda))
+
+
+@pytest.mark.parametrize("quant_b", [True, False])
+def test_a_tokens_bits_do_not_depend_on_the_batch(cuda, quant_b):
+    """Up to 32 tokens and from 33 on other kernels form the products; below 128 tokens their fp32 sums are the same (chains of 128
+    rows within 1024, and those in order), so a token's results are the same bits in a batch of 32 and of 100."""
+    case = op.make_case(100, 1, 64, seed=77, h=1280, q_lora_rank=1536, n=32, quant_b=quant_b)
+    first = {k: v[:32].contiguous() if k in ("x", "cos", "sin", "cache_index") else v for k, v in case.items()}
+    assert case["x"].shape[0] == 100 and case["cos"].shape[0] == 100
+    many, few = run(case, cuda), run(first, cuda)
+    for name in ("q_norm", "q_norm_scale", "q_nope", "q_rope"):
+        assert torch.equal(many[name][:32], few[name]), name
 
 
 def test_bf16_form_reference_case_b4_s2(cuda):
