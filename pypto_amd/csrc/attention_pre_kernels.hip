@@ -195,7 +195,85 @@ __global__ __launch_bounds__(256) void apq_gemm_kernel(AttnPreArgs a)
     }
 }
 
-// The projection at prefill sizes and larger decode batches (attention_pre_big): a workgroup owns 32 TB tokens x 256 outputs - two heads - over one
+// The projection of a rank's few heads at small prefill sizes (attention_pre_kernel): a workgroup owns 128 tokens x 128 outputs
+// over one split of the contraction, so that 14 heads fill the chip where tiles of 256 outputs leave most of it idle (14 heads:
+// 144 tokens 21.4 us a call against 23.1, 28 heads, 64 tokens: 19.8 / 21.7).  It walks the split in stages of 128 rows, both
+// operands staged through LDS with the next stage's global loads in flight while the current stage is multiplied.  Wave (wr, wc) owns tokens [64 wr, +64) x outputs [64 wc, +64):
+// every operand fragment read from LDS feeds four MFMAs, and the weights are read once per 128 tokens instead of once
+// per 32.  Same int32 partial sums as apq_gemm_kernel (exact, so neither the tiling nor the split shows).
+// grid (n_out / 128, splits, token tiles of 128), 256 lanes.
+constexpr int BTOK = 128, BK = 128;
+constexpr int BQROW = BK + 16; // bytes per LDS row of the [token][k] int8 tile (padded against bank conflicts)
+__global__ __launch_bounds__(256, 3) void apq_gemm_mid_kernel(AttnPreArgs a, int per)
+{
+    __shared__ __align__(16) uint8_t wl[BK * AROW];
+    __shared__ __align__(16) uint8_t ql[BTOK * BQROW];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int l16 = lane & 15, g = lane >> 4, wr = wave >> 1, wc = wave & 1;
+    const int col0 = blockIdx.x * AD, split = blockIdx.y, tok0 = blockIdx.z * BTOK;
+    const int st0 = split * per, stages = min(a.h / BK, st0 + per) - st0; // this split's stages of 128 rows
+    // 128 rows x 128 bytes of either operand per stage = 4 pieces of 16 bytes per lane (rows tid / 8 + 32 i, piece tid % 8)
+    const int srow = tid >> 3, spc = tid & 7;
+    const int8_t* wp = a.w + ((int64_t)st0 * BK + srow) * a.n_out + col0 + 16 * spc;
+    const int8_t* qp[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) qp[i] = a.x_q + (int64_t)min(tok0 + srow + 32 * i, a.t - 1) * a.h + (int64_t)st0 * BK + 16 * spc;
+    u32x4 wst[4], qst[4];
+    auto load = [&](int st) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) qst[i] = *reinterpret_cast<const u32x4*>(qp[i] + st * BK);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) wst[i] = *reinterpret_cast<const u32x4*>(wp + ((int64_t)st * BK + 32 * i) * a.n_out);
+    };
+    i32x4 acc[4][4]; // [db][tb]
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb) acc[db][tb] = i32x4{0, 0, 0, 0};
+    load(0);
+    for (int st = 0; st < stages; ++st) {
+        __syncthreads(); // everyone is done with the previous stage's tiles
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            u32x2* d = reinterpret_cast<u32x2*>(wl + (srow + 32 * i) * AROW + 16 * spc);
+            d[0] = u32x2{wst[i][0], wst[i][1]};
+            d[1] = u32x2{wst[i][2], wst[i][3]};
+            *reinterpret_cast<u32x4*>(ql + (srow + 32 * i) * BQROW + 16 * spc) = qst[i];
+        }
+        __syncthreads();
+        load(min(st + 1, stages - 1)); // (unconditional: past the end the last stage is fetched again and dropped)
+#pragma unroll
+        for (int ks = 0; ks < BK / 64; ++ks) {
+            i32x4 qf[4], wf[4];
+#pragma unroll
+            for (int tb = 0; tb < 4; ++tb)
+                qf[tb] = *reinterpret_cast<const i32x4*>(ql + (64 * wr + 16 * tb + l16) * BQROW + ks * 64 + 16 * g);
+            // (the byte-transposing read: see apq_gemm_kernel)
+#pragma unroll
+            for (int db = 0; db < 4; ++db) {
+                const uint8_t* p = wl + (ks * 64 + 16 * g + (l16 >> 1)) * AROW + 64 * wc + 16 * db + 8 * (l16 & 1);
+                const v2i lo = lds_read_tr8(p), hi = lds_read_tr8(p + 8 * AROW);
+                wf[db] = i32x4{lo[0], lo[1], hi[0], hi[1]};
+            }
+#pragma unroll
+            for (int db = 0; db < 4; ++db)
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb)
+                    acc[db][tb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[db], qf[tb], acc[db][tb], 0, 0, 0);
+        }
+    }
+    // register e of acc[db][tb]: output 64 wc + 16 db + 4 g + e, token 64 wr + 16 tb + l16
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) {
+        const int tok = tok0 + 64 * wr + 16 * tb + l16;
+        if (tok >= a.t) continue;
+        int32_t* dst = a.part + ((int64_t)split * a.t + tok) * a.n_out + col0 + 64 * wc + 4 * g;
+#pragma unroll
+        for (int db = 0; db < 4; ++db) *reinterpret_cast<i32x4*>(dst + 16 * db) = acc[db][tb];
+    }
+}
+
+// The projection at prefill sizes and larger decode batches (attention_pre_kernel): a workgroup owns 32 TB tokens x 256 outputs - two heads - over one
 // split of the contraction (gemm_tile.h; an odd last head is taken twice and dropped).  An XCD takes neighbouring heads.  Where one split covers the whole contraction the head's epilogue runs on the
 // tile: the sums never go to memory (777 tokens x 112 heads: 45 MB written and read again, and a kernel of 87 K small
 // workgroups).  Same operations in the same order as apq_head_kernel, so the same bits: its sum over the 128 squares is a
@@ -430,19 +508,25 @@ bool attention_pre_supported(int64_t h, int64_t d, int64_t half)
 
 static uint64_t align256(uint64_t v) { return (v + 255) & ~(uint64_t)255; }
 
-// stages of 256 contraction rows per workgroup of the projection: as many (1, 2 or 4) as still leave 448 workgroups
+// stages of 256 contraction rows per workgroup of apq_gemm_kernel: as many (1, 2 or 4) as still leave enough workgroups
+// (14 heads, 33 tokens, 560 workgroups of one stage: 17.0 us a call, 280 of two 15.6; 28 heads, 32 tokens: 18.9 / 18.1)
 static int stages_per_split(int64_t t, int64_t h, int64_t n_out)
 {
     const int64_t wgs = (n_out / AD) * (h / AK) * ((t + ATOK - 1) / ATOK);
-    return wgs >= 8 * 448 ? 4 : wgs >= 2 * 448 ? 2 : 1;
+    return wgs >= 8 * 448 ? 4 : wgs >= 480 ? 2 : 1;
+}
+
+// stages of 128 rows per workgroup of apq_gemm_mid_kernel - all of them while that still leaves 256 workgroups, otherwise as
+// many as do
+static int mid_stages_per_split(int64_t t, int64_t h, int64_t n_out)
+{
+    const int64_t tiles = (n_out / AD) * ((t + BTOK - 1) / BTOK), stages = h / BK;
+    const int64_t splits = std::min<int64_t>(stages, std::max<int64_t>(1, (256 + tiles - 1) / tiles));
+    return (int)((stages + splits - 1) / splits);
 }
 
 // Prefill sizes: token blocks of the tile and stages of 128 rows per workgroup of apq_gemm_big_kernel, by the time they should
 // take in ns (gt_time_ns); partial sums are written, read again at 8 TB/s (the caches hold them) and cost the head kernel.
-// From 33 tokens on (a second token tile of apq_gemm_kernel: 14 heads 16.3 against 15.7 us a call, 64 tokens 19.5 / 18.1), and
-// from 9 where the weights are large (112 heads: 12 tokens 24.8 against 22.2 us, 24: 29.6 / 24.3, 100: 77 / 32; 28 heads and 12
-// tokens are the same, 14 heads 13.1 / 14.3).
-static bool attention_pre_big(int64_t t, int64_t n_out) { return t >= 33 || (t >= 9 && n_out >= 8192); }
 struct BigPlan { int tb, per; };
 static BigPlan big_plan(int64_t t, int64_t h, int64_t n_out)
 {
@@ -460,18 +544,35 @@ static BigPlan big_plan(int64_t t, int64_t h, int64_t n_out)
     return best;
 }
 
+// The projection's kernel.  The streamed one up to 32 tokens, but only up to 8 where the weights are large (112 heads: 12 tokens
+// 24.8 us a call against 22.2 by tiles of 256 outputs, 24: 29.6 / 24.3, 100: 77 / 32; 28 heads and 12 tokens are the same, 14
+// heads 13.1 / 14.3), and up to 128 tokens with up to 16 heads (14 heads, 128 x 128 tiles in the middle, 256 outputs last: 33 tokens
+// 15.6 / 16.6 / 17.0, 97: 19.9 / 20.6 / 21.3, 128: 22.4 / 22.4 / 23.6, 129: 22.5 / 21.0 / 23.2).  128 x 128 tiles with up to 16 heads
+// up to 192 tokens, with up to 32 up to 160, and again where a third token tile has just begun (14 heads: 160 tokens 22.6
+// against 23.9, 192: 23.7 / 24.0, 224: 24.8 / 24.5, 257: 25.8 / 26.8, 320: 28.0 / 26.8; 28 heads: 97 tokens 22.7 / 23.8, 160:
+// 25.2 / 26.5, 161: 25.3 / 24.7, 288: 31.9 / 32.6; 56 heads, 64 tokens: 24.8 / 22.6).
+enum class ApqKernel { stream, mid, tiles };
+static ApqKernel attention_pre_kernel(int64_t t, int64_t n_out)
+{
+    if (t <= 8 || (t <= 32 && n_out < 8192) || (t <= 128 && n_out <= 16 * AD)) return ApqKernel::stream;
+    const int64_t two_tiles = n_out <= 16 * AD ? 192 : 160;
+    return n_out <= 32 * AD && (t <= two_tiles || (t > 256 && t <= 288)) ? ApqKernel::mid : ApqKernel::tiles;
+}
+
 int attention_pre_ksplits(int64_t t, int64_t h, int64_t n_out)
 {
-    if (attention_pre_big(t, n_out)) {
-        const int per = big_plan(t, h, n_out).per;
-        return (int)((h / GT_KI8 + per - 1) / per);
-    }
-    const int per = stages_per_split(t, h, n_out);
-    return (int)((h / AK + per - 1) / per);
+    const ApqKernel kernel = attention_pre_kernel(t, n_out);
+    const int per = kernel == ApqKernel::tiles ? big_plan(t, h, n_out).per
+                                               : kernel == ApqKernel::mid ? mid_stages_per_split(t, h, n_out) : stages_per_split(t, h, n_out);
+    const int rows = kernel == ApqKernel::tiles ? GT_KI8 : kernel == ApqKernel::mid ? BK : AK;
+    return (int)((h / rows + per - 1) / per);
 }
 
 // one split at prefill sizes: the projection's workgroups finish their heads themselves, no sums go through memory
-static bool attention_pre_whole(int64_t t, int64_t n_out, int ksplits) { return attention_pre_big(t, n_out) && ksplits == 1; }
+static bool attention_pre_whole(int64_t t, int64_t n_out, int ksplits)
+{
+    return attention_pre_kernel(t, n_out) == ApqKernel::tiles && ksplits == 1;
+}
 
 uint64_t attention_pre_workspace_bytes(int64_t t, int64_t h, int64_t n_out)
 {
@@ -503,15 +604,18 @@ hipError_t attention_pre_launch(const AttnPreArgs& a, hipStream_t stream)
         const dim3 grid(a.n_out / AD, a.ksplits, (a.t + ATOK - 1) / ATOK);
         const int per = stages_per_split(a.t, a.h, a.n_out);
         if (a.ksplits != attention_pre_ksplits(a.t, a.h, a.n_out)) return hipErrorInvalidValue;
-        const bool tiles = attention_pre_big(a.t, a.n_out);
-        const BigPlan big = tiles ? big_plan(a.t, a.h, a.n_out) : BigPlan{};
-        if (tiles)
+        const ApqKernel kernel = attention_pre_kernel(a.t, a.n_out);
+        if (kernel == ApqKernel::tiles) {
+            const BigPlan big = big_plan(a.t, a.h, a.n_out);
             gt_dispatch(big.tb, [&](auto tb) {
                 constexpr int TB = decltype(tb)::value;
                 hipLaunchKernelGGL((whole ? apq_gemm_big_kernel<TB, true> : apq_gemm_big_kernel<TB, false>),
                                    dim3((a.n_out / AD + 1) / 2, a.ksplits, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream, a,
                                    big.per);
             });
+        } else if (kernel == ApqKernel::mid)
+            hipLaunchKernelGGL(apq_gemm_mid_kernel, dim3(a.n_out / AD, a.ksplits, (a.t + BTOK - 1) / BTOK), dim3(256), 0, stream, a,
+                               mid_stages_per_split(a.t, a.h, a.n_out));
         else if (per == 4)
             hipLaunchKernelGGL(apq_gemm_kernel<4>, grid, dim3(256), 0, stream, a);
         else if (per == 2)

@@ -141,9 +141,8 @@ def test_token_counts(cuda, t):
 
 @pytest.mark.parametrize("t,h,q_heads,kv_heads", [(128, 1024, 4, 2), (200, 5120, 12, 1), (300, 6400, 30, 3), (513, 256, 2, 1)])
 def test_prefill_token_counts(cuda, t, h, q_heads, kv_heads):
-    """128 tokens and more run the projection kernel that owns a 128 x 128 output tile: token counts that end inside a
-    tile, a contraction split into several workgroups with a short last split (6400 = 50 stages of 128), a contraction
-    of two stages taken whole."""
+    """Prefill sizes over all projection kernels: token counts that end inside a tile, a contraction split into several
+    workgroups with a short last split (6400 = 50 stages of 128), a contraction of two stages taken whole."""
     case = op.make_case(t, h=h, q_heads=q_heads, kv_heads=kv_heads, seed=t + h)
     check(case, run(case, cuda))
 
@@ -157,10 +156,32 @@ def test_whole_model_heads(cuda):
 @pytest.mark.parametrize("t,q_heads,kv_heads,half", [(128, 3, 1, 20), (129, 2, 1, 64), (1300, 48, 2, 32), (1500, 48, 2, 8), (1800, 48, 2, 1),
                                                      (2100, 47, 2, 32), (9, 62, 1, 32), (31, 60, 3, 32)])
 def test_prefill_in_one_split(cuda, t, q_heads, kv_heads, half):
-    """One split over the contraction (short here): the projection's workgroups finish their heads themselves.  Tiles of 128,
-    160, 192, 224 and 256 tokens with a remainder, an odd number of heads, rotary halves of whole and of broken pieces."""
+    """A short contraction, which the tiles of 256 outputs take in one split: their workgroups finish their heads themselves.  Tiles
+    of 128, 160, 192, 224 and 256 tokens with a remainder, an odd number of heads, rotary halves of whole and of broken pieces (the
+    first two cases run the streamed kernel and 128 x 128 tiles)."""
     case = op.make_case(t, h=256, q_heads=q_heads, kv_heads=kv_heads, half=half, seed=40 + t)
     check(case, run(case, cuda))
+
+
+@pytest.mark.parametrize("t,h,q_heads,kv_heads,half", [
+    (33, 5120, 12, 1, 32), (128, 6400, 14, 1, 20), (128, 1024, 15, 1, 64), (129, 6400, 12, 1, 64), (160, 256, 30, 1, 20), (192, 5120, 12, 2, 1), (160, 5120, 26, 2, 1), (161, 256, 26, 2, 32),
+    (193, 512, 3, 1, 20), (200, 256, 2, 1, 64), (257, 1024, 12, 1, 8), (288, 256, 30, 1, 64), (289, 1024, 12, 1, 32), (33, 512, 31, 1, 32)])
+def test_projection_kernels_at_the_edges_of_their_ranges(cuda, t, h, q_heads, kv_heads, half):
+    """Up to 16 heads: streamed up to 128 tokens, 128 x 128 tiles up to 192 and from 257 to 288; up to 32 heads: 128 x 128 tiles
+    from 33 to 160 tokens; wider tiles elsewhere.  Short last splits, token tiles with remainders of 1 to all rows."""
+    case = op.make_case(t, h=h, q_heads=q_heads, kv_heads=kv_heads, half=half, seed=t + h + half)
+    check(case, run(case, cuda))
+
+
+def test_a_tokens_bits_do_not_depend_on_the_projection_kernel(cuda):
+    # int32 sums are exact and the head epilogues the same operations: streamed, 128 x 128 and wide tiles in one and in several splits
+    case = op.make_case(300, h=1024, seed=3)
+    rows = ("hidden_states", "residual", "cos", "sin")
+    full = run(case, cuda)
+    for t in (20, 33, 128, 150, 200, 256, 260):
+        got = run({k: v[:t].contiguous() if k in rows else v for k, v in case.items()}, cuda)
+        for name in ("query", "key", "value", "residual_res"):
+            assert torch.equal(got[name], full[name][:t]), (t, name)
 
 
 @pytest.mark.parametrize("h,half", [(256, 64), (6144, 16), (6400, 1), (16384, 32)])
