@@ -890,8 +890,11 @@ __global__ __launch_bounds__(256, 2) void fused_qb_big_kernel(MlaPrologArgs m, P
         prolog_q_big_body<QB_DEPTH>(p, blockIdx.x - nqb, blockIdx.y * QB_TOK, lds);
 }
 
-// Above 256 tokens the two products in one launch of gemm_tile.h's tiles: the index heads' part alone is half a round of
-// workgroups up to 512 tokens (call of 257 tokens 94 -> 80 us, 512: 124 -> 104, 1501: the same).  grid (index heads / 2 rounded up + n * 192 / 256 rounded up, token tiles), 512 lanes
+constexpr int FUSED_T = 2048;
+// Above 256 tokens the two products in one launch of gemm_tile.h's tiles where that takes no more rounds of workgroups: the index
+// heads' part alone is half a round up to 512 tokens (call of 257 tokens 94 -> 80 us, 512: 124 -> 104).  Its tiles are up to
+// 224 tokens; where the query product's own of 256 save a round, and a round counts, the two are launches of their own (1024
+// tokens: 191 us in one, 184 in two, 1200: 219 / 208, 2048: the same, 4096: 680 / 691).  grid (index heads / 2 rounded up + n * 192 / 256 rounded up, token tiles), 512 lanes
 template <int TB>
 __global__ __launch_bounds__(GT_LANES, 2) void fused_qb_wide_kernel(MlaPrologArgs m, PrologArgs p)
 {
@@ -902,6 +905,13 @@ __global__ __launch_bounds__(GT_LANES, 2) void fused_qb_wide_kernel(MlaPrologArg
         prolog_q_wide_body<TB>(p, 2 * blockIdx.x, tok0, lds);
     else
         mla_qb_wide_body<TB>(m, blockIdx.x - nqt, tok0, lds);
+}
+// the index heads' part; grid (index heads / 2 rounded up, token tiles), 512 lanes
+template <int TB>
+__global__ __launch_bounds__(GT_LANES, 2) void fused_q_wide_kernel(PrologArgs p)
+{
+    __shared__ __align__(16) uint8_t lds[prolog_q_wide_lds(TB)];
+    prolog_q_wide_body<TB>(p, 2 * blockIdx.x, blockIdx.y * 32 * TB, lds);
 }
 
 // ------------------------------------------------------------------------------------------------ q_b[:, head, :128] @ w_uk[head]
@@ -1094,20 +1104,28 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
             if (p && a.t <= BIG_T2) {
                 hipLaunchKernelGGL(fused_qb_big_kernel, dim3(qgrid.x + p->n, qgrid.y), dim3(256), 0, stream, a, *p);
             } else {
-                const int cols = (a.n * MQH + 255) / 256, qcols = p ? (p->n + 1) / 2 : 0;
+                const int cols = (a.n * MQH + 255) / 256, qcols = p ? (p->n + 1) / 2 : 0, stages = a.r / GT_KI8;
+                const GtPlan alone = gt_token_blocks(a.t, cols, stages, 8), q_alone = gt_token_blocks(a.t, qcols, stages, 7);
+                const GtPlan both = gt_token_blocks(a.t, cols + qcols, stages, 7);
                 if (a.t <= BIG_T2)
                     hipLaunchKernelGGL(mla_qb_big_kernel<QB_DEPTH>, qgrid, dim3(256), 0, stream, a);
-                else if (p)
-                    gt_dispatch(gt_token_blocks(a.t, cols + qcols, a.r / GT_KI8, 7), [&](auto tb) {
+                else if (p && (both.ns <= alone.ns + q_alone.ns || a.t >= FUSED_T))
+                    gt_dispatch(both.tb, [&](auto tb) {
                         constexpr int TB = decltype(tb)::value < 7 ? decltype(tb)::value : 7;
                         hipLaunchKernelGGL(fused_qb_wide_kernel<TB>, dim3(qcols + cols, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream,
                                            a, *p);
                     });
-                else
-                    gt_dispatch(gt_token_blocks(a.t, cols, a.r / GT_KI8, 8), [&](auto tb) {
+                else {
+                    gt_dispatch(alone.tb, [&](auto tb) {
                         constexpr int TB = decltype(tb)::value;
                         hipLaunchKernelGGL(mla_qb_wide_kernel<TB>, dim3(cols, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream, a);
                     });
+                    if (p)
+                        gt_dispatch(q_alone.tb, [&](auto tb) {
+                            constexpr int TB = decltype(tb)::value < 7 ? decltype(tb)::value : 7;
+                            hipLaunchKernelGGL(fused_q_wide_kernel<TB>, dim3(qcols, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream, *p);
+                        });
+                }
             }
         } else if (p) {
             hipLaunchKernelGGL(fused_qb_kernel, dim3(a.n * MQH / 128 + p->n), dim3(256), 0, stream, a, *p);

@@ -164,6 +164,15 @@ def test_prefill_index_query_tiles(cuda, t, n, r, h):
     check_against_oracle(mla_case, idx_case, fused)
 
 
+@pytest.mark.parametrize("t,n", [(775, 64), (1447, 16), (1762, 8)])
+def test_prefill_products_in_two_launches(cuda, t, n):
+    # shapes where one launch over both int8 products would take a round of workgroups more than one for each
+    mla_case, idx_case = op.make_fused_case(t, 1, 64, seed=80 + n, n_idx=64, h=256, q_lora_rank=128, n=n)
+    fused = run_fused(mla_case, idx_case, cuda, entry="mla_indexer_prolog_quant_p")
+    same_as_separate(fused, run_separate(mla_case, idx_case, cuda), idx_case)
+    check_against_oracle(mla_case, idx_case, fused)
+
+
 def test_index_head_counts_without_the_side_by_side_kernels(cuda):
     # 32 index heads: x @ w_proj is half an output tile wide, so the fused entry runs the two operators back to back
     mla_case, idx_case = op.make_fused_case(5, 1, 300, seed=23, n_idx=32, h=512, q_lora_rank=256, n=4)
