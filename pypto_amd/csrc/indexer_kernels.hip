@@ -150,21 +150,21 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v)
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// The workgroup's histograms (S1 query tokens, one span of keys) go to its own slots, as 16-bit counts (a span has at
-// most 4096 keys), two per lane.  The span-0 workgroup also clears the select kernel's list counters of its query tokens and
-// leaves it the (logarithm of the) passes of a span.  256 lanes.
+// The workgroup's histograms (S1 query tokens, `slots` runs of keys from slot `first` on) go to its own slots, as 16-bit counts (a
+// slot has at most 2048 keys), two per lane.  The first workgroup of a sequence also clears the select kernel's list counters of
+// its query tokens.  256 lanes.
 template <int S1>
-__device__ __forceinline__ void flush_span_hist(const IndexerArgs& a, const uint32_t (*hist)[SBINS], int row0, int span, int passes_log2, int tid)
+__device__ __forceinline__ void flush_span_hist(const IndexerArgs& a, const uint32_t (*hist)[S1][SBINS], int row0, int first, int slots, int tid)
 {
     if (tid < SBINS / 2) {
+        for (int h = 0; h < slots; ++h)
 #pragma unroll
-        for (int s = 0; s < S1; ++s) {
-            const int64_t slot = (int64_t)(row0 + s) * a.pchunks + span;
-            reinterpret_cast<uint32_t*>(a.span_hist + slot * SBINS)[tid] = hist[s][2 * tid] | (hist[s][2 * tid + 1] << 16);
-        }
+            for (int s = 0; s < S1; ++s) {
+                const int64_t slot = (int64_t)(row0 + s) * a.pchunks + first + h;
+                reinterpret_cast<uint32_t*>(a.span_hist + slot * SBINS)[tid] = hist[h][s][2 * tid] | (hist[h][s][2 * tid + 1] << 16);
+            }
     }
-    if (span == 0 && tid < 4 * S1) a.counters[(int64_t)row0 * 4 + tid] = 0u;
-    if (span == 0 && tid == 0) *a.passes_log2 = (uint32_t)passes_log2; // (every sequence's workgroup writes the same)
+    if (first == 0 && tid < 4 * S1) a.counters[(int64_t)row0 * 4 + tid] = 0u;
 }
 
 // S1 query tokens of one sequence share every key fragment.
@@ -172,7 +172,7 @@ __device__ __forceinline__ void flush_span_hist(const IndexerArgs& a, const uint
 template <int S1, bool POW2, bool F32>
 __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a)
 {
-    __shared__ __align__(16) uint32_t hist[S1][SBINS];
+    __shared__ __align__(16) uint32_t hist[1][S1][SBINS];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, g = lane >> 4;
     const int bi = blockIdx.y;
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a)
     if (blockIdx.x * (CHUNK * PASSES) >= L) return;
     const int row0 = bi * a.s1 + sgrp * S1;
 
-    for (int i = tid; i < S1 * SBINS; i += 256) (&hist[0][0])[i] = 0;
+    for (int i = tid; i < S1 * SBINS; i += 256) (&hist[0][0][0])[i] = 0;
 
     // int8 A fragments: head hb*16 + l16, bytes 64*ks + 16*g .. +15
     i32x4 qf[S1][4][2];
@@ -262,13 +262,13 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a)
             if (ok && g == 0) {
                 const float sc = sum[0] * (present[j] ? ScaleOf<F32>::f32(ksb[j]) : 0.f);
                 a.scores[(int64_t)(row0 + s) * a.score_stride + tok] = sc;
-                if (a.use_hist && tok < eff) atomicAdd(&hist[s][score_bin(score_key(sc))], 1u);
+                if (a.use_hist && tok < eff) atomicAdd(&hist[0][s][score_bin(score_key(sc))], 1u);
             }
         }
     }
     } // pass
     __syncthreads();
-    if (a.use_hist) flush_span_hist<S1>(a, hist, row0, (int)blockIdx.x, __builtin_ctz(PASSES), tid);
+    if (a.use_hist) flush_span_hist<S1>(a, hist, row0, (int)blockIdx.x, 1, tid);
 }
 
 // relu(a) * 2^-11 and relu(b) * 2^-11, each rounded once to fp16, packed (a in the low half).  The int32 sums arrive
@@ -306,7 +306,8 @@ constexpr int SCAN_SEQS = 256; // sequences whose lengths a wavefront looks at
 template <int S1, bool F32, int PPASSES, bool MAY>
 __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kernel(IndexerArgs a)
 {
-    __shared__ __align__(16) uint32_t hist[S1][SBINS];
+    constexpr int SLOT = PPASSES < PASSES ? PPASSES : PASSES; // passes to a histogram slot
+    __shared__ __align__(16) uint32_t hist[PPASSES / SLOT][S1][SBINS];
     __shared__ __align__(16) float s_sc[S1][CHUNK * PPASSES]; // the workgroup's scores, written out in one burst at the end
     __shared__ __align__(16) uint8_t s_keys[4][64 * D];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -460,7 +461,7 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
                 wa[s][mm] = __builtin_shufflevector(qlo * wlo, qhi * whi, 0, 1, 2, 3, 4, 5, 6, 7);
             }
         }
-    for (int i = tid; i < S1 * SBINS; i += 256) (&hist[0][0])[i] = 0;
+    for (int i = tid; i < PPASSES / SLOT * S1 * SBINS; i += 256) (&hist[0][0][0])[i] = 0;
     __syncthreads();
 
     auto compute_half = [&](int hh, typename ScaleOf<F32>::raw ksc) {
@@ -495,7 +496,7 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
             const float sc = res[s] * ks;
             s_sc[s][tok - span * span_keys] = sc;
             const int eff = L - (a.s1 - 1 - (sgrp * S1 + s));
-            if (a.use_hist && tok < eff) atomicAdd(&hist[s][score_bin(score_key(sc))], 1u);
+            if (a.use_hist && tok < eff) atomicAdd(&hist[hh / (2 * SLOT)][s][score_bin(score_key(sc))], 1u);
         }
     };
 
@@ -527,7 +528,7 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
             if (4 * (tid + 256 * i) < span_keys)
                 *reinterpret_cast<f32x4*>(dst + 4 * (tid + 256 * i)) = *reinterpret_cast<const f32x4*>(&s_sc[s][4 * (tid + 256 * i)]);
     }
-    if (a.use_hist) flush_span_hist<S1>(a, hist, row0, span, passes_log2, tid);
+    if (a.use_hist) flush_span_hist<S1>(a, hist, row0, span * passes / SLOT, max(passes / SLOT, 1), tid);
 }
 
 __global__ void indexer_fill_kernel(int32_t* p, int n, int32_t v)
@@ -586,7 +587,6 @@ __global__ __launch_bounds__(256) void indexer_select_kernel(IndexerArgs a)
     constexpr int GROUP = 32;
     const int sg = tid >> 5, oct = tid & 31;
     const uint16_t* sh = a.span_hist + (int64_t)row * a.pchunks * SBINS + 8 * oct;
-    const int shift = __builtin_ctz(CHUNK) + (int)(*a.passes_log2 & 15u); // (not written, and not used, if no sequence has keys)
     u32x4 cv[GROUP / 8];
 #pragma unroll
     for (int j = 0; j < GROUP / 8; ++j) cv[j] = *reinterpret_cast<const u32x4*>(sh + (int64_t)min(sg + 8 * j, a.pchunks - 1) * SBINS);
@@ -599,7 +599,8 @@ __global__ __launch_bounds__(256) void indexer_select_kernel(IndexerArgs a)
     const int n = max(len - (a.s1 - 1 - (row - bi * a.s1)), 0);
     // (a workgroup past the row's end leaves further down, behind the first use of what was requested above: an exit
     // here would let the compiler move those requests behind the wait for the length - two round trips instead of one)
-    const int nsp = n > 0 ? min(((len - 1) >> shift) + 1, a.pchunks) : 0; // spans whose workgroup ran
+    const int slot_keys = CHUNK * a.min_passes;
+    const int nsp = min((len + slot_keys - 1) / slot_keys, a.pchunks); // slots whose workgroup ran
     if (tid == 0) s_bin = 0xffffffffu; // n <= k: no threshold bin, everything is a winner
 
     uint32_t acc[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
@@ -1300,7 +1301,7 @@ hipError_t topk_launch(const float* x, float* values, int32_t* indices, int64_t 
 }
 
 // workspace: scores [t, stride] f32 | span_hist [t, spans, 256] u16 | counters [t, 4] u32 | winners [t, 2048] u64 |
-// ties [t, 8192] u64 | passes_log2 u32; spans = stride / span
+// ties [t, 8192] u64; spans: histogram slots
 static uint64_t align256(uint64_t x) { return (x + 255) & ~(uint64_t)255; }
 
 // Passes of 512 keys per workgroup of the paged score kernel: as many as leave SCORE_GROUPS workgroups, eight at most.  Where
@@ -1321,7 +1322,7 @@ uint64_t indexer_workspace_bytes(int b, int s1, int stride)
     const int passes = pick_passes(b, s1, stride);
     const uint64_t spans = (uint64_t)stride / (CHUNK * std::min(passes, PASSES)); // (the unpaged kernel's spans: PASSES)
     return align256((uint64_t)t * stride * 4) + align256((uint64_t)t * spans * SBINS * 2) + align256((uint64_t)t * 4 * 4) +
-           align256((uint64_t)t * (MAX_K + TIE_CAP) * 8) + 256;
+           align256((uint64_t)t * (MAX_K + TIE_CAP) * 8);
 }
 
 void indexer_bind_workspace(IndexerArgs& a, void* ws)
@@ -1338,8 +1339,6 @@ void indexer_bind_workspace(IndexerArgs& a, void* ws)
     p += align256((uint64_t)t * 4 * 4);
     a.winners = reinterpret_cast<uint64_t*>(p);
     a.ties = a.winners + (uint64_t)t * MAX_K;
-    p += align256((uint64_t)t * (MAX_K + TIE_CAP) * 8);
-    a.passes_log2 = reinterpret_cast<uint32_t*>(p);
     a.pchunks = (int32_t)spans;
 }
 

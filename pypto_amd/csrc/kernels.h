@@ -53,14 +53,13 @@ struct IndexerArgs {
     uint32_t* counters;          // workspace [t, 4]: winners, ties (cleared by the score kernel)
     uint64_t* winners;           // workspace [t, 2048]
     uint64_t* ties;              // workspace [t, 8192]
-    uint32_t* passes_log2;       // workspace: of a span (the score kernel's choice)
     int64_t n_blocks;
     int32_t b, s1, nh, block_size, bt_stride, k, score_stride;
     int32_t max_ctx; // set by indexer_launch: bt_stride * block_size, the longest sequence the page table can address
     bool scales_f32; // q_scale and k_scale are fp32: w_scale = fp16(q_scale * fp32(weight)), k_scale enters the score as it is
     int32_t span;    // set by indexer_bind_workspace: keys per workgroup of the score kernel for full page tables
-    int32_t pchunks; // set by indexer_bind_workspace: histogram slots (spans of keys) per query token
-    int32_t min_passes; // set by indexer_launch: passes of 512 keys per workgroup of the score kernel at least
+    int32_t pchunks; // set by indexer_bind_workspace: histogram slots per query token
+    int32_t min_passes; // set by indexer_launch: passes of 512 keys per workgroup of the score kernel at least (with histograms: to a slot)
     bool use_hist;   // set by indexer_launch: the selection needs the score kernel's histograms
 };
 
