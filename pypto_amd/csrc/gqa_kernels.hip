@@ -21,8 +21,8 @@
 // waited for the sub-tile in flight as well (loads complete in order): 1077 -> 868 us.
 //   Chunks are chosen on the device from the lengths (choose_chunk): as long as they can be while the workgroups fill the
 // chip a whole number of times.  Two row tiles per workgroup (two query tokens of a sequence) share every K and V byte.
-//   64 sequences of 4096 .. 32768 tokens, 96 / 8 heads: 1090 us with fixed chunks of 1024, 796 now (4.8 GB); 8
-// sequences up to 8192, 12 / 1 heads: 21 us, 13.5 now, most of it the chain lengths - page table - keys - merge.
+//   64 sequences of 4096 .. 32768 tokens, 96 / 8 heads: 1090 us with fixed chunks of 1024, 797 now (4.8 GB); 8
+// sequences up to 8192, 12 / 1 heads: 19.5 us, 13 now, most of it the chain lengths - page table - keys - merge.
 //
 //   S^T[token, head] = K Q^T : v_mfma_f32_16x16x32_bf16, A = K rows (lane = token l%16, 8 dims at 8*(l/16) + 32*j), B = Q
 //       (resident, heads padded to 16).

@@ -16,8 +16,11 @@
 // (v_mfma_f32_16x16x32_f16: row 0 of A holds w_scale, B is the fp16 tile just produced; every product of two
 // fp16 values is exact in fp32, so this is the golden's fp32 sum up to the order of additions).  Scores go to
 // a dense fp32 row per query token, and their order-preserving keys into a 256-bin histogram in LDS (score_bin:
-// quarter octaves).  Every workgroup owns a span of its sequence's keys and leaves its histogram in a slot of
+// quarter octaves).  Every workgroup owns a span of its sequence's keys and leaves its histogram in one or two slots of
 // its own in the workspace (16-bit counts): plain stores, nothing to clear beforehand and no global atomics.
+//
+// Score rows of up to 32768 keys (by the page table's reach) are selected by one kernel (indexer_row_topk_kernel), without
+// histograms; longer ones by two:
 //
 // indexer_select_kernel: every workgroup adds up the spans' histograms of its query token, finds the bin B that
 // holds the k-th largest key, and files its 4096 scores: bins above B are winners, bin B goes to a tie list (both
@@ -26,7 +29,7 @@
 //
 // indexer_topk_kernel: one workgroup per query token takes the winners, picks the missing krem entries out of
 // the tie list by radix-selecting on the 64-bit words (key << 32 | ~index) (so equal keys resolve to the
-// smaller index), and bitonic-sorts the k words.  A tie list that overflowed its capacity (e.g. all scores
+// smaller index), and puts the k words in order (order_words).  A tie list that overflowed its capacity (e.g. all scores
 // equal) falls back to radix-selecting over the whole score row.
 #include <algorithm>
 #include <type_traits>
@@ -295,10 +298,10 @@ __device__ __forceinline__ uint32_t relu_scale_pack(int a, int b)
 // in every row of the head-sum operand, so every lane group holds the 16 scores of a key group and lane group g keeps those
 // of key group g - after four key groups lane l holds the score of key l of the 64, next to that key's scale (loaded with one
 // 128-byte instruction per 64 keys).
-// A workgroup takes `passes` passes of 512 keys, as score_passes has it for the batch's lengths: PPASSES, what it has for full
-// page tables, or fewer (where the selection needs the spans' histograms, no fewer than there are slots for).  Short contexts under
-// wide tables would otherwise be few long workgroups (32 sequences of 8192 keys under 1024 columns: 24.7 us with spans of
-// 4096 keys).
+// A workgroup takes `passes` passes of 512 keys: PPASSES, pick_passes' choice for full page tables, or fewer, by the lengths, while
+// there would be fewer than SCORE_GROUPS_MIN workgroups (where the selection needs histograms, no fewer than fill a slot).  Short
+// contexts under wide tables would otherwise be few long workgroups (32 sequences of 8192 keys under 1024 columns: 24.7 us
+// with spans of 4096 keys, 14.7 with 2048).
 // MAY: loads past the caches' retention, where the batch's keys do not fit the last-level cache - which needs the whole-row
 // loads: taken in operand layout, a row is two loads of half a cache line, and a line that is not kept in between is fetched
 // twice (32 x 64 K keys, 272 MB: 56.8 us in operand layout, 65.0 with non-temporal loads; 57.8 and 52.7 this way).

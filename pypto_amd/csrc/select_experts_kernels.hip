@@ -3,8 +3,9 @@
 // python/tests/ut/interpreter/_ops/moe_gating_topk.py:223-287 (groups, -inf fill, scaling factor).
 //
 // The whole problem is a few MB (8192 x 160 logits): what bounds the kernels is vector instruction issue (many tokens) and
-// the length of one wavefront's instruction chain (few), both mostly the sigmoid and the arg-max rounds.  Groups are ranked by counting (rank of g = number of groups that come before g
-// in the order "value descending, index ascending"), experts by top_k rounds of an arg-max on (ordered score, ~id).
+// the length of one wavefront's instruction chain (few), both mostly the sigmoid and the choice of the experts.  Groups are ranked
+// by counting (rank of g = number of groups that come before g in the order "value descending, index ascending"), experts by
+// merging sorted lists of (ordered score, ~id), or by top_k rounds of an arg-max on them where more than eight are selected.
 // select_experts_rows_kernel puts four tokens in a wavefront (the router's shapes); select_experts_kernel, one token per
 // wavefront, takes the shapes with more than 16 groups or 16 selected experts.
 #include <hip/hip_runtime.h>
@@ -183,8 +184,8 @@ __global__ __launch_bounds__(64) void select_experts_kernel(SelectExpertsArgs a)
 // Up to eight selected experts (TOP8): every lane sorts its own and keeps eight, and four merges with the lanes 8, 4, 2 and 1
 // places away leave the row's eight in order in all of its lanes - about 300 instructions where eight arg-max rounds over
 // score and id took 800.  More: rounds of an arg-max.  The selected experts' sigmoid values are read back from LDS.
-// 8192 tokens x 160 experts, 8 of 4 of 8 groups: 11.1 us with the library's exp and the rounds, 7.7 now; 8 tokens: 9.2
-// us, 4.8 now (what is left is one wavefront's chain: loads, 33 dependent double-precision steps, the merges).
+// A call with 160 experts, 8 of 4 of 8 groups: 8192 tokens 10.2 us with the library's exp and the rounds, 7.0 now; 8 tokens
+// 7.6, 5.2 now (what is left is one wavefront's chain: loads, 33 dependent double-precision steps, the merges).
 template <int N>
 __device__ __forceinline__ uint32_t row_ror(uint32_t v)
 {

@@ -71,6 +71,13 @@ def test_row_slices_that_start_off_a_16_byte_boundary(cuda):
     assert torch.equal(idx.cpu(), gi) and torch.equal(vals.cpu(), gv)
 
 
+@pytest.mark.parametrize("n,k", [(300_000, 2048), (1 << 20, 2048), (1 << 20, 64), ((1 << 24) - 3, 2048), (1 << 24, 1)])
+def test_rows_up_to_the_longest(cuda, n, k):
+    # beyond some 400 K elements the sampled pivot cannot hold 2048 of them and the row is selected by counting passes
+    g = torch.Generator().manual_seed(n + k)
+    check(torch.randn((1, n), generator=g), k, None, True, cuda)
+
+
 def test_long_rows_go_through_the_radix_select(cuda):
     g = torch.Generator().manual_seed(6)
     x = torch.randn((3, 131072), generator=g)
