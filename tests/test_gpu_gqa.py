@@ -103,6 +103,27 @@ def test_forced_chunks_agree(cuda):
         check(out.cpu(), case, f"chunk {chunk}")
 
 
+@pytest.mark.parametrize("act,cols", [([3000, 500], 2000), ([3, 200] * 130 + [700], 100)])
+def test_forced_chunks_under_a_wide_page_table(cuda, act, cols):
+    # more units than workgroups: walked by lengths (few sequences) and by the chunks' places (many)
+    from pypto_amd import _runtime
+    lib = _runtime.load_library()
+    case = gqa.make_case(len(act), 1, 12, 1, act, seed=len(act))
+    bt = case["block_table"]
+    wide = torch.full((len(act), cols), -1, dtype=bt.dtype)
+    wide[:, :bt.shape[1]] = bt
+    ts = [case["q"].to(cuda), case["k"].to(cuda), case["v"].to(cuda), wide.to(cuda), torch.tensor(act, dtype=torch.int32, device=cuda)]
+    out = torch.zeros_like(ts[0])
+    d = _runtime.describe(ts + [out])
+    p = _runtime.GqaParams(case["softmax_scale"], 128)
+    n = lib.pto_gqa_decode_workspace(d, 6, ctypes.byref(p))
+    ws = torch.empty(n, dtype=torch.uint8, device=cuda)
+    rc = lib.pto_gqa_decode_launch(d, 6, ctypes.byref(p), ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream, 0)
+    assert rc == 0, lib.pto_last_error()
+    torch.cuda.synchronize()
+    check(out.cpu(), case, f"{len(act)} sequences, {cols} columns")
+
+
 def test_full_size_config4_sample(cuda):
     # the benchmark's GQA configuration (b=64, 96/8 heads, contexts U[4096, 32768]); the oracle checks 6 of the sequences
     g = torch.Generator().manual_seed(44)
@@ -159,9 +180,12 @@ def test_keys_beyond_the_last_level_cache(cuda):
 
 
 @pytest.mark.parametrize("s1,nq,nkv,act,cols", [(1, 12, 1, [3, 200] * 150 + [9000], 2100), (2, 12, 1, [3, 200] * 150 + [9000], 700),
-                                                (1, 12, 1, [5, 300, 0, 129] * 10, 3000), (2, 24, 2, [700, 4097], 8192), (1, 96, 8, [300] * 40, 1024)])
+                                                (1, 12, 1, [5, 300, 0, 129] * 10, 3000), (2, 24, 2, [700, 4097], 8192), (1, 96, 8, [300] * 40, 1024),
+                                                (1, 8, 8, [3, 200] * 150 + [9000], 2100), (2, 96, 8, [60, 3] * 20, 1024),
+                                                (2, 8, 8, [3, 40] * 550, 600)])
 def test_page_tables_wider_than_the_contexts(cuda, s1, nq, nkv, act, cols):
-    # a serving loop's page tables, as wide as its longest context may get, over short contexts
+    # a serving loop's page tables, as wide as its longest context may get, over short contexts: workgroups that walk the units
+    # (one and two row tiles, batches that the device-side choice takes and larger ones), some of them with a second one
     case = gqa.make_case(len(act), s1, nq, nkv, act, seed=len(act) + cols)
     bt = case["block_table"]
     wide = torch.full((len(act), cols), -1, dtype=bt.dtype)
