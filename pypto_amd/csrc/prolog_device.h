@@ -49,6 +49,102 @@ __device__ __forceinline__ void rope_tile(uint8_t* xt, const uint16_t* csl, int 
     }
 }
 
+// What follows the index query's product for one head and 32 TB tokens, 256 lanes (ht), on the bf16 tile xt [32 TB][XROW] - the one
+// place for the operations behind every form of the product: Hadamard and quantisation here, the rotary embedding in front of them in
+// prolog_q_finish (from memory) or rope_tile (from LDS).  had: hadamard_q, smax: per-wave maxima.  Every lane of the workgroup
+// passes its barriers; heads past the last one are dropped.
+template <int TB>
+__device__ __forceinline__ void prolog_q_quantise(const PrologArgs& a, int head, int tok0, int ht, const uint8_t* had, const uint8_t* xt,
+                                                  float (*smax)[32 * TB])
+{
+#pragma clang fp contract(off)
+    const int lane = ht & 63, hwave = ht >> 6, l32 = lane & 31, hl = lane >> 5;
+    // Y^T[n, token] = H^T[n, k] . X^T[k, token]: wave w of a head owns n in [32 w, 32 w + 32) for the blocks of 32 tokens.  A (H^T) by
+    // transposing reads of the row-major H: lane jj of 16-lane group G points at row k0 + 4 hl + jj / 4 (+ 8), columns 32 w + 16 (G & 1)
+    // + 4 (jj & 3); they hand lane half hl the contraction rows {4 hl .. 4 hl + 3} and {8 + 4 hl .. 8 + 4 hl + 3} of a 16-row step, so
+    // the B operand takes the same rows of X: two 8-byte pieces
+    f32x16 y[TB];
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) y[tb][e] = 0.f;
+    {
+        const int jj = lane & 15, mh = (lane >> 4) & 1;
+        const uint8_t* hp = had + (4 * hl + (jj >> 2)) * (PD * 2) + (32 * hwave + 16 * mh + 4 * (jj & 3)) * 2;
+        const uint8_t* xp = xt + l32 * XROW + hl * 8;
+#pragma unroll
+        for (int ks = 0; ks < PD / 16; ++ks) {
+            const s16x4 lo = lds_read_tr(hp + ks * 16 * (PD * 2));
+            const s16x4 hi = lds_read_tr(hp + (ks * 16 + 8) * (PD * 2));
+            const bf16x8 av = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb) {
+                const u32x2 b0 = *reinterpret_cast<const u32x2*>(xp + 32 * tb * XROW + ks * 32);
+                const u32x2 b1 = *reinterpret_cast<const u32x2*>(xp + 32 * tb * XROW + ks * 32 + 16);
+                const bf16x8 bv = __builtin_bit_cast(bf16x8, u32x4{b0[0], b0[1], b1[0], b1[1]});
+                y[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, y[tb], 0, 0, 0);
+            }
+        }
+    }
+    // register e of y[tb]: n = 32 w + 8 (e/4) + 4 hl + e%4, token 32 tb + l32.  Round to bf16, per-token absmax over the 128 n
+    float mx[TB];
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) {
+        mx[tb] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            y[tb][e] = bf16_to_f32(f32_to_bf16(y[tb][e]));
+            mx[tb] = fmaxf(mx[tb], fabsf(y[tb][e]));
+        }
+        mx[tb] = fmaxf(mx[tb], __shfl_xor(mx[tb], 32));
+        if (hl == 0) smax[hwave][32 * tb + l32] = mx[tb];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) {
+        const int tl = 32 * tb + l32;
+        const float m = fmaxf(fmaxf(smax[0][tl], smax[1][tl]), fmaxf(smax[2][tl], smax[3][tl]));
+        const float sq = quant_scale(m);
+        const int gt = tok0 + tl;
+        if (gt < a.t && head < a.n) {
+            int8_t* qo = a.q_int8 + ((int64_t)gt * a.n + head) * PD + 32 * hwave + 4 * hl;
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) {
+                uint32_t pk = 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(y[tb][4 * e4 + e] * sq) & 0xffu) << (8 * e);
+                *reinterpret_cast<uint32_t*>(qo + 8 * e4) = pk;
+            }
+            if (hwave == 0 && hl == 0) a.q_scale[(int64_t)gt * a.n + head] = __builtin_bit_cast(uint16_t, (_Float16)(1.0f / sq));
+        }
+    }
+}
+template <int TB>
+__device__ __forceinline__ void prolog_q_finish(const PrologArgs& a, int head, int tok0, int ht, const uint8_t* had, uint8_t* xt,
+                                                float (*smax)[32 * TB])
+{
+#pragma clang fp contract(off)
+    // rotary on the first 64 dims: 32 pairs a token (the arithmetic of rope_tile)
+#pragma unroll 4
+    for (int it = 0; it < TB * 32 * 32 / 256; ++it) {
+        const int item = ht + 256 * it;
+        const int tok = item >> 5, i = item & 31;
+        uint16_t* row = reinterpret_cast<uint16_t*>(xt + tok * XROW);
+        const int64_t gtc = (int64_t)min(tok0 + tok, a.t - 1) * PROPE;
+        const uint16_t* cosp = a.cos + gtc;
+        const uint16_t* sinp = a.sin + gtc;
+        const float x1 = bf16_to_f32(row[i]), x2 = bf16_to_f32(row[i + 32]);
+        const float c1 = bf16_to_f32(cosp[i]), c2 = bf16_to_f32(cosp[i + 32]);
+        const float s1 = bf16_to_f32(sinp[i]), s2 = bf16_to_f32(sinp[i + 32]);
+        const float o1 = x1 * c1 + (-x2) * s1;
+        const float o2 = x2 * c2 + x1 * s2;
+        row[i] = f32_to_bf16(o1);
+        row[i + 32] = f32_to_bf16(o2);
+    }
+    __syncthreads();
+    prolog_q_quantise<TB>(a, head, tok0, ht, had, xt, smax);
+}
+
 // ------------------------------------------------------------------------------------------------ query path
 // One workgroup of 1024 lanes = 4 groups of 4 wavefronts per (head, token tile of 32); plds is its dynamic LDS
 // (prolog_q_lds_bytes).
@@ -197,54 +293,7 @@ __device__ __forceinline__ void prolog_q_body(const PrologArgs& a, int head, int
     __syncthreads();
     rope_tile(xt, csl, tid);
     __syncthreads();
-
-    // Y^T[n, token] = H^T[n, k] . X^T[k, token]: wave w owns n in [32 w, 32 w + 32).  A (H^T) by transposing reads of
-    // the row-major H: lane jj of 16-lane group G points at row k0 + 4*hl + jj/4 (+ 8), columns 32 w + 16 (G&1) + 4 (jj&3)
-    f32x16 y;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) y[e] = 0.f;
-    {
-        const int jj = lane & 15, mh = (lane >> 4) & 1;
-        const uint8_t* hp = had + (4 * hl + (jj >> 2)) * (PD * 2) + (32 * wave + 16 * mh + 4 * (jj & 3)) * 2;
-        // the transposing reads hand lane half hl the contraction rows {4 hl .. 4 hl + 3} and {8 + 4 hl .. 8 + 4 hl + 3} of
-        // a 16-row step, so the B operand takes the same rows of X: two 8-byte pieces
-        const uint8_t* xp = xt + l32 * XROW + hl * 8;
-#pragma unroll
-        for (int ks = 0; ks < PD / 16; ++ks) {
-            const s16x4 lo = lds_read_tr(hp + ks * 16 * (PD * 2));
-            const s16x4 hi = lds_read_tr(hp + (ks * 16 + 8) * (PD * 2));
-            const bf16x8 av = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            const u32x2 b0 = *reinterpret_cast<const u32x2*>(xp + ks * 32);
-            const u32x2 b1 = *reinterpret_cast<const u32x2*>(xp + ks * 32 + 16);
-            const bf16x8 bv = __builtin_bit_cast(bf16x8, u32x4{b0[0], b0[1], b1[0], b1[1]});
-            y = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, y, 0, 0, 0);
-        }
-    }
-    // register e: n = 32 w + 8 (e/4) + 4 hl + e%4, token l32.  Round to bf16, then per-token absmax over the 128 n
-    float yb[16], mx = 0.f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        yb[e] = bf16_to_f32(f32_to_bf16(y[e]));
-        mx = fmaxf(mx, fabsf(yb[e]));
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    if (hl == 0) smax[wave][l32] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(smax[0][l32], smax[1][l32]), fmaxf(smax[2][l32], smax[3][l32]));
-    const float sq = quant_scale(mx);
-    const int gt = tok0 + l32;
-    if (gt < a.t) {
-        int8_t* qo = a.q_int8 + ((int64_t)gt * a.n + head) * PD + 32 * wave + 4 * hl;
-#pragma unroll
-        for (int e4 = 0; e4 < 4; ++e4) {
-            uint32_t pk = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(yb[4 * e4 + e] * sq) & 0xffu) << (8 * e);
-            *reinterpret_cast<uint32_t*>(qo + 8 * e4) = pk;
-        }
-        if (wave == 0 && hl == 0)
-            a.q_scale[(int64_t)gt * a.n + head] = __builtin_bit_cast(uint16_t, (_Float16)(1.0f / sq));
-    }
+    prolog_q_quantise<1>(a, head, tok0, tid, had, xt, smax);
 }
 
 // ------------------------------------------------------------------------------------------------ query path, prefill sizes
@@ -359,167 +408,7 @@ __device__ __forceinline__ void prolog_q_big_body(const PrologArgs& a, int head,
         }
     }
     __syncthreads();
-    // rotary on the first 64 dims: 128 tokens x 32 pairs, 16 items per lane (the arithmetic of rope_tile)
-#pragma unroll 4
-    for (int it = 0; it < QB_TOK * 32 / 256; ++it) {
-        const int item = tid + 256 * it;
-        const int tok = item >> 5, i = item & 31;
-        uint16_t* row = reinterpret_cast<uint16_t*>(xt + tok * XROW);
-        const int64_t gtc = (int64_t)min(tok0 + tok, a.t - 1) * PROPE;
-        const uint16_t* cosp = a.cos + gtc;
-        const uint16_t* sinp = a.sin + gtc;
-        const float x1 = bf16_to_f32(row[i]), x2 = bf16_to_f32(row[i + 32]);
-        const float c1 = bf16_to_f32(cosp[i]), c2 = bf16_to_f32(cosp[i + 32]);
-        const float s1 = bf16_to_f32(sinp[i]), s2 = bf16_to_f32(sinp[i + 32]);
-        const float o1 = x1 * c1 + (-x2) * s1;
-        const float o2 = x2 * c2 + x1 * s2;
-        row[i] = f32_to_bf16(o1);
-        row[i + 32] = f32_to_bf16(o2);
-    }
-    __syncthreads();
-    // Y^T[n, token] = H^T[n, k] . X^T[k, token]: wave w owns n in [32 w, 32 w + 32) for the four blocks of 32 tokens
-    // (operand addressing as in prolog_q_body)
-    f32x16 y[4];
-#pragma unroll
-    for (int tb = 0; tb < 4; ++tb)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) y[tb][e] = 0.f;
-    {
-        const int jj = lane & 15, mh = (lane >> 4) & 1;
-        const uint8_t* hp = had + (4 * hl + (jj >> 2)) * (PD * 2) + (32 * wave + 16 * mh + 4 * (jj & 3)) * 2;
-        const uint8_t* xp = xt + l32 * XROW + hl * 8;
-#pragma unroll
-        for (int ks = 0; ks < PD / 16; ++ks) {
-            const s16x4 lo = lds_read_tr(hp + ks * 16 * (PD * 2));
-            const s16x4 hi = lds_read_tr(hp + (ks * 16 + 8) * (PD * 2));
-            const bf16x8 av = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-            for (int tb = 0; tb < 4; ++tb) {
-                const u32x2 b0 = *reinterpret_cast<const u32x2*>(xp + 32 * tb * XROW + ks * 32);
-                const u32x2 b1 = *reinterpret_cast<const u32x2*>(xp + 32 * tb * XROW + ks * 32 + 16);
-                const bf16x8 bv = __builtin_bit_cast(bf16x8, u32x4{b0[0], b0[1], b1[0], b1[1]});
-                y[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, y[tb], 0, 0, 0);
-            }
-        }
-    }
-    // register e of y[tb]: n = 32 w + 8 (e/4) + 4 hl + e%4, token 32 tb + l32.  Round to bf16, per-token absmax over the 128 n
-    float mx[4];
-#pragma unroll
-    for (int tb = 0; tb < 4; ++tb) {
-        mx[tb] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            y[tb][e] = bf16_to_f32(f32_to_bf16(y[tb][e]));
-            mx[tb] = fmaxf(mx[tb], fabsf(y[tb][e]));
-        }
-        mx[tb] = fmaxf(mx[tb], __shfl_xor(mx[tb], 32));
-        if (hl == 0) smax[wave][32 * tb + l32] = mx[tb];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int tb = 0; tb < 4; ++tb) {
-        const int tl = 32 * tb + l32;
-        const float m = fmaxf(fmaxf(smax[0][tl], smax[1][tl]), fmaxf(smax[2][tl], smax[3][tl]));
-        const float sq = quant_scale(m);
-        const int gt = tok0 + tl;
-        if (gt < a.t) {
-            int8_t* qo = a.q_int8 + ((int64_t)gt * a.n + head) * PD + 32 * wave + 4 * hl;
-#pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) {
-                uint32_t pk = 0;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(y[tb][4 * e4 + e] * sq) & 0xffu) << (8 * e);
-                *reinterpret_cast<uint32_t*>(qo + 8 * e4) = pk;
-            }
-            if (wave == 0 && hl == 0) a.q_scale[(int64_t)gt * a.n + head] = __builtin_bit_cast(uint16_t, (_Float16)(1.0f / sq));
-        }
-    }
-}
-// What follows the product for one head and TOK = 32 TB tokens, 256 lanes (ht): rotary, Hadamard, quantisation of the bf16 tile
-// xt [TOK][XROW]; had: hadamard_q, smax: per-wave maxima.  Every lane of the workgroup passes its barriers; heads past the last
-// one are dropped.
-template <int TB>
-__device__ __forceinline__ void prolog_q_finish(const PrologArgs& a, int head, int tok0, int ht, const uint8_t* had, uint8_t* xt,
-                                                float (*smax)[32 * TB])
-{
-#pragma clang fp contract(off)
-    constexpr int TOK = 32 * TB;
-    const int lane = ht & 63, hwave = ht >> 6, l32 = lane & 31, hl = lane >> 5;
-    // rotary on the first 64 dims: 32 pairs a token (the arithmetic of rope_tile)
-#pragma unroll 4
-    for (int it = 0; it < TOK * 32 / 256; ++it) {
-        const int item = ht + 256 * it;
-        const int tok = item >> 5, i = item & 31;
-        uint16_t* row = reinterpret_cast<uint16_t*>(xt + tok * XROW);
-        const int64_t gtc = (int64_t)min(tok0 + tok, a.t - 1) * PROPE;
-        const uint16_t* cosp = a.cos + gtc;
-        const uint16_t* sinp = a.sin + gtc;
-        const float x1 = bf16_to_f32(row[i]), x2 = bf16_to_f32(row[i + 32]);
-        const float c1 = bf16_to_f32(cosp[i]), c2 = bf16_to_f32(cosp[i + 32]);
-        const float s1 = bf16_to_f32(sinp[i]), s2 = bf16_to_f32(sinp[i + 32]);
-        const float o1 = x1 * c1 + (-x2) * s1;
-        const float o2 = x2 * c2 + x1 * s2;
-        row[i] = f32_to_bf16(o1);
-        row[i + 32] = f32_to_bf16(o2);
-    }
-    __syncthreads();
-    // Y^T[n, token] = H^T[n, k] . X^T[k, token]: wave w of a head owns n in [32 w, 32 w + 32) for the blocks of 32 tokens
-    // (operand addressing as in prolog_q_body)
-    f32x16 y[TB];
-#pragma unroll
-    for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) y[tb][e] = 0.f;
-    {
-        const int jj = lane & 15, mh = (lane >> 4) & 1;
-        const uint8_t* hp = had + (4 * hl + (jj >> 2)) * (PD * 2) + (32 * hwave + 16 * mh + 4 * (jj & 3)) * 2;
-        const uint8_t* xp = xt + l32 * XROW + hl * 8;
-#pragma unroll
-        for (int ks = 0; ks < PD / 16; ++ks) {
-            const s16x4 lo = lds_read_tr(hp + ks * 16 * (PD * 2));
-            const s16x4 hi = lds_read_tr(hp + (ks * 16 + 8) * (PD * 2));
-            const bf16x8 av = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-            for (int tb = 0; tb < TB; ++tb) {
-                const u32x2 b0 = *reinterpret_cast<const u32x2*>(xp + 32 * tb * XROW + ks * 32);
-                const u32x2 b1 = *reinterpret_cast<const u32x2*>(xp + 32 * tb * XROW + ks * 32 + 16);
-                const bf16x8 bv = __builtin_bit_cast(bf16x8, u32x4{b0[0], b0[1], b1[0], b1[1]});
-                y[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, y[tb], 0, 0, 0);
-            }
-        }
-    }
-    // register e of y[tb]: n = 32 w + 8 (e/4) + 4 hl + e%4, token 32 tb + l32.  Round to bf16, per-token absmax over the 128 n
-    float mx[TB];
-#pragma unroll
-    for (int tb = 0; tb < TB; ++tb) {
-        mx[tb] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            y[tb][e] = bf16_to_f32(f32_to_bf16(y[tb][e]));
-            mx[tb] = fmaxf(mx[tb], fabsf(y[tb][e]));
-        }
-        mx[tb] = fmaxf(mx[tb], __shfl_xor(mx[tb], 32));
-        if (hl == 0) smax[hwave][32 * tb + l32] = mx[tb];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int tb = 0; tb < TB; ++tb) {
-        const int tl = 32 * tb + l32;
-        const float m = fmaxf(fmaxf(smax[0][tl], smax[1][tl]), fmaxf(smax[2][tl], smax[3][tl]));
-        const float sq = quant_scale(m);
-        const int gt = tok0 + tl;
-        if (gt < a.t && head < a.n) {
-            int8_t* qo = a.q_int8 + ((int64_t)gt * a.n + head) * PD + 32 * hwave + 4 * hl;
-#pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) {
-                uint32_t pk = 0;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(y[tb][4 * e4 + e] * sq) & 0xffu) << (8 * e);
-                *reinterpret_cast<uint32_t*>(qo + 8 * e4) = pk;
-            }
-            if (hwave == 0 && hl == 0) a.q_scale[(int64_t)gt * a.n + head] = __builtin_bit_cast(uint16_t, (_Float16)(1.0f / sq));
-        }
-    }
+    prolog_q_finish<QB_TOK / 32>(a, head, tok0, tid, had, xt, smax);
 }
 
 // Above 256 tokens: 32 TB tokens x two heads per workgroup (gemm_tile.h), four waves to a head behind the product; the
