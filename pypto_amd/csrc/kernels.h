@@ -25,6 +25,8 @@ struct SfaArgs {
     int32_t b, s1, nq, topk, topk_stride, block_size, bt_stride, nsplit;
     int32_t split_cap; // set by sfa_launch: capacity (tokens) of the per-split LDS arrays
     int32_t bt_cached; // set by sfa_launch: the sequence's page table fits in LDS
+    uint32_t page_mul; // set by sfa_launch: idx / block_size = idx * page_mul >> page_shift
+    int32_t page_shift;
     float softmax_scale;
     bool quant;
 };

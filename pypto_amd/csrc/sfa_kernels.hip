@@ -11,25 +11,31 @@
 //
 // Work decomposition.  One workgroup of eight wavefronts owns one (query token, KV split, group of 128 heads) and
 // walks its share of the token's top-k list in tiles of 32 selected cache rows; every gathered row is dequantised
-// once for all 128 heads.  The dequantised tile sits row-major in LDS (16-byte chunks XOR-swizzled with the row),
-// double buffered, and serves as K (row reads) and as V (transposing reads, ds_read_b64_tr_b16).  All eight
-// wavefronts issue MFMAs (v_mfma_f32_32x32x16_bf16), two per SIMD, and each has two roles:
-//   * scores: wave (hg, kh) computes S^T = K Q^T for the 32 heads of group hg over half of the 576-wide
-//     contraction (nope columns [256 kh, 256 kh + 256) and rope columns [32 kh, 32 kh + 32)); its Q slice is the B
-//     operand, resident in registers but for a few k-steps parked in LDS;
-//   * values: wave (hh, dq) accumulates O^T = V^T P~ for the 64 heads of half hh and 128 of the 512 value
-//     columns (128 accumulator registers); every V^T fragment read from LDS feeds two MFMAs.
-// Between the two, per tile: the kh = 1 wave of a pair hands its partial S to the kh = 0 wave through LDS; the
-// kh = 0 wave runs the online softmax (one head per lane) and leaves P~ (bf16, already in B-operand order), the
-// rescale factors and a flag in LDS for the value role; and every wave produces its share of the next tile (four of
-// the 32 rows): dequantises it out of the registers its gather landed in, stores it to the other LDS stage and issues
-// the gather of the tile after.  Two workgroup barriers per tile.  All waves run the same phase at the same time on
-// purpose: two waves of a SIMD issuing MFMAs keep the matrix pipe fed (one wave alone gets its LDS operands at half
-// the rate), and two waves issuing vector work fill the vector port (one wave alone issues at about half its rate);
-// running the phases of two wave groups one barrier interval apart was measured and is slower.
+// once for all 128 heads.  The dequantised tile sits row-major in LDS (16-byte chunks XOR-swizzled with the row), three
+// tiles deep, and serves as K (row reads) and as V (transposing reads, ds_read_b64_tr_b16).  A SIMD holds a pair of
+// wavefronts, which owns 32 heads; the two do different work, so that one has vector and memory work to do while the other
+// issues MFMAs (v_mfma_f32_32x32x16_bf16):
+//   * the score wave holds Q (B operand, 30 of its 36 k-steps in registers, six parked in LDS), computes S^T = K Q^T over
+//     the whole contraction, runs the online softmax (one head per lane) and accumulates O^T = V^T P~ for the first 128
+//     value columns, with P~ straight out of its registers: S^T comes out in the B-operand order of the values product;
+//   * the value wave produces the tiles - eight of the 32 rows each: gather into registers, dequantisation, store to LDS -
+//     with the matrix instructions of the other 384 value columns between the pieces; P~ and the rescale factors come to it
+//     through LDS.
+// Between two barriers, one per tile: the scores and the softmax of tile i, the values of tile i - 1, the production of
+// tile i + 1 and the gather of tile i + 2.  Nothing is exchanged within a tile.
+//
+// What bounds it: nothing alone.  A tile takes 3450 ticks of a CU (1000 query tokens, 2048 rows each), of which the matrix
+// pipes are busy 2176, the vector ports about 2250 (380 instructions a SIMD and the matrix instructions' issue) and LDS
+// about 2100; the kernel before, whose eight wavefronts all went through the same phases between two barriers a tile,
+// took 5150.  Measured on the way: four wavefronts with 512 registers each, 32 heads and no pairs, 4170 (a single
+// wavefront's issue slots); eight of 16 heads with 16x16x32 instructions, 5460 (three operand fragments in flight are
+// too few); the value wave's products before or after its production 3660 and 3770, interleaved without its raised
+// priority 4060 (the older score wave takes every slot and then waits at the barrier).
 //
 // KV splits write their output normalised by their own sum as fp16, in the accumulators' fragment order, plus (m, l);
 // sfa_combine_kernel merges them and turns the result into rows.
+#include <utility>
+
 #include "common.h"
 #include "kernels.h"
 #include "timing.h"
@@ -40,38 +46,33 @@ namespace {
 constexpr int T = 32;                  // selected rows per tile
 constexpr int DN = 512;                // nope / value width
 constexpr int DR = 64;                 // rope width
-constexpr int KSTEPS = (DN + DR) / 16; // 36 MFMA k-steps for S, 18 per wave of a pair
+constexpr int KSTEPS = (DN + DR) / 16; // 36 MFMA k-steps for S
 constexpr int KROW = (DN + DR) * 2;    // 1152 bytes per tile row = 72 chunks of 16 bytes
 constexpr int STAGE = T * KROW;        // 36864
 constexpr int MAX_SPLIT_TOKENS = 2048; // largest share of a top-k list one workgroup may own
 constexpr int HEADS_PER_WG = 128;
-// of a wave's 18 k-steps of Q, NREG stay in registers and the others are parked in LDS (16 bytes per lane each): with
-// the 128 accumulator registers of the values role, the wave's share of a gathered tile and the operand fragments in
-// flight this is what fits the 256 registers a wave has at two waves per SIMD without spilling
-constexpr int NREG_SM = 12, NREG_PR = 12;
-// of the 8 tile rows a pair of waves produces, the KH = 1 wave takes NR_PR and the softmax wave the others
-constexpr int NR_PR = 4;
-// operand fragments read ahead of the MFMA that uses them, in the scores and in the values phase (deeper costs
-// registers the kernel does not have)
-constexpr int S_AHEAD = 2, PV_AHEAD = 1;
-constexpr int NPARK_SM = KSTEPS / 2 - NREG_SM, NPARK_PR = KSTEPS / 2 - NREG_PR;
-// LDS layout: two tile stages | partial S, 4 KB per head group | P~, 2 KB per head group | rescale factors [4][32],
-// flags [4] | parked Q | per-split arrays sized by SfaArgs::split_cap (validity words, rows) |
-// this sequence's page table (when it fits)
-constexpr int XBUF_OFF = 2 * STAGE;
-constexpr int PBUF_OFF = XBUF_OFF + 4 * 4096;
-constexpr int ALPHA_OFF = PBUF_OFF + 4 * 2048;
-constexpr int FLAG_OFF = ALPHA_OFF + 4 * 32 * 4;
-constexpr int QPARK_OFF = FLAG_OFF + 16;
-constexpr int SPLIT_OFF = QPARK_OFF + 4 * (NPARK_SM + NPARK_PR) * 1024;
+constexpr int WAVES = 8, PAIRS = 4;    // a pair of waves, one of each role, to 32 heads
+constexpr int NDB = DN / 32;           // 16 blocks of 32 value columns ...
+constexpr int NDB_S = 4;               // ... of which the score wave of a pair takes the first four
+// of the score wave's 36 k-steps of Q, every sixth is parked in LDS (16 bytes per lane each): what its 256 registers do not
+// hold beside its part of O and the scores
+constexpr int PARK_EVERY = 6, NPARK = KSTEPS / PARK_EVERY, NREG = KSTEPS - NPARK;
+// LDS layout: three tile stages | parked Q | P~ [2][pair], 2 KB each | rescale factors [2][pair][32], flags [2][pair] |
+// per-split arrays sized by SfaArgs::split_cap (validity words, rows).  While the share is looked up, this sequence's page
+// table lies in front (when it fits); then the query, on its way to operand layout.
+constexpr int QPARK_OFF = 3 * STAGE;
+constexpr int PBUF_OFF = QPARK_OFF + PAIRS * NPARK * 1024;
+constexpr int ALPHA_OFF = PBUF_OFF + 2 * PAIRS * 2048;
+constexpr int FLAG_OFF = ALPHA_OFF + 2 * PAIRS * 32 * 4;
+constexpr int SPLIT_OFF = FLAG_OFF + 2 * PAIRS * 4;
 constexpr int LDS_LIMIT = 160 * 1024;
 constexpr int OUT_ROW = DN * 2;  // epilogue staging: 128 heads x 512 values of 16 bits, reusing the front of LDS
-constexpr int OUT_LSUM_OFF = HEADS_PER_WG * OUT_ROW; // the epilogue's row sums, behind the staging area (in the parked Q, dead by then)
+constexpr int LSUM_OFF = ALPHA_OFF; // the epilogue's row sums [pair][32], where the rescale factors were
 constexpr int QROW = KROW;       // start-up staging of Q: 128 heads x 1152 bytes
-static_assert(HEADS_PER_WG * QROW <= SPLIT_OFF, "the query of 128 heads fits below the per-split arrays");
+constexpr int BT_MAX = 2048;     // entries of a page table that is looked up in LDS
+static_assert(HEADS_PER_WG * QROW <= SPLIT_OFF && HEADS_PER_WG * OUT_ROW <= LSUM_OFF && BT_MAX * 4 <= SPLIT_OFF, "what uses the front of LDS ends below the per-split arrays");
 __host__ __device__ constexpr int tmask_bytes(int cap) { return (cap / T + 2) * 4; }
 __host__ __device__ constexpr int split_bytes(int cap) { return tmask_bytes(cap) + cap * 4; }
-static_assert(OUT_LSUM_OFF >= QPARK_OFF && OUT_LSUM_OFF + HEADS_PER_WG * 4 <= SPLIT_OFF, "the epilogue's row sums lie in the parked Q, which nothing reads after the last tile's scores");
 static_assert(QPARK_OFF % 16 == 0 && SPLIT_OFF % 16 == 0, "16-byte LDS accesses");
 static_assert(SPLIT_OFF + split_bytes(MAX_SPLIT_TOKENS) <= LDS_LIMIT, "a whole top-k list must fit one workgroup");
 
@@ -85,170 +86,167 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 // addressed by lanes i/4, 4 + i/4, 8 + i/4 and 12 + i/4 of the group.
 __device__ __forceinline__ s16x4 lds_read_tr(uint8_t* p) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p); }
 
-// chunk swizzle of tile row t: a bijection of t % 8, so that 8 consecutive rows (b128 column reads) and the
-// 4 consecutive rows of a transpose read both land on distinct banks
-__device__ __forceinline__ int swz(int t) { return ((t & 3) << 1) | ((t >> 2) & 1); }
+// Chunk swizzle of tile row t.  A row is 32 banks more than a multiple of the 64, so rows of one parity share their
+// banks.  A b128 read serves 16 lanes at a time, 16 rows in the scores' K fragments: the eight rows of a parity need eight
+// different values.  A transposing read serves 32 lanes, 64 bytes of four rows: two neighbouring rows of a parity need
+// different values of bit 2.  (4.0 and 2.5 ticks of the CU's LDS per read, its full rate; with a bijection of t % 8, as
+// b128 reads of eight lanes would want, the K fragments took 8.0.)
+__host__ __device__ constexpr int swz(int t) { return ((t & 2) << 1) | ((t >> 2) & 3); }
 
-// A wavefront's share of one gathered tile, in registers: NR of the tile's 32 rows (this lane's 8 columns of each), 8
-// bytes of the tile's rope columns, and one of the share's 4 NR dequantisation scales.  The two waves of a pair (same
-// head group hg) share rows 8 hg .. 8 hg + 7: the first NR_PR go to the KH = 1 wave, the others to the softmax wave.
-template <bool QUANT, int NR>
-struct RawTile;
-template <int NR>
-struct RawTile<true, NR> {
-    u32x2 nope[NR]; // NR rows x 8 int8
-    u32x2 rope;     // row tid/16, bytes 8 (tid%16) ..
-    float sc;       // lanes 0 .. 4 NR - 1: scale of (row lane/4 of the share, column group lane%4)
-};
-template <int NR>
-struct RawTile<false, NR> {
-    u32x4 nope[NR]; // NR rows x 8 bf16
-    u32x2 rope;
-};
-
-// Byte offset `row * stride` of a wave-uniform row, pinned in scalar registers so that the load that follows takes a
-// scalar base and the lane's 32-bit offset (no 64-bit vector arithmetic per row).  An offset, not an address: the
-// pointer it is added to keeps its address space, and the load stays a global one.
-__device__ __forceinline__ uint64_t row_offset(uint32_t row, uint32_t stride)
+// f(integral_constant 0), f(integral_constant 1) .. f(integral_constant N - 1), written out
+template <class F, int... I>
+__device__ __forceinline__ void unroll_seq(std::integer_sequence<int, I...>, F&& f)
 {
-    const uint64_t p = (uint64_t)row * stride;
-    uint32_t lo = (uint32_t)p, hi = (uint32_t)(p >> 32);
-    asm volatile("" : "+s"(lo), "+s"(hi));
-    return ((uint64_t)hi << 32) | lo;
+    (f(std::integral_constant<int, I>{}), ...);
 }
+template <int N, class F>
+__device__ __forceinline__ void unroll(F&& f)
+{
+    unroll_seq(std::make_integer_sequence<int, N>{}, static_cast<F&&>(f));
+}
+
+// v, in a form that the compiler does not keep what follows from it in registers across the tiles: it would spill other
+// such values, and a spilled value read back waits for every gather in flight
+__device__ __forceinline__ int fresh(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// A value wave's share of one gathered tile, in registers: rows 8 pair .. 8 pair + 7 of the tile and 16 bytes of the rope
+// columns of row lane / 8 of them.  int8: 16 columns (of the row's 512) of rows 4 (lane / 32) .. + 3 and the dequantisation
+// scale of (row lane % 8, column group lane / 8 % 4) - 16 bytes a lane, because a load occupies the memory pipe by its
+// lanes, not by its bytes.  bf16: 8 columns of all eight rows.
+template <bool QUANT>
+struct RawTile;
+template <>
+struct RawTile<true> {
+    static constexpr int LOADS = 4;
+    u32x4 nope[LOADS];
+    u32x4 rope;
+    float sc;
+};
+template <>
+struct RawTile<false> {
+    static constexpr int LOADS = 8;
+    u32x4 nope[LOADS];
+    u32x4 rope;
+};
 
 // rows[] holds valid cache rows only (absent entries point at row 0); the tile's validity word says which rows are
 // absent, and their data is zeroed when it is consumed, so that no load depends on it.  All loads are unconditional.
-// The share is rows pair0 + E0 .. pair0 + E0 + NR - 1 of the tile, pair0 a multiple of 8.
-template <int NR>
-struct RowRefs {
-    uint64_t off[NR];  // byte offsets of the share's rows in the nope cache (scalar registers)
-    uint32_t rope_row; // this lane's row for the rope columns
-    uint32_t sc_row;   // this lane's row for the scales
-};
-template <bool QUANT, int NR, int E0>
-__device__ __forceinline__ void prepare_rows(RowRefs<NR>& f, const SfaArgs& a, const int* rows, int tile, int pair0, int lane, int tid)
+// r points at the share's eight rows in LDS; what a load needs is read from there a few steps ahead of it (a register instead of ten).
+// An address is one 64-bit multiply-add in the vector unit: the row comes out of LDS in every lane, and in scalar
+// registers it would take a read of the lane, two multiplies and two additions per row, all issued by the same wave.
+template <bool QUANT, int K>
+__device__ __forceinline__ uint32_t nope_row(const int* r, int lane)
 {
-    // the pair's eight rows are the same for every lane: two 16-byte LDS reads, then scalar address arithmetic
-    const u32x4 ra = *reinterpret_cast<const u32x4*>(rows + tile * T + pair0);
-    const u32x4 rb = *reinterpret_cast<const u32x4*>(rows + tile * T + pair0 + 4);
-    f.rope_row = (uint32_t)rows[tile * T + (tid >> 4)];
-    if constexpr (QUANT) {
-        const int l = lane < 4 * NR ? lane : 0;
-        f.sc_row = (uint32_t)rows[tile * T + pair0 + E0 + (l >> 2)];
-    }
-#pragma unroll
-    for (int e = 0; e < NR; ++e) {
-        const uint32_t row = __builtin_amdgcn_readfirstlane(E0 + e < 4 ? ra[(E0 + e) & 3] : rb[(E0 + e) & 3]);
-        f.off[e] = row_offset(row, a.kn_stride);
-    }
+    return (uint32_t)(QUANT ? r[4 * (fresh(lane) >> 5) + K] : r[K]);
 }
-template <bool QUANT, int NR>
-__device__ __forceinline__ void issue_raw(RawTile<QUANT, NR>& r, const RowRefs<NR>& f, const SfaArgs& a, int lane, int tid)
+__device__ __forceinline__ uint32_t rope_row(const int* r, int lane) { return (uint32_t)r[fresh(lane) >> 3]; }
+__device__ __forceinline__ uint32_t scale_row(const int* r, int lane) { return (uint32_t)r[fresh(lane) & 7]; }
+template <bool QUANT, int K>
+__device__ __forceinline__ void gather_nope(RawTile<QUANT>& r, uint32_t row, const SfaArgs& a, int lane)
 {
-#pragma unroll
-    for (int e = 0; e < NR; ++e) {
-        const uint8_t* rp = a.kn + f.off[e];
-        if constexpr (QUANT)
-            r.nope[e] = *reinterpret_cast<const u32x2*>(rp + lane * 8);
-        else
-            r.nope[e] = *reinterpret_cast<const u32x4*>(rp + lane * 16);
-    }
-    r.rope = *reinterpret_cast<const u32x2*>(a.kr + (uint64_t)f.rope_row * a.kr_stride + (tid & 15) * 8);
-    if constexpr (QUANT) {
-        const int l = lane < 4 * NR ? lane : 0;
-        r.sc = *reinterpret_cast<const float*>(a.ks + (uint64_t)f.sc_row * a.ks_stride + (l & 3) * 4);
-    }
+    const int l = QUANT ? lane & 31 : fresh(lane);
+    r.nope[K] = *reinterpret_cast<const u32x4*>(a.kn + l * 16 + (uint64_t)row * a.kn_stride);
 }
-template <bool QUANT, int NR, int E0>
-__device__ __forceinline__ void load_raw(RawTile<QUANT, NR>& r, const SfaArgs& a, const int* rows, int tile, int pair0,
-                                         int lane, int tid)
+template <bool QUANT>
+__device__ __forceinline__ void gather_rope(RawTile<QUANT>& r, uint32_t row, const SfaArgs& a, int lane)
 {
-    RowRefs<NR> f;
-    prepare_rows<QUANT, NR, E0>(f, a, rows, tile, pair0, lane, tid);
-    issue_raw<QUANT, NR>(r, f, a, lane, tid);
+    lane = fresh(lane);
+    r.rope = *reinterpret_cast<const u32x4*>(a.kr + (lane & 7) * 16 + (uint64_t)row * a.kr_stride);
+}
+template <bool QUANT>
+__device__ __forceinline__ void gather_scale(RawTile<QUANT>& r, uint32_t row, const SfaArgs& a, int lane)
+{
+    lane = fresh(lane);
+    if constexpr (QUANT) r.sc = *reinterpret_cast<const float*>(a.ks + ((lane >> 3) & 3) * 4 + (uint64_t)row * a.ks_stride);
+}
+template <bool QUANT>
+__device__ __forceinline__ void gather_tile(RawTile<QUANT>& t, const SfaArgs& a, const int* r, int lane)
+{
+    gather_scale<QUANT>(t, scale_row(r, lane), a, lane);
+    unroll<RawTile<QUANT>::LOADS>([&](auto k) { gather_nope<QUANT, k>(t, nope_row<QUANT, k>(r, lane), a, lane); });
+    gather_rope<QUANT>(t, rope_row(r, lane), a, lane);
 }
 
-// int8 -> fp32 -> * scale with one conversion and one fma per element: byte k of w holds x + 128 (the caller
-// flips the sign bits), so x * s = fma(float(byte), s, -128 s); -128 s is exact, hence one rounding, the same
-// as rounding the product x * s.
-__device__ __forceinline__ float dq(uint32_t w, int k, float s, float neg128s)
-{
-    return __builtin_fmaf((float)((w >> (8 * k)) & 0xffu), s, neg128s);
-}
+// Dequantisation of the share.  Two int8 of a row at a time: their bytes, sign bits flipped, are x + 128 and as the low
+// bytes of two fp16 read (x + 128) 2^-24 (fp16 denormals, exact); one fma per element with the scale times 2^24 and -128
+// times the scale, both exact (scales up to 2^103), rounds once, like the product x * s that the golden rounds.  (A
+// conversion per element instead of one byte permute for two costs a quarter more instructions.)  In 35 pieces: a piece is the permute of one
+// pair, the fmas of the pair before and the packing of the one before that, because a wave issues a vector instruction
+// that depends on the one ahead of it at half the rate of an independent one.
+constexpr int PIECES = 35;
+template <bool QUANT>
+struct Production {
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    float v;          // the loaded scale, of (row lane % 8, column group lane / 8 % 4)
+    float sc;         // the scale of the row to come
+    float s, c;       // of the row in hand: times 2^24 and times -128
+    int from;         // where the scales of this lane's rows and columns are: 4 times the lane
+    f16x2 h;
+    float f0, f1;
+    uint32_t pk[4];
+    uint32_t at;      // LDS address of this lane's first chunk, stage included
 
-// Dequantise the share and store it, and the lane's rope piece, into an LDS stage; `present` is the tile's validity word.
-// Two rows at a time, instruction class by instruction class (16 conversions, 16 multiply-adds, 8 packs): a wave issues
-// a vector instruction that depends on the one before it at half the rate of an independent one, and the scheduler,
-// left alone, emits each element's conversion - multiply-add - pack chain back to back.
-template <bool QUANT, int NR>
-__device__ __forceinline__ void dequant_store(const RawTile<QUANT, NR>& r, uint8_t* stage, uint32_t present, int row0,
-                                              int lane, int tid)
-{
-    float sc[NR];
-    if constexpr (QUANT) {
-        // the scale of (row e, this lane's group of 128 columns) sits in lane 4e + lane/16; an absent row is stored as
-        // zeros (scale 0)
-#pragma unroll
-        for (int e = 0; e < NR; ++e)
-            sc[e] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (4 * e + (lane >> 4)), __builtin_bit_cast(int, r.sc)));
-#pragma unroll
-        for (int e = 0; e < NR; ++e) sc[e] = ((present >> (row0 + e)) & 1u) ? sc[e] : 0.f;
-    }
-#pragma unroll
-    for (int e0 = 0; e0 < NR; e0 += 2) {
-        constexpr int G = 2;
+    __device__ __forceinline__ void begin(const RawTile<QUANT>& r, uint32_t present, uint32_t stage, int pair, int lane)
+    {
+        lane = fresh(lane);
         if constexpr (QUANT) {
-            float f[G][8], c[G];
-            uint32_t pk[G][4];
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (e0 + g >= NR) break;
-                const uint32_t w0 = r.nope[e0 + g][0] ^ 0x80808080u, w1 = r.nope[e0 + g][1] ^ 0x80808080u;
-                c[g] = -128.f * sc[e0 + g];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    f[g][k] = (float)((w0 >> (8 * k)) & 0xffu);
-                    f[g][4 + k] = (float)((w1 >> (8 * k)) & 0xffu);
-                }
+            v = r.sc;
+            if (present != 0xffffffffu) { // (an absent row is stored as zeros)
+                if (!((present >> (8 * pair + (lane & 7))) & 1u)) v = 0.f;
             }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (e0 + g >= NR) break;
-#pragma unroll
-                for (int k = 0; k < 8; ++k) f[g][k] = __builtin_fmaf(f[g][k], sc[e0 + g], c[g]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (e0 + g >= NR) break;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) pk[g][k] = pack_bf16x2(f[g][2 * k], f[g][2 * k + 1]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (e0 + g >= NR) break;
-                const int t = row0 + e0 + g;
-                *reinterpret_cast<u32x4*>(stage + t * KROW + ((lane ^ swz(t)) << 4)) = u32x4{pk[g][0], pk[g][1], pk[g][2], pk[g][3]};
-            }
+            from = 4 * (4 * (lane >> 5) + (lane & 24));
+            fetch_scale<0>();
+            // rows t = 8 pair + 4 (lane / 32) + k, chunks 2 (lane % 32) and the next: swz(t) is swz(t - k) ^ 4 (k / 2)
+            const int t = 8 * pair + 4 * (lane >> 5);
+            at = stage + t * KROW + (((2 * (lane & 31)) ^ swz(t)) << 4);
         } else {
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (e0 + g >= NR) break;
-                const int t = row0 + e0 + g;
-                const u32x4 v = ((present >> t) & 1u) ? r.nope[e0 + g] : u32x4{0u, 0u, 0u, 0u};
-                *reinterpret_cast<u32x4*>(stage + t * KROW + ((lane ^ swz(t)) << 4)) = v;
-            }
+            at = stage + 8 * pair * KROW + ((lane ^ swz(8 * pair)) << 4); // rows 8 pair + k, chunk lane
         }
     }
+    template <int K>
+    __device__ __forceinline__ void fetch_scale()
     {
-        const int t = tid >> 4, piece = tid & 15;
-        const u32x2 rp = ((present >> t) & 1u) ? r.rope : u32x2{0u, 0u};
-        *reinterpret_cast<u32x2*>(stage + t * KROW + DN * 2 + (((piece >> 1) ^ swz(t)) << 4) + (piece & 1) * 8) = rp;
+        sc = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from + 4 * K, __builtin_bit_cast(int, v)));
     }
-}
+    template <int P>
+    __device__ __forceinline__ void piece(const RawTile<QUANT>& r, uint32_t present, uint8_t* lds, uint32_t stage, int pair, int lane)
+    {
+        if constexpr (QUANT) {
+            if constexpr (P >= 2 && P < 34) {
+                constexpr int K = (P - 2) / 8, H = (P - 2) / 4 % 2, Q = (P - 2) % 4;
+                pk[Q] = pack_bf16x2(f0, f1);
+                if constexpr (Q == 3) *reinterpret_cast<u32x4*>(lds + (at ^ (16 * H + 64 * (K / 2))) + K * KROW) = u32x4{pk[0], pk[1], pk[2], pk[3]};
+            }
+            if constexpr (P >= 1 && P < 33) {
+                f0 = __builtin_fmaf((float)h[0], s, c);
+                f1 = __builtin_fmaf((float)h[1], s, c);
+            }
+            if constexpr (P < 32) {
+                constexpr int K = P / 8, J = P % 8;
+                if constexpr (J == 0) {
+                    s = sc * 16777216.f;
+                    c = sc * -128.f;
+                }
+                if constexpr (J == 1 && K < 3) fetch_scale<K + 1>();
+                h = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0u, r.nope[K][J / 2] ^ 0x80808080u, J % 2 ? 0x0c030c02u : 0x0c010c00u));
+            }
+        } else if constexpr (P < 32 && P % 4 == 3) {
+            constexpr int K = P / 4; // (a multiple of eight rows changes swz only in the bits that `at` has)
+            u32x4 v = r.nope[K];
+            if (!((present >> (8 * pair + K)) & 1u)) v = u32x4{0u, 0u, 0u, 0u};
+            *reinterpret_cast<u32x4*>(lds + (at ^ (swz(K) << 4)) + K * KROW) = v;
+        }
+        if constexpr (P == 34) { // (an absent row's scores are masked: its rope columns may be anything)
+            lane = fresh(lane);
+            const int t = 8 * pair + (lane >> 3);
+            *reinterpret_cast<u32x4*>(lds + stage + t * KROW + DN * 2 + (((lane & 7) ^ swz(t)) << 4)) = r.rope;
+        }
+    }
+};
 
 // A workgroup's share of a token's top-k list: tiles [tile0, tile0 + ntiles) of the first `cur` entries.
 struct SplitRange {
@@ -284,7 +282,7 @@ __device__ __forceinline__ SplitRange resolve_split(const SfaArgs& a, int bi, in
     const int act = a.act_seq[bi];
     // this sequence's page table -> LDS (saves one dependent global load per selected token); a table that fits LDS
     // has at most BT_PER_LANE entries per lane
-    constexpr int BT_PER_LANE = (LDS_LIMIT - SPLIT_OFF) / 4 / NT + 1;
+    constexpr int BT_PER_LANE = BT_MAX / NT;
     const bool bt_cached = a.bt_cached != 0;
     int btv[BT_PER_LANE];
     if (bt_cached) {
@@ -302,21 +300,23 @@ __device__ __forceinline__ SplitRange resolve_split(const SfaArgs& a, int bi, in
     if (r.tile0 != guess.tile0) fetch(r.tile0 * T); // block-uniform
     const int tok0 = r.tile0 * T;
     const int ntiles_even = (r.ntiles + 1) & ~1; // whole wavefronts of entries
-    const int64_t max_logical = (int64_t)a.bt_stride * a.block_size;
+    // (as unsigned numbers: an unused entry, -1, is past every limit)
+    const uint32_t max_logical = (uint32_t)min((int64_t)a.bt_stride * a.block_size, (int64_t)1 << 31);
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < PER_LANE; ++j) {
         const int i = tid + NT * j;
         if (i >= ntiles_even * T) break; // wave-uniform: tiles are 32 wide, waves 64
-        const int idx = (i < r.ntiles * T && tok0 + i < r.cur) ? my_idx[j] : -1;
+        const uint32_t idx = (i < r.ntiles * T && tok0 + i < r.cur) ? (uint32_t)my_idx[j] : 0xffffffffu;
         int row = -1;
-        if (idx >= 0 && idx < max_logical) {
+        if (idx < max_logical) {
+            const uint32_t slot = (uint32_t)((uint64_t)idx * a.page_mul >> a.page_shift); // idx / block_size
             int page; // (two loads under a branch, not one load from a selected pointer: that would be a generic-address load)
             if (bt_cached)
-                page = bt_lds[idx / a.block_size];
+                page = bt_lds[slot];
             else
-                page = a.block_table[(int64_t)bi * a.bt_stride + idx / a.block_size];
-            const int64_t pr = (int64_t)page * a.block_size + idx % a.block_size;
+                page = a.block_table[(int64_t)bi * a.bt_stride + slot];
+            const int64_t pr = (int64_t)page * a.block_size + (idx - slot * a.block_size);
             if (page >= 0 && pr < a.n_rows) row = (int)pr;
         }
         rows[i] = max(row, 0);
@@ -330,389 +330,440 @@ __device__ __forceinline__ SplitRange resolve_split(const SfaArgs& a, int bi, in
     return r;
 }
 
-// Half of S^T[token, head] = K[token, :] . Q[head, :] for one wave: its 18 k-steps (kstep_of).  One accumulation
-// chain; the K fragments (and the parked Q fragments) are read AHEAD k-steps before the MFMA that uses them.
-template <int NREG, int KH>
-__device__ __forceinline__ void s_partial(f32x16& s, const uint8_t* stage, const uint32_t (&s_off)[4], const bf16x8 (&q)[NREG],
-                                          const uint8_t* qpark)
+// k-step of position i of a wave's 36: the two halves of the contraction one after the other, each its 16 nope steps and
+// its 2 rope steps
+__host__ __device__ constexpr int kstep_at(int i) { return i < 16 ? i : i < 18 ? i + 16 : i < 34 ? i - 2 : i; }
+constexpr bool parked(int i) { return i % PARK_EVERY == PARK_EVERY - 1; }
+// operand fragments read ahead of the matrix instruction that uses them: K, V in the score wave, V in the value wave (more
+// are registers that the waves do not have; four K fragments: 3650 ticks a tile, three in the value wave: 4000)
+constexpr int KD = 3, VD_S = 3, VD_V = 2;
+#define STEP_FENCE() __builtin_amdgcn_sched_barrier(0)
+
+// (fmaxf has the compiler quiet every operand first; the scores are sums of products, which are no signalling NaN)
+__device__ __forceinline__ float max3(float a, float b, float c)
 {
-    constexpr int AHEAD = S_AHEAD, N = KSTEPS / 2;
-    static_assert(NREG >= AHEAD && NREG <= N, "the first reads are of k-steps whose Q fragment is in registers");
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = 0.f;
-    bf16x8 kf[N], qp[N];
-    auto fetch = [&](int i) {
-        // nope k-step 16 KH + i: chunks 32 KH + 2 i + hl; rope k-step 32 + 2 KH + (i - 16): chunks 64 + 2 (2 KH + i - 16) + hl
-        kf[i] = *reinterpret_cast<const bf16x8*>(i < 16 ? stage + s_off[i & 3] + KH * 512 + (i >> 2) * 128
-                                                        : stage + s_off[2 * KH + i - 16] + DN * 2);
-        if (i >= NREG) qp[i] = *reinterpret_cast<const bf16x8*>(qpark + (i - NREG) * 1024);
-    };
-#pragma unroll
-    for (int i = 0; i < AHEAD; ++i) fetch(i);
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        if (i + AHEAD < N) fetch(i + AHEAD);
-        const bf16x8 qi = i < NREG ? q[i < NREG ? i : 0] : qp[i];
-        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qi, s, 0, 0, 0);
-    }
-    // issue order: AHEAD fetches, then (MFMA, fetch) pairs, then the last MFMAs; a fetch is one LDS read for a
-    // k-step whose Q fragment is in registers and two for a parked one
-    __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
-#pragma unroll
-    for (int i = 0; i < NREG - AHEAD; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-#pragma unroll
-    for (int i = NREG - AHEAD; i < N - AHEAD; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
 }
 
-// The body of one wavefront.  KH = 0: the softmax wave of its pair; KH = 1: the wave that hands its partial S over.
-template <bool QUANT, int KH>
+// O^T blocks DB0 .. DB0 + N - 1 of a pair's 32 heads: V^T fragments from a tile by transposing reads, P~ in two fragments of
+// 16 tokens.
+template <int DB0, int N, int VD>
+struct Values {
+    f32x16 o[N];
+    uint32_t off;       // this lane's place in a stage
+    uint32_t at[2][2];  // the same in the stage in use, for the second eight rows and odd blocks too
+    s16x4 lo[VD], hi[VD];
+
+    __device__ __forceinline__ void init(int lane)
+    {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+        // lane jj of 16-lane group G points at row 4*hl + jj/4 (+ 8*h2 + 16*j), columns 32*db + 16*(G&1) + 4*(jj&3) -> chunk
+        // 4*db + 2*(G&1) + (jj&3)/2.  Eight rows on, the swizzle differs in bit 1; in odd blocks, the chunk in bit 2; a stage
+        // is a multiple of 128 bytes, so that an exclusive or in these bits stays inside a row's group of eight chunks.
+        const int hl = lane >> 5, jj = lane & 15, mh = (lane >> 4) & 1, t = 4 * hl + (jj >> 2);
+        off = t * KROW + (((2 * mh + ((jj & 3) >> 1)) ^ swz(t)) << 4) + (jj & 1) * 8;
+    }
+    // fragment n: token block n / N, column block n % N
+    template <int n>
+    __device__ __forceinline__ void fetch(uint8_t* lds)
+    {
+        constexpr int j = n / N, db = DB0 + n % N, step = 16 * j * KROW + (db >> 1) * 128;
+        lo[n % VD] = lds_read_tr(lds + at[0][db & 1] + step);
+        hi[n % VD] = lds_read_tr(lds + at[1][db & 1] + step + 8 * KROW);
+    }
+    __device__ __forceinline__ void ahead(uint8_t* lds, int stage)
+    {
+        at[0][0] = off + stage;
+        at[0][1] = at[0][0] ^ 64;
+        at[1][0] = at[0][0] ^ 32;
+        at[1][1] = at[0][0] ^ 96;
+        unroll<VD>([&](auto n) { fetch<n>(lds); });
+    }
+    template <int n>
+    __device__ __forceinline__ void step(uint8_t* lds, const u32x4& p)
+    {
+        const s16x8 v = __builtin_shufflevector(lo[n % VD], hi[n % VD], 0, 1, 2, 3, 4, 5, 6, 7);
+        o[n % N] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, v), __builtin_bit_cast(bf16x8, p), o[n % N], 0, 0, 0);
+        if constexpr (n + VD < 2 * N) fetch<n + VD>(lds);
+    }
+    // (fragments 0 .. VD - 1 have been requested)
+    __device__ __forceinline__ void add(uint8_t* lds, const u32x4 (&p)[2])
+    {
+        unroll<2 * N>([&](auto n) {
+            step<n>(lds, p[n / N]);
+            STEP_FENCE();
+        });
+    }
+    __device__ __forceinline__ void scale(float f)
+    {
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i] *= f;
+    }
+    // Epilogue.  Register r of o[i] holds dim 32*(DB0 + i) + 8*(r/4) + 4*hl + r%4 of the lane's head: four consecutive dims,
+    // and the other half-wave holds the four next to them.
+    // A split's share, normalised by its own sum, in fp16 (|value| <= max |V| and 2^-11 relative rounding, a quarter
+    // of the final bf16 rounding, half the bytes of fp32 for this kernel to write and the merge to read).  It leaves
+    // in fragment order, straight from the accumulators: [token][split][head group][column group dq 4][head half 2]
+    // [head block 2][i 4][half 2][lane 64] x 8 fp16 (block 4 dq + i) - every store instruction writes 1 KB of
+    // consecutive bytes, and nothing is staged.  The merge kernel reads the same order and does the transposition to
+    // rows once, for the output, instead of once per split here.  (Streaming stores: 34 MB leave the chip's 256
+    // workgroups at once and are read back once.)
+    __device__ __forceinline__ void store_partial(_Float16* base, float mul)
+    {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+                const int db = DB0 + i;
+                uint32_t x[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    x[k] = __builtin_bit_cast(uint32_t, f16x2{(_Float16)(o[i][8 * h + 2 * k] * mul), (_Float16)(o[i][8 * h + 2 * k + 1] * mul)});
+                __builtin_nontemporal_store(u32x4{x[0], x[1], x[2], x[3]}, reinterpret_cast<u32x4*>(base + (db >> 2) * 16384 + ((db & 3) * 2 + h) * 512));
+            }
+    }
+    // One split: the output itself, bf16 rows [head][512] of 1024 bytes in LDS.  v_permlane32_swap pairs up the two
+    // half-waves' four-dim pieces - the lower half-wave ends up with the 8 dims of block g = 2 gp, the upper one with those
+    // of block 2 gp + 1 - so that a lane stores 16 bytes; the chunks of a row are XOR-swizzled with the head (16 rows of a
+    // store meet all banks).
+    __device__ __forceinline__ void stage_rows(uint8_t* orow, int hrow, int hl, float mul)
+    {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+            for (int gp = 0; gp < 2; ++gp) {
+                uint32_t x[2][2]; // [block 2 gp, 2 gp + 1][pair of dims]
+#pragma unroll
+                for (int g = 0; g < 2; ++g)
+#pragma unroll
+                    for (int k = 0; k < 2; ++k)
+                        x[g][k] = pack_bf16x2(o[i][4 * (2 * gp + g) + 2 * k] * mul, o[i][4 * (2 * gp + g) + 2 * k + 1] * mul);
+                // the swap exchanges the upper half-wave of its first operand with the lower half-wave of its second
+                const auto e0 = __builtin_amdgcn_permlane32_swap(x[0][0], x[1][0], false, false);
+                const auto e1 = __builtin_amdgcn_permlane32_swap(x[0][1], x[1][1], false, false);
+                const int c = 4 * (DB0 + i) + 2 * gp + hl;
+                *reinterpret_cast<u32x4*>(orow + ((c ^ (hrow & 15)) << 4)) = u32x4{(uint32_t)e0[0], (uint32_t)e1[0], (uint32_t)e0[1], (uint32_t)e1[1]};
+            }
+    }
+};
+
+// The body of one wavefront.  SCORES: the pair's score wave (waves 0 .. 3), which holds Q and does the scores, the softmax and
+// the values of the first NDB_S column blocks; else its value wave (waves 4 .. 7), which produces the tiles, eight rows of
+// each, and does the values of the other blocks.
+template <bool QUANT, bool SCORES>
 __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32_t* tmask, int* rows, int* bt_lds, int tid)
 {
+    constexpr int NT = 64 * WAVES;
     const int tq = blockIdx.x, sp = blockIdx.y, hz = blockIdx.z;
     const int bi = tq / a.s1, si = tq - bi * a.s1;
-    constexpr int NREG = KH ? NREG_PR : NREG_SM;
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6); // (scalar: what follows from it is too)
+    const int lane = tid & 63, pair = __builtin_amdgcn_readfirstlane(tid >> 6) & (PAIRS - 1); // (scalar: what follows from it is too)
     const int l32 = lane & 31, hl = lane >> 5;
-    const int hg = wave & 3;              // scores role: heads [32 hg, 32 hg + 32) of the workgroup's 128, contraction half KH = wave / 4
-    const int hh = wave & 1, dq = wave >> 1; // values role: heads [64 hh, 64 hh + 64), value columns [128 dq, 128 dq + 128)
     const int head0 = hz * HEADS_PER_WG;
-    const int head = head0 + hg * 32 + l32;
-    const bool head_ok = head < a.nq;
-    const bool s_active = head0 + hg * 32 < a.nq;
-    const bool pv_active = head0 + hh * 64 < a.nq;
+    const int hrow = pair * 32 + l32, head = head0 + hrow;
+    const bool active = head0 + pair * 32 < a.nq; // (a pair without heads works on copies of the last one, and stores nothing)
 
     // The query of the workgroup's 128 heads, requested right behind the few loads the look-up of the share starts with
     // (it is the largest piece of the start-up traffic and depends on nothing).  Fetched as whole cache lines - in each of four rounds of 128 nope
     // columns a lane takes four 16-byte pieces, 16 consecutive lanes one head's 256 bytes; then the rope columns, two
     // pieces per lane - because a load in operand layout (a lane pair per head) costs the texture addresser one line per
     // lane pair.  The operand layout is made on the way through LDS further down.
-    u32x4 qraw[4][4], qraw_rope[2];
+    constexpr int QN = HEADS_PER_WG * 16 / NT, QR = HEADS_PER_WG * 8 / NT;
+    u32x4 qraw[4][QN], qraw_rope[QR];
     auto request_q = [&]() {
         const int64_t qrow0 = (int64_t)tq * a.nq;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int p = tid + 512 * j;
+            for (int j = 0; j < QN; ++j) {
+                const int p = tid + NT * j;
                 const int64_t row = qrow0 + min(head0 + (p >> 4), a.nq - 1);
                 qraw[r][j] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const __bf16*>(a.q_nope) + row * DN + 128 * r + 8 * (p & 15));
             }
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int p = tid + 512 * j;
+        for (int j = 0; j < QR; ++j) {
+            const int p = tid + NT * j;
             const int64_t row = qrow0 + min(head0 + (p >> 3), a.nq - 1);
             qraw_rope[j] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const __bf16*>(a.q_rope) + row * DR + 8 * (p & 7));
         }
     };
 
-    const SplitRange share = resolve_split<512>(a, bi, si, tq, sp, tmask, rows, bt_lds, tid, lane, request_q);
+    const SplitRange share = resolve_split<NT>(a, bi, si, tq, sp, tmask, rows, bt_lds, tid, lane, request_q);
     const int ntiles = share.ntiles, last = ntiles - 1;
 
-    // Production: this wave's share of every tile (rows row0 .. row0 + NR - 1 and 8 bytes of the rope columns).  The
-    // share of tile i+1 is dequantised out of `raw` and stored between the two MFMA phases of tile i, and `raw` is
-    // refilled at once with the share of tile i+2 (past the end the last tile is loaded again and stored into a stage
-    // nobody reads: every path has the same loads in flight).
-    constexpr int NR = KH ? NR_PR : 8 - NR_PR, E0 = KH ? 0 : NR_PR;
-    const int pair0 = 8 * hg, row0 = pair0 + E0;
-    RawTile<QUANT, NR> raw;
-    if (ntiles > 0) load_raw<QUANT, NR, E0>(raw, a, rows, 0, pair0, lane, tid);
+    RawTile<QUANT> raw;
+    if (!SCORES && ntiles > 0) gather_tile<QUANT>(raw, a, rows + 8 * pair, lane);
 
-    // Q into operand layout: this lane's head (hg, l32) and its slice - the 16 k-steps of nope columns
-    // [256 KH, 256 KH + 256) and the 2 of rope columns [32 KH, 32 KH + 32); B operand layout: head = column, 8
-    // consecutive k per half-wave.  One trip through LDS (all of it below the per-split arrays is still unused).
-    bf16x8 q[NREG];
-    uint8_t* qpark = smem + QPARK_OFF + (KH ? 4 * NPARK_SM * 1024 + hg * (NPARK_PR * 1024) : hg * (NPARK_SM * 1024)) + lane * 16;
+    // Q into operand layout: this lane's head and the 36 k-steps; B operand layout: head = column, 8 consecutive k per
+    // half-wave.  One trip through LDS (all of it below the per-split arrays is still unused).
+    bf16x8 q[SCORES ? NREG : 1];
+    uint8_t* qpark = smem + QPARK_OFF + pair * (NPARK * 1024) + lane * 16;
     {
         // (a negative softmax_scale is applied as its magnitude to the negated query: the row statistics below are
         // taken on the raw scores, which needs a factor that commutes with max)
         const uint32_t f = a.softmax_scale < 0.f ? 0x80008000u : 0u;
         const u32x4 qflip = {f, f, f, f};
-        // all 128 heads' rows at once: row h at h * QROW, its 72 16-byte chunks (64 nope, 8 rope) XOR-swizzled with h
-        // so that the 8 lanes of a b128 access hit distinct banks although a row is a multiple of 128 bytes
+        // all 128 heads' rows at once: row h at h * QROW, its 72 16-byte chunks (64 nope, 8 rope) swizzled like a tile's
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int pp = tid + 512 * j, h = pp >> 4, c = 16 * r + (pp & 15);
-                *reinterpret_cast<u32x4*>(smem + h * QROW + ((c ^ (h & 7)) << 4)) = qraw[r][j];
+            for (int j = 0; j < QN; ++j) {
+                const int pp = tid + NT * j, h = pp >> 4, c = 16 * r + (pp & 15);
+                *reinterpret_cast<u32x4*>(smem + h * QROW + ((c ^ swz(h)) << 4)) = qraw[r][j];
             }
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int pp = tid + 512 * j, h = pp >> 3, c = 64 + (pp & 7);
-            *reinterpret_cast<u32x4*>(smem + h * QROW + ((c ^ (h & 7)) << 4)) = qraw_rope[j];
+        for (int j = 0; j < QR; ++j) {
+            const int pp = tid + NT * j, h = pp >> 3, c = 64 + (pp & 7);
+            *reinterpret_cast<u32x4*>(smem + h * QROW + ((c ^ swz(h)) << 4)) = qraw_rope[j];
         }
         __syncthreads();
-        // k-step i of this wave's 18: nope chunks 2 (16 KH + i) + hl, rope chunks 64 + 2 (2 KH + i - 16) + hl
-        u32x4 qa[KSTEPS / 2];
-        {
-            const int h = hg * 32 + l32;
-            const uint8_t* row = smem + h * QROW;
+        u32x4 qa[KSTEPS];
+        if constexpr (SCORES) {
 #pragma unroll
-            for (int i = 0; i < KSTEPS / 2; ++i) {
-                const int c = (i < 16 ? 2 * (16 * KH + i) : 64 + 2 * (2 * KH + i - 16)) + hl;
-                qa[i] = *reinterpret_cast<const u32x4*>(row + ((c ^ (h & 7)) << 4)) ^ qflip;
+            for (int i = 0; i < KSTEPS; ++i)
+                qa[i] = *reinterpret_cast<const u32x4*>(smem + hrow * QROW + (((2 * kstep_at(i) + hl) ^ swz(hrow)) << 4)) ^ qflip;
+        }
+        __syncthreads(); // the score waves have their fragments: the rows' space is free for the parked fragments and the tiles
+        if constexpr (SCORES) {
+#pragma unroll
+            for (int i = 0; i < KSTEPS; ++i) {
+                const bf16x8 v = __builtin_bit_cast(bf16x8, qa[i]);
+                if (parked(i))
+                    *reinterpret_cast<bf16x8*>(qpark + (i / PARK_EVERY) * 1024) = v;
+                else
+                    q[SCORES ? i - i / PARK_EVERY : 0] = v;
             }
         }
-        __syncthreads(); // every wave has its fragments: the rows' space is free for the parked fragments and the tiles
-#pragma unroll
-        for (int i = 0; i < KSTEPS / 2; ++i) {
-            const bf16x8 v = __builtin_bit_cast(bf16x8, qa[i]);
-            if (i < NREG)
-                q[i < NREG ? i : 0] = v;
-            else
-                *reinterpret_cast<bf16x8*>(qpark + (i - NREG) * 1024) = v;
-        }
-    }
-    if (ntiles > 0) {
-        dequant_store<QUANT, NR>(raw, smem, __builtin_amdgcn_readfirstlane(tmask[0]), row0, lane, tid);
-        load_raw<QUANT, NR, E0>(raw, a, rows, min(1, last), pair0, lane, tid);
     }
 
-    f32x16 o[4][2]; // O^T blocks [value columns 32 (4 dq + i) ..][heads 64 hh + 32 hb ..]
+    Values<SCORES ? 0 : NDB_S, SCORES ? NDB_S : NDB - NDB_S, SCORES ? VD_S : VD_V> val;
+    val.init(lane);
+    // P~ of tile i lies in buffer i % 2, the order the S^T registers hold the tokens in, and the factor by which what was
+    // summed before is to be multiplied, where the flag says so
+    uint8_t* pbuf = smem + PBUF_OFF + pair * 2048; // (+ 16 lane)
+    float* alpha_lds = reinterpret_cast<float*>(smem + ALPHA_OFF) + pair * 32;
+    uint32_t* flag_lds = reinterpret_cast<uint32_t*>(smem + FLAG_OFF) + pair;
+    float* lsum = reinterpret_cast<float*>(smem + LSUM_OFF) + pair * 32;
+    // Between two barriers: the scores and the softmax of tile `it`, the values of tile it - 1, the production of tile it + 1
+    // and the gather of tile it + 2.
+    int st_old = 2 * STAGE, st = 0, st_new = STAGE; // stages of the tiles it - 1, it, it + 1
+    auto turn = [&]() {
+        const int t = st_old;
+        st_old = st;
+        st = st_new;
+        st_new = t;
+    };
+    float l_tot, m_out = 0.f;
+    if constexpr (SCORES) {
+        // S operand (b128): row l32, chunk 2*ks + hl of k-step ks; swizzled offsets of the four chunk positions 2 m + hl
+        // inside a group of eight chunks
+        uint32_t s_off[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+        for (int m = 0; m < 4; ++m) s_off[m] = l32 * KROW + (((2 * m + hl) ^ swz(l32)) << 4);
+        bf16x8 kf[KD], qp;
+        auto fetch_k = [&](auto ic) {
+            constexpr int i = ic, ks = kstep_at(i);
+            kf[i % KD] = *reinterpret_cast<const bf16x8*>(smem + st + s_off[ks & 3] + (ks >> 2) * 128);
+            if constexpr (parked(i)) qp = *reinterpret_cast<const bf16x8*>(qpark + (i / PARK_EVERY) * 1024);
+        };
+        float m_run = -INFINITY; // running max of S * scale * log2(e)
+        float l_run = 0.f;       // this lane's share of sum exp
+        float alpha = 1.f;
+        bool rescale = false;
+        // (never exactly zero: a masked score is -inf, and -inf * 0 would be NaN; 2^(s * 1e-30) is 1 for every finite s, so
+        // a zero scale still gives every attended row the same weight)
+        const float c_log2 = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, fmaxf(fabsf(a.softmax_scale) * 1.4426950408889634f, 1e-30f))));
+        u32x4 p[2];
+        auto tile = [&](int it) {
+            f32x16 s0, s1;
+            const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            STEP_FENCE();
+            unroll<KSTEPS>([&](auto ic) {
+                constexpr int i = ic;
+                const bf16x8 qi = parked(i) ? qp : q[i - i / PARK_EVERY];
+                f32x16& s = i < KSTEPS / 2 ? s0 : s1;
+                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i % KD], qi, i % (KSTEPS / 2) == 0 ? zero : s, 0, 0, 0);
+                if constexpr (i + KD < KSTEPS) fetch_k(std::integral_constant<int, i + KD>{});
+                STEP_FENCE();
+            });
+            const uint32_t valid = __builtin_amdgcn_readfirstlane(tmask[it]);
 #pragma unroll
-        for (int hb = 0; hb < 2; ++hb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o[i][hb][r] = 0.f;
-    float m_run = -INFINITY; // running max of S * scale * log2(e)          (softmax wave)
-    float l_run = 0.f;       // this lane's share of sum exp                (softmax wave)
-    // (never exactly zero: a masked score is -inf, and -inf * 0 would be NaN; 2^(s * 1e-30) is 1 for every finite s, so
-    // a zero scale still gives every attended row the same weight)
-    const float c_log2 = fmaxf(fabsf(a.softmax_scale) * 1.4426950408889634f, 1e-30f);
-
-    // S operand (b128): row l32, chunk 2*ks + hl of k-step ks; swizzled offsets of the four chunk positions 2 m + hl
-    // inside a group of eight chunks
-    uint32_t s_off[4];
-    {
-        const int sw = swz(l32);
-#pragma unroll
-        for (int m = 0; m < 4; ++m) s_off[m] = l32 * KROW + (((2 * m + hl) ^ sw) << 4);
-    }
-    // V^T operand (transpose read): lane jj of 16-lane group G points at row 4*hl + jj/4 (+ 16*j + 8*h2), columns
-    // 32*db + 16*(G&1) + 4*(jj&3) with db = 4*dq + i -> chunk 16*dq + 4*i + 2*(G&1) + (jj&3)/2; swizzled offsets for even
-    // and odd i
-    uint32_t v_off[2];
-    {
-        const int jj = lane & 15, mh = (lane >> 4) & 1;
-        const int cl = 2 * mh + ((jj & 3) >> 1);
-        const int sw = ((jj >> 2) << 1) | hl;
-        const uint32_t base = (4 * hl + (jj >> 2)) * KROW + (jj & 1) * 8 + dq * 256;
-        v_off[0] = base + ((cl ^ sw) << 4);
-        v_off[1] = base + (((4 + cl) ^ sw) << 4);
-    }
-    uint8_t* xbuf = smem + XBUF_OFF + hg * 4096 + lane * 16;
-    uint8_t* pbuf = smem + PBUF_OFF + hg * 2048 + lane * 16;
-    float* alpha_lds = reinterpret_cast<float*>(smem + ALPHA_OFF);
-    uint32_t* flag_lds = reinterpret_cast<uint32_t*>(smem + FLAG_OFF);
-    if (tid < 4) flag_lds[tid] = 0u;
-    __syncthreads(); // tile 0 stored, Q parked
-
-    // Two barriers per tile: partial S handed over | P~ and the next tile ready.
-    for (int it = 0; it < ntiles; ++it) {
-        uint8_t* stage = smem + (it & 1) * STAGE;
-        const uint32_t valid = __builtin_amdgcn_readfirstlane(tmask[it]);
-        RowRefs<NR> next_rows; // of the tile after next, looked up under the score MFMAs
-        prepare_rows<QUANT, NR, E0>(next_rows, a, rows, min(it + 2, last), pair0, lane, tid);
-        f32x16 s;
-        if (s_active) s_partial<NREG, KH>(s, stage, s_off, q, qpark);
-        if (KH == 1 && s_active) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<f32x4*>(xbuf + g * 1024) = f32x4{s[4 * g], s[4 * g + 1], s[4 * g + 2], s[4 * g + 3]};
-        }
-        __syncthreads(); // the partial S of the KH = 1 waves is in LDS
-        if (KH == 0 && s_active && valid != 0u) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x4 p = *reinterpret_cast<const f32x4*>(xbuf + g * 1024);
-                s[4 * g] += p[0];
-                s[4 * g + 1] += p[1];
-                s[4 * g + 2] += p[2];
-                s[4 * g + 3] += p[3];
-            }
-            // register r holds token 8*(r/4) + 4*hl + r%4 for head l32; statistics on the raw scores (the factor
-            // is not negative, so it commutes with max), exponent argument by one fma per score
-            float mx = -INFINITY;
+            for (int r = 0; r < 16; ++r) s0[r] += s1[r];
             if (valid != 0xffffffffu) {
-                // (the half-wave's shift first: the bit positions left are compile-time constants)
+                // register r holds token 8*(r/4) + 4*hl + r%4 for head l32 (the half-wave's shift first: the bit
+                // positions left are compile-time constants)
                 const uint32_t vh = valid >> (4 * hl);
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s[r] = ((vh >> (8 * (r >> 2) + (r & 3))) & 1u) ? s[r] : -INFINITY;
+                for (int r = 0; r < 16; ++r) s0[r] = ((vh >> (8 * (r >> 2) + (r & 3))) & 1u) ? s0[r] : -INFINITY;
             }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
-            {
-                // maximum over both halves of the wavefront without a trip through LDS: v_permlane32_swap exchanges the
-                // upper half of its first operand with the lower half of its second
-                const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, mx), __builtin_bit_cast(unsigned, mx), false, false);
-                mx = fmaxf(__builtin_bit_cast(float, (unsigned)sw[0]), __builtin_bit_cast(float, (unsigned)sw[1])) * c_log2;
-            }
+            // statistics on the raw scores (the factor is not negative, so it commutes with max)
+            float x0 = max3(s0[0], s0[1], s0[2]), x1 = max3(s0[3], s0[4], s0[5]), x2 = max3(s0[6], s0[7], s0[8]);
+            float x3 = max3(s0[9], s0[10], s0[11]), x4 = max3(s0[12], s0[13], s0[14]);
+            x0 = max3(x0, x1, s0[15]);
+            x2 = max3(x2, x3, x4);
+            // maximum over both halves of the wavefront without a trip through LDS: v_permlane32_swap exchanges the
+            // upper half of its first operand with the lower half of its second.  (The multiplication is the compiler's own:
+            // the swap needs wait states behind an instruction that writes its operand, which the compiler leaves behind
+            // one that it knows)
+            const float mx = max3(x0, x2, x2) * c_log2;
+            const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, mx), __builtin_bit_cast(unsigned, mx), false, false);
             // The reference exponent only follows the running maximum when it has grown by more than 2^8: until
             // then P~ = 2^(z - m_run) may exceed 1 (by at most 2^8, no issue for bf16 or the fp32 sums), which
             // makes the rescale of the accumulator registers a rare event.  Every P~, l and O stay relative to
             // the same m_run, so the result is unchanged.
-            const float m_new = fmaxf(m_run, mx);
-            const bool rescale = __any(m_new > m_run + 8.f);
+            const float m_new = max3(m_run, __builtin_bit_cast(float, (unsigned)sw[0]), __builtin_bit_cast(float, (unsigned)sw[1]));
+            rescale = __any(m_new > m_run + 8.f);
             if (rescale) {
-                const float alpha = __builtin_amdgcn_exp2f(m_run - m_new); // 0 on the first tile (m_run = -inf)
+                alpha = __builtin_amdgcn_exp2f(m_run - m_new); // 0 on the first tile (m_run = -inf)
                 l_run *= alpha;
                 m_run = m_new;
-                if (hl == 0) alpha_lds[hg * 32 + l32] = alpha;
+                if (hl == 0) alpha_lds[(it & 1) * (PAIRS * 32) + l32] = alpha;
             }
-            if (lane == 0) flag_lds[hg] = rescale ? 1u : 0u;
-            uint32_t pb[8];
-#pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c_log2, -m_run));
-                const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r + 1], c_log2, -m_run));
-                l_run += p0 + p1;
-                pb[r >> 1] = pack_bf16x2(p0, p1);
-            }
+            if (lane == 0) flag_lds[(it & 1) * PAIRS] = rescale ? 1u : 0u;
+            const float m_use = valid != 0u ? m_run : 0.f; // (a tile without rows: every score is -inf, every P~ 0)
             // P~ in the order the S^T registers hold the tokens: k-slot s of half hl in block j is token
             // 16*j + 8*(s/4) + 4*hl + s%4 - which is also how the V^T fragments are read
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-                *reinterpret_cast<u32x4*>(pbuf + j * 1024) = u32x4{pb[4 * j], pb[4 * j + 1], pb[4 * j + 2], pb[4 * j + 3]};
-        }
-        {
-            // the next tile: out of the registers into the other stage, then the gather of the tile after
-            const int nx = min(it + 1, last);
-            dequant_store<QUANT, NR>(raw, smem + ((it + 1) & 1) * STAGE, __builtin_amdgcn_readfirstlane(tmask[nx]), row0, lane, tid);
-            issue_raw<QUANT, NR>(raw, next_rows, a, lane, tid);
-        }
-        __syncthreads(); // P~ and the next tile are in LDS
-        if (pv_active && valid != 0u) {
-            // O^T[dim, head] += V^T[dim, token] . P~[token, head]
+            for (int r = 0; r < 16; ++r) s0[r] = __builtin_fmaf(s0[r], c_log2, -m_use);
 #pragma unroll
-            for (int hb = 0; hb < 2; ++hb) {
-                const uint32_t f = __builtin_amdgcn_readfirstlane(flag_lds[2 * hh + hb]);
-                if (f) {
-                    const float alpha = alpha_lds[(2 * hh + hb) * 32 + l32];
+            for (int r = 0; r < 16; ++r) s0[r] = __builtin_amdgcn_exp2f(s0[r]);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) o[i][hb][r] *= alpha;
-                }
+            for (int r = 0; r < 16; r += 2) {
+                l_run += s0[r] + s0[r + 1];
+                p[r >> 3][(r & 7) >> 1] = pack_bf16x2(s0[r], s0[r + 1]);
             }
-            bf16x8 pf[2][2];
 #pragma unroll
-            for (int hb = 0; hb < 2; ++hb)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    pf[hb][j] = *reinterpret_cast<const bf16x8*>(smem + PBUF_OFF + (2 * hh + hb) * 2048 + j * 1024 + lane * 16);
-            // 8 V^T fragments (token block j, column block i), two transpose reads each, feeding two MFMAs each;
-            // the reads run AHEAD fragments ahead
-            constexpr int AHEAD = PV_AHEAD;
-            s16x4 lo[8], hi[8];
-            auto vread = [&](int n) {
-                const int j = n >> 2, i = n & 3;
-                uint8_t* vp = stage + v_off[i & 1] + (16 * j) * KROW + (i >> 1) * 128;
-                lo[n] = lds_read_tr(vp);
-                hi[n] = lds_read_tr(vp + 8 * KROW);
-            };
-#pragma unroll
-            for (int n = 0; n < AHEAD; ++n) vread(n);
-#pragma unroll
-            for (int n = 0; n < 8; ++n) {
-                if (n + AHEAD < 8) vread(n + AHEAD);
-                const s16x8 both = __builtin_shufflevector(lo[n], hi[n], 0, 1, 2, 3, 4, 5, 6, 7);
-                const bf16x8 vf = __builtin_bit_cast(bf16x8, both);
-#pragma unroll
-                for (int hb = 0; hb < 2; ++hb)
-                    o[n & 3][hb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[hb][n >> 2], o[n & 3][hb], 0, 0, 0);
+            for (int j = 0; j < 2; ++j) *reinterpret_cast<u32x4*>(pbuf + (it & 1) * (PAIRS * 2048) + j * 1024 + lane * 16) = p[j];
+        };
+        __syncthreads(); // tile 0 stored, Q parked
+        if (ntiles > 0) {
+            unroll<KD>(fetch_k);
+            tile(0);
+            rescale = false; // (there is nothing to rescale yet)
+            __syncthreads();
+            turn();
+            for (int it = 1; it < ntiles; ++it) {
+                val.ahead(smem, st_old);
+                unroll<KD>(fetch_k);
+                if (rescale) val.scale(alpha);
+                val.add(smem, p);
+                tile(it);
+                __syncthreads();
+                turn();
             }
+            val.ahead(smem, st_old);
+            if (rescale) val.scale(alpha);
+            val.add(smem, p);
+        }
+        l_tot = l_run + __shfl_xor(l_run, 32);
+        m_out = m_run;
+    } else {
+        Production<QUANT> prod;
+        // Tile `tile` out of registers into a stage.  A load's registers are free as soon as their last pair is in hand: the
+        // rows of the tile after are requested right behind that.
+        constexpr int LOADS = RawTile<QUANT>::LOADS;
+        constexpr int STEPS = 2 * (NDB - NDB_S);
+        auto produce = [&](int tile, int stage, auto&& between) {
+            const uint32_t present = __builtin_amdgcn_readfirstlane(tmask[tile]);
+            const int* next = rows + min(tile + 1, last) * T + 8 * pair;
+            uint32_t row, row1;
+            prod.begin(raw, present, stage, pair, lane);
+            STEP_FENCE();
+            unroll<PIECES>([&](auto ic) {
+                constexpr int i = ic, per = 32 / LOADS, K = i / per;
+                between(ic);
+                prod.template piece<i>(raw, present, smem, stage, pair, lane);
+                if constexpr (i < 32 && i % per == per - 3) row = nope_row<QUANT, K>(next, lane);
+                if constexpr (i < 32 && i % per == per - 1) gather_nope<QUANT, K>(raw, row, a, lane);
+                if constexpr (i == 28) row1 = scale_row(next, lane);
+                if constexpr (i == 30) gather_scale<QUANT>(raw, row1, a, lane);
+                if constexpr (i == 32) row1 = rope_row(next, lane);
+                STEP_FENCE();
+            });
+            gather_rope<QUANT>(raw, row1, a, lane);
+        };
+        u32x4 p, p1;
+        const uint8_t* pb;
+        auto values = [&](int it) {
+            pb = pbuf + (it & 1) * (PAIRS * 2048) + fresh(lane) * 16;
+            p = *reinterpret_cast<const u32x4*>(pb);
+            val.ahead(smem, st_old);
+            if (__builtin_amdgcn_readfirstlane(flag_lds[(it & 1) * PAIRS])) val.scale(alpha_lds[(it & 1) * (PAIRS * 32) + (fresh(lane) & 31)]);
+            STEP_FENCE();
+        };
+        auto value_step = [&](auto nc) {
+            constexpr int n = nc;
+            if constexpr (n == STEPS / 2 - 2) p1 = *reinterpret_cast<const u32x4*>(pb + 1024);
+            val.template step<n>(smem, n < STEPS / 2 ? p : p1);
+            STEP_FENCE();
+        };
+        auto nothing = [](auto) {};
+        if (ntiles > 0) produce(0, 0, nothing);
+        __syncthreads(); // tile 0 stored, Q parked
+        if (ntiles > 0) {
+            if (last > 0) produce(1, st_new, nothing);
+            __syncthreads();
+            turn();
+            __builtin_amdgcn_s_setprio(1); // (the score wave is the older one of the SIMD and would take every slot)
+            for (int it = 1; it < last; ++it) {
+                values(it - 1);
+                produce(it + 1, st_new, [&](auto ic) {
+                    constexpr int i = ic, n0 = i * STEPS / PIECES, n1 = (i + 1) * STEPS / PIECES;
+                    if constexpr (n1 > n0) value_step(std::integral_constant<int, n0>{});
+                });
+                __syncthreads();
+                turn();
+            }
+            if (last > 0) {
+                values(last - 1);
+                unroll<STEPS>(value_step);
+                __syncthreads();
+                turn();
+            }
+            values(last);
+            unroll<STEPS>(value_step);
         }
     }
 
-    // Epilogue.  The softmax waves publish the row sums (in a part of LDS the staging area below does not reach) and every
-    // wave normalises its O^T blocks.  Register r of o[i][hb] holds dim 32*(4*dq + i) + 8*(r/4) + 4*hl + r%4 of head
-    // 64*hh + 32*hb + l32: four consecutive dims, and the other half-wave holds the four next to them.
-    float* lsum = reinterpret_cast<float*>(smem + OUT_LSUM_OFF);
-    if (KH == 0) {
-        const float l_tot = l_run + __shfl_xor(l_run, 32);
-        if (hl == 0) lsum[hg * 32 + l32] = s_active ? l_tot : 0.f;
-        if (a.nsplit > 1 && head_ok && hl == 0) {
-            const int64_t prow = ((int64_t)tq * a.nsplit + sp) * a.nq + head;
-            a.part_ml[prow * 2] = m_run;
-            a.part_ml[prow * 2 + 1] = l_tot;
-        }
-    }
-    __syncthreads(); // row sums published; nobody reads a tile, P~ or parked Q any more
-    if (a.nsplit > 1) {
-        // A split's share, normalised by its own sum, in fp16 (|value| <= max |V| and 2^-11 relative rounding, a quarter
-        // of the final bf16 rounding, half the bytes of fp32 for this kernel to write and the merge to read).  It leaves
-        // in fragment order, straight from the accumulators: [token][split][head group][wave 8][hb 2][i 4][half 2]
-        // [lane 64] x 8 fp16 - every store instruction writes 1 KB of consecutive bytes, and nothing is staged.  The
-        // merge kernel reads the same order and does the transposition to rows once, for the output, instead of once
-        // per split here.  (Streaming stores: 34 MB leave the chip's 256 workgroups at once and are read back once.)
-        if (pv_active) {
-            const int wave = tid >> 6;
-            _Float16* wbase = a.part_o + ((((int64_t)tq * a.nsplit + sp) * gridDim.z + hz) * 8 + wave) * 8192 + lane * 8;
-#pragma unroll
-            for (int hb = 0; hb < 2; ++hb) {
-                const float l = lsum[64 * hh + 32 * hb + l32];
-                const float mul = l > 0.f ? 1.f / l : 0.f;
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-                        uint32_t w[4];
-#pragma unroll
-                        for (int k = 0; k < 4; ++k)
-                            w[k] = __builtin_bit_cast(uint32_t, f16x2{(_Float16)(o[i][hb][8 * h + 2 * k] * mul), (_Float16)(o[i][hb][8 * h + 2 * k + 1] * mul)});
-                        __builtin_nontemporal_store(u32x4{w[0], w[1], w[2], w[3]}, reinterpret_cast<u32x4*>(wbase + ((hb * 4 + i) * 2 + h) * 512));
-                    }
+    // The score waves publish the row sums; every wave normalises its own blocks.
+    __syncthreads(); // nobody reads a tile, P~ or a factor any more
+    if constexpr (SCORES) {
+        if (hl == 0) {
+            lsum[l32] = l_tot;
+            if (a.nsplit > 1 && head < a.nq) {
+                const int64_t prow = ((int64_t)tq * a.nsplit + sp) * a.nq + head;
+                a.part_ml[prow * 2] = m_out;
+                a.part_ml[prow * 2 + 1] = l_tot;
             }
-        }
-        return;
-    }
-    // One split: the output itself, bf16 rows.  v_permlane32_swap pairs up the two half-waves' four-dim pieces - the lower
-    // half-wave ends up with the 8 dims of block g = 2 gp, the upper one with those of block 2 gp + 1 - so that a lane
-    // stores 16 bytes; all 128 heads' rows are staged in LDS as [head][512] rows of 1024 bytes (everything below
-    // OUT_LSUM_OFF is free now), the 16-byte chunks of a row XOR-swizzled with the head so that the 8 lanes of a b128
-    // access hit distinct banks, and all 512 lanes copy the rows out, a wavefront writing one whole row per instruction.
-    if (pv_active) {
-#pragma unroll
-        for (int hb = 0; hb < 2; ++hb) {
-            const int hrow = 64 * hh + 32 * hb + l32;
-            const float l = lsum[hrow];
-            const float mul = l > 0.f ? 1.f / l : 0.f;
-            uint8_t* orow = smem + hrow * OUT_ROW;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int gp = 0; gp < 2; ++gp) {
-                    uint32_t w[2][2]; // [block 2 gp, 2 gp + 1][pair of dims]
-#pragma unroll
-                    for (int g = 0; g < 2; ++g)
-#pragma unroll
-                        for (int k = 0; k < 2; ++k)
-                            w[g][k] = pack_bf16x2(o[i][hb][4 * (2 * gp + g) + 2 * k] * mul, o[i][hb][4 * (2 * gp + g) + 2 * k + 1] * mul);
-                    // the swap exchanges the upper half-wave of its first operand with the lower half-wave of its second
-                    const auto s0 = __builtin_amdgcn_permlane32_swap(w[0][0], w[1][0], false, false);
-                    const auto s1 = __builtin_amdgcn_permlane32_swap(w[0][1], w[1][1], false, false);
-                    const int c = 4 * (4 * dq + i) + 2 * gp + hl;
-                    *reinterpret_cast<u32x4*>(orow + ((c ^ (hrow & 7)) << 4)) = u32x4{(uint32_t)s0[0], (uint32_t)s1[0], (uint32_t)s0[1], (uint32_t)s1[1]};
-                }
         }
     }
     __syncthreads();
-#pragma unroll 4
-    for (int id = tid; id < HEADS_PER_WG * (DN / 8); id += 512) {
-        const int hrow = id / (DN / 8), c = id % (DN / 8);
-        const int oh = head0 + hrow;
-        if (oh >= a.nq) break; // (wave-uniform: a wavefront copies one row)
-        const u32x4 v = *reinterpret_cast<const u32x4*>(smem + hrow * OUT_ROW + ((c ^ (hrow & 7)) << 4));
-        *reinterpret_cast<u32x4*>(reinterpret_cast<uint8_t*>(a.out) + (((int64_t)tq * a.nq + oh) * DN + c * 8) * 2) = v;
+    if constexpr (!SCORES) l_tot = lsum[l32];
+    const float mul = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    if (a.nsplit > 1) {
+        if (active) val.store_partial(a.part_o + ((((int64_t)tq * a.nsplit + sp) * gridDim.z + hz) * 8 + (pair >> 1)) * 8192 + (pair & 1) * 4096 + lane * 8, mul);
+        return;
+    }
+    val.stage_rows(smem + hrow * OUT_ROW, hrow, hl, mul);
+    __syncthreads();
+    // a wavefront copies whole rows, one per instruction
+    const int row0 = pair * 32 + (SCORES ? 0 : 16);
+#pragma unroll
+    for (int k0 = 0; k0 < 16; k0 += 8) {
+        u32x4 v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = *reinterpret_cast<const u32x4*>(smem + (row0 + k0 + k) * OUT_ROW + ((lane ^ (k0 + k)) << 4));
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int oh = head0 + row0 + k0 + k;
+            if (oh < a.nq) // (wave-uniform)
+                *reinterpret_cast<u32x4*>(reinterpret_cast<uint8_t*>(a.out) + (((int64_t)tq * a.nq + oh) * DN + lane * 8) * 2) = v[k];
+        }
     }
 }
 
@@ -720,21 +771,18 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
 // token as the fastest grid dimension the splits of one token run on one XCD (when the token count is a multiple of 8)
 // and share its L2 for the token's queries.
 template <bool QUANT>
-__global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2))) void sfa_decode_kernel(
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * WAVES, 64 * WAVES), amdgpu_waves_per_eu(2, 2))) void sfa_decode_kernel(
     SfaArgs a)
 {
     extern __shared__ __align__(16) uint8_t smem[];
     uint32_t* tmask = reinterpret_cast<uint32_t*>(smem + SPLIT_OFF);
     int* rows = reinterpret_cast<int*>(smem + SPLIT_OFF + tmask_bytes(a.split_cap));
-    int* bt_lds = reinterpret_cast<int*>(smem + SPLIT_OFF + split_bytes(a.split_cap));
-
-    const int tid = threadIdx.x;
-
-    // Both kinds of wavefront run the same barrier sequence: one before the first tile, two per tile, the epilogue's.
-    if (tid < 256)
-        sfa_wave<QUANT, 0>(a, smem, tmask, rows, bt_lds, tid);
+    int* bt_lds = reinterpret_cast<int*>(smem);
+    // both roles run the same barrier sequence
+    if (threadIdx.x < 64 * PAIRS)
+        sfa_wave<QUANT, true>(a, smem, tmask, rows, bt_lds, threadIdx.x);
     else
-        sfa_wave<QUANT, 1>(a, smem, tmask, rows, bt_lds, tid);
+        sfa_wave<QUANT, false>(a, smem, tmask, rows, bt_lds, threadIdx.x);
 }
 
 // attention_out <- 0 (cache without rows: every selected entry is absent)
@@ -906,10 +954,15 @@ hipError_t sfa_launch(const SfaArgs& a, hipStream_t stream)
     }
     SfaArgs args = a;
     const int tiles = (a.topk + T - 1) / T;
+    // division of a 31-bit index by the page size as a multiplication: with 2^(l-1) < block_size <= 2^l and the multiplier
+    // 2^(31+l) / block_size rounded up (less than 2^32), the excess of the product is less than 2^(31+l) / block_size
+    int l = 0;
+    while (((int64_t)1 << l) < a.block_size) ++l;
+    args.page_mul = (uint32_t)((((uint64_t)1 << (31 + l)) + (uint32_t)a.block_size - 1) / (uint32_t)a.block_size);
+    args.page_shift = 31 + l;
     args.split_cap = (((tiles + a.nsplit - 1) / a.nsplit + 1) & ~1) * T;
-    int smem_bytes = SPLIT_OFF + split_bytes(args.split_cap);
-    args.bt_cached = smem_bytes + a.bt_stride * 4 <= LDS_LIMIT ? 1 : 0;
-    if (args.bt_cached) smem_bytes += a.bt_stride * 4;
+    const int smem_bytes = SPLIT_OFF + split_bytes(args.split_cap);
+    args.bt_cached = a.bt_stride <= BT_MAX ? 1 : 0;
     static DeviceOnce attr_done[2];
     auto kern = a.quant ? sfa_decode_kernel<true> : sfa_decode_kernel<false>;
     {
@@ -923,7 +976,7 @@ hipError_t sfa_launch(const SfaArgs& a, hipStream_t stream)
     dim3 grid(t, a.nsplit, hgroups);
     {
         ScopedKernelTimer tm(KID_SFA_DECODE, stream);
-        hipLaunchKernelGGL(kern, grid, dim3(512), smem_bytes, stream, args);
+        hipLaunchKernelGGL(kern, grid, dim3(64 * WAVES), smem_bytes, stream, args);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

@@ -126,6 +126,49 @@ def test_absent_entries_inside_the_list_are_skipped(cuda):
     full_check(out, ref_case, "absent entries")
 
 
+def run_with_splits(case, dev, splits):
+    """The C ABI with a forced number of KV splits."""
+    from pypto_amd import _runtime
+    lib = _runtime.load_library()
+    b, nq, topk, q = case["b"], case["nq"], case["topk"], case["q"]
+    ts = [q[..., :512].reshape(-1, 512).contiguous().to(dev), q[..., 512:].reshape(-1, 64).contiguous().to(dev),
+          case["kn"].to(dev), case["kr"].to(dev), case["kn_scales"].to(dev), case["topk_indices"].to(dev),
+          case["block_table"].to(dev), torch.tensor(case["act_seq"], dtype=torch.int32, device=dev),
+          torch.zeros((b, 1, nq, 512), dtype=torch.bfloat16, device=dev)]
+    d = _runtime.describe(ts)
+    p = _runtime.SfaParams(nq, 1, case["softmax_scale"], topk, case["block_size"], case["block_table"].shape[1], splits)
+    n = lib.pto_sfa_quant_workspace(d, 9, ctypes.byref(p))
+    ws = torch.empty(max(n, 1), dtype=torch.uint8, device=dev)
+    assert lib.pto_sfa_quant_launch(d, 9, ctypes.byref(p), ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream, 0) == 0, lib.pto_last_error()
+    torch.cuda.synchronize()
+    return ts[8].cpu()
+
+
+@pytest.mark.parametrize("quant", [True, False])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_lists_around_tile_boundaries(cuda, quant, splits):
+    """No tile, one, two, three and more tiles of 32 entries, whole and ragged: every start and end of the tile pipeline.
+    40 heads leave half of a head group's waves without work and one with eight heads."""
+    acts = [0, 1, 31, 32, 33, 64, 65, 96, 97, 129, 256]
+    case = osfa.make_case(len(acts), 40, 1, acts, topk=256, block_size=48, seed=31, dist="bench", quant=quant, softmax_scale=192 ** -0.5)
+    out = run_with_splits(case, cuda, splits)
+    assert (out[0] == 0).all()
+    full_check(out, case, f"lists of {acts}")
+
+
+@pytest.mark.parametrize("dead", [(0, 32), (32, 64), (224, 256), (16, 240)])
+def test_tiles_without_a_present_entry(cuda, dead):
+    """Whole tiles of absent entries at the start, inside and at the end of a list, and all but two half tiles: the result
+    is attention over the entries that remain."""
+    case = osfa.make_case(1, 128, 1, [700], topk=256, seed=32, dist="bench", softmax_scale=192 ** -0.5)
+    tk = case["topk_indices"].clone()
+    tk[0, dead[0]:dead[1]] = -1
+    keep = [j for j in range(256) if not dead[0] <= j < dead[1]]
+    ref = dict(case, topk_indices=case["topk_indices"][:, keep].contiguous(), topk=len(keep))
+    for splits in (1, 4):
+        full_check(run_with_splits(dict(case, topk_indices=tk), cuda, splits), ref, f"absent {dead}, {splits} splits")
+
+
 def test_forced_kv_splits_agree(cuda):
     """Drives the C ABI directly: 1, 2, 4 and 16 KV splits of the same problem."""
     from pypto_amd import _runtime
