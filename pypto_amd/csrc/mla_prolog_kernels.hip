@@ -472,102 +472,114 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb16_wide_kernel(MlaPrologArg
 __device__ __forceinline__ float wave_sum(float v) { return wave_sum_butterfly(v); }
 __device__ __forceinline__ float wave_max(float v) { return wave_max_f32(v); }
 
-// one workgroup of 256 lanes per token; S: splits whose partial sums are in flight together
+// Columns col0 + tid + 256 j, j < NJ, of a token's row: partial sums in a fixed order, rounded to bf16, into buf (n columns; S:
+// splits whose partial sums are in flight together).  Every load is unconditional (columns past the end re-read the last
+// one and are dropped): a load under a condition makes the compiler wait for it on the spot, one memory round trip per load.
+template <int S, int NJ>
+__device__ __forceinline__ void mla_sums(const MlaPrologArgs& a, int tok, int col0, int n, float* buf)
+{
+    const int tid = threadIdx.x;
+    int cj[NJ];
+    float sum[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        cj[j] = col0 + min(256 * j + tid, n - 1);
+        sum[j] = 0.f;
+    }
+    // (a split past the end re-reads the last one and adds zero)
+    for (int s0 = 0; s0 < a.ksplits; s0 += S) {
+        float v[S][NJ];
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+            const float* p = a.xa_part + ((int64_t)min(s0 + i, a.ksplits - 1) * a.t + tok) * a.ncols;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) v[i][j] = p[cj[j]];
+        }
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) sum[j] += s0 + i < a.ksplits ? v[i][j] : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+        if (256 * j + tid < n) buf[256 * j + tid] = round_bf16(sum[j]);
+}
+
+// The two norms of a token are independent chains of loads, reductions and barriers: a workgroup of 256 lanes for either (one
+// workgroup for both, one chain behind the other: 1.6 us more a call, at 1 token as at 600).
+// Query: RmsNorm over r, then per-token quantisation.
 template <int S>
-__device__ __forceinline__ void mla_norm_body(const MlaPrologArgs& a, int tok)
+__device__ __forceinline__ void mla_norm_query_body(const MlaPrologArgs& a, int tok)
 {
 #pragma clang fp contract(off)
-    __shared__ float buf[MAX_R + MKV];
+    __shared__ float buf[MAX_R];
     __shared__ float red[8];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int r = a.r, ncols = r + MKV;
-    // everything that does not depend on the sums is loaded first, so that its latency hides behind them
-    const int64_t row = a.cache_index[tok];
-    const bool row_ok = row >= 0 && row < a.cache_rows;
+    const int r = a.r;
+    // (what does not depend on the sums is loaded first, so that its latency hides behind them)
     constexpr int NQ = MAX_R / 256;
     uint16_t gq[NQ];
 #pragma unroll
     for (int j = 0; j < NQ; ++j) gq[j] = 256 * j + tid < r ? a.gamma_cq[256 * j + tid] : (uint16_t)0;
+    mla_sums<S, NQ>(a, tok, 0, r, buf);
+    __syncthreads();
+    const float coff = 1.0f / (float)r;
+    float ss = 0.f;
+    for (int c = tid; c < r; c += 256) ss += (buf[c] * buf[c]) * coff;
+    ss = wave_sum(ss);
+    if (lane == 0) red[wave] = ss;
+    __syncthreads();
+    const float y = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) + a.eps_cq);
+    float mx = 0.f;
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {
+        const int c = 256 * j + tid;
+        if (c < r) {
+            const float v = round_bf16(bf16_to_f32(gq[j]) * (buf[c] * y));
+            buf[c] = v;
+            mx = fmaxf(mx, fabsf(v));
+        }
+    }
+    mx = wave_max(mx);
+    if (lane == 0) red[4 + wave] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));
+    if (a.quant) {
+        const float sq = quant_scale(mx);
+        // four values per lane and store
+        for (int c = 4 * tid; c < r; c += 1024) {
+            uint32_t pk = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(buf[c + e] * sq) & 0xffu) << (8 * e);
+            *reinterpret_cast<uint32_t*>(a.q_norm + (int64_t)tok * r + c) = pk;
+        }
+        if (tid == 0) a.q_norm_scale[tok] = 1.0f / sq;
+    } else { // bf16 form: q_norm is the normalised row itself
+        uint16_t* qo = reinterpret_cast<uint16_t*>(a.q_norm) + (int64_t)tok * r;
+        for (int c = 4 * tid; c < r; c += 1024)
+            *reinterpret_cast<u32x2*>(qo + c) = u32x2{(uint32_t)f32_to_bf16(buf[c]) | ((uint32_t)f32_to_bf16(buf[c + 1]) << 16),
+                                                      (uint32_t)f32_to_bf16(buf[c + 2]) | ((uint32_t)f32_to_bf16(buf[c + 3]) << 16)};
+    }
+}
+
+// Key: RmsNorm over 512 (lane: elements tid and tid + 256), groups of 128 quantised on their own, rotary, the cache rows.
+template <int S>
+__device__ __forceinline__ void mla_norm_key_body(const MlaPrologArgs& a, int tok)
+{
+#pragma clang fp contract(off)
+    __shared__ float buf[MKV];
+    __shared__ float red[8];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t row = a.cache_index[tok];
+    const bool row_ok = row >= 0 && row < a.cache_rows;
     const uint16_t gk0 = a.gamma_ckv[tid], gk1 = a.gamma_ckv[256 + tid];
     const int ri = tid & 31;
     const float rc0 = bf16_to_f32(a.cos[(int64_t)tok * MROPE + ri]), rc1 = bf16_to_f32(a.cos[(int64_t)tok * MROPE + ri + 32]);
     const float rs0 = bf16_to_f32(a.sin[(int64_t)tok * MROPE + ri]), rs1 = bf16_to_f32(a.sin[(int64_t)tok * MROPE + ri + 32]);
-    // q_a and kv: partial sums in a fixed order, rounded to bf16 (lane: columns tid + 256 j; all of a split's loads in
-    // flight together)
-    {
-        constexpr int NJ = (MAX_R + MKV + 255) / 256;
-        // every load is unconditional (columns past the end re-read the last one and are dropped below): a load under
-        // a condition makes the compiler wait for it on the spot, one memory round trip per load
-        int cj[NJ];
-        float sum[NJ];
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            cj[j] = min(256 * j + tid, ncols - 1);
-            sum[j] = 0.f;
-        }
-        // (a split past the end re-reads the last one and adds zero)
-        for (int s0 = 0; s0 < a.ksplits; s0 += S) {
-            float v[S][NJ];
-#pragma unroll
-            for (int i = 0; i < S; ++i) {
-                const float* p = a.xa_part + ((int64_t)min(s0 + i, a.ksplits - 1) * a.t + tok) * a.ncols;
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) v[i][j] = p[cj[j]];
-            }
-#pragma unroll
-            for (int i = 0; i < S; ++i)
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) sum[j] += s0 + i < a.ksplits ? v[i][j] : 0.f;
-        }
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-            if (256 * j + tid < ncols) buf[256 * j + tid] = round_bf16(sum[j]);
-    }
+    mla_sums<S, (MKV + 255) / 256>(a, tok, a.r, MKV, buf);
     __syncthreads();
-    // query: RmsNorm over r, then per-token quantisation
     {
-        const float coff = 1.0f / (float)r;
-        float ss = 0.f;
-        for (int c = tid; c < r; c += 256) ss += (buf[c] * buf[c]) * coff;
-        ss = wave_sum(ss);
-        if (lane == 0) red[wave] = ss;
-        __syncthreads();
-        const float y = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) + a.eps_cq);
-        float mx = 0.f;
-#pragma unroll
-        for (int j = 0; j < NQ; ++j) {
-            const int c = 256 * j + tid;
-            if (c < r) {
-                const float v = round_bf16(bf16_to_f32(gq[j]) * (buf[c] * y));
-                buf[c] = v;
-                mx = fmaxf(mx, fabsf(v));
-            }
-        }
-        mx = wave_max(mx);
-        if (lane == 0) red[4 + wave] = mx;
-        __syncthreads();
-        mx = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));
-        if (a.quant) {
-            const float sq = quant_scale(mx);
-            // four values per lane and store
-            for (int c = 4 * tid; c < r; c += 1024) {
-                uint32_t pk = 0;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(buf[c + e] * sq) & 0xffu) << (8 * e);
-                *reinterpret_cast<uint32_t*>(a.q_norm + (int64_t)tok * r + c) = pk;
-            }
-            if (tid == 0) a.q_norm_scale[tok] = 1.0f / sq;
-        } else { // bf16 form: q_norm is the normalised row itself
-            uint16_t* qo = reinterpret_cast<uint16_t*>(a.q_norm) + (int64_t)tok * r;
-            for (int c = 4 * tid; c < r; c += 1024)
-                *reinterpret_cast<u32x2*>(qo + c) = u32x2{(uint32_t)f32_to_bf16(buf[c]) | ((uint32_t)f32_to_bf16(buf[c + 1]) << 16),
-                                                          (uint32_t)f32_to_bf16(buf[c + 2]) | ((uint32_t)f32_to_bf16(buf[c + 3]) << 16)};
-        }
-    }
-    __syncthreads();
-    // key: RmsNorm over 512 (lane: elements tid and tid + 256), groups of 128 quantised on their own
-    {
-        const float x0 = buf[r + tid], x1 = buf[r + 256 + tid];
+        const float x0 = buf[tid], x1 = buf[256 + tid];
         float ss = wave_sum((x0 * x0) * (1.0f / MC) + (x1 * x1) * (1.0f / MC));
         if (lane == 0) red[wave] = ss;
         __syncthreads();
@@ -600,12 +612,28 @@ __device__ __forceinline__ void mla_norm_body(const MlaPrologArgs& a, int tok)
     }
     // key rotary: pair i = elements (2i, 2i+1) -> positions (i, 32 + i)
     if (tid < MROPE / 2 && row_ok) {
-        const float xe = buf[r + MC + 2 * tid], xo = buf[r + MC + 2 * tid + 1];
+        const float xe = buf[MC + 2 * tid], xo = buf[MC + 2 * tid + 1];
         const float o1 = xe * rc0 + (-xo) * rs0;
         const float o2 = xo * rc1 + xe * rs1;
         a.kr_cache[row * MROPE + tid] = f32_to_bf16(o1);
         a.kr_cache[row * MROPE + 32 + tid] = f32_to_bf16(o2);
     }
+}
+
+// The head of a weight slice, read and dropped: the first `rows` rows of 16 `pieces` bytes (rows a multiple of what 256 lanes
+// cover in one go, up to 24 times that), so that the workgroup of the next launch that streams the slice finds them in
+// its XCD's L2.
+__device__ __forceinline__ void touch_rows(const uint8_t* base, int64_t stride, int rows, int pieces)
+{
+    const int per = 256 / pieces, row = threadIdx.x / pieces, n = rows / per;
+    const uint8_t* p = base + row * stride + (threadIdx.x % pieces) * 16;
+    u32x4 v[24];
+#pragma unroll
+    for (int i = 0; i < 24; ++i)
+        if (i < n) v[i] = *reinterpret_cast<const u32x4*>(p + i * per * stride);
+#pragma unroll
+    for (int i = 0; i < 24; ++i)
+        if (i < n) asm volatile("" ::"v"(v[i]));
 }
 
 // ------------------------------------------------------------------------------------------------ q_norm @ w_uq_qr
@@ -641,11 +669,31 @@ __device__ __forceinline__ void mla_qb_body(const MlaPrologArgs& a, int tile, ui
     qb_store_blocks<MTOK>(a, lds, 2 * tile, 0);
 }
 
-// grid (tokens), 256 lanes
-template <int S>
-__global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a)
+// Decode batches: while the norms' few workgroups go through their chains, the rest of the chip has nothing to do, and the
+// next launch starts with a stream of weights.  The workgroups from `first` on (a multiple of eight: workgroups go to the XCDs
+// round-robin) read the head of the slice that the workgroup of the same number past `first` streams next (bf16 form, 24 tokens:
+// 41.5 us a call without, 41.3 / 40.8 / 40.5 with 32 / 64 / 96 KB of a slice; int8, 2 tokens: 30.1, 29.7 / 29.3 / 29.2).
+constexpr int TOUCH_BYTES = 96 * 1024; // of a slice: 32 workgroups of an XCD leave a quarter of its 4 MB L2
+
+__device__ __forceinline__ void mla_touch(const MlaPrologArgs& a, int tile)
 {
-    mla_norm_body<S>(a, blockIdx.x);
+    const int64_t stride = (int64_t)a.n * MQH * (a.quant ? 1 : 2);
+    const int pieces = a.quant ? 8 : 16; // 128 outputs (the half tile that the bf16 form may end with is not asked for)
+    const int rows = min(a.r, TOUCH_BYTES / (16 * pieces)) & ~31;
+    touch_rows(static_cast<const uint8_t*>(a.w_uq_qr) + (int64_t)tile * 16 * pieces, stride, rows, pieces);
+}
+
+// grid (2 x tokens: query, key | touching workgroups from `first` on), 256 lanes
+template <int S>
+__global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a, int first)
+{
+    const int id = blockIdx.x;
+    if (id < a.t)
+        mla_norm_query_body<S>(a, id);
+    else if (id < 2 * a.t)
+        mla_norm_key_body<S>(a, id - a.t);
+    else if (id >= first)
+        mla_touch(a, id - first);
 }
 
 // grid (n * 192 / 128), 256 lanes
@@ -852,15 +900,24 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb_wide_kernel(MlaPrologArgs 
 // The fused operator runs the two prologs' per-token kernels side by side in one launch, and likewise the two int8
 // GEMMs on q_norm (192 + 64 workgroups at model sizes: one per compute unit); the indexer's x @ [w_k | w_proj] rides along
 // in mla_xa_kernel as three more output tiles.
-// grid (tokens, 2), 256 lanes: y = 0 the MLA norms and cache rows, y = 1 the indexer's key path and weights (128 lanes)
+// grid (3 x tokens: the MLA norms, the indexer's key path and weights (128 lanes) | touching workgroups from `first` on), 256 lanes
 template <int S>
-__global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, PrologArgs p)
+__global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, PrologArgs p, int first)
 {
-    if (blockIdx.y == 0) {
-        mla_norm_body<S>(m, blockIdx.x);
-    } else {
+    const int id = blockIdx.x;
+    if (id < m.t)
+        mla_norm_query_body<S>(m, id);
+    else if (id < 2 * m.t)
+        mla_norm_key_body<S>(m, id - m.t);
+    else if (id < 3 * m.t) {
         if (threadIdx.x >= 128) return; // the barriers inside are among the two remaining waves
-        prolog_k_body<S>(p, blockIdx.x);
+        prolog_k_body<S>(p, id - 2 * m.t);
+    } else if (id >= first) {
+        const int tile = id - first, nqb = m.n * MQH / 128;
+        if (tile < nqb)
+            mla_touch(m, tile);
+        else
+            touch_rows(reinterpret_cast<const uint8_t*>(p.w_qb) + (int64_t)(tile - nqb) * PD, (int64_t)p.n * PD, min(p.r, TOUCH_BYTES / PD) & ~31, 8);
     }
 }
 
@@ -1085,12 +1142,14 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         ScopedKernelTimer tm(KID_MLA_NORM, stream);
         // all partial sums of an output in flight at once for the usual seven splits and fewer, none of them twice for one or two
         const int in_flight = a.ksplits <= 2 ? 2 : a.ksplits <= 4 ? 4 : 8;
+        const int norms = (p ? 3 : 2) * a.t, first = (norms + 7) / 8 * 8;
+        const unsigned grid = big ? norms : first + a.n * MQH / 128 + (p ? p->n : 0); // (the kernels above BIG_T tokens do not wait for their weights)
         if (p)
             hipLaunchKernelGGL((in_flight == 2 ? fused_norm_kernel<2> : in_flight == 4 ? fused_norm_kernel<4> : fused_norm_kernel<8>),
-                               dim3(a.t, 2), dim3(256), 0, stream, a, *p);
+                               dim3(grid), dim3(256), 0, stream, a, *p, first);
         else
             hipLaunchKernelGGL((in_flight == 2 ? mla_norm_kernel<2> : in_flight == 4 ? mla_norm_kernel<4> : mla_norm_kernel<8>),
-                               dim3(a.t), dim3(256), 0, stream, a);
+                               dim3(grid), dim3(256), 0, stream, a, first);
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
     {
