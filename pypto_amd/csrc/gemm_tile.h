@@ -1,10 +1,13 @@
 // Main loop of the products at prefill sizes: a workgroup of 512 lanes owns 32 TB tokens (128 to 256) x 256 outputs.
 //
-// What bounds these products at prefill sizes is what the CUs draw from the L2: with the matrix instructions taken out, the
-// copies of 128 x 128 tiles alone (1.03 GB for 777 tokens x 5120 x 14336) take 77 of the product's 87 us, 13 TB/s, wherever the
-// tiles lie, and staging through registers under two barriers a stage took 99 us.  So the tile is as large as LDS and registers
-// hold: 537 MB and 74 us there, where the copies alone take 72 (a round trip per stage) and the rest alone 59; a ring of five
-// half stages with the fragments read a stage ahead is no faster.  And
+// What bounds these products at prefill sizes is first what the CUs draw from the L2: with the matrix instructions taken out, the
+// copies of 128 x 128 tiles alone (1.03 GB for 777 tokens x 5120 x 14336) take 77 us, 13 TB/s, wherever the tiles lie.  So the
+// tile is as large as LDS and registers hold (537 MB there).  Then a CU's own pipes: of a stage of 224 x 256 x 128 the matrix
+// instructions take 1792 ticks, the LDS reads and the copies' writes some 1250, the copies' instructions 960, and the loop is as
+// good as these overlap.  40 such stages take 122.6 K ticks with the copies issued first and the fragments read in front of
+// their products, 111 K with the copies between the matrix instructions, 107 K with the products half a stage behind the reads
+// besides (a call of 777 tokens x 112 heads 90.8 us, 88.7, 86.4; 1024 tokens 101.0, 98.3, 95.9).  The waves' priorities make no
+// difference: the second wave of a SIMD is done when it would be anyway, the first waits for it at the barrier.  And
 //  - a stage's operands are copied to LDS by the memory pipe itself (global_load_lds_dwordx4: no registers, no LDS store
 //    instructions), into the buffer that is not being read, so that a stage has one barrier;
 //  - rows of 128 bytes are kept unpadded (a copy writes 64 lanes x 16 bytes in a row) and spread over the banks by
@@ -26,13 +29,20 @@ namespace {
 
 constexpr int GT_LANES = 512;
 constexpr int GT_KI8 = 128;                  // contraction rows per stage
+constexpr int gt_lds_bytes(int tb) // of an int8 tile's stages
+{
+    const int q = 32 * tb * 128, w = 2 * 128 * 128;
+    return (3 * (q + w) <= 160 * 1024 ? 3 : 2) * q + 3 * w;
+}
 template <int TB>
 struct GtTile {
     static constexpr int TOK = 32 * TB;             // tokens of the tile
     static constexpr int QBYTES = TOK * 128;        // a stage in LDS: token rows | [2] weight rows, 128 bytes each
-    static constexpr int STAGE = QBYTES + 2 * 128 * 128;
-    static constexpr int RING = 3 * STAGE <= 160 * 1024 ? 3 : 2; // stages in LDS, one workgroup to a CU: up to 160 tokens two in flight
-    static constexpr int LDS = RING * STAGE;
+    static constexpr int WBYTES = 2 * 128 * 128, STAGE = QBYTES + WBYTES;
+    // stages in LDS, one workgroup to a CU: two in flight, of the token rows above 160 tokens one (what LDS holds)
+    static constexpr int WRING = 3, RING = 3 * STAGE <= 160 * 1024 ? 3 : 2;
+    static constexpr int WOFF = RING * QBYTES, LDS = gt_lds_bytes(TB); // int8: the token rows' buffers, the weights'
+    static_assert(LDS == WOFF + WRING * WBYTES && LDS <= 160 * 1024, "");
 };
 
 typedef __attribute__((address_space(3))) uint8_t gt_lds;
@@ -77,6 +87,43 @@ __device__ __forceinline__ void gt_stages(int stages, Copy&& copy, Multiply&& mu
     gt_landed<0>();
 }
 
+// The tiles' loop: the operands in rings of their own, the weights one stage further ahead where they have one more buffer, and
+// the copies between the matrix instructions.  A copy keeps the CU's texture addresser busy for 16 ticks: issued in one go at
+// the head of a stage, the 60 of a 224 x 256 tile held the last wave up for 960 ticks, after which all matrix instructions
+// were still to come.  copy_q(i, stage, byte offset of the buffer), i < QC, and copy_w(..), i < WC: one copy of a wave;
+// multiply(byte offsets of both, issue): calls issue(i) for all QC + WC in order, somewhere.
+template <int QRING, int QSTAGE, int QC, int WRING, int WSTAGE, int WC, class CopyQ, class CopyW, class Multiply>
+__device__ __forceinline__ void gt_tile_stages(int stages, CopyQ&& copy_q, CopyW&& copy_w, Multiply&& multiply)
+{
+    static_assert(QRING == WRING || QRING + 1 == WRING, "the order of the copies that the wait counts on");
+    // behind a stage's token rows: the weights of their round, where those are of a later stage, and the rounds since
+    constexpr int BEHIND = (QRING - 2) * (QC + WC) + (QRING < WRING ? WC : 0);
+#pragma unroll
+    for (int s = 0; s < WRING - 1; ++s) { // (the token rows of the first stage with the weights of the last one ahead)
+        if (s >= WRING - QRING)
+#pragma unroll
+            for (int i = 0; i < QC; ++i) copy_q(i, min(s - (WRING - QRING), stages - 1), (s - (WRING - QRING)) * QSTAGE);
+#pragma unroll
+        for (int i = 0; i < WC; ++i) copy_w(i, min(s, stages - 1), s * WSTAGE);
+    }
+    int qin = (QRING - 1) * QSTAGE, qout = 0, win = (WRING - 1) * WSTAGE, wout = 0;
+    for (int st = 0; st < stages; ++st) {
+        gt_landed<BEHIND>(); // stage st is there, and everyone is done with the buffers of the stage before
+        const int qst = min(st + QRING - 1, stages - 1), wst = min(st + WRING - 1, stages - 1);
+        multiply(st, qout, wout, [&](int i) {
+            if (i < QC)
+                copy_q(i, qst, qin);
+            else
+                copy_w(i - QC, wst, win);
+        });
+        qin = qin == (QRING - 1) * QSTAGE ? 0 : qin + QSTAGE;
+        qout = qout == (QRING - 1) * QSTAGE ? 0 : qout + QSTAGE;
+        win = win == (WRING - 1) * WSTAGE ? 0 : win + WSTAGE;
+        wout = wout == (WRING - 1) * WSTAGE ? 0 : wout + WSTAGE;
+    }
+    gt_landed<0>();
+}
+
 // acc[nb][tb] += w[k, col0 + ..]^T . q[token, k], int8.  w0, w1: first contraction row of the two halves' columns, ldw bytes a
 // row; q: [t, ldq], column of the first contraction row.  Register e of acc[nb][tb]: output 64 wc + 16 nb + 4 g + e, token
 // 16 TB wr + 16 tb + l16.
@@ -101,41 +148,60 @@ __device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t*
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) wo[i] = (uint32_t)((row + 64 * i) * (int)ldw + 16 * (pos ^ (((row >> 1) & 3) | ((row >> 2) & 4))));
-    auto copy = [&](int st, int b) {
-#pragma unroll
-        for (int i = 0; i < QC; ++i) gt_copy(qb + st * GT_KI8, qo[i], lds + b + qd[i]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            gt_copy((i < 2 ? w0 : w1) + (int64_t)st * GT_KI8 * ldw, wo[i & 1], lds + b + T::QBYTES + 8192 * i + 1024 * wave);
+    auto copy_q = [&](int i, int st, int b) { gt_copy(qb + st * GT_KI8, qo[i], lds + b + qd[i]); };
+    auto copy_w = [&](int i, int st, int b) {
+        gt_copy((i < 2 ? w0 : w1) + (int64_t)st * GT_KI8 * ldw, wo[i & 1], lds + T::WOFF + b + 8192 * i + 1024 * wave);
     };
     // token fragments: row 16 TB wr + 16 tb + l16, piece 4 ks + g.  Weight fragments by the byte-transposing read, which hands
     // lane i of a 16-lane group byte i % 8 of the chunks addressed by lanes i / 8, i / 8 + 2, ...: lane i points at row i / 2
     // (+ 8 for the second read), half i % 2 of the 16-column piece 4 (wc & 1) + nb, and gets column i over rows 0 .. 7
     const uint8_t* qr = lds + (16 * TB * wr + l16) * 128;
     const int qpos = 16 * (g ^ ((l16 >> 1) & 7));
-    const uint8_t* wrow = lds + T::QBYTES + (wc >> 1) * 16384 + (16 * g + (l16 >> 1)) * 128 + 8 * (l16 & 1);
+    const uint8_t* wrow = lds + T::WOFF + (wc >> 1) * 16384 + (16 * g + (l16 >> 1)) * 128 + 8 * (l16 & 1);
     int wpos[4];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) wpos[nb] = 16 * ((4 * (wc & 1) + nb) ^ (((l16 >> 2) & 3) | ((g & 1) << 2)));
-    gt_stages<T::RING, T::STAGE, QC + 4>(stages, copy, [&](int, int b) {
+    // Half a stage behind: what follows a barrier is the second half of the stage before, whose fragments are in registers,
+    // while the first half's are read.  (With the reads of a stage in front of its own products the matrix pipes waited
+    // some 600 ticks of 2760 for all eight waves' fragments to come out of LDS.)
+    i32x4 qf[2][TB], wf[2][4];
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            i32x4 qf[TB], wf[4];
+    for (int tb = 0; tb < TB; ++tb) qf[1][tb] = i32x4{0, 0, 0, 0}; // ("the stage before" the first: products of zero)
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) wf[1][nb] = i32x4{0, 0, 0, 0};
+    auto mfma = [&](int ks, auto&& between) {
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb)
+                acc[nb][tb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[ks][nb], qf[ks][tb], acc[nb][tb], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            between(tb);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    gt_tile_stages<T::RING, T::QBYTES, QC, T::WRING, T::WBYTES, 4>(stages, copy_q, copy_w, [&](int, int b, int bw, auto&& issue) {
+        auto read = [&](int ks) {
 #pragma unroll
             for (int nb = 0; nb < 4; ++nb) {
-                const uint8_t* p = wrow + b + 8192 * ks + wpos[nb];
+                const uint8_t* p = wrow + bw + 8192 * ks + wpos[nb];
                 const v2i lo = lds_read_tr8(p), hi = lds_read_tr8(p + 1024);
-                wf[nb] = i32x4{lo[0], lo[1], hi[0], hi[1]};
+                wf[ks][nb] = i32x4{lo[0], lo[1], hi[0], hi[1]};
             }
 #pragma unroll
-            for (int tb = 0; tb < TB; ++tb) qf[tb] = *reinterpret_cast<const i32x4*>(qr + b + 2048 * tb + (qpos ^ (64 * ks)));
-#pragma unroll
-            for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-                for (int nb = 0; nb < 4; ++nb)
-                    acc[nb][tb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[nb], qf[tb], acc[nb][tb], 0, 0, 0);
-        }
+            for (int tb = 0; tb < TB; ++tb) qf[ks][tb] = *reinterpret_cast<const i32x4*>(qr + b + 2048 * tb + (qpos ^ (64 * ks)));
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        read(0);
+        mfma(1, [&](int tb) {
+            if (tb < QC + 4) issue(tb);
+        });
+        read(1);
+        mfma(0, [&](int tb) {
+            if (TB + tb < QC + 4) issue(TB + tb);
+        });
     });
+    mfma(1, [](int) {});
 }
 
 // Up to 32 tokens x 128 outputs, 256 lanes: a stream of weights, five stages of 128 rows in flight straight to LDS.  Wave w owns
@@ -208,19 +274,14 @@ __device__ __forceinline__ void gt_product_bf16(f32x16 (&sum)[2][2], const uint1
         xo[i] = (uint32_t)(min(row + 64 * i, t - 1 - tok0) * (int)ldx * 2 + 16 * (pos ^ ((row >> 1) & 7)));
 #pragma unroll
     for (int i = 0; i < 4; ++i) wo[i] = (uint32_t)(row * ld[i] * 2 + 16 * (pos ^ ((row << 1) & 4)));
-    auto copy = [&](int st, int b) {
-        uint8_t* d = lds + b + 1024 * wave;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) gt_copy(xb + st * GT_KBF, xo[i], d + 8192 * i);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) gt_copy(src[i] + (int64_t)st * GT_KBF * ld[i], wo[i], d + T::QBYTES + 8192 * i);
-    };
+    auto copy_x = [&](int i, int st, int b) { gt_copy(xb + st * GT_KBF, xo[i], lds + b + 1024 * wave + 8192 * i); };
+    auto copy_w = [&](int i, int st, int b) { gt_copy(src[i] + (int64_t)st * GT_KBF * ld[i], wo[i], lds + T::WOFF + b + 1024 * wave + 8192 * i); };
     // token fragments: row 64 wr + 32 tb + l32, piece 2 ks + hl.  Weight fragments by 16-bit transposing reads: lane jj of a
     // 16-lane group points at row 8 hl + jj / 4 (+ 4 for the second read) of the step, columns 16 mh + 4 (jj & 3), and gets
     // column 16 mh + jj over those rows
     const uint8_t* xr = lds + (64 * wr + l32) * 128;
     const int xf = (l32 >> 1) & 7;
-    const uint8_t* wrow = lds + T::QBYTES + wc * 8192 + (8 * hl + (jj >> 2)) * 128 + 8 * (jj & 1);
+    const uint8_t* wrow = lds + T::WOFF + wc * 8192 + (8 * hl + (jj >> 2)) * 128 + 8 * (jj & 1);
     const int wpos = 16 * ((2 * mh + ((jj >> 1) & 1)) ^ ((jj >> 1) & 4));
     static_assert(GROUP % CHAIN == 0 && CHAIN % GT_KBF == 0, "whole chains");
     constexpr bool TWO = GROUP > CHAIN; // (else a chain goes straight to the sums)
@@ -245,31 +306,56 @@ __device__ __forceinline__ void gt_product_bf16(f32x16 (&sum)[2][2], const uint1
                     from[tb][nb][e] = 0.f;
                 }
     };
-    gt_stages<T::RING, T::STAGE, 6>(stages, copy, [&](int st, int b) {
+    // (a step behind, as in gt_product_i8: after a barrier the last step of the stage before, and with it the end of a chain)
+    constexpr int STEPS = GT_KBF / 16;
+    bf16x8 xv[2][2], wv[2][2];
 #pragma unroll
-        for (int ks = 0; ks < GT_KBF / 16; ++ks) {
-            bf16x8 xv[2], wv[2];
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xv[1][i][e] = wv[1][i][e] = (__bf16)0.f;
+    auto mfma = [&](int set, auto&& between) {
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) {
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+                acc[tb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv[set][tb], wv[set][nb], acc[tb][nb], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            between(tb);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto finish = [&](int done, bool last) { // `done` stages are summed up
+        if constexpr (TWO) {
+            if (done % (CHAIN / GT_KBF) == 0 || last) add(part, acc);
+            if (done % (GROUP / GT_KBF) == 0 || last) add(sum, part);
+        } else {
+            if (done % (CHAIN / GT_KBF) == 0 || last) add(sum, acc);
+        }
+    };
+    static_assert(STEPS % 2 == 0, "the last step's fragments are in set 1");
+    gt_tile_stages<T::RING, T::QBYTES, 2, T::WRING, T::WBYTES, 4>(stages, copy_x, copy_w, [&](int st, int b, int bw, auto&& issue) {
+        auto read = [&](int ks) {
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
-                const uint8_t* p = wrow + b + 2048 * ks + (wpos ^ (64 * nb));
+                const uint8_t* p = wrow + bw + 2048 * ks + (wpos ^ (64 * nb));
                 const s16x4 lo = lds_read_tr(p), hi = lds_read_tr(p + 512);
-                wv[nb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                wv[ks & 1][nb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
             }
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb) xv[tb] = *reinterpret_cast<const bf16x8*>(xr + b + 4096 * tb + 16 * ((2 * ks + hl) ^ xf));
+            for (int tb = 0; tb < 2; ++tb) xv[ks & 1][tb] = *reinterpret_cast<const bf16x8*>(xr + b + 4096 * tb + 16 * ((2 * ks + hl) ^ xf));
+            __builtin_amdgcn_sched_barrier(0);
+        };
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb) acc[tb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv[tb], wv[nb], acc[tb][nb], 0, 0, 0);
-        }
-        const bool last = st + 1 == stages;
-        if constexpr (TWO) {
-            if ((st + 1) % (CHAIN / GT_KBF) == 0 || last) add(part, acc);
-            if ((st + 1) % (GROUP / GT_KBF) == 0 || last) add(sum, part);
-        } else {
-            if ((st + 1) % (CHAIN / GT_KBF) == 0 || last) add(sum, acc);
+        for (int ks = 0; ks < STEPS; ++ks) {
+            read(ks);
+            mfma(1 - (ks & 1), [&](int tb) {
+                if (2 * ks + tb < 6) issue(2 * ks + tb);
+            });
+            if (ks == 0 && st > 0) finish(st, false);
         }
     });
+    mfma(1, [](int) {});
+    finish(stages, true);
 }
 
 // Token blocks TB (4 .. most) of an int8 product's tile, by the time it should take in ns: the grid runs in rounds of one

@@ -851,7 +851,7 @@ __global__ __launch_bounds__(256, 2) void mla_qb_big_kernel(MlaPrologArgs a)
 // them.  128 x 128 tiles through registers took 109 us at 1501 tokens, bound by the operands' way into LDS.
 constexpr int mla_qb_wide_lds(int tb) // the product's stages, or four blocks of the output tile
 {
-    const int tok = 32 * tb, stage = tok * 128 + 2 * 128 * 128, ring = (3 * stage <= 160 * 1024 ? 3 : 2) * stage;
+    const int tok = 32 * tb, ring = gt_lds_bytes(tb);
     return 4 * tok * QBS_ROW > ring ? 4 * tok * QBS_ROW : ring;
 }
 template <int TB>

@@ -416,7 +416,7 @@ __device__ __forceinline__ void prolog_q_big_body(const PrologArgs& a, int head,
 // and dropped.
 constexpr int prolog_q_wide_lds(int tb) // the product's stages, or hadamard_q | [2] bf16 tiles | [2] per-wave maxima
 {
-    const int tok = 32 * tb, stage = tok * 128 + 2 * 128 * 128, ring = (3 * stage <= 160 * 1024 ? 3 : 2) * stage;
+    const int tok = 32 * tb, ring = gt_lds_bytes(tb);
     const int epi = PD * PD * 2 + 2 * tok * XROW + 2 * 4 * tok * 4;
     return epi > ring ? epi : ring;
 }
