@@ -273,11 +273,41 @@ __global__ __launch_bounds__(256, 3) void apq_gemm_mid_kernel(AttnPreArgs a, int
     }
 }
 
-// The projection at prefill sizes and larger decode batches (attention_pre_kernel): a workgroup owns 32 TB tokens x 256 outputs - two heads - over one
-// split of the contraction (gemm_tile.h; an odd last head is taken twice and dropped).  An XCD takes neighbouring heads.  Where one split covers the whole contraction the head's epilogue runs on the
-// tile: the sums never go to memory (777 tokens x 112 heads: 45 MB written and read again, and a kernel of 87 K small
-// workgroups).  Same operations in the same order as apq_head_kernel, so the same bits: its sum over the 128 squares is a
-// butterfly over dims 32, 16, .. 1 apart, which here are register, lane and register exchanges.
+// the upper or the lower bf16 of a register
+__device__ __forceinline__ float half_of(uint32_t v, int upper)
+{
+    return __builtin_bit_cast(float, upper ? v & 0xffff0000u : v << 16);
+}
+// a over lanes l and l + 32 in the lower half, b in the upper; of rows of 16 lanes: a over rows 0 and 1, b, a over rows 2 and 3, b
+__device__ __forceinline__ float add_halves32(float a, float b)
+{
+    const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    return __builtin_bit_cast(float, (unsigned)sw[0]) + __builtin_bit_cast(float, (unsigned)sw[1]);
+}
+__device__ __forceinline__ float add_rows16(float a, float b)
+{
+    const auto sw = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    return __builtin_bit_cast(float, (unsigned)sw[0]) + __builtin_bit_cast(float, (unsigned)sw[1]);
+}
+
+// The projection at prefill sizes and larger decode batches (attention_pre_kernel): a workgroup owns 32 TB tokens x 256 outputs -
+// two heads - over one split of the contraction (gemm_tile.h; an odd last head is taken twice and dropped).  An XCD takes
+// neighbouring heads.  Where one split covers the whole contraction the head's epilogue runs on the tile: the sums never go to
+// memory (777 tokens x 112 heads: 45 MB written and read again, and a kernel of 87 K small workgroups).  Same operations in the
+// same order as apq_head_kernel, so the same bits: its sum over the 128 squares is a butterfly over dims 32, 16, .. 1 apart, which
+// here are register, lane and register exchanges.
+//
+// All tiles reach the epilogue together, so nothing covers it; it is bound by its vector instructions, 14336 to 32768 elements to a
+// SIMD.  At 224 tokens it took 38 K ticks beside the product's 99 K, of which a division per element and sums exchanged through
+// LDS 21 K, rotary pairs from an LDS tile with their cos and sin two loads at a time 15 K; now 20 K:
+//  - a quotient is two fused multiply-adds on the product with the reciprocal, which for a bf16 dividend gives the rounded
+//    quotient for every pair of mantissas (all 2^30 compared).  It needs that no step under- or overflows: positive scales of
+//    2^-60 to 2^60 (a value is 0 or a scale times 1 to 2^32) and divisors of 2^-20 to 2^100, or the wave divides;
+//  - pairs of rotary dims 16 or 32 apart are registers of one lane, whose cos and sin are loaded before the sums.  The half of a
+//    head that has none belongs to every second wave: the two waves of a SIMD get one of each (gt_wave_across);
+//  - each wave turns 16 tokens x 64 dims at a time into rows through LDS of its own and stores them while it goes on.
+// (777 tokens x 112 heads 82.4 -> 75.0 us a call, 1024 tokens 95.9 -> 88.9.)
+// Other rotary widths have pairs in two waves or in broken pieces: the tile goes through LDS.
 // grid (heads / 2 rounded up, splits, token tiles), 512 lanes.
 template <int TB, bool WHOLE>
 __global__ __launch_bounds__(GT_LANES, 2) void apq_gemm_big_kernel(AttnPreArgs a, int per)
@@ -287,7 +317,7 @@ __global__ __launch_bounds__(GT_LANES, 2) void apq_gemm_big_kernel(AttnPreArgs a
     constexpr int OROW = AD * 2 + 16; // bytes per LDS row of a head's bf16 output tile (padded against bank conflicts)
     constexpr int EPI = 2 * T::TOK * OROW + 4 * T::TOK * 4; // two heads' output tiles, sums of squares of [wc][tokens]
     __shared__ __align__(16) uint8_t lds[WHOLE && EPI > T::LDS ? EPI : T::LDS];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = gt_wave_across();
     const int l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
     const int tile = gridDim.x % 8 == 0 ? (int)(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8) : (int)blockIdx.x;
     const int heads = a.q_heads + 2 * a.kv_heads, head0 = 2 * tile, head = head0 + (wc >> 1); // of the tile, of this wave
@@ -300,7 +330,7 @@ __global__ __launch_bounds__(GT_LANES, 2) void apq_gemm_big_kernel(AttnPreArgs a
         for (int tb = 0; tb < TB; ++tb) acc[db][tb] = i32x4{0, 0, 0, 0};
     const int8_t* w = a.w + (int64_t)st0 * GT_KI8 * a.n_out;
     gt_product_i8<TB>(acc, w + head0 * AD, w + min(head0 + 1, heads - 1) * AD, a.n_out, a.x_q + (int64_t)st0 * GT_KI8, a.h, tok0, a.t,
-                      stages, lds);
+                      stages, lds, wave);
     const bool live = head < heads;
     const int hw = 64 * (wc & 1), col0 = min(head, heads - 1) * AD; // this wave's half of its head; the head's columns
     // register e of acc[db][tb]: dim hw + 16 db + 4 g + e of the head, token 16 TB wr + 16 tb + l16
@@ -319,18 +349,45 @@ __global__ __launch_bounds__(GT_LANES, 2) void apq_gemm_big_kernel(AttnPreArgs a
     const bool is_q = head < a.q_heads, is_v = head >= a.q_heads + a.kv_heads; // uniform over the wave
     const uint16_t* gp = is_q ? a.q_gamma : a.k_gamma;
     const uint16_t* bp = is_q ? a.q_bias : a.k_bias;
-    float y[4][TB][4]; // [db][tb][e]
+    uint32_t y[4][TB][2]; // [db][tb][e / 2], bf16
+    float least = HUGE_VALF, most = 0.f; // of the scales
 #pragma unroll
     for (int db = 0; db < 4; ++db) {
         const int dim = hw + 16 * db + 4 * g;
         const f32x4 deq = *reinterpret_cast<const f32x4*>(a.deq + col0 + dim);
         const i32x4 qb = *reinterpret_cast<const i32x4*>(a.qbias + col0 + dim);
+        least = fminf(fminf(least, deq[0]), fminf(deq[1], fminf(deq[2], deq[3])));
+        most = fmaxf(fmaxf(most, deq[0]), fmaxf(deq[1], fmaxf(deq[2], deq[3])));
 #pragma unroll
         for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) y[db][tb][e] = round_bf16((float)(acc[db][tb][e] + qb[e]) * deq[e]);
+            for (int e = 0; e < 4; e += 2)
+                y[db][tb][e / 2] = pack_bf16x2((float)(acc[db][tb][e] + qb[e]) * deq[e], (float)(acc[db][tb][e + 1] + qb[e + 1]) * deq[e + 1]);
     }
+    __builtin_amdgcn_sched_barrier(0); // (the loads below once the sums' registers are free)
+    const bool here = hw == 0 && !is_v && (a.half == 16 || a.half == 32); // rotary pairs of this wave, in one lane each
+    u32x2 cosr[TB][2], sinr[TB][2], gr[4], br[4];
     if (!is_v) {
+#pragma unroll
+        for (int db = 0; db < 4; ++db) {
+            gr[db] = *reinterpret_cast<const u32x2*>(gp + hw + 16 * db + 4 * g);
+            br[db] = *reinterpret_cast<const u32x2*>(bp + hw + 16 * db + 4 * g);
+        }
+        if (here) {
+            const uint16_t* cp = a.cos + (int64_t)tok0 * a.half;
+            const uint16_t* sp = a.sin + (int64_t)tok0 * a.half;
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) { // (16 dims: the same ones twice)
+                    const uint32_t at = min(16 * TB * wr + 16 * tb + l16, a.t - 1 - tok0) * a.half + (16 * i & (a.half - 1)) + 4 * g;
+                    cosr[tb][i] = *reinterpret_cast<const u32x2*>(cp + at);
+                    sinr[tb][i] = *reinterpret_cast<const u32x2*>(sp + at);
+                }
+        }
+        // sums of squares: over dims 32, 16 (registers), 8, 4 (16-lane rows), 2, 1 (registers) apart.  An exchange adds up two
+        // values at once, one to either half of the lanes, then to every other row: the four values of e, then four token blocks
+        float s[(TB + 3) / 4 * 4];
 #pragma unroll
         for (int tb = 0; tb < TB; ++tb) {
             float m[4];
@@ -338,40 +395,122 @@ __global__ __launch_bounds__(GT_LANES, 2) void apq_gemm_big_kernel(AttnPreArgs a
             for (int e = 0; e < 4; ++e) {
                 float sq[4];
 #pragma unroll
-                for (int db = 0; db < 4; ++db) sq[db] = (y[db][tb][e] * y[db][tb][e]) * (1.0f / AD);
-                m[e] = (sq[0] + sq[2]) + (sq[1] + sq[3]); // dims 32, then 16 apart
-                m[e] += __shfl_xor(m[e], 32, 64);         // 8
-                m[e] += __shfl_xor(m[e], 16, 64);         // 4
+                for (int db = 0; db < 4; ++db) {
+                    const float v = half_of(y[db][tb][e >> 1], e & 1);
+                    sq[db] = (v * v) * (1.0f / AD);
+                }
+                m[e] = (sq[0] + sq[2]) + (sq[1] + sq[3]);
             }
-            const float s = (m[0] + m[2]) + (m[1] + m[3]); // 2, 1
-            if (g == 0) sums[wc * T::TOK + 16 * TB * wr + 16 * tb + l16] = s;
+            s[tb] = add_rows16(add_halves32(m[0], m[2]), add_halves32(m[1], m[3])); // in row e the sum for e
+        }
+#pragma unroll
+        for (int tb = TB; tb < (int)(sizeof(s) / sizeof(float)); ++tb) s[tb] = s[TB - 1];
+#pragma unroll
+        for (int tb = 0; tb < TB; tb += 4) {
+            const float sum = add_rows16(add_halves32(s[tb], s[tb + 1]), add_halves32(s[tb + 2], s[tb + 3]));
+            const int mine = min(tb + ((g & 1) << 1 | g >> 1), TB - 1); // rows 0, 1, 2, 3: blocks 0, 2, 1, 3
+            sums[wc * T::TOK + 16 * TB * wr + 16 * mine + l16] = sum;
         }
     }
     __syncthreads();
     if (!is_v) {
+        float denom[TB];
+        bool plain = least >= 0x1p-60f && most <= 0x1p60f;
 #pragma unroll
         for (int tb = 0; tb < TB; ++tb) {
             const int tl = 16 * TB * wr + 16 * tb + l16;
-            const float denom = sqrtf((sums[(wc & 2) * T::TOK + tl] + sums[(wc | 1) * T::TOK + tl]) + a.eps);
+            denom[tb] = sqrtf((sums[(wc & 2) * T::TOK + tl] + sums[(wc | 1) * T::TOK + tl]) + a.eps);
+            plain = plain && denom[tb] >= 0x1p-20f && denom[tb] <= 0x1p100f;
+        }
+        auto norm = [&](auto quotient) {
 #pragma unroll
-            for (int db = 0; db < 4; ++db) {
-                const int dim = hw + 16 * db + 4 * g;
-                const u32x2 gr = *reinterpret_cast<const u32x2*>(gp + dim), br = *reinterpret_cast<const u32x2*>(bp + dim);
+            for (int tb = 0; tb < TB; ++tb) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int sh = (e & 1) * 16;
-                    y[db][tb][e] = (y[db][tb][e] / denom) * bf16_bits_to_f32((gr[e >> 1] >> sh) & 0xffffu) +
-                                   bf16_bits_to_f32((br[e >> 1] >> sh) & 0xffffu);
+                for (int db = 0; db < 4; ++db) // (taken apart anew, not kept in fp32 since the sums)
+                    asm("" : "+v"(y[db][tb][0]), "+v"(y[db][tb][1]));
+                const float r = 1.0f / denom[tb];
+#pragma unroll
+                for (int db = 0; db < 4; ++db)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        float x[2];
+#pragma unroll
+                        for (int e = 0; e < 2; ++e)
+                            x[e] = quotient(half_of(y[db][tb][i], e), denom[tb], r) * half_of(gr[db][i], e) + half_of(br[db][i], e);
+                        y[db][tb][i] = pack_bf16x2(x[0], x[1]);
+                    }
+            }
+        };
+        if (__all(plain))
+            norm([](float x, float d, float r) {
+                const float q = x * r;
+                return __builtin_fmaf(__builtin_fmaf(-q, d, x), r, q);
+            });
+        else
+            norm([](float x, float d, float) { return x / d; });
+    }
+    if (a.half == 16 || a.half == 32) {
+        auto rotate = [&](auto first, auto second, int tb, int j) { // blocks of 16 dims that hold a pair's dims
+            uint32_t(&lo)[2] = y[decltype(first)::value][tb];
+            uint32_t(&hi)[2] = y[decltype(second)::value][tb];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                float r[2][2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const float x1 = half_of(lo[i], e), x2 = half_of(hi[i], e), c = half_of(cosr[tb][j][i], e), sn = half_of(sinr[tb][j][i], e);
+                    r[0][e] = x1 * c - x2 * sn;
+                    r[1][e] = x2 * c + x1 * sn;
                 }
+                lo[i] = pack_bf16x2(r[0][0], r[0][1]);
+                hi[i] = pack_bf16x2(r[1][0], r[1][1]);
+            }
+        };
+        using std::integral_constant;
+        constexpr integral_constant<int, 0> b0{};
+        constexpr integral_constant<int, 1> b1{};
+        constexpr integral_constant<int, 2> b2{};
+        constexpr integral_constant<int, 3> b3{};
+        if (here) {
+            if (a.half == 32) {
+#pragma unroll
+                for (int tb = 0; tb < TB; ++tb) rotate(b0, b2, tb, 0), rotate(b1, b3, tb, 1);
+            } else {
+#pragma unroll
+                for (int tb = 0; tb < TB; ++tb) rotate(b0, b1, tb, 0);
             }
         }
+        // 16 tokens x 64 dims at a time to where the wave alone reads them back as pieces of 16 bytes
+        constexpr int WROW = 128 + 16;
+        uint8_t* own = lds + wave * (2 * 16 * WROW);
+        static_assert(8 * 2 * 16 * WROW <= 2 * T::TOK * OROW, "the sums lie behind");
+        uint16_t* dst = is_v ? a.v + (int64_t)(head - a.q_heads - a.kv_heads) * AD
+                             : is_q ? a.q + (int64_t)head * AD
+                                    : a.k + (int64_t)(head - a.q_heads) * AD;
+        const int64_t pitch = (int64_t)(is_q ? a.q_heads : a.kv_heads) * AD;
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {
+            uint8_t* at = own + (tb & 1) * (16 * WROW);
+#pragma unroll
+            for (int db = 0; db < 4; ++db)
+                *reinterpret_cast<u32x2*>(at + l16 * WROW + 32 * db + 8 * g) = u32x2{y[db][tb][0], y[db][tb][1]};
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int row = 8 * i + (lane >> 3), tok = tok0 + 16 * TB * wr + 16 * tb + row;
+                const u32x4 o = *reinterpret_cast<const u32x4*>(at + row * WROW + 16 * (lane & 7));
+                if (tok < a.t && live) *reinterpret_cast<u32x4*>(dst + (int64_t)tok * pitch + hw + 8 * (lane & 7)) = o;
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        return;
     }
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
         for (int db = 0; db < 4; ++db)
             *reinterpret_cast<u32x2*>(lds + ((wc >> 1) * T::TOK + 16 * TB * wr + 16 * tb + l16) * OROW + (hw + 16 * db + 4 * g) * 2) =
-                u32x2{pack_bf16x2(y[db][tb][0], y[db][tb][1]), pack_bf16x2(y[db][tb][2], y[db][tb][3])};
+                u32x2{y[db][tb][0], y[db][tb][1]};
     __syncthreads();
     // tokens x 16 pieces of 8 dims, a head to four waves; a piece's rotary partners are half dims further on or back
     const int ohead = head0 + (tid >> 8), otid = tid & 255;

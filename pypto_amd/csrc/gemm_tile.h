@@ -124,15 +124,24 @@ __device__ __forceinline__ void gt_tile_stages(int stages, CopyQ&& copy_q, CopyW
     gt_landed<0>();
 }
 
-// acc[nb][tb] += w[k, col0 + ..]^T . q[token, k], int8.  w0, w1: first contraction row of the two halves' columns, ldw bytes a
+// Waves by their number; and with the column blocks of the second token half exchanged in pairs, so that the two waves of a SIMD
+// (numbers four apart) have an even and an odd one, for epilogues that give these different work.
+__device__ __forceinline__ int gt_wave() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+__device__ __forceinline__ int gt_wave_across()
+{
+    const int wave = gt_wave();
+    return wave ^ (wave >> 2);
+}
+
+// acc[nb][tb] += w[k, col0 + ..]^T . q[token, k], int8, by wave 4 wr + wc.  w0, w1: first contraction row of the two halves' columns, ldw bytes a
 // row; q: [t, ldq], column of the first contraction row.  Register e of acc[nb][tb]: output 64 wc + 16 nb + 4 g + e, token
 // 16 TB wr + 16 tb + l16.
 template <int TB>
 __device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t* w0, const int8_t* w1, int64_t ldw, const int8_t* q,
-                                              int64_t ldq, int tok0, int t, int stages, uint8_t* lds)
+                                              int64_t ldq, int tok0, int t, int stages, uint8_t* lds, int wave)
 {
     using T = GtTile<TB>;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
     const int l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
     // copy i of a wave: rows 64 i + 8 wave + lane / 8 of either operand
     const int row = 8 * wave + (lane >> 3), pos = lane & 7;

@@ -868,7 +868,8 @@ __device__ __forceinline__ void mla_qb_wide_body(const MlaPrologArgs& a, int til
 #pragma unroll
         for (int tb = 0; tb < TB; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
     const int8_t* w = static_cast<const int8_t*>(a.w_uq_qr);
-    gt_product_i8<TB>(acc, w + col0, w + min(col0 + 128, nq - 128), nq, a.q_norm, a.r, tok0, a.t, a.r / GT_KI8, lds);
+    gt_product_i8<TB>(acc, w + col0, w + min(col0 + 128, nq - 128), nq, a.q_norm, a.r, tok0, a.t, a.r / GT_KI8, lds,
+                      gt_wave());
     // register e of acc[nb][tb]: output 64 wc + 16 nb + 4 g + e, token 16 TB wr + 16 tb + l16
     f32x4 ws[4];
 #pragma unroll

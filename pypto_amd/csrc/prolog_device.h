@@ -434,7 +434,8 @@ __device__ __forceinline__ void prolog_q_wide_body(const PrologArgs& a, int head
     for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
         for (int tb = 0; tb < TB; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
-    gt_product_i8<TB>(acc, a.w_qb + head0 * PD, a.w_qb + min(head0 + 1, a.n - 1) * PD, nd, a.q_norm, a.r, tok0, a.t, a.r / GT_KI8, lds);
+    gt_product_i8<TB>(acc, a.w_qb + head0 * PD, a.w_qb + min(head0 + 1, a.n - 1) * PD, nd, a.q_norm, a.r, tok0, a.t, a.r / GT_KI8, lds,
+                      gt_wave());
     uint8_t* had = lds;
 #pragma unroll
     for (int i = 0; i < PD * PD * 2 / 16 / 512; ++i) reinterpret_cast<u32x4*>(had)[tid + 512 * i] = reinterpret_cast<const u32x4*>(a.had_q)[tid + 512 * i];

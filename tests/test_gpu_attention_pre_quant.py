@@ -173,6 +173,32 @@ def test_projection_kernels_at_the_edges_of_their_ranges(cuda, t, h, q_heads, kv
     check(case, run(case, cuda))
 
 
+@pytest.mark.parametrize("t,q_heads,kv_heads,half,scales", [
+    (1300, 48, 2, 16, "plain"), (1500, 48, 2, 32, "least"), (1800, 48, 2, 16, "signs"), (2100, 47, 2, 32, "zeros"), (1025, 47, 2, 16, "below"),
+    (1300, 48, 2, 32, "most"), (1301, 48, 2, 64, "below"), (1499, 48, 2, 8, "above")])
+def test_heads_finished_on_the_tiles_have_the_bits_of_the_head_kernel(cuda, t, q_heads, kv_heads, half, scales):
+    """Tiles in one split against the streamed kernel with its head kernel, bit by bit, on the first and the last tokens and around the
+    tiles' borders: pairs of rotary dims inside a wave's tile (16 and 32 a half) and across, scales at both ends of the range in
+    which a quotient is taken by the reciprocal (2^-60 to 2^60), beyond it, negative and zero."""
+    case = op.make_case(t, h=256, q_heads=q_heads, kv_heads=kv_heads, half=half, seed=70 + t)
+    deq = case["atten_qkv_deq_scale"]
+    n = deq.numel()
+    if scales == "signs":
+        deq[torch.arange(n) % 5 == 0] *= -1
+    elif scales == "zeros":
+        deq[torch.arange(n) % 3 == 0] = 0
+        deq[:128] = 0
+    elif scales != "plain":
+        deq[torch.arange(n) % 7 == 0] = {"least": 2.0 ** -60, "below": 2.0 ** -75, "most": 2.0 ** 60, "above": 2.0 ** 61}[scales]
+    full = run(case, cuda)
+    rows = ("hidden_states", "residual", "cos", "sin")
+    for t0 in (0, 124, 188, 252, t - 8):
+        got = run({k: v[t0:t0 + 8].contiguous() if k in rows else v for k, v in case.items()}, cuda)
+        for name in ("query", "key", "value"):
+            assert torch.isfinite(got[name]).all()
+            assert torch.equal(got[name], full[name][t0:t0 + 8]), (t0, name)
+
+
 def test_a_tokens_bits_do_not_depend_on_the_projection_kernel(cuda):
     # int32 sums are exact and the head epilogues the same operations: streamed, 128 x 128 and wide tiles in one and in several splits
     case = op.make_case(300, h=1024, seed=3)

@@ -153,3 +153,21 @@ def test_reference_test_distribution_runs():
     assert out["query"].shape == (8, 1536) and out["key"].shape == (8, 128)
     for k in ("query", "key", "value", "residual_res"):
         assert torch.isfinite(out[k].float()).all()
+
+
+def test_quotient_of_a_bf16_by_its_reciprocal_is_the_rounded_quotient():
+    """What the projection's tiles compute in place of x / d where nothing under- or overflows: with r = fp32(1 / d) and q = fp32(x r),
+    q + (x - q d) r by two fused multiply-adds is fp32(x / d) for every bf16 x.  Both sides scale with powers of two, so the
+    mantissas are all there is: 128 of x, and of the 2^23 of d (all agree) every 61st and those at both ends.  fp64 holds the
+    products of the fused operations exactly; the sum of the second is rounded to odd there, and then to fp32."""
+    m = np.unique(np.concatenate([np.arange(0, 1 << 23, 61), np.arange(4096), (1 << 23) - 1 - np.arange(4096)]))
+    d = (1 + m / 2.0 ** 23).astype(np.float32)
+    r = np.float32(1) / d
+    for x in (1 + np.arange(128) / 128).astype(np.float32):
+        q = (x * r).astype(np.float64)
+        p = (np.float64(x) - q * d).astype(np.float32) * r.astype(np.float64)
+        s = q + p
+        err = p - (s - q)  # exact: |p| < |q|
+        even = (s.view(np.int64) & 1) == 0
+        s = np.where((err != 0) & even, np.nextafter(s, np.where(err > 0, np.inf, -np.inf)), s)
+        assert (s.astype(np.float32) == x / d).all(), x
