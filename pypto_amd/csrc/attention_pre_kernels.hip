@@ -273,11 +273,6 @@ __global__ __launch_bounds__(256, 3) void apq_gemm_mid_kernel(AttnPreArgs a, int
     }
 }
 
-// the upper or the lower bf16 of a register
-__device__ __forceinline__ float half_of(uint32_t v, int upper)
-{
-    return __builtin_bit_cast(float, upper ? v & 0xffff0000u : v << 16);
-}
 // a over lanes l and l + 32 in the lower half, b in the upper; of rows of 16 lanes: a over rows 0 and 1, b, a over rows 2 and 3, b
 __device__ __forceinline__ float add_halves32(float a, float b)
 {

@@ -26,6 +26,11 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t v) { return __builtin_bit_
 __device__ __forceinline__ float quant_scale(float mx) { return (1.0f / mx) * 127.0f; }
 __device__ __forceinline__ uint16_t f32_to_bf16(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 __device__ __forceinline__ float round_bf16(float f) { return bf16_to_f32(f32_to_bf16(f)); }
+// the upper or the lower bf16 of a register
+__device__ __forceinline__ float half_of(uint32_t v, int upper)
+{
+    return __builtin_bit_cast(float, upper ? v & 0xffff0000u : v << 16);
+}
 
 
 } // namespace

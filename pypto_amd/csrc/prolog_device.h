@@ -13,7 +13,7 @@ constexpr int PD = 128;      // index head dim
 constexpr int PROPE = 64;    // rotary dims
 constexpr int PTOK = 32;     // tokens per workgroup tile
 constexpr int XW_K = 256;    // contraction rows per workgroup of the x @ [w_k | w_proj] product
-constexpr int XROW = PD * 2 + 16; // bytes per LDS row of the 32 x 128 bf16 tile (padded)
+constexpr int XROW = PD * 2 + 8; // bytes per LDS row of the 32 x 128 bf16 tile (padded: 32 rows two banks apart)
 constexpr int QK = 128;      // contraction rows per stage of prolog_q_kernel
 constexpr int QROW = 136;    // bytes per LDS row of a [k][128] int8 weight stage (padded, 8-byte aligned)
 constexpr int QGROUPS = 4;   // wave groups of prolog_q_kernel, each with its own stages
@@ -72,18 +72,26 @@ __device__ __forceinline__ void prolog_q_quantise(const PrologArgs& a, int head,
         const int jj = lane & 15, mh = (lane >> 4) & 1;
         const uint8_t* hp = had + (4 * hl + (jj >> 2)) * (PD * 2) + (32 * hwave + 16 * mh + 4 * (jj & 3)) * 2;
         const uint8_t* xp = xt + l32 * XROW + hl * 8;
-#pragma unroll
-        for (int ks = 0; ks < PD / 16; ++ks) {
+        bf16x8 av[2], bv[2][TB]; // a step's operands are read while the step before is multiplied
+        auto read = [&](int ks) {
             const s16x4 lo = lds_read_tr(hp + ks * 16 * (PD * 2));
             const s16x4 hi = lds_read_tr(hp + (ks * 16 + 8) * (PD * 2));
-            const bf16x8 av = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            av[ks & 1] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
             for (int tb = 0; tb < TB; ++tb) {
                 const u32x2 b0 = *reinterpret_cast<const u32x2*>(xp + 32 * tb * XROW + ks * 32);
                 const u32x2 b1 = *reinterpret_cast<const u32x2*>(xp + 32 * tb * XROW + ks * 32 + 16);
-                const bf16x8 bv = __builtin_bit_cast(bf16x8, u32x4{b0[0], b0[1], b1[0], b1[1]});
-                y[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, y[tb], 0, 0, 0);
+                bv[ks & 1][tb] = __builtin_bit_cast(bf16x8, u32x4{b0[0], b0[1], b1[0], b1[1]});
             }
+        };
+        read(0);
+#pragma unroll
+        for (int ks = 0; ks < PD / 16; ++ks) {
+            if (ks + 1 < PD / 16) read(ks + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb) y[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[ks & 1], bv[ks & 1][tb], y[tb], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
     // register e of y[tb]: n = 32 w + 8 (e/4) + 4 hl + e%4, token 32 tb + l32.  Round to bf16, per-token absmax over the 128 n
@@ -106,15 +114,20 @@ __device__ __forceinline__ void prolog_q_quantise(const PrologArgs& a, int head,
         const float m = fmaxf(fmaxf(smax[0][tl], smax[1][tl]), fmaxf(smax[2][tl], smax[3][tl]));
         const float sq = quant_scale(m);
         const int gt = tok0 + tl;
+        // pieces of 4 dims, 8 apart; with the other lane half's: 16 dims in a row to a lane, one store
+        uint32_t pk[4];
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4) {
+            uint32_t r[4]; // at most 127: behind 1.5 * 2^23 the low byte is the value rounded to even (0 of a NaN)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[e] = __builtin_bit_cast(uint32_t, y[tb][4 * e4 + e] * sq + 12582912.f);
+            pk[e4] = __builtin_amdgcn_perm(r[1], r[0], 0x0c0c0400u) | __builtin_amdgcn_perm(r[3], r[2], 0x04000c0cu);
+        }
+        const auto even = __builtin_amdgcn_permlane32_swap(pk[0], pk[2], false, false);
+        const auto odd = __builtin_amdgcn_permlane32_swap(pk[1], pk[3], false, false);
         if (gt < a.t && head < a.n) {
-            int8_t* qo = a.q_int8 + ((int64_t)gt * a.n + head) * PD + 32 * hwave + 4 * hl;
-#pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) {
-                uint32_t pk = 0;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(y[tb][4 * e4 + e] * sq) & 0xffu) << (8 * e);
-                *reinterpret_cast<uint32_t*>(qo + 8 * e4) = pk;
-            }
+            *reinterpret_cast<u32x4*>(a.q_int8 + ((int64_t)gt * a.n + head) * PD + 32 * hwave + 16 * hl) =
+                u32x4{(unsigned)even[0], (unsigned)even[1], (unsigned)odd[0], (unsigned)odd[1]};
             if (hwave == 0 && hl == 0) a.q_scale[(int64_t)gt * a.n + head] = __builtin_bit_cast(uint16_t, (_Float16)(1.0f / sq));
         }
     }
@@ -411,9 +424,27 @@ __device__ __forceinline__ void prolog_q_big_body(const PrologArgs& a, int head,
     prolog_q_finish<QB_TOK / 32>(a, head, tok0, tid, had, xt, smax);
 }
 
+// 4 x 4 pieces of 8 bytes, [row of 16 lanes][register]: out[j] of row g = x[g] of row j
+__device__ __forceinline__ void transpose_rows(uint32_t (&out)[4][2], const u32x4 (&x)[2])
+{
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const auto a = __builtin_amdgcn_permlane32_swap(x[0][i], x[1][i], false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(x[0][2 + i], x[1][2 + i], false, false);
+        const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)a[0], (unsigned)b[0], false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)a[1], (unsigned)b[1], false, false);
+        out[0][i] = lo[0], out[1][i] = lo[1], out[2][i] = hi[0], out[3][i] = hi[1];
+    }
+}
+
 // Above 256 tokens: 32 TB tokens x two heads per workgroup (gemm_tile.h), four waves to a head behind the product; the
 // operations are prolog_q_big_body's, so are the bits (51 us at 1501 tokens there).  512 lanes; an odd last head is taken twice
 // and dropped.
+// Nothing covers what follows the product, which at 192 tokens x 1536 rows took 33 K ticks beside the product's 30 K: rotary pairs
+// out of LDS, cos and sin loaded in single elements; pairs of LDS rows in the same banks in front of the Hadamard product; four
+// stores of 4 bytes a lane.  Now 22 K: pairs are rotated where they are, in registers of a lane, by one wave of each SIMD
+// (gt_wave_across), cos and sin loaded 16 bytes at a time (loads of 8 cost the memory pipe twice as much, 13 K ticks in all, not 8);
+// rows two banks apart; one store of 16 bytes.  Call of 1501 tokens 239.6 -> 232.9 us, 300: 80.7 -> 76.5.
 constexpr int prolog_q_wide_lds(int tb) // the product's stages, or hadamard_q | [2] bf16 tiles | [2] per-wave maxima
 {
     const int tok = 32 * tb, ring = gt_lds_bytes(tb);
@@ -426,7 +457,7 @@ __device__ __forceinline__ void prolog_q_wide_body(const PrologArgs& a, int head
 #pragma clang fp contract(off)
     constexpr int TOK = 32 * TB;
     static_assert(prolog_q_wide_lds(TB) <= 160 * 1024 && prolog_q_wide_lds(TB) >= GtTile<TB>::LDS, "LDS");
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = gt_wave_across();
     const int l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
     const int64_t nd = (int64_t)a.n * PD;
     i32x4 acc[4][TB]; // [nb][tb]
@@ -435,36 +466,79 @@ __device__ __forceinline__ void prolog_q_wide_body(const PrologArgs& a, int head
 #pragma unroll
         for (int tb = 0; tb < TB; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
     gt_product_i8<TB>(acc, a.w_qb + head0 * PD, a.w_qb + min(head0 + 1, a.n - 1) * PD, nd, a.q_norm, a.r, tok0, a.t, a.r / GT_KI8, lds,
-                      gt_wave());
-    uint8_t* had = lds;
+                      wave);
+    u32x4 hadr[PD * PD * 2 / 16 / 512];
 #pragma unroll
-    for (int i = 0; i < PD * PD * 2 / 16 / 512; ++i) reinterpret_cast<u32x4*>(had)[tid + 512 * i] = reinterpret_cast<const u32x4*>(a.had_q)[tid + 512 * i];
+    for (int i = 0; i < PD * PD * 2 / 16 / 512; ++i) hadr[i] = reinterpret_cast<const u32x4*>(a.had_q)[tid + 512 * i];
     // register e of acc[nb][tb]: dim 64 (wc & 1) + 16 nb + 4 g + e of head wc / 2, token 16 TB wr + 16 tb + l16
+    const int hw = 64 * (wc & 1);
+    uint32_t y[4][TB][2]; // bf16
     {
-        uint8_t* xt = lds + PD * PD * 2 + (wc >> 1) * TOK * XROW;
         f32x4 ws[4];
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb)
-            ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + (int64_t)min(head0 + (wc >> 1), a.n - 1) * PD + 64 * (wc & 1) + 16 * nb + 4 * g);
+            ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + (int64_t)min(head0 + (wc >> 1), a.n - 1) * PD + hw + 16 * nb + 4 * g);
 #pragma unroll
         for (int tb = 0; tb < TB; ++tb) {
-            const int tl = 16 * TB * wr + 16 * tb + l16;
-            const float qs = a.q_norm_scale[min(tok0 + tl, a.t - 1)];
+            const float qs = a.q_norm_scale[min(tok0 + 16 * TB * wr + 16 * tb + l16, a.t - 1)];
 #pragma unroll
             for (int nb = 0; nb < 4; ++nb) {
                 float v[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs) * ws[nb][e];
-                *reinterpret_cast<u32x2*>(xt + tl * XROW + (64 * (wc & 1) + 16 * nb + 4 * g) * 2) =
-                    u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+                y[nb][tb][0] = pack_bf16x2(v[0], v[1]);
+                y[nb][tb][1] = pack_bf16x2(v[2], v[3]);
             }
         }
     }
+    __builtin_amdgcn_sched_barrier(0); // (the loads below once the sums' registers are free)
+    if (hw == 0) { // rotary pairs are 32 dims apart: registers of a lane
+        const uint16_t* cp = a.cos + (int64_t)tok0 * PROPE;
+        const uint16_t* sp = a.sin + (int64_t)tok0 * PROPE;
+        // a lane loads dims 16 g .. 16 g + 15 of its token, four pieces of 4, and gets its pieces 16 nb + 4 g by exchange of rows
+        u32x4 cr[TB][2], sr[TB][2];
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const uint32_t at = min(16 * TB * wr + 16 * tb + l16, a.t - 1 - tok0) * PROPE + 16 * g + 8 * i;
+                cr[tb][i] = *reinterpret_cast<const u32x4*>(cp + at);
+                sr[tb][i] = *reinterpret_cast<const u32x4*>(sp + at);
+            }
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {
+            uint32_t c[4][2], sn[4][2];
+            transpose_rows(c, cr[tb]);
+            transpose_rows(sn, sr[tb]);
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    float o[2][2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) { // (the arithmetic of rope_tile)
+                        const float x1 = half_of(y[nb][tb][i], e), x2 = half_of(y[nb + 2][tb][i], e);
+                        o[0][e] = x1 * half_of(c[nb][i], e) + (-x2) * half_of(sn[nb][i], e);
+                        o[1][e] = x2 * half_of(c[nb + 2][i], e) + x1 * half_of(sn[nb + 2][i], e);
+                    }
+                    y[nb][tb][i] = pack_bf16x2(o[0][0], o[0][1]);
+                    y[nb + 2][tb][i] = pack_bf16x2(o[1][0], o[1][1]);
+                }
+        }
+    }
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb)
+            *reinterpret_cast<u32x2*>(lds + PD * PD * 2 + ((wc >> 1) * TOK + 16 * TB * wr + 16 * tb + l16) * XROW + (hw + 16 * nb + 4 * g) * 2) =
+                u32x2{y[nb][tb][0], y[nb][tb][1]};
+#pragma unroll
+    for (int i = 0; i < PD * PD * 2 / 16 / 512; ++i) reinterpret_cast<u32x4*>(lds)[tid + 512 * i] = hadr[i];
     __syncthreads();
     const int hs = tid >> 8, ht = tid & 255, head = head0 + hs; // from here on four waves to a head
     uint8_t* xt = lds + PD * PD * 2 + hs * TOK * XROW;
     float(*smax)[TOK] = reinterpret_cast<float(*)[TOK]>(lds + PD * PD * 2 + 2 * TOK * XROW + hs * 4 * TOK * 4);
-    prolog_q_finish<TB>(a, head, tok0, ht, lds, xt, smax);
+    prolog_q_quantise<TB>(a, head, tok0, ht, lds, xt, smax);
 }
 
 // Up to 32 tokens: one head per workgroup of 256 lanes behind the streamed product; the bits of prolog_q_body.
