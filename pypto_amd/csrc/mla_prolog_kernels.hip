@@ -952,17 +952,24 @@ constexpr int FUSED_T = 2048;
 // Above 256 tokens the two products in one launch of gemm_tile.h's tiles where that takes no more rounds of workgroups: the index
 // heads' part alone is half a round up to 512 tokens (call of 257 tokens 94 -> 80 us, 512: 124 -> 104).  Its tiles are up to
 // 224 tokens; where the query product's own of 256 save a round, and a round counts, the two are launches of their own (1024
-// tokens: 191 us in one, 184 in two, 1200: 219 / 208, 2048: the same, 4096: 680 / 691).  grid (index heads / 2 rounded up + n * 192 / 256 rounded up, token tiles), 512 lanes
+// tokens: 191 us in one, 184 in two, 1200: 219 / 208, 2048: the same, 4096: 680 / 691).
+// The index heads' tiles take the longer, 26 us at 192 tokens against 19, and come first, those of all tokens: as columns of each
+// token tile they began again in the last round of workgroups (104 us for the kernel at 1501 tokens,
+// 92 so; the call 240.8 -> 236.8, no difference where the rounds come out even).
+// grid ((index heads / 2 rounded up + n * 192 / 256 rounded up) x token tiles), 512 lanes
 template <int TB>
 __global__ __launch_bounds__(GT_LANES, 2) void fused_qb_wide_kernel(MlaPrologArgs m, PrologArgs p)
 {
     constexpr int A = mla_qb_wide_lds(TB), B = prolog_q_wide_lds(TB);
     __shared__ __align__(16) uint8_t lds[A > B ? A : B];
-    const int nqt = (p.n + 1) / 2, tok0 = blockIdx.y * 32 * TB;
-    if ((int)blockIdx.x < nqt)
-        prolog_q_wide_body<TB>(p, 2 * blockIdx.x, tok0, lds);
-    else
-        mla_qb_wide_body<TB>(m, blockIdx.x - nqt, tok0, lds);
+    const int nqt = (p.n + 1) / 2, nqb = (m.n * MQH + 255) / 256, rows = (m.t + 32 * TB - 1) / (32 * TB);
+    int id = blockIdx.x;
+    if (id < nqt * rows)
+        prolog_q_wide_body<TB>(p, 2 * (id % nqt), id / nqt * 32 * TB, lds);
+    else {
+        id -= nqt * rows;
+        mla_qb_wide_body<TB>(m, id % nqb, id / nqb * 32 * TB, lds);
+    }
 }
 // the index heads' part; grid (index heads / 2 rounded up, token tiles), 512 lanes
 template <int TB>
@@ -1172,7 +1179,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
                 else if (p && (both.ns <= alone.ns + q_alone.ns || a.t >= FUSED_T))
                     gt_dispatch(both.tb, [&](auto tb) {
                         constexpr int TB = decltype(tb)::value < 7 ? decltype(tb)::value : 7;
-                        hipLaunchKernelGGL(fused_qb_wide_kernel<TB>, dim3(qcols + cols, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream,
+                        hipLaunchKernelGGL(fused_qb_wide_kernel<TB>, dim3((qcols + cols) * ((a.t + 32 * TB - 1) / (32 * TB))), dim3(GT_LANES), 0, stream,
                                            a, *p);
                     });
                 else {
