@@ -472,37 +472,45 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb16_wide_kernel(MlaPrologArg
 __device__ __forceinline__ float wave_sum(float v) { return wave_sum_butterfly(v); }
 __device__ __forceinline__ float wave_max(float v) { return wave_max_f32(v); }
 
-// Columns col0 + tid + 256 j, j < NJ, of a token's row: partial sums in a fixed order, rounded to bf16, into buf (n columns; S:
-// splits whose partial sums are in flight together).  Every load is unconditional (columns past the end re-read the last
-// one and are dropped): a load under a condition makes the compiler wait for it on the spot, one memory round trip per load.
-template <int S, int NJ>
-__device__ __forceinline__ void mla_sums(const MlaPrologArgs& a, int tok, int col0, int n, float* buf)
+// Columns col0 + 4 tid + 1024 j .. + 3, j < NP, of a token's row: partial sums in a fixed order, rounded to bf16, into x and buf (n
+// columns, a multiple of 4; S: splits whose partial sums are in flight together).  Four columns a load: a load costs the memory
+// pipe its 64 lanes whatever their width, and single columns were 64 loads a lane of the query's chain at seven splits (with the
+// indexer's key path, prolog_k_body: call of 1 token 34.6 -> 33.0 us, MLA alone 38.5 -> 36.4, 1501 tokens 232 -> 225).  Every
+// load is unconditional (columns past the end re-read the last ones and are dropped): a load under a condition makes the compiler
+// wait for it on the spot, one memory round trip per load.
+template <int S, int NP>
+__device__ __forceinline__ void mla_sums(const MlaPrologArgs& a, int tok, int col0, int n, float (&x)[NP][4], float* buf)
 {
     const int tid = threadIdx.x;
-    int cj[NJ];
-    float sum[NJ];
+    int cj[NP];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        cj[j] = col0 + min(256 * j + tid, n - 1);
-        sum[j] = 0.f;
+    for (int j = 0; j < NP; ++j) {
+        cj[j] = col0 + min(1024 * j + 4 * tid, n - 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[j][e] = 0.f;
     }
     // (a split past the end re-reads the last one and adds zero)
     for (int s0 = 0; s0 < a.ksplits; s0 += S) {
-        float v[S][NJ];
+        f32x4 v[S][NP];
 #pragma unroll
         for (int i = 0; i < S; ++i) {
             const float* p = a.xa_part + ((int64_t)min(s0 + i, a.ksplits - 1) * a.t + tok) * a.ncols;
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) v[i][j] = p[cj[j]];
+            for (int j = 0; j < NP; ++j) v[i][j] = *reinterpret_cast<const f32x4*>(p + cj[j]);
         }
 #pragma unroll
         for (int i = 0; i < S; ++i)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) sum[j] += s0 + i < a.ksplits ? v[i][j] : 0.f;
+            for (int j = 0; j < NP; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[j][e] += s0 + i < a.ksplits ? v[i][j][e] : 0.f;
     }
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
-        if (256 * j + tid < n) buf[256 * j + tid] = round_bf16(sum[j]);
+    for (int j = 0; j < NP; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[j][e] = round_bf16(x[j][e]);
+        if (1024 * j + 4 * tid < n) *reinterpret_cast<f32x4*>(buf + 1024 * j + 4 * tid) = f32x4{x[j][0], x[j][1], x[j][2], x[j][3]};
+    }
 }
 
 // The two norms of a token are independent chains of loads, reductions and barriers: a workgroup of 256 lanes for either (one
@@ -512,16 +520,17 @@ template <int S>
 __device__ __forceinline__ void mla_norm_query_body(const MlaPrologArgs& a, int tok)
 {
 #pragma clang fp contract(off)
-    __shared__ float buf[MAX_R];
+    __shared__ __align__(16) float buf[MAX_R];
     __shared__ float red[8];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = a.r;
     // (what does not depend on the sums is loaded first, so that its latency hides behind them)
-    constexpr int NQ = MAX_R / 256;
-    uint16_t gq[NQ];
+    constexpr int NP = MAX_R / 1024;
+    u32x2 gq[NP];
+    float x[NP][4];
 #pragma unroll
-    for (int j = 0; j < NQ; ++j) gq[j] = 256 * j + tid < r ? a.gamma_cq[256 * j + tid] : (uint16_t)0;
-    mla_sums<S, NQ>(a, tok, 0, r, buf);
+    for (int j = 0; j < NP; ++j) gq[j] = *reinterpret_cast<const u32x2*>(a.gamma_cq + min(1024 * j + 4 * tid, r - 4));
+    mla_sums<S, NP>(a, tok, 0, r, x, buf);
     __syncthreads();
     const float coff = 1.0f / (float)r;
     float ss = 0.f;
@@ -530,35 +539,36 @@ __device__ __forceinline__ void mla_norm_query_body(const MlaPrologArgs& a, int 
     if (lane == 0) red[wave] = ss;
     __syncthreads();
     const float y = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) + a.eps_cq);
-    float mx = 0.f;
+    float mx = 0.f; // (columns past the end are the last ones again)
 #pragma unroll
-    for (int j = 0; j < NQ; ++j) {
-        const int c = 256 * j + tid;
-        if (c < r) {
-            const float v = round_bf16(bf16_to_f32(gq[j]) * (buf[c] * y));
-            buf[c] = v;
-            mx = fmaxf(mx, fabsf(v));
+    for (int j = 0; j < NP; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            x[j][e] = round_bf16(half_of(gq[j][e >> 1], e & 1) * (x[j][e] * y));
+            mx = fmaxf(mx, fabsf(x[j][e]));
         }
-    }
     mx = wave_max(mx);
     if (lane == 0) red[4 + wave] = mx;
     __syncthreads();
     mx = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));
     if (a.quant) {
         const float sq = quant_scale(mx);
-        // four values per lane and store
-        for (int c = 4 * tid; c < r; c += 1024) {
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            const int c = 1024 * j + 4 * tid;
             uint32_t pk = 0;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(buf[c + e] * sq) & 0xffu) << (8 * e);
-            *reinterpret_cast<uint32_t*>(a.q_norm + (int64_t)tok * r + c) = pk;
+            for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(x[j][e] * sq) & 0xffu) << (8 * e);
+            if (c < r) *reinterpret_cast<uint32_t*>(a.q_norm + (int64_t)tok * r + c) = pk;
         }
         if (tid == 0) a.q_norm_scale[tok] = 1.0f / sq;
     } else { // bf16 form: q_norm is the normalised row itself
         uint16_t* qo = reinterpret_cast<uint16_t*>(a.q_norm) + (int64_t)tok * r;
-        for (int c = 4 * tid; c < r; c += 1024)
-            *reinterpret_cast<u32x2*>(qo + c) = u32x2{(uint32_t)f32_to_bf16(buf[c]) | ((uint32_t)f32_to_bf16(buf[c + 1]) << 16),
-                                                      (uint32_t)f32_to_bf16(buf[c + 2]) | ((uint32_t)f32_to_bf16(buf[c + 3]) << 16)};
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            const int c = 1024 * j + 4 * tid;
+            if (c < r) *reinterpret_cast<u32x2*>(qo + c) = u32x2{pack_bf16x2(x[j][0], x[j][1]), pack_bf16x2(x[j][2], x[j][3])};
+        }
     }
 }
 
@@ -567,7 +577,7 @@ template <int S>
 __device__ __forceinline__ void mla_norm_key_body(const MlaPrologArgs& a, int tok)
 {
 #pragma clang fp contract(off)
-    __shared__ float buf[MKV];
+    __shared__ __align__(16) float buf[MKV];
     __shared__ float red[8];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t row = a.cache_index[tok];
@@ -576,7 +586,8 @@ __device__ __forceinline__ void mla_norm_key_body(const MlaPrologArgs& a, int to
     const int ri = tid & 31;
     const float rc0 = bf16_to_f32(a.cos[(int64_t)tok * MROPE + ri]), rc1 = bf16_to_f32(a.cos[(int64_t)tok * MROPE + ri + 32]);
     const float rs0 = bf16_to_f32(a.sin[(int64_t)tok * MROPE + ri]), rs1 = bf16_to_f32(a.sin[(int64_t)tok * MROPE + ri + 32]);
-    mla_sums<S, (MKV + 255) / 256>(a, tok, a.r, MKV, buf);
+    float x[1][4];
+    mla_sums<S, 1>(a, tok, a.r, MKV, x, buf);
     __syncthreads();
     {
         const float x0 = buf[tid], x1 = buf[256 + tid];
@@ -683,8 +694,9 @@ __device__ __forceinline__ void mla_touch(const MlaPrologArgs& a, int tile)
     touch_rows(static_cast<const uint8_t*>(a.w_uq_qr) + (int64_t)tile * 16 * pieces, stride, rows, pieces);
 }
 
-// grid (2 x tokens: query, key | touching workgroups from `first` on), 256 lanes
-template <int S>
+// grid (2 x tokens: query, key | TOUCH: touching workgroups from `first` on), 256 lanes.  Without them (above 32 tokens) 40 registers
+// instead of 98, all of a token's chain that a SIMD can hold.
+template <int S, bool TOUCH>
 __global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a, int first)
 {
     const int id = blockIdx.x;
@@ -692,8 +704,9 @@ __global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a, int firs
         mla_norm_query_body<S>(a, id);
     else if (id < 2 * a.t)
         mla_norm_key_body<S>(a, id - a.t);
-    else if (id >= first)
-        mla_touch(a, id - first);
+    else if constexpr (TOUCH) {
+        if (id >= first) mla_touch(a, id - first);
+    }
 }
 
 // grid (n * 192 / 128), 256 lanes
@@ -901,8 +914,9 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb_wide_kernel(MlaPrologArgs 
 // The fused operator runs the two prologs' per-token kernels side by side in one launch, and likewise the two int8
 // GEMMs on q_norm (192 + 64 workgroups at model sizes: one per compute unit); the indexer's x @ [w_k | w_proj] rides along
 // in mla_xa_kernel as three more output tiles.
-// grid (3 x tokens: the MLA norms, the indexer's key path and weights (128 lanes) | touching workgroups from `first` on), 256 lanes
-template <int S>
+// grid (3 x tokens: the MLA norms, the indexer's key path and weights (128 lanes) | TOUCH: touching workgroups from `first` on),
+// 256 lanes
+template <int S, bool TOUCH>
 __global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, PrologArgs p, int first)
 {
     const int id = blockIdx.x;
@@ -913,7 +927,7 @@ __global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, Prolog
     else if (id < 3 * m.t) {
         if (threadIdx.x >= 128) return; // the barriers inside are among the two remaining waves
         prolog_k_body<S>(p, id - 2 * m.t);
-    } else if (id >= first) {
+    } else if (TOUCH && id >= first) {
         const int tile = id - first, nqb = m.n * MQH / 128;
         if (tile < nqb)
             mla_touch(m, tile);
@@ -1152,12 +1166,26 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         const int in_flight = a.ksplits <= 2 ? 2 : a.ksplits <= 4 ? 4 : 8;
         const int norms = (p ? 3 : 2) * a.t, first = (norms + 7) / 8 * 8;
         const unsigned grid = big ? norms : first + a.n * MQH / 128 + (p ? p->n : 0); // (the kernels above BIG_T tokens do not wait for their weights)
-        if (p)
-            hipLaunchKernelGGL((in_flight == 2 ? fused_norm_kernel<2> : in_flight == 4 ? fused_norm_kernel<4> : fused_norm_kernel<8>),
-                               dim3(grid), dim3(256), 0, stream, a, *p, first);
+        auto launch = [&](auto splits, auto touch) {
+            constexpr int S = decltype(splits)::value;
+            constexpr bool TOUCH = decltype(touch)::value;
+            if (p)
+                hipLaunchKernelGGL((fused_norm_kernel<S, TOUCH>), dim3(grid), dim3(256), 0, stream, a, *p, first);
+            else
+                hipLaunchKernelGGL((mla_norm_kernel<S, TOUCH>), dim3(grid), dim3(256), 0, stream, a, first);
+        };
+        auto launch_with = [&](auto touch) {
+            if (in_flight == 2)
+                launch(std::integral_constant<int, 2>{}, touch);
+            else if (in_flight == 4)
+                launch(std::integral_constant<int, 4>{}, touch);
+            else
+                launch(std::integral_constant<int, 8>{}, touch);
+        };
+        if (big)
+            launch_with(std::false_type{});
         else
-            hipLaunchKernelGGL((in_flight == 2 ? mla_norm_kernel<2> : in_flight == 4 ? mla_norm_kernel<4> : mla_norm_kernel<8>),
-                               dim3(grid), dim3(256), 0, stream, a, first);
+            launch_with(std::true_type{});
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
     {

@@ -604,7 +604,7 @@ __device__ __forceinline__ void prolog_k_body(const PrologArgs& a, int tok)
 {
 #pragma clang fp contract(off)
     __shared__ float red[2];
-    __shared__ float kb[PD];
+    __shared__ __align__(16) float kb[PD], yb[PD];
     const int tid = threadIdx.x;
     // everything that does not depend on the sums is loaded first (its latency hides behind them), and no load sits
     // under a condition (the compiler would wait for it on the spot)
@@ -612,27 +612,37 @@ __device__ __forceinline__ void prolog_k_body(const PrologArgs& a, int tok)
     const float gam = bf16_to_f32(a.ln_gamma[tid]), bet = bf16_to_f32(a.ln_beta[tid]);
     const int ri = tid & (PROPE - 1);
     const float rc = bf16_to_f32(a.cos[(int64_t)tok * PROPE + ri]), rs = bf16_to_f32(a.sin[(int64_t)tok * PROPE + ri]);
-    uint16_t hk[PD]; // this lane's column of hadamard_k
-#pragma unroll
-    for (int k = 0; k < PD; ++k) hk[k] = a.had_k[k * PD + tid];
     float kv = 0.f, wv = 0.f;
     const int wcol = PD + min(tid, a.n - 1);
     // S splits' loads in flight together (a split past the end re-reads the last one and adds zero); the order of the
     // additions is the order of the splits
-    for (int s0 = 0; s0 < a.ksplits; s0 += S) {
-        float v0[S], v1[S];
+    float v0[S], v1[S];
+    auto load = [&](int s0) {
 #pragma unroll
         for (int j = 0; j < S; ++j) {
             const float* p = a.xw_part + ((int64_t)min(s0 + j, a.ksplits - 1) * a.t + tok) * a.xw_stride + a.xw_col0;
             v0[j] = p[tid];
             v1[j] = p[wcol];
         }
+    };
+    auto add = [&](int s0) {
 #pragma unroll
         for (int j = 0; j < S; ++j) {
             kv += s0 + j < a.ksplits ? v0[j] : 0.f;
             wv += s0 + j < a.ksplits ? v1[j] : 0.f;
         }
-    }
+    };
+    load(0);
+    __builtin_amdgcn_sched_barrier(0);
+    // the Hadamard matrix behind the sums in the memory pipe: the wave's half of the rows, two columns to a lane (a wave per half of
+    // the columns asked for twice as many loads, 256 of 2 bytes a lane, in front of the sums)
+    const int hw = __builtin_amdgcn_readfirstlane(tid >> 6), hc = 2 * (tid & 63);
+    uint32_t hk[PD / 2];
+#pragma unroll
+    for (int k = 0; k < PD / 2; ++k) hk[k] = *reinterpret_cast<const uint32_t*>(a.had_k + (PD / 2 * hw + k) * PD + hc);
+    __builtin_amdgcn_sched_barrier(0);
+    add(0);
+    for (int s0 = S; s0 < a.ksplits; s0 += S) load(s0), add(s0);
     // LayerNorm in fp32 (biased variance), -> bf16
     const float mean = block_sum128(kv, red) / (float)PD;
     const float dlt = kv - mean;
@@ -650,11 +660,23 @@ __device__ __forceinline__ void prolog_k_body(const PrologArgs& a, int tok)
     __syncthreads();
     kb[tid] = kr;
     __syncthreads();
-    // hadamard: y[n] = sum_k kr[k] H[k][n], fp32, -> bf16
-    float y = 0.f;
+    // hadamard: y[n] = sum_k kr[k] H[k][n], fp32, k in order (the second wave goes on from the first's sums), -> bf16
+#pragma unroll 1
+    for (int part = 0; part < 2; ++part) {
+        if (hw == part) {
+            float2 h = part ? *reinterpret_cast<const float2*>(yb + hc) : float2{0.f, 0.f};
 #pragma unroll
-    for (int k = 0; k < PD; ++k) y = __builtin_fmaf(kb[k], bf16_to_f32(hk[k]), y);
-    y = bf16_to_f32(f32_to_bf16(y));
+            for (int k = 0; k < PD / 2; ++k) {
+                asm("" : "+v"(hk[k])); // (taken apart here, not in front of the loop for 64 registers more)
+                const float x = kb[PD / 2 * hw + k];
+                h.x = __builtin_fmaf(x, half_of(hk[k], 0), h.x);
+                h.y = __builtin_fmaf(x, half_of(hk[k], 1), h.y);
+            }
+            *reinterpret_cast<float2*>(yb + hc) = h;
+        }
+        __syncthreads();
+    }
+    const float y = bf16_to_f32(f32_to_bf16(yb[tid]));
     const float mx = block_max128(fabsf(y), red);
     const float sq = quant_scale(mx);
     if (row >= 0 && row < a.cache_rows) {
