@@ -22,7 +22,7 @@
 //                    key's rotary embedding, the three cache writes, q_norm / q_norm_scale
 //   mla_qb_kernel    int8 MFMA GEMM q_norm @ w_uq_qr, 128 outputs x 32 tokens per workgroup, weights streamed to LDS
 //                    (gemm_tile.h); dequantisation and the query's rotary embedding on the tile
-//   mla_wuk_kernel   per (head, 128 outputs): q_b[:, head, :128] @ w_uk[head]
+//   mla_wuk_kernel   per (head, 128 outputs): q_b[:, head, :128] @ w_uk[head]; above 64 tokens per head (mla_wuk_wide_kernel)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -994,90 +994,170 @@ __global__ __launch_bounds__(GT_LANES, 2) void fused_q_wide_kernel(PrologArgs p)
 }
 
 // ------------------------------------------------------------------------------------------------ q_b[:, head, :128] @ w_uk[head]
-// grid (heads, 512 / 128, z), 256 lanes: wave w owns outputs [32 w, 32 w + 32) of the tile.  The head's 128 x 128 weight
-// tile stays in LDS while the workgroup walks the token tiles z, z + gridDim.z, ... (one at decode sizes; at prefill
-// sizes the weights are then read once per workgroup instead of once per token tile); the next tile's operand rows are
-// requested before the current tile's products.  TB blocks of 32 tokens per tile: 1 at decode sizes; 2 at prefill
-// sizes, where every weight fragment read from LDS then feeds two MFMAs.
+// Up to 32 TB tokens (TB 1 or 2), grid (heads, 512 / 128), 256 lanes: wave w owns outputs [32 w, 32 w + 32) of the tile.
 template <int TB>
 __global__ __launch_bounds__(256) void mla_wuk_kernel(MlaPrologArgs a)
 {
-    constexpr int WTOK = MTOK * TB;    // tokens per tile
+    constexpr int WTOK = MTOK * TB;    // tokens
     constexpr int OROW = 128 * 2 + 16; // bytes per LDS row of the WTOK x 128 bf16 output tile (padded)
     __shared__ __align__(16) uint8_t wl[MNOPE * TROW];
-    __shared__ __align__(16) uint8_t bt[WTOK * OROW]; // the token tile's operand rows
-    __shared__ __align__(16) uint8_t ot[WTOK * OROW]; // its outputs
+    __shared__ __align__(16) uint8_t bt[WTOK * OROW]; // the operand rows
+    __shared__ __align__(16) uint8_t ot[WTOK * OROW]; // the outputs
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, hl = lane >> 5;
     const int head = blockIdx.x, ct = blockIdx.y;
-    const int ttiles = (a.t + WTOK - 1) / WTOK;
     const uint16_t* src = a.w_uk + (int64_t)head * MNOPE * MC + ct * 128;
-    // a tile's operand rows: WTOK tokens x 256 bytes, fetched once by the workgroup in 16-byte pieces (16 lanes per row) and
+    // the operand rows: WTOK tokens x 256 bytes, fetched once by the workgroup in 16-byte pieces (16 lanes per row) and
     // handed to the waves through LDS - a wave loading its own operand would fetch a different row with every lane pair,
     // which costs the texture addresser a cycle per row and instruction, four times over for the four waves
     const int prow = tid >> 4, pcol = tid & 15;
-    auto fetch = [&](u32x4 (&q)[2 * TB], int tt) {
+    u32x4 q[2 * TB];
 #pragma unroll
-        for (int i = 0; i < 2 * TB; ++i)
-            q[i] = *reinterpret_cast<const u32x4*>(a.qb_nope + ((int64_t)min(tt * WTOK + prow + 16 * i, a.t - 1) * a.n + head) * MNOPE +
-                                                   8 * pcol);
-    };
-    auto park = [&](const u32x4 (&q)[2 * TB]) {
-#pragma unroll
-        for (int i = 0; i < 2 * TB; ++i) *reinterpret_cast<u32x4*>(bt + (prow + 16 * i) * OROW + 16 * pcol) = q[i];
-    };
-    u32x4 q0[2 * TB];
-    fetch(q0, blockIdx.z);
+    for (int i = 0; i < 2 * TB; ++i)
+        q[i] = *reinterpret_cast<const u32x4*>(a.qb_nope + ((int64_t)min(prow + 16 * i, a.t - 1) * a.n + head) * MNOPE + 8 * pcol);
 #pragma unroll
     for (int i = tid; i < MNOPE * 16; i += 256) {
         const int k = i >> 4, c = i & 15;
         *reinterpret_cast<u32x4*>(wl + k * TROW + c * 16) = *reinterpret_cast<const u32x4*>(src + (int64_t)k * MC + c * 8);
     }
-    park(q0);
+#pragma unroll
+    for (int i = 0; i < 2 * TB; ++i) *reinterpret_cast<u32x4*>(bt + (prow + 16 * i) * OROW + 16 * pcol) = q[i];
     __syncthreads();
     const int jj = lane & 15, mh = (lane >> 4) & 1;
     const uint8_t* hp = wl + (8 * hl + (jj >> 2)) * TROW + (32 * wave + 16 * mh + 4 * (jj & 3)) * 2;
-    for (int tt = blockIdx.z; tt < ttiles; tt += gridDim.z) {
-        // the rows of the tile after this one, if there is one (uniform over the workgroup)
-        const bool more = tt + (int)gridDim.z < ttiles;
-        u32x4 qn[2 * TB];
-        if (more) fetch(qn, tt + gridDim.z);
-        f32x16 acc[TB];
+    f32x16 acc[TB];
 #pragma unroll
-        for (int tb = 0; tb < TB; ++tb)
+    for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[tb][e] = 0.f;
+        for (int e = 0; e < 16; ++e) acc[tb][e] = 0.f;
+    // (the weight fragment by transposing reads: see gemm_tr_tile)
+#pragma unroll
+    for (int ks = 0; ks < MNOPE / 16; ++ks) {
+        const s16x4 lo = lds_read_tr(hp + ks * 16 * TROW);
+        const s16x4 hi = lds_read_tr(hp + (ks * 16 + 4) * TROW);
+        const bf16x8 av = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {
+            const bf16x8 bx = *reinterpret_cast<const bf16x8*>(bt + (32 * tb + l32) * OROW + (ks * 16 + 8 * hl) * 2);
+            acc[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bx, acc[tb], 0, 0, 0);
+        }
+    }
+    // through LDS, so that a token's 128 outputs leave as one 256-byte run (16 lanes x 16 bytes)
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4) {
+            const u32x2 pk = {(uint32_t)f32_to_bf16(acc[tb][4 * e4]) | ((uint32_t)f32_to_bf16(acc[tb][4 * e4 + 1]) << 16),
+                              (uint32_t)f32_to_bf16(acc[tb][4 * e4 + 2]) | ((uint32_t)f32_to_bf16(acc[tb][4 * e4 + 3]) << 16)};
+            *reinterpret_cast<u32x2*>(ot + (32 * tb + l32) * OROW + (32 * wave + 8 * e4 + 4 * hl) * 2) = pk;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2 * TB; ++i) {
+        const int tok = prow + 16 * i;
+        if (tok < a.t)
+            *reinterpret_cast<u32x4*>(a.q_nope + ((int64_t)tok * a.n + head) * MC + ct * 128 + 8 * pcol) =
+                *reinterpret_cast<const u32x4*>(ot + tok * OROW + 16 * pcol);
+    }
+}
+
+// The same product above 64 tokens, with the same sums in the same order.  Bound by the outputs' way to memory (1501 tokens x 128
+// heads: 197 MB out, 49 in, 47 us at the rate of a large copy).  By tiles of 64 tokens x 128 outputs, two workgroups to a CU with
+// the weights in LDS, every tile's rows were read four times over and a tile passed two barriers: 65 us.  So a workgroup of 512
+// lanes owns a head's whole 512 outputs and walks the token tiles of 64, z of them side by side (z: one workgroup to a CU); wave w
+// owns outputs [64 w, +64), whose weights stay in its registers (64 a lane) and whose outputs leave through LDS of its own; a
+// tile's rows are in one of two buffers, and one barrier ends it.  Call of 1501 tokens 236.7 -> 224.5 us, 300: 81.7 -> 77.2, 128:
+// 56.4 -> 54.7; at 64 tokens, a single tile for half as many waves, 48.9 -> 49.4, so not there.  grid (heads, z), 512 lanes.
+constexpr int WW_TOK = 64;
+__global__ __launch_bounds__(512, 2) void mla_wuk_wide_kernel(MlaPrologArgs a)
+{
+    constexpr int BROW = MNOPE * 2 + 16; // bytes per LDS row of a tile's operand rows (padded)
+    constexpr int OROW = 64 * 2 + 16;    // of a wave's 64 outputs, or of its slice of the weights
+    constexpr int OWN = 2 * 32 * OROW;   // two blocks of 32 tokens of a wave's outputs
+    constexpr int BT = WW_TOK * BROW, WL = MNOPE * OROW;
+    __shared__ __align__(16) uint8_t lds[8 * WL]; // the weights on their way to the registers; then [2] operand rows, outputs
+    static_assert(2 * BT + 8 * OWN <= 8 * WL, "LDS");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, hl = lane >> 5, head = blockIdx.x;
+    const int ttiles = (a.t + WW_TOK - 1) / WW_TOK;
+    const int prow = tid >> 4, pcol = tid & 15; // the operand rows' pieces of 16 bytes, 32 rows a load
+    auto fetch = [&](u32x4 (&q)[2], int tt) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            q[i] = *reinterpret_cast<const u32x4*>(a.qb_nope + ((int64_t)min(tt * WW_TOK + prow + 32 * i, a.t - 1) * a.n + head) * MNOPE + 8 * pcol);
+    };
+    auto park = [&](const u32x4 (&q)[2], uint8_t* bt) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(bt + (prow + 32 * i) * BROW + 16 * pcol) = q[i];
+    };
+    u32x4 q[2];
+    fetch(q, blockIdx.y);
+    bf16x8 w[2][MNOPE / 16];
+    {
+        const uint16_t* src = a.w_uk + (int64_t)head * MNOPE * MC + 64 * wave;
+        uint8_t* wl = lds + wave * WL;
+        const int r = lane >> 3, c = lane & 7;
+        u32x4 x[MNOPE / 8];
+#pragma unroll
+        for (int i = 0; i < MNOPE / 8; ++i) x[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)(8 * i + r) * MC + 8 * c);
+#pragma unroll
+        for (int i = 0; i < MNOPE / 8; ++i) *reinterpret_cast<u32x4*>(wl + (8 * i + r) * OROW + 16 * c) = x[i];
+        __builtin_amdgcn_wave_barrier();
         // (the weight fragment by transposing reads: see gemm_tr_tile)
+        const int jj = lane & 15, mh = (lane >> 4) & 1;
+        const uint8_t* hp = wl + (8 * hl + (jj >> 2)) * OROW + (16 * mh + 4 * (jj & 3)) * 2;
 #pragma unroll
-        for (int ks = 0; ks < MNOPE / 16; ++ks) {
-            const s16x4 lo = lds_read_tr(hp + ks * 16 * TROW);
-            const s16x4 hi = lds_read_tr(hp + (ks * 16 + 4) * TROW);
-            const bf16x8 av = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-            for (int tb = 0; tb < TB; ++tb) {
-                const bf16x8 bx = *reinterpret_cast<const bf16x8*>(bt + (32 * tb + l32) * OROW + (ks * 16 + 8 * hl) * 2);
-                acc[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bx, acc[tb], 0, 0, 0);
+            for (int ks = 0; ks < MNOPE / 16; ++ks) {
+                const s16x4 lo = lds_read_tr(hp + 64 * nb + ks * 16 * OROW), hi = lds_read_tr(hp + 64 * nb + (ks * 16 + 4) * OROW);
+                w[nb][ks] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
             }
-        }
-        // through LDS, so that a token's 128 outputs leave as one 256-byte run (16 lanes x 16 bytes)
+    }
+    __syncthreads(); // every wave has its weights
+    park(q, lds);
+    __syncthreads();
+    uint8_t* own = lds + 2 * BT + wave * OWN;
+    uint16_t* dst = a.q_nope + (int64_t)head * MC + 64 * wave + 8 * (lane & 7);
+    for (int tt = blockIdx.y, cur = 0; tt < ttiles; tt += gridDim.y, cur ^= 1) {
+        const bool more = tt + (int)gridDim.y < ttiles; // (uniform over the workgroup)
+        if (more) fetch(q, tt + gridDim.y);
+        const uint8_t* bt = lds + cur * BT + l32 * BROW + 16 * hl;
+        f32x16 acc[2][2];
 #pragma unroll
-        for (int tb = 0; tb < TB; ++tb)
+        for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) {
-                const u32x2 pk = {(uint32_t)f32_to_bf16(acc[tb][4 * e4]) | ((uint32_t)f32_to_bf16(acc[tb][4 * e4 + 1]) << 16),
-                                  (uint32_t)f32_to_bf16(acc[tb][4 * e4 + 2]) | ((uint32_t)f32_to_bf16(acc[tb][4 * e4 + 3]) << 16)};
-                *reinterpret_cast<u32x2*>(ot + (32 * tb + l32) * OROW + (32 * wave + 8 * e4 + 4 * hl) * 2) = pk;
+            for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[tb][nb][e] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < MNOPE / 16; ++ks)
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) {
+                const bf16x8 bx = *reinterpret_cast<const bf16x8*>(bt + 32 * tb * BROW + 32 * ks);
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) acc[tb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[nb][ks], bx, acc[tb][nb], 0, 0, 0);
             }
-        __syncthreads(); // outputs parked; every wave is done with the operand rows
+        if (more) park(q, lds + (cur ^ 1) * BT); // (read last before the barrier behind the tile before)
+        // through LDS of the wave's own, so that a token's 64 outputs leave as one run of 128 bytes
 #pragma unroll
-        for (int i = 0; i < 2 * TB; ++i) {
-            const int tok = prow + 16 * i;
-            if (tt * WTOK + tok < a.t)
-                *reinterpret_cast<u32x4*>(a.q_nope + ((int64_t)(tt * WTOK + tok) * a.n + head) * MC + ct * 128 + 8 * pcol) =
-                    *reinterpret_cast<const u32x4*>(ot + tok * OROW + 16 * pcol);
+        for (int tb = 0; tb < 2; ++tb) {
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                for (int e4 = 0; e4 < 4; ++e4)
+                    *reinterpret_cast<u32x2*>(own + (32 * tb + l32) * OROW + (32 * nb + 8 * e4 + 4 * hl) * 2) =
+                        u32x2{pack_bf16x2(acc[tb][nb][4 * e4], acc[tb][nb][4 * e4 + 1]), pack_bf16x2(acc[tb][nb][4 * e4 + 2], acc[tb][nb][4 * e4 + 3])};
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = 32 * tb + 8 * i + (lane >> 3), tok = tt * WW_TOK + row;
+                const u32x4 o = *reinterpret_cast<const u32x4*>(own + row * OROW + 16 * (lane & 7));
+                if (tok < a.t) *reinterpret_cast<u32x4*>(dst + (int64_t)tok * a.n * MC) = o;
+            }
+            __builtin_amdgcn_wave_barrier();
         }
-        if (more) park(qn);
-        __syncthreads();
+        __syncthreads(); // the next tile's rows are parked, this one's read
     }
 }
 
@@ -1231,15 +1311,13 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
     if ((e = hipGetLastError()) != hipSuccess) return e;
     {
         ScopedKernelTimer tm(KID_MLA_WUK, stream);
-        // token tiles per workgroup: one while that leaves the grid at about a thousand workgroups or fewer, more beyond
-        if (big) {
-            const int wtiles = (a.t + 2 * MTOK - 1) / (2 * MTOK);
-            const int zdim = std::min(wtiles, std::max(1, 1024 / (a.n * (MC / 128))));
-            hipLaunchKernelGGL(mla_wuk_kernel<2>, dim3(a.n, MC / 128, zdim), dim3(256), 0, stream, a);
-        } else {
-            const int zdim = std::min(ttiles, std::max(1, 1024 / (a.n * (MC / 128))));
-            hipLaunchKernelGGL(mla_wuk_kernel<1>, dim3(a.n, MC / 128, zdim), dim3(256), 0, stream, a);
-        }
+        if (a.t > WW_TOK) {
+            const int wtiles = (a.t + WW_TOK - 1) / WW_TOK, zdim = std::min(wtiles, std::max(1, 256 / a.n));
+            hipLaunchKernelGGL(mla_wuk_wide_kernel, dim3(a.n, zdim), dim3(512), 0, stream, a);
+        } else if (big)
+            hipLaunchKernelGGL(mla_wuk_kernel<2>, dim3(a.n, MC / 128), dim3(256), 0, stream, a);
+        else
+            hipLaunchKernelGGL(mla_wuk_kernel<1>, dim3(a.n, MC / 128), dim3(256), 0, stream, a);
     }
     return hipGetLastError();
 }

@@ -233,6 +233,14 @@ def test_prefill_query_tiles(cuda, t, n):
     check(case, run(case, cuda, entry="mla_prolog_quant_p"))
 
 
+@pytest.mark.parametrize("t,n", [(64, 4), (65, 4), (127, 128), (193, 2), (193, 128), (193, 258)])
+def test_prefill_absorbed_tiles(cuda, t, n):
+    # q_nope @ w_uk above 64 tokens: tiles of 64 tokens with remainders of one to all rows, one tile to a workgroup, two, and (258 heads: more
+    # than workgroups that fit side by side) all of them
+    case = op.make_case(t, 1, 64, seed=60 + t, h=256, q_lora_rank=128, n=n)
+    check(case, run(case, cuda, entry="mla_prolog_quant_p"))
+
+
 @pytest.mark.parametrize("t,n", [(33, 2), (128, 6), (129, 4), (300, 2)])
 def test_bf16_form_prefill_tiles(cuda, t, n):
     # from 33 tokens on the query product owns 128 tokens x 256 outputs: remainders of both, chains of 128 rows
