@@ -83,6 +83,24 @@ __device__ __forceinline__ float wave_sum_butterfly(float v)
     return v;
 }
 
+// The same from 32 lanes apart down to 1: rotations of a row serve for 8 and 4, since by then its halves, then quarters, repeat.
+__device__ __forceinline__ float wave_sum_descending(float v)
+{
+    {
+        const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+        v = __builtin_bit_cast(float, (unsigned)sw[0]) + __builtin_bit_cast(float, (unsigned)sw[1]);
+    }
+    {
+        const auto sw = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+        v = __builtin_bit_cast(float, (unsigned)sw[0]) + __builtin_bit_cast(float, (unsigned)sw[1]);
+    }
+    v += dpp_perm_f32<0x128>(v); // row_ror:8
+    v += dpp_perm_f32<0x124>(v); // row_ror:4
+    v += dpp_perm_f32<0x4E>(v);  // quad_perm [2, 3, 0, 1]
+    v += dpp_perm_f32<0xB1>(v);  // quad_perm [1, 0, 3, 2]
+    return v;
+}
+
 // Two fp32 -> one dword holding two bf16 (round to nearest even), low half = a.
 __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b)
 {
