@@ -374,16 +374,13 @@ inline int64_t gt_time_ns(int64_t wgs, int64_t stages, int tb)
 {
     return (wgs + 255) / 256 * (stages * (tb + 2) * 160 + 12000) + wgs * stages * (tb + 8) * 4096 / 26000;
 }
-struct GtPlan {
-    int tb;
-    int64_t ns;
-};
-inline GtPlan gt_token_blocks(int64_t t, int64_t cols, int64_t stages, int most)
+inline int gt_token_blocks(int64_t t, int64_t cols, int64_t stages, int most)
 {
-    GtPlan best = {4, INT64_MAX};
+    int best = 4;
+    int64_t best_ns = INT64_MAX;
     for (int tb = 4; tb <= most; ++tb) {
         const int64_t ns = gt_time_ns(cols * ((t + 32 * tb - 1) / (32 * tb)), stages, tb);
-        if (ns < best.ns) best = {tb, ns};
+        if (ns < best_ns) best = tb, best_ns = ns;
     }
     return best;
 }

@@ -18,7 +18,7 @@
 // MFMA operands want (contraction contiguous per lane), so every weight tile goes through LDS and is read back
 // transposed: bf16 tiles with ds_read_b64_tr_b16, the int8 tile with ds_read_b64_tr_b8.
 //   mla_xa_kernel    x @ [w_dq | w_dkv_kr], 256 contraction rows x 128 outputs per workgroup, fp32 partials
-//   mla_norm_kernel  one workgroup per token: fixed-order sum of the partials, both RmsNorms, the quantisations, the
+//   mla_norm_kernel  two workgroups per token: fixed-order sum of the partials, an RmsNorm each, the quantisations, the
 //                    key's rotary embedding, the three cache writes, q_norm / q_norm_scale
 //   mla_qb_kernel    int8 MFMA GEMM q_norm @ w_uq_qr, 128 outputs x 32 tokens per workgroup, weights streamed to LDS
 //                    (gemm_tile.h); dequantisation and the query's rotary embedding on the tile
@@ -962,11 +962,10 @@ __global__ __launch_bounds__(256, 2) void fused_qb_big_kernel(MlaPrologArgs m, P
         prolog_q_big_body<QB_DEPTH>(p, blockIdx.x - nqb, blockIdx.y * QB_TOK, lds);
 }
 
-constexpr int FUSED_T = 2048;
-// Above 256 tokens the two products in one launch of gemm_tile.h's tiles where that takes no more rounds of workgroups: the index
-// heads' part alone is half a round up to 512 tokens (call of 257 tokens 94 -> 80 us, 512: 124 -> 104).  Its tiles are up to
-// 224 tokens; where the query product's own of 256 save a round, and a round counts, the two are launches of their own (1024
-// tokens: 191 us in one, 184 in two, 1200: 219 / 208, 2048: the same, 4096: 680 / 691).
+// Above 256 tokens the two products in one launch of gemm_tile.h's tiles: the index heads' part alone is half a round of workgroups
+// up to 512 tokens (call of 257 tokens 83.0 us as two launches, 72.2 as one, 512: 104.4 / 96.3, 1024: 163.6 / 160.7, 1344: 211.5 /
+// 194.6, 4096: 604.7 / 591.0).  Its tiles are up to 224 tokens; where the query product's own of 256 save a round the two are the
+// same (900 tokens 153.9 / 154.0, 2048: 314.5 / 316.6).
 // The index heads' tiles take the longer, 26 us at 192 tokens against 19, and come first, those of all tokens: as columns of each
 // token tile they began again in the last round of workgroups (104 us for the kernel at 1501 tokens,
 // 92 so; the call 240.8 -> 236.8, no difference where the rounds come out even).
@@ -984,13 +983,6 @@ __global__ __launch_bounds__(GT_LANES, 2) void fused_qb_wide_kernel(MlaPrologArg
         id -= nqt * rows;
         mla_qb_wide_body<TB>(m, id % nqb, id / nqb * 32 * TB, lds);
     }
-}
-// the index heads' part; grid (index heads / 2 rounded up, token tiles), 512 lanes
-template <int TB>
-__global__ __launch_bounds__(GT_LANES, 2) void fused_q_wide_kernel(PrologArgs p)
-{
-    __shared__ __align__(16) uint8_t lds[prolog_q_wide_lds(TB)];
-    prolog_q_wide_body<TB>(p, 2 * blockIdx.x, blockIdx.y * 32 * TB, lds);
 }
 
 // ------------------------------------------------------------------------------------------------ q_b[:, head, :128] @ w_uk[head]
@@ -1280,27 +1272,19 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
                 hipLaunchKernelGGL(fused_qb_big_kernel, dim3(qgrid.x + p->n, qgrid.y), dim3(256), 0, stream, a, *p);
             } else {
                 const int cols = (a.n * MQH + 255) / 256, qcols = p ? (p->n + 1) / 2 : 0, stages = a.r / GT_KI8;
-                const GtPlan alone = gt_token_blocks(a.t, cols, stages, 8), q_alone = gt_token_blocks(a.t, qcols, stages, 7);
-                const GtPlan both = gt_token_blocks(a.t, cols + qcols, stages, 7);
                 if (a.t <= BIG_T2)
                     hipLaunchKernelGGL(mla_qb_big_kernel<QB_DEPTH>, qgrid, dim3(256), 0, stream, a);
-                else if (p && (both.ns <= alone.ns + q_alone.ns || a.t >= FUSED_T))
-                    gt_dispatch(both.tb, [&](auto tb) {
+                else if (p)
+                    gt_dispatch(gt_token_blocks(a.t, cols + qcols, stages, 7), [&](auto tb) {
                         constexpr int TB = decltype(tb)::value < 7 ? decltype(tb)::value : 7;
                         hipLaunchKernelGGL(fused_qb_wide_kernel<TB>, dim3((qcols + cols) * ((a.t + 32 * TB - 1) / (32 * TB))), dim3(GT_LANES), 0, stream,
                                            a, *p);
                     });
-                else {
-                    gt_dispatch(alone.tb, [&](auto tb) {
+                else
+                    gt_dispatch(gt_token_blocks(a.t, cols, stages, 8), [&](auto tb) {
                         constexpr int TB = decltype(tb)::value;
                         hipLaunchKernelGGL(mla_qb_wide_kernel<TB>, dim3(cols, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream, a);
                     });
-                    if (p)
-                        gt_dispatch(q_alone.tb, [&](auto tb) {
-                            constexpr int TB = decltype(tb)::value < 7 ? decltype(tb)::value : 7;
-                            hipLaunchKernelGGL(fused_q_wide_kernel<TB>, dim3(qcols, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream, *p);
-                        });
-                }
             }
         } else if (p) {
             hipLaunchKernelGGL(fused_qb_kernel, dim3(a.n * MQH / 128 + p->n), dim3(256), 0, stream, a, *p);
