@@ -49,8 +49,7 @@ constexpr int MQROW = 136;         // bytes per LDS row of a [k][128] int8 weigh
 constexpr int BIG_T = 33;         // token count from which the kernels that own an output tile take over: the others read the
                                   // weights once per 32 tokens (fused prolog, 33 tokens: 63.6 against 47.2 us, 96: 87 / 55, 127:
                                   // 108 / 59; 24 tokens: 43.6 / 46.8)
-constexpr int BIG_T2 = 256;       // token count above which the tiles are 256 outputs wide (127 tokens: 59 against 87 us, 256: 83 /
-                                  // 94, 257: 106 / 94)
+constexpr int BIG_T2 = 256;       // token count above which the x product's tiles are 256 outputs wide, in splits of its own
 
 // 32 outputs x 32 tokens += W[KSTEPS steps of 16 rows, outputs]^T . X[tokens, k]: A by transposing reads of the [k][n]
 // tile in LDS, rows of ROWB bytes.  Lane jj of a 16-lane group points at row 8 hl + jj / 4 (+ 4 for the second read) of
@@ -716,13 +715,13 @@ __global__ __launch_bounds__(256) void mla_qb_kernel(MlaPrologArgs a)
     mla_qb_body(a, blockIdx.x, lds);
 }
 
-// The same product at 33 to 256 tokens: a workgroup owns 128 tokens x 128 outputs and walks the
+// The same product at 33 to 128 tokens beside the index heads' (fused_qb_big_kernel): a workgroup owns 128 tokens x 128 outputs and walks the
 // contraction in stages of 128 rows, both operands staged through LDS with the next stage's global loads in flight.  Wave
 // (wr, wc) owns tokens [64 wr, +64) x outputs [64 wc, +64): every operand fragment read from LDS feeds four MFMAs.  The
 // int32 sums are exact, so the results are the bits of mla_qb_kernel's.  The outputs go through LDS (in place of the
 // operand tiles, which are no longer needed) so that they leave as the 128-byte runs they are in memory - a 128-column
 // tile holds two 64-column segments, each either half of a head's 128 first dims or a head's 64 rotary dims, rotated
-// into place on the way.  grid (n * 192 / 128, token tiles of 128), 256 lanes.
+// into place on the way.  256 lanes.
 constexpr int QG_TOK = 128, QG_K = 128;
 constexpr int QG_QROW = QG_K + 16;       // bytes per LDS row of the [token][k] int8 tile (padded against bank conflicts)
 constexpr int QG_OROW = 128 * 2 + 16;    // bytes per LDS row of the [token][128 outputs] bf16 tile
@@ -853,15 +852,9 @@ __device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0
     }
 }
 
-template <int DEPTH>
-__global__ __launch_bounds__(256, 2) void mla_qb_big_kernel(MlaPrologArgs a)
-{
-    __shared__ __align__(16) uint8_t stage_lds[QG_STAGE_BYTES];
-    mla_qb_big_body<DEPTH>(a, blockIdx.x * 128, blockIdx.y * QG_TOK, stage_lds);
-}
-
-// Above 256 tokens: 32 TB tokens x 256 outputs per workgroup (gemm_tile.h), the same exact sums and the same operations behind
-// them.  128 x 128 tiles through registers took 109 us at 1501 tokens, bound by the operands' way into LDS.
+// From 33 tokens on, above 128 beside the index heads': 32 TB tokens x 256 outputs per workgroup (gemm_tile.h), the same exact sums
+// and the same operations behind them.  128 x 128 tiles through registers are bound by the operands' way into LDS: MLA prolog of 40
+// tokens 41.0 us a call against 38.8, 128: 50.0 / 48.5, 200: 66.2 / 57.2.
 constexpr int mla_qb_wide_lds(int tb) // the product's stages, or four blocks of the output tile
 {
     const int tok = 32 * tb, ring = gt_lds_bytes(tb);
@@ -948,21 +941,22 @@ __global__ __launch_bounds__(256) void fused_qb_kernel(MlaPrologArgs m, PrologAr
         prolog_q_stream_body(p, blockIdx.x - nqb, lds);
 }
 
-// The same pair at 33 to 256 tokens: both products per 128 tokens, side by side.  The indexer's epilogue sets the LDS (68 KB:
-// two workgroups to a CU), so both run with three stages of loads in flight.
-// grid (n * 192 / 128 + index heads, token tiles of 128), 256 lanes
+// The same pair at 33 to 128 tokens: both products side by side.  The indexer's epilogue sets the LDS (68 KB:
+// two workgroups to a CU), so both run with three stages of loads in flight.  With tiles of 256 outputs half as many workgroups have
+// the index heads' epilogue to hide: call of 64 tokens 47.9 us here, 48.5 there, 128: 54.1 / 55.4; 129: 66.7 / 63.9, 256: 75.1 / 70.0.
+// grid (n * 192 / 128 + index heads), 256 lanes
 __global__ __launch_bounds__(256, 2) void fused_qb_big_kernel(MlaPrologArgs m, PrologArgs p)
 {
     static_assert(QB_LDS_BYTES >= QG_STAGE_BYTES && QB_TOK == QG_TOK, "one LDS block and one token tiling serve both bodies");
     __shared__ __align__(16) uint8_t lds[QB_LDS_BYTES];
     const int nqb = m.n * MQH / 128;
     if ((int)blockIdx.x < nqb)
-        mla_qb_big_body<QB_DEPTH>(m, blockIdx.x * 128, blockIdx.y * QG_TOK, lds);
+        mla_qb_big_body<QB_DEPTH>(m, blockIdx.x * 128, 0, lds);
     else
-        prolog_q_big_body<QB_DEPTH>(p, blockIdx.x - nqb, blockIdx.y * QB_TOK, lds);
+        prolog_q_big_body<QB_DEPTH>(p, blockIdx.x - nqb, 0, lds);
 }
 
-// Above 256 tokens the two products in one launch of gemm_tile.h's tiles: the index heads' part alone is half a round of workgroups
+// Above 128 tokens the two products in one launch of gemm_tile.h's tiles: the index heads' part alone is half a round of workgroups
 // up to 512 tokens (call of 257 tokens 83.0 us as two launches, 72.2 as one, 512: 104.4 / 96.3, 1024: 163.6 / 160.7, 1344: 211.5 /
 // 194.6, 4096: 604.7 / 591.0).  Its tiles are up to 224 tokens; where the query product's own of 256 save a round the two are the
 // same (900 tokens 153.9 / 154.0, 2048: 314.5 / 316.6).
@@ -1267,14 +1261,11 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         } else if (!a.quant) {
             hipLaunchKernelGGL(mla_qb16_kernel, dim3((a.n * MQH + 127) / 128), dim3(256), 0, stream, a);
         } else if (big) {
-            const dim3 qgrid(a.n * MQH / 128, (a.t + QG_TOK - 1) / QG_TOK);
-            if (p && a.t <= BIG_T2) {
-                hipLaunchKernelGGL(fused_qb_big_kernel, dim3(qgrid.x + p->n, qgrid.y), dim3(256), 0, stream, a, *p);
+            if (p && a.t <= QG_TOK) {
+                hipLaunchKernelGGL(fused_qb_big_kernel, dim3(a.n * MQH / 128 + p->n), dim3(256), 0, stream, a, *p);
             } else {
                 const int cols = (a.n * MQH + 255) / 256, qcols = p ? (p->n + 1) / 2 : 0, stages = a.r / GT_KI8;
-                if (a.t <= BIG_T2)
-                    hipLaunchKernelGGL(mla_qb_big_kernel<QB_DEPTH>, qgrid, dim3(256), 0, stream, a);
-                else if (p)
+                if (p)
                     gt_dispatch(gt_token_blocks(a.t, cols + qcols, stages, 7), [&](auto tb) {
                         constexpr int TB = decltype(tb)::value < 7 ? decltype(tb)::value : 7;
                         hipLaunchKernelGGL(fused_qb_wide_kernel<TB>, dim3((qcols + cols) * ((a.t + 32 * TB - 1) / (32 * TB))), dim3(GT_LANES), 0, stream,

@@ -164,6 +164,15 @@ def test_prefill_index_query_tiles(cuda, t, n, r, h):
     check_against_oracle(mla_case, idx_case, fused)
 
 
+@pytest.mark.parametrize("t,n", [(128, 6), (129, 6), (160, 64), (193, 2), (256, 2)])
+def test_products_around_the_narrow_tiles_limit(cuda, t, n):
+    # up to 128 tokens tiles of 128 outputs, above of 256 with a remainder of one token, half a tile (two heads) and whole tiles
+    mla_case, idx_case = op.make_fused_case(t, 1, 64, seed=80 + n, n_idx=64, h=256, q_lora_rank=128, n=n)
+    fused = run_fused(mla_case, idx_case, cuda, entry="mla_indexer_prolog_quant_p")
+    same_as_separate(fused, run_separate(mla_case, idx_case, cuda), idx_case)
+    check_against_oracle(mla_case, idx_case, fused)
+
+
 @pytest.mark.parametrize("t,n", [(775, 64), (1447, 16), (1762, 8)])
 def test_prefill_products_in_two_launches(cuda, t, n):
     # shapes where one launch over both int8 products would take a round of workgroups more than one for each
