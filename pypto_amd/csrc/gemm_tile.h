@@ -59,12 +59,16 @@ __device__ __forceinline__ void gt_copy(const void* base, uint32_t offset, uint8
                  : "memory");
 }
 
-// all but the last N of this wave's copies have landed, and with the barrier everybody's
+// All but the last N of this wave's copies have landed and all of its LDS reads are done, and with the barrier everybody's.  The
+// wait for the reads is written out: gt_product_i8's and gt_product_bf16's last reads of a stage are used behind this barrier
+// only, and what is copied right behind it goes into the buffer that they read.  Left to __syncthreads, the compiler drops that
+// wait where the reads come over the loop's back edge (12 to 14 of them were outstanding at the barrier).  They were issued a
+// half stage of matrix instructions before: no time.
 template <int N>
 __device__ __forceinline__ void gt_landed()
 {
     static_assert(N < 64, "the counter's six bits");
-    __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | (N >> 4 << 14)); // vmcnt(N)
+    __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | (N >> 4 << 14)); // vmcnt(N) lgkmcnt(0)
     __syncthreads();
 }
 
