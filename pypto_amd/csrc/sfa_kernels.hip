@@ -176,7 +176,8 @@ __device__ __forceinline__ void gather_tile(RawTile<QUANT>& t, const SfaArgs& a,
 // times the scale, both exact (scales up to 2^103), rounds once, like the product x * s that the golden rounds.  (A
 // conversion per element instead of one byte permute for two costs a quarter more instructions.)  In 35 pieces: a piece is the permute of one
 // pair, the fmas of the pair before and the packing of the one before that, because a wave issues a vector instruction
-// that depends on the one ahead of it at half the rate of an independent one.
+// that depends on the one ahead of it at half the rate of an independent one.  A share with a scale from 2^104 on, where 2^24
+// times the scale overflows and the product with an int8 need not, is stored once more by plain_share.
 constexpr int PIECES = 35;
 template <bool QUANT>
 struct Production {
@@ -189,6 +190,7 @@ struct Production {
     float f0, f1;
     uint32_t pk[4];
     uint32_t at;      // LDS address of this lane's first chunk, stage included
+    bool large;       // uniform: some scale of the share is 2^104 or more
 
     __device__ __forceinline__ void begin(const RawTile<QUANT>& r, uint32_t present, uint32_t stage, int pair, int lane)
     {
@@ -198,6 +200,7 @@ struct Production {
             if (present != 0xffffffffu) { // (an absent row is stored as zeros)
                 if (!((present >> (8 * pair + (lane & 7))) & 1u)) v = 0.f;
             }
+            large = __any(fabsf(v) >= 0x1p104f);
             from = 4 * (4 * (lane >> 5) + (lane & 24));
             fetch_scale<0>();
             // rows t = 8 pair + 4 (lane / 32) + k, chunks 2 (lane % 32) and the next: swz(t) is swz(t - k) ^ 4 (k / 2)
@@ -247,6 +250,27 @@ struct Production {
         }
     }
 };
+
+// The int8 columns of a wave's share by the plain product, from memory: r points at the share's eight rows.
+__device__ __forceinline__ void plain_share(const SfaArgs& a, const int* r, uint32_t present, uint8_t* stage, int pair, int lane)
+{
+    lane = fresh(lane);
+#pragma unroll 1
+    for (int e = 0; e < 8; ++e) {
+        const int t = 8 * pair + e;
+        const uint32_t row = (uint32_t)r[e];
+        const u32x2 x = *reinterpret_cast<const u32x2*>(a.kn + lane * 8 + (uint64_t)row * a.kn_stride);
+        const float sc = *reinterpret_cast<const float*>(a.ks + (lane >> 4) * 4 + (uint64_t)row * a.ks_stride);
+        const float s = (present >> t) & 1u ? sc : 0.f;
+        uint32_t pk[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int w = (int)(x[k >> 1] >> (k & 1 ? 16 : 0));
+            pk[k] = pack_bf16x2((float)(int8_t)w * s, (float)(int8_t)(w >> 8) * s);
+        }
+        *reinterpret_cast<u32x4*>(stage + t * KROW + ((lane ^ swz(t)) << 4)) = u32x4{pk[0], pk[1], pk[2], pk[3]};
+    }
+}
 
 // A workgroup's share of a token's top-k list: tiles [tile0, tile0 + ntiles) of the first `cur` entries.
 struct SplitRange {
@@ -686,6 +710,8 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
                 STEP_FENCE();
             });
             gather_rope<QUANT>(raw, row1, a, lane);
+            if constexpr (QUANT)
+                if (__builtin_expect(prod.large, false)) plain_share(a, rows + tile * T + 8 * pair, present, smem + stage, pair, lane);
         };
         u32x4 p, p1;
         const uint8_t* pb;

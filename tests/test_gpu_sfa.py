@@ -169,6 +169,25 @@ def test_tiles_without_a_present_entry(cuda, dead):
         full_check(run_with_splits(dict(case, topk_indices=tk), cuda, splits), ref, f"absent {dead}, {splits} splits")
 
 
+@pytest.mark.parametrize("power", [108, 110, 111, 112])
+def test_scales_whose_fast_dequantisation_overflows(cuda, power):
+    """Cache scales around 2^104, from where the dequantisation's 2^24 times the scale is infinite and the values are not: with the
+    nope query divided by the same power of two every score is the same and every output exactly that power larger.  Scales of
+    0.005 to 0.02: none of 2^104 or more, some and all, in tiles with absent entries too.  (Query values below 2^-6 are set to
+    zero, so that all are normal bf16 after the division.)"""
+    case = osfa.make_case(3, 40, 1, [300, 64, 33], topk=128, block_size=32, seed=41, dist="bench", softmax_scale=192 ** -0.5)
+    case["topk_indices"][0, 5:40:3] = -1
+    case["kn_scales"][::5, 1] *= -1
+    nope = case["q"][..., :512]
+    nope[nope.abs() < 2.0 ** -6] = 0
+    ref = run_with_splits(case, cuda, 1)
+    large = dict(case, q=case["q"].clone(), kn_scales=case["kn_scales"] * 2.0 ** power)
+    large["q"][..., :512] = (nope.float() * 2.0 ** -power).to(torch.bfloat16)
+    out = run_with_splits(large, cuda, 1)
+    assert torch.isfinite(out).all()
+    assert torch.equal(out.double(), ref.double() * 2.0 ** power)
+
+
 def test_forced_kv_splits_agree(cuda):
     """Drives the C ABI directly: 1, 2, 4 and 16 KV splits of the same problem."""
     from pypto_amd import _runtime
