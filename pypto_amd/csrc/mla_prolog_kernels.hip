@@ -22,7 +22,7 @@
 //                    key's rotary embedding, the three cache writes, q_norm / q_norm_scale
 //   mla_qb_kernel    int8 MFMA GEMM q_norm @ w_uq_qr, 128 outputs x 32 tokens per workgroup, weights streamed to LDS
 //                    (gemm_tile.h); dequantisation and the query's rotary embedding on the tile
-//   mla_wuk_kernel   per (head, 128 outputs): q_b[:, head, :128] @ w_uk[head]; above 64 tokens per head (mla_wuk_wide_kernel)
+//   mla_wuk_kernel   per (head, 128 outputs): q_b[:, head, :128] @ w_uk[head]; for many tokens or heads per head (mla_wuk_wide_kernel)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -980,7 +980,8 @@ __global__ __launch_bounds__(GT_LANES, 2) void fused_qb_wide_kernel(MlaPrologArg
 }
 
 // ------------------------------------------------------------------------------------------------ q_b[:, head, :128] @ w_uk[head]
-// Up to 32 TB tokens (TB 1 or 2), grid (heads, 512 / 128), 256 lanes: wave w owns outputs [32 w, 32 w + 32) of the tile.
+// Tiles of 32 TB tokens (TB 1 or 2) x 128 outputs, one to a workgroup: grid (heads, 512 / 128, token tiles), 256 lanes; wave w owns
+// outputs [32 w, 32 w + 32) of the tile.
 template <int TB>
 __global__ __launch_bounds__(256) void mla_wuk_kernel(MlaPrologArgs a)
 {
@@ -991,7 +992,7 @@ __global__ __launch_bounds__(256) void mla_wuk_kernel(MlaPrologArgs a)
     __shared__ __align__(16) uint8_t ot[WTOK * OROW]; // the outputs
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, hl = lane >> 5;
-    const int head = blockIdx.x, ct = blockIdx.y;
+    const int head = blockIdx.x, ct = blockIdx.y, tok0 = blockIdx.z * WTOK;
     const uint16_t* src = a.w_uk + (int64_t)head * MNOPE * MC + ct * 128;
     // the operand rows: WTOK tokens x 256 bytes, fetched once by the workgroup in 16-byte pieces (16 lanes per row) and
     // handed to the waves through LDS - a wave loading its own operand would fetch a different row with every lane pair,
@@ -1000,7 +1001,7 @@ __global__ __launch_bounds__(256) void mla_wuk_kernel(MlaPrologArgs a)
     u32x4 q[2 * TB];
 #pragma unroll
     for (int i = 0; i < 2 * TB; ++i)
-        q[i] = *reinterpret_cast<const u32x4*>(a.qb_nope + ((int64_t)min(prow + 16 * i, a.t - 1) * a.n + head) * MNOPE + 8 * pcol);
+        q[i] = *reinterpret_cast<const u32x4*>(a.qb_nope + ((int64_t)min(tok0 + prow + 16 * i, a.t - 1) * a.n + head) * MNOPE + 8 * pcol);
 #pragma unroll
     for (int i = tid; i < MNOPE * 16; i += 256) {
         const int k = i >> 4, c = i & 15;
@@ -1041,19 +1042,24 @@ __global__ __launch_bounds__(256) void mla_wuk_kernel(MlaPrologArgs a)
 #pragma unroll
     for (int i = 0; i < 2 * TB; ++i) {
         const int tok = prow + 16 * i;
-        if (tok < a.t)
-            *reinterpret_cast<u32x4*>(a.q_nope + ((int64_t)tok * a.n + head) * MC + ct * 128 + 8 * pcol) =
+        if (tok0 + tok < a.t)
+            *reinterpret_cast<u32x4*>(a.q_nope + ((int64_t)(tok0 + tok) * a.n + head) * MC + ct * 128 + 8 * pcol) =
                 *reinterpret_cast<const u32x4*>(ot + tok * OROW + 16 * pcol);
     }
 }
 
-// The same product above 64 tokens, with the same sums in the same order.  Bound by the outputs' way to memory (1501 tokens x 128
+// The same product for more tiles than WUK_TILES, with the same sums in the same order.  Bound by the outputs' way to memory (1501 tokens x 128
 // heads: 197 MB out, 49 in, 47 us at the rate of a large copy).  By tiles of 64 tokens x 128 outputs, two workgroups to a CU with
 // the weights in LDS, every tile's rows were read four times over and a tile passed two barriers: 65 us.  So a workgroup of 512
 // lanes owns a head's whole 512 outputs and walks the token tiles of 64, z of them side by side (z: one workgroup to a CU); wave w
 // owns outputs [64 w, +64), whose weights stay in its registers (64 a lane) and whose outputs leave through LDS of its own; a
 // tile's rows are in one of two buffers, and one barrier ends it.  Call of 1501 tokens 236.7 -> 224.5 us, 300: 81.7 -> 77.2, 128:
-// 56.4 -> 54.7; at 64 tokens, a single tile for half as many waves, 48.9 -> 49.4, so not there.  grid (heads, z), 512 lanes.
+// 56.4 -> 54.7; at 64 tokens, a single tile for half as many waves, 48.9 -> 49.4, so not there.
+// Where the tiles of 128 outputs all fit side by side, two workgroups to a CU, they are the faster ones: a workgroup here starts
+// with four times their weights.  The kernel, wide and by tiles: 16 heads x 128 tokens 5.6 us and 4.1, 512: 6.4 / 5.8, 1024: 8.1 /
+// 9.3; 64 heads x 128 tokens 6.8 / 6.2, 192: 7.4 / 8.4; 128 heads x 65 tokens 7.7 / 10.2 (256 heads 15.1 / 16.8).
+// grid (heads, z), 512 lanes.
+constexpr int WUK_TILES = 2 * 256;
 constexpr int WW_TOK = 64;
 __global__ __launch_bounds__(512, 2) void mla_wuk_wide_kernel(MlaPrologArgs a)
 {
@@ -1286,13 +1292,13 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
     if ((e = hipGetLastError()) != hipSuccess) return e;
     {
         ScopedKernelTimer tm(KID_MLA_WUK, stream);
-        if (a.t > WW_TOK) {
-            const int wtiles = (a.t + WW_TOK - 1) / WW_TOK, zdim = std::min(wtiles, std::max(1, 256 / a.n));
-            hipLaunchKernelGGL(mla_wuk_wide_kernel, dim3(a.n, zdim), dim3(512), 0, stream, a);
-        } else if (big)
-            hipLaunchKernelGGL(mla_wuk_kernel<2>, dim3(a.n, MC / 128), dim3(256), 0, stream, a);
-        else
+        const int wtiles = (a.t + WW_TOK - 1) / WW_TOK;
+        if (!big)
             hipLaunchKernelGGL(mla_wuk_kernel<1>, dim3(a.n, MC / 128), dim3(256), 0, stream, a);
+        else if (wtiles == 1 || (int64_t)a.n * (MC / 128) * wtiles <= WUK_TILES)
+            hipLaunchKernelGGL(mla_wuk_kernel<2>, dim3(a.n, MC / 128, wtiles), dim3(256), 0, stream, a);
+        else
+            hipLaunchKernelGGL(mla_wuk_wide_kernel, dim3(a.n, std::min(wtiles, std::max(1, 256 / a.n))), dim3(512), 0, stream, a);
     }
     return hipGetLastError();
 }

@@ -233,10 +233,11 @@ def test_prefill_query_tiles(cuda, t, n):
     check(case, run(case, cuda, entry="mla_prolog_quant_p"))
 
 
-@pytest.mark.parametrize("t,n", [(64, 4), (65, 4), (127, 128), (193, 2), (193, 128), (193, 258)])
+@pytest.mark.parametrize("t,n", [(64, 4), (65, 4), (127, 128), (193, 2), (193, 128), (193, 258), (256, 32), (257, 32), (127, 64), (129, 64)])
 def test_prefill_absorbed_tiles(cuda, t, n):
-    # q_nope @ w_uk above 64 tokens: tiles of 64 tokens with remainders of one to all rows, one tile to a workgroup, two, and (258 heads: more
-    # than workgroups that fit side by side) all of them
+    # q_nope @ w_uk by tiles of 64 tokens with remainders of one to all rows: up to 512 tiles x 128 outputs a workgroup each (256 x 32
+    # and 127 x 64 the last ones), beyond a head's tiles to workgroups of its own: one each, two, and (258 heads: more than workgroups
+    # that fit side by side) all of them
     case = op.make_case(t, 1, 64, seed=60 + t, h=256, q_lora_rank=128, n=n)
     check(case, run(case, cuda, entry="mla_prolog_quant_p"))
 
