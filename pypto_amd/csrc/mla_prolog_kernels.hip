@@ -681,22 +681,33 @@ __device__ __forceinline__ void mla_qb_body(const MlaPrologArgs& a, int tile, ui
 
 // Decode batches: while the norms' few workgroups go through their chains, the rest of the chip has nothing to do, and the
 // next launch starts with a stream of weights.  The workgroups from `first` on (a multiple of eight: workgroups go to the XCDs
-// round-robin) read the head of the slice that the workgroup of the same number past `first` streams next (bf16 form, 24 tokens:
-// 41.5 us a call without, 41.3 / 40.8 / 40.5 with 32 / 64 / 96 KB of a slice; int8, 2 tokens: 30.1, 29.7 / 29.3 / 29.2).
-constexpr int TOUCH_BYTES = 96 * 1024; // of a slice: 32 workgroups of an XCD leave a quarter of its 4 MB L2
+// round-robin) read the head of the slice that the workgroup of the same number past `first` streams next, `bytes` of it.
+//
+// How much: what an XCD's slices come to has to stay in its 4 MB L2 beside all else, and has to be there when the norms are done.
+// 96 KB of each slice, however many there are, took longer than none from about 250 slices on.  Weights out of HBM (six sets
+// in turn), us a call with none / 96 KB / 2 MB to an XCD: int8, 8 tokens, 128 heads 33.8 / 33.5 / 33.2, 192: 45.8 / 47.1 / 45.9,
+// 256: 48.0 / 51.5 / 47.9; bf16, 32 tokens, 144 heads 46.2 / 47.0 / 46.5, 256: 65.2 / 67.9 / 64.8; fused, 8 tokens, 144 heads
+// 47.9 / 48.6 / 47.0, 256: 52.4 / 55.9 / 52.3.  The fused operator's norms take longer; to 256 slices they cover 3 MB (128 heads,
+// 1 token 36.4, 35.5 with 3 MB, 36.0 with 2; 64 heads 33.8 / 32.3).
+constexpr int TOUCH_BYTES = 96 * 1024; // of a slice, at most: touch_rows' registers
+inline int touch_bytes(int slices, bool fused)
+{
+    const int xcd = fused && slices <= 256 ? 3 << 20 : 2 << 20;
+    return std::min(TOUCH_BYTES, xcd / ((slices + 7) / 8));
+}
 
-__device__ __forceinline__ void mla_touch(const MlaPrologArgs& a, int tile)
+__device__ __forceinline__ void mla_touch(const MlaPrologArgs& a, int tile, int bytes)
 {
     const int64_t stride = (int64_t)a.n * MQH * (a.quant ? 1 : 2);
     const int pieces = a.quant ? 8 : 16; // 128 outputs (the half tile that the bf16 form may end with is not asked for)
-    const int rows = min(a.r, TOUCH_BYTES / (16 * pieces)) & ~31;
+    const int rows = min(a.r, bytes / (16 * pieces)) & ~31;
     touch_rows(static_cast<const uint8_t*>(a.w_uq_qr) + (int64_t)tile * 16 * pieces, stride, rows, pieces);
 }
 
 // grid (2 x tokens: query, key | TOUCH: touching workgroups from `first` on), 256 lanes.  Without them (above 32 tokens) 40 registers
 // instead of 98, all of a token's chain that a SIMD can hold.
 template <int S, bool TOUCH>
-__global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a, int first)
+__global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a, int first, int touch)
 {
     const int id = blockIdx.x;
     if (id < a.t)
@@ -704,7 +715,7 @@ __global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a, int firs
     else if (id < 2 * a.t)
         mla_norm_key_body<S>(a, id - a.t);
     else if constexpr (TOUCH) {
-        if (id >= first) mla_touch(a, id - first);
+        if (id >= first) mla_touch(a, id - first, touch);
     }
 }
 
@@ -910,7 +921,7 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb_wide_kernel(MlaPrologArgs 
 // grid (3 x tokens: the MLA norms, the indexer's key path and weights (128 lanes) | TOUCH: touching workgroups from `first` on),
 // 256 lanes
 template <int S, bool TOUCH>
-__global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, PrologArgs p, int first)
+__global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, PrologArgs p, int first, int touch)
 {
     const int id = blockIdx.x;
     if (id < m.t)
@@ -923,9 +934,9 @@ __global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, Prolog
     } else if (TOUCH && id >= first) {
         const int tile = id - first, nqb = m.n * MQH / 128;
         if (tile < nqb)
-            mla_touch(m, tile);
+            mla_touch(m, tile, touch);
         else
-            touch_rows(reinterpret_cast<const uint8_t*>(p.w_qb) + (int64_t)(tile - nqb) * PD, (int64_t)p.n * PD, min(p.r, TOUCH_BYTES / PD) & ~31, 8);
+            touch_rows(reinterpret_cast<const uint8_t*>(p.w_qb) + (int64_t)(tile - nqb) * PD, (int64_t)p.n * PD, min(p.r, touch / PD) & ~31, 8);
     }
 }
 
@@ -1237,14 +1248,16 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         // all partial sums of an output in flight at once for the usual seven splits and fewer, none of them twice for one or two
         const int in_flight = a.ksplits <= 2 ? 2 : a.ksplits <= 4 ? 4 : 8;
         const int norms = (p ? 3 : 2) * a.t, first = (norms + 7) / 8 * 8;
-        const unsigned grid = big ? norms : first + a.n * MQH / 128 + (p ? p->n : 0); // (the kernels above BIG_T tokens do not wait for their weights)
+        const int slices = a.n * MQH / 128 + (p ? p->n : 0), bytes = touch_bytes(slices, p != nullptr);
+        const bool ahead = !big && bytes >= 32 * 256; // (32 rows; the kernels above BIG_T tokens do not wait for their weights)
+        const unsigned grid = ahead ? first + slices : norms;
         auto launch = [&](auto splits, auto touch) {
             constexpr int S = decltype(splits)::value;
             constexpr bool TOUCH = decltype(touch)::value;
             if (p)
-                hipLaunchKernelGGL((fused_norm_kernel<S, TOUCH>), dim3(grid), dim3(256), 0, stream, a, *p, first);
+                hipLaunchKernelGGL((fused_norm_kernel<S, TOUCH>), dim3(grid), dim3(256), 0, stream, a, *p, first, bytes);
             else
-                hipLaunchKernelGGL((mla_norm_kernel<S, TOUCH>), dim3(grid), dim3(256), 0, stream, a, first);
+                hipLaunchKernelGGL((mla_norm_kernel<S, TOUCH>), dim3(grid), dim3(256), 0, stream, a, first, bytes);
         };
         auto launch_with = [&](auto touch) {
             if (in_flight == 2)
@@ -1254,10 +1267,10 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
             else
                 launch(std::integral_constant<int, 8>{}, touch);
         };
-        if (big)
-            launch_with(std::false_type{});
-        else
+        if (ahead)
             launch_with(std::true_type{});
+        else
+            launch_with(std::false_type{});
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
     {

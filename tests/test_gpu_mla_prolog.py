@@ -249,6 +249,13 @@ def test_bf16_form_prefill_tiles(cuda, t, n):
     check_bf16_form(case, run(case, cuda))
 
 
+@pytest.mark.parametrize("n,quant_b", [(130, True), (172, True), (258, True), (172, False), (258, False)])
+def test_decode_batches_of_many_heads(cuda, n, quant_b):
+    # the norms' launch reads 85, 60, 41 KB of each slice of the query weights ahead: parts of 512 rows and all of them
+    case = op.make_case(3, 1, 64, seed=90, h=256, q_lora_rank=512, n=n, quant_b=quant_b)
+    (check if quant_b else check_bf16_form)(case, run(case, cuda))
+
+
 @pytest.mark.parametrize("quant_b", [True, False])
 def test_a_tokens_bits_do_not_depend_on_the_batch(cuda, quant_b):
     """Up to 32 tokens and from 33 on other kernels form the products; below 128 tokens their fp32 sums are the same (chains of 128
