@@ -821,14 +821,18 @@ __device__ __forceinline__ void order_words(const uint64_t (&w)[PER], uint32_t m
     // bitonic sort, descending, two words per lane and 2048 words.  A compare-exchange step of stride <= 64 stays inside
     // the 128 words owned by one wavefront (lane i of wave w handles the pair (128w + 2i - i%stride, + stride)),
     // so only the steps of stride >= 128 need a workgroup barrier; the others rely on LDS operations of one
-    // wavefront completing in order.
+    // wavefront completing in order.  The wait for them in front of the barrier that follows is written out: they come to it over
+    // the loops' back edges, and left to __syncthreads the compiler drops it.
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < PER; ++h) buf[tid + 1024 * h] = (uint32_t)(tid + 1024 * h) < m ? w[h] : 0ull;
     __syncthreads();
     for (int size = 2; size <= 1024 * PER; size <<= 1) {
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            if (stride >= 128) __syncthreads();
+            if (stride >= 128) {
+                __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0)
+                __syncthreads();
+            }
 #pragma unroll
             for (int q = 0; q < PER / 2; ++q) {
                 const int i = tid + 1024 * q;
