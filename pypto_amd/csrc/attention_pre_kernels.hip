@@ -40,7 +40,7 @@ constexpr int ATOK = 32;     // tokens per workgroup of apq_gemm_kernel
 constexpr int AMAX_H = 16384;
 
 // sum over the 256 lanes of a workgroup in a fixed order; red is 4 floats of LDS (in the lanes' own network: six dependent
-// permutes through LDS here and in apq_head_kernel were 0.45 us of a decode layer's 31.3)
+// permutes through LDS here and in apq_head_kernel were 0.4 us of the 12.1 of a call of 8 tokens x 14 heads)
 __device__ __forceinline__ float block_sum_256(float v, float* red, int tid)
 {
     v = wave_sum_descending(v);
@@ -297,11 +297,13 @@ __device__ __forceinline__ float add_rows16(float a, float b)
 // LDS 21 K, rotary pairs from an LDS tile with their cos and sin two loads at a time 15 K; now 20 K:
 //  - a quotient is two fused multiply-adds on the product with the reciprocal, which for a bf16 dividend gives the rounded
 //    quotient for every pair of mantissas (all 2^30 compared).  It needs that no step under- or overflows: positive scales of
-//    2^-60 to 2^60 (a value is 0 or a scale times 1 to 2^32) and divisors of 2^-20 to 2^100, or the wave divides;
+//    2^-60 to 2^60 (a value is 0 or a scale times 1 to 2^32) and divisors of 2^-20 to 2^100, or the wave divides.  (A divisor is
+//    the root of an fp32, below 2^64 where it is finite: the least quotient but 0 is above 2^-124, no subnormal);
 //  - pairs of rotary dims 16 or 32 apart are registers of one lane, whose cos and sin are loaded before the sums.  The half of a
 //    head that has none belongs to every second wave: the two waves of a SIMD get one of each (gt_wave_across);
 //  - each wave turns 16 tokens x 64 dims at a time into rows through LDS of its own and stores them while it goes on.
-// (777 tokens x 112 heads 82.4 -> 75.0 us a call, 1024 tokens 95.9 -> 88.9.)
+// (777 tokens x 112 heads 82.4 -> 75.0 us a call, 1024 tokens 95.9 -> 88.9.  Tiles of 256 tokens keep 4 registers in scratch memory
+// from there on; the product's loop has none.)
 // Other rotary widths have pairs in two waves or in broken pieces: the tile goes through LDS.
 // grid (heads / 2 rounded up, splits, token tiles), 512 lanes.
 template <int TB, bool WHOLE>

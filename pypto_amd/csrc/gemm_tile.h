@@ -37,7 +37,8 @@ constexpr int gt_lds_bytes(int tb) // of an int8 tile's stages
 template <int TB>
 struct GtTile {
     static constexpr int TOK = 32 * TB;             // tokens of the tile
-    static constexpr int QBYTES = TOK * 128;        // a stage in LDS: token rows | [2] weight rows, 128 bytes each
+    static constexpr int QBYTES = TOK * 128;        // a stage's token rows, 128 bytes each, and [2] weight rows: either
+                                                    // operand in a ring of its own
     static constexpr int WBYTES = 2 * 128 * 128, STAGE = QBYTES + WBYTES;
     // stages in LDS, one workgroup to a CU: two in flight, of the token rows above 160 tokens one (what LDS holds)
     static constexpr int WRING = 3, RING = 3 * STAGE <= 160 * 1024 ? 3 : 2;

@@ -726,8 +726,8 @@ __global__ __launch_bounds__(256) void mla_qb_kernel(MlaPrologArgs a)
     mla_qb_body(a, blockIdx.x, lds);
 }
 
-// The same product at 33 to 128 tokens beside the index heads' (fused_qb_big_kernel): a workgroup owns 128 tokens x 128 outputs and walks the
-// contraction in stages of 128 rows, both operands staged through LDS with the next stage's global loads in flight.  Wave
+// The same product at 33 to 128 tokens beside the index heads' (fused_qb_big_kernel): a workgroup owns all tokens x 128 outputs and walks
+// the contraction in stages of 128 rows, both operands staged through LDS with the next stage's global loads in flight.  Wave
 // (wr, wc) owns tokens [64 wr, +64) x outputs [64 wc, +64): every operand fragment read from LDS feeds four MFMAs.  The
 // int32 sums are exact, so the results are the bits of mla_qb_kernel's.  The outputs go through LDS (in place of the
 // operand tiles, which are no longer needed) so that they leave as the 128-byte runs they are in memory - a 128-column
@@ -738,10 +738,9 @@ constexpr int QG_QROW = QG_K + 16;       // bytes per LDS row of the [token][k] 
 constexpr int QG_OROW = 128 * 2 + 16;    // bytes per LDS row of the [token][128 outputs] bf16 tile
 constexpr int QG_STAGE_BYTES = QG_K * MQROW + QG_TOK * QG_QROW;
 static_assert(QG_TOK * QG_OROW <= QG_STAGE_BYTES, "the output tile takes the operand tiles' place");
-// DEPTH: stages whose loads are in flight (register sets used round-robin): the grid leaves at most two workgroups to a CU at
+// QB_DEPTH stages' loads are in flight (register sets used round-robin): the grid leaves at most two workgroups to a CU at
 // these sizes, and the twelve stages of a tile are otherwise twelve memory latencies in a row.
-template <int DEPTH>
-__device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0, int tok0, uint8_t* stage_lds)
+__device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0, uint8_t* stage_lds)
 {
 #pragma clang fp contract(off)
     // stage_lds: QG_STAGE_BYTES, [128 k][MQROW] weights | [128 tokens][QG_QROW] q_norm
@@ -757,8 +756,8 @@ __device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0
     const int8_t* wp = static_cast<const int8_t*>(a.w_uq_qr) + (int64_t)srow * nq + col0 + 16 * spc;
     const int8_t* qp[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) qp[i] = a.q_norm + (int64_t)min(tok0 + srow + 32 * i, a.t - 1) * r + 16 * spc;
-    u32x4 wst[DEPTH][4], qst[DEPTH][4];
+    for (int i = 0; i < 4; ++i) qp[i] = a.q_norm + (int64_t)min(srow + 32 * i, a.t - 1) * r + 16 * spc;
+    u32x4 wst[QB_DEPTH][4], qst[QB_DEPTH][4];
     auto load = [&](int st, int u) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) qst[u][i] = *reinterpret_cast<const u32x4*>(qp[i] + st * QG_K);
@@ -769,7 +768,7 @@ __device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0
     float qs_pre[4];
     f32x4 ws_pre[4];
 #pragma unroll
-    for (int tb = 0; tb < 4; ++tb) qs_pre[tb] = a.q_norm_scale[min(tok0 + 64 * wr + 16 * tb + l16, a.t - 1)];
+    for (int tb = 0; tb < 4; ++tb) qs_pre[tb] = a.q_norm_scale[min(64 * wr + 16 * tb + l16, a.t - 1)];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) ws_pre[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + col0 + 64 * wc + 16 * nb + 4 * g);
     i32x4 acc[4][4]; // [nb][tb]
@@ -778,10 +777,10 @@ __device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0
 #pragma unroll
         for (int tb = 0; tb < 4; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
 #pragma unroll
-    for (int u = 0; u < DEPTH; ++u) load(min(u, stages - 1), u);
-    for (int st0 = 0; st0 < stages; st0 += DEPTH) {
+    for (int u = 0; u < QB_DEPTH; ++u) load(min(u, stages - 1), u);
+    for (int st0 = 0; st0 < stages; st0 += QB_DEPTH) {
 #pragma unroll
-        for (int u = 0; u < DEPTH; ++u) {
+        for (int u = 0; u < QB_DEPTH; ++u) {
             if (st0 + u < stages) { // (uniform over the workgroup)
                 __syncthreads(); // everyone is done with the previous stage's tiles
     #pragma unroll
@@ -792,7 +791,7 @@ __device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0
                     *reinterpret_cast<u32x4*>(ql + (srow + 32 * i) * QG_QROW + 16 * spc) = qst[u][i];
                 }
                 __syncthreads();
-                load(min(st0 + u + DEPTH, stages - 1), u); // (unconditional: past the end the last stage is fetched again and dropped)
+                load(min(st0 + u + QB_DEPTH, stages - 1), u); // (unconditional: past the end the last stage is fetched again and dropped)
     #pragma unroll
                 for (int ks = 0; ks < QG_K / 64; ++ks) {
                     i32x4 qf[4], wf[4];
@@ -834,7 +833,7 @@ __device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0
                 const u32x2 pk = {(uint32_t)vb[0] | ((uint32_t)vb[1] << 16), (uint32_t)vb[2] | ((uint32_t)vb[3] << 16)};
                 *reinterpret_cast<u32x2*>(ot + tl * QG_OROW + cl * 2) = pk;
             } else {
-                const int64_t gtc = (int64_t)min(tok0 + tl, a.t - 1) * MROPE;
+                const int64_t gtc = (int64_t)min(tl, a.t - 1) * MROPE;
                 const uint16_t* cp = a.cos + gtc;
                 const uint16_t* snp = a.sin + gtc;
                 uint16_t* seg = reinterpret_cast<uint16_t*>(ot + tl * QG_OROW) + (cl - (d - MNOPE)); // the head's 64 rotary dims
@@ -855,10 +854,9 @@ __device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int pc = tid + 256 * i, tl = pc >> 4, sg = (pc >> 3) & 1, c = pc & 7;
-        const int gt = tok0 + tl;
-        if (gt >= a.t) continue;
+        if (tl >= a.t) continue;
         const int col = col0 + 64 * sg, head = col / MQH, d0 = col % MQH;
-        uint16_t* dst = d0 < MNOPE ? a.qb_nope + ((int64_t)gt * a.n + head) * MNOPE + d0 : a.q_rope + ((int64_t)gt * a.n + head) * MROPE;
+        uint16_t* dst = d0 < MNOPE ? a.qb_nope + ((int64_t)tl * a.n + head) * MNOPE + d0 : a.q_rope + ((int64_t)tl * a.n + head) * MROPE;
         *reinterpret_cast<u32x4*>(dst + 8 * c) = *reinterpret_cast<const u32x4*>(ot + tl * QG_OROW + (64 * sg + 8 * c) * 2);
     }
 }
@@ -962,7 +960,7 @@ __global__ __launch_bounds__(256, 2) void fused_qb_big_kernel(MlaPrologArgs m, P
     __shared__ __align__(16) uint8_t lds[QB_LDS_BYTES];
     const int nqb = m.n * MQH / 128;
     if ((int)blockIdx.x < nqb)
-        mla_qb_big_body<QB_DEPTH>(m, blockIdx.x * 128, 0, lds);
+        mla_qb_big_body(m, blockIdx.x * 128, lds);
     else
         prolog_q_big_body<QB_DEPTH>(p, blockIdx.x - nqb, 0, lds);
 }

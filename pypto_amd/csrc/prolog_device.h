@@ -118,7 +118,8 @@ __device__ __forceinline__ void prolog_q_quantise(const PrologArgs& a, int head,
         uint32_t pk[4];
 #pragma unroll
         for (int e4 = 0; e4 < 4; ++e4) {
-            uint32_t r[4]; // at most 127: behind 1.5 * 2^23 the low byte is the value rounded to even (0 of a NaN)
+            uint32_t r[4]; // at most 127: behind 1.5 * 2^23 the low byte is the value rounded to even (0 of a NaN, and of an infinity by a scale
+                           // that a maximum below 2^-121 makes infinite: the golden's bytes)
 #pragma unroll
             for (int e = 0; e < 4; ++e) r[e] = __builtin_bit_cast(uint32_t, y[tb][4 * e4 + e] * sq + 12582912.f);
             pk[e4] = __builtin_amdgcn_perm(r[1], r[0], 0x0c0c0400u) | __builtin_amdgcn_perm(r[3], r[2], 0x04000c0cu);
@@ -437,7 +438,7 @@ __device__ __forceinline__ void transpose_rows(uint32_t (&out)[4][2], const u32x
     }
 }
 
-// Above 256 tokens: 32 TB tokens x two heads per workgroup (gemm_tile.h), four waves to a head behind the product; the
+// Above 128 tokens: 32 TB tokens x two heads per workgroup (gemm_tile.h), four waves to a head behind the product; the
 // operations are prolog_q_big_body's, so are the bits (51 us at 1501 tokens there).  512 lanes; an odd last head is taken twice
 // and dropped.
 // Nothing covers what follows the product, which at 192 tokens x 1536 rows took 33 K ticks beside the product's 30 K: rotary pairs

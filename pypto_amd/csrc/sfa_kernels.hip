@@ -69,7 +69,8 @@ constexpr int LDS_LIMIT = 160 * 1024;
 constexpr int OUT_ROW = DN * 2;  // epilogue staging: 128 heads x 512 values of 16 bits, reusing the front of LDS
 constexpr int LSUM_OFF = ALPHA_OFF; // the epilogue's row sums [pair][32], where the rescale factors were
 constexpr int QROW = KROW;       // start-up staging of Q: 128 heads x 1152 bytes
-constexpr int BT_MAX = 2048;     // entries of a page table that is looked up in LDS
+constexpr int BT_MAX = 2048;     // entries of a page table that is looked up in LDS (a wider one is read from memory, out of the L2: 24
+                                 // tokens of 50 to 56 K contexts, 1750 entries each in LDS or 3500 in memory, 36.0 us a call either way)
 static_assert(HEADS_PER_WG * QROW <= SPLIT_OFF && HEADS_PER_WG * OUT_ROW <= LSUM_OFF && BT_MAX * 4 <= SPLIT_OFF, "what uses the front of LDS ends below the per-split arrays");
 __host__ __device__ constexpr int tmask_bytes(int cap) { return (cap / T + 2) * 4; }
 __host__ __device__ constexpr int split_bytes(int cap) { return tmask_bytes(cap) + cap * 4; }
@@ -78,7 +79,6 @@ static_assert(SPLIT_OFF + split_bytes(MAX_SPLIT_TOKENS) <= LDS_LIMIT, "a whole t
 
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
@@ -820,8 +820,8 @@ __global__ void sfa_zero_kernel(uint32_t* out, int64_t n_words)
 
 // out[row, :] = sum_s (2^(m_s - M) l_s / L) o_s[row, :] with L = sum_s 2^(m_s - M) l_s and o_s the split's normalised
 // output.  The partials lie in the fragment order the attention kernel's accumulators have (see its epilogue).  One
-// workgroup merges, for one token, what wave wv of the attention workgroups left for head block hb: 32 heads x 128
-// value columns; its wavefront i takes column block i, a lane owning for its head (l32) the four 4-column runs at
+// workgroup merges, for one token, what the attention workgroups left for column group wv / 2, head half wv % 2 and head
+// block hb: 32 heads x 128 value columns; its wavefront i takes column block i, a lane owning for its head (l32) the four 4-column runs at
 // 32 i + 16 h + 8 g + 4 hl.  Splits are taken G at a time (G = 2, 4 or 8: the smallest that covers the split count,
 // eight for more than eight splits), every load of a group requested before any is used (splits past the last are the
 // last again with weight 0).  The workgroup then turns its 32 x 128 block through LDS
