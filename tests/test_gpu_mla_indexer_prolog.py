@@ -145,7 +145,7 @@ def test_prefill_entry_ragged_tiles_small_sizes(cuda):
 def test_prefill_sizes_fused_equals_separate_and_oracle(cuda):
     # 128 tokens and more: the first product of both calls runs the kernel that owns an output tile, and so does the
     # separate call's int8 product (exact, so still the fused call's bits)
-    # (up to 256 tokens the two int8 products of the fused call share a launch, above they are launches of their own)
+    # (the two int8 products of the fused call always share a launch; above 128 tokens that of the wide tiles)
     for b, seed in ((150, 24), (300, 25)):
         mla_case, idx_case = op.make_fused_case(b, 1, 300, seed=seed, n_idx=64, h=1280, q_lora_rank=256, n=4)
         fused = run_fused(mla_case, idx_case, cuda, entry="mla_indexer_prolog_quant_p")
@@ -173,9 +173,10 @@ def test_products_around_the_narrow_tiles_limit(cuda, t, n):
     check_against_oracle(mla_case, idx_case, fused)
 
 
-@pytest.mark.parametrize("t,n", [(775, 64), (1447, 16), (1762, 8)])
-def test_prefill_products_in_two_launches(cuda, t, n):
-    # shapes where one launch over both int8 products would take a round of workgroups more than one for each
+@pytest.mark.parametrize("t,n", [(257, 64), (775, 64), (1447, 16), (1762, 8), (961, 64), (1793, 64)])
+def test_index_head_tiles_ahead_of_the_query_tiles(cuda, t, n):
+    # one launch holds the index heads' tiles of all token tiles (32 each), then the query product's (48, 12 or 6 each): three to
+    # twelve token tiles of 128, 160 (three shapes), 192 and 224 tokens, the last of 135, 7, 2 tokens or one
     mla_case, idx_case = op.make_fused_case(t, 1, 64, seed=80 + n, n_idx=64, h=256, q_lora_rank=128, n=n)
     fused = run_fused(mla_case, idx_case, cuda, entry="mla_indexer_prolog_quant_p")
     same_as_separate(fused, run_separate(mla_case, idx_case, cuda), idx_case)
