@@ -268,6 +268,71 @@ __device__ __forceinline__ void gt_stream_i8(i32x4 (&acc)[2][2], const int8_t* w
         });
 }
 
+// 33 to 160 tokens x 128 outputs, 512 lanes: a stream of weights still, all tokens beside them, three or more stages in flight.  Wave (wr, wc) owns tokens [16 TT wr,
+// +16 TT) x two blocks of 16 outputs 32 apart, gt_batch_block(wc, nb): what a rotary embedding pairs is in one lane.  Register e of
+// acc[nb][tb]: output 16 gt_batch_block + 4 g + e, token 16 TT wr + 16 tb + l16.
+template <int TT>
+struct GtBatch {
+    static constexpr int TOK = 32 * TT, QBYTES = TOK * 128, STAGE = QBYTES + 128 * 128, FIT = 160 * 1024 / STAGE, RING = FIT < 6 ? FIT : 6, LDS = RING * STAGE;
+};
+__device__ __forceinline__ int gt_batch_block(int wc, int nb) { return (wc & 1) + 2 * nb + 4 * (wc >> 1); }
+template <int TT>
+__device__ __forceinline__ void gt_batch_i8(i32x4 (&acc)[2][TT], const int8_t* w, int64_t ldw, const int8_t* q, int64_t ldq, int t, int stages,
+                                            uint8_t* lds)
+{
+    using T = GtBatch<TT>;
+    const int lane = threadIdx.x & 63, wave = gt_wave();
+    const int l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
+    // copies of a wave: token rows 64 i + 8 w + lane / 8 (the last rows again where eight waves have more hands than rows), weight rows alike
+    const int row = 8 * wave + (lane >> 3), pos = lane & 7;
+    constexpr int QC = (TT + 1) / 2;
+    uint32_t qo[QC], wo[2];
+    int qd[QC];
+#pragma unroll
+    for (int i = 0; i < QC; ++i) {
+        const int c = min(8 * i + wave, 4 * TT - 1), qrow = 8 * c + (lane >> 3);
+        qd[i] = 1024 * c;
+        qo[i] = (uint32_t)(min(qrow, t - 1) * (int)ldq + 16 * (pos ^ ((qrow >> 1) & 7)));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) wo[i] = (uint32_t)((row + 64 * i) * (int)ldw + 16 * (pos ^ (((row >> 1) & 3) | ((row >> 2) & 4))));
+    const uint8_t* qr = lds + (16 * TT * wr + l16) * 128;
+    const int qpos = 16 * (g ^ ((l16 >> 1) & 7));
+    const uint8_t* wrow = lds + T::QBYTES + (16 * g + (l16 >> 1)) * 128 + 8 * (l16 & 1);
+    int wpos[2]; // (transposing reads: see gt_product_i8)
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) wpos[nb] = 16 * (gt_batch_block(wc, nb) ^ (((l16 >> 2) & 3) | ((g & 1) << 2)));
+    gt_stages<T::RING, T::STAGE, QC + 2>(
+        stages,
+        [&](int st, int b) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) gt_copy(w + (int64_t)st * GT_KI8 * ldw, wo[i], lds + b + T::QBYTES + 8192 * i + 1024 * wave);
+#pragma unroll
+            for (int i = 0; i < QC; ++i) gt_copy(q + st * GT_KI8, qo[i], lds + b + qd[i]);
+        },
+        [&](int, int b) {
+            i32x4 qf[2][TT], wf[2][2];
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) {
+                    const uint8_t* p = wrow + b + 8192 * ks + wpos[nb];
+                    const v2i lo = lds_read_tr8(p), hi = lds_read_tr8(p + 1024);
+                    wf[ks][nb] = i32x4{lo[0], lo[1], hi[0], hi[1]};
+                }
+#pragma unroll
+                for (int tb = 0; tb < TT; ++tb) qf[ks][tb] = *reinterpret_cast<const i32x4*>(qr + b + 2048 * tb + (qpos ^ (64 * ks)));
+            }
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int tb = 0; tb < TT; ++tb)
+#pragma unroll
+                    for (int nb = 0; nb < 2; ++nb)
+                        acc[nb][tb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[ks][nb], qf[ks][tb], acc[nb][tb], 0, 0, 0);
+        });
+}
+
 // The same loop in bf16 for 128 tokens x 256 outputs, the outputs in four blocks of 64 columns at src[i], ld[i] values a row;
 // x: [t, ldx], column of the first contraction row.  Wave (wr, wc) owns tokens [64 wr, +64) x block wc.  Register e of
 // sum[tb][nb]: token 64 wr + 32 tb + 8 (e / 4) + 4 hl + e % 4, column 32 nb + lane % 32 of the block.  Sums are chains of at most

@@ -45,10 +45,9 @@ constexpr int XA_K = 256;         // contraction rows per stage of mla_xa_kernel
 constexpr int XA_SPLIT = 1024;    // contraction rows per workgroup of mla_xa_kernel (one fp32 partial sum each)
 constexpr int XROW2 = 64 * 2 + 16; // bytes per LDS row of a [k][64] bf16 weight tile (padded against bank conflicts)
 constexpr int TROW = 128 * 2 + 32; // bytes per LDS row of a [k][128] bf16 weight tile (padded against bank conflicts)
-constexpr int MQROW = 136;         // bytes per LDS row of a [k][128] int8 weight tile (padded, 8-byte aligned)
-constexpr int BIG_T = 33;         // token count from which the kernels that own an output tile take over: the others read the
-                                  // weights once per 32 tokens (fused prolog, 33 tokens: 63.6 against 47.2 us, 96: 87 / 55, 127:
-                                  // 108 / 59; 24 tokens: 43.6 / 46.8)
+constexpr int BIG_T = 33;         // token count from which the kernels that hold more than 32 tokens take over: the others read the
+                                  // weights once per 32 tokens (fused prolog, 32 tokens 32.0 us and 33: 33.0; with the weights read
+                                  // twice 63.6)
 constexpr int BIG_T2 = 256;       // token count above which the x product's tiles are 256 outputs wide, in splits of its own
 
 // 32 outputs x 32 tokens += W[KSTEPS steps of 16 rows, outputs]^T . X[tokens, k]: A by transposing reads of the [k][n]
@@ -166,102 +165,94 @@ __global__ __launch_bounds__(1024) void mla_xa_kernel(MlaPrologArgs a)
     xa_body(a.x, a.h, a.h, src, ld, a.xa_part, a.ncols, blockIdx.y * 64, blockIdx.x, blockIdx.z * MTOK, a.t, xa_lds);
 }
 
-// The same product at 33 to 256 tokens: a workgroup owns an output tile of 128 tokens x 64 columns
-// over one 1024-row split of the contraction and walks it in stages of 64 rows, both operands staged through LDS, so
-// that the weights are read once per 128 tokens instead of once per 32 and a token row's piece is fetched by 8
-// neighbouring lanes as one 128-byte run.  The global loads of BG_DEPTH stages are in flight at any time (register
-// sets used round-robin): a stage's multiplication takes a few hundred nanoseconds and a load comes back after one to
-// two microseconds, so with one stage ahead the sixteen stages of a split were sixteen memory latencies in a row
-// (29 us at 512 tokens with 256 x 64 tiles; a 256 x 128 tile that halves the operand traffic but leaves one
-// workgroup per CU was slower still: 33 us).  Wave w owns tokens [32 w, +32) x the 64 columns.  x is the A operand here,
-// so a result register holds one token's value for 32 consecutive columns across the lanes and the partial sums leave
-// as 128-byte runs.  grid (splits, output tiles of 64, token tiles), 256 lanes.
-constexpr int BG_KS = 64;               // contraction rows per stage
-constexpr int BG_XROW = BG_KS * 2 + 16; // bytes per LDS row of the [token][k] tile (padded against bank conflicts)
-// DEPTH: stages whose loads are in flight.  CHAINS: sums are chains of 128 rows added up in order, which are mla_xa_kernel's
-// sums bit for bit (a decode step's selection can hang on the last bit of a score, so batches that cross the kernels' border
-// see the same numbers); otherwise one chain of a split's rows.  (With chains two workgroups to a CU: the grid has no more
-// below 128 tokens, and three leave too few registers.)
-template <int DEPTH, bool CHAINS>
-__global__ __launch_bounds__(256, CHAINS ? 2 : 3) void mla_xa_big_kernel(MlaPrologArgs a)
+// The same product at 33 to 256 tokens: a workgroup owns all tokens x 64 columns over one 1024-row split of the contraction and
+// streams it in stages of 64 rows straight to LDS (gemm_tile.h), so that the weights are read once.  x is the A operand here, so a
+// result register holds one token's value for 32 consecutive columns across the lanes and the partial sums leave as 128-byte runs.
+// The sums are chains of 128 rows added up in order, which are mla_xa_kernel's bit for bit (a decode step's selection can hang on
+// the last bit of a score, so batches that cross the kernels' border see the same numbers).
+// What bounds it: the weights' stream (34 MB, 6.5 us), and from some 100 tokens on what 252 workgroups draw of x from the L2 (2 KB a
+// token and split each, 10 TB/s).  Tiles of 128 tokens through registers, four stages of loads in flight and two barriers a stage,
+// took 13.3 us at 40 tokens and 20.9 at 160 (two tiles); so 10.4 and 16.0.  Call of the fused prolog, with mla_qb_batch_kernel's
+// change: 33 tokens 40.1 -> 33.0 us, 64: 42.7 -> 34.6, 96: 45.5 -> 40.3, 128: 47.0 -> 45.2, 160: 58.3 -> 53.1, 256: 66.9 -> 64.7.
+// grid (splits, output tiles of 64), 512 lanes: up to four blocks of 32 tokens wave w owns block w / 2 x 32 columns, above block w x 64.
+constexpr int XB_KS = 64; // contraction rows per stage
+template <int TT>
+__global__ __launch_bounds__(512, 2) void mla_xa_batch_kernel(MlaPrologArgs a)
 {
-    constexpr int TOK = 128;
-    static_assert((XA_SPLIT / BG_KS) % DEPTH == 0 && XA_K % (BG_KS * DEPTH) == 0, "whole rounds of stages in every split");
-    __shared__ __align__(16) uint8_t wt[BG_KS * XROW2];
-    __shared__ __align__(16) uint8_t xt[TOK * BG_XROW];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int XBYTES = TT * 32 * 128, STAGE = XBYTES + XB_KS * 128, FIT = 160 * 1024 / STAGE, RING = FIT < 8 ? FIT : 8;
+    constexpr int NB = TT <= 4 ? 1 : 2, XC = (TT + 1) / 2;
+    static_assert(XA_K % (2 * XB_KS) == 0, "whole chains of 128 rows in every split");
+    __shared__ __align__(16) uint8_t lds[RING * STAGE];
+    const int lane = threadIdx.x & 63, wave = gt_wave();
     const int l32 = lane & 31, hl = lane >> 5, jj = lane & 15, mh = (lane >> 4) & 1;
     int ld;
     const uint16_t* src = xa_source(a, blockIdx.y, ld);
-    const int split = blockIdx.x, tok0 = blockIdx.z * TOK, col0 = blockIdx.y * 64;
-    const int kbeg = split * XA_SPLIT;
-    const int stages = (min(a.h, kbeg + XA_SPLIT) - kbeg) / BG_KS; // a multiple of DEPTH (h is one of 256)
-    const int srow = tid >> 3, spc = tid & 7;
-    const uint16_t* xp[4];
+    const int split = blockIdx.x, kbeg = split * XA_SPLIT, stages = (min(a.h, kbeg + XA_SPLIT) - kbeg) / XB_KS;
+    const uint16_t* x = a.x + kbeg;
+    src += (int64_t)kbeg * ld;
+    // copies of a wave (layout and exchange of the pieces: gemm_tile.h): token rows 64 i + 8 w + lane / 8 (the last rows again where
+    // eight waves have more hands than rows), weight rows 8 w + lane / 8
+    const int row = 8 * wave + (lane >> 3), pos = lane & 7;
+    uint32_t xo[XC];
+    int xd[XC];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) xp[i] = a.x + (int64_t)min(tok0 + srow + 32 * i, a.t - 1) * a.h + kbeg + 8 * spc;
-    const uint16_t* wp = src + (int64_t)(kbeg + srow) * ld + 8 * spc;
-    u32x4 xs[DEPTH][4], ws[DEPTH][2];
-    auto load = [&](int st, int u) {
+    for (int i = 0; i < XC; ++i) {
+        const int c = min(8 * i + wave, 4 * TT - 1), xrow = 8 * c + (lane >> 3);
+        xd[i] = 1024 * c;
+        xo[i] = (uint32_t)(min(xrow, a.t - 1) * a.h * 2 + 16 * (pos ^ ((xrow >> 1) & 7)));
+    }
+    const uint32_t wo = (uint32_t)(row * ld * 2 + 16 * (pos ^ ((row << 1) & 4)));
+    const int tb = TT <= 4 ? wave >> 1 : wave, nb0 = TT <= 4 ? wave & 1 : 0;
+    const bool busy = tb < TT; // (the barriers are everybody's)
+    const uint8_t* xr = lds + (32 * (busy ? tb : 0) + l32) * 128;
+    const int xf = (l32 >> 1) & 7;
+    const uint8_t* wrow = lds + XBYTES + (8 * hl + (jj >> 2)) * 128 + 8 * (jj & 1);
+    const int wpos = 16 * ((4 * nb0 + 2 * mh + ((jj >> 1) & 1)) ^ ((jj >> 1) & 4));
+    f32x16 acc[NB], sum[NB];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) xs[u][i] = *reinterpret_cast<const u32x4*>(xp[i] + st * BG_KS);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) ws[u][i] = *reinterpret_cast<const u32x4*>(wp + (int64_t)(st * BG_KS + 32 * i) * ld);
-    };
-    f32x16 acc[2], sum[2];
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[nb][e] = sum[nb][e] = 0.f;
-    const uint8_t* xr = xt + (32 * wave + l32) * BG_XROW + 16 * hl;
-    const uint8_t* hp = wt + (8 * hl + (jj >> 2)) * XROW2 + (16 * mh + 4 * (jj & 3)) * 2;
+    gt_stages<RING, STAGE, XC + 1>(
+        stages,
+        [&](int st, int b) {
+            gt_copy(src + (int64_t)st * XB_KS * ld, wo, lds + b + XBYTES + 1024 * wave);
 #pragma unroll
-    for (int u = 0; u < DEPTH; ++u) load(u, u);
-    for (int st0 = 0; st0 < stages; st0 += DEPTH) {
+            for (int i = 0; i < XC; ++i) gt_copy(x + st * XB_KS, xo[i], lds + b + xd[i]);
+        },
+        [&](int st, int b) {
+            if (!busy) return;
+            bf16x8 xv[XB_KS / 16], wv[XB_KS / 16][NB];
 #pragma unroll
-        for (int u = 0; u < DEPTH; ++u) {
-            __syncthreads(); // everyone is done with the previous stage's tiles
+            for (int ks = 0; ks < XB_KS / 16; ++ks) {
+                xv[ks] = *reinterpret_cast<const bf16x8*>(xr + b + 16 * ((2 * ks + hl) ^ xf));
 #pragma unroll
-            for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(xt + (srow + 32 * i) * BG_XROW + 16 * spc) = xs[u][i];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(wt + (srow + 32 * i) * XROW2 + 16 * spc) = ws[u][i];
-            __syncthreads();
-            load(min(st0 + u + DEPTH, stages - 1), u); // (unconditional: past the end the last stage is fetched again and dropped)
-#pragma unroll
-            for (int ks = 0; ks < BG_KS / 16; ++ks) {
-                bf16x8 wf[2];
-                const bf16x8 xf = *reinterpret_cast<const bf16x8*>(xr + ks * 32);
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb) {
-                    const s16x4 lo = lds_read_tr(hp + 64 * nb + ks * 16 * XROW2);
-                    const s16x4 hi = lds_read_tr(hp + 64 * nb + (ks * 16 + 4) * XROW2);
-                    wf[nb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-                }
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, wf[nb], acc[nb], 0, 0, 0);
-            }
-            if constexpr (CHAINS) {
-                if (u % (128 / BG_KS) == 128 / BG_KS - 1) {
-#pragma unroll
-                    for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-                        for (int e = 0; e < 16; ++e) {
-                            sum[nb][e] += acc[nb][e];
-                            acc[nb][e] = 0.f;
-                        }
+                for (int nb = 0; nb < NB; ++nb) {
+                    const uint8_t* p = wrow + b + 2048 * ks + (wpos ^ (64 * nb));
+                    const s16x4 lo = lds_read_tr(p), hi = lds_read_tr(p + 512);
+                    wv[ks][nb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
                 }
             }
-        }
-    }
-    if constexpr (!CHAINS) sum[0] = acc[0], sum[1] = acc[1];
-    // register e of sum[nb]: token 32 w + 8 (e / 4) + 4 hl + e % 4, column 32 nb + lane % 32
+#pragma unroll
+            for (int ks = 0; ks < XB_KS / 16; ++ks)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv[ks], wv[ks][nb], acc[nb], 0, 0, 0);
+            if (st & 1) {
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) sum[nb][e] += acc[nb][e], acc[nb][e] = 0.f;
+            }
+        });
+    if (!busy) return;
+    // register e of sum[nb]: token 32 tb + 8 (e / 4) + 4 hl + e % 4, column 32 (nb0 + nb) + lane % 32
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-        const int gt = tok0 + 32 * wave + 8 * (e >> 2) + 4 * hl + (e & 3);
-        if (gt >= a.t) continue;
-        float* out = a.xa_part + ((int64_t)split * a.t + gt) * a.ncols + col0 + l32;
+        const int tok = 32 * tb + 8 * (e >> 2) + 4 * hl + (e & 3);
+        if (tok >= a.t) continue;
+        float* out = a.xa_part + ((int64_t)split * a.t + tok) * a.ncols + blockIdx.y * 64 + 32 * nb0 + l32;
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) out[32 * nb] = sum[nb][e];
+        for (int nb = 0; nb < NB; ++nb) out[32 * nb] = sum[nb][e];
     }
 }
 
@@ -310,22 +301,22 @@ static int xa_wide_rows(int64_t t, int64_t h, int64_t r)
 }
 
 // Four blocks of 64 outputs of q_b, TOK tokens each, from LDS rows of QBS_ROW bytes (padded against bank conflicts) to memory in
-// 16-byte pieces: a block is half of a head's 128 first dims, or its rotary dims, rotated on the way.  Two waves to a block (two
-// blocks: 256 lanes).
+// 16-byte pieces: a block is half of a head's 128 first dims, or its rotary dims, rotated on the way.  PER lanes to a block (two waves: two
+// blocks in 256 lanes).
 constexpr int QBS_ROW = 64 * 2 + 16;
-template <int TOK>
+template <int TOK, int PER = 128>
 __device__ __forceinline__ void qb_store_blocks(const MlaPrologArgs& a, const uint8_t* lds, int block0, int tok0)
 {
 #pragma clang fp contract(off)
     const int tid = threadIdx.x, blocks = a.n * MQH / 64;
-    const int bl = tid >> 7, block = block0 + bl, head = block / 3; // two waves to a block
+    const int bl = tid / PER, block = block0 + bl, head = block / 3;
     if (block >= blocks) return;
     const uint8_t* tile = lds + bl * TOK * QBS_ROW;
     if (block % 3 < 2) { // 8 pieces of 8 dims
         uint16_t* dst = a.qb_nope + head * MNOPE + block % 3 * 64 + 8 * (tid & 7);
 #pragma unroll
-        for (int i = 0; i < TOK / 16; ++i) {
-            const int tl = ((tid >> 3) & 15) + 16 * i;
+        for (int i = 0; i < TOK * 8 / PER; ++i) {
+            const int tl = (tid % PER >> 3) + PER / 8 * i;
             if (tok0 + tl < a.t)
                 *reinterpret_cast<u32x4*>(dst + (int64_t)(tok0 + tl) * a.n * MNOPE) =
                     *reinterpret_cast<const u32x4*>(tile + tl * QBS_ROW + 16 * (tid & 7));
@@ -333,9 +324,9 @@ __device__ __forceinline__ void qb_store_blocks(const MlaPrologArgs& a, const ui
     } else { // 4 times 8 pairs, rotated into the two halves
         const int i0 = 8 * (tid & 3);
 #pragma unroll
-        for (int i = 0; i < TOK / 32; ++i) {
-            const int tl = ((tid >> 2) & 31) + 32 * i, gt = tok0 + tl;
-            if (gt >= a.t) continue;
+        for (int i = 0; i < (TOK * 4 + PER - 1) / PER; ++i) {
+            const int tl = (tid % PER >> 2) + PER / 4 * i, gt = tok0 + tl;
+            if (tl >= TOK || gt >= a.t) continue;
             const u32x4* x = reinterpret_cast<const u32x4*>(tile + tl * QBS_ROW + 4 * i0);
             const uint16_t* cp = a.cos + (int64_t)gt * MROPE + i0;
             const uint16_t* sp = a.sin + (int64_t)gt * MROPE + i0;
@@ -726,144 +717,9 @@ __global__ __launch_bounds__(256) void mla_qb_kernel(MlaPrologArgs a)
     mla_qb_body(a, blockIdx.x, lds);
 }
 
-// The same product at 33 to 128 tokens beside the index heads' (fused_qb_big_kernel): a workgroup owns all tokens x 128 outputs and walks
-// the contraction in stages of 128 rows, both operands staged through LDS with the next stage's global loads in flight.  Wave
-// (wr, wc) owns tokens [64 wr, +64) x outputs [64 wc, +64): every operand fragment read from LDS feeds four MFMAs.  The
-// int32 sums are exact, so the results are the bits of mla_qb_kernel's.  The outputs go through LDS (in place of the
-// operand tiles, which are no longer needed) so that they leave as the 128-byte runs they are in memory - a 128-column
-// tile holds two 64-column segments, each either half of a head's 128 first dims or a head's 64 rotary dims, rotated
-// into place on the way.  256 lanes.
-constexpr int QG_TOK = 128, QG_K = 128;
-constexpr int QG_QROW = QG_K + 16;       // bytes per LDS row of the [token][k] int8 tile (padded against bank conflicts)
-constexpr int QG_OROW = 128 * 2 + 16;    // bytes per LDS row of the [token][128 outputs] bf16 tile
-constexpr int QG_STAGE_BYTES = QG_K * MQROW + QG_TOK * QG_QROW;
-static_assert(QG_TOK * QG_OROW <= QG_STAGE_BYTES, "the output tile takes the operand tiles' place");
-// QB_DEPTH stages' loads are in flight (register sets used round-robin): the grid leaves at most two workgroups to a CU at
-// these sizes, and the twelve stages of a tile are otherwise twelve memory latencies in a row.
-__device__ __forceinline__ void mla_qb_big_body(const MlaPrologArgs& a, int col0, uint8_t* stage_lds)
-{
-#pragma clang fp contract(off)
-    // stage_lds: QG_STAGE_BYTES, [128 k][MQROW] weights | [128 tokens][QG_QROW] q_norm
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int l16 = lane & 15, g = lane >> 4, wr = wave >> 1, wc = wave & 1;
-    const int r = a.r;
-    const int64_t nq = (int64_t)a.n * MQH;
-    uint8_t* wl = stage_lds;
-    uint8_t* ql = stage_lds + QG_K * MQROW;
-    const int stages = r / QG_K;
-    // 128 rows x 128 bytes of either operand per stage = 4 pieces of 16 bytes per lane (rows tid / 8 + 32 i, piece tid % 8)
-    const int srow = tid >> 3, spc = tid & 7;
-    const int8_t* wp = static_cast<const int8_t*>(a.w_uq_qr) + (int64_t)srow * nq + col0 + 16 * spc;
-    const int8_t* qp[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) qp[i] = a.q_norm + (int64_t)min(srow + 32 * i, a.t - 1) * r + 16 * spc;
-    u32x4 wst[QB_DEPTH][4], qst[QB_DEPTH][4];
-    auto load = [&](int st, int u) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) qst[u][i] = *reinterpret_cast<const u32x4*>(qp[i] + st * QG_K);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) wst[u][i] = *reinterpret_cast<const u32x4*>(wp + ((int64_t)st * QG_K + 32 * i) * nq);
-    };
-    // the epilogue's scales, requested first
-    float qs_pre[4];
-    f32x4 ws_pre[4];
-#pragma unroll
-    for (int tb = 0; tb < 4; ++tb) qs_pre[tb] = a.q_norm_scale[min(64 * wr + 16 * tb + l16, a.t - 1)];
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) ws_pre[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + col0 + 64 * wc + 16 * nb + 4 * g);
-    i32x4 acc[4][4]; // [nb][tb]
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb)
-#pragma unroll
-        for (int tb = 0; tb < 4; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
-#pragma unroll
-    for (int u = 0; u < QB_DEPTH; ++u) load(min(u, stages - 1), u);
-    for (int st0 = 0; st0 < stages; st0 += QB_DEPTH) {
-#pragma unroll
-        for (int u = 0; u < QB_DEPTH; ++u) {
-            if (st0 + u < stages) { // (uniform over the workgroup)
-                __syncthreads(); // everyone is done with the previous stage's tiles
-    #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    u32x2* d = reinterpret_cast<u32x2*>(wl + (srow + 32 * i) * MQROW + 16 * spc);
-                    d[0] = u32x2{wst[u][i][0], wst[u][i][1]};
-                    d[1] = u32x2{wst[u][i][2], wst[u][i][3]};
-                    *reinterpret_cast<u32x4*>(ql + (srow + 32 * i) * QG_QROW + 16 * spc) = qst[u][i];
-                }
-                __syncthreads();
-                load(min(st0 + u + QB_DEPTH, stages - 1), u); // (unconditional: past the end the last stage is fetched again and dropped)
-    #pragma unroll
-                for (int ks = 0; ks < QG_K / 64; ++ks) {
-                    i32x4 qf[4], wf[4];
-    #pragma unroll
-                    for (int tb = 0; tb < 4; ++tb)
-                        qf[tb] = *reinterpret_cast<const i32x4*>(ql + (64 * wr + 16 * tb + l16) * QG_QROW + ks * 64 + 16 * g);
-                    // (the byte-transposing read: see gt_product_i8)
-    #pragma unroll
-                    for (int nb = 0; nb < 4; ++nb) {
-                        const uint8_t* p = wl + (ks * 64 + 16 * g + (l16 >> 1)) * MQROW + 64 * wc + 16 * nb + 8 * (l16 & 1);
-                        const v2i lo = lds_read_tr8(p), hi = lds_read_tr8(p + 8 * MQROW);
-                        wf[nb] = i32x4{lo[0], lo[1], hi[0], hi[1]};
-                    }
-    #pragma unroll
-                    for (int nb = 0; nb < 4; ++nb)
-    #pragma unroll
-                        for (int tb = 0; tb < 4; ++tb)
-                            acc[nb][tb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[nb], qf[tb], acc[nb][tb], 0, 0, 0);
-                }
-            }
-        }
-    }
-    __syncthreads(); // the operand tiles are free: the output tile takes their place
-    // register e of acc[nb][tb]: output col0 + 64 wc + 16 nb + 4 g + e, token 64 wr + 16 tb + l16
-    uint8_t* ot = stage_lds;
-#pragma unroll
-    for (int tb = 0; tb < 4; ++tb) {
-        const int tl = 64 * wr + 16 * tb + l16;
-        const float qs = qs_pre[tb];
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-            const int cl = 64 * wc + 16 * nb + 4 * g; // column inside the tile
-            const int d = (col0 + cl) % MQH;
-            const f32x4 ws = ws_pre[nb];
-            uint16_t vb[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) vb[e] = f32_to_bf16(((float)acc[nb][tb][e] * qs) * ws[e]);
-            if (d < MNOPE) {
-                const u32x2 pk = {(uint32_t)vb[0] | ((uint32_t)vb[1] << 16), (uint32_t)vb[2] | ((uint32_t)vb[3] << 16)};
-                *reinterpret_cast<u32x2*>(ot + tl * QG_OROW + cl * 2) = pk;
-            } else {
-                const int64_t gtc = (int64_t)min(tl, a.t - 1) * MROPE;
-                const uint16_t* cp = a.cos + gtc;
-                const uint16_t* snp = a.sin + gtc;
-                uint16_t* seg = reinterpret_cast<uint16_t*>(ot + tl * QG_OROW) + (cl - (d - MNOPE)); // the head's 64 rotary dims
-#pragma unroll
-                for (int pr = 0; pr < 2; ++pr) {
-                    const int i = (d - MNOPE) / 2 + pr;
-                    const float xe = bf16_to_f32(vb[2 * pr]), xo = bf16_to_f32(vb[2 * pr + 1]);
-                    const float o1 = xe * bf16_to_f32(cp[i]) + (-xo) * bf16_to_f32(snp[i]);
-                    const float o2 = xo * bf16_to_f32(cp[i + 32]) + xe * bf16_to_f32(snp[i + 32]);
-                    seg[i] = f32_to_bf16(o1);
-                    seg[i + 32] = f32_to_bf16(o2);
-                }
-            }
-        }
-    }
-    __syncthreads();
-    // 128 tokens x 2 segments x 128 bytes = 8 pieces of 16 bytes per lane
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int pc = tid + 256 * i, tl = pc >> 4, sg = (pc >> 3) & 1, c = pc & 7;
-        if (tl >= a.t) continue;
-        const int col = col0 + 64 * sg, head = col / MQH, d0 = col % MQH;
-        uint16_t* dst = d0 < MNOPE ? a.qb_nope + ((int64_t)tl * a.n + head) * MNOPE + d0 : a.q_rope + ((int64_t)tl * a.n + head) * MROPE;
-        *reinterpret_cast<u32x4*>(dst + 8 * c) = *reinterpret_cast<const u32x4*>(ot + tl * QG_OROW + (64 * sg + 8 * c) * 2);
-    }
-}
-
-// From 33 tokens on, above 128 beside the index heads': 32 TB tokens x 256 outputs per workgroup (gemm_tile.h), the same exact sums
-// and the same operations behind them.  128 x 128 tiles through registers are bound by the operands' way into LDS: MLA prolog of 40
-// tokens 41.0 us a call against 38.8, 128: 50.0 / 48.5, 200: 66.2 / 57.2.
+// For more tokens than mla_qb_batch_kernel takes (qb_batch): 32 TB tokens x 256 outputs per workgroup (gemm_tile.h), the same exact
+// sums and the same operations behind them.  128 x 128 tiles through registers are bound by the operands' way into LDS: MLA prolog
+// of 200 tokens 66.2 us a call against 57.2.
 constexpr int mla_qb_wide_lds(int tb) // the product's stages, or four blocks of the output tile
 {
     const int tok = 32 * tb, ring = gt_lds_bytes(tb);
@@ -912,6 +768,50 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb_wide_kernel(MlaPrologArgs 
     mla_qb_wide_body<TB>(a, blockIdx.x, blockIdx.y * 32 * TB, lds);
 }
 
+// 33 to QB_BATCH_T tokens: 128 outputs per workgroup of 512 lanes, all tokens, the weights streamed (gt_batch_i8); the same exact sums
+// and the same operations behind them.  Its 192 workgroups at model sizes keep twice as many CUs at the weights as tiles of 256
+// outputs.  Call of 40 tokens 33.8 -> 30.6 us, 96: 37.9 -> 35.0, 160: 50.6 -> 46.4.
+template <int TT>
+__device__ __forceinline__ void mla_qb_batch_body(const MlaPrologArgs& a, int tile, uint8_t* lds)
+{
+#pragma clang fp contract(off)
+    using T = GtBatch<TT>;
+    static_assert(2 * T::TOK * QBS_ROW <= T::LDS, "the output tile takes the stages' place");
+    const int lane = threadIdx.x & 63, wave = gt_wave(), l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3, col0 = 128 * tile;
+    float qs[TT];
+    f32x4 ws[2];
+#pragma unroll
+    for (int tb = 0; tb < TT; ++tb) qs[tb] = a.q_norm_scale[min(16 * TT * wr + 16 * tb + l16, a.t - 1)];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + col0 + 16 * gt_batch_block(wc, nb) + 4 * g);
+    i32x4 acc[2][TT];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int tb = 0; tb < TT; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
+    gt_batch_i8<TT>(acc, static_cast<const int8_t*>(a.w_uq_qr) + col0, (int64_t)a.n * MQH, a.q_norm, a.r, a.t, a.r / GT_KI8, lds);
+#pragma unroll
+    for (int tb = 0; tb < TT; ++tb)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs[tb]) * ws[nb][e];
+            const int cb = gt_batch_block(wc, nb);
+            *reinterpret_cast<u32x2*>(lds + ((cb >> 2) * T::TOK + 16 * TT * wr + 16 * tb + l16) * QBS_ROW + (16 * (cb & 3) + 4 * g) * 2) =
+                u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        }
+    __syncthreads();
+    qb_store_blocks<T::TOK, 256>(a, lds, 2 * tile, 0);
+}
+// grid (n * 192 / 128), 512 lanes
+template <int TT>
+__global__ __launch_bounds__(GT_LANES, 2) void mla_qb_batch_kernel(MlaPrologArgs a)
+{
+    __shared__ __align__(16) uint8_t lds[GtBatch<TT>::LDS];
+    mla_qb_batch_body<TT>(a, blockIdx.x, lds);
+}
+
 // ------------------------------------------------------------------------------------------------ fused with the indexer prolog
 // The fused operator runs the two prologs' per-token kernels side by side in one launch, and likewise the two int8
 // GEMMs on q_norm (192 + 64 workgroups at model sizes: one per compute unit); the indexer's x @ [w_k | w_proj] rides along
@@ -950,22 +850,20 @@ __global__ __launch_bounds__(256) void fused_qb_kernel(MlaPrologArgs m, PrologAr
         prolog_q_stream_body(p, blockIdx.x - nqb, lds);
 }
 
-// The same pair at 33 to 128 tokens: both products side by side.  The indexer's epilogue sets the LDS (68 KB:
-// two workgroups to a CU), so both run with three stages of loads in flight.  With tiles of 256 outputs half as many workgroups have
-// the index heads' epilogue to hide: call of 64 tokens 47.9 us here, 48.5 there, 128: 54.1 / 55.4; 129: 66.7 / 63.9, 256: 75.1 / 70.0.
-// grid (n * 192 / 128 + index heads), 256 lanes
-__global__ __launch_bounds__(256, 2) void fused_qb_big_kernel(MlaPrologArgs m, PrologArgs p)
+// The same pair at 33 to QB_BATCH_T tokens.  The kernel at model sizes: 40 tokens 13.8 us, 96: 16.0, 128: 18.4, 160: 22.1; tiles of
+// 128 x 128 through registers, three stages of loads in flight and two barriers a stage, took 20.7 up to 128 tokens, tiles of 256
+// outputs 24.4 at 160.  grid (index heads + n * 192 / 128), 512 lanes
+template <int TT>
+__global__ __launch_bounds__(GT_LANES, 2) void fused_qb_batch_kernel(MlaPrologArgs m, PrologArgs p)
 {
-    static_assert(QB_LDS_BYTES >= QG_STAGE_BYTES && QB_TOK == QG_TOK, "one LDS block and one token tiling serve both bodies");
-    __shared__ __align__(16) uint8_t lds[QB_LDS_BYTES];
-    const int nqb = m.n * MQH / 128;
-    if ((int)blockIdx.x < nqb)
-        mla_qb_big_body(m, blockIdx.x * 128, lds);
+    __shared__ __align__(16) uint8_t lds[GtBatch<TT>::LDS];
+    if ((int)blockIdx.x < p.n) // (the index heads have the longer epilogue)
+        prolog_q_batch_body<TT>(p, blockIdx.x, lds);
     else
-        prolog_q_big_body<QB_DEPTH>(p, blockIdx.x - nqb, 0, lds);
+        mla_qb_batch_body<TT>(m, blockIdx.x - p.n, lds);
 }
 
-// Above 128 tokens the two products in one launch of gemm_tile.h's tiles: the index heads' part alone is half a round of workgroups
+// For more tokens than that (qb_batch) the two products in one launch of gemm_tile.h's tiles: the index heads' part alone is half a round of workgroups
 // up to 512 tokens (call of 257 tokens 83.0 us as two launches, 72.2 as one, 512: 104.4 / 96.3, 1024: 163.6 / 160.7, 1344: 211.5 /
 // 194.6, 4096: 604.7 / 591.0).  Its tiles are up to 224 tokens; where the query product's own of 256 save a round the two are the
 // same (900 tokens 153.9 / 154.0, 2048: 314.5 / 316.6).
@@ -1218,6 +1116,35 @@ static hipError_t set_lds_limits()
     });
 }
 
+// f(integral constant: blocks of 32 tokens) for 33 to 256 tokens
+template <class F>
+static void token_blocks(int t, F&& f)
+{
+    switch ((t + 31) / 32) {
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 5: f(std::integral_constant<int, 5>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    case 7: f(std::integral_constant<int, 7>{}); break;
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    default: f(std::integral_constant<int, 2>{}); break;
+    }
+}
+
+// The int8 products by workgroups of 128 outputs and all tokens: one round of workgroups to the CUs, one to a CU.  Alone to 160
+// tokens where they are one round (us a call, tiles of 256 outputs and these: 40 tokens, 16 heads 31.7 / 26.7, 160 heads 36.4 / 34.5,
+// 192: 37.8 / 41.7; 150 tokens, 16 heads 39.9 / 38.0, 160: 55.2 / 52.2, 192: 61.4 / 71.4; 128 heads, 192 tokens 50.9 / 50.7, 224:
+// 52.2 / 53.5).  Beside the index heads' up to 128 tokens (against 128 x 128 tiles, 96 tokens: 16 heads 39.6 / 35.5, 256 heads, two
+// rounds: 69.1 / 65.4), to 160 where 256 outputs leave the chip half empty and these fill it (150 tokens, 16 heads 45.7 / 46.4, 64:
+// 49.0 / 49.7, 192: 70.3 / 74.4; 160 tokens, 128 heads 58.3 / 55.9, 192 tokens: 61.9 / 61.7).
+constexpr int QB_BATCH_T = 160;
+static bool qb_batch(const MlaPrologArgs& a, const PrologArgs* p)
+{
+    const int slices = a.n * MQH / 128 + (p ? p->n : 0);
+    if (a.t > QB_BATCH_T) return false;
+    return p ? a.t <= 128 || (slices > 192 && slices <= 256) : slices <= 256;
+}
+
 // p == nullptr: the MLA prolog on its own; otherwise the fused operator (m and p bound by fused_prolog_bind)
 static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hipStream_t stream)
 {
@@ -1230,7 +1157,10 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         ScopedKernelTimer tm(KID_MLA_XA, stream);
         if (big)
             if (a.t <= BIG_T2)
-                hipLaunchKernelGGL((a.t < 128 ? mla_xa_big_kernel<4, true> : mla_xa_big_kernel<4, false>), dim3(a.ksplits, a.ncols / 64, (a.t + 127) / 128), dim3(256), 0, stream, a);
+                token_blocks(a.t, [&](auto tt) {
+                    constexpr int TT = decltype(tt)::value;
+                    hipLaunchKernelGGL(mla_xa_batch_kernel<TT>, dim3(a.ksplits, a.ncols / 64), dim3(512), 0, stream, a);
+                });
             else {
                 const int xtiles = (a.t + 127) / 128, ntiles = (a.ncols + 255) / 256, rows = xa_wide_rows(a.t, a.h, a.r);
                 if (a.ksplits != (a.h + rows - 1) / rows) return hipErrorInvalidValue;
@@ -1278,8 +1208,14 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         } else if (!a.quant) {
             hipLaunchKernelGGL(mla_qb16_kernel, dim3((a.n * MQH + 127) / 128), dim3(256), 0, stream, a);
         } else if (big) {
-            if (p && a.t <= QG_TOK) {
-                hipLaunchKernelGGL(fused_qb_big_kernel, dim3(a.n * MQH / 128 + p->n), dim3(256), 0, stream, a, *p);
+            if (qb_batch(a, p)) {
+                token_blocks(a.t, [&](auto tt) {
+                    constexpr int TT = decltype(tt)::value < QB_BATCH_T / 32 ? decltype(tt)::value : QB_BATCH_T / 32;
+                    if (p)
+                        hipLaunchKernelGGL(fused_qb_batch_kernel<TT>, dim3(a.n * MQH / 128 + p->n), dim3(GT_LANES), 0, stream, a, *p);
+                    else
+                        hipLaunchKernelGGL(mla_qb_batch_kernel<TT>, dim3(a.n * MQH / 128), dim3(GT_LANES), 0, stream, a);
+                });
             } else {
                 const int cols = (a.n * MQH + 255) / 256, qcols = p ? (p->n + 1) / 2 : 0, stages = a.r / GT_KI8;
                 if (p)

@@ -579,6 +579,79 @@ __device__ __forceinline__ void prolog_q_stream_body(const PrologArgs& a, int he
     __syncthreads();
     prolog_q_finish<1>(a, head, 0, tid, had, xt, reinterpret_cast<float(*)[PTOK]>(lds + PTOK * XROW));
 }
+
+// 33 to 160 tokens: one head per workgroup of 512 lanes behind the streamed product of all tokens; two groups of four waves to the
+// halves of the tokens behind it.  Rotary pairs are registers of a lane; hadamard_q, cos and sin come ahead of the stages.  lds: the stages, afterwards hadamard_q | bf16 tile | [2] per-wave maxima
+template <int TT>
+__device__ __forceinline__ void prolog_q_batch_body(const PrologArgs& a, int head, uint8_t* lds)
+{
+#pragma clang fp contract(off)
+    using T = GtBatch<TT>;
+    constexpr int HB = (TT + 1) / 2, HTOK = 32 * HB; // token blocks of a group
+    static_assert(PD * PD * 2 + 2 * HTOK * XROW + 2 * 4 * HTOK * 4 <= T::LDS, "the epilogue takes the stages' place");
+    const int tid = threadIdx.x, lane = tid & 63, wave = gt_wave(), l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
+    float qs[TT];
+    f32x4 ws[2];
+#pragma unroll
+    for (int tb = 0; tb < TT; ++tb) qs[tb] = a.q_norm_scale[min(16 * TT * wr + 16 * tb + l16, a.t - 1)];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + (int64_t)head * PD + 16 * gt_batch_block(wc, nb) + 4 * g);
+    u32x4 hadr[PD * PD * 2 / 16 / 512];
+#pragma unroll
+    for (int i = 0; i < PD * PD * 2 / 16 / 512; ++i) hadr[i] = reinterpret_cast<const u32x4*>(a.had_q)[tid + 512 * i];
+    // cos and sin of the rotary dims 16 wc + 4 g .. + 3 and the ones 32 on (waves 0 and 1 of a row)
+    u32x2 cs[TT][2], sn[TT][2];
+#pragma unroll
+    for (int tb = 0; tb < TT; ++tb)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int at = min(16 * TT * wr + 16 * tb + l16, a.t - 1) * PROPE + 32 * i + 16 * (wc & 1) + 4 * g;
+            cs[tb][i] = *reinterpret_cast<const u32x2*>(a.cos + at);
+            sn[tb][i] = *reinterpret_cast<const u32x2*>(a.sin + at);
+        }
+    i32x4 acc[2][TT];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int tb = 0; tb < TT; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
+    gt_batch_i8<TT>(acc, a.w_qb + head * PD, (int64_t)a.n * PD, a.q_norm, a.r, a.t, a.r / GT_KI8, lds);
+    uint8_t* xt = lds + PD * PD * 2;
+#pragma unroll
+    for (int tb = 0; tb < TT; ++tb) {
+        uint32_t y[2][2];
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs[tb]) * ws[nb][e];
+            y[nb][0] = pack_bf16x2(v[0], v[1]);
+            y[nb][1] = pack_bf16x2(v[2], v[3]);
+        }
+        if (wc < 2) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                float o[2][2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) { // (the arithmetic of rope_tile)
+                    const float x1 = half_of(y[0][i], e), x2 = half_of(y[1][i], e);
+                    o[0][e] = x1 * half_of(cs[tb][0][i], e) + (-x2) * half_of(sn[tb][0][i], e);
+                    o[1][e] = x2 * half_of(cs[tb][1][i], e) + x1 * half_of(sn[tb][1][i], e);
+                }
+                y[0][i] = pack_bf16x2(o[0][0], o[0][1]);
+                y[1][i] = pack_bf16x2(o[1][0], o[1][1]);
+            }
+        }
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+            *reinterpret_cast<u32x2*>(xt + (16 * TT * wr + 16 * tb + l16) * XROW + (16 * gt_batch_block(wc, nb) + 4 * g) * 2) = u32x2{y[nb][0], y[nb][1]};
+    }
+#pragma unroll
+    for (int i = 0; i < PD * PD * 2 / 16 / 512; ++i) reinterpret_cast<u32x4*>(lds)[tid + 512 * i] = hadr[i];
+    __syncthreads();
+    const int hs = tid >> 8; // (of an odd number of blocks the second group has one less: rows past the tile, dropped)
+    float(*smax)[HTOK] = reinterpret_cast<float(*)[HTOK]>(xt + 2 * HTOK * XROW + hs * 4 * HTOK * 4);
+    prolog_q_quantise<HB>(a, head, HTOK * hs, tid & 255, lds, xt + HTOK * hs * XROW, smax);
+}
 constexpr int PROLOG_BIG_T = 128;   // token count from which the query product runs per 128 tokens
 
 // ------------------------------------------------------------------------------------------------ key path, weights

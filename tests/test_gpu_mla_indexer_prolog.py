@@ -173,6 +173,16 @@ def test_products_around_the_narrow_tiles_limit(cuda, t, n):
     check_against_oracle(mla_case, idx_case, fused)
 
 
+@pytest.mark.parametrize("t,n", [(33, 6), (64, 6), (65, 2), (96, 128), (97, 6), (128, 258), (129, 128), (160, 96), (161, 96), (150, 64)])
+def test_streamed_products_of_33_to_160_tokens(cuda, t, n):
+    # token blocks of 32: two to five with remainders of one and all rows, the last head count of one round of workgroups and one past
+    # it (258 heads), and the tiles that take over
+    mla_case, idx_case = op.make_fused_case(t, 1, 64, seed=90 + n, n_idx=64, h=512, q_lora_rank=384, n=n)
+    fused = run_fused(mla_case, idx_case, cuda, entry="mla_indexer_prolog_quant_p")
+    same_as_separate(fused, run_separate(mla_case, idx_case, cuda), idx_case)
+    check_against_oracle(mla_case, idx_case, fused)
+
+
 @pytest.mark.parametrize("t,n", [(257, 64), (775, 64), (1447, 16), (1762, 8), (961, 64), (1793, 64)])
 def test_index_head_tiles_ahead_of_the_query_tiles(cuda, t, n):
     # one launch holds the index heads' tiles of all token tiles (32 each), then the query product's (48, 12 or 6 each): three to

@@ -268,6 +268,20 @@ def test_a_tokens_bits_do_not_depend_on_the_batch(cuda, quant_b):
         assert torch.equal(many[name][:32], few[name]), name
 
 
+@pytest.mark.parametrize("t,n,quant_b", [(33, 2, True), (65, 4, True), (97, 128, True), (129, 6, True), (160, 170, True), (160, 172, True),
+                                         (161, 6, True), (193, 2, True), (225, 2, True), (256, 4, True), (64, 4, False), (200, 4, False)])
+def test_streamed_products_have_the_bits_of_the_decode_kernels(cuda, t, n, quant_b):
+    """33 to 256 tokens: two to eight blocks of 32 with remainders of one and all rows; the x product over splits of 1024 and 256
+    rows, whose sums are the decode kernel's (chains of 128 rows, added up in order), the int8 product's are exact: the last tokens'
+    results are the bits of a call of those tokens alone."""
+    case = op.make_case(t, 1, 64, seed=170 + t, h=1280, q_lora_rank=768, n=n, quant_b=quant_b)
+    last = {k: v[-20:].contiguous() if k in ("x", "cos", "sin", "cache_index") else v for k, v in case.items()}
+    many, few = run(case, cuda), run(last, cuda)
+    for name in ("q_norm", "q_norm_scale", "q_nope", "q_rope"):
+        assert torch.equal(many[name][-20:], few[name]), name
+    (check if quant_b else check_bf16_form)(case, many, **({} if quant_b else {"outliers": 1e-4}))
+
+
 def test_bf16_form_reference_case_b4_s2(cuda):
     # the reference's test_b4_s64k2_pa_nd_bf16_d: no quantisation anywhere (empty dequant_scale, bf16 w_uq_qr and cache)
     case = op.make_case(4, 2, 1024, seed=18, quant_b=False)
