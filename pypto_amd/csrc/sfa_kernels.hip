@@ -14,9 +14,9 @@
 // once for all 128 heads.  The dequantised tile sits row-major in LDS (16-byte chunks XOR-swizzled with the row), three
 // tiles deep, and serves as K (row reads) and as V (transposing reads, ds_read_b64_tr_b16).  A SIMD holds a pair of
 // wavefronts, which owns 32 heads; the two do different work, so that one has vector and memory work to do while the other
-// issues MFMAs (v_mfma_f32_32x32x16_bf16):
-//   * the score wave holds Q (B operand, 30 of its 36 k-steps in registers, six parked in LDS), computes S^T = K Q^T over
-//     the whole contraction, runs the online softmax (one head per lane) and accumulates O^T = V^T P~ for the first 128
+// issues MFMAs (v_mfma_f32_16x16x32_bf16):
+//   * the score wave holds Q (B operand, 30 of its 36 fragments in registers, six parked in LDS), computes S^T = K Q^T over
+//     the whole contraction, runs the online softmax (two heads per lane) and accumulates O^T = V^T P~ for the first 128
 //     value columns, with P~ straight out of its registers: S^T comes out in the B-operand order of the values product;
 //   * the value wave produces the tiles - eight of the 32 rows each: gather into registers, dequantisation, store to LDS -
 //     with the matrix instructions of the other 384 value columns between the pieces; P~ and the rescale factors come to it
@@ -24,13 +24,15 @@
 // Between two barriers, one per tile: the scores and the softmax of tile i, the values of tile i - 1, the production of
 // tile i + 1 and the gather of tile i + 2.  Nothing is exchanged within a tile.
 //
-// What bounds it: nothing alone.  A tile takes 3450 ticks of a CU (1000 query tokens, 2048 rows each), of which the matrix
-// pipes are busy 2176, the vector ports about 2250 (380 instructions a SIMD and the matrix instructions' issue) and LDS
-// about 2100; the kernel before, whose eight wavefronts all went through the same phases between two barriers a tile,
-// took 5150.  Measured on the way: four wavefronts with 512 registers each, 32 heads and no pairs, 4170 (a single
-// wavefront's issue slots); eight of 16 heads with 16x16x32 instructions, 5460 (three operand fragments in flight are
-// too few); the value wave's products before or after its production 3660 and 3770, interleaved without its raised
-// priority 4060 (the older score wave takes every slot and then waits at the barrier).
+// What bounds it: where every CU has long lists (1000 query tokens, 2048 rows each), the chip's power.  Its clock falls to 1.65 GHz
+// there, from 2.35, and the time follows the energy of a tile more than its ticks: v_mfma_f32_16x16x32_bf16 adds up twice the
+// products per accumulator it reads and writes of v_mfma_f32_32x32x16_bf16, and takes 3900 ticks a tile here where that one took
+// 3580, but 546 us for the 1000 tokens instead of 572.  (Matrix instructions alone, out of registers, on random numbers: 1.82
+// PFLOP/s and 1.63; on zeros, at full clock, 2.3 either way.  Only the values in the one and the scores in the other: 572.)  Short
+// of that the issue of the two waves of a SIMD: a tile's values, scores and softmax take the score wave 0.8, 1.9 and 1.0 K ticks, the
+// production and the values the value wave 3.5 K; the matrix pipes are busy 2.3 K, LDS 2.0 K.  Not faster: the values between the
+// pieces of the softmax, or between the scores; more fragments ahead; the int8 shares' stores free of bank conflicts (LDS 1.8 K);
+// equal priorities (4700).
 //
 // KV splits write their output normalised by their own sum as fp16, in the accumulators' fragment order, plus (m, l);
 // sfa_combine_kernel merges them and turns the result into rows.
@@ -46,20 +48,20 @@ namespace {
 constexpr int T = 32;                  // selected rows per tile
 constexpr int DN = 512;                // nope / value width
 constexpr int DR = 64;                 // rope width
-constexpr int KSTEPS = (DN + DR) / 16; // 36 MFMA k-steps for S
+constexpr int KSTEPS = (DN + DR) / 32; // 18 MFMA k-steps for S
 constexpr int KROW = (DN + DR) * 2;    // 1152 bytes per tile row = 72 chunks of 16 bytes
 constexpr int STAGE = T * KROW;        // 36864
 constexpr int MAX_SPLIT_TOKENS = 2048; // largest share of a top-k list one workgroup may own
 constexpr int HEADS_PER_WG = 128;
 constexpr int WAVES = 8, PAIRS = 4;    // a pair of waves, one of each role, to 32 heads
-constexpr int NDB = DN / 32;           // 16 blocks of 32 value columns ...
-constexpr int NDB_S = 4;               // ... of which the score wave of a pair takes the first four
-// of the score wave's 36 k-steps of Q, every sixth is parked in LDS (16 bytes per lane each): what its 256 registers do not
-// hold beside its part of O and the scores
-constexpr int PARK_EVERY = 6, NPARK = KSTEPS / PARK_EVERY, NREG = KSTEPS - NPARK;
+constexpr int NDB = DN / 16;           // 32 blocks of 16 value columns ...
+constexpr int NDB_S = 8;               // ... of which the score wave of a pair takes the first eight
+// of the score wave's 36 fragments of Q (k-step, block of 16 heads), every sixth is parked in LDS (16 bytes per lane each): what its
+// 256 registers do not hold beside its part of O and the scores
+constexpr int QFRAGS = 2 * KSTEPS, PARK_EVERY = 6, NPARK = QFRAGS / PARK_EVERY, NREG = QFRAGS - NPARK;
 // LDS layout: three tile stages | parked Q | P~ [2][pair], 2 KB each | rescale factors [2][pair][32], flags [2][pair] |
-// per-split arrays sized by SfaArgs::split_cap (validity words, rows).  While the share is looked up, this sequence's page
-// table lies in front (when it fits); then the query, on its way to operand layout.
+// per-split arrays sized by SfaArgs::split_cap (validity words, rows).  At the start the query lies in front, on its way to operand
+// layout, and behind it this sequence's page table (when it fits), while the share is looked up.
 constexpr int QPARK_OFF = 3 * STAGE;
 constexpr int PBUF_OFF = QPARK_OFF + PAIRS * NPARK * 1024;
 constexpr int ALPHA_OFF = PBUF_OFF + 2 * PAIRS * 2048;
@@ -68,10 +70,12 @@ constexpr int SPLIT_OFF = FLAG_OFF + 2 * PAIRS * 4;
 constexpr int LDS_LIMIT = 160 * 1024;
 constexpr int OUT_ROW = DN * 2;  // epilogue staging: 128 heads x 512 values of 16 bits, reusing the front of LDS
 constexpr int LSUM_OFF = ALPHA_OFF; // the epilogue's row sums [pair][32], where the rescale factors were
-constexpr int QROW = KROW;       // start-up staging of Q: 128 heads x 1152 bytes
-constexpr int BT_MAX = 2048;     // entries of a page table that is looked up in LDS (a wider one is read from memory, out of the L2: 24
+// start-up: each pair's query in LDS of its own, [32 heads] x 1024 bytes of nope columns, then x 128 of rope columns; behind them
+// the page table
+constexpr int QPAIR = 32 * (DN + DR) * 2, BT_OFF = PAIRS * QPAIR;
+constexpr int BT_MAX = 1280;     // entries of a page table that is looked up in LDS (a wider one is read from memory, out of the L2: 24
                                  // tokens of 50 to 56 K contexts, 1750 entries each in LDS or 3500 in memory, 36.0 us a call either way)
-static_assert(HEADS_PER_WG * QROW <= SPLIT_OFF && HEADS_PER_WG * OUT_ROW <= LSUM_OFF && BT_MAX * 4 <= SPLIT_OFF, "what uses the front of LDS ends below the per-split arrays");
+static_assert(HEADS_PER_WG * OUT_ROW <= LSUM_OFF && BT_OFF + BT_MAX * 4 <= SPLIT_OFF && BT_OFF % 16 == 0, "what uses the front of LDS ends below the per-split arrays");
 __host__ __device__ constexpr int tmask_bytes(int cap) { return (cap / T + 2) * 4; }
 __host__ __device__ constexpr int split_bytes(int cap) { return tmask_bytes(cap) + cap * 4; }
 static_assert(QPARK_OFF % 16 == 0 && SPLIT_OFF % 16 == 0, "16-byte LDS accesses");
@@ -88,10 +92,9 @@ __device__ __forceinline__ s16x4 lds_read_tr(uint8_t* p) { return __builtin_amdg
 
 // Chunk swizzle of tile row t.  A row is 32 banks more than a multiple of the 64, so rows of one parity share their
 // banks.  A b128 read serves 16 lanes at a time, 16 rows in the scores' K fragments: the eight rows of a parity need eight
-// different values.  A transposing read serves 32 lanes, 64 bytes of four rows: two neighbouring rows of a parity need
-// different values of bit 2.  (4.0 and 2.5 ticks of the CU's LDS per read, its full rate; with a bijection of t % 8, as
-// b128 reads of eight lanes would want, the K fragments took 8.0.)
-__host__ __device__ constexpr int swz(int t) { return ((t & 2) << 1) | ((t >> 2) & 3); }
+// different values.  A transposing read serves 32 lanes, 32 bytes of eight rows: the four rows of a parity need different
+// values of bits 1 and 2.
+__host__ __device__ constexpr int swz(int t) { return ((t & 2) << 1) | (((t >> 1) ^ (t >> 2)) & 2) | ((t >> 3) & 1); }
 
 // f(integral_constant 0), f(integral_constant 1) .. f(integral_constant N - 1), written out
 template <class F, int... I>
@@ -287,11 +290,14 @@ __device__ __forceinline__ SplitRange split_range(int cur, int nsplit, int sp)
 // Resolves the workgroup's share: logical indices -> physical cache rows (absent entries: row 0 and a cleared bit in
 // the tile's validity word), in LDS.  NT lanes.  The sequence's length, its page table and the share's top-k entries
 // are requested together: the entries are fetched for the share a full list would give (the usual case) and only
-// fetched again if the length, once known, moves the share.  `between` runs after those requests and before the first
-// wait for them.  Returns the share.
-template <int NT, class Between>
+// fetched again if the length, once known, moves the share.  The other waves pass its two barriers beside it.  Returns the share.
+__device__ __forceinline__ SplitRange share_of(const SfaArgs& a, int act, int si, int sp)
+{
+    return split_range(min(max(act - a.s1 + 1 + si, 0), a.topk), a.nsplit, sp);
+}
+template <int NT>
 __device__ __forceinline__ SplitRange resolve_split(const SfaArgs& a, int bi, int si, int tq, int sp, uint32_t* tmask,
-                                                    int* rows, int* bt_lds, int tid, int lane, Between&& between)
+                                                    int* rows, int* bt_lds, int tid, int lane)
 {
     constexpr int PER_LANE = MAX_SPLIT_TOKENS / NT;
     const int32_t* list = a.topk_idx + (int64_t)tq * a.topk_stride;
@@ -314,13 +320,12 @@ __device__ __forceinline__ SplitRange resolve_split(const SfaArgs& a, int bi, in
         for (int j = 0; j < BT_PER_LANE; ++j)
             if (tid + NT * j < a.bt_stride) btv[j] = a.block_table[(int64_t)bi * a.bt_stride + tid + NT * j];
     }
-    between(); // the caller's own loads, behind the ones above and ahead of the first wait for them
     if (bt_cached) {
 #pragma unroll
         for (int j = 0; j < BT_PER_LANE; ++j)
             if (tid + NT * j < a.bt_stride) bt_lds[tid + NT * j] = btv[j];
     }
-    const SplitRange r = split_range(min(max(act - a.s1 + 1 + si, 0), a.topk), a.nsplit, sp);
+    const SplitRange r = share_of(a, act, si, sp);
     if (r.tile0 != guess.tile0) fetch(r.tile0 * T); // block-uniform
     const int tok0 = r.tile0 * T;
     const int ntiles_even = (r.ntiles + 1) & ~1; // whole wavefronts of entries
@@ -354,13 +359,13 @@ __device__ __forceinline__ SplitRange resolve_split(const SfaArgs& a, int bi, in
     return r;
 }
 
-// k-step of position i of a wave's 36: the two halves of the contraction one after the other, each its 16 nope steps and
-// its 2 rope steps
-__host__ __device__ constexpr int kstep_at(int i) { return i < 16 ? i : i < 18 ? i + 16 : i < 34 ? i - 2 : i; }
-constexpr bool parked(int i) { return i % PARK_EVERY == PARK_EVERY - 1; }
-// operand fragments read ahead of the matrix instruction that uses them: K, V in the score wave, V in the value wave (more
-// are registers that the waves do not have; four K fragments: 3650 ticks a tile, three in the value wave: 4000)
-constexpr int KD = 3, VD_S = 3, VD_V = 2;
+// k-step of position i of 18: the two halves of the contraction one after the other, each its eight nope steps and its rope step
+__host__ __device__ constexpr int kstep_at(int i) { return i < 8 ? i : i == 8 ? 16 : i < 17 ? i - 1 : i; }
+// fragments of Q: 2 (position) + block of 16 heads
+constexpr bool parked(int f) { return f % PARK_EVERY == PARK_EVERY - 1; }
+// operand fragments read ahead of the matrix instructions that use them: K, V in the score wave, V in the value wave (more
+// are registers that the waves do not have)
+constexpr int KD = 4, VD_S = 3, VD_V = 2;
 #define STEP_FENCE() __builtin_amdgcn_sched_barrier(0)
 
 // (fmaxf has the compiler quiet every operand first; the scores are sums of products, which are no signalling NaN)
@@ -371,13 +376,28 @@ __device__ __forceinline__ float max3(float a, float b, float c)
     return r;
 }
 
-// O^T blocks DB0 .. DB0 + N - 1 of a pair's 32 heads: V^T fragments from a tile by transposing reads, P~ in two fragments of
-// 16 tokens.
+// Over the four lanes of a wavefront that are 16 apart: the maxima of a and of b, in every one of them.  (Without a trip through LDS:
+// v_permlane32_swap exchanges the upper half of its first operand with the lower half of its second, v_permlane16_swap the odd
+// rows of 16 lanes of the first with the even rows of the second.  They need wait states behind an instruction that writes their
+// operands, which the compiler leaves behind one that it knows: no inline assembly for those.)
+__device__ __forceinline__ void max_over_rows(float a, float b, float& ma, float& mb)
+{
+    const auto h = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    const unsigned x = __builtin_bit_cast(unsigned, fmaxf(__builtin_bit_cast(float, (unsigned)h[0]), __builtin_bit_cast(float, (unsigned)h[1])));
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    const unsigned y = __builtin_bit_cast(unsigned, fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1])));
+    const auto m = __builtin_amdgcn_permlane32_swap(y, y, false, false); // (lower half of y: a's maxima, upper: b's)
+    ma = __builtin_bit_cast(float, (unsigned)m[0]);
+    mb = __builtin_bit_cast(float, (unsigned)m[1]);
+}
+
+// O^T blocks DB0 .. DB0 + N - 1 of a pair's 32 heads, each 16 value columns x two blocks of 16 heads: V^T fragments of all 32 tokens of
+// a tile by transposing reads, P~ in one fragment per block of heads.
 template <int DB0, int N, int VD>
 struct Values {
-    f32x16 o[N];
+    f32x4 o[N][2];
     uint32_t off;       // this lane's place in a stage
-    uint32_t at[2][2];  // the same in the stage in use, for the second eight rows and odd blocks too
+    uint32_t at[4];     // the same in the stage in use, for the blocks n % 4
     s16x4 lo[VD], hi[VD];
 
     __device__ __forceinline__ void init(int lane)
@@ -385,97 +405,106 @@ struct Values {
 #pragma unroll
         for (int i = 0; i < N; ++i)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
-        // lane jj of 16-lane group G points at row 4*hl + jj/4 (+ 8*h2 + 16*j), columns 32*db + 16*(G&1) + 4*(jj&3) -> chunk
-        // 4*db + 2*(G&1) + (jj&3)/2.  Eight rows on, the swizzle differs in bit 1; in odd blocks, the chunk in bit 2; a stage
-        // is a multiple of 128 bytes, so that an exclusive or in these bits stays inside a row's group of eight chunks.
-        const int hl = lane >> 5, jj = lane & 15, mh = (lane >> 4) & 1, t = 4 * hl + (jj >> 2);
-        off = t * KROW + (((2 * mh + ((jj & 3) >> 1)) ^ swz(t)) << 4) + (jj & 1) * 8;
+            for (int b = 0; b < 2; ++b) o[i][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // lane jj of row g of 16 lanes points at tile row 4 g + jj / 4 (+ 16: the same swizzle), columns 16 n + 4 (jj & 3) -> chunk 2 n +
+        // (jj & 3) / 2, and gets column 16 n + jj of the rows 4 g .. 4 g + 3.  n % 4 is bits 1 and 2 of the chunk; a stage is a multiple
+        // of 128 bytes, so that an exclusive or in these bits stays inside a row's group of eight chunks.
+        const int jj = lane & 15, t = 4 * (lane >> 4) + (jj >> 2);
+        off = t * KROW + ((((jj & 3) >> 1) ^ swz(t)) << 4) + (jj & 1) * 8;
     }
-    // fragment n: token block n / N, column block n % N
     template <int n>
     __device__ __forceinline__ void fetch(uint8_t* lds)
     {
-        constexpr int j = n / N, db = DB0 + n % N, step = 16 * j * KROW + (db >> 1) * 128;
-        lo[n % VD] = lds_read_tr(lds + at[0][db & 1] + step);
-        hi[n % VD] = lds_read_tr(lds + at[1][db & 1] + step + 8 * KROW);
+        constexpr int db = DB0 + n, step = (db >> 2) * 128;
+        lo[n % VD] = lds_read_tr(lds + at[db & 3] + step);
+        hi[n % VD] = lds_read_tr(lds + at[db & 3] + step + 16 * KROW);
     }
     __device__ __forceinline__ void ahead(uint8_t* lds, int stage)
     {
-        at[0][0] = off + stage;
-        at[0][1] = at[0][0] ^ 64;
-        at[1][0] = at[0][0] ^ 32;
-        at[1][1] = at[0][0] ^ 96;
+        at[0] = off + stage;
+        at[1] = at[0] ^ 32;
+        at[2] = at[0] ^ 64;
+        at[3] = at[0] ^ 96;
         unroll<VD>([&](auto n) { fetch<n>(lds); });
     }
     template <int n>
-    __device__ __forceinline__ void step(uint8_t* lds, const u32x4& p)
+    __device__ __forceinline__ void step(uint8_t* lds, const u32x4 (&p)[2])
     {
-        const s16x8 v = __builtin_shufflevector(lo[n % VD], hi[n % VD], 0, 1, 2, 3, 4, 5, 6, 7);
-        o[n % N] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, v), __builtin_bit_cast(bf16x8, p), o[n % N], 0, 0, 0);
-        if constexpr (n + VD < 2 * N) fetch<n + VD>(lds);
+        const bf16x8 v = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo[n % VD], hi[n % VD], 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+        for (int b = 0; b < 2; ++b) o[n][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, __builtin_bit_cast(bf16x8, p[b]), o[n][b], 0, 0, 0);
+        if constexpr (n + VD < N) fetch<n + VD>(lds);
     }
     // (fragments 0 .. VD - 1 have been requested)
     __device__ __forceinline__ void add(uint8_t* lds, const u32x4 (&p)[2])
     {
-        unroll<2 * N>([&](auto n) {
-            step<n>(lds, p[n / N]);
+        unroll<N>([&](auto n) {
+            step<n>(lds, p);
             STEP_FENCE();
         });
     }
-    __device__ __forceinline__ void scale(float f)
+    __device__ __forceinline__ void scale(float f0, float f1)
     {
 #pragma unroll
-        for (int i = 0; i < N; ++i) o[i] *= f;
+        for (int i = 0; i < N; ++i) {
+            o[i][0] *= f0;
+            o[i][1] *= f1;
+        }
     }
-    // Epilogue.  Register r of o[i] holds dim 32*(DB0 + i) + 8*(r/4) + 4*hl + r%4 of the lane's head: four consecutive dims,
-    // and the other half-wave holds the four next to them.
+    // Epilogue.  Register e of o[i][b] holds dim 16 (DB0 + i) + 4 g + e of head 16 b + lane % 16.
     // A split's share, normalised by its own sum, in fp16 (|value| <= max |V| and 2^-11 relative rounding, a quarter
     // of the final bf16 rounding, half the bytes of fp32 for this kernel to write and the merge to read).  It leaves
-    // in fragment order, straight from the accumulators: [token][split][head group][column group dq 4][head half 2]
-    // [head block 2][i 4][half 2][lane 64] x 8 fp16 (block 4 dq + i) - every store instruction writes 1 KB of
+    // in fragment order, straight from the accumulators: [token][split][head group][column group dq 4][pair 4][i 4][block of
+    // heads 2][lane 64] x 8 fp16, dims 4 g .. + 3 of column blocks 8 dq + 2 i and the next - every store instruction writes 1 KB of
     // consecutive bytes, and nothing is staged.  The merge kernel reads the same order and does the transposition to
     // rows once, for the output, instead of once per split here.  (Streaming stores: 34 MB leave the chip's 256
     // workgroups at once and are read back once.)
-    __device__ __forceinline__ void store_partial(_Float16* base, float mul)
+    __device__ __forceinline__ void store_partial(_Float16* base, const float (&mul)[2])
     {
 #pragma unroll
-        for (int i = 0; i < N; ++i)
+        for (int i = 0; i < N / 2; ++i)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
+            for (int b = 0; b < 2; ++b) {
                 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-                const int db = DB0 + i;
+                const int cb = DB0 / 2 + i;
                 uint32_t x[4];
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
-                    x[k] = __builtin_bit_cast(uint32_t, f16x2{(_Float16)(o[i][8 * h + 2 * k] * mul), (_Float16)(o[i][8 * h + 2 * k + 1] * mul)});
-                __builtin_nontemporal_store(u32x4{x[0], x[1], x[2], x[3]}, reinterpret_cast<u32x4*>(base + (db >> 2) * 16384 + ((db & 3) * 2 + h) * 512));
+                    x[k] = __builtin_bit_cast(uint32_t, f16x2{(_Float16)(o[2 * i + (k >> 1)][b][2 * (k & 1)] * mul[b]),
+                                                              (_Float16)(o[2 * i + (k >> 1)][b][2 * (k & 1) + 1] * mul[b])});
+                __builtin_nontemporal_store(u32x4{x[0], x[1], x[2], x[3]}, reinterpret_cast<u32x4*>(base + (cb >> 2) * 16384 + ((cb & 3) * 2 + b) * 512));
             }
     }
-    // One split: the output itself, bf16 rows [head][512] of 1024 bytes in LDS.  v_permlane32_swap pairs up the two
-    // half-waves' four-dim pieces - the lower half-wave ends up with the 8 dims of block g = 2 gp, the upper one with those
-    // of block 2 gp + 1 - so that a lane stores 16 bytes; the chunks of a row are XOR-swizzled with the head (16 rows of a
-    // store meet all banks).
-    __device__ __forceinline__ void stage_rows(uint8_t* orow, int hrow, int hl, float mul)
+    // One split: the output itself, bf16 rows [head][512] of 1024 bytes in LDS (orow: the pair's first).  v_permlane16_swap pairs up
+    // four-dim pieces of neighbouring rows of lanes - an even row ends up with 8 dims of the first of two blocks, an odd one with
+    // those of the second - so that a lane stores 16 bytes; the chunks of a row are XOR-swizzled with the head (16 rows of a store
+    // meet all banks).
+    __device__ __forceinline__ void stage_rows(uint8_t* orow, int l16, int g, const float (&mul)[2])
     {
 #pragma unroll
-        for (int i = 0; i < N; ++i)
+        for (int i = 0; i < N; i += 2)
 #pragma unroll
-            for (int gp = 0; gp < 2; ++gp) {
-                uint32_t x[2][2]; // [block 2 gp, 2 gp + 1][pair of dims]
+            for (int b = 0; b < 2; ++b) {
+                uint32_t x[2][2]; // [block i, i + 1][pair of dims]
 #pragma unroll
-                for (int g = 0; g < 2; ++g)
+                for (int j = 0; j < 2; ++j)
 #pragma unroll
-                    for (int k = 0; k < 2; ++k)
-                        x[g][k] = pack_bf16x2(o[i][4 * (2 * gp + g) + 2 * k] * mul, o[i][4 * (2 * gp + g) + 2 * k + 1] * mul);
-                // the swap exchanges the upper half-wave of its first operand with the lower half-wave of its second
-                const auto e0 = __builtin_amdgcn_permlane32_swap(x[0][0], x[1][0], false, false);
-                const auto e1 = __builtin_amdgcn_permlane32_swap(x[0][1], x[1][1], false, false);
-                const int c = 4 * (DB0 + i) + 2 * gp + hl;
-                *reinterpret_cast<u32x4*>(orow + ((c ^ (hrow & 15)) << 4)) = u32x4{(uint32_t)e0[0], (uint32_t)e1[0], (uint32_t)e0[1], (uint32_t)e1[1]};
+                    for (int k = 0; k < 2; ++k) x[j][k] = pack_bf16x2(o[i + j][b][2 * k] * mul[b], o[i + j][b][2 * k + 1] * mul[b]);
+                const auto e0 = __builtin_amdgcn_permlane16_swap(x[0][0], x[1][0], false, false);
+                const auto e1 = __builtin_amdgcn_permlane16_swap(x[0][1], x[1][1], false, false);
+                const int c = 2 * (DB0 + i + (g & 1)) + (g >> 1);
+                *reinterpret_cast<u32x4*>(orow + (16 * b + l16) * OUT_ROW + ((c ^ l16) << 4)) = u32x4{(uint32_t)e0[0], (uint32_t)e1[0], (uint32_t)e0[1], (uint32_t)e1[1]};
             }
     }
 };
+
+// 64 lanes x 16 bytes from base + each lane's offset to 1 KB of LDS at d, in lane order, without registers in between; base and d are
+// wave-uniform.  (Written out: the compiler would wait for it before every other LDS read.)
+typedef __attribute__((address_space(3))) uint8_t lds_u8;
+__device__ __forceinline__ void copy_to_lds(const void* base, uint32_t offset, uint8_t* d)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"((lds_u8*)d), "v"(offset), "s"(base) : "memory");
+}
 
 // The body of one wavefront.  SCORES: the pair's score wave (waves 0 .. 3), which holds Q and does the scores, the softmax and
 // the values of the first NDB_S column blocks; else its value wave (waves 4 .. 7), which produces the tiles, eight rows of
@@ -483,90 +512,76 @@ struct Values {
 template <bool QUANT, bool SCORES>
 __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32_t* tmask, int* rows, int* bt_lds, int tid)
 {
-    constexpr int NT = 64 * WAVES;
     const int tq = blockIdx.x, sp = blockIdx.y, hz = blockIdx.z;
     const int bi = tq / a.s1, si = tq - bi * a.s1;
     const int lane = tid & 63, pair = __builtin_amdgcn_readfirstlane(tid >> 6) & (PAIRS - 1); // (scalar: what follows from it is too)
-    const int l32 = lane & 31, hl = lane >> 5;
+    const int l16 = lane & 15, g = lane >> 4;
     const int head0 = hz * HEADS_PER_WG;
-    const int hrow = pair * 32 + l32, head = head0 + hrow;
+    const int hrow = pair * 32 + l16, head = head0 + hrow; // (and the ones 16 on)
     const bool active = head0 + pair * 32 < a.nq; // (a pair without heads works on copies of the last one, and stores nothing)
 
-    // The query of the workgroup's 128 heads, requested right behind the few loads the look-up of the share starts with
-    // (it is the largest piece of the start-up traffic and depends on nothing).  Fetched as whole cache lines - in each of four rounds of 128 nope
-    // columns a lane takes four 16-byte pieces, 16 consecutive lanes one head's 256 bytes; then the rope columns, two
-    // pieces per lane - because a load in operand layout (a lane pair per head) costs the texture addresser one line per
-    // lane pair.  The operand layout is made on the way through LDS further down.
-    constexpr int QN = HEADS_PER_WG * 16 / NT, QR = HEADS_PER_WG * 8 / NT;
-    u32x4 qraw[4][QN], qraw_rope[QR];
-    auto request_q = [&]() {
-        const int64_t qrow0 = (int64_t)tq * a.nq;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int j = 0; j < QN; ++j) {
-                const int p = tid + NT * j;
-                const int64_t row = qrow0 + min(head0 + (p >> 4), a.nq - 1);
-                qraw[r][j] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const __bf16*>(a.q_nope) + row * DN + 128 * r + 8 * (p & 15));
-            }
-#pragma unroll
-        for (int j = 0; j < QR; ++j) {
-            const int p = tid + NT * j;
-            const int64_t row = qrow0 + min(head0 + (p >> 3), a.nq - 1);
-            qraw_rope[j] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const __bf16*>(a.q_rope) + row * DR + 8 * (p & 7));
-        }
-    };
-
-    const SplitRange share = resolve_split<NT>(a, bi, si, tq, sp, tmask, rows, bt_lds, tid, lane, request_q);
-    const int ntiles = share.ntiles, last = ntiles - 1;
-
-    RawTile<QUANT> raw;
-    if (!SCORES && ntiles > 0) gather_tile<QUANT>(raw, a, rows + 8 * pair, lane);
-
-    // Q into operand layout: this lane's head and the 36 k-steps; B operand layout: head = column, 8 consecutive k per
-    // half-wave.  One trip through LDS (all of it below the per-split arrays is still unused).
+    // The start.  The score waves copy the query of their 32 heads to LDS, a head's nope columns to an instruction, and read their operand
+    // fragments from there, while the value waves look up the share and gather the first two tiles: 8 K ticks until the first tile is
+    // stored, where all waves did one after the other, the query through registers, 12 K.  (A load in operand layout would cost the
+    // texture addresser a line per lane.)  The 16-byte chunks of a nope row are exchanged by the head's last four bits, of a rope row by
+    // the three above the last: the 16 lanes that a read serves meet all banks.
+    constexpr int NT = 64 * PAIRS;
+    const int ht = tid & (NT - 1);
     bf16x8 q[SCORES ? NREG : 1];
     uint8_t* qpark = smem + QPARK_OFF + pair * (NPARK * 1024) + lane * 16;
-    {
+    SplitRange share;
+    RawTile<QUANT> raw0, raw;
+    if constexpr (SCORES) {
+        const int act = a.act_seq[bi];
+        uint8_t* qrows = smem + pair * QPAIR;
+        const int64_t qrow0 = (int64_t)tq * a.nq;
+#pragma unroll
+        for (int h = 0; h < 32; ++h)
+            copy_to_lds(static_cast<const uint8_t*>(a.q_nope) + (qrow0 + min(head0 + 32 * pair + h, a.nq - 1)) * (DN * 2), (uint32_t)((lane ^ (h & 15)) * 16),
+                        qrows + h * (DN * 2));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int h = 8 * i + (lane >> 3);
+            copy_to_lds(static_cast<const uint8_t*>(a.q_rope) + qrow0 * (DR * 2),
+                        (uint32_t)(min(head0 + 32 * pair + h, a.nq - 1) * (DR * 2) + (((lane & 7) ^ ((h >> 1) & 7)) * 16)), qrows + 32 * DN * 2 + i * 1024);
+        }
+        share = share_of(a, act, si, sp);
+        __syncthreads(); // (the look-up's)
+        __syncthreads(); // rows[] / tmask[] ready
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         // (a negative softmax_scale is applied as its magnitude to the negated query: the row statistics below are
         // taken on the raw scores, which needs a factor that commutes with max)
         const uint32_t f = a.softmax_scale < 0.f ? 0x80008000u : 0u;
         const u32x4 qflip = {f, f, f, f};
-        // all 128 heads' rows at once: row h at h * QROW, its 72 16-byte chunks (64 nope, 8 rope) swizzled like a tile's
+        // B operand layout: head = column, 8 consecutive k per row of 16 lanes
+        u32x4 qa[QFRAGS];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int j = 0; j < QN; ++j) {
-                const int pp = tid + NT * j, h = pp >> 4, c = 16 * r + (pp & 15);
-                *reinterpret_cast<u32x4*>(smem + h * QROW + ((c ^ swz(h)) << 4)) = qraw[r][j];
-            }
-#pragma unroll
-        for (int j = 0; j < QR; ++j) {
-            const int pp = tid + NT * j, h = pp >> 3, c = 64 + (pp & 7);
-            *reinterpret_cast<u32x4*>(smem + h * QROW + ((c ^ swz(h)) << 4)) = qraw_rope[j];
-        }
-        __syncthreads();
-        u32x4 qa[KSTEPS];
-        if constexpr (SCORES) {
-#pragma unroll
-            for (int i = 0; i < KSTEPS; ++i)
-                qa[i] = *reinterpret_cast<const u32x4*>(smem + hrow * QROW + (((2 * kstep_at(i) + hl) ^ swz(hrow)) << 4)) ^ qflip;
+        for (int i = 0; i < QFRAGS; ++i) {
+            const int ks = kstep_at(i >> 1), h = 16 * (i & 1) + l16;
+            qa[i] = *reinterpret_cast<const u32x4*>(ks < DN / 32 ? qrows + h * (DN * 2) + (((4 * ks + g) ^ l16) << 4)
+                                                                 : qrows + 32 * DN * 2 + h * (DR * 2) + (((4 * (ks - DN / 32) + g) ^ ((h >> 1) & 7)) << 4)) ^ qflip;
         }
         __syncthreads(); // the score waves have their fragments: the rows' space is free for the parked fragments and the tiles
-        if constexpr (SCORES) {
 #pragma unroll
-            for (int i = 0; i < KSTEPS; ++i) {
-                const bf16x8 v = __builtin_bit_cast(bf16x8, qa[i]);
-                if (parked(i))
-                    *reinterpret_cast<bf16x8*>(qpark + (i / PARK_EVERY) * 1024) = v;
-                else
-                    q[SCORES ? i - i / PARK_EVERY : 0] = v;
-            }
+        for (int i = 0; i < QFRAGS; ++i) {
+            const bf16x8 v = __builtin_bit_cast(bf16x8, qa[i]);
+            if (parked(i))
+                *reinterpret_cast<bf16x8*>(qpark + (i / PARK_EVERY) * 1024) = v;
+            else
+                q[SCORES ? i - i / PARK_EVERY : 0] = v;
         }
+    } else {
+        share = resolve_split<NT>(a, bi, si, tq, sp, tmask, rows, bt_lds, ht, lane);
+        if (share.ntiles > 0) {
+            gather_tile<QUANT>(raw0, a, rows + 8 * pair, lane);
+            gather_tile<QUANT>(raw, a, rows + min(1, share.ntiles - 1) * T + 8 * pair, lane);
+        }
+        __syncthreads(); // the score waves have their fragments
     }
+    const int ntiles = share.ntiles, last = ntiles - 1;
 
     Values<SCORES ? 0 : NDB_S, SCORES ? NDB_S : NDB - NDB_S, SCORES ? VD_S : VD_V> val;
-    val.init(lane);
+    if constexpr (SCORES) val.init(lane);
     // P~ of tile i lies in buffer i % 2, the order the S^T registers hold the tokens in, and the factor by which what was
     // summed before is to be multiplied, where the flag says so
     uint8_t* pbuf = smem + PBUF_OFF + pair * 2048; // (+ 16 lane)
@@ -582,87 +597,107 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
         st = st_new;
         st_new = t;
     };
-    float l_tot, m_out = 0.f;
+    float l_tot[2], m_out[2] = {0.f, 0.f};
     if constexpr (SCORES) {
-        // S operand (b128): row l32, chunk 2*ks + hl of k-step ks; swizzled offsets of the four chunk positions 2 m + hl
-        // inside a group of eight chunks
-        uint32_t s_off[4];
+        // S operand (b128): tile rows l16 and 16 + l16 (the same swizzle), chunk 4 ks + g of k-step ks; swizzled offsets of the two
+        // chunk positions inside a group of eight chunks
+        uint32_t s_off[2];
 #pragma unroll
-        for (int m = 0; m < 4; ++m) s_off[m] = l32 * KROW + (((2 * m + hl) ^ swz(l32)) << 4);
+        for (int m = 0; m < 2; ++m) s_off[m] = l16 * KROW + (((4 * m + g) ^ swz(l16)) << 4);
+        // fragment n of a tile: position n / 2, rows 16 (n % 2) ..
         bf16x8 kf[KD], qp;
-        auto fetch_k = [&](auto ic) {
-            constexpr int i = ic, ks = kstep_at(i);
-            kf[i % KD] = *reinterpret_cast<const bf16x8*>(smem + st + s_off[ks & 3] + (ks >> 2) * 128);
-            if constexpr (parked(i)) qp = *reinterpret_cast<const bf16x8*>(qpark + (i / PARK_EVERY) * 1024);
+        auto fetch_k = [&](auto nc) {
+            constexpr int n = nc, ks = kstep_at(n >> 1);
+            kf[n % KD] = *reinterpret_cast<const bf16x8*>(smem + st + s_off[ks & 1] + (ks >> 1) * 128 + (n & 1) * 16 * KROW);
+            if constexpr (!(n & 1) && parked(n + 1)) qp = *reinterpret_cast<const bf16x8*>(qpark + (n / PARK_EVERY) * 1024);
         };
-        float m_run = -INFINITY; // running max of S * scale * log2(e)
-        float l_run = 0.f;       // this lane's share of sum exp
-        float alpha = 1.f;
+        static_assert(PARK_EVERY % 2 == 0 && KD < PARK_EVERY, "a parked fragment is its k-step's second, and out of use when the next one is read");
+        float m_run[2] = {-INFINITY, -INFINITY}; // running max of S * scale * log2(e)
+        float l_run[2] = {0.f, 0.f};             // this lane's share of sum exp
+        float alpha[2] = {1.f, 1.f};
         bool rescale = false;
         // (never exactly zero: a masked score is -inf, and -inf * 0 would be NaN; 2^(s * 1e-30) is 1 for every finite s, so
         // a zero scale still gives every attended row the same weight)
         const float c_log2 = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, fmaxf(fabsf(a.softmax_scale) * 1.4426950408889634f, 1e-30f))));
         u32x4 p[2];
         auto tile = [&](int it) {
-            f32x16 s0, s1;
-            const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            f32x4 s0[2][2]; // [block of 16 rows][block of 16 heads]
+            const uint32_t present = tmask[it];
             STEP_FENCE();
-            unroll<KSTEPS>([&](auto ic) {
-                constexpr int i = ic;
-                const bf16x8 qi = parked(i) ? qp : q[i - i / PARK_EVERY];
-                f32x16& s = i < KSTEPS / 2 ? s0 : s1;
-                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i % KD], qi, i % (KSTEPS / 2) == 0 ? zero : s, 0, 0, 0);
-                if constexpr (i + KD < KSTEPS) fetch_k(std::integral_constant<int, i + KD>{});
+            unroll<QFRAGS>([&](auto nc) {
+                constexpr int n = nc, i = n >> 1;
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    constexpr int f = 2 * i;
+                    const bf16x8 qi = b == 1 && parked(f + 1) ? qp : q[f + b - (f + b) / PARK_EVERY];
+                    f32x4& s = s0[n & 1][b];
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[n % KD], qi, i == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : s, 0, 0, 0);
+                }
+                if constexpr (n + KD < QFRAGS) fetch_k(std::integral_constant<int, n + KD>{});
                 STEP_FENCE();
             });
-            const uint32_t valid = __builtin_amdgcn_readfirstlane(tmask[it]);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s0[r] += s1[r];
+            const uint32_t valid = __builtin_amdgcn_readfirstlane(present);
             if (valid != 0xffffffffu) {
-                // register r holds token 8*(r/4) + 4*hl + r%4 for head l32 (the half-wave's shift first: the bit
+                // register e of s0[rb][b] holds row 16 rb + 4 g + e for head 16 b + l16 (the lanes' shift first: the bit
                 // positions left are compile-time constants)
-                const uint32_t vh = valid >> (4 * hl);
+                const uint32_t vh = valid >> (4 * g);
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s0[r] = ((vh >> (8 * (r >> 2) + (r & 3))) & 1u) ? s0[r] : -INFINITY;
+                for (int r = 0; r < 16; ++r) {
+                    f32x4& x = s0[r >> 3][(r >> 2) & 1];
+                    x[r & 3] = ((vh >> (16 * (r >> 3) + (r & 3))) & 1u) ? x[r & 3] : -INFINITY;
+                }
             }
-            // statistics on the raw scores (the factor is not negative, so it commutes with max)
-            float x0 = max3(s0[0], s0[1], s0[2]), x1 = max3(s0[3], s0[4], s0[5]), x2 = max3(s0[6], s0[7], s0[8]);
-            float x3 = max3(s0[9], s0[10], s0[11]), x4 = max3(s0[12], s0[13], s0[14]);
-            x0 = max3(x0, x1, s0[15]);
-            x2 = max3(x2, x3, x4);
-            // maximum over both halves of the wavefront without a trip through LDS: v_permlane32_swap exchanges the
-            // upper half of its first operand with the lower half of its second.  (The multiplication is the compiler's own:
-            // the swap needs wait states behind an instruction that writes its operand, which the compiler leaves behind
-            // one that it knows)
-            const float mx = max3(x0, x2, x2) * c_log2;
-            const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, mx), __builtin_bit_cast(unsigned, mx), false, false);
+            // P~ in the order the S^T registers hold the rows: k-slot s of lanes g is row 4 g + s % 4 + 16 (s / 4) - which is also how the
+            // V^T fragments are read.  Relative to the running maximum as it was, while the maximum of this tile is on its way between
+            // the lanes.
+            float l_tile[2], mx[2], m_new[2];
+            auto probabilities = [&](auto between) {
+                unroll<2>([&](auto bc) {
+                    constexpr int b = bc;
+                    const float m_use = valid != 0u ? m_run[b] : 0.f; // (a tile without rows: every score is -inf, every P~ 0)
+                    l_tile[b] = 0.f;
+                    unroll<4>([&](auto rc) {
+                        constexpr int r = 2 * rc;
+                        const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s0[r >> 2][b][r & 3], c_log2, -m_use));
+                        const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s0[r >> 2][b][(r & 3) + 1], c_log2, -m_use));
+                        l_tile[b] += e0 + e1;
+                        p[b][r >> 1] = pack_bf16x2(e0, e1);
+                        between(std::integral_constant<int, 4 * b + r / 2>{});
+                    });
+                });
+            };
+            probabilities([&](auto ic) {
+                constexpr int i = ic;
+                // statistics on the raw scores (the factor is not negative, so it commutes with max)
+                if constexpr (i == 0 || i == 1) {
+                    const float x0 = max3(s0[0][i][0], s0[0][i][1], s0[0][i][2]), x1 = max3(s0[0][i][3], s0[1][i][0], s0[1][i][1]);
+                    mx[i] = max3(x0, x1, max3(s0[1][i][2], s0[1][i][3], x0)) * c_log2;
+                }
+                if constexpr (i == 2) max_over_rows(mx[0], mx[1], m_new[0], m_new[1]);
+            });
             // The reference exponent only follows the running maximum when it has grown by more than 2^8: until
             // then P~ = 2^(z - m_run) may exceed 1 (by at most 2^8, no issue for bf16 or the fp32 sums), which
             // makes the rescale of the accumulator registers a rare event.  Every P~, l and O stay relative to
             // the same m_run, so the result is unchanged.
-            const float m_new = max3(m_run, __builtin_bit_cast(float, (unsigned)sw[0]), __builtin_bit_cast(float, (unsigned)sw[1]));
-            rescale = __any(m_new > m_run + 8.f);
+#pragma unroll
+            for (int b = 0; b < 2; ++b) m_new[b] = fmaxf(m_run[b], m_new[b]);
+            rescale = __any(m_new[0] > m_run[0] + 8.f || m_new[1] > m_run[1] + 8.f);
             if (rescale) {
-                alpha = __builtin_amdgcn_exp2f(m_run - m_new); // 0 on the first tile (m_run = -inf)
-                l_run *= alpha;
-                m_run = m_new;
-                if (hl == 0) alpha_lds[(it & 1) * (PAIRS * 32) + l32] = alpha;
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    alpha[b] = __builtin_amdgcn_exp2f(m_run[b] - m_new[b]); // 0 on the first tile (m_run = -inf)
+                    l_run[b] *= alpha[b];
+                    m_run[b] = m_new[b];
+                    if (g == 0) alpha_lds[(it & 1) * (PAIRS * 32) + 16 * b + l16] = alpha[b];
+                }
+                probabilities([](auto) {});
             }
             if (lane == 0) flag_lds[(it & 1) * PAIRS] = rescale ? 1u : 0u;
-            const float m_use = valid != 0u ? m_run : 0.f; // (a tile without rows: every score is -inf, every P~ 0)
-            // P~ in the order the S^T registers hold the tokens: k-slot s of half hl in block j is token
-            // 16*j + 8*(s/4) + 4*hl + s%4 - which is also how the V^T fragments are read
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s0[r] = __builtin_fmaf(s0[r], c_log2, -m_use);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s0[r] = __builtin_amdgcn_exp2f(s0[r]);
-#pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                l_run += s0[r] + s0[r + 1];
-                p[r >> 3][(r & 7) >> 1] = pack_bf16x2(s0[r], s0[r + 1]);
+            for (int b = 0; b < 2; ++b) {
+                l_run[b] += l_tile[b];
+                *reinterpret_cast<u32x4*>(pbuf + (it & 1) * (PAIRS * 2048) + b * 1024 + lane * 16) = p[b];
             }
-#pragma unroll
-            for (int j = 0; j < 2; ++j) *reinterpret_cast<u32x4*>(pbuf + (it & 1) * (PAIRS * 2048) + j * 1024 + lane * 16) = p[j];
         };
         __syncthreads(); // tile 0 stored, Q parked
         if (ntiles > 0) {
@@ -674,25 +709,30 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
             for (int it = 1; it < ntiles; ++it) {
                 val.ahead(smem, st_old);
                 unroll<KD>(fetch_k);
-                if (rescale) val.scale(alpha);
+                if (rescale) val.scale(alpha[0], alpha[1]);
                 val.add(smem, p);
                 tile(it);
                 __syncthreads();
                 turn();
             }
             val.ahead(smem, st_old);
-            if (rescale) val.scale(alpha);
+            if (rescale) val.scale(alpha[0], alpha[1]);
             val.add(smem, p);
         }
-        l_tot = l_run + __shfl_xor(l_run, 32);
-        m_out = m_run;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const float l = l_run[b] + __shfl_xor(l_run[b], 16);
+            l_tot[b] = l + __shfl_xor(l, 32);
+            m_out[b] = m_run[b];
+        }
     } else {
         Production<QUANT> prod;
         // Tile `tile` out of registers into a stage.  A load's registers are free as soon as their last pair is in hand: the
         // rows of the tile after are requested right behind that.
         constexpr int LOADS = RawTile<QUANT>::LOADS;
-        constexpr int STEPS = 2 * (NDB - NDB_S);
-        auto produce = [&](int tile, int stage, auto&& between) {
+        constexpr int STEPS = NDB - NDB_S;
+        auto produce = [&](RawTile<QUANT>& raw, auto regather, int tile, int stage, auto&& between) {
+            constexpr bool GATHER = decltype(regather)::value;
             const uint32_t present = __builtin_amdgcn_readfirstlane(tmask[tile]);
             const int* next = rows + min(tile + 1, last) * T + 8 * pair;
             uint32_t row, row1;
@@ -702,43 +742,48 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
                 constexpr int i = ic, per = 32 / LOADS, K = i / per;
                 between(ic);
                 prod.template piece<i>(raw, present, smem, stage, pair, lane);
-                if constexpr (i < 32 && i % per == per - 3) row = nope_row<QUANT, K>(next, lane);
-                if constexpr (i < 32 && i % per == per - 1) gather_nope<QUANT, K>(raw, row, a, lane);
-                if constexpr (i == 28) row1 = scale_row(next, lane);
-                if constexpr (i == 30) gather_scale<QUANT>(raw, row1, a, lane);
-                if constexpr (i == 32) row1 = rope_row(next, lane);
+                if constexpr (GATHER) {
+                    if constexpr (i < 32 && i % per == per - 3) row = nope_row<QUANT, K>(next, lane);
+                    if constexpr (i < 32 && i % per == per - 1) gather_nope<QUANT, K>(raw, row, a, lane);
+                    if constexpr (i == 28) row1 = scale_row(next, lane);
+                    if constexpr (i == 30) gather_scale<QUANT>(raw, row1, a, lane);
+                    if constexpr (i == 32) row1 = rope_row(next, lane);
+                }
                 STEP_FENCE();
             });
-            gather_rope<QUANT>(raw, row1, a, lane);
+            if constexpr (GATHER) gather_rope<QUANT>(raw, row1, a, lane);
             if constexpr (QUANT)
                 if (__builtin_expect(prod.large, false)) plain_share(a, rows + tile * T + 8 * pair, present, smem + stage, pair, lane);
         };
-        u32x4 p, p1;
-        const uint8_t* pb;
+        u32x4 p[2];
         auto values = [&](int it) {
-            pb = pbuf + (it & 1) * (PAIRS * 2048) + fresh(lane) * 16;
-            p = *reinterpret_cast<const u32x4*>(pb);
+            const uint8_t* pb = pbuf + (it & 1) * (PAIRS * 2048) + fresh(lane) * 16;
+#pragma unroll
+            for (int b = 0; b < 2; ++b) p[b] = *reinterpret_cast<const u32x4*>(pb + 1024 * b);
             val.ahead(smem, st_old);
-            if (__builtin_amdgcn_readfirstlane(flag_lds[(it & 1) * PAIRS])) val.scale(alpha_lds[(it & 1) * (PAIRS * 32) + (fresh(lane) & 31)]);
+            if (__builtin_amdgcn_readfirstlane(flag_lds[(it & 1) * PAIRS])) {
+                const float* al = alpha_lds + (it & 1) * (PAIRS * 32) + (fresh(lane) & 15);
+                val.scale(al[0], al[16]);
+            }
             STEP_FENCE();
         };
         auto value_step = [&](auto nc) {
             constexpr int n = nc;
-            if constexpr (n == STEPS / 2 - 2) p1 = *reinterpret_cast<const u32x4*>(pb + 1024);
-            val.template step<n>(smem, n < STEPS / 2 ? p : p1);
+            val.template step<n>(smem, p);
             STEP_FENCE();
         };
         auto nothing = [](auto) {};
-        if (ntiles > 0) produce(0, 0, nothing);
+        if (ntiles > 0) produce(raw0, std::false_type{}, 0, 0, nothing);
         __syncthreads(); // tile 0 stored, Q parked
+        val.init(lane);  // (while the score wave has the first tile)
         if (ntiles > 0) {
-            if (last > 0) produce(1, st_new, nothing);
+            if (last > 0) produce(raw, std::true_type{}, 1, st_new, nothing);
             __syncthreads();
             turn();
             __builtin_amdgcn_s_setprio(1); // (the score wave is the older one of the SIMD and would take every slot)
             for (int it = 1; it < last; ++it) {
                 values(it - 1);
-                produce(it + 1, st_new, [&](auto ic) {
+                produce(raw, std::true_type{}, it + 1, st_new, [&](auto ic) {
                     constexpr int i = ic, n0 = i * STEPS / PIECES, n1 = (i + 1) * STEPS / PIECES;
                     if constexpr (n1 > n0) value_step(std::integral_constant<int, n0>{});
                 });
@@ -759,23 +804,30 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
     // The score waves publish the row sums; every wave normalises its own blocks.
     __syncthreads(); // nobody reads a tile, P~ or a factor any more
     if constexpr (SCORES) {
-        if (hl == 0) {
-            lsum[l32] = l_tot;
-            if (a.nsplit > 1 && head < a.nq) {
-                const int64_t prow = ((int64_t)tq * a.nsplit + sp) * a.nq + head;
-                a.part_ml[prow * 2] = m_out;
-                a.part_ml[prow * 2 + 1] = l_tot;
+        if (g == 0) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                lsum[16 * b + l16] = l_tot[b];
+                if (a.nsplit > 1 && head + 16 * b < a.nq) {
+                    const int64_t prow = ((int64_t)tq * a.nsplit + sp) * a.nq + head + 16 * b;
+                    a.part_ml[prow * 2] = m_out[b];
+                    a.part_ml[prow * 2 + 1] = l_tot[b];
+                }
             }
         }
     }
     __syncthreads();
-    if constexpr (!SCORES) l_tot = lsum[l32];
-    const float mul = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    float mul[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        if constexpr (!SCORES) l_tot[b] = lsum[16 * b + l16];
+        mul[b] = l_tot[b] > 0.f ? 1.f / l_tot[b] : 0.f;
+    }
     if (a.nsplit > 1) {
         if (active) val.store_partial(a.part_o + ((((int64_t)tq * a.nsplit + sp) * gridDim.z + hz) * 8 + (pair >> 1)) * 8192 + (pair & 1) * 4096 + lane * 8, mul);
         return;
     }
-    val.stage_rows(smem + hrow * OUT_ROW, hrow, hl, mul);
+    val.stage_rows(smem + pair * 32 * OUT_ROW, l16, g, mul);
     __syncthreads();
     // a wavefront copies whole rows, one per instruction
     const int row0 = pair * 32 + (SCORES ? 0 : 16);
@@ -803,7 +855,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * WAVES, 64 * WAVES), a
     extern __shared__ __align__(16) uint8_t smem[];
     uint32_t* tmask = reinterpret_cast<uint32_t*>(smem + SPLIT_OFF);
     int* rows = reinterpret_cast<int*>(smem + SPLIT_OFF + tmask_bytes(a.split_cap));
-    int* bt_lds = reinterpret_cast<int*>(smem);
+    int* bt_lds = reinterpret_cast<int*>(smem + BT_OFF);
     // both roles run the same barrier sequence
     if (threadIdx.x < 64 * PAIRS)
         sfa_wave<QUANT, true>(a, smem, tmask, rows, bt_lds, threadIdx.x);
@@ -820,9 +872,9 @@ __global__ void sfa_zero_kernel(uint32_t* out, int64_t n_words)
 
 // out[row, :] = sum_s (2^(m_s - M) l_s / L) o_s[row, :] with L = sum_s 2^(m_s - M) l_s and o_s the split's normalised
 // output.  The partials lie in the fragment order the attention kernel's accumulators have (see its epilogue).  One
-// workgroup merges, for one token, what the attention workgroups left for column group wv / 2, head half wv % 2 and head
-// block hb: 32 heads x 128 value columns; its wavefront i takes column block i, a lane owning for its head (l32) the four 4-column runs at
-// 32 i + 16 h + 8 g + 4 hl.  Splits are taken G at a time (G = 2, 4 or 8: the smallest that covers the split count,
+// workgroup merges, for one token, what the attention workgroups left for column group wv / 2 and pair 2 (wv % 2) + hb: 32 heads x
+// 128 value columns; its wavefront i takes 32 columns, a lane owning for its two heads (16 b + l16) the two 4-column runs at
+// 32 i + 16 j + 4 g.  Splits are taken G at a time (G = 2, 4 or 8: the smallest that covers the split count,
 // eight for more than eight splits), every load of a group requested before any is used (splits past the last are the
 // last again with weight 0).  The workgroup then turns its 32 x 128 block through LDS
 // and writes the 256-byte row pieces, 16 lanes a piece.
@@ -834,7 +886,7 @@ __global__ __launch_bounds__(256) void sfa_combine_kernel(const void* __restrict
 {
     __shared__ __align__(16) uint8_t tr[32 * CROW];
     const _Float16* part_o = static_cast<const _Float16*>(part_o_fp16); // (a plain pointer type keeps the symbol readable)
-    const int lane = threadIdx.x & 63, l32 = lane & 31, hl = lane >> 5;
+    const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
     const int i = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int task = blockIdx.x; // ((tq * hgroups + hz) * 8 + wv) * 2 + hb
     const int hb = task & 1, wv = (task >> 1) & 7;
@@ -842,58 +894,61 @@ __global__ __launch_bounds__(256) void sfa_combine_kernel(const void* __restrict
     const int hh = wv & 1, dq = wv >> 1;
     const int head_base = hz * HEADS_PER_WG + 64 * hh + 32 * hb;
     if (head_base >= nq) return; // (a head block past the last head: nothing was written for it)
-    const int headc = min(head_base + l32, nq - 1);
     float acc[2][8];
 #pragma unroll
     for (int x = 0; x < 16; ++x) (&acc[0][0])[x] = 0.f;
-    float M = -INFINITY, L = 0.f;
+    float M[2] = {-INFINITY, -INFINITY}, L[2] = {0.f, 0.f};
     const int64_t split_stride = (int64_t)hgroups * 8 * 8192; // fp16 elements between two splits of a token
     const _Float16* frag0 = part_o + (((int64_t)tq * nsplit * hgroups + hz) * 8 + wv) * 8192 + (hb * 4 + i) * 1024; // (the workgroup's four wavefronts read 8 KB in a row per split)
-    const float* ml0 = part_ml + (int64_t)tq * nsplit * nq * 2;
+    const float2* ml0 = reinterpret_cast<const float2*>(part_ml) + (int64_t)tq * nsplit * nq;
     for (int s0 = 0; s0 < nsplit; s0 += G) {
         f16x8 v[G][2];
-        float m[G], l[G];
+        float2 ml[G][2];
 #pragma unroll
         for (int j = 0; j < G; ++j) {
             const int s = min(s0 + j, nsplit - 1);
             const _Float16* base = frag0 + s * split_stride;
 #pragma unroll
-            for (int h = 0; h < 2; ++h) v[j][h] = *reinterpret_cast<const f16x8*>(base + h * 512 + lane * 8);
-            m[j] = ml0[((int64_t)s * nq + headc) * 2];
-            l[j] = s0 + j < nsplit ? ml0[((int64_t)s * nq + headc) * 2 + 1] : 0.f;
-        }
-        // the group's maximum joins the running one: what was summed so far is rescaled once per group
-        float Mg = M;
-#pragma unroll
-        for (int j = 0; j < G; ++j) Mg = l[j] > 0.f ? fmaxf(Mg, m[j]) : Mg;
-        if (Mg != -INFINITY) { // (otherwise nothing attended in these splits)
-            if (s0 > 0) {
-                const float back = exp2f(M - Mg); // 0 while nothing has been summed (M = -inf)
-                L *= back;
-#pragma unroll
-                for (int x = 0; x < 16; ++x) (&acc[0][0])[x] *= back;
+            for (int b = 0; b < 2; ++b) {
+                v[j][b] = *reinterpret_cast<const f16x8*>(base + b * 512 + lane * 8);
+                ml[j][b] = ml0[(int64_t)s * nq + min(head_base + 16 * b + l16, nq - 1)];
+                if (s0 + j >= nsplit) ml[j][b].y = 0.f;
             }
-            M = Mg;
+        }
 #pragma unroll
-            for (int j = 0; j < G; ++j) {
-                const float w = l[j] > 0.f ? exp2f(m[j] - M) * l[j] : 0.f;
-                L += w;
+        for (int b = 0; b < 2; ++b) {
+            // the group's maximum joins the running one: what was summed so far is rescaled once per group
+            float Mg = M[b];
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
+            for (int j = 0; j < G; ++j) Mg = ml[j][b].y > 0.f ? fmaxf(Mg, ml[j][b].x) : Mg;
+            if (Mg != -INFINITY) { // (otherwise nothing attended in these splits)
+                if (s0 > 0) {
+                    const float back = exp2f(M[b] - Mg); // 0 while nothing has been summed (M = -inf)
+                    L[b] *= back;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) acc[h][e] += (float)v[j][h][e] * w;
+                    for (int e = 0; e < 8; ++e) acc[b][e] *= back;
+                }
+                M[b] = Mg;
+#pragma unroll
+                for (int j = 0; j < G; ++j) {
+                    const float w = ml[j][b].y > 0.f ? exp2f(ml[j][b].x - Mg) * ml[j][b].y : 0.f;
+                    L[b] += w;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) acc[b][e] += (float)v[j][b][e] * w;
+                }
             }
         }
     }
-    const float inv = L > 0.f ? 1.f / L : 0.f;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int b = 0; b < 2; ++b) {
+        const float inv = L[b] > 0.f ? 1.f / L[b] : 0.f;
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            const float* x = &acc[h][4 * g];
+        for (int j = 0; j < 2; ++j) {
+            const float* x = &acc[b][4 * j];
             const u32x2 w = {pack_bf16x2(x[0] * inv, x[1] * inv), pack_bf16x2(x[2] * inv, x[3] * inv)};
-            *reinterpret_cast<u32x2*>(tr + l32 * CROW + (32 * i + 16 * h + 8 * g + 4 * hl) * 2) = w;
+            *reinterpret_cast<u32x2*>(tr + (16 * b + l16) * CROW + (32 * i + 16 * j + 4 * g) * 2) = w;
         }
+    }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
