@@ -64,10 +64,11 @@ struct SfaPlan {
     uint64_t ws_bytes;
 };
 
-// Common checks of both attention entry points once the cache streams are resolved.
+// Common checks of both attention entry points once the cache streams are resolved.  scratch: bytes of workspace there are, which the
+// choice of the KV splits keeps to where it has one.
 int plan_sfa(const char* op, const PtoTensorDesc& qn, const PtoTensorDesc& qr, const PtoTensorDesc& tk,
              const PtoTensorDesc& bt, const PtoTensorDesc& act, const PtoTensorDesc& out, int64_t out_rows,
-             const PtoSfaParams* p, SfaPlan* plan)
+             const PtoSfaParams* p, SfaPlan* plan, uint64_t scratch)
 {
     if (p == nullptr) return fail(PTO_ERR_PARAM, "%s: params is null", op);
     if (p->nq <= 0) return fail(PTO_ERR_PARAM, "%s: nq must be positive, got %d", op, p->nq);
@@ -108,10 +109,10 @@ int plan_sfa(const char* op, const PtoTensorDesc& qn, const PtoTensorDesc& qr, c
     a.block_size = p->block_size;
     a.bt_stride = (int32_t)bt.shape[1];
     a.softmax_scale = p->softmax_scale;
-    a.nsplit = p->kv_splits > 0 ? p->kv_splits : pto::sfa_pick_splits((int)t, p->nq, p->topk);
+    a.splits = p->kv_splits > 0 ? pto::SfaSplits{(int32_t)t, p->kv_splits, p->kv_splits} : pto::sfa_pick_splits((int)t, p->nq, p->topk, scratch);
     a.part_o = nullptr;
     a.part_ml = nullptr;
-    plan->ws_bytes = pto::sfa_workspace_bytes((int)t, p->nq, a.nsplit);
+    plan->ws_bytes = pto::sfa_workspace_bytes((int)t, p->nq, a.splits);
     return PTO_OK;
 }
 
@@ -123,11 +124,11 @@ int bind_workspace(const char* op, SfaPlan* plan, void* ws, uint64_t ws_bytes)
                     (unsigned long long)plan->ws_bytes, (unsigned long long)(ws ? ws_bytes : 0));
     pto::SfaArgs& a = plan->args;
     a.part_o = static_cast<_Float16*>(ws);
-    a.part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + pto::sfa_partials_bytes(a.b * a.s1, a.nq, a.nsplit));
+    a.part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + pto::sfa_partials_bytes(a.b * a.s1, a.nq, a.splits));
     return PTO_OK;
 }
 
-int plan_sfa_quant(const PtoTensorDesc* ts, uint32_t n, const PtoSfaParams* p, SfaPlan* plan)
+int plan_sfa_quant(const PtoTensorDesc* ts, uint32_t n, const PtoSfaParams* p, SfaPlan* plan, uint64_t scratch)
 {
     const char* op = "sparse_flash_attention_quant";
     if (ts == nullptr || n != 9) return fail(PTO_ERR_ARG_COUNT, "%s: expected 9 tensors, got %u", op, n);
@@ -152,7 +153,7 @@ int plan_sfa_quant(const PtoTensorDesc* ts, uint32_t n, const PtoSfaParams* p, S
     if (n_rows > 0x7fffffff) return fail(PTO_ERR_SHAPE, "%s: cache has too many rows", op);
     if (p && ts[8].shape[2] != p->nq) return fail(PTO_ERR_SHAPE, "%s: attention_out dim 2 must equal nq", op);
     const int64_t out_rows = ts[8].shape[0] * ts[8].shape[1] * ts[8].shape[2];
-    if ((rc = plan_sfa(op, ts[0], ts[1], ts[5], ts[6], ts[7], ts[8], out_rows, p, plan))) return rc;
+    if ((rc = plan_sfa(op, ts[0], ts[1], ts[5], ts[6], ts[7], ts[8], out_rows, p, plan, scratch))) return rc;
     if (ts[8].shape[0] != plan->args.b) return fail(PTO_ERR_SHAPE, "%s: attention_out dim 0 must equal the batch", op);
     pto::SfaArgs& a = plan->args;
     a.quant = quant;
@@ -166,7 +167,7 @@ int plan_sfa_quant(const PtoTensorDesc* ts, uint32_t n, const PtoSfaParams* p, S
     return PTO_OK;
 }
 
-int plan_sfa_antiquant(const PtoTensorDesc* ts, uint32_t n, const PtoSfaParams* p, SfaPlan* plan)
+int plan_sfa_antiquant(const PtoTensorDesc* ts, uint32_t n, const PtoSfaParams* p, SfaPlan* plan, uint64_t scratch)
 {
     const char* op = "sparse_attention_antiquant";
     if (ts == nullptr || n != 7) return fail(PTO_ERR_ARG_COUNT, "%s: expected 7 tensors, got %u", op, n);
@@ -181,7 +182,7 @@ int plan_sfa_antiquant(const PtoTensorDesc* ts, uint32_t n, const PtoSfaParams* 
     if (ts[2].shape[1] != 656) return fail(PTO_ERR_SHAPE, "%s: nope_cache rows must be 656 bytes, got %lld", op, (long long)ts[2].shape[1]);
     if (ts[6].shape[1] != 512) return fail(PTO_ERR_SHAPE, "%s: attention_out last dim must be 512", op);
     if (ts[2].shape[0] > 0x7fffffff) return fail(PTO_ERR_SHAPE, "%s: cache has too many rows", op);
-    if ((rc = plan_sfa(op, ts[0], ts[1], ts[3], ts[4], ts[5], ts[6], ts[6].shape[0], p, plan))) return rc;
+    if ((rc = plan_sfa(op, ts[0], ts[1], ts[3], ts[4], ts[5], ts[6], ts[6].shape[0], p, plan, scratch))) return rc;
     pto::SfaArgs& a = plan->args;
     a.quant = true;
     a.kn = static_cast<const uint8_t*>(ts[2].addr);
@@ -941,14 +942,14 @@ static int select_experts_launch_async(const PtoTensorDesc* tensors, uint32_t n_
 uint64_t pto_sfa_quant_workspace(const PtoTensorDesc* tensors, uint32_t n_tensors, const PtoSfaParams* params)
 {
     SfaPlan plan;
-    return plan_sfa_quant(tensors, n_tensors, params, &plan) == PTO_OK ? plan.ws_bytes : 0;
+    return plan_sfa_quant(tensors, n_tensors, params, &plan, UINT64_MAX) == PTO_OK ? plan.ws_bytes : 0;
 }
 
 static int sfa_quant_launch_async(const PtoTensorDesc* tensors, uint32_t n_tensors, const PtoSfaParams* params, void* workspace,
                          uint64_t workspace_bytes, void* hip_stream)
 {
     SfaPlan plan;
-    int rc = plan_sfa_quant(tensors, n_tensors, params, &plan);
+    int rc = plan_sfa_quant(tensors, n_tensors, params, &plan, workspace ? workspace_bytes : 0);
     if (rc) return rc;
     return launch_sfa("sparse_flash_attention_quant", &plan, workspace, workspace_bytes, hip_stream);
 }
@@ -958,7 +959,7 @@ int pto_sfa_quant_launch_noalloc(const PtoTensorDesc* tensors, uint32_t n_tensor
 {
     const char* op = "sparse_flash_attention_quant (no-allocation entry)";
     SfaPlan plan;
-    int rc = plan_sfa_quant(tensors, n_tensors, params, &plan);
+    int rc = plan_sfa_quant(tensors, n_tensors, params, &plan, pto::SFA_STATIC_SCRATCH_BYTES);
     if (rc) return rc;
     if (plan.ws_bytes > pto::SFA_STATIC_SCRATCH_BYTES)
         return fail(PTO_ERR_WORKSPACE, "%s: this problem needs %llu bytes of scratch, the library's own scratch array holds %llu; use pto_sfa_quant_launch with a workspace",
@@ -974,14 +975,14 @@ int pto_sfa_quant_launch_noalloc(const PtoTensorDesc* tensors, uint32_t n_tensor
 uint64_t pto_sfa_antiquant_workspace(const PtoTensorDesc* tensors, uint32_t n_tensors, const PtoSfaParams* params)
 {
     SfaPlan plan;
-    return plan_sfa_antiquant(tensors, n_tensors, params, &plan) == PTO_OK ? plan.ws_bytes : 0;
+    return plan_sfa_antiquant(tensors, n_tensors, params, &plan, UINT64_MAX) == PTO_OK ? plan.ws_bytes : 0;
 }
 
 static int sfa_antiquant_launch_async(const PtoTensorDesc* tensors, uint32_t n_tensors, const PtoSfaParams* params,
                              void* workspace, uint64_t workspace_bytes, void* hip_stream)
 {
     SfaPlan plan;
-    int rc = plan_sfa_antiquant(tensors, n_tensors, params, &plan);
+    int rc = plan_sfa_antiquant(tensors, n_tensors, params, &plan, workspace ? workspace_bytes : 0);
     if (rc) return rc;
     return launch_sfa("sparse_attention_antiquant", &plan, workspace, workspace_bytes, hip_stream);
 }

@@ -36,6 +36,7 @@
 //
 // KV splits write their output normalised by their own sum as fp16, in the accumulators' fragment order, plus (m, l);
 // sfa_combine_kernel merges them and turns the result into rows.
+#include <algorithm>
 #include <utility>
 
 #include "common.h"
@@ -291,17 +292,17 @@ __device__ __forceinline__ SplitRange split_range(int cur, int nsplit, int sp)
 // the tile's validity word), in LDS.  NT lanes.  The sequence's length, its page table and the share's top-k entries
 // are requested together: the entries are fetched for the share a full list would give (the usual case) and only
 // fetched again if the length, once known, moves the share.  The other waves pass its two barriers beside it.  Returns the share.
-__device__ __forceinline__ SplitRange share_of(const SfaArgs& a, int act, int si, int sp)
+__device__ __forceinline__ SplitRange share_of(const SfaArgs& a, int act, int si, int nsplit, int sp)
 {
-    return split_range(min(max(act - a.s1 + 1 + si, 0), a.topk), a.nsplit, sp);
+    return split_range(min(max(act - a.s1 + 1 + si, 0), a.topk), nsplit, sp);
 }
 template <int NT>
-__device__ __forceinline__ SplitRange resolve_split(const SfaArgs& a, int bi, int si, int tq, int sp, uint32_t* tmask,
+__device__ __forceinline__ SplitRange resolve_split(const SfaArgs& a, int bi, int si, int tq, int nsplit, int sp, uint32_t* tmask,
                                                     int* rows, int* bt_lds, int tid, int lane)
 {
     constexpr int PER_LANE = MAX_SPLIT_TOKENS / NT;
     const int32_t* list = a.topk_idx + (int64_t)tq * a.topk_stride;
-    const SplitRange guess = split_range(a.topk, a.nsplit, sp);
+    const SplitRange guess = split_range(a.topk, nsplit, sp);
     int my_idx[PER_LANE];
     auto fetch = [&](int tok0) {
 #pragma unroll
@@ -325,7 +326,7 @@ __device__ __forceinline__ SplitRange resolve_split(const SfaArgs& a, int bi, in
         for (int j = 0; j < BT_PER_LANE; ++j)
             if (tid + NT * j < a.bt_stride) bt_lds[tid + NT * j] = btv[j];
     }
-    const SplitRange r = share_of(a, act, si, sp);
+    const SplitRange r = share_of(a, act, si, nsplit, sp);
     if (r.tile0 != guess.tile0) fetch(r.tile0 * T); // block-uniform
     const int tok0 = r.tile0 * T;
     const int ntiles_even = (r.ntiles + 1) & ~1; // whole wavefronts of entries
@@ -512,7 +513,17 @@ __device__ __forceinline__ void copy_to_lds(const void* base, uint32_t offset, u
 template <bool QUANT, bool SCORES>
 __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32_t* tmask, int* rows, int* bt_lds, int tid)
 {
-    const int tq = blockIdx.x, sp = blockIdx.y, hz = blockIdx.z;
+    int tq = blockIdx.x, sp = blockIdx.y, nsplit = gridDim.y;
+    const int hz = blockIdx.z;
+    if (a.mixed) { // the tokens before t1 first, split by split, then the others
+        const int w1 = a.splits.t1 * a.splits.first;
+        const bool first = tq < w1;
+        const int w = first ? tq : tq - w1, tokens = first ? a.splits.t1 : a.b * a.s1 - a.splits.t1;
+        nsplit = first ? a.splits.first : a.splits.rest;
+        sp = w / tokens;
+        tq = w - sp * tokens + (first ? 0 : a.splits.t1);
+    }
+    const int64_t part = a.mixed ? a.splits.partial(tq) : (int64_t)tq * nsplit;
     const int bi = tq / a.s1, si = tq - bi * a.s1;
     const int lane = tid & 63, pair = __builtin_amdgcn_readfirstlane(tid >> 6) & (PAIRS - 1); // (scalar: what follows from it is too)
     const int l16 = lane & 15, g = lane >> 4;
@@ -545,7 +556,7 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
             copy_to_lds(static_cast<const uint8_t*>(a.q_rope) + qrow0 * (DR * 2),
                         (uint32_t)(min(head0 + 32 * pair + h, a.nq - 1) * (DR * 2) + (((lane & 7) ^ ((h >> 1) & 7)) * 16)), qrows + 32 * DN * 2 + i * 1024);
         }
-        share = share_of(a, act, si, sp);
+        share = share_of(a, act, si, nsplit, sp);
         __syncthreads(); // (the look-up's)
         __syncthreads(); // rows[] / tmask[] ready
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -571,7 +582,7 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
                 q[SCORES ? i - i / PARK_EVERY : 0] = v;
         }
     } else {
-        share = resolve_split<NT>(a, bi, si, tq, sp, tmask, rows, bt_lds, ht, lane);
+        share = resolve_split<NT>(a, bi, si, tq, nsplit, sp, tmask, rows, bt_lds, ht, lane);
         if (share.ntiles > 0) {
             gather_tile<QUANT>(raw0, a, rows + 8 * pair, lane);
             gather_tile<QUANT>(raw, a, rows + min(1, share.ntiles - 1) * T + 8 * pair, lane);
@@ -636,6 +647,7 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
                 if constexpr (n + KD < QFRAGS) fetch_k(std::integral_constant<int, n + KD>{});
                 STEP_FENCE();
             });
+            val.ahead(smem, st); // (this tile's values, behind the barrier)
             const uint32_t valid = __builtin_amdgcn_readfirstlane(present);
             if (valid != 0xffffffffu) {
                 // register e of s0[rb][b] holds row 16 rb + 4 g + e for head 16 b + l16 (the lanes' shift first: the bit
@@ -707,7 +719,6 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
             __syncthreads();
             turn();
             for (int it = 1; it < ntiles; ++it) {
-                val.ahead(smem, st_old);
                 unroll<KD>(fetch_k);
                 if (rescale) val.scale(alpha[0], alpha[1]);
                 val.add(smem, p);
@@ -715,7 +726,6 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
                 __syncthreads();
                 turn();
             }
-            val.ahead(smem, st_old);
             if (rescale) val.scale(alpha[0], alpha[1]);
             val.add(smem, p);
         }
@@ -760,7 +770,6 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
             const uint8_t* pb = pbuf + (it & 1) * (PAIRS * 2048) + fresh(lane) * 16;
 #pragma unroll
             for (int b = 0; b < 2; ++b) p[b] = *reinterpret_cast<const u32x4*>(pb + 1024 * b);
-            val.ahead(smem, st_old);
             if (__builtin_amdgcn_readfirstlane(flag_lds[(it & 1) * PAIRS])) {
                 const float* al = alpha_lds + (it & 1) * (PAIRS * 32) + (fresh(lane) & 15);
                 val.scale(al[0], al[16]);
@@ -778,21 +787,24 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
         val.init(lane);  // (while the score wave has the first tile)
         if (ntiles > 0) {
             if (last > 0) produce(raw, std::true_type{}, 1, st_new, nothing);
+            val.ahead(smem, st); // (this tile's values, behind the barrier)
             __syncthreads();
             turn();
             __builtin_amdgcn_s_setprio(1); // (the score wave is the older one of the SIMD and would take every slot)
             for (int it = 1; it < last; ++it) {
                 values(it - 1);
                 produce(raw, std::true_type{}, it + 1, st_new, [&](auto ic) {
-                    constexpr int i = ic, n0 = i * STEPS / PIECES, n1 = (i + 1) * STEPS / PIECES;
+                    constexpr int i = ic, n0 = i < 3 ? 0 : (i - 3) * STEPS / (PIECES - 3), n1 = i < 3 ? 0 : (i - 2) * STEPS / (PIECES - 3);
                     if constexpr (n1 > n0) value_step(std::integral_constant<int, n0>{});
                 });
+                val.ahead(smem, st);
                 __syncthreads();
                 turn();
             }
             if (last > 0) {
                 values(last - 1);
                 unroll<STEPS>(value_step);
+                val.ahead(smem, st);
                 __syncthreads();
                 turn();
             }
@@ -808,8 +820,8 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
                 lsum[16 * b + l16] = l_tot[b];
-                if (a.nsplit > 1 && head + 16 * b < a.nq) {
-                    const int64_t prow = ((int64_t)tq * a.nsplit + sp) * a.nq + head + 16 * b;
+                if (nsplit > 1 && head + 16 * b < a.nq) {
+                    const int64_t prow = (part + sp) * a.nq + head + 16 * b;
                     a.part_ml[prow * 2] = m_out[b];
                     a.part_ml[prow * 2 + 1] = l_tot[b];
                 }
@@ -823,8 +835,8 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
         if constexpr (!SCORES) l_tot[b] = lsum[16 * b + l16];
         mul[b] = l_tot[b] > 0.f ? 1.f / l_tot[b] : 0.f;
     }
-    if (a.nsplit > 1) {
-        if (active) val.store_partial(a.part_o + ((((int64_t)tq * a.nsplit + sp) * gridDim.z + hz) * 8 + (pair >> 1)) * 8192 + (pair & 1) * 4096 + lane * 8, mul);
+    if (nsplit > 1) {
+        if (active) val.store_partial(a.part_o + (((part + sp) * gridDim.z + hz) * 8 + (pair >> 1)) * 8192 + (pair & 1) * 4096 + lane * 8, mul);
         return;
     }
     val.stage_rows(smem + pair * 32 * OUT_ROW, l16, g, mul);
@@ -845,8 +857,8 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
     }
 }
 
-// grid (query token, KV split, group of 128 heads).  Workgroups go to the XCDs round-robin in launch order, so with the
-// token as the fastest grid dimension the splits of one token run on one XCD (when the token count is a multiple of 8)
+// grid (query tokens, KV splits, groups of 128 heads); where the tokens do not all have the same splits, (their sum, 1, groups).  Workgroups go to the XCDs round-robin in launch order, so with the
+// token as the fastest dimension the splits of one token run on one XCD (when the token count is a multiple of 8)
 // and share its L2 for the token's queries.
 template <bool QUANT>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * WAVES, 64 * WAVES), amdgpu_waves_per_eu(2, 2))) void sfa_decode_kernel(
@@ -873,22 +885,18 @@ __global__ void sfa_zero_kernel(uint32_t* out, int64_t n_words)
 // out[row, :] = sum_s (2^(m_s - M) l_s / L) o_s[row, :] with L = sum_s 2^(m_s - M) l_s and o_s the split's normalised
 // output.  The partials lie in the fragment order the attention kernel's accumulators have (see its epilogue).  One
 // workgroup merges, for one token, what the attention workgroups left for column group wv / 2 and pair 2 (wv % 2) + hb: 32 heads x
-// 128 value columns; its wavefront i takes 32 columns, a lane owning for its two heads (16 b + l16) the two 4-column runs at
-// 32 i + 16 j + 4 g.  Splits are taken G at a time (G = 2, 4 or 8: the smallest that covers the split count,
+// 128 value columns; its wavefront i takes 16 of the heads and 64 columns, a lane owning for its head (16 (i % 2) + l16) the four
+// 4-column runs at 16 j + 4 g of these.  Splits are taken G at a time (G = 2, 4 or 8: the smallest that covers the split count,
 // eight for more than eight splits), every load of a group requested before any is used (splits past the last are the
 // last again with weight 0).  The workgroup then turns its 32 x 128 block through LDS
 // and writes the 256-byte row pieces, 16 lanes a piece.
 constexpr int CROW = 128 * 2 + 16; // LDS row of the merge's transposition: 128 bf16 plus one 16-byte chunk of padding
 template <int G>
-__global__ __launch_bounds__(256) void sfa_combine_kernel(const void* __restrict__ part_o_fp16,
-                                                          const float* __restrict__ part_ml, void* out, int nq,
-                                                          int nsplit, int hgroups)
+__device__ __forceinline__ void merge_splits(const _Float16* part_o, const float* part_ml, void* out, int nq, int nsplit, int64_t partial, int hgroups,
+                                             int task, uint8_t* tr)
 {
-    __shared__ __align__(16) uint8_t tr[32 * CROW];
-    const _Float16* part_o = static_cast<const _Float16*>(part_o_fp16); // (a plain pointer type keeps the symbol readable)
     const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
     const int i = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int task = blockIdx.x; // ((tq * hgroups + hz) * 8 + wv) * 2 + hb
     const int hb = task & 1, wv = (task >> 1) & 7;
     const int th = task >> 4, hz = th % hgroups, tq = th / hgroups;
     const int hh = wv & 1, dq = wv >> 1;
@@ -897,58 +905,55 @@ __global__ __launch_bounds__(256) void sfa_combine_kernel(const void* __restrict
     float acc[2][8];
 #pragma unroll
     for (int x = 0; x < 16; ++x) (&acc[0][0])[x] = 0.f;
-    float M[2] = {-INFINITY, -INFINITY}, L[2] = {0.f, 0.f};
+    float M = -INFINITY, L = 0.f;
+    const int b = i & 1, cb = i & 2; // the wavefront's block of 16 heads and first of two column blocks
     const int64_t split_stride = (int64_t)hgroups * 8 * 8192; // fp16 elements between two splits of a token
-    const _Float16* frag0 = part_o + (((int64_t)tq * nsplit * hgroups + hz) * 8 + wv) * 8192 + (hb * 4 + i) * 1024; // (the workgroup's four wavefronts read 8 KB in a row per split)
-    const float2* ml0 = reinterpret_cast<const float2*>(part_ml) + (int64_t)tq * nsplit * nq;
+    const _Float16* frag0 = part_o + ((partial * hgroups + hz) * 8 + wv) * 8192 + hb * 4096 + cb * 1024 + b * 512; // (the workgroup's four wavefronts read 8 KB in a row per split)
+    const float2* ml0 = reinterpret_cast<const float2*>(part_ml) + partial * nq + min(head_base + 16 * b + l16, nq - 1);
     for (int s0 = 0; s0 < nsplit; s0 += G) {
         f16x8 v[G][2];
-        float2 ml[G][2];
+        float2 ml[G];
 #pragma unroll
         for (int j = 0; j < G; ++j) {
             const int s = min(s0 + j, nsplit - 1);
             const _Float16* base = frag0 + s * split_stride;
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                v[j][b] = *reinterpret_cast<const f16x8*>(base + b * 512 + lane * 8);
-                ml[j][b] = ml0[(int64_t)s * nq + min(head_base + 16 * b + l16, nq - 1)];
-                if (s0 + j >= nsplit) ml[j][b].y = 0.f;
-            }
+            for (int h = 0; h < 2; ++h) v[j][h] = *reinterpret_cast<const f16x8*>(base + h * 1024 + lane * 8);
+            ml[j] = ml0[(int64_t)s * nq];
+            if (s0 + j >= nsplit) ml[j].y = 0.f;
         }
+        // the group's maximum joins the running one: what was summed so far is rescaled once per group
+        float Mg = M;
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            // the group's maximum joins the running one: what was summed so far is rescaled once per group
-            float Mg = M[b];
+        for (int j = 0; j < G; ++j) Mg = ml[j].y > 0.f ? fmaxf(Mg, ml[j].x) : Mg;
+        if (Mg != -INFINITY) { // (otherwise nothing attended in these splits)
+            if (s0 > 0) {
+                const float back = exp2f(M - Mg); // 0 while nothing has been summed (M = -inf)
+                L *= back;
 #pragma unroll
-            for (int j = 0; j < G; ++j) Mg = ml[j][b].y > 0.f ? fmaxf(Mg, ml[j][b].x) : Mg;
-            if (Mg != -INFINITY) { // (otherwise nothing attended in these splits)
-                if (s0 > 0) {
-                    const float back = exp2f(M[b] - Mg); // 0 while nothing has been summed (M = -inf)
-                    L[b] *= back;
+                for (int x = 0; x < 16; ++x) (&acc[0][0])[x] *= back;
+            }
+            M = Mg;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) acc[b][e] *= back;
-                }
-                M[b] = Mg;
+            for (int j = 0; j < G; ++j) {
+                const float w = ml[j].y > 0.f ? exp2f(ml[j].x - M) * ml[j].y : 0.f;
+                L += w;
 #pragma unroll
-                for (int j = 0; j < G; ++j) {
-                    const float w = ml[j][b].y > 0.f ? exp2f(ml[j][b].x - Mg) * ml[j][b].y : 0.f;
-                    L[b] += w;
+                for (int h = 0; h < 2; ++h)
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) acc[b][e] += (float)v[j][b][e] * w;
-                }
+                    for (int e = 0; e < 8; ++e) acc[h][e] += (float)v[j][h][e] * w;
             }
         }
     }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        const float inv = L[b] > 0.f ? 1.f / L[b] : 0.f;
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const float* x = &acc[b][4 * j];
+            const float* x = &acc[h][4 * j];
             const u32x2 w = {pack_bf16x2(x[0] * inv, x[1] * inv), pack_bf16x2(x[2] * inv, x[3] * inv)};
-            *reinterpret_cast<u32x2*>(tr + (16 * b + l16) * CROW + (32 * i + 16 * j + 4 * g) * 2) = w;
+            *reinterpret_cast<u32x2*>(tr + (16 * b + l16) * CROW + (32 * (cb + h) + 16 * j + 4 * g) * 2) = w;
         }
-    }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -957,6 +962,27 @@ __global__ __launch_bounds__(256) void sfa_combine_kernel(const void* __restrict
         if (head_base + r < nq)
             *reinterpret_cast<u32x4*>(reinterpret_cast<uint8_t*>(out) + (((int64_t)tq * nq + head_base + r) * DN + 128 * dq + 8 * c) * 2) = w;
     }
+}
+
+// grid (tokens with several splits x head groups x 16), 256 lanes.  G of the tokens before t1 and of the others (0: these, or those, have
+// a single split); both in one launch: a second one for a few tokens costs more than the registers of the wider merge.
+template <int G1, int G2>
+__global__ __launch_bounds__(256) void sfa_combine_kernel(const void* __restrict__ part_o_fp16, const float* __restrict__ part_ml, void* out, int nq,
+                                                          SfaSplits splits, int hgroups)
+{
+    __shared__ __align__(16) uint8_t tr[32 * CROW];
+    const _Float16* part_o = static_cast<const _Float16*>(part_o_fp16); // (a plain pointer type keeps the symbol readable)
+    const int task = blockIdx.x + (G1 == 0 ? splits.t1 * hgroups * 16 : 0); // ((tq * hgroups + hz) * 8 + wv) * 2 + hb
+    const int tq = (task >> 4) / hgroups;
+    if constexpr (G1 != 0 && G2 != 0) {
+        if (tq < splits.t1)
+            merge_splits<G1>(part_o, part_ml, out, nq, splits.first, (int64_t)tq * splits.first, hgroups, task, tr);
+        else
+            merge_splits<G2>(part_o, part_ml, out, nq, splits.rest, splits.partial(tq), hgroups, task, tr);
+    } else if constexpr (G1 != 0)
+        merge_splits<G1>(part_o, part_ml, out, nq, splits.first, (int64_t)tq * splits.first, hgroups, task, tr);
+    else
+        merge_splits<G2>(part_o, part_ml, out, nq, splits.rest, (int64_t)(tq - splits.t1) * splits.rest, hgroups, task, tr);
 }
 
 int num_cus()
@@ -974,31 +1000,51 @@ int num_cus()
 
 } // namespace
 
-int sfa_pick_splits(int t, int nq, int topk)
+// The KV splits.  One number for all tokens: one workgroup to a CU, and no more than share the tiles as well - nine splits of 64 tiles
+// are eight tiles each like eight splits, but leave more partials, and a second group of them to the merge (26 tokens: 77.0 us a pass
+// with nine, 73.9 with eight).  Or two: whole rounds of workgroups of the first tokens, and as many splits of the rest as fill the CUs
+// once more.  300 tokens in one split each are two rounds, the second for 44 of them.  By the time that either should take, in ns:
+// a tile (where more CUs work, the chip's clock falls: 150 workgroups 1700, 200: 1780, 256: 2030), the two ends of a workgroup, a
+// partial result's way to memory and back, the merge's launch.
+// Prefill calls of 2048 rows a token, one split for each and so: 129 tokens 108 -> 99 us, 257: 239 -> 156, 300: 245 -> 175, 360:
+// 247 -> 207, 520: 391 -> 296, 700: 409 -> 396.  (Two splits for 128 tokens and the rest in more where that is less by the formula: 144 tokens
+// 109 us as before, 160 by one split each 117, by two 115.)
+constexpr int64_t TILE_NS = 1550, TILE_FULL_NS = 480, ENDS_NS = 7000, PARTIAL_NS = 45, MERGE_NS = 2500;
+SfaSplits sfa_pick_splits(int t, int nq, int topk, uint64_t scratch)
 {
-    const int hgroups = (nq + HEADS_PER_WG - 1) / HEADS_PER_WG;
+    const int hgroups = (nq + HEADS_PER_WG - 1) / HEADS_PER_WG, cus = std::max(1, num_cus() / hgroups); // (of a head group)
     const int tiles = (topk + T - 1) / T;
-    int n = num_cus() / (t * hgroups > 0 ? t * hgroups : 1);
-    n = n < 1 ? 1 : n;
-    n = n > tiles ? tiles : n;
-    n = n > 16 ? 16 : n;
-    // no more than share the tiles as well: nine splits of 64 tiles are eight tiles each like eight splits, but leave more
-    // partials, and a second group of them to the merge (26 tokens: 77.0 us a pass with nine, 73.9 with eight)
-    const int per = (tiles + n - 1) / n;
-    return (tiles + per - 1) / per;
+    auto even = [&](int n) { // no more splits than n, and no more than share the tiles as well
+        n = std::max(1, std::min({n, tiles, 16}));
+        const int per = (tiles + n - 1) / n;
+        return (tiles + per - 1) / per;
+    };
+    // w workgroups of a token's n-th part
+    auto round_ns = [&](int n, int64_t w) { return (tiles + n - 1) / n * (TILE_NS + TILE_FULL_NS * std::min<int64_t>(w, cus) * std::min<int64_t>(w, cus) / (cus * cus)) + ENDS_NS; };
+    auto partials_ns = [&](const SfaSplits& s) { return s.partials(t) > 0 ? s.partials(t) * hgroups * PARTIAL_NS + MERGE_NS : 0; };
+    const int n = even(cus / std::max(t, 1));
+    SfaSplits best = {t, n, n};
+    const int64_t wgs = (int64_t)t * n, whole = wgs / cus;
+    int64_t best_ns = whole * round_ns(n, cus) + (wgs > whole * cus ? round_ns(n, wgs - whole * cus) : 0) + partials_ns(best);
+    for (int first = 1; first <= 2; ++first) {
+        const int per_round = cus / first, rounds = per_round > 0 ? t / per_round : 0, t1 = rounds * per_round;
+        if (t1 == 0 || t1 == t || even(first) != first || (first > 1 && rounds > 1)) continue;
+        const SfaSplits s = {t1, first, even(cus / (t - t1))};
+        const int64_t ns = rounds * round_ns(first, cus) + round_ns(s.rest, (int64_t)(t - t1) * s.rest) + partials_ns(s);
+        if (ns < best_ns && sfa_workspace_bytes(t, nq, s) <= scratch) best = s, best_ns = ns;
+    }
+    return best;
 }
 
-uint64_t sfa_partials_bytes(int t, int nq, int nsplit)
+uint64_t sfa_partials_bytes(int t, int nq, const SfaSplits& splits)
 {
-    if (nsplit <= 1) return 0;
     const int hgroups = (nq + HEADS_PER_WG - 1) / HEADS_PER_WG; // (whole 128-head groups: the partials lie in fragment order)
-    return (uint64_t)t * nsplit * hgroups * HEADS_PER_WG * DN * sizeof(_Float16);
+    return (uint64_t)splits.partials(t) * hgroups * HEADS_PER_WG * DN * sizeof(_Float16);
 }
 
-uint64_t sfa_workspace_bytes(int t, int nq, int nsplit)
+uint64_t sfa_workspace_bytes(int t, int nq, const SfaSplits& splits)
 {
-    if (nsplit <= 1) return 0;
-    return sfa_partials_bytes(t, nq, nsplit) + (uint64_t)t * nsplit * nq * 2 * sizeof(float);
+    return sfa_partials_bytes(t, nq, splits) + (uint64_t)splits.partials(t) * nq * 2 * sizeof(float);
 }
 
 // Scratch for callers that cannot allocate (sfa_static_scratch): one array per GPU the library runs on, held until the
@@ -1041,7 +1087,8 @@ hipError_t sfa_launch(const SfaArgs& a, hipStream_t stream)
     while (((int64_t)1 << l) < a.block_size) ++l;
     args.page_mul = (uint32_t)((((uint64_t)1 << (31 + l)) + (uint32_t)a.block_size - 1) / (uint32_t)a.block_size);
     args.page_shift = 31 + l;
-    args.split_cap = (((tiles + a.nsplit - 1) / a.nsplit + 1) & ~1) * T;
+    const int fewest = a.splits.t1 == t ? a.splits.first : a.splits.t1 == 0 ? a.splits.rest : std::min(a.splits.first, a.splits.rest); // of a token
+    args.split_cap = (((tiles + fewest - 1) / fewest + 1) & ~1) * T;
     const int smem_bytes = SPLIT_OFF + split_bytes(args.split_cap);
     args.bt_cached = a.bt_stride <= BT_MAX ? 1 : 0;
     static DeviceOnce attr_done[2];
@@ -1054,18 +1101,29 @@ hipError_t sfa_launch(const SfaArgs& a, hipStream_t stream)
         if (e != hipSuccess) return e;
     }
     const int hgroups = (a.nq + HEADS_PER_WG - 1) / HEADS_PER_WG;
-    dim3 grid(t, a.nsplit, hgroups);
+    const int one = a.splits.t1 == t ? a.splits.first : a.splits.t1 == 0 || a.splits.first == a.splits.rest ? a.splits.rest : 0; // all tokens' splits
+    args.mixed = one == 0;
+    const int64_t wgs = (int64_t)a.splits.t1 * a.splits.first + (int64_t)(t - a.splits.t1) * a.splits.rest;
+    if (wgs > 0x7fffffff / (64 * WAVES)) return hipErrorInvalidValue;
+    const dim3 grid = one ? dim3(t, one, hgroups) : dim3((unsigned)wgs, 1, hgroups);
     {
         ScopedKernelTimer tm(KID_SFA_DECODE, stream);
         hipLaunchKernelGGL(kern, grid, dim3(64 * WAVES), smem_bytes, stream, args);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (a.nsplit > 1) {
+    const int n1 = a.splits.t1 > 0 && a.splits.first > 1 ? a.splits.first : 0, n2 = a.splits.t1 < t && a.splits.rest > 1 ? a.splits.rest : 0;
+    if (n1 || n2) {
         ScopedKernelTimer tm(KID_SFA_COMBINE, stream);
-        auto merge = a.nsplit <= 2 ? sfa_combine_kernel<2> : a.nsplit <= 4 ? sfa_combine_kernel<4> : sfa_combine_kernel<8>;
-        hipLaunchKernelGGL(merge, dim3(t * hgroups * 16), dim3(256), 0, stream, static_cast<const void*>(a.part_o),
-                           a.part_ml, a.out, a.nq, a.nsplit, hgroups);
+        const int tokens = (n1 ? a.splits.t1 : 0) + (n2 ? t - a.splits.t1 : 0);
+        auto group = [](int n) { return n == 0 ? 0 : n <= 2 ? 2 : n <= 4 ? 4 : 8; };
+        const int g1 = group(n1), g2 = group(n2);
+        // (two numbers of splits: the first is two)
+        auto merge = g1 && g2 ? (g2 <= 4 ? sfa_combine_kernel<2, 4> : sfa_combine_kernel<2, 8>)
+                   : g1 ? (g1 == 2 ? sfa_combine_kernel<2, 0> : g1 == 4 ? sfa_combine_kernel<4, 0> : sfa_combine_kernel<8, 0>)
+                        : (g2 == 2 ? sfa_combine_kernel<0, 2> : g2 == 4 ? sfa_combine_kernel<0, 4> : sfa_combine_kernel<0, 8>);
+        hipLaunchKernelGGL(merge, dim3(tokens * hgroups * 16), dim3(256), 0, stream, static_cast<const void*>(a.part_o),
+                           a.part_ml, a.out, a.nq, a.splits, hgroups);
         e = hipGetLastError();
     }
     return e;

@@ -216,6 +216,37 @@ def test_forced_kv_splits_agree(cuda):
         assert count_violations(o, outs[0], 2e-3, 2.0 ** -5) == 0
 
 
+@pytest.mark.parametrize("t,first,rest", [(18, 1, 8), (17, 1, 16), (35, 1, 5), (9, 2, 16)])
+def test_tokens_with_different_splits(cuda, t, first, rest):
+    """2048 heads are 16 workgroups a token: 16 tokens fill the CUs.  A few more than that, or than half of it in two splits each: the
+    first tokens in whole rounds, the rest in as many splits as fill the CUs once more - each the bits of a call with that many
+    splits for all.  Without the workspace that this asks for: one split for all, whose partial results need none."""
+    from pypto_amd import _runtime
+    case = osfa.make_case(t, 2048, 1, [2100] * t, topk=2048, seed=71, dist="bench", softmax_scale=192 ** -0.5)
+    lib = _runtime.load_library()
+    ts = [case["q"][..., :512].reshape(-1, 512).contiguous().to(cuda), case["q"][..., 512:].reshape(-1, 64).contiguous().to(cuda)]
+    ts += [case[k].to(cuda) for k in ("kn", "kr", "kn_scales", "topk_indices", "block_table")]
+    ts += [torch.tensor(case["act_seq"], dtype=torch.int32, device=cuda), torch.zeros((t, 1, 2048, 512), dtype=torch.bfloat16, device=cuda)]
+    d = _runtime.describe(ts)
+
+    def run(splits, own_workspace=True):
+        ts[8].fill_(float("nan"))
+        p = _runtime.SfaParams(2048, 1, case["softmax_scale"], 2048, case["block_size"], case["block_table"].shape[1], splits)
+        n = lib.pto_sfa_quant_workspace(d, 9, ctypes.byref(p))
+        ws = torch.empty(max(n, 1), dtype=torch.uint8, device=cuda)
+        stream = torch.cuda.current_stream().cuda_stream
+        rc = lib.pto_sfa_quant_launch(d, 9, ctypes.byref(p), ws.data_ptr() if own_workspace else None, n if own_workspace else 0, stream, 1)
+        assert rc == 0, lib.pto_last_error()
+        return n, ts[8].cpu()
+
+    whole = t // (16 // first) * (16 // first)
+    n, out = run(0)
+    assert n == (whole * (first if first > 1 else 0) + (t - whole) * rest) * 2048 * (512 * 2 + 8)
+    assert torch.equal(out[:whole], run(first)[1][:whole]) and torch.equal(out[whole:], run(rest)[1][whole:])
+    one = run(1)[1]
+    assert torch.equal(run(0, own_workspace=False)[1], one)
+
+
 @pytest.mark.parametrize("nq,splits", [(128, 1), (128, 5), (33, 2), (1, 3)])
 def test_page_tables_around_the_widest_in_lds(cuda, nq, splits):
     """1280 entries lie in LDS while the shares are looked up, behind the query of four times 32 heads; 1281 are read from memory:
