@@ -561,8 +561,17 @@ __device__ __forceinline__ uint32_t block_suffix_sum(uint32_t v, uint32_t* tmp)
     __syncthreads();
     if (lane == 0) tmp[wave] = v;
     __syncthreads();
-    uint32_t add = 0;
-    for (int w = wave + 1; w < NWAVES; ++w) add += tmp[w];
+    // the totals of the wavefronts behind this one: one read, summed up between the lanes (up to 15 reads in a row took three times as
+    // long as all the rest)
+    static_assert(NWAVES == 4 || NWAVES == 16, "sums over lanes of a row that repeat");
+    uint32_t add = tmp[lane & (NWAVES - 1)];
+    add = (lane & (NWAVES - 1)) > wave ? add : 0u;
+    if constexpr (NWAVES == 16) {
+        add += dpp_from<0x128, 0xf>(add, 0u); // row_ror:8, 4
+        add += dpp_from<0x124, 0xf>(add, 0u);
+    }
+    add += dpp_from<0x122, 0xf>(add, 0u); // row_ror:2, 1
+    add += dpp_from<0x121, 0xf>(add, 0u);
     return v + add;
 }
 
@@ -742,11 +751,13 @@ __device__ __forceinline__ void radix_select64(Each&& for_each, Emit&& emit, uin
     }
 }
 
-// A word's group for ordering: a non-decreasing function of its key with values 0 .. 2047.  `kind` 0 cuts the scores'
+// A word's group for ordering: a non-decreasing function of its key with values 0 .. 2^BITS - 1.  `kind` 0 cuts the scores'
 // range into equal steps (rounding is monotone: neither the difference nor the product turns two scores around), kind 1
 // the range of their ordered keys - steps in proportion to the magnitude.
 __device__ __forceinline__ float key_to_score(uint32_t key) { return __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key); }
+template <int BITS>
 struct KeyGroups {
+    static constexpr uint32_t LAST = (1u << BITS) - 1u;
     uint32_t kmin, kmax;
     float fmin, per;
     int shift;
@@ -755,13 +766,13 @@ struct KeyGroups {
     {
         fmin = key_to_score(lo);
         const float span = key_to_score(hi) - fmin;
-        per = 2047.0f / span;
-        shift = max(0, 21 - (int)__builtin_clz((hi - lo) | 1u));
+        per = (float)LAST / span;
+        shift = max(0, 32 - BITS - (int)__builtin_clz((hi - lo) | 1u));
         linear_ok = span > 0.f && span < __builtin_inff() && per < __builtin_inff();
     }
     __device__ __forceinline__ uint32_t of(uint32_t key, int kind) const
     {
-        return kind == 0 ? min((uint32_t)((key_to_score(key) - fmin) * per), 2047u) : (key - kmin) >> shift;
+        return kind == 0 ? min((uint32_t)((key_to_score(key) - fmin) * per), LAST) : (key - kmin) >> shift;
     }
 };
 
@@ -772,49 +783,57 @@ struct KeyGroups {
 // selection ends.  If those crowd (more than GROUP_CAP words in one), equal steps of the keys; if these do too (heavily tied
 // scores), a bitonic sort.  (Steps of the keys alone crowd near zero, and a row whose selection reaches scores of both signs
 // then paid for the sort: 18 us against 8.)
-// Workgroup of 1024 lanes; buf has 1024 PER words, hist and start 2048, tmp 16.
+// 4096 groups: where the selection ends, which is where the scores of a bell are densest, 2048 hold 7 words on the average and up to 15
+// (8192: as many ticks won in the comparisons as lost in the scan).
+// Workgroup of 1024 lanes; buf has 1024 PER words, start ORDER_GROUPS (16-byte aligned), tmp 16.
 constexpr uint32_t GROUP_CAP = 64;
+constexpr int ORDER_BITS = 12, ORDER_GROUPS = 1 << ORDER_BITS;
 template <int PER, class Write>
-__device__ __forceinline__ void order_words(const uint64_t (&w)[PER], uint32_t m, uint32_t kmin, uint32_t kmax, uint64_t* buf, uint32_t* hist,
-                                            uint32_t* start, uint32_t* tmp, uint32_t* s_flag, int k, Write&& write)
+__device__ __forceinline__ void order_words(const uint64_t (&w)[PER], uint32_t m, uint32_t kmin, uint32_t kmax, uint64_t* buf, uint32_t* start,
+                                            uint32_t* tmp, uint32_t* s_flag, int k, Write&& write)
 {
     const int tid = threadIdx.x;
-    const KeyGroups groups(kmin, kmax);
+    const KeyGroups<ORDER_BITS> groups(kmin, kmax);
     uint32_t bin[PER];
     for (int kind = groups.linear_ok ? 0 : 1; kind < 2; ++kind) { // (block-uniform)
         __syncthreads();
-        hist[tid] = 0;
-        hist[tid + 1024] = 0;
+        reinterpret_cast<u32x4*>(start)[tid] = u32x4{0u, 0u, 0u, 0u};
         if (tid == 0) *s_flag = 0;
         __syncthreads();
 #pragma unroll
         for (int h = 0; h < PER; ++h) {
             bin[h] = groups.of((uint32_t)(w[h] >> 32), kind);
-            if ((uint32_t)(tid + 1024 * h) < m) atomicAdd(&hist[bin[h]], 1u);
+            if ((uint32_t)(tid + 1024 * h) < m) atomicAdd(&start[bin[h]], 1u);
         }
         __syncthreads();
         {
-            const uint32_t h_lo = hist[2 * tid], h_hi = hist[2 * tid + 1]; // lane t owns bins 2t and 2t+1
-            if (h_lo > GROUP_CAP || h_hi > GROUP_CAP) *s_flag = 1;
-            const uint32_t incl = block_suffix_sum<16>(h_lo + h_hi, tmp);
-            start[2 * tid + 1] = incl - h_lo - h_hi; // slots taken by the higher bins
-            start[2 * tid] = incl - h_lo;
+            const u32x4 c = reinterpret_cast<const u32x4*>(start)[tid]; // lane t owns groups 4 t .. 4 t + 3
+            if (max(max(c[0], c[1]), max(c[2], c[3])) > GROUP_CAP) *s_flag = 1;
+            const uint32_t incl = block_suffix_sum<16>((c[0] + c[1]) + (c[2] + c[3]), tmp);
+            // slots taken by the higher groups
+            const uint32_t s0 = incl - c[0], s1 = s0 - c[1], s2 = s1 - c[2];
+            reinterpret_cast<u32x4*>(start)[tid] = u32x4{s0, s1, s2, s2 - c[3]};
         }
         __syncthreads();
         if (*s_flag == 0) {
 #pragma unroll
             for (int h = 0; h < PER; ++h)
-                if ((uint32_t)(tid + 1024 * h) < m) buf[atomicAdd(&start[bin[h]], 1u)] = w[h]; // (start ends up as the bin's end)
+                if ((uint32_t)(tid + 1024 * h) < m) buf[atomicAdd(&start[bin[h]], 1u)] = w[h]; // (start ends up as the group's end)
             __syncthreads();
+            // By place now, so that neighbouring lanes compare neighbouring words and write next to each other.  (A word's own lane
+            // went all over LDS and the output for it: 5 K of the 32 K ticks of a row of 20000, this way 2 K.)
 #pragma unroll
-            for (int h = 0; h < PER; ++h)
-                if ((uint32_t)(tid + 1024 * h) < m) {
-                    const uint32_t c = hist[bin[h]], s0 = start[bin[h]] - c;
-                    if ((int)s0 >= k) continue;
-                    uint32_t rank = s0;
-                    for (uint32_t j = 0; j < c; ++j) rank += buf[s0 + j] > w[h] ? 1u : 0u;
-                    if ((int)rank < k) write((int)rank, w[h]);
-                }
+            for (int h = 0; h < PER; ++h) {
+                const uint32_t i = (uint32_t)(tid + 1024 * h);
+                if (i >= m) break;
+                const uint64_t x = buf[i];
+                const uint32_t b = groups.of((uint32_t)(x >> 32), kind);
+                const uint32_t s0 = b + 1 < ORDER_GROUPS ? start[b + 1] : 0u, end = start[b]; // (a group begins where the next higher one ends)
+                if ((int)s0 >= k) break;
+                uint32_t rank = s0;
+                for (uint32_t j = s0; j < end; ++j) rank += buf[j] > x ? 1u : 0u;
+                if ((int)rank < k) write((int)rank, x);
+            }
             return;
         }
     }
@@ -871,7 +890,7 @@ __global__ __launch_bounds__(1024) void indexer_topk_kernel(IndexerArgs a)
 {
     __shared__ uint32_t hist[NBINS];
     __shared__ uint64_t cand[MAX_K];
-    __shared__ uint64_t tie[TIE_CAP];
+    __shared__ __align__(16) uint64_t tie[TIE_CAP];
     __shared__ uint32_t tmp[16];
     __shared__ uint32_t s_bin, s_krem, s_cnt, s_out;
 
@@ -1010,7 +1029,7 @@ __global__ __launch_bounds__(1024) void indexer_topk_kernel(IndexerArgs a)
         }
     }
     block_key_range(kmin, kmax, tmp);
-    order_words<2>(w, m, kmin, kmax, cand, hist, reinterpret_cast<uint32_t*>(tie), tmp, &s_bin, k,
+    order_words<2>(w, m, kmin, kmax, cand, reinterpret_cast<uint32_t*>(tie), tmp, &s_bin, k,
                    [&](int rank, uint64_t word) { out[rank] = word_index(word); });
 }
 
@@ -1065,20 +1084,23 @@ __global__ __launch_bounds__(1024) void topk_sort_kernel(const float* __restrict
 
 // The k (<= MAX_K) first words of a row in descending word order, by one workgroup of 1024 lanes in one pass over the row:
 // calls write(rank, word).  Bound by latency, not by bytes: a chain of memory round trips, LDS passes and barriers.
-//   1. ROW_SAMPLES elements, evenly spaced, are counted in equal steps of their scores' range; a suffix scan gives a pivot
-//      that somewhat more than k elements of the row should reach (four standard deviations of the sample count more).
+//   1. A sample, evenly spaced, is counted in equal steps of its scores' range; a suffix scan gives a pivot
+//      that somewhat more than k elements of the row should reach (four standard deviations of the sample count more).  Where the
+//      row is all in registers it is every fourth of a lane's elements, another fourth in each of four wavefronts: 4096 requested
+//      from memory one by one, a line each, took the memory pipe 4 K of the 32 K ticks of a row of 20000.  Longer rows pay that:
+//      four of a lane's (eight: 2 rows of 65536 24.6 us, not 23.0).
 //   2. The row - requested before anything else - is filtered: the words that reach the pivot go to
-//      LDS, a wavefront's with one counter update per 16 elements of a lane.
+//      LDS, a wavefront's with one counter update per 16 elements of a lane.  (16 wavefronts share four SIMDs: instructions bound
+//      this, so the index is looked at only where the row ends and the smallest key is the pivot, not a minimum.)
 //   3. If at least k and at most ROW_CAP did (else: row_select_exact), they are put in order by order_words, which drops
 //      those behind the k-th.
 // Rows of up to ROW_CAP elements skip 1 and keep everything.  NPT: elements per lane; 0: rows of any length, 32 elements per
 // lane (128 KB) in flight.  `VEC` consecutive elements go to one lane (4: `load4(i)`, 16-byte aligned and readable up to the next
 // multiple of 4096 elements, `cap`), so that the requests are wide.
-constexpr int ROW_CAP = 4096, ROW_SAMPLES = 4096;
+constexpr int ROW_CAP = 4096;
 struct RowLds {
     uint64_t buf[ROW_CAP];
-    uint32_t hist[NBINS];
-    uint32_t start[NBINS];
+    uint32_t hist[ORDER_GROUPS]; // (the sample's and the radix select's: the first NBINS)
     uint32_t tmp[16];
     uint32_t bin, krem, cnt, out;
 };
@@ -1148,25 +1170,47 @@ __device__ __forceinline__ void select_row(RowLds& lds, int cap, int k, Load&& l
     }
     uint32_t pivot = 0u;
     if (n > ROW_CAP) { // block-uniform
-        constexpr int PER = ROW_SAMPLES / 1024;
+        float per_element; // samples
+        constexpr int PER = AHEAD * CH / 4, FAR = PER < 4 ? PER : 4; // (of a lane: out of its registers, from memory)
         uint32_t key[PER], kmin = 0xffffffffu, kmax = 0u;
-        float sv[PER];
+        if (NPT > 0 || n <= 1024 * AHEAD * CH) { // block-uniform
+            // every fourth of the lane's elements, from one of the first four on in turn
+            auto sample = [&](auto first) {
 #pragma unroll
-        for (int q = 0; q < PER; ++q) sv[q] = load((int)(((int64_t)(tid + 1024 * q) * n) / ROW_SAMPLES));
+                for (int q = 0; q < PER; ++q) {
+                    const int j = 4 * q + first;
+                    key[q] = index(j) < n ? max(score_key(v[j / CH][j % CH]), 1u) : 0u; // (0: no element)
+                }
+            };
+            switch (__builtin_amdgcn_readfirstlane(tid >> 6) & 3) {
+            case 0: sample(std::integral_constant<int, 0>{}); break;
+            case 1: sample(std::integral_constant<int, 1>{}); break;
+            case 2: sample(std::integral_constant<int, 2>{}); break;
+            default: sample(std::integral_constant<int, 3>{}); break;
+            }
+            per_element = 0.25f;
+        } else {
+            float sv[FAR];
+#pragma unroll
+            for (int q = 0; q < FAR; ++q) sv[q] = load((int)(((int64_t)(tid + 1024 * q) * n) / (1024 * FAR)));
+#pragma unroll
+            for (int q = 0; q < PER; ++q) key[q] = q < FAR ? max(score_key(sv[q < FAR ? q : 0]), 1u) : 0u;
+            per_element = 1024.f * FAR / (float)n;
+        }
 #pragma unroll
         for (int q = 0; q < PER; ++q) {
-            key[q] = score_key(sv[q]);
-            kmin = min(kmin, key[q]);
+            kmin = min(kmin, key[q] - 1u);
             kmax = max(kmax, key[q]);
         }
         __syncthreads();
         block_key_range(kmin, kmax, lds.tmp);
-        const KeyGroups groups(kmin, kmax);
+        const KeyGroups<11> groups(kmin + 1u, kmax);
         if (groups.linear_ok) {
 #pragma unroll
-            for (int q = 0; q < PER; ++q) atomicAdd(&lds.hist[groups.of(key[q], 0)], 1u);
+            for (int q = 0; q < PER; ++q)
+                if (key[q] != 0u) atomicAdd(&lds.hist[groups.of(key[q], 0)], 1u);
             __syncthreads();
-            const float expect = (float)k * ((float)ROW_SAMPLES / (float)n);
+            const float expect = (float)k * per_element;
             const uint32_t target = (uint32_t)(expect + 4.f * __builtin_sqrtf(expect)) + 2u;
             const uint32_t h_lo = lds.hist[2 * tid], h_hi = lds.hist[2 * tid + 1]; // lane t owns bins 2t and 2t+1
             const uint32_t incl = block_suffix_sum<16>(h_lo + h_hi, lds.tmp);
@@ -1185,25 +1229,43 @@ __device__ __forceinline__ void select_row(RowLds& lds, int cap, int k, Load&& l
     uint32_t bottom = 0xffffffffu, top = 0u; // smallest and largest key that reached the pivot
     auto filter = [&](int j0, const float (&from)[CH]) { // elements j0 .. j0 + CH - 1 of the lane
         uint32_t key[CH], count = 0;
+        bool in[CH];
 #pragma unroll
-        for (int j = 0; j < CH; ++j) {
-            const uint32_t u = max(score_key(from[j]), 1u); // (0: no element; only NaNs have keys that low)
-            key[j] = index(j0 + j) < n && u >= pivot ? u : 0u;
-            top = max(top, key[j]);
-            bottom = min(bottom, key[j] - 1u);
-            count += key[j] != 0u ? 1u : 0u;
+        for (int j4 = 0; j4 < CH; j4 += 4) { // (block-uniform: past the row's end nothing, inside it without a look at the index)
+            const int begin = 1024 * (j0 + j4);
+#pragma unroll
+            for (int j = j4; j < j4 + 4; ++j) in[j] = false;
+            if (begin >= n) continue;
+#pragma unroll
+            for (int j = j4; j < j4 + 4; ++j) {
+                key[j] = score_key(from[j]);
+                in[j] = key[j] >= pivot;
+            }
+            if (begin + 4096 > n) {
+#pragma unroll
+                for (int j = j4; j < j4 + 4; ++j) in[j] = in[j] && index(j0 + j) < n;
+            }
+#pragma unroll
+            for (int j = j4; j < j4 + 4; ++j) count += in[j] ? 1u : 0u;
         }
         const uint32_t incl = wave_prefix_sum(count);
         const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
         if (total == 0u) return; // wave-uniform
         uint32_t at = 0;
         if (lane == 0) at = atomicAdd(&lds.out, total);
-        at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) + incl - count;
+        at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+        if (at + total > ROW_CAP) return; // (wave-uniform; the row is selected exactly)
+        at += incl - count;
 #pragma unroll
-        for (int j = 0; j < CH; ++j) {
-            if (key[j] != 0u && at < ROW_CAP) lds.buf[at] = make_cand(key[j], index(j0 + j));
-            at += key[j] != 0u ? 1u : 0u;
-        }
+        for (int j = 0; j < CH; ++j)
+            if (in[j]) {
+                lds.buf[at++] = make_cand(key[j], index(j0 + j));
+                top = max(top, key[j]);
+            }
+        if (pivot == 0u) // (else the pivot bounds them: block-uniform)
+#pragma unroll
+            for (int j = 0; j < CH; ++j)
+                if (in[j]) bottom = min(bottom, key[j]);
     };
     if constexpr (NPT > 0) {
         filter(0, v[0]);
@@ -1224,7 +1286,7 @@ __device__ __forceinline__ void select_row(RowLds& lds, int cap, int k, Load&& l
         atomicMax(&lds.tmp[15], top);
     }
     __syncthreads();
-    uint32_t m = lds.out, kmin = lds.tmp[14] + 1u, kmax = lds.tmp[15];
+    uint32_t m = lds.out, kmin = pivot == 0u ? lds.tmp[14] : pivot, kmax = lds.tmp[15];
     const bool exact = m < (uint32_t)k || m > ROW_CAP; // block-uniform
     if (exact) {
         row_select_exact(lds, n, k, load);
@@ -1249,7 +1311,7 @@ __device__ __forceinline__ void select_row(RowLds& lds, int cap, int k, Load&& l
             }
         block_key_range(kmin, kmax, lds.tmp);
     }
-    order_words<ROW_CAP / 1024>(w, m, kmin, kmax, lds.buf, lds.hist, lds.start, lds.tmp, &lds.cnt, k, write);
+    order_words<ROW_CAP / 1024>(w, m, kmin, kmax, lds.buf, lds.hist, lds.tmp, &lds.cnt, k, write);
 }
 
 // The indexer's selection as one kernel over the score rows, for rows of at most INDEXER_ROW_MAX keys: no histograms, no
@@ -1257,7 +1319,7 @@ __device__ __forceinline__ void select_row(RowLds& lds, int cap, int k, Load&& l
 template <int NPT>
 __global__ __launch_bounds__(1024) void indexer_row_topk_kernel(IndexerArgs a)
 {
-    __shared__ RowLds lds;
+    __shared__ __align__(16) RowLds lds;
     const int tid = threadIdx.x, row = blockIdx.x;
     const float* x = a.scores + (int64_t)row * a.score_stride;
     int32_t* out = a.topk_res + (int64_t)row * a.k;
@@ -1271,13 +1333,14 @@ __global__ __launch_bounds__(1024) void indexer_row_topk_kernel(IndexerArgs a)
                        [&](int rank, uint64_t w) { out[rank] = word_index(w); });
 }
 
-// 16 rows of 20000, k = 2048: 14.6 us (counting passes that read the row twice per 11 bits, and a bitonic sort of all selected
-// words: 53); 2 rows of 4440, k = 563: 7 us (the row sorted whole: 66).
+// With the gather that uses it, k = 2048: 16 rows of 20000 20.6 us, 2 rows of 65536 23.0, 4 rows of 200000 47.1 (the sample always
+// from memory, every index looked at, half the groups and each word compared by the lane that had read it: 23.5, 24.7, 53.8).
+// Counting passes over the row and a bitonic sort of the selected words took the selection from 15 to 53 us for the first.
 template <int NPT>
 __global__ __launch_bounds__(1024) void topk_select_kernel(const float* __restrict__ x, float* __restrict__ values,
                                                            int32_t* __restrict__ indices, int n, int k, int largest)
 {
-    __shared__ RowLds lds;
+    __shared__ __align__(16) RowLds lds;
     const float* row = x + (int64_t)blockIdx.x * n;
     auto load = [&](int i) { return largest ? row[i] : -row[i]; };
     int32_t* out_i = indices + (int64_t)blockIdx.x * k;

@@ -114,3 +114,22 @@ def test_row_lengths_at_the_kernels_edges(cuda, n):
     for k in (1, min(n, 2048)):
         check(x, k, None, True, cuda)
     check(x, min(n, 100), None, False, cuda)
+
+
+@pytest.mark.parametrize("n,k", [(4097, 2048), (4100, 1), (16383, 2048), (16384, 100), (16385, 2048), (32767, 1000), (32768, 2048),
+                                 (32769, 2048), (65537, 5)])
+def test_rows_around_the_sample_and_what_registers_hold(cuda, n, k):
+    """Rows just within and beyond what a lane's registers hold: the sample comes from them, or from memory.  Scores the sample sees
+    as they are (a bell), sorted by position, alternating with the lanes of a wavefront, tied, and with infinities and zeros of both
+    signs; selections bit for bit."""
+    g = torch.Generator().manual_seed(n)
+    bell = torch.randn((1, n), generator=g)
+    lanes = bell + 8 * ((torch.arange(n) % 4) == 1).float()        # all the best in one of every four elements
+    blocks = bell + 8 * ((torch.arange(n) // 64 % 4) == 2).float()  # all the best in one wavefront of every four
+    special = bell.clone()
+    special[0, ::7], special[0, 1::7] = 0.0, -0.0
+    special[0, 5], special[0, n - 1] = float("inf"), float("-inf")
+    tied = torch.randint(-40, 40, (1, n), generator=g).float()
+    x = torch.cat([bell, bell.sort(-1).values, lanes, blocks, special, tied])
+    for largest in (True, False):
+        check(x, k, -1, largest, cuda)
