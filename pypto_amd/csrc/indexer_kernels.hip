@@ -73,13 +73,13 @@ __device__ __forceinline__ _Float16 round_f32_product_to_f16(float a, float b)
 // w_scale = q_scale * weight rounded once to fp16: the fp16 product of two fp16 values, or - fp32 scales - the fp32
 // product of the scale and the widened weight
 template <bool F32>
-__device__ __forceinline__ _Float16 w_scale_of(const void* q_scale, const uint16_t* weights, int64_t h)
+__device__ __forceinline__ _Float16 w_scale_of(typename ScaleOf<F32>::raw q_scale, uint16_t weight)
 {
-    const _Float16 w = __builtin_bit_cast(_Float16, weights[h]);
+    const _Float16 w = __builtin_bit_cast(_Float16, weight);
     if constexpr (F32)
-        return round_f32_product_to_f16(static_cast<const float*>(q_scale)[h], (float)w);
+        return round_f32_product_to_f16(q_scale, (float)w);
     else
-        return (_Float16)(__builtin_bit_cast(_Float16, static_cast<const uint16_t*>(q_scale)[h]) * w);
+        return (_Float16)(__builtin_bit_cast(_Float16, q_scale) * w);
 }
 __device__ __forceinline__ uint32_t score_key(float f) { return f32_to_ordered(f + 0.0f); } // -0 -> +0
 // Bin of a score key in the selection histogram, non-decreasing in the key: quarter octaves (sign, exponent, two
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256) void indexer_score_kernel(IndexerArgs a)
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const int64_t h = (int64_t)(row0 + s) * a.nh + 32 * mm + 16 * (e >> 2) + 4 * g + (e & 3);
-                wa[s][mm][e] = l16 == 0 ? w_scale_of<F32>(a.q_scale, a.weights, h) : (_Float16)0.f; // one fp16 rounding
+                wa[s][mm][e] = l16 == 0 ? w_scale_of<F32>(static_cast<const typename ScaleOf<F32>::raw*>(a.q_scale)[h], a.weights[h]) : (_Float16)0.f; // one fp16 rounding
             }
     }
     __syncthreads(); // histogram zeroed
@@ -312,6 +312,7 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
     constexpr int SLOT = PPASSES < PASSES ? PPASSES : PASSES; // passes to a histogram slot
     __shared__ __align__(16) uint32_t hist[PPASSES / SLOT][S1][SBINS];
     __shared__ __align__(16) float s_sc[S1][CHUNK * PPASSES]; // the workgroup's scores, written out in one burst at the end
+    __shared__ __align__(16) _Float16 s_w[S1][64];
     __shared__ __align__(16) uint8_t s_keys[4][64 * D];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, g = lane >> 4;
@@ -370,6 +371,7 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
         int fseq = -1, fspan = 0;
 #pragma unroll
         for (int j = 0; j < SCAN_SEQS / 64; ++j) {
+            if (64 * j >= a.b) break;
             const int len = min(lens[j], a.max_ctx);
             const uint32_t cnt = (lane + 64 * j < a.b && len > 0) ? ((uint32_t)((len - 1) / CHUNK) >> passes_log2) + 1u : 0u;
             const uint32_t incl = wave_prefix_sum(cnt), excl = incl - cnt;
@@ -425,20 +427,28 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
     uint8_t* key_dst = keys + (lane >> 3) * D + (((lane & 7) ^ (lane >> 3)) << 4);
     const uint8_t* key_src0 = keys + l16 * D + ((g ^ (l16 & 7)) << 4);
     const uint8_t* key_src1 = keys + l16 * D + (((g + 4) ^ (l16 & 7)) << 4);
-    // The key loads go out first; the query and its scales follow them (memory operations complete in order, and the
-    // first MFMA needs all of them).  Every memory operation from here on is unconditional, so that the number in
-    // flight is the same on every path into the loop and the waits can count them.
+    // The query and its scales go through LDS too, whole rows to an instruction and once to a workgroup.  (Taken by every wavefront
+    // in operand layout, neighbouring lanes in different rows, the 8 S1 loads of the query alone kept the load path busy for most of the
+    // 4.5 us before the first product: now 3.0 with two query tokens.  13 sequences of 1000 .. 40000 keys, two query tokens, through
+    // selection and attention 63.9 -> 59.9 us; 64 of them 153 -> 146.7; one sequence of 4096, a layer 62.1 -> 60.4.)
+    // They are requested first, then the keys and their scales (memory operations complete in order).  Every memory operation from
+    // here on is unconditional, so that the number in flight is the same on every path into the loop and the waits can count them.
+    i32x4 qraw[2 * S1];
+#pragma unroll
+    for (int i = 0; i < 2 * S1; ++i)
+        qraw[i] = *reinterpret_cast<const i32x4*>(a.q + ((int64_t)row0 * a.nh + (wave * 2 * S1 + i) * 8) * D + 16 * lane);
+    // one head's w_scale to a lane, of query token wave % S1
+    const int64_t w_at = (int64_t)(row0 + wave % S1) * a.nh + lane;
+    const uint16_t w_raw = a.weights[w_at];
+    const typename ScaleOf<F32>::raw qs_raw = static_cast<const typename ScaleOf<F32>::raw*>(a.q_scale)[w_at];
     load_half(0);
-    // int8 A fragments: head hb*16 + l16, bytes 64*ks + 16*g .. +15
-    i32x4 qf[S1][4][2];
+    for (int i = tid; i < PPASSES / SLOT * S1 * SBINS; i += 256) (&hist[0][0][0])[i] = 0;
+    // (row r of s_keys: head r % 64 of query token r / 64; the chunks XOR-ed as the keys')
 #pragma unroll
-    for (int s = 0; s < S1; ++s)
-#pragma unroll
-        for (int hb = 0; hb < 4; ++hb) {
-            const int8_t* qp = a.q + ((int64_t)(row0 + s) * a.nh + hb * 16 + l16) * D + 16 * g;
-            qf[s][hb][0] = *reinterpret_cast<const i32x4*>(qp);
-            qf[s][hb][1] = *reinterpret_cast<const i32x4*>(qp + 64);
-        }
+    for (int i = 0; i < 2 * S1; ++i)
+        *reinterpret_cast<i32x4*>(&s_keys[0][0] + (wave * 2 * S1 + i) * 8 * D + (lane >> 3) * D + (((lane & 7) ^ (lane >> 3)) << 4)) = qraw[i];
+    s_w[wave % S1][lane] = w_scale_of<F32>(qs_raw, w_raw);
+    __syncthreads();
     // fp16 A fragments of the head sum, the same in every row: k-slot (g, e) of MFMA mm is head
     // 32*mm + 16*(e/4) + 4*g + e%4 - the head whose int32 result this lane group holds in that slot; the value is
     // q_scale * weights in one fp16 rounding
@@ -448,23 +458,19 @@ __global__ __launch_bounds__(256, S1 == 1 ? 3 : 2) void indexer_score_paged_kern
 #pragma unroll
         for (int mm = 0; mm < 2; ++mm) {
             typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-            const int64_t h = (int64_t)(row0 + s) * a.nh + 32 * mm + 4 * g;
-            const f16x4 wlo = *reinterpret_cast<const f16x4*>(a.weights + h), whi = *reinterpret_cast<const f16x4*>(a.weights + h + 16);
-            if constexpr (F32) {
-                const f32x4 qlo = *reinterpret_cast<const f32x4*>(static_cast<const float*>(a.q_scale) + h);
-                const f32x4 qhi = *reinterpret_cast<const f32x4*>(static_cast<const float*>(a.q_scale) + h + 16);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    wa[s][mm][e] = round_f32_product_to_f16(qlo[e], (float)wlo[e]);
-                    wa[s][mm][4 + e] = round_f32_product_to_f16(qhi[e], (float)whi[e]);
-                }
-            } else {
-                const uint16_t* qs = static_cast<const uint16_t*>(a.q_scale);
-                const f16x4 qlo = *reinterpret_cast<const f16x4*>(qs + h), qhi = *reinterpret_cast<const f16x4*>(qs + h + 16);
-                wa[s][mm] = __builtin_shufflevector(qlo * wlo, qhi * whi, 0, 1, 2, 3, 4, 5, 6, 7);
-            }
+            const _Float16* wp = &s_w[s][32 * mm + 4 * g];
+            wa[s][mm] = __builtin_shufflevector(*reinterpret_cast<const f16x4*>(wp), *reinterpret_cast<const f16x4*>(wp + 16), 0, 1, 2, 3, 4, 5, 6, 7);
         }
-    for (int i = tid; i < PPASSES / SLOT * S1 * SBINS; i += 256) (&hist[0][0][0])[i] = 0;
+    // int8 A fragments: head hb*16 + l16, bytes 64*ks + 16*g .. +15
+    i32x4 qf[S1][4][2];
+#pragma unroll
+    for (int s = 0; s < S1; ++s)
+#pragma unroll
+        for (int hb = 0; hb < 4; ++hb) {
+            const uint8_t* qp = &s_keys[0][0] + (s * 64 + hb * 16 + l16) * D;
+            qf[s][hb][0] = *reinterpret_cast<const i32x4*>(qp + ((g ^ (l16 & 7)) << 4));
+            qf[s][hb][1] = *reinterpret_cast<const i32x4*>(qp + (((g + 4) ^ (l16 & 7)) << 4));
+        }
     __syncthreads();
 
     auto compute_half = [&](int hh, typename ScaleOf<F32>::raw ksc) {
