@@ -218,10 +218,11 @@ __device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t*
     mfma(1, [](int) {});
 }
 
-// Up to 32 tokens x 128 outputs, 256 lanes: a stream of weights, five stages of 128 rows in flight straight to LDS.  Wave w owns
-// outputs [32 w, +32).  Register e of acc[nb][tb]: output 32 w + 16 nb + 4 g + e, token 16 tb + l16.
+// Up to 32 tokens x 128 outputs, 256 lanes: a stream of weights, three stages of 128 rows in flight straight to LDS (with five, or
+// two, the fused prolog of 8 tokens takes 0.4 us longer: 28.4 us, weights out of HBM 32.8).  Wave w owns outputs [32 w, +32).
+// Register e of acc[nb][tb]: output 32 w + 16 nb + 4 g + e, token 16 tb + l16.
 struct GtStream {
-    static constexpr int TOK = 32, QBYTES = TOK * 128, STAGE = QBYTES + 128 * 128, RING = 6, LDS = RING * STAGE;
+    static constexpr int TOK = 32, QBYTES = TOK * 128, STAGE = QBYTES + 128 * 128, RING = 4, LDS = RING * STAGE;
 };
 __device__ __forceinline__ void gt_stream_i8(i32x4 (&acc)[2][2], const int8_t* w, int64_t ldw, const int8_t* q, int64_t ldq, int t,
                                              int stages, uint8_t* lds)
@@ -268,12 +269,13 @@ __device__ __forceinline__ void gt_stream_i8(i32x4 (&acc)[2][2], const int8_t* w
         });
 }
 
-// 33 to 160 tokens x 128 outputs, 512 lanes: a stream of weights still, all tokens beside them, three or more stages in flight.  Wave (wr, wc) owns tokens [16 TT wr,
-// +16 TT) x two blocks of 16 outputs 32 apart, gt_batch_block(wc, nb): what a rotary embedding pairs is in one lane.  Register e of
-// acc[nb][tb]: output 16 gt_batch_block + 4 g + e, token 16 TT wr + 16 tb + l16.
+// 33 to 160 tokens x 128 outputs, 512 lanes: a stream of weights still, all tokens beside them, two stages in flight (fused prolog of 40
+// tokens, weights out of HBM, 38.1 us; with three 38.6, with five 39.2).  Wave (wr, wc) owns tokens [16 TT wr, +16 TT) x two blocks of
+// 16 outputs 32 apart, gt_batch_block(wc, nb): what a rotary embedding pairs is in one lane.  Register e of acc[nb][tb]: output
+// 16 gt_batch_block + 4 g + e, token 16 TT wr + 16 tb + l16.
 template <int TT>
 struct GtBatch {
-    static constexpr int TOK = 32 * TT, QBYTES = TOK * 128, STAGE = QBYTES + 128 * 128, FIT = 160 * 1024 / STAGE, RING = FIT < 6 ? FIT : 6, LDS = RING * STAGE;
+    static constexpr int TOK = 32 * TT, QBYTES = TOK * 128, STAGE = QBYTES + 128 * 128, FIT = 160 * 1024 / STAGE, RING = FIT < 3 ? FIT : 3, LDS = RING * STAGE;
 };
 __device__ __forceinline__ int gt_batch_block(int wc, int nb) { return (wc & 1) + 2 * nb + 4 * (wc >> 1); }
 template <int TT>

@@ -17,7 +17,7 @@
 // by that read.  All four weight matrices are stored with the output dimension contiguous, the opposite of what the
 // MFMA operands want (contraction contiguous per lane), so every weight tile goes through LDS and is read back
 // transposed: bf16 tiles with ds_read_b64_tr_b16, the int8 tile with ds_read_b64_tr_b8.
-//   mla_xa_kernel    x @ [w_dq | w_dkv_kr], 256 contraction rows x 128 outputs per workgroup, fp32 partials
+//   mla_xa_kernel    x @ [w_dq | w_dkv_kr], 1024 contraction rows x 64 outputs per workgroup, fp32 partials
 //   mla_norm_kernel  two workgroups per token: fixed-order sum of the partials, an RmsNorm each, the quantisations, the
 //                    key's rotary embedding, the three cache writes, q_norm / q_norm_scale
 //   mla_qb_kernel    int8 MFMA GEMM q_norm @ w_uq_qr, 128 outputs x 32 tokens per workgroup, weights streamed to LDS
@@ -41,101 +41,13 @@ namespace {
 constexpr int MTOK = 32;          // tokens per workgroup tile
 constexpr int MNOPE = 128, MROPE = 64, MQH = MNOPE + MROPE, MC = 512, MKV = MC + MROPE;
 constexpr int MAX_R = 2048;       // largest q_lora_rank (LDS of mla_norm_kernel)
-constexpr int XA_K = 256;         // contraction rows per stage of mla_xa_kernel
+constexpr int XA_K = 256;         // the hidden size is a multiple
 constexpr int XA_SPLIT = 1024;    // contraction rows per workgroup of mla_xa_kernel (one fp32 partial sum each)
-constexpr int XROW2 = 64 * 2 + 16; // bytes per LDS row of a [k][64] bf16 weight tile (padded against bank conflicts)
 constexpr int TROW = 128 * 2 + 32; // bytes per LDS row of a [k][128] bf16 weight tile (padded against bank conflicts)
-constexpr int BIG_T = 33;         // token count from which the kernels that hold more than 32 tokens take over: the others read the
-                                  // weights once per 32 tokens (fused prolog, 32 tokens 32.0 us and 33: 33.0; with the weights read
+constexpr int BIG_T = 33;         // token count from which the query kernels that hold more than 32 tokens take over: the others read the
+                                  // weights once per 32 tokens (fused prolog, 32 tokens 30.5 us and 40: 31.2; with the weights read
                                   // twice 63.6)
 constexpr int BIG_T2 = 256;       // token count above which the x product's tiles are 256 outputs wide, in splits of its own
-
-// 32 outputs x 32 tokens += W[KSTEPS steps of 16 rows, outputs]^T . X[tokens, k]: A by transposing reads of the [k][n]
-// tile in LDS, rows of ROWB bytes.  Lane jj of a 16-lane group points at row 8 hl + jj / 4 (+ 4 for the second read) of
-// the step, columns 16 mh + 4 (jj & 3); a read hands lane i the column 16 mh + i over the four rows its group's lanes
-// i / 4, i / 4 + 4, ... point at, so lane half hl ends up with the contraction rows 8 hl .. 8 hl + 7 of the step - and B
-// takes the same rows of X with ONE 16-byte load per step (x[token][16 ks + 8 hl ..]: 32 bytes contiguous per token row
-// and instruction; narrower pieces cost the texture addresser twice the cycles, and it is what bounds these loads:
-// every lane pair reads a different row).  Register e of the result: output 8 (e / 4) + 4 hl + e % 4, token lane % 32.
-// The B operand is loaded by its own call so that a caller can put these loads ahead of a prefetch in program order:
-// memory operations complete in order, and a wait for loads issued after a prefetch would wait for the prefetch too.
-template <int KSTEPS>
-__device__ __forceinline__ void load_b_rows(u32x4 (&b)[KSTEPS], const uint16_t* xrow, int lane)
-{
-    const uint16_t* xp = xrow + (lane >> 5) * 8;
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) b[ks] = *reinterpret_cast<const u32x4*>(xp + ks * 16);
-}
-template <int KSTEPS, int ROWB>
-__device__ __forceinline__ void gemm_tr_tile(f32x16& acc, const uint8_t* wtile, int ncol0, const u32x4 (&b)[KSTEPS], int lane)
-{
-    const int jj = lane & 15, mh = (lane >> 4) & 1, hl = lane >> 5;
-    const uint8_t* hp = wtile + (8 * hl + (jj >> 2)) * ROWB + (ncol0 + 16 * mh + 4 * (jj & 3)) * 2;
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-        const s16x4 lo = lds_read_tr(hp + ks * 16 * ROWB);
-        const s16x4 hi = lds_read_tr(hp + (ks * 16 + 4) * ROWB);
-        const bf16x8 av = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, __builtin_bit_cast(bf16x8, b[ks]), acc, 0, 0, 0);
-    }
-}
-
-// ------------------------------------------------------------------------------------------------ x @ [w_dq | w_dkv_kr]
-// grid (ceil(h / 1024), output tiles of 64, token tiles of 32), 1024 lanes = 4 groups of 4 wavefronts.  Group g takes rows
-// [256 g, 256 g + 256) of the workgroup's 1024 contraction rows: 256 rows x 64 outputs of weights, loaded in one go (every
-// load of the workgroup is in flight at once - at decode sizes the kernel is a single pass over the weights and its
-// duration is one memory latency plus the transfer), transposed through the group's LDS buffer.  Within a group wave w
-// owns the 32 outputs of block w & 1 over rows [128 (w >> 1), + 128).  The eight partial sums of an output are added
-// through LDS in a fixed order; fp32 partial sums per 1024-row split go to the workspace.
-// x [t, ldx] (bf16) times the 64 output columns at src (row stride ld), contraction rows [split * 1024, ..) of kdim;
-// the workgroup's fp32 partial sums go to part_out[(split * t + token) * ncols + col0 + ..]
-__device__ __forceinline__ void xa_body(const uint16_t* x, int ldx, int kdim, const uint16_t* src, int ld, float* part_out,
-                                        int ncols, int col0, int split, int tok0, int t, uint8_t* xa_lds)
-{
-    const int tid = threadIdx.x & 255, grp = threadIdx.x >> 8, lane = tid & 63, wave = tid >> 6;
-    const int l32 = lane & 31, hl = lane >> 5;
-    const int stages = min(XA_SPLIT, kdim - split * XA_SPLIT) / XA_K; // 256-row stages of this split (4 but for the last)
-    const int sg = min(grp, stages - 1);                              // idle groups re-read the last stage and drop it
-    const int64_t kbase = (int64_t)split * XA_SPLIT + sg * XA_K;
-    uint8_t* wl = xa_lds + grp * (XA_K * XROW2);
-    const int nb = wave & 1, kh = wave >> 1;
-    // the B operand first, then the weights (memory operations complete in order)
-    u32x4 bx[8];
-    load_b_rows<8>(bx, x + (int64_t)min(tok0 + l32, t - 1) * ldx + kbase + 128 * kh, lane);
-    // 256 rows x 128 bytes = 8 pieces of 16 bytes per lane (rows tid/8 + 32 i, piece tid%8)
-    const int srow = tid >> 3, spc = tid & 7;
-    const uint16_t* sp = src + (kbase + srow) * ld + 8 * spc;
-    u32x4 stg[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) stg[i] = *reinterpret_cast<const u32x4*>(sp + (int64_t)(32 * i) * ld);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4*>(wl + (srow + 32 * i) * XROW2 + 16 * spc) = stg[i];
-    __syncthreads();
-    f32x16 acc;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-    gemm_tr_tile<8, XROW2>(acc, wl + 128 * kh * XROW2, 32 * nb, bx, lane);
-    __syncthreads();
-    // partial sums of (group, row half) -> LDS; the two collecting waves add them in the order of the rows
-    float* red = reinterpret_cast<float*>(xa_lds);
-    const int part = 2 * grp + kh;
-    if (part > 0 && grp < stages) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) red[((part * 2 + nb) * 16 + e) * 64 + lane] = acc[e];
-    }
-    __syncthreads();
-    if (part > 0) return;
-    for (int pp = 1; pp < 2 * stages; ++pp)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[e] += red[((pp * 2 + nb) * 16 + e) * 64 + lane];
-    const int gt = tok0 + l32;
-    if (gt < t) {
-        float* out = part_out + ((int64_t)split * t + gt) * ncols + col0 + 32 * nb + 4 * hl;
-#pragma unroll
-        for (int e4 = 0; e4 < 4; ++e4)
-            *reinterpret_cast<f32x4*>(out + 8 * e4) = f32x4{acc[4 * e4], acc[4 * e4 + 1], acc[4 * e4 + 2], acc[4 * e4 + 3]};
-    }
-}
 
 // Output tile `tile` (64 columns) of x @ [w_dq | w_dkv_kr | w_k | w_proj]: its weight columns and their row stride.
 __device__ __forceinline__ const uint16_t* xa_source(const MlaPrologArgs& a, int tile, int& ld)
@@ -157,29 +69,25 @@ __device__ __forceinline__ const uint16_t* xa_source(const MlaPrologArgs& a, int
     return a.w_proj + (tile - qtiles - MKV / 64 - PD / 64) * 64;
 }
 
-__global__ __launch_bounds__(1024) void mla_xa_kernel(MlaPrologArgs a)
-{
-    extern __shared__ __align__(16) uint8_t xa_lds[]; // [4 groups][256 k][64 n] bf16, rows of XROW2 bytes
-    int ld;
-    const uint16_t* src = xa_source(a, blockIdx.y, ld);
-    xa_body(a.x, a.h, a.h, src, ld, a.xa_part, a.ncols, blockIdx.y * 64, blockIdx.x, blockIdx.z * MTOK, a.t, xa_lds);
-}
-
-// The same product at 33 to 256 tokens: a workgroup owns all tokens x 64 columns over one 1024-row split of the contraction and
-// streams it in stages of 64 rows straight to LDS (gemm_tile.h), so that the weights are read once.  x is the A operand here, so a
-// result register holds one token's value for 32 consecutive columns across the lanes and the partial sums leave as 128-byte runs.
-// The sums are chains of 128 rows added up in order, which are mla_xa_kernel's bit for bit (a decode step's selection can hang on
-// the last bit of a score, so batches that cross the kernels' border see the same numbers).
+// ------------------------------------------------------------------------------------------------ x @ [w_dq | w_dkv_kr]
+// Up to 256 tokens a workgroup owns all tokens x 64 columns over one 1024-row split of the contraction and streams it in stages of
+// 64 rows straight to LDS (gemm_tile.h), so that the weights are read once.  x is the A operand here, so a result register holds one
+// token's value for 32 consecutive columns across the lanes and the partial sums leave as 128-byte runs.  The sums are chains of 128
+// rows added up in order, whatever the number of tokens (a decode step's selection can hang on the last bit of a score, so batches of
+// different sizes see the same numbers).
 // What bounds it: the weights' stream (34 MB, 6.5 us), and from some 100 tokens on what 252 workgroups draw of x from the L2 (2 KB a
-// token and split each, 10 TB/s).  Tiles of 128 tokens through registers, four stages of loads in flight and two barriers a stage,
-// took 13.3 us at 40 tokens and 20.9 at 160 (two tiles); so 10.4 and 16.0.  Call of the fused prolog, with mla_qb_batch_kernel's
-// change: 33 tokens 40.1 -> 33.0 us, 64: 42.7 -> 34.6, 96: 45.5 -> 40.3, 128: 47.0 -> 45.2, 160: 58.3 -> 53.1, 256: 66.9 -> 64.7.
+// token and split each, 10 TB/s).
+// To 32 tokens 1024 lanes with the whole split in registers, the token rows in operand layout (a different row with every lane: a
+// cycle of the texture addresser each, 8192 to a workgroup): a call of the bf16 form of 24 tokens 34.6 us, 32.6 this way, the fused
+// operator of 8 and 32 tokens 30.5 -> 29.3 and 32.4 -> 30.7.  Above, tiles of 128 tokens through registers took 13.3 us at 40 tokens
+// and 20.9 at 160 (two tiles); so 10.4 and 16.0.
+// Three stages ahead: with seven 33.4 at 24 tokens, with eleven 34.3 (fused, 96 tokens: 40.3 with seven, 39.0 with three; two ahead are as good).
 // grid (splits, output tiles of 64), 512 lanes: up to four blocks of 32 tokens wave w owns block w / 2 x 32 columns, above block w x 64.
 constexpr int XB_KS = 64; // contraction rows per stage
 template <int TT>
-__global__ __launch_bounds__(512, 2) void mla_xa_batch_kernel(MlaPrologArgs a)
+__global__ __launch_bounds__(512, 2) void mla_xa_kernel(MlaPrologArgs a)
 {
-    constexpr int XBYTES = TT * 32 * 128, STAGE = XBYTES + XB_KS * 128, FIT = 160 * 1024 / STAGE, RING = FIT < 8 ? FIT : 8;
+    constexpr int XBYTES = TT * 32 * 128, STAGE = XBYTES + XB_KS * 128, FIT = 160 * 1024 / STAGE, RING = FIT < 4 ? FIT : 4;
     constexpr int NB = TT <= 4 ? 1 : 2, XC = (TT + 1) / 2;
     static_assert(XA_K % (2 * XB_KS) == 0, "whole chains of 128 rows in every split");
     __shared__ __align__(16) uint8_t lds[RING * STAGE];
@@ -356,14 +264,14 @@ __device__ __forceinline__ void qb_store_blocks(const MlaPrologArgs& a, const ui
 }
 
 // bf16 form of the operator, up to 32 tokens: q_b = q_norm (bf16 [t, r]) @ w_uq_qr (bf16 [r, n * 192]), a stream of 75 MB of
-// weights.  A workgroup owns 128 outputs (192 of them at model sizes) and keeps six stages of 64 rows x 256 bytes in flight
-// straight to LDS.  Splits of 1024 rows loaded in one go through registers, their fp32 partial sums through memory and a kernel
+// weights.  A workgroup owns 128 outputs (192 of them at model sizes) and keeps three stages of 64 rows x 256 bytes in flight
+// straight to LDS (call of 24 tokens 30.8 us, with six 31.3; out of HBM 35.9 and 36.3).  Splits of 1024 rows loaded in one go through registers, their fp32 partial sums through memory and a kernel
 // behind them took 24.4 + 4.8 us at 24 tokens.  The sums: chains of 128 rows added up in order, then splits of 1024 rows.
 // grid (n * 192 / 128 rounded up), 256 lanes: wave w owns outputs [32 w, +32).
 __global__ __launch_bounds__(256) void mla_qb16_kernel(MlaPrologArgs a)
 {
 #pragma clang fp contract(off)
-    constexpr int XB = MTOK * 128, STAGE = XB + 2 * 64 * 128, RING = 7; // a stage: token rows | [2] weight rows of 128 bytes
+    constexpr int XB = MTOK * 128, STAGE = XB + 2 * 64 * 128, RING = 4; // a stage: token rows | [2] weight rows of 128 bytes
     static_assert(2 * MTOK * QBS_ROW <= RING * STAGE, "the output tile takes the stages' place");
     __shared__ __align__(16) uint8_t lds[RING * STAGE];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -924,7 +832,9 @@ __global__ __launch_bounds__(256) void mla_wuk_kernel(MlaPrologArgs a)
     for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[tb][e] = 0.f;
-    // (the weight fragment by transposing reads: see gemm_tr_tile)
+    // The weight fragment by transposing reads.  Lane jj of a 16-lane group points at row 8 hl + jj / 4 (+ 4 for the second read) of the
+    // step, columns 16 mh + 4 (jj & 3); a read hands lane i the column 16 mh + i over the four rows its group's lanes i / 4, i / 4 + 4,
+    // .. point at, so lane half hl ends up with the contraction rows 8 hl .. 8 hl + 7 - and B takes the same rows with one 16-byte read.
 #pragma unroll
     for (int ks = 0; ks < MNOPE / 16; ++ks) {
         const s16x4 lo = lds_read_tr(hp + ks * 16 * TROW);
@@ -1002,7 +912,7 @@ __global__ __launch_bounds__(512, 2) void mla_wuk_wide_kernel(MlaPrologArgs a)
 #pragma unroll
         for (int i = 0; i < MNOPE / 8; ++i) *reinterpret_cast<u32x4*>(wl + (8 * i + r) * OROW + 16 * c) = x[i];
         __builtin_amdgcn_wave_barrier();
-        // (the weight fragment by transposing reads: see gemm_tr_tile)
+        // (the weight fragment by transposing reads: see mla_wuk_kernel)
         const int jj = lane & 15, mh = (lane >> 4) & 1;
         const uint8_t* hp = wl + (8 * hl + (jj >> 2)) * OROW + (16 * mh + 4 * (jj & 3)) * 2;
 #pragma unroll
@@ -1107,20 +1017,12 @@ void fused_prolog_bind(MlaPrologArgs& m, PrologArgs& p, void* ws)
     p.ksplits = m.ksplits;
 }
 
-static hipError_t set_lds_limits()
-{
-    static DeviceOnce once;
-    return once.run([] {
-        return hipFuncSetAttribute(reinterpret_cast<const void*>(mla_xa_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   4 * XA_K * XROW2);
-    });
-}
-
-// f(integral constant: blocks of 32 tokens) for 33 to 256 tokens
+// f(integral constant: blocks of 32 tokens) for up to 256 tokens
 template <class F>
 static void token_blocks(int t, F&& f)
 {
     switch ((t + 31) / 32) {
+    case 1: f(std::integral_constant<int, 1>{}); break;
     case 3: f(std::integral_constant<int, 3>{}); break;
     case 4: f(std::integral_constant<int, 4>{}); break;
     case 5: f(std::integral_constant<int, 5>{}); break;
@@ -1150,25 +1052,21 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
 {
     if (a.t == 0) return hipSuccess;
     const int ttiles = (a.t + MTOK - 1) / MTOK;
-    hipError_t e = set_lds_limits();
-    if (e != hipSuccess) return e;
+    hipError_t e;
     const bool big = a.t >= BIG_T; // the kernels that own an output tile
     {
         ScopedKernelTimer tm(KID_MLA_XA, stream);
-        if (big)
-            if (a.t <= BIG_T2)
-                token_blocks(a.t, [&](auto tt) {
-                    constexpr int TT = decltype(tt)::value;
-                    hipLaunchKernelGGL(mla_xa_batch_kernel<TT>, dim3(a.ksplits, a.ncols / 64), dim3(512), 0, stream, a);
-                });
-            else {
-                const int xtiles = (a.t + 127) / 128, ntiles = (a.ncols + 255) / 256, rows = xa_wide_rows(a.t, a.h, a.r);
-                if (a.ksplits != (a.h + rows - 1) / rows) return hipErrorInvalidValue;
-                hipLaunchKernelGGL(mla_xa_wide_kernel, dim3((xtiles * ntiles * a.ksplits + 7) / 8 * 8), dim3(GT_LANES), 0, stream, a, xtiles,
-                                   ntiles, rows);
-            }
-        else
-            hipLaunchKernelGGL(mla_xa_kernel, dim3(a.ksplits, a.ncols / 64, ttiles), dim3(1024), 4 * XA_K * XROW2, stream, a);
+        if (a.t <= BIG_T2) {
+            token_blocks(a.t, [&](auto tt) {
+                constexpr int TT = decltype(tt)::value;
+                hipLaunchKernelGGL(mla_xa_kernel<TT>, dim3(a.ksplits, a.ncols / 64), dim3(512), 0, stream, a);
+            });
+        } else {
+            const int xtiles = (a.t + 127) / 128, ntiles = (a.ncols + 255) / 256, rows = xa_wide_rows(a.t, a.h, a.r);
+            if (a.ksplits != (a.h + rows - 1) / rows) return hipErrorInvalidValue;
+            hipLaunchKernelGGL(mla_xa_wide_kernel, dim3((xtiles * ntiles * a.ksplits + 7) / 8 * 8), dim3(GT_LANES), 0, stream, a, xtiles,
+                               ntiles, rows);
+        }
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
     {
@@ -1210,7 +1108,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         } else if (big) {
             if (qb_batch(a, p)) {
                 token_blocks(a.t, [&](auto tt) {
-                    constexpr int TT = decltype(tt)::value < QB_BATCH_T / 32 ? decltype(tt)::value : QB_BATCH_T / 32;
+                    constexpr int TT = std::clamp(decltype(tt)::value, 2, QB_BATCH_T / 32);
                     if (p)
                         hipLaunchKernelGGL(fused_qb_batch_kernel<TT>, dim3(a.n * MQH / 128 + p->n), dim3(GT_LANES), 0, stream, a, *p);
                     else
