@@ -773,8 +773,8 @@ __global__ __launch_bounds__(GT_LANES, 2) void fused_qb_batch_kernel(MlaPrologAr
 
 // For more tokens than that (qb_batch) the two products in one launch of gemm_tile.h's tiles: the index heads' part alone is half a round of workgroups
 // up to 512 tokens (call of 257 tokens 83.0 us as two launches, 72.2 as one, 512: 104.4 / 96.3, 1024: 163.6 / 160.7, 1344: 211.5 /
-// 194.6, 4096: 604.7 / 591.0).  Its tiles are up to 224 tokens; where the query product's own of 256 save a round the two are the
-// same (900 tokens 153.9 / 154.0, 2048: 314.5 / 316.6).
+// 194.6, 4096: 604.7 / 591.0).  Tiles of 128 to 256 tokens, by modelled time (with 224 at most: 512 tokens 94.5 us a call, 1024: 159.8,
+// 1501: 215.7; so 91.9, 153.6, 207.0).
 // The index heads' tiles take the longer, 26 us at 192 tokens against 19, and come first, those of all tokens: as columns of each
 // token tile they began again in the last round of workgroups (104 us for the kernel at 1501 tokens,
 // 92 so; the call 240.8 -> 236.8, no difference where the rounds come out even).
@@ -1117,8 +1117,8 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
             } else {
                 const int cols = (a.n * MQH + 255) / 256, qcols = p ? (p->n + 1) / 2 : 0, stages = a.r / GT_KI8;
                 if (p)
-                    gt_dispatch(gt_token_blocks(a.t, cols + qcols, stages, 7), [&](auto tb) {
-                        constexpr int TB = decltype(tb)::value < 7 ? decltype(tb)::value : 7;
+                    gt_dispatch(gt_token_blocks(a.t, cols + qcols, stages, 8), [&](auto tb) {
+                        constexpr int TB = decltype(tb)::value;
                         hipLaunchKernelGGL(fused_qb_wide_kernel<TB>, dim3((qcols + cols) * ((a.t + 32 * TB - 1) / (32 * TB))), dim3(GT_LANES), 0, stream,
                                            a, *p);
                     });

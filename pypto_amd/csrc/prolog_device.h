@@ -446,9 +446,12 @@ __device__ __forceinline__ void transpose_rows(uint32_t (&out)[4][2], const u32x
 // stores of 4 bytes a lane.  Now 22 K: pairs are rotated where they are, in registers of a lane, by one wave of each SIMD
 // (gt_wave_across), cos and sin loaded 16 bytes at a time (loads of 8 cost the memory pipe twice as much, 13 K ticks in all, not 8);
 // rows two banks apart; one store of 16 bytes.  Call of 1501 tokens 239.6 -> 232.9 us, 300: 80.7 -> 76.5.
+// 256 tokens' tiles of both heads do not fit LDS: there the two halves of the tokens, which are two rows of waves, go through one
+// after the other (three rounds of workgroups for 1501 tokens instead of four of 192: a call 215.7 -> 207.0 us).
+constexpr int prolog_q_wide_parts(int tb) { return tb > 7 ? 2 : 1; }
 constexpr int prolog_q_wide_lds(int tb) // the product's stages, or hadamard_q | [2] bf16 tiles | [2] per-wave maxima
 {
-    const int tok = 32 * tb, ring = gt_lds_bytes(tb);
+    const int tok = 32 * tb / prolog_q_wide_parts(tb), ring = gt_lds_bytes(tb);
     const int epi = PD * PD * 2 + 2 * tok * XROW + 2 * 4 * tok * 4;
     return epi > ring ? epi : ring;
 }
@@ -456,7 +459,8 @@ template <int TB>
 __device__ __forceinline__ void prolog_q_wide_body(const PrologArgs& a, int head0, int tok0, uint8_t* lds)
 {
 #pragma clang fp contract(off)
-    constexpr int TOK = 32 * TB;
+    constexpr int PARTS = prolog_q_wide_parts(TB), TILE = 32 * TB / PARTS;
+    static_assert(PARTS == 1 || TILE == 16 * TB, "a part is a row of waves");
     static_assert(prolog_q_wide_lds(TB) <= 160 * 1024 && prolog_q_wide_lds(TB) >= GtTile<TB>::LDS, "LDS");
     const int tid = threadIdx.x, lane = tid & 63, wave = gt_wave_across();
     const int l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
@@ -527,19 +531,25 @@ __device__ __forceinline__ void prolog_q_wide_body(const PrologArgs& a, int head
                 }
         }
     }
-#pragma unroll
-    for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb)
-            *reinterpret_cast<u32x2*>(lds + PD * PD * 2 + ((wc >> 1) * TOK + 16 * TB * wr + 16 * tb + l16) * XROW + (hw + 16 * nb + 4 * g) * 2) =
-                u32x2{y[nb][tb][0], y[nb][tb][1]};
+    const int hs = tid >> 8, ht = tid & 255, head = head0 + hs; // behind the tile four waves to a head
+    uint8_t* xt = lds + PD * PD * 2 + hs * TILE * XROW;
+    float(*smax)[TILE] = reinterpret_cast<float(*)[TILE]>(lds + PD * PD * 2 + 2 * TILE * XROW + hs * 4 * TILE * 4);
 #pragma unroll
     for (int i = 0; i < PD * PD * 2 / 16 / 512; ++i) reinterpret_cast<u32x4*>(lds)[tid + 512 * i] = hadr[i];
-    __syncthreads();
-    const int hs = tid >> 8, ht = tid & 255, head = head0 + hs; // from here on four waves to a head
-    uint8_t* xt = lds + PD * PD * 2 + hs * TOK * XROW;
-    float(*smax)[TOK] = reinterpret_cast<float(*)[TOK]>(lds + PD * PD * 2 + 2 * TOK * XROW + hs * 4 * TOK * 4);
-    prolog_q_quantise<TB>(a, head, tok0, ht, lds, xt, smax);
+#pragma unroll
+    for (int part = 0; part < PARTS; ++part) {
+        if (part > 0) __syncthreads(); // the tile and the maxima before are read
+        if (PARTS == 1 || wr == part) {
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+                for (int nb = 0; nb < 4; ++nb)
+                    *reinterpret_cast<u32x2*>(lds + PD * PD * 2 + ((wc >> 1) * TILE + 16 * TB * wr - part * TILE + 16 * tb + l16) * XROW +
+                                              (hw + 16 * nb + 4 * g) * 2) = u32x2{y[nb][tb][0], y[nb][tb][1]};
+        }
+        __syncthreads();
+        prolog_q_quantise<TB / PARTS>(a, head, tok0 + part * TILE, ht, lds, xt, smax);
+    }
 }
 
 // Up to 32 tokens: one head per workgroup of 256 lanes behind the streamed product; the bits of prolog_q_body.

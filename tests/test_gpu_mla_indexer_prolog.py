@@ -193,6 +193,16 @@ def test_index_head_tiles_ahead_of_the_query_tiles(cuda, t, n):
     check_against_oracle(mla_case, idx_case, fused)
 
 
+@pytest.mark.parametrize("t,n,r", [(673, 64, 256), (768, 64, 128), (1793, 38, 384)])
+def test_index_head_tiles_of_256_tokens(cuda, t, n, r):
+    # tiles of 256 tokens, whose halves of 128 go through LDS one after the other: the last tile of 161 tokens (both halves), of all
+    # 256 and of one (the second half empty)
+    mla_case, idx_case = op.make_fused_case(t, 1, 64, seed=100 + n, n_idx=64, h=256, q_lora_rank=r, n=n)
+    fused = run_fused(mla_case, idx_case, cuda, entry="mla_indexer_prolog_quant_p")
+    same_as_separate(fused, run_separate(mla_case, idx_case, cuda), idx_case)
+    check_against_oracle(mla_case, idx_case, fused)
+
+
 def test_index_head_counts_without_the_side_by_side_kernels(cuda):
     # 32 index heads: x @ w_proj is half an output tile wide, so the fused entry runs the two operators back to back
     mla_case, idx_case = op.make_fused_case(5, 1, 300, seed=23, n_idx=32, h=512, q_lora_rank=256, n=4)
