@@ -164,8 +164,8 @@ __global__ __launch_bounds__(512, 2) void mla_xa_kernel(MlaPrologArgs a)
     }
 }
 
-// Above 256 tokens the workgroup owns 128 tokens x 256 outputs (gemm_tile.h) over one split of the contraction, a multiple of
-// 256 rows chosen so that the workgroups fill the CUs once: few splits, so few partial sums.  Seven splits of 1024 rows
+// Above 256 tokens the workgroup owns 128 tokens x 256 outputs (gemm_tile.h) over one split of the contraction, whole stages of
+// 64 rows, so that the workgroups fill the CUs once: few splits, so few partial sums.  Seven splits of 1024 rows
 // with 256 x 64 tiles wrote 97 MB of partial sums at 1501 tokens, which the norm kernel read again.  An XCD takes neighbouring
 // workgroups in the order token tile, output tile, split.  grid (workgroups rounded up to a multiple of 8), 512 lanes.
 __global__ __launch_bounds__(GT_LANES, 2) void mla_xa_wide_kernel(MlaPrologArgs a, int ttiles, int ntiles, int rows)
@@ -199,13 +199,14 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_xa_wide_kernel(MlaPrologArgs 
             for (int nb = 0; nb < 2; ++nb) out[32 * nb] = acc[tb][nb][e];
         }
 }
-// its contraction rows per split: as many splits of at least 256 rows as there are CUs for, and no more than the workspace
-// holds.  The same with and without the indexer's columns (counted in), so that the fused operator's sums are the others'.
+// its contraction rows per split: as many splits as there are CUs for, and no more than the workspace holds, as even as whole
+// stages allow (in pieces of 256 rows, where three or five splits of 7168 end on an emptier one: fused prolog of 600 tokens 108.6 us a
+// call, so 107.1, 1024: 155.2 / 154.2; bf16 form of 600 118.4 / 116.4).  The same with and without the indexer's columns (counted in), so that the fused operator's sums are the others'.
 static int xa_wide_rows(int64_t t, int64_t h, int64_t r)
 {
     const int64_t tiles = ((t + 127) / 128) * ((r + MKV + PD + 64 + 255) / 256), most = (h + XA_SPLIT - 1) / XA_SPLIT;
     const int64_t splits = std::max<int64_t>(1, std::min<int64_t>(most, 256 / tiles));
-    return (int)((h / XA_K + splits - 1) / splits) * XA_K;
+    return (int)((h / GT_KBF + splits - 1) / splits) * GT_KBF;
 }
 
 // Four blocks of 64 outputs of q_b, TOK tokens each, from LDS rows of QBS_ROW bytes (padded against bank conflicts) to memory in

@@ -203,6 +203,15 @@ def test_index_head_tiles_of_256_tokens(cuda, t, n, r):
     check_against_oracle(mla_case, idx_case, fused)
 
 
+@pytest.mark.parametrize("t,n,h", [(300, 6, 1280), (300, 2, 2816)])
+def test_x_product_in_splits_of_whole_stages(cuda, t, n, h):
+    # two splits of ten stages of 64 rows, and of 15, 15 and 14: no multiples of the 256 that the hidden size is one of
+    mla_case, idx_case = op.make_fused_case(t, 1, 64, seed=110 + n, n_idx=64, h=h, q_lora_rank=128, n=n)
+    fused = run_fused(mla_case, idx_case, cuda, entry="mla_indexer_prolog_quant_p")
+    same_as_separate(fused, run_separate(mla_case, idx_case, cuda), idx_case)
+    check_against_oracle(mla_case, idx_case, fused)
+
+
 def test_index_head_counts_without_the_side_by_side_kernels(cuda):
     # 32 index heads: x @ w_proj is half an output tile wide, so the fused entry runs the two operators back to back
     mla_case, idx_case = op.make_fused_case(5, 1, 300, seed=23, n_idx=32, h=512, q_lora_rank=256, n=4)
