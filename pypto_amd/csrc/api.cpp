@@ -64,8 +64,8 @@ struct SfaPlan {
     uint64_t ws_bytes;
 };
 
-// Common checks of both attention entry points once the cache streams are resolved.  scratch: bytes of workspace there are, which the
-// choice of the KV splits keeps to where it has one.
+// Common checks of both attention entry points once the cache streams are resolved.  scratch: bytes of workspace that the choice of the
+// KV splits may use for tokens that one split each would do for (sfa_pick_splits).
 int plan_sfa(const char* op, const PtoTensorDesc& qn, const PtoTensorDesc& qr, const PtoTensorDesc& tk,
              const PtoTensorDesc& bt, const PtoTensorDesc& act, const PtoTensorDesc& out, int64_t out_rows,
              const PtoSfaParams* p, SfaPlan* plan, uint64_t scratch)
@@ -109,7 +109,7 @@ int plan_sfa(const char* op, const PtoTensorDesc& qn, const PtoTensorDesc& qr, c
     a.block_size = p->block_size;
     a.bt_stride = (int32_t)bt.shape[1];
     a.softmax_scale = p->softmax_scale;
-    a.splits = p->kv_splits > 0 ? pto::SfaSplits{(int32_t)t, p->kv_splits, p->kv_splits} : pto::sfa_pick_splits((int)t, p->nq, p->topk, scratch);
+    a.splits = p->kv_splits > 0 ? pto::SfaSplits{0, p->kv_splits} : pto::sfa_pick_splits((int)t, p->nq, p->topk, scratch);
     a.part_o = nullptr;
     a.part_ml = nullptr;
     plan->ws_bytes = pto::sfa_workspace_bytes((int)t, p->nq, a.splits);
@@ -123,7 +123,7 @@ int bind_workspace(const char* op, SfaPlan* plan, void* ws, uint64_t ws_bytes)
         return fail(PTO_ERR_WORKSPACE, "%s: workspace of %llu bytes required, got %llu", op,
                     (unsigned long long)plan->ws_bytes, (unsigned long long)(ws ? ws_bytes : 0));
     pto::SfaArgs& a = plan->args;
-    a.part_o = static_cast<_Float16*>(ws);
+    a.part_o = ws;
     a.part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + pto::sfa_partials_bytes(a.b * a.s1, a.nq, a.splits));
     return PTO_OK;
 }

@@ -6,18 +6,14 @@
 namespace pto {
 
 // ---------------------------------------------------------------- sparse flash attention
-// KV splits of the query tokens: `first` in each of the tokens before t1, `rest` in the others.  A token with more than one has as many
+// KV splits of the query tokens: one in each of the tokens before t1, n in the others.  A token with more than one has as many
 // partial results, in the order of the tokens; one with a single split writes its output itself.
 struct SfaSplits {
-    int32_t t1, first, rest;
-#ifdef __HIPCC__
-    __host__ __device__
-#endif
-    int64_t partial(int token) const // the first one of a token that has any
-    {
-        return token < t1 ? (int64_t)token * first : (first > 1 ? (int64_t)t1 * first : 0) + (int64_t)(token - t1) * rest;
-    }
-    int64_t partials(int t) const { return (first > 1 ? (int64_t)t1 * first : 0) + (rest > 1 ? (int64_t)(t - t1) * rest : 0); }
+    int32_t t1, n;
+    int64_t partials(int t) const { return n > 1 ? (int64_t)(t - t1) * n : 0; }
+    // Where all tokens are split, partial results are fp16.  Where some are not, the others' are fp32, which is what all of them have
+    // without the splits: the same range, and the same rounding to the output's type, for every token of the call.
+    bool fp32() const { return t1 > 0; }
 };
 
 struct SfaArgs {
@@ -34,11 +30,10 @@ struct SfaArgs {
     const int32_t* block_table; // [b, bt_stride]
     const int32_t* act_seq;     // [b]
     void* out;                  // [t*nq, 512] bf16
-    _Float16* part_o;           // [partial, head groups, 128 x 512] fp16 in the accumulators' fragment order: each split's output normalised by its own sum
+    void* part_o;               // [partial, head groups, 128 x 512] fp16 or fp32 (SfaSplits::fp32) in the accumulators' fragment order: each split's output normalised by its own sum
     float* part_ml;             // [partial, nq, 2]  fp32 (running max in log2 units, sum)
     int32_t b, s1, nq, topk, topk_stride, block_size, bt_stride;
     SfaSplits splits;
-    int32_t mixed;     // set by sfa_launch: the tokens do not all have the same number of splits
     int32_t split_cap; // set by sfa_launch: capacity (tokens) of the per-split LDS arrays
     int32_t bt_cached; // set by sfa_launch: the sequence's page table fits in LDS
     uint32_t page_mul; // set by sfa_launch: idx / block_size = idx * page_mul >> page_shift
@@ -47,9 +42,9 @@ struct SfaArgs {
     bool quant;
 };
 
-SfaSplits sfa_pick_splits(int t, int nq, int topk, uint64_t scratch); // scratch: bytes that the choice's partials should fit
+SfaSplits sfa_pick_splits(int t, int nq, int topk, uint64_t scratch); // scratch: bytes that the partial results of a last round's tokens may take
 uint64_t sfa_workspace_bytes(int t, int nq, const SfaSplits& splits);
-uint64_t sfa_partials_bytes(int t, int nq, const SfaSplits& splits); // the fp16 partials at the front of that workspace; (m, l) follow
+uint64_t sfa_partials_bytes(int t, int nq, const SfaSplits& splits); // the partial results at the front of that workspace; (m, l) follow
 hipError_t sfa_launch(const SfaArgs& a, hipStream_t stream);
 // Device address, on the current device, of the library's own scratch array of SFA_STATIC_SCRATCH_BYTES bytes (looked up
 // once per device).  Every call on a GPU shares that GPU's array.

@@ -34,7 +34,7 @@
 // pieces of the softmax, or between the scores; more fragments ahead; the int8 shares' stores free of bank conflicts (LDS 1.8 K);
 // equal priorities (4700).
 //
-// KV splits write their output normalised by their own sum as fp16, in the accumulators' fragment order, plus (m, l);
+// KV splits write their output normalised by their own sum as fp16 or fp32, in the accumulators' fragment order, plus (m, l);
 // sfa_combine_kernel merges them and turns the result into rows.
 #include <algorithm>
 #include <utility>
@@ -454,9 +454,11 @@ struct Values {
     }
     // Epilogue.  Register e of o[i][b] holds dim 16 (DB0 + i) + 4 g + e of head 16 b + lane % 16.
     // A split's share, normalised by its own sum, in fp16 (|value| <= max |V| and 2^-11 relative rounding, a quarter
-    // of the final bf16 rounding, half the bytes of fp32 for this kernel to write and the merge to read).  It leaves
+    // of the final bf16 rounding, half the bytes of fp32 for this kernel to write and the merge to read) where every token of the
+    // call is split, in fp32 where only a last round's are.  It leaves
     // in fragment order, straight from the accumulators: [token][split][head group][column group dq 4][pair 4][i 4][block of
-    // heads 2][lane 64] x 8 fp16, dims 4 g .. + 3 of column blocks 8 dq + 2 i and the next - every store instruction writes 1 KB of
+    // heads 2][lane 64] x 8 fp16, dims 4 g .. + 3 of column blocks 8 dq + 2 i and the next, or [column block 2][lane 64] x 4 fp32 in
+    // place of the last two - every store instruction writes 1 KB of
     // consecutive bytes, and nothing is staged.  The merge kernel reads the same order and does the transposition to
     // rows once, for the output, instead of once per split here.  (Streaming stores: 34 MB leave the chip's 256
     // workgroups at once and are read back once.)
@@ -474,6 +476,16 @@ struct Values {
                     x[k] = __builtin_bit_cast(uint32_t, f16x2{(_Float16)(o[2 * i + (k >> 1)][b][2 * (k & 1)] * mul[b]),
                                                               (_Float16)(o[2 * i + (k >> 1)][b][2 * (k & 1) + 1] * mul[b])});
                 __builtin_nontemporal_store(u32x4{x[0], x[1], x[2], x[3]}, reinterpret_cast<u32x4*>(base + (cb >> 2) * 16384 + ((cb & 3) * 2 + b) * 512));
+            }
+    }
+    __device__ __forceinline__ void store_partial(float* base, const float (&mul)[2])
+    {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const int cb = (DB0 + i) / 2;
+                __builtin_nontemporal_store(o[i][b] * mul[b], reinterpret_cast<f32x4*>(base + (cb >> 2) * 16384 + ((cb & 3) * 2 + b) * 512 + (i & 1) * 256));
             }
     }
     // One split: the output itself, bf16 rows [head][512] of 1024 bytes in LDS (orow: the pair's first).  v_permlane16_swap pairs up
@@ -510,20 +522,20 @@ __device__ __forceinline__ void copy_to_lds(const void* base, uint32_t offset, u
 // The body of one wavefront.  SCORES: the pair's score wave (waves 0 .. 3), which holds Q and does the scores, the softmax and
 // the values of the first NDB_S column blocks; else its value wave (waves 4 .. 7), which produces the tiles, eight rows of
 // each, and does the values of the other blocks.
-template <bool QUANT, bool SCORES>
+template <bool QUANT, bool SOME, bool SCORES>
 __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32_t* tmask, int* rows, int* bt_lds, int tid)
 {
     int tq = blockIdx.x, sp = blockIdx.y, nsplit = gridDim.y;
     const int hz = blockIdx.z;
-    if (a.mixed) { // the tokens before t1 first, split by split, then the others
-        const int w1 = a.splits.t1 * a.splits.first;
-        const bool first = tq < w1;
-        const int w = first ? tq : tq - w1, tokens = first ? a.splits.t1 : a.b * a.s1 - a.splits.t1;
-        nsplit = first ? a.splits.first : a.splits.rest;
-        sp = w / tokens;
-        tq = w - sp * tokens + (first ? 0 : a.splits.t1);
+    if constexpr (SOME) { // the tokens before t1 first, then the others, split by split
+        const int w = tq - a.splits.t1, tokens = a.b * a.s1 - a.splits.t1;
+        if (w >= 0) {
+            nsplit = a.splits.n;
+            sp = __builtin_amdgcn_readfirstlane(w / tokens); // (a division is vector code)
+            tq -= sp * tokens;
+        }
     }
-    const int64_t part = a.mixed ? a.splits.partial(tq) : (int64_t)tq * nsplit;
+    const int64_t part = (int64_t)(tq - (SOME ? a.splits.t1 : 0)) * nsplit; // (of a token with several splits: its first partial result)
     const int bi = tq / a.s1, si = tq - bi * a.s1;
     const int lane = tid & 63, pair = __builtin_amdgcn_readfirstlane(tid >> 6) & (PAIRS - 1); // (scalar: what follows from it is too)
     const int l16 = lane & 15, g = lane >> 4;
@@ -836,7 +848,10 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
         mul[b] = l_tot[b] > 0.f ? 1.f / l_tot[b] : 0.f;
     }
     if (nsplit > 1) {
-        if (active) val.store_partial(a.part_o + (((part + sp) * gridDim.z + hz) * 8 + (pair >> 1)) * 8192 + (pair & 1) * 4096 + lane * 8, mul);
+        using P = typename std::conditional<SOME, float, _Float16>::type;
+        const int64_t at = (((part + sp) * gridDim.z + hz) * 8 + (pair >> 1)) * 8192 + (pair & 1) * 4096;
+        // (counted in fp16 up to the lane's 16 bytes: counted in P the int8 value wave had a gather's registers spilled in every tile)
+        if (active) val.store_partial(reinterpret_cast<P*>(static_cast<_Float16*>(a.part_o) + at * (sizeof(P) / 2) + lane * 8), mul);
         return;
     }
     val.stage_rows(smem + pair * 32 * OUT_ROW, l16, g, mul);
@@ -857,10 +872,11 @@ __device__ __forceinline__ void sfa_wave(const SfaArgs& a, uint8_t* smem, uint32
     }
 }
 
-// grid (query tokens, KV splits, groups of 128 heads); where the tokens do not all have the same splits, (their sum, 1, groups).  Workgroups go to the XCDs round-robin in launch order, so with the
+// grid (query tokens, KV splits, groups of 128 heads); SOME: where only the tokens from t1 on are split, (sum of the splits, 1, groups).
+// Workgroups go to the XCDs round-robin in launch order, so with the
 // token as the fastest dimension the splits of one token run on one XCD (when the token count is a multiple of 8)
 // and share its L2 for the token's queries.
-template <bool QUANT>
+template <bool QUANT, bool SOME>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * WAVES, 64 * WAVES), amdgpu_waves_per_eu(2, 2))) void sfa_decode_kernel(
     SfaArgs a)
 {
@@ -870,9 +886,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * WAVES, 64 * WAVES), a
     int* bt_lds = reinterpret_cast<int*>(smem + BT_OFF);
     // both roles run the same barrier sequence
     if (threadIdx.x < 64 * PAIRS)
-        sfa_wave<QUANT, true>(a, smem, tmask, rows, bt_lds, threadIdx.x);
+        sfa_wave<QUANT, SOME, true>(a, smem, tmask, rows, bt_lds, threadIdx.x);
     else
-        sfa_wave<QUANT, false>(a, smem, tmask, rows, bt_lds, threadIdx.x);
+        sfa_wave<QUANT, SOME, false>(a, smem, tmask, rows, bt_lds, threadIdx.x);
 }
 
 // attention_out <- 0 (cache without rows: every selected entry is absent)
@@ -890,15 +906,21 @@ __global__ void sfa_zero_kernel(uint32_t* out, int64_t n_words)
 // eight for more than eight splits), every load of a group requested before any is used (splits past the last are the
 // last again with weight 0).  The workgroup then turns its 32 x 128 block through LDS
 // and writes the 256-byte row pieces, 16 lanes a piece.
+// grid (tokens with several splits x head groups x 16), 256 lanes; token0: the first of these tokens.  P: type of the partials.
 constexpr int CROW = 128 * 2 + 16; // LDS row of the merge's transposition: 128 bf16 plus one 16-byte chunk of padding
-template <int G>
-__device__ __forceinline__ void merge_splits(const _Float16* part_o, const float* part_ml, void* out, int nq, int nsplit, int64_t partial, int hgroups,
-                                             int task, uint8_t* tr)
+template <int G, class P>
+__global__ __launch_bounds__(256) void sfa_combine_kernel(const P* __restrict__ part_o, const float* __restrict__ part_ml, void* out, int nq, int nsplit,
+                                                          int token0, int hgroups)
 {
+    constexpr bool FP32 = std::is_same<P, float>::value;
+    typedef float f32x8 __attribute__((ext_vector_type(8)));
+    __shared__ __align__(16) uint8_t tr[32 * CROW];
     const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
     const int i = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int task = blockIdx.x; // ((token - token0) * hgroups + hz) * 8 + wv) * 2 + hb
     const int hb = task & 1, wv = (task >> 1) & 7;
-    const int th = task >> 4, hz = th % hgroups, tq = th / hgroups;
+    const int th = task >> 4, hz = th % hgroups, tq = token0 + th / hgroups;
+    const int64_t partial = (int64_t)(tq - token0) * nsplit;
     const int hh = wv & 1, dq = wv >> 1;
     const int head_base = hz * HEADS_PER_WG + 64 * hh + 32 * hb;
     if (head_base >= nq) return; // (a head block past the last head: nothing was written for it)
@@ -907,18 +929,24 @@ __device__ __forceinline__ void merge_splits(const _Float16* part_o, const float
     for (int x = 0; x < 16; ++x) (&acc[0][0])[x] = 0.f;
     float M = -INFINITY, L = 0.f;
     const int b = i & 1, cb = i & 2; // the wavefront's block of 16 heads and first of two column blocks
-    const int64_t split_stride = (int64_t)hgroups * 8 * 8192; // fp16 elements between two splits of a token
-    const _Float16* frag0 = part_o + ((partial * hgroups + hz) * 8 + wv) * 8192 + hb * 4096 + cb * 1024 + b * 512; // (the workgroup's four wavefronts read 8 KB in a row per split)
+    const int64_t split_stride = (int64_t)hgroups * 8 * 8192; // elements between two splits of a token
+    const P* frag0 = part_o + ((partial * hgroups + hz) * 8 + wv) * 8192 + hb * 4096 + cb * 1024 + b * 512; // (the workgroup's four wavefronts read 8 or 16 KB in a row per split)
     const float2* ml0 = reinterpret_cast<const float2*>(part_ml) + partial * nq + min(head_base + 16 * b + l16, nq - 1);
     for (int s0 = 0; s0 < nsplit; s0 += G) {
-        f16x8 v[G][2];
+        typename std::conditional<FP32, f32x8, f16x8>::type v[G][2];
         float2 ml[G];
 #pragma unroll
         for (int j = 0; j < G; ++j) {
             const int s = min(s0 + j, nsplit - 1);
-            const _Float16* base = frag0 + s * split_stride;
+            const P* base = frag0 + s * split_stride;
 #pragma unroll
-            for (int h = 0; h < 2; ++h) v[j][h] = *reinterpret_cast<const f16x8*>(base + h * 1024 + lane * 8);
+            for (int h = 0; h < 2; ++h) {
+                if constexpr (FP32) {
+                    const f32x4 *lo = reinterpret_cast<const f32x4*>(base + h * 1024) + lane, *hi = lo + 64;
+                    v[j][h] = __builtin_shufflevector(*lo, *hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                } else
+                    v[j][h] = *reinterpret_cast<const f16x8*>(base + h * 1024 + lane * 8);
+            }
             ml[j] = ml0[(int64_t)s * nq];
             if (s0 + j >= nsplit) ml[j].y = 0.f;
         }
@@ -964,27 +992,6 @@ __device__ __forceinline__ void merge_splits(const _Float16* part_o, const float
     }
 }
 
-// grid (tokens with several splits x head groups x 16), 256 lanes.  G of the tokens before t1 and of the others (0: these, or those, have
-// a single split); both in one launch: a second one for a few tokens costs more than the registers of the wider merge.
-template <int G1, int G2>
-__global__ __launch_bounds__(256) void sfa_combine_kernel(const void* __restrict__ part_o_fp16, const float* __restrict__ part_ml, void* out, int nq,
-                                                          SfaSplits splits, int hgroups)
-{
-    __shared__ __align__(16) uint8_t tr[32 * CROW];
-    const _Float16* part_o = static_cast<const _Float16*>(part_o_fp16); // (a plain pointer type keeps the symbol readable)
-    const int task = blockIdx.x + (G1 == 0 ? splits.t1 * hgroups * 16 : 0); // ((tq * hgroups + hz) * 8 + wv) * 2 + hb
-    const int tq = (task >> 4) / hgroups;
-    if constexpr (G1 != 0 && G2 != 0) {
-        if (tq < splits.t1)
-            merge_splits<G1>(part_o, part_ml, out, nq, splits.first, (int64_t)tq * splits.first, hgroups, task, tr);
-        else
-            merge_splits<G2>(part_o, part_ml, out, nq, splits.rest, splits.partial(tq), hgroups, task, tr);
-    } else if constexpr (G1 != 0)
-        merge_splits<G1>(part_o, part_ml, out, nq, splits.first, (int64_t)tq * splits.first, hgroups, task, tr);
-    else
-        merge_splits<G2>(part_o, part_ml, out, nq, splits.rest, (int64_t)(tq - splits.t1) * splits.rest, hgroups, task, tr);
-}
-
 int num_cus()
 {
     static std::atomic<int> cached[64]; // per device ordinal; 0 = not asked yet
@@ -1002,14 +1009,15 @@ int num_cus()
 
 // The KV splits.  One number for all tokens: one workgroup to a CU, and no more than share the tiles as well - nine splits of 64 tiles
 // are eight tiles each like eight splits, but leave more partials, and a second group of them to the merge (26 tokens: 77.0 us a pass
-// with nine, 73.9 with eight).  Or two: whole rounds of workgroups of the first tokens, and as many splits of the rest as fill the CUs
-// once more.  300 tokens in one split each are two rounds, the second for 44 of them.  By the time that either should take, in ns:
+// with nine, 73.9 with eight).  Where that is one split each and the tokens are some whole rounds of workgroups and a few more: as many
+// splits of these few as fill the CUs once more, where the last round takes less so.  By the time that either should take, in ns:
 // a tile (where more CUs work, the chip's clock falls: 150 workgroups 1700, 200: 1780, 256: 2030), the two ends of a workgroup, a
 // partial result's way to memory and back, the merge's launch.
-// Prefill calls of 2048 rows a token, one split for each and so: 129 tokens 108 -> 99 us, 257: 239 -> 156, 300: 245 -> 175, 360:
-// 247 -> 207, 520: 391 -> 296, 700: 409 -> 396.  (Two splits for 128 tokens and the rest in more where that is less by the formula: 144 tokens
-// 109 us as before, 160 by one split each 117, by two 115.)
-constexpr int64_t TILE_NS = 1550, TILE_FULL_NS = 480, ENDS_NS = 7000, PARTIAL_NS = 45, MERGE_NS = 2500;
+// Prefill calls of 128 heads and 2048 rows a token, one split each and so, int8 cache: 257 tokens 239 -> 162 us, 300: 249 -> 182, 360:
+// 253 -> 213, 384: 252 -> 224, 520: 378 -> 300, 640: 388 -> 358, 800: 514 -> 452; bf16 cache, 300: 248 -> 183, 384: 251 -> 224, packed rows the same.
+// (With fp16 partial results 300 take 175, and 129 in two splits each 102 instead of 118 - but calls of one split a token have fp32 sums
+// to the end, and their range.  rms error of the last round's tokens against 64 bits, 300 tokens: one split 2.163e-3, so 2.141e-3.)
+constexpr int64_t TILE_NS = 1550, TILE_FULL_NS = 480, ENDS_NS = 7000, PARTIAL_NS = 90, MERGE_NS = 2500;
 SfaSplits sfa_pick_splits(int t, int nq, int topk, uint64_t scratch)
 {
     const int hgroups = (nq + HEADS_PER_WG - 1) / HEADS_PER_WG, cus = std::max(1, num_cus() / hgroups); // (of a head group)
@@ -1019,27 +1027,20 @@ SfaSplits sfa_pick_splits(int t, int nq, int topk, uint64_t scratch)
         const int per = (tiles + n - 1) / n;
         return (tiles + per - 1) / per;
     };
-    // w workgroups of a token's n-th part
-    auto round_ns = [&](int n, int64_t w) { return (tiles + n - 1) / n * (TILE_NS + TILE_FULL_NS * std::min<int64_t>(w, cus) * std::min<int64_t>(w, cus) / (cus * cus)) + ENDS_NS; };
-    auto partials_ns = [&](const SfaSplits& s) { return s.partials(t) > 0 ? s.partials(t) * hgroups * PARTIAL_NS + MERGE_NS : 0; };
-    const int n = even(cus / std::max(t, 1));
-    SfaSplits best = {t, n, n};
-    const int64_t wgs = (int64_t)t * n, whole = wgs / cus;
-    int64_t best_ns = whole * round_ns(n, cus) + (wgs > whole * cus ? round_ns(n, wgs - whole * cus) : 0) + partials_ns(best);
-    for (int first = 1; first <= 2; ++first) {
-        const int per_round = cus / first, rounds = per_round > 0 ? t / per_round : 0, t1 = rounds * per_round;
-        if (t1 == 0 || t1 == t || even(first) != first || (first > 1 && rounds > 1)) continue;
-        const SfaSplits s = {t1, first, even(cus / (t - t1))};
-        const int64_t ns = rounds * round_ns(first, cus) + round_ns(s.rest, (int64_t)(t - t1) * s.rest) + partials_ns(s);
-        if (ns < best_ns && sfa_workspace_bytes(t, nq, s) <= scratch) best = s, best_ns = ns;
-    }
-    return best;
+    const int last = t % cus; // tokens of the last round, by one split each
+    if (t < cus || last == 0) return {0, even(cus / std::max(t, 1))};
+    auto round_ns = [&](int n) { // of the last round, its tokens in n splits each
+        const int64_t w = (int64_t)last * n;
+        return (tiles + n - 1) / n * (TILE_NS + TILE_FULL_NS * w * w / ((int64_t)cus * cus)) + ENDS_NS + (n > 1 ? w * hgroups * PARTIAL_NS + MERGE_NS : 0);
+    };
+    const SfaSplits some = {t - last, even(cus / last)};
+    return some.n > 1 && round_ns(some.n) < round_ns(1) && sfa_workspace_bytes(t, nq, some) <= scratch ? some : SfaSplits{0, 1};
 }
 
 uint64_t sfa_partials_bytes(int t, int nq, const SfaSplits& splits)
 {
     const int hgroups = (nq + HEADS_PER_WG - 1) / HEADS_PER_WG; // (whole 128-head groups: the partials lie in fragment order)
-    return (uint64_t)splits.partials(t) * hgroups * HEADS_PER_WG * DN * sizeof(_Float16);
+    return (uint64_t)splits.partials(t) * hgroups * HEADS_PER_WG * DN * (splits.fp32() ? sizeof(float) : sizeof(_Float16));
 }
 
 uint64_t sfa_workspace_bytes(int t, int nq, const SfaSplits& splits)
@@ -1087,43 +1088,38 @@ hipError_t sfa_launch(const SfaArgs& a, hipStream_t stream)
     while (((int64_t)1 << l) < a.block_size) ++l;
     args.page_mul = (uint32_t)((((uint64_t)1 << (31 + l)) + (uint32_t)a.block_size - 1) / (uint32_t)a.block_size);
     args.page_shift = 31 + l;
-    const int fewest = a.splits.t1 == t ? a.splits.first : a.splits.t1 == 0 ? a.splits.rest : std::min(a.splits.first, a.splits.rest); // of a token
+    const int t1 = a.splits.t1, n = a.splits.n, fewest = t1 > 0 ? 1 : n; // splits of a token
     args.split_cap = (((tiles + fewest - 1) / fewest + 1) & ~1) * T;
     const int smem_bytes = SPLIT_OFF + split_bytes(args.split_cap);
     args.bt_cached = a.bt_stride <= BT_MAX ? 1 : 0;
-    static DeviceOnce attr_done[2];
-    auto kern = a.quant ? sfa_decode_kernel<true> : sfa_decode_kernel<false>;
+    static DeviceOnce attr_done[2][2];
+    auto kern = t1 > 0 ? (a.quant ? sfa_decode_kernel<true, true> : sfa_decode_kernel<false, true>)
+                       : (a.quant ? sfa_decode_kernel<true, false> : sfa_decode_kernel<false, false>);
     {
-        hipError_t e = attr_done[a.quant].run([&] {
+        hipError_t e = attr_done[t1 > 0][a.quant].run([&] {
             return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        LDS_LIMIT);
         });
         if (e != hipSuccess) return e;
     }
     const int hgroups = (a.nq + HEADS_PER_WG - 1) / HEADS_PER_WG;
-    const int one = a.splits.t1 == t ? a.splits.first : a.splits.t1 == 0 || a.splits.first == a.splits.rest ? a.splits.rest : 0; // all tokens' splits
-    args.mixed = one == 0;
-    const int64_t wgs = (int64_t)a.splits.t1 * a.splits.first + (int64_t)(t - a.splits.t1) * a.splits.rest;
-    if (wgs > 0x7fffffff / (64 * WAVES)) return hipErrorInvalidValue;
-    const dim3 grid = one ? dim3(t, one, hgroups) : dim3((unsigned)wgs, 1, hgroups);
+    const dim3 grid = t1 > 0 ? dim3(t1 + (t - t1) * n, 1, hgroups) : dim3(t, n, hgroups);
     {
         ScopedKernelTimer tm(KID_SFA_DECODE, stream);
         hipLaunchKernelGGL(kern, grid, dim3(64 * WAVES), smem_bytes, stream, args);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const int n1 = a.splits.t1 > 0 && a.splits.first > 1 ? a.splits.first : 0, n2 = a.splits.t1 < t && a.splits.rest > 1 ? a.splits.rest : 0;
-    if (n1 || n2) {
+    if (n > 1) {
         ScopedKernelTimer tm(KID_SFA_COMBINE, stream);
-        const int tokens = (n1 ? a.splits.t1 : 0) + (n2 ? t - a.splits.t1 : 0);
-        auto group = [](int n) { return n == 0 ? 0 : n <= 2 ? 2 : n <= 4 ? 4 : 8; };
-        const int g1 = group(n1), g2 = group(n2);
-        // (two numbers of splits: the first is two)
-        auto merge = g1 && g2 ? (g2 <= 4 ? sfa_combine_kernel<2, 4> : sfa_combine_kernel<2, 8>)
-                   : g1 ? (g1 == 2 ? sfa_combine_kernel<2, 0> : g1 == 4 ? sfa_combine_kernel<4, 0> : sfa_combine_kernel<8, 0>)
-                        : (g2 == 2 ? sfa_combine_kernel<0, 2> : g2 == 4 ? sfa_combine_kernel<0, 4> : sfa_combine_kernel<0, 8>);
-        hipLaunchKernelGGL(merge, dim3(tokens * hgroups * 16), dim3(256), 0, stream, static_cast<const void*>(a.part_o),
-                           a.part_ml, a.out, a.nq, a.splits, hgroups);
+        const dim3 merges((t - t1) * hgroups * 16);
+        if (t1 > 0) {
+            auto merge = n <= 2 ? sfa_combine_kernel<2, float> : n <= 4 ? sfa_combine_kernel<4, float> : sfa_combine_kernel<8, float>;
+            hipLaunchKernelGGL(merge, merges, dim3(256), 0, stream, static_cast<const float*>(a.part_o), a.part_ml, a.out, a.nq, n, t1, hgroups);
+        } else {
+            auto merge = n <= 2 ? sfa_combine_kernel<2, _Float16> : n <= 4 ? sfa_combine_kernel<4, _Float16> : sfa_combine_kernel<8, _Float16>;
+            hipLaunchKernelGGL(merge, merges, dim3(256), 0, stream, static_cast<const _Float16*>(a.part_o), a.part_ml, a.out, a.nq, n, t1, hgroups);
+        }
         e = hipGetLastError();
     }
     return e;
