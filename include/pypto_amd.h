@@ -9,7 +9,7 @@
  * point it replaces; the launch is asynchronous on the caller's HIP stream unless `sync` is non-zero, in which case
  * it returns after the stream has drained (pypto_bundle_api.h:41-44: "sync!=0 waits for completion"); 0 means success.
  * Besides the reference's (workspace, stream, sync) a launch takes `workspace_bytes`, so that a short workspace is
- * refused instead of overrun.
+ * refused instead of overrun (or, where an attention call can do with less or none, not used: PtoSfaParams.kv_splits).
  *
  * Tensor descriptors use the reference's layout (pypto_bundle_api.h:30-35) and its DataType numbering
  * (framework/include/tilefwk/data_type.h:33-65).  All tensors are dense row-major device memory on the
@@ -62,7 +62,10 @@ typedef struct {
     int32_t topk;
     int32_t block_size;
     int32_t max_blocknum_perbatch;
-    int32_t kv_splits; /* 0 = choose from the problem size; >0 forces the number of KV splits per query token */
+    int32_t kv_splits; /* >0 forces the number of KV splits per query token; 0 = choose from the problem size.  Calls of more query
+                          tokens than the GPU has room for at once can have the last ones split, which is faster: the workspace
+                          reported is for that.  Launched with less (or none), every token of such a call has one split, which needs
+                          no workspace; the outputs' last bits differ between the two */
 } PtoSfaParams;
 
 /* Scalar arguments of lightning_indexer_decode
@@ -94,10 +97,11 @@ int pto_sfa_quant_launch(const PtoTensorDesc* tensors, uint32_t n_tensors, const
 /*
  * The allocation-free launch of sparse_flash_attention_quant: pto_sfa_quant_launch without the workspace arguments.
  * It has no counterpart in the reference.  It is for callers that cannot allocate device memory - code under HIP graph
- * capture, tight serving loops, harnesses that forbid it: the scratch the KV splits need (what
- * pto_sfa_quant_workspace reports) lives in an array inside the library, 40 MiB on every GPU the library runs on, held
- * until the process ends.  A problem that needs more is refused with PTO_ERR_WORKSPACE.  Every call on a GPU shares that
- * GPU's array: calls that overlap in time on one GPU (two streams, two threads) race; calls on one stream do not.
+ * capture, tight serving loops, harnesses that forbid it: the scratch the KV splits need lives in an array inside the
+ * library, 40 MiB on every GPU the library runs on, held until the process ends.  A problem that needs more is refused with
+ * PTO_ERR_WORKSPACE.  Calls that can do without scratch do (kv_splits = 0 and more query tokens than half the GPU has room for at
+ * once: one split each, the bits of pto_sfa_quant_launch without a workspace).  All others on a GPU share that GPU's array: those
+ * that overlap in time on one GPU (two streams, two threads) race; calls on one stream do not.
  * Tensors and parameters as for pto_sfa_quant_launch.
  */
 int pto_sfa_quant_launch_noalloc(const PtoTensorDesc* tensors, uint32_t n_tensors, const PtoSfaParams* params,

@@ -959,7 +959,7 @@ int pto_sfa_quant_launch_noalloc(const PtoTensorDesc* tensors, uint32_t n_tensor
 {
     const char* op = "sparse_flash_attention_quant (no-allocation entry)";
     SfaPlan plan;
-    int rc = plan_sfa_quant(tensors, n_tensors, params, &plan, pto::SFA_STATIC_SCRATCH_BYTES);
+    int rc = plan_sfa_quant(tensors, n_tensors, params, &plan, 0); // (the shared array is for calls that need it)
     if (rc) return rc;
     if (plan.ws_bytes > pto::SFA_STATIC_SCRATCH_BYTES)
         return fail(PTO_ERR_WORKSPACE, "%s: this problem needs %llu bytes of scratch, the library's own scratch array holds %llu; use pto_sfa_quant_launch with a workspace",

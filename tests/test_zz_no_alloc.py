@@ -3,7 +3,7 @@
 pto_sfa_quant_launch_noalloc takes no workspace: the partial results of the KV splits go to an array that lives in the
 library (one per GPU, held until the process ends).  Its output must equal pto_sfa_quant_launch's bit for bit - the same
 kernels run on the same split - on two calls in a row, the second on a smaller problem (the array keeps what the
-first call left in it).
+first call left in it).  Where one split a token fills the GPU it uses no scratch, and equals that entry without a workspace.
 """
 import ctypes
 
@@ -18,7 +18,7 @@ from _cases import sfa_golden
 pytestmark = pytest.mark.gpu
 
 
-def both_entries(case, dev):
+def both_entries(case, dev, workspace=True):
     from pypto_amd import _runtime
     lib = _runtime.load_library()
     fn = lib.pto_sfa_quant_launch_noalloc
@@ -40,9 +40,9 @@ def both_entries(case, dev):
             rc = fn(d, 9, ctypes.byref(p), stream, 1)
         else:
             n = lib.pto_sfa_quant_workspace(d, 9, ctypes.byref(p))
-            assert n > 0, "the case must need scratch, or the test shows nothing"
+            assert n > 0 or not workspace, "the case must need scratch, or the test shows nothing"
             ws = torch.empty(n, dtype=torch.uint8, device=dev)
-            rc = lib.pto_sfa_quant_launch(d, 9, ctypes.byref(p), ws.data_ptr(), n, stream, 1)
+            rc = lib.pto_sfa_quant_launch(d, 9, ctypes.byref(p), ws.data_ptr() if workspace else None, n if workspace else 0, stream, 1)
         assert rc == 0, lib.pto_last_error().decode()
         outs.append(out.cpu())
     return outs
@@ -57,6 +57,16 @@ def test_no_alloc_entry_matches_the_workspace_entry_twice(cuda):
         assert torch.equal(got, want)
         # and on its own against the oracle, to the attention tests' bar (every element within 1e-2 + 2e-2 |golden|)
         assert count_violations(got, sfa_golden(case), 1e-2, 2e-2) == 0
+
+
+@pytest.mark.parametrize("t", [129, 144, 256, 257, 300])
+def test_no_alloc_entry_without_scratch(cuda, t):
+    """More tokens than half of the 256 workgroups that run at once: one split each, also where the workspace entry splits the last
+    ones (257 and 300), so that calls on two streams share nothing."""
+    case = osfa.make_case(t, 40, 1, [300] * (t - 1) + [2100], topk=2048, seed=73, dist="bench", softmax_scale=192 ** -0.5)
+    want, got = both_entries(case, cuda, workspace=False)
+    assert torch.equal(got, want)
+    assert count_violations(got, sfa_golden(case), 1e-2, 2e-2) == 0
 
 
 def test_no_alloc_entry_rejects_what_does_not_fit(cuda):
