@@ -99,15 +99,18 @@ __global__ __launch_bounds__(512, 2) void mla_xa_kernel(MlaPrologArgs a)
     const uint16_t* x = a.x + kbeg;
     src += (int64_t)kbeg * ld;
     // copies of a wave (layout and exchange of the pieces: gemm_tile.h): token rows 64 i + 8 w + lane / 8 (the last rows again where
-    // eight waves have more hands than rows), weight rows 8 w + lane / 8
+    // eight waves have more hands than rows), weight rows 8 w + lane / 8.  Eight token rows are a base of their own: all of them can be
+    // more than 4 GB
     const int row = 8 * wave + (lane >> 3), pos = lane & 7;
+    const uint16_t* xp[XC];
     uint32_t xo[XC];
     int xd[XC];
 #pragma unroll
     for (int i = 0; i < XC; ++i) {
-        const int c = min(8 * i + wave, 4 * TT - 1), xrow = 8 * c + (lane >> 3);
+        const int c = min(8 * i + wave, 4 * TT - 1), xrow = 8 * c + (lane >> 3), xrow0 = min(8 * c, a.t - 1);
         xd[i] = 1024 * c;
-        xo[i] = (uint32_t)(min(xrow, a.t - 1) * a.h * 2 + 16 * (pos ^ ((xrow >> 1) & 7)));
+        xp[i] = x + (int64_t)xrow0 * a.h;
+        xo[i] = (uint32_t)(min(xrow, a.t - 1) - xrow0) * a.h * 2 + 16 * (pos ^ ((xrow >> 1) & 7));
     }
     const uint32_t wo = (uint32_t)(row * ld * 2 + 16 * (pos ^ ((row << 1) & 4)));
     const int tb = TT <= 4 ? wave >> 1 : wave, nb0 = TT <= 4 ? wave & 1 : 0;
@@ -126,7 +129,7 @@ __global__ __launch_bounds__(512, 2) void mla_xa_kernel(MlaPrologArgs a)
         [&](int st, int b) {
             gt_copy(src + (int64_t)st * XB_KS * ld, wo, lds + b + XBYTES + 1024 * wave);
 #pragma unroll
-            for (int i = 0; i < XC; ++i) gt_copy(x + st * XB_KS, xo[i], lds + b + xd[i]);
+            for (int i = 0; i < XC; ++i) gt_copy(xp[i] + st * XB_KS, xo[i], lds + b + xd[i]);
         },
         [&](int st, int b) {
             if (!busy) return;

@@ -282,6 +282,20 @@ def test_streamed_products_have_the_bits_of_the_decode_kernels(cuda, t, n, quant
     (check if quant_b else check_bf16_form)(case, many, **({} if quant_b else {"outliers": 1e-4}))
 
 
+def test_token_rows_beyond_4_gb(cuda):
+    """256 rows of 8421632 values, of which the last begins just beyond 4 GB: its results are the bits of a call of the last 20
+    tokens alone."""
+    h, r, n = 256 * 32897, 128, 2
+    case = op.make_case(256, 1, 64, seed=181, h=256, q_lora_rank=r, n=n)
+    g = torch.Generator(device=cuda).manual_seed(182)
+    for name, shape in (("x", (256, h)), ("w_dq", (h, r)), ("w_dkv_kr", (h, 576))):
+        case[name] = torch.empty(shape, dtype=torch.bfloat16, device=cuda).uniform_(-1, 1, generator=g)
+    many = run(case, cuda)
+    few = run({k: v[-20:].contiguous() if k in ("x", "cos", "sin", "cache_index") else v for k, v in case.items()}, cuda)
+    for name in ("q_norm", "q_norm_scale", "q_nope", "q_rope"):
+        assert torch.isfinite(many[name].float()).all() and torch.equal(many[name][-20:], few[name]), name
+
+
 def test_bf16_form_reference_case_b4_s2(cuda):
     # the reference's test_b4_s64k2_pa_nd_bf16_d: no quantisation anywhere (empty dequant_scale, bf16 w_uq_qr and cache)
     case = op.make_case(4, 2, 1024, seed=18, quant_b=False)
