@@ -906,13 +906,14 @@ __global__ void sfa_zero_kernel(uint32_t* out, int64_t n_words)
 // eight for more than eight splits), every load of a group requested before any is used (splits past the last are the
 // last again with weight 0).  The workgroup then turns its 32 x 128 block through LDS
 // and writes the 256-byte row pieces, 16 lanes a piece.
-// grid (tokens with several splits x head groups x 16), 256 lanes; token0: the first of these tokens.  P: type of the partials.
+// grid (tokens with several splits x head groups x 16), 256 lanes; token0: the first of these tokens.
 constexpr int CROW = 128 * 2 + 16; // LDS row of the merge's transposition: 128 bf16 plus one 16-byte chunk of padding
-template <int G, class P>
-__global__ __launch_bounds__(256) void sfa_combine_kernel(const P* __restrict__ part_o, const float* __restrict__ part_ml, void* out, int nq, int nsplit,
-                                                          int token0, int hgroups)
+template <int G, bool FP32>
+__global__ __launch_bounds__(256) void sfa_combine_kernel(const void* __restrict__ partials, const float* __restrict__ part_ml, void* out, int nq,
+                                                          int nsplit, int token0, int hgroups)
 {
-    constexpr bool FP32 = std::is_same<P, float>::value;
+    using P = typename std::conditional<FP32, float, _Float16>::type;
+    const P* part_o = static_cast<const P*>(partials); // (a plain pointer type keeps the symbol readable)
     typedef float f32x8 __attribute__((ext_vector_type(8)));
     __shared__ __align__(16) uint8_t tr[32 * CROW];
     const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
@@ -1113,13 +1114,9 @@ hipError_t sfa_launch(const SfaArgs& a, hipStream_t stream)
     if (n > 1) {
         ScopedKernelTimer tm(KID_SFA_COMBINE, stream);
         const dim3 merges((t - t1) * hgroups * 16);
-        if (t1 > 0) {
-            auto merge = n <= 2 ? sfa_combine_kernel<2, float> : n <= 4 ? sfa_combine_kernel<4, float> : sfa_combine_kernel<8, float>;
-            hipLaunchKernelGGL(merge, merges, dim3(256), 0, stream, static_cast<const float*>(a.part_o), a.part_ml, a.out, a.nq, n, t1, hgroups);
-        } else {
-            auto merge = n <= 2 ? sfa_combine_kernel<2, _Float16> : n <= 4 ? sfa_combine_kernel<4, _Float16> : sfa_combine_kernel<8, _Float16>;
-            hipLaunchKernelGGL(merge, merges, dim3(256), 0, stream, static_cast<const _Float16*>(a.part_o), a.part_ml, a.out, a.nq, n, t1, hgroups);
-        }
+        auto merge = t1 > 0 ? (n <= 2 ? sfa_combine_kernel<2, true> : n <= 4 ? sfa_combine_kernel<4, true> : sfa_combine_kernel<8, true>)
+                            : (n <= 2 ? sfa_combine_kernel<2, false> : n <= 4 ? sfa_combine_kernel<4, false> : sfa_combine_kernel<8, false>);
+        hipLaunchKernelGGL(merge, merges, dim3(256), 0, stream, static_cast<const void*>(a.part_o), a.part_ml, a.out, a.nq, n, t1, hgroups);
         e = hipGetLastError();
     }
     return e;
