@@ -285,10 +285,12 @@ __device__ __forceinline__ void gt_batch_i8(i32x4 (&acc)[2][TT], const int8_t* w
     using T = GtBatch<TT>;
     const int lane = threadIdx.x & 63, wave = gt_wave();
     const int l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
-    // copies of a wave: token rows 64 i + 8 w + lane / 8 (the last rows again where eight waves have more hands than rows), weight rows alike
+    // copies of a wave: token rows 64 i + 8 w + lane / 8 (the last rows again where eight waves have more hands than rows), weight rows
+    // alike, eight of them from a base of their own (128 can be more than 4 GB)
     const int row = 8 * wave + (lane >> 3), pos = lane & 7;
+    w += (int64_t)(8 * wave) * ldw;
     constexpr int QC = (TT + 1) / 2;
-    uint32_t qo[QC], wo[2];
+    uint32_t qo[QC], wo;
     int qd[QC];
 #pragma unroll
     for (int i = 0; i < QC; ++i) {
@@ -296,8 +298,7 @@ __device__ __forceinline__ void gt_batch_i8(i32x4 (&acc)[2][TT], const int8_t* w
         qd[i] = 1024 * c;
         qo[i] = (uint32_t)(min(qrow, t - 1) * (int)ldq + 16 * (pos ^ ((qrow >> 1) & 7)));
     }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) wo[i] = (uint32_t)((row + 64 * i) * (int)ldw + 16 * (pos ^ (((row >> 1) & 3) | ((row >> 2) & 4))));
+    wo = (uint32_t)(lane >> 3) * (uint32_t)ldw + 16 * (pos ^ (((row >> 1) & 3) | ((row >> 2) & 4))); // (the same 64 rows on)
     const uint8_t* qr = lds + (16 * TT * wr + l16) * 128;
     const int qpos = 16 * (g ^ ((l16 >> 1) & 7));
     const uint8_t* wrow = lds + T::QBYTES + (16 * g + (l16 >> 1)) * 128 + 8 * (l16 & 1);
@@ -308,7 +309,7 @@ __device__ __forceinline__ void gt_batch_i8(i32x4 (&acc)[2][TT], const int8_t* w
         stages,
         [&](int st, int b) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) gt_copy(w + (int64_t)st * GT_KI8 * ldw, wo[i], lds + b + T::QBYTES + 8192 * i + 1024 * wave);
+            for (int i = 0; i < 2; ++i) gt_copy(w + (int64_t)(st * GT_KI8 + 64 * i) * ldw, wo, lds + b + T::QBYTES + 8192 * i + 1024 * wave);
 #pragma unroll
             for (int i = 0; i < QC; ++i) gt_copy(q + st * GT_KI8, qo[i], lds + b + qd[i]);
         },

@@ -212,6 +212,19 @@ def test_x_product_in_splits_of_whole_stages(cuda, t, n, h):
     check_against_oracle(mla_case, idx_case, fused)
 
 
+def test_query_weights_whose_last_rows_lie_beyond_4_gb(cuda):
+    # 33 tokens, 128 rows of 33818880 outputs: the last heads' results are the bits of a call of these heads alone
+    n, r = 176140, 128
+    mla_case, idx_case = op.make_fused_case(33, 1, 64, seed=121, n_idx=64, h=256, q_lora_rank=r, n=2)
+    small = run_fused(mla_case, idx_case, cuda)
+    g = torch.Generator(device=cuda).manual_seed(122)
+    many = dict(mla_case, w_uq_qr=torch.randint(-127, 128, (r, n * 192), generator=g, device=cuda, dtype=torch.int8),
+                w_qb_scale=torch.full((n * 192, 1), 1e-3, device=cuda), w_uk=torch.zeros((n, 128, 512), dtype=torch.bfloat16, device=cuda))
+    many["w_uq_qr"][:, -384:], many["w_qb_scale"][-384:], many["w_uk"][-2:] = (mla_case[k].to(cuda) for k in ("w_uq_qr", "w_qb_scale", "w_uk"))
+    big = run_fused(many, idx_case, cuda)
+    assert torch.equal(big["q_nope"][:, -2:], small["q_nope"]) and torch.equal(big["q_rope"][:, -2:], small["q_rope"])
+
+
 def test_index_head_counts_without_the_side_by_side_kernels(cuda):
     # 32 index heads: x @ w_proj is half an output tile wide, so the fused entry runs the two operators back to back
     mla_case, idx_case = op.make_fused_case(5, 1, 300, seed=23, n_idx=32, h=512, q_lora_rank=256, n=4)
