@@ -1041,14 +1041,16 @@ static void token_blocks(int t, F&& f)
 // tokens where they are one round (us a call, tiles of 256 outputs and these: 40 tokens, 16 heads 31.7 / 26.7, 160 heads 36.4 / 34.5,
 // 192: 37.8 / 41.7; 150 tokens, 16 heads 39.9 / 38.0, 160: 55.2 / 52.2, 192: 61.4 / 71.4; 128 heads, 192 tokens 50.9 / 50.7, 224:
 // 52.2 / 53.5).  Beside the index heads' up to 128 tokens (against 128 x 128 tiles, 96 tokens: 16 heads 39.6 / 35.5, 256 heads, two
-// rounds: 69.1 / 65.4), to 160 where 256 outputs leave the chip half empty and these fill it (150 tokens, 16 heads 45.7 / 46.4, 64:
-// 49.0 / 49.7, 192: 70.3 / 74.4; 160 tokens, 128 heads 58.3 / 55.9, 192 tokens: 61.9 / 61.7).
+// rounds: 69.1 / 65.4), to 160 where 256 outputs leave the chip half empty and these fill it: by slices of 128 outputs, index heads among
+// them, at 129, 145 and 160 tokens 88: 41.4 / 41.4, 41.1 / 41.8, 41.5 / 42.5; 160: 45.4 / 45.2, 44.4 / 45.0, 44.8 / 45.7; 172: 45.5 / 44.9,
+// 45.5 / 45.3, 46.1 / 46.1; 184: 46.4 / 45.3, 46.4 / 45.6, 46.8 / 46.6; 196: 49.7 / 47.0, 50.0 / 47.3, 50.9 / 48.5; 256: 52.6 / 50.2, 51.7 / 49.5,
+// 52.4 / 50.2 (352, two rounds, at 150: 70.3 / 74.4; 256 slices, 192 tokens: 61.9 / 61.7).
 constexpr int QB_BATCH_T = 160;
 static bool qb_batch(const MlaPrologArgs& a, const PrologArgs* p)
 {
     const int slices = a.n * MQH / 128 + (p ? p->n : 0);
     if (a.t > QB_BATCH_T) return false;
-    return p ? a.t <= 128 || (slices > 192 && slices <= 256) : slices <= 256;
+    return p ? a.t <= 128 || (slices > 172 && slices <= 256) : slices <= 256;
 }
 
 // p == nullptr: the MLA prolog on its own; otherwise the fused operator (m and p bound by fused_prolog_bind)

@@ -173,7 +173,7 @@ def test_products_around_the_narrow_tiles_limit(cuda, t, n):
     check_against_oracle(mla_case, idx_case, fused)
 
 
-@pytest.mark.parametrize("t,n", [(33, 6), (64, 6), (65, 2), (96, 128), (97, 6), (128, 258), (129, 128), (160, 96), (161, 96), (150, 64)])
+@pytest.mark.parametrize("t,n", [(33, 6), (64, 6), (65, 2), (96, 128), (97, 6), (128, 258), (129, 128), (160, 96), (161, 96), (150, 64), (145, 72), (145, 74)])
 def test_streamed_products_of_33_to_160_tokens(cuda, t, n):
     # token blocks of 32: two to five with remainders of one and all rows, the last head count of one round of workgroups and one past
     # it (258 heads), and the tiles that take over
