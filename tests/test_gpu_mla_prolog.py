@@ -258,7 +258,7 @@ def test_decode_batches_of_many_heads(cuda, n, quant_b):
 
 @pytest.mark.parametrize("quant_b", [True, False])
 def test_a_tokens_bits_do_not_depend_on_the_batch(cuda, quant_b):
-    """Up to 32 tokens and from 33 on other kernels form the products; below 128 tokens their fp32 sums are the same (chains of 128
+    """Up to 32 tokens and from 33 on other kernels form the products; up to 256 tokens their fp32 sums are the same (chains of 128
     rows within 1024, and those in order), so a token's results are the same bits in a batch of 32 and of 100."""
     case = op.make_case(100, 1, 64, seed=77, h=1280, q_lora_rank=1536, n=32, quant_b=quant_b)
     first = {k: v[:32].contiguous() if k in ("x", "cos", "sin", "cache_index") else v for k, v in case.items()}
