@@ -951,6 +951,7 @@ __global__ __launch_bounds__(256) void sfa_combine_kernel(const void* __restrict
             ml[j] = ml0[(int64_t)s * nq];
             if (s0 + j >= nsplit) ml[j].y = 0.f;
         }
+        if constexpr (FP32) STEP_FENCE(); // (left alone, fewer of the loads are in flight: 8 tokens of 16 splits 14.4 us, so 10.5; 44 of 5: 13.4 / 13.0)
         // the group's maximum joins the running one: what was summed so far is rescaled once per group
         float Mg = M;
 #pragma unroll
@@ -1014,9 +1015,9 @@ int num_cus()
 // splits of these few as fill the CUs once more, where the last round takes less so.  By the time that either should take, in ns:
 // a tile (where more CUs work, the chip's clock falls: 150 workgroups 1700, 200: 1780, 256: 2030), the two ends of a workgroup, a
 // partial result's way to memory and back, the merge's launch.
-// Prefill calls of 128 heads and 2048 rows a token, one split each and so, int8 cache: 257 tokens 239 -> 162 us, 300: 249 -> 182, 360:
-// 253 -> 213, 384: 252 -> 224, 520: 378 -> 300, 640: 388 -> 358, 800: 514 -> 452; bf16 cache, 300: 248 -> 183, 384: 251 -> 224, packed rows the same.
-// (With fp16 partial results 300 take 175, and 129 in two splits each 102 instead of 118 - but calls of one split a token have fp32 sums
+// Prefill calls of 128 heads and 2048 rows a token, one split each and so, int8 cache: 257 tokens 239 -> 159 us, 300: 244 -> 177, 360:
+// 246 -> 208, 384: 247 -> 218, 520: 370 -> 287, 640: 377 -> 348, 800: 500 -> 437; bf16 cache and packed rows within 1 us of these.
+// (With fp16 partial results 300 take 170, and 129 in two splits each 102 instead of 118 - but calls of one split a token have fp32 sums
 // to the end, and their range.  rms error of the last round's tokens against 64 bits, 300 tokens: one split 2.163e-3, so 2.141e-3.)
 constexpr int64_t TILE_NS = 1550, TILE_FULL_NS = 480, ENDS_NS = 7000, PARTIAL_NS = 90, MERGE_NS = 2500;
 SfaSplits sfa_pick_splits(int t, int nq, int topk, uint64_t scratch)
