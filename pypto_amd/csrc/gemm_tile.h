@@ -6,8 +6,12 @@
 // instructions take 1792 ticks, the LDS reads and the copies' writes some 1250, the copies' instructions 960, and the loop is as
 // good as these overlap.  40 such stages take 122.6 K ticks with the copies issued first and the fragments read in front of
 // their products, 111 K with the copies between the matrix instructions, 107 K with the products half a stage behind the reads
-// besides (a call of 777 tokens x 112 heads 90.8 us, 88.7, 86.4; 1024 tokens 101.0, 98.3, 95.9).  The waves' priorities make no
-// difference: the second wave of a SIMD is done when it would be anyway, the first waits for it at the barrier.  And
+// besides (a call of 777 tokens x 112 heads 90.8 us, 88.7, 86.4; 1024 tokens 101.0, 98.3, 95.9).  With the reads between the matrix
+// instructions too, instead of in one go behind the barrier, a stage by itself takes 2295 ticks, not 2440 (256 tokens 2490 / 2717, 128:
+// 1488 / 1551; calls of 777 and 1024 tokens 75.6 -> 71.8 us and 79.9 -> 78.7).  Below that the chip's power decides: matrix
+// instructions 78 % of the time hold the clock at 1.85 GHz (four waves with half again the tile each read a quarter less of LDS, and
+// the compiler moves their sums between register files: 57 -> 74 us at 256 tokens).  The waves' priorities make no difference: the
+// second wave of a SIMD is done when it would be anyway, the first waits for it at the barrier.  And
 //  - a stage's operands are copied to LDS by the memory pipe itself (global_load_lds_dwordx4: no registers, no LDS store
 //    instructions), into the buffer that is not being read, so that a stage has one barrier;
 //  - rows of 128 bytes are kept unpadded (a copy writes 64 lanes x 16 bytes in a row) and spread over the banks by
@@ -195,23 +199,20 @@ __device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t*
         }
     };
     gt_tile_stages<T::RING, T::QBYTES, QC, T::WRING, T::WBYTES, 4>(stages, copy_q, copy_w, [&](int, int b, int bw, auto&& issue) {
-        auto read = [&](int ks) {
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-                const uint8_t* p = wrow + bw + 8192 * ks + wpos[nb];
+        auto read = [&](int ks, int i) { // token block i's fragment, and with the first four the weights'
+            if (i < 4) {
+                const uint8_t* p = wrow + bw + 8192 * ks + wpos[i];
                 const v2i lo = lds_read_tr8(p), hi = lds_read_tr8(p + 1024);
-                wf[ks][nb] = i32x4{lo[0], lo[1], hi[0], hi[1]};
+                wf[ks][i] = i32x4{lo[0], lo[1], hi[0], hi[1]};
             }
-#pragma unroll
-            for (int tb = 0; tb < TB; ++tb) qf[ks][tb] = *reinterpret_cast<const i32x4*>(qr + b + 2048 * tb + (qpos ^ (64 * ks)));
-            __builtin_amdgcn_sched_barrier(0);
+            qf[ks][i] = *reinterpret_cast<const i32x4*>(qr + b + 2048 * i + (qpos ^ (64 * ks)));
         };
-        read(0);
         mfma(1, [&](int tb) {
+            read(0, tb);
             if (tb < QC + 4) issue(tb);
         });
-        read(1);
         mfma(0, [&](int tb) {
+            read(1, tb);
             if (TB + tb < QC + 4) issue(TB + tb);
         });
     });
