@@ -533,6 +533,251 @@ __device__ __forceinline__ void mla_norm_key_body(const MlaPrologArgs& a, int to
     }
 }
 
+// The fused operator's norms where the x product has at most four splits (above 640 tokens at model sizes): a wavefront to each of a
+// token's three chains, the sums of the workgroups above bit for bit - what they spread over four wavefronts (lane l of wave w: columns
+// l + 64 w + 256 i) are four sums of a lane here, and no barrier is passed.
+// What bounds it: the partial sums' way from memory (28 MB at 1501 tokens).  A workgroup to a chain went through barriers with
+// eight chains in flight to a CU, and every token's fetched hadamard_k's 32 KB out of the L2 in 128 loads: the kernel at 1501 tokens 15.1 us, so 11.6,
+// a call 210.7 -> 208.1, 900: 140.4 / 138.1.  The MLA prolog's two chains alone are as fast either way (1024 tokens 8.3 / 8.4).
+// request(i, split) asks for what a chain reads of a split, all S of them in flight together (a split past the end is the last one
+// again, dropped), add(i, first, real) adds it up in order.
+template <int S, class Request, class Add>
+__device__ __forceinline__ void each_split(int ksplits, Request&& request, Add&& add)
+{
+#pragma unroll
+    for (int i = 0; i < S; ++i) request(i, min(i, ksplits - 1));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < S; ++i) add(i, i == 0, i < ksplits);
+}
+
+template <int S, int NP>
+__device__ __forceinline__ void mla_norm_query_wave(const MlaPrologArgs& a, int tok, float* buf)
+{
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & 63, r = a.r;
+    f32x4 x[NP], v[S][NP];
+    each_split<S>(
+        a.ksplits,
+        [&](int i, int split) {
+            const float* p = a.xa_part + ((int64_t)split * a.t + tok) * a.ncols;
+#pragma unroll
+            for (int j = 0; j < NP; ++j) v[i][j] = *reinterpret_cast<const f32x4*>(p + min(256 * j + 4 * lane, r - 4));
+        },
+        [&](int i, bool first, bool real) {
+#pragma unroll
+            for (int j = 0; j < NP; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[j][e] = first ? v[i][j][e] : x[j][e] + (real ? v[i][j][e] : 0.f);
+        });
+    u32x2 gq[NP];
+#pragma unroll
+    for (int j = 0; j < NP; ++j) gq[j] = *reinterpret_cast<const u32x2*>(a.gamma_cq + min(256 * j + 4 * lane, r - 4));
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[j][e] = round_bf16(x[j][e]);
+        *reinterpret_cast<f32x4*>(buf + 256 * j + 4 * lane) = 256 * j + 4 * lane < r ? x[j] : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    __builtin_amdgcn_wave_barrier();
+    const float coff = 1.0f / (float)r;
+    float ss[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        ss[w] = 0.f;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const float b = buf[256 * i + 64 * w + lane]; // (zero past the end)
+            ss[w] += (b * b) * coff;
+        }
+    }
+#pragma unroll
+    for (int w = 0; w < 4; ++w) ss[w] = wave_sum(ss[w]);
+    const float y = 1.0f / sqrtf(((ss[0] + ss[1]) + (ss[2] + ss[3])) + a.eps_cq);
+    float mx = 0.f; // (columns past the end are the last ones again)
+#pragma unroll
+    for (int j = 0; j < NP; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            x[j][e] = round_bf16(half_of(gq[j][e >> 1], e & 1) * (x[j][e] * y));
+            mx = fmaxf(mx, fabsf(x[j][e]));
+        }
+    if (a.quant) {
+        const float sq = quant_scale(wave_max(mx));
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            const int c = 256 * j + 4 * lane;
+            uint32_t pk = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(x[j][e] * sq) & 0xffu) << (8 * e);
+            if (c < r) *reinterpret_cast<uint32_t*>(a.q_norm + (int64_t)tok * r + c) = pk;
+        }
+        if (lane == 0) a.q_norm_scale[tok] = 1.0f / sq;
+    } else {
+        uint16_t* qo = reinterpret_cast<uint16_t*>(a.q_norm) + (int64_t)tok * r;
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            const int c = 256 * j + 4 * lane;
+            if (c < r) *reinterpret_cast<u32x2*>(qo + c) = u32x2{pack_bf16x2(x[j][0], x[j][1]), pack_bf16x2(x[j][2], x[j][3])};
+        }
+    }
+}
+
+// lane l: columns l + 64 m of the 512 normalised ones, and (l < 32) the rotary pair 2 l, 2 l + 1
+template <int S>
+__device__ __forceinline__ void mla_norm_key_wave(const MlaPrologArgs& a, int tok)
+{
+#pragma clang fp contract(off)
+    constexpr int M = MC / 64;
+    const int lane = threadIdx.x & 63, ri = lane & 31;
+    const int64_t row = a.cache_index[tok];
+    uint16_t gk[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) gk[m] = a.gamma_ckv[64 * m + lane];
+    const float rc0 = bf16_to_f32(a.cos[(int64_t)tok * MROPE + ri]), rc1 = bf16_to_f32(a.cos[(int64_t)tok * MROPE + ri + 32]);
+    const float rs0 = bf16_to_f32(a.sin[(int64_t)tok * MROPE + ri]), rs1 = bf16_to_f32(a.sin[(int64_t)tok * MROPE + ri + 32]);
+    float x[M], pv[S][M];
+    float2 pair, pp[S];
+    each_split<S>(
+        a.ksplits,
+        [&](int i, int split) {
+            const float* p = a.xa_part + ((int64_t)split * a.t + tok) * a.ncols + a.r;
+#pragma unroll
+            for (int m = 0; m < M; ++m) pv[i][m] = p[64 * m + lane];
+            pp[i] = *reinterpret_cast<const float2*>(p + MC + 2 * ri);
+        },
+        [&](int i, bool first, bool real) {
+#pragma unroll
+            for (int m = 0; m < M; ++m) x[m] = first ? pv[i][m] : x[m] + (real ? pv[i][m] : 0.f);
+            pair.x = first ? pp[i].x : pair.x + (real ? pp[i].x : 0.f);
+            pair.y = first ? pp[i].y : pair.y + (real ? pp[i].y : 0.f);
+        });
+    const bool row_ok = row >= 0 && row < a.cache_rows;
+    float ss[4], v[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) x[m] = round_bf16(x[m]);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) ss[w] = wave_sum((x[w] * x[w]) * (1.0f / MC) + (x[w + 4] * x[w + 4]) * (1.0f / MC));
+    const float y = 1.0f / sqrtf(((ss[0] + ss[1]) + (ss[2] + ss[3])) + a.eps_ckv);
+#pragma unroll
+    for (int m = 0; m < M; ++m) v[m] = round_bf16(bf16_to_f32(gk[m]) * (x[m] * y));
+    if (a.quant) {
+#pragma unroll
+        for (int g = 0; g < M / 2; ++g) { // groups of 128
+            const float sq = quant_scale(wave_max(fmaxf(fabsf(v[2 * g]), fabsf(v[2 * g + 1]))));
+            if (row_ok) {
+                a.kv_cache[row * MC + 128 * g + lane] = (int8_t)(int)__builtin_rintf(v[2 * g] * sq);
+                a.kv_cache[row * MC + 128 * g + 64 + lane] = (int8_t)(int)__builtin_rintf(v[2 * g + 1] * sq);
+                if (lane == 0) a.k_scale_cache[row * 4 + g] = 1.0f / sq;
+            }
+        }
+    } else if (row_ok) {
+        uint16_t* kvo = reinterpret_cast<uint16_t*>(a.kv_cache) + row * MC;
+#pragma unroll
+        for (int m = 0; m < M; ++m) kvo[64 * m + lane] = f32_to_bf16(v[m]);
+    }
+    if (lane < MROPE / 2 && row_ok) {
+        const float xe = round_bf16(pair.x), xo = round_bf16(pair.y);
+        a.kr_cache[row * MROPE + lane] = f32_to_bf16(xe * rc0 + (-xo) * rs0);
+        a.kr_cache[row * MROPE + 32 + lane] = f32_to_bf16(xo * rc1 + xe * rs1);
+    }
+}
+
+// The indexer's key path and weights (prolog_k_body's arithmetic); had: hadamard_k in LDS
+template <int S>
+__device__ __forceinline__ void prolog_k_wave(const PrologArgs& a, int tok, const uint32_t* had)
+{
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & 63;
+    const int64_t row = a.k_cache_index[tok];
+    float gam[2], bet[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        gam[m] = bf16_to_f32(a.ln_gamma[64 * m + lane]);
+        bet[m] = bf16_to_f32(a.ln_beta[64 * m + lane]);
+    }
+    const float rc = bf16_to_f32(a.cos[(int64_t)tok * PROPE + lane]), rs = bf16_to_f32(a.sin[(int64_t)tok * PROPE + lane]);
+    float kv[2], wv[2], v0[S][2], v1[S][2];
+    each_split<S>(
+        a.ksplits,
+        [&](int i, int split) {
+            const float* p = a.xw_part + ((int64_t)split * a.t + tok) * a.xw_stride + a.xw_col0;
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                v0[i][m] = p[64 * m + lane];
+                v1[i][m] = p[PD + min(64 * m + lane, a.n - 1)];
+            }
+        },
+        [&](int i, bool first, bool real) {
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                kv[m] = first ? v0[i][m] : kv[m] + (real ? v0[i][m] : 0.f);
+                wv[m] = first ? v1[i][m] : wv[m] + (real ? v1[i][m] : 0.f);
+            }
+        });
+    const float mean = (wave_sum(kv[0]) + wave_sum(kv[1])) / (float)PD;
+    float dlt[2], kb[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) dlt[m] = kv[m] - mean;
+    const float var = (wave_sum(dlt[0] * dlt[0]) + wave_sum(dlt[1] * dlt[1])) / (float)PD;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        float xn = dlt[m] / sqrtf(var + a.eps);
+        xn = xn * gam[m] + bet[m];
+        kb[m] = round_bf16(xn);
+    }
+    // rotary on the first 64 dims: the partner is 32 lanes away
+    const float far = __shfl_xor(kb[0], 32);
+    kb[0] = round_bf16(kb[0] * rc + (lane < 32 ? -far : far) * rs);
+    // hadamard: columns 2 l, 2 l + 1, k in order
+    float2 h = {0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < PD; ++k) {
+        const float x = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, kb[k >> 6]), k & 63));
+        const uint32_t hk = had[64 * k + lane];
+        h.x = __builtin_fmaf(x, half_of(hk, 0), h.x);
+        h.y = __builtin_fmaf(x, half_of(hk, 1), h.y);
+    }
+    const float y0 = round_bf16(h.x), y1 = round_bf16(h.y);
+    const float sq = quant_scale(wave_max(fmaxf(fabsf(y0), fabsf(y1))));
+    if (row >= 0 && row < a.cache_rows) {
+        const uint32_t q0 = (uint32_t)(int)__builtin_rintf(y0 * sq) & 0xffu, q1 = (uint32_t)(int)__builtin_rintf(y1 * sq) & 0xffu;
+        *reinterpret_cast<uint16_t*>(a.k_cache + row * PD + 2 * lane) = (uint16_t)(q0 | (q1 << 8));
+        if (lane == 0) a.k_scale_cache[row] = __builtin_bit_cast(uint16_t, (_Float16)(1.0f / sq));
+    }
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+        if (64 * m + lane < a.n) {
+            const float w = bf16_to_f32(f32_to_bf16(wv[m]));
+            a.weights[(int64_t)tok * a.n + 64 * m + lane] = __builtin_bit_cast(uint16_t, (_Float16)((w * a.wscale_n) * a.wscale_d));
+        }
+}
+
+// grid (3 ceil(t / 4): the indexer's keys, queries, keys; four tokens to a workgroup), 256 lanes
+template <int S, int NP>
+__global__ __launch_bounds__(256) void fused_norm_wide_kernel(MlaPrologArgs m, PrologArgs p)
+{
+    constexpr int QB = 4 * NP * 256 * 4, HB = PD * PD * 2;
+    __shared__ __align__(16) uint8_t lds[HB > QB ? HB : QB];
+    const int groups = (m.t + 3) / 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int part = blockIdx.x / groups, tok = 4 * (blockIdx.x % groups) + wave;
+    if (part == 0) {
+        u32x4 h[HB / 4096];
+#pragma unroll
+        for (int i = 0; i < HB / 4096; ++i) h[i] = reinterpret_cast<const u32x4*>(p.had_k)[threadIdx.x + 256 * i];
+#pragma unroll
+        for (int i = 0; i < HB / 4096; ++i) reinterpret_cast<u32x4*>(lds)[threadIdx.x + 256 * i] = h[i];
+        __syncthreads();
+    }
+    if (tok >= m.t) return;
+    if (part == 0)
+        prolog_k_wave<S>(p, tok, reinterpret_cast<const uint32_t*>(lds));
+    else if (part == 1)
+        mla_norm_query_wave<S, NP>(m, tok, reinterpret_cast<float*>(lds) + wave * NP * 256);
+    else
+        mla_norm_key_wave<S>(m, tok);
+}
+
 // The head of a weight slice, read and dropped: the first `rows` rows of 16 `pieces` bytes (rows a multiple of what 256 lanes
 // cover in one go, up to 24 times that), so that the workgroup of the next launch that streams the slice finds them in
 // its XCD's L2.
@@ -1099,7 +1344,22 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
             else
                 launch(std::integral_constant<int, 8>{}, touch);
         };
-        if (ahead)
+        if (p && a.t > BIG_T2 && a.ksplits <= 4) {
+            auto wide = [&](auto splits, auto pieces) {
+                hipLaunchKernelGGL((fused_norm_wide_kernel<decltype(splits)::value, decltype(pieces)::value>), dim3(3 * ((a.t + 3) / 4)), dim3(256), 0,
+                                   stream, a, *p);
+            };
+            auto wide_with = [&](auto splits) {
+                if (a.r <= 1536)
+                    wide(splits, std::integral_constant<int, 6>{});
+                else
+                    wide(splits, std::integral_constant<int, MAX_R / 256>{});
+            };
+            if (in_flight == 2)
+                wide_with(std::integral_constant<int, 2>{});
+            else
+                wide_with(std::integral_constant<int, 4>{});
+        } else if (ahead)
             launch_with(std::true_type{});
         else
             launch_with(std::false_type{});
