@@ -233,6 +233,33 @@ def test_forced_kv_splits_agree(cuda):
         assert count_violations(o, outs[0], 2e-3, 2.0 ** -5) == 0
 
 
+@pytest.mark.parametrize("nq,splits,quant", [(128, 8, True), (128, 9, True), (33, 12, True), (130, 16, True), (200, 17, False), (1, 32, True),
+                                             (96, 33, True), (128, 64, True)])
+def test_merge_of_more_than_eight_splits(cuda, nq, splits, quant):
+    """Four wavefronts take every fourth split, four or eight of them at a time: 9 and 12 (the last ones missing), 16, 17 and 32 in one go,
+    33 and 64 in more; lists of no entry, of one tile and of some leave splits without a tile, and heads end inside the blocks of 16."""
+    case = osfa.make_case(4, nq, 1, [2300, 0, 31, 1500], topk=2048, seed=90 + splits, dist="bench", quant=quant, softmax_scale=192 ** -0.5)
+    case["topk_indices"][0, 96:512] = -1 # whole tiles without a present entry: splits that attended to nothing
+    keep = torch.cat([case["topk_indices"][:, :96], case["topk_indices"][:, 512:]], dim=1).contiguous()
+    out = run_with_splits(case, cuda, splits)
+    assert (out[1] == 0).all()
+    one = run_with_splits(case, cuda, 1)
+    # splits differ only in where P~ is rounded to bf16 (relative to each split's own maximum)
+    assert count_violations(out, one, 2e-3, 2.0 ** -5) == 0
+    first = dict(case, b=1, q=case["q"][:1].contiguous(), act_seq=case["act_seq"][:1], block_table=case["block_table"][:1].contiguous(),
+                 topk=keep.shape[1], topk_indices=keep[:1].contiguous())
+    golds = [sfa_golden(first), sfa_golden(first, flash=True, s2_tile=512)]
+    check_rms_vs_fp64(out[:1], first, golds, f"{nq} heads, {splits} splits")
+
+
+def test_a_single_token_has_up_to_32_splits(cuda):
+    case = osfa.make_case(1, 128, 1, [5000], topk=2048, seed=95, dist="bench", softmax_scale=192 ** -0.5)
+    out = run_sfa(case, cuda)
+    full_check(out, case, "one token")
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert torch.equal(out, run_with_splits(case, cuda, 32))
+
+
 @pytest.mark.parametrize("t,rest", [(18, 8), (17, 16), (35, 5), (16, 1), (15, 1), (9, 1)])
 def test_tokens_with_different_splits(cuda, t, rest):
     """2048 heads are 16 workgroups a token: 16 tokens fill the CUs.  With a few more, the first tokens are whole rounds of one split
