@@ -24,6 +24,7 @@
 #include <stdint.h>
 
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "prolog_common.h"
@@ -93,6 +94,56 @@ __device__ __forceinline__ void gt_stages(int stages, Copy&& copy, Multiply&& mu
         in = in == (RING - 1) * STAGE ? 0 : in + STAGE;
         out = out == (RING - 1) * STAGE ? 0 : out + STAGE;
     }
+    gt_landed<0>();
+}
+
+// f(integral_constant 0) .. f(integral_constant N - 1), written out
+template <class F, int... I>
+__device__ __forceinline__ void gt_unroll_seq(std::integer_sequence<int, I...>, F&& f)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void gt_unroll(F&& f)
+{
+    gt_unroll_seq(std::make_integer_sequence<int, N>{}, static_cast<F&&>(f));
+}
+
+// The same with MORE stages of something else behind them, whose copies (as many) follow without a gap: copy_more(stage, byte offset),
+// between() in front of the first of them (what it leaves in LDS is there for multiply_more), multiply_more(integral constant stage,
+// byte offset).
+template <int RING, int STAGE, int COPIES, int MORE, class Copy, class Multiply, class CopyMore, class Between, class MultiplyMore>
+__device__ __forceinline__ void gt_stages_more(int stages, Copy&& copy, Multiply&& multiply, CopyMore&& copy_more, Between&& between,
+                                               MultiplyMore&& multiply_more)
+{
+    static_assert(MORE >= RING - 1, "no copies past the end");
+    auto any = [&](int st, int b) { // (uniform)
+        if (st < stages)
+            copy(st, b);
+        else
+            copy_more(st - stages, b);
+    };
+#pragma unroll
+    for (int s = 0; s < RING - 1; ++s) any(s, s * STAGE);
+    int in = (RING - 1) * STAGE, out = 0;
+    auto turn = [&]() {
+        in = in == (RING - 1) * STAGE ? 0 : in + STAGE;
+        out = out == (RING - 1) * STAGE ? 0 : out + STAGE;
+    };
+    for (int st = 0; st < stages; ++st) {
+        gt_landed<(RING - 2) * COPIES>();
+        any(st + RING - 1, in);
+        multiply(st, out);
+        turn();
+    }
+    between();
+    gt_unroll<MORE>([&](auto ic) {
+        constexpr int c = ic, ahead = c + RING - 2 < MORE - 1 ? RING - 2 : MORE - 1 - c;
+        gt_landed<ahead * COPIES>();
+        if constexpr (c + RING - 1 < MORE) copy_more(c + RING - 1, in);
+        multiply_more(ic, out);
+        turn();
+    });
     gt_landed<0>();
 }
 
@@ -222,11 +273,13 @@ __device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t*
 // Up to 32 tokens x 128 outputs, 256 lanes: a stream of weights, three stages of 128 rows in flight straight to LDS (with five, or
 // two, the fused prolog of 8 tokens takes 0.4 us longer: 28.4 us, weights out of HBM 32.8).  Wave w owns outputs [32 w, +32).
 // Register e of acc[nb][tb]: output 32 w + 16 nb + 4 g + e, token 16 tb + l16.
-struct GtStream {
+struct GtStream { // (a stage's token rows first)
     static constexpr int TOK = 32, QBYTES = TOK * 128, STAGE = QBYTES + 128 * 128, RING = 4, LDS = RING * STAGE;
 };
-__device__ __forceinline__ void gt_stream_i8(i32x4 (&acc)[2][2], const int8_t* w, int64_t ldw, const int8_t* q, int64_t ldq, int t,
-                                             int stages, uint8_t* lds)
+// The outputs are two times 64 that lie `gap` columns apart (0: 128 in a row).  run(copy, multiply) goes through the stages.
+template <class Run>
+__device__ __forceinline__ void gt_stream_i8(i32x4 (&acc)[2][2], const int8_t* w, int gap, int64_t ldw, const int8_t* q, int64_t ldq, int t,
+                                             uint8_t* lds, Run&& run)
 {
     using T = GtStream;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -236,13 +289,15 @@ __device__ __forceinline__ void gt_stream_i8(i32x4 (&acc)[2][2], const int8_t* w
     const uint32_t qo = (uint32_t)(min(row, t - 1) * (int)ldq + 16 * (pos ^ ((row >> 1) & 7)));
     uint32_t wo[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) wo[i] = (uint32_t)((row + 32 * i) * (int)ldw + 16 * (pos ^ (((row >> 1) & 3) | ((row >> 2) & 4))));
+    for (int i = 0; i < 4; ++i) {
+        const int piece = pos ^ (((row >> 1) & 3) | ((row >> 2) & 4));
+        wo[i] = (uint32_t)((row + 32 * i) * (int)ldw + 16 * piece + (piece >= 4 ? gap : 0));
+    }
     const uint8_t* qr = lds + l16 * 128;
     const int qpos = 16 * (g ^ ((l16 >> 1) & 7));
     const uint8_t* wrow = lds + T::QBYTES + (16 * g + (l16 >> 1)) * 128 + 8 * (l16 & 1);
     const int wf0 = ((l16 >> 2) & 3) | ((g & 1) << 2); // (transposing reads: see gt_product_i8)
-    gt_stages<T::RING, T::STAGE, 5>(
-        stages,
+    run(
         [&](int st, int b) {
             uint8_t* d = lds + b + 1024 * wave;
             gt_copy(q + st * GT_KI8, qo, d);
@@ -268,6 +323,12 @@ __device__ __forceinline__ void gt_stream_i8(i32x4 (&acc)[2][2], const int8_t* w
                         acc[nb][tb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[nb], qf[tb], acc[nb][tb], 0, 0, 0);
             }
         });
+}
+__device__ __forceinline__ void gt_stream_i8(i32x4 (&acc)[2][2], const int8_t* w, int64_t ldw, const int8_t* q, int64_t ldq, int t,
+                                             int stages, uint8_t* lds)
+{
+    using T = GtStream;
+    gt_stream_i8(acc, w, 0, ldw, q, ldq, t, lds, [&](auto&& copy, auto&& multiply) { gt_stages<T::RING, T::STAGE, 5>(stages, copy, multiply); });
 }
 
 // 33 to 160 tokens x 128 outputs, 512 lanes: a stream of weights still, all tokens beside them, two stages in flight (fused prolog of 40

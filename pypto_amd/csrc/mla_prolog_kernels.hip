@@ -23,6 +23,7 @@
 //   mla_qb_kernel    int8 MFMA GEMM q_norm @ w_uq_qr, 128 outputs x 32 tokens per workgroup, weights streamed to LDS
 //                    (gemm_tile.h); dequantisation and the query's rotary embedding on the tile
 //   mla_wuk_kernel   per (head, 128 outputs): q_b[:, head, :128] @ w_uk[head]; for many tokens or heads per head (mla_wuk_wide_kernel)
+// Up to 32 tokens and 170 heads the last two are one kernel, mla_head_kernel: a head's dims and its absorbed product in one workgroup.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -214,14 +215,14 @@ static int xa_wide_rows(int64_t t, int64_t h, int64_t r)
 
 // Four blocks of 64 outputs of q_b, TOK tokens each, from LDS rows of QBS_ROW bytes (padded against bank conflicts) to memory in
 // 16-byte pieces: a block is half of a head's 128 first dims, or its rotary dims, rotated on the way.  PER lanes to a block (two waves: two
-// blocks in 256 lanes).
+// blocks in 256 lanes); step: from one of them to the next.
 constexpr int QBS_ROW = 64 * 2 + 16;
 template <int TOK, int PER = 128>
-__device__ __forceinline__ void qb_store_blocks(const MlaPrologArgs& a, const uint8_t* lds, int block0, int tok0)
+__device__ __forceinline__ void qb_store_blocks(const MlaPrologArgs& a, const uint8_t* lds, int block0, int tok0, int step = 1)
 {
 #pragma clang fp contract(off)
     const int tid = threadIdx.x, blocks = a.n * MQH / 64;
-    const int bl = tid / PER, block = block0 + bl, head = block / 3;
+    const int bl = tid / PER, block = block0 + step * bl, head = block / 3;
     if (block >= blocks) return;
     const uint8_t* tile = lds + bl * TOK * QBS_ROW;
     if (block % 3 < 2) { // 8 pieces of 8 dims
@@ -271,21 +272,20 @@ __device__ __forceinline__ void qb_store_blocks(const MlaPrologArgs& a, const ui
 // weights.  A workgroup owns 128 outputs (192 of them at model sizes) and keeps three stages of 64 rows x 256 bytes in flight
 // straight to LDS (call of 24 tokens 30.8 us, with six 31.3; out of HBM 35.9 and 36.3).  Splits of 1024 rows loaded in one go through registers, their fp32 partial sums through memory and a kernel
 // behind them took 24.4 + 4.8 us at 24 tokens.  The sums: chains of 128 rows added up in order, then splits of 1024 rows.
-// grid (n * 192 / 128 rounded up), 256 lanes: wave w owns outputs [32 w, +32).
-__global__ __launch_bounds__(256) void mla_qb16_kernel(MlaPrologArgs a)
+// 256 lanes: wave w owns outputs [32 w, +32); the two blocks of 64 begin at w0 and w1.  run(copy, multiply) goes through the stages.
+// Register e of sum: output 32 w + 8 (e / 4) + 4 hl + e % 4, token lane % 32.
+struct Qb16Stream { // a stage: token rows | [2] weight rows of 128 bytes
+    static constexpr int XB = MTOK * 128, STAGE = XB + 2 * 64 * 128, RING = 4, LDS = RING * STAGE;
+};
+template <class Run>
+__device__ __forceinline__ void qb16_stream(f32x16& sum, const MlaPrologArgs& a, const uint16_t* w0, const uint16_t* w1, uint8_t* lds, Run&& run)
 {
 #pragma clang fp contract(off)
-    constexpr int XB = MTOK * 128, STAGE = XB + 2 * 64 * 128, RING = 4; // a stage: token rows | [2] weight rows of 128 bytes
-    static_assert(2 * MTOK * QBS_ROW <= RING * STAGE, "the output tile takes the stages' place");
-    __shared__ __align__(16) uint8_t lds[RING * STAGE];
+    constexpr int XB = Qb16Stream::XB;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, hl = lane >> 5, jj = lane & 15, mh = (lane >> 4) & 1;
-    const int nq = a.n * MQH, block0 = 2 * blockIdx.x;
+    const int nq = a.n * MQH;
     const uint16_t* x = reinterpret_cast<const uint16_t*>(a.q_norm);
-    const uint16_t* src[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) // (a block past the last one: that one again, dropped below)
-        src[i] = static_cast<const uint16_t*>(a.w_uq_qr) + min(block0 + i, nq / 64 - 1) * 64;
     // copies of a wave (layout and exchange of the pieces: gemm_tile.h): token rows 8 w + lane / 8, weight rows 32 i + that
     const int row = 8 * wave + (lane >> 3), pos = lane & 7;
     const uint32_t xo = (uint32_t)(min(row, a.t - 1) * a.r * 2 + 16 * (pos ^ ((row >> 1) & 7)));
@@ -296,17 +296,16 @@ __global__ __launch_bounds__(256) void mla_qb16_kernel(MlaPrologArgs a)
     const int xf = (l32 >> 1) & 7;
     const uint8_t* wrow = lds + XB + (wave >> 1) * 8192 + (8 * hl + (jj >> 2)) * 128 + 8 * (jj & 1);
     const int wpos = 16 * ((4 * (wave & 1) + 2 * mh + ((jj >> 1) & 1)) ^ ((jj >> 1) & 4));
-    f32x16 acc, part, sum;
+    f32x16 acc, part;
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = part[e] = sum[e] = 0.f;
     const int stages = a.r / 64;
-    gt_stages<RING, STAGE, 5>(
-        stages,
+    run(
         [&](int st, int b) {
             uint8_t* d = lds + b + 1024 * wave;
             gt_copy(x + st * 64, xo, d);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) gt_copy(src[i >> 1] + (int64_t)st * 64 * nq, wo[i & 1], d + XB + 4096 * i);
+            for (int i = 0; i < 4; ++i) gt_copy((i < 2 ? w0 : w1) + (int64_t)st * 64 * nq, wo[i & 1], d + XB + 4096 * i);
         },
         [&](int st, int b) {
 #pragma unroll
@@ -327,13 +326,28 @@ __global__ __launch_bounds__(256) void mla_qb16_kernel(MlaPrologArgs a)
                 for (int e = 0; e < 16; ++e) sum[e] += part[e], part[e] = 0.f;
             }
         });
-    // register e: output 32 w + 8 (e / 4) + 4 hl + e % 4, token lane % 32
+}
+// the sums as bf16 rows [2 blocks][32 tokens] of QBS_ROW bytes
+__device__ __forceinline__ void qb16_tile(const f32x16& sum, uint8_t* tile)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, hl = lane >> 5;
 #pragma unroll
     for (int e4 = 0; e4 < 4; ++e4)
-        *reinterpret_cast<u32x2*>(lds + ((wave >> 1) * MTOK + l32) * QBS_ROW + (32 * (wave & 1) + 8 * e4 + 4 * hl) * 2) =
+        *reinterpret_cast<u32x2*>(tile + ((wave >> 1) * MTOK + l32) * QBS_ROW + (32 * (wave & 1) + 8 * e4 + 4 * hl) * 2) =
             u32x2{pack_bf16x2(sum[4 * e4], sum[4 * e4 + 1]), pack_bf16x2(sum[4 * e4 + 2], sum[4 * e4 + 3])};
+}
+// grid (n * 192 / 128), 256 lanes
+__global__ __launch_bounds__(256) void mla_qb16_kernel(MlaPrologArgs a)
+{
+    using S = Qb16Stream;
+    static_assert(2 * MTOK * QBS_ROW <= S::LDS, "the output tile takes the stages' place");
+    __shared__ __align__(16) uint8_t lds[S::LDS];
+    const uint16_t* w = static_cast<const uint16_t*>(a.w_uq_qr) + 128 * blockIdx.x;
+    f32x16 sum;
+    qb16_stream(sum, a, w, w + 64, lds, [&](auto&& copy, auto&& multiply) { gt_stages<S::RING, S::STAGE, 5>(a.r / 64, copy, multiply); });
+    qb16_tile(sum, lds);
     __syncthreads();
-    qb_store_blocks<MTOK>(a, lds, block0, 0);
+    qb_store_blocks<MTOK>(a, lds, 2 * blockIdx.x, 0);
 }
 
 // The bf16 form at more tokens: 128 tokens x 256 outputs per workgroup over the whole contraction (gemm_tile.h), the epilogue
@@ -780,11 +794,11 @@ __global__ __launch_bounds__(256) void fused_norm_wide_kernel(MlaPrologArgs m, P
 
 // The head of a weight slice, read and dropped: the first `rows` rows of 16 `pieces` bytes (rows a multiple of what 256 lanes
 // cover in one go, up to 24 times that), so that the workgroup of the next launch that streams the slice finds them in
-// its XCD's L2.
-__device__ __forceinline__ void touch_rows(const uint8_t* base, int64_t stride, int rows, int pieces)
+// its XCD's L2.  The second half of a row's pieces lies `gap` bytes further on.
+__device__ __forceinline__ void touch_rows(const uint8_t* base, int64_t stride, int rows, int pieces, int gap)
 {
-    const int per = 256 / pieces, row = threadIdx.x / pieces, n = rows / per;
-    const uint8_t* p = base + row * stride + (threadIdx.x % pieces) * 16;
+    const int per = 256 / pieces, row = threadIdx.x / pieces, n = rows / per, piece = threadIdx.x % pieces;
+    const uint8_t* p = base + row * stride + piece * 16 + (2 * piece >= pieces ? gap : 0);
     u32x4 v[24];
 #pragma unroll
     for (int i = 0; i < 24; ++i)
@@ -796,35 +810,165 @@ __device__ __forceinline__ void touch_rows(const uint8_t* base, int64_t stride, 
 
 // ------------------------------------------------------------------------------------------------ q_norm @ w_uq_qr
 // Up to 32 tokens: 128 outputs per workgroup of 256 lanes behind the streamed product (gemm_tile.h); dequantisation and the
-// query's rotary embedding on the tile.  The int32 sums are exact.
-__device__ __forceinline__ void mla_qb_body(const MlaPrologArgs& a, int tile, uint8_t* lds)
-{
-#pragma clang fp contract(off)
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4, col0 = 128 * tile;
+// query's rotary embedding on the tile.  The int32 sums are exact.  The outputs are two times 64, `gap` columns apart.
+struct QbScales {
     float qs[2];
     f32x4 ws[2];
+    __device__ __forceinline__ void load(const MlaPrologArgs& a, int col0, int gap)
+    {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb) qs[tb] = a.q_norm_scale[min(16 * tb + l16, a.t - 1)];
+        for (int tb = 0; tb < 2; ++tb) qs[tb] = a.q_norm_scale[min(16 * tb + l16, a.t - 1)];
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + col0 + 32 * wave + 16 * nb + 4 * g);
-    i32x4 acc[2][2];
+        for (int nb = 0; nb < 2; ++nb)
+            ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + col0 + (wave >> 1) * gap + 32 * wave + 16 * nb + 4 * g);
+    }
+    // bf16 rows [2 blocks][32 tokens] of QBS_ROW bytes
+    __device__ __forceinline__ void tile(const i32x4 (&acc)[2][2], uint8_t* to) const
+    {
+#pragma clang fp contract(off)
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
+        for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
-    gt_stream_i8(acc, static_cast<const int8_t*>(a.w_uq_qr) + col0, (int64_t)a.n * MQH, a.q_norm, a.r, a.t, a.r / GT_KI8, lds);
+            for (int nb = 0; nb < 2; ++nb) {
+                float v[4];
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs[tb]) * ws[nb][e];
-            *reinterpret_cast<u32x2*>(lds + ((wave >> 1) * MTOK + 16 * tb + l16) * QBS_ROW + (32 * (wave & 1) + 16 * nb + 4 * g) * 2) =
-                u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-        }
+                for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs[tb]) * ws[nb][e];
+                *reinterpret_cast<u32x2*>(to + ((wave >> 1) * MTOK + 16 * tb + l16) * QBS_ROW + (32 * (wave & 1) + 16 * nb + 4 * g) * 2) =
+                    u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+            }
+    }
+};
+__device__ __forceinline__ void mla_qb_body(const MlaPrologArgs& a, int tile, uint8_t* lds)
+{
+    QbScales scales;
+    scales.load(a, 128 * tile, 0);
+    i32x4 acc[2][2] = {};
+    gt_stream_i8(acc, static_cast<const int8_t*>(a.w_uq_qr) + 128 * tile, (int64_t)a.n * MQH, a.q_norm, a.r, a.t, a.r / GT_KI8, lds);
+    scales.tile(acc, lds);
     __syncthreads();
     qb_store_blocks<MTOK>(a, lds, 2 * tile, 0);
+}
+
+// Up to 32 tokens and one workgroup to a CU (head_units): a head's 128 first dims of q_b in one workgroup, which goes on to
+// the absorbed product with the head's w_uk, whose 128 KB follow the other weights through the same stages; the rotary dims of two heads
+// in another.  The three workgroups of two heads, which share cache lines of the int8 weights, go to one XCD.
+// A kernel of its own for the absorbed product, 512 workgroups behind a launch and a round trip of q_b through memory, took 4.2 to 5 us.
+constexpr int WUK_CHUNKS = MC / 64; // stages of w_uk: 128 rows x 64 columns
+struct HeadUnit {
+    int head, col0, gap; // (the first) head, first output, from the first 64 outputs to the others
+    bool nope;
+};
+__device__ __forceinline__ HeadUnit head_unit(const MlaPrologArgs& a, int id)
+{
+    const bool even = a.n % 16 == 0; // (whole rounds of the XCDs)
+    const int pair = even ? id / 24 * 8 + id % 8 : id / 3, k = even ? id / 8 % 3 : id % 3;
+    return k < 2 ? HeadUnit{2 * pair + k, (2 * pair + k) * MQH, 0, true} : HeadUnit{2 * pair, 2 * pair * MQH + MNOPE, MQH - 64, false};
+}
+struct Absorbed { // wave w: columns 32 (w % 2) of the chunks 2 i + w / 2
+    static constexpr int TILE = 2 * MTOK * QBS_ROW, OROW = MC * 2 + 16; // bytes of q_b's tile, of an LDS row of the outputs
+    f32x16 acc[WUK_CHUNKS / 2];
+
+    // five copies of a wave, as many as a stage of the other weights (the first is not used)
+    static __device__ __forceinline__ void copy(const MlaPrologArgs& a, int head, int c, uint8_t* slot)
+    {
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int row = 8 * wave + (lane >> 3), pos = lane & 7;
+        const uint16_t* w = a.w_uk + (int64_t)head * MNOPE * MC + 64 * c;
+        const uint32_t at = (uint32_t)(row * MC * 2 + 16 * (pos ^ ((row << 1) & 4)));
+        uint8_t* d = slot + 1024 * wave;
+        gt_copy(w, at, d);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gt_copy(w + 32 * i * MC, at, d + MTOK * 128 + 4096 * i);
+    }
+    // (the operands and the order of mla_wuk_kernel)
+    template <int C>
+    __device__ __forceinline__ void multiply(const uint8_t* tile, const uint8_t* slot)
+    {
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        if ((wave >> 1) != (C & 1)) return;
+        const int l32 = lane & 31, hl = lane >> 5, jj = lane & 15, mh = (lane >> 4) & 1;
+        const uint8_t* wrow = slot + MTOK * 128 + (8 * hl + (jj >> 2)) * 128 + 8 * (jj & 1) +
+                              16 * ((4 * (wave & 1) + 2 * mh + ((jj >> 1) & 1)) ^ ((jj >> 1) & 4));
+        f32x16& o = acc[C / 2];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[e] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < MNOPE / 16; ++ks) {
+            const s16x4 lo = lds_read_tr(wrow + 2048 * ks), hi = lds_read_tr(wrow + 2048 * ks + 512);
+            const bf16x8 wv = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            const bf16x8 xv = *reinterpret_cast<const bf16x8*>(tile + ((ks >> 2) * MTOK + l32) * QBS_ROW + 32 * (ks & 3) + 16 * hl);
+            o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv, xv, o, 0, 0, 0);
+        }
+    }
+    // through LDS, a token's 512 outputs to a wavefront's store
+    __device__ __forceinline__ void store(const MlaPrologArgs& a, int head, uint8_t* lds) const
+    {
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l32 = lane & 31, hl = lane >> 5;
+#pragma unroll
+        for (int i = 0; i < WUK_CHUNKS / 2; ++i)
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4)
+                *reinterpret_cast<u32x2*>(lds + l32 * OROW + (64 * (2 * i + (wave >> 1)) + 32 * (wave & 1) + 8 * e4 + 4 * hl) * 2) =
+                    u32x2{pack_bf16x2(acc[i][4 * e4], acc[i][4 * e4 + 1]), pack_bf16x2(acc[i][4 * e4 + 2], acc[i][4 * e4 + 3])};
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < MTOK / 4; ++i) {
+            const int tok = 4 * i + wave;
+            if (tok < a.t) // (wave-uniform)
+                *reinterpret_cast<u32x4*>(a.q_nope + ((int64_t)tok * a.n + head) * MC + 8 * lane) = *reinterpret_cast<const u32x4*>(lds + tok * OROW + 16 * lane);
+        }
+    }
+};
+constexpr int HEAD_LDS = GtStream::LDS + Absorbed::TILE; // the stages, later the outputs | q_b's tile
+static_assert(Qb16Stream::STAGE == GtStream::STAGE && Qb16Stream::RING == GtStream::RING && Qb16Stream::XB == GtStream::QBYTES &&
+                  GtStream::QBYTES == MTOK * 128 && MTOK * Absorbed::OROW <= GtStream::LDS, "one layout");
+// lds: HEAD_LDS bytes
+template <bool QUANT>
+__device__ __forceinline__ void mla_head_body(const MlaPrologArgs& a, int id, uint8_t* lds)
+{
+    using S = GtStream;
+    const HeadUnit u = head_unit(a, id);
+    uint8_t* tile = lds + S::LDS;
+    QbScales scales;
+    i32x4 acc[2][2] = {};
+    f32x16 sum;
+    if constexpr (QUANT) scales.load(a, u.col0, u.gap);
+    const int stages = a.r / (QUANT ? GT_KI8 : 64);
+    auto product = [&](auto&& run) {
+        if constexpr (QUANT)
+            gt_stream_i8(acc, static_cast<const int8_t*>(a.w_uq_qr) + u.col0, u.gap, (int64_t)a.n * MQH, a.q_norm, a.r, a.t, lds, run);
+        else
+            qb16_stream(sum, a, static_cast<const uint16_t*>(a.w_uq_qr) + u.col0, static_cast<const uint16_t*>(a.w_uq_qr) + u.col0 + 64 + u.gap, lds, run);
+    };
+    auto to_tile = [&]() {
+        if constexpr (QUANT)
+            scales.tile(acc, tile);
+        else
+            qb16_tile(sum, tile);
+    };
+    if (u.nope) { // uniform over the workgroup
+        Absorbed o;
+        product([&](auto&& copy, auto&& multiply) {
+            gt_stages_more<S::RING, S::STAGE, 5, WUK_CHUNKS>(
+                stages, copy, multiply, [&](int c, int b) { Absorbed::copy(a, u.head, c, lds + b); }, to_tile,
+                [&](auto ic, int b) { o.template multiply<decltype(ic)::value>(tile, lds + b); });
+        });
+        o.store(a, u.head, lds);
+    } else {
+        product([&](auto&& copy, auto&& multiply) { gt_stages<S::RING, S::STAGE, 5>(stages, copy, multiply); });
+        to_tile();
+        __syncthreads();
+        qb_store_blocks<MTOK>(a, tile, 3 * u.head + 2, 0, 3);
+    }
+}
+// grid (n * 192 / 128), 256 lanes
+template <bool QUANT>
+__global__ __launch_bounds__(256) void mla_head_kernel(MlaPrologArgs a)
+{
+    __shared__ __align__(16) uint8_t lds[HEAD_LDS];
+    mla_head_body<QUANT>(a, blockIdx.x, lds);
 }
 
 // Decode batches: while the norms' few workgroups go through their chains, the rest of the chip has nothing to do, and the
@@ -844,18 +988,19 @@ inline int touch_bytes(int slices, bool fused)
     return std::min(TOUCH_BYTES, xcd / ((slices + 7) / 8));
 }
 
-__device__ __forceinline__ void mla_touch(const MlaPrologArgs& a, int tile, int bytes)
+__device__ __forceinline__ void mla_touch(const MlaPrologArgs& a, int tile, int bytes, bool heads)
 {
-    const int64_t stride = (int64_t)a.n * MQH * (a.quant ? 1 : 2);
-    const int pieces = a.quant ? 8 : 16; // 128 outputs (the half tile that the bf16 form may end with is not asked for)
+    const int value = a.quant ? 1 : 2, pieces = 8 * value; // 128 outputs
+    const int64_t stride = (int64_t)a.n * MQH * value;
     const int rows = min(a.r, bytes / (16 * pieces)) & ~31;
-    touch_rows(static_cast<const uint8_t*>(a.w_uq_qr) + (int64_t)tile * 16 * pieces, stride, rows, pieces);
+    const HeadUnit u = heads ? head_unit(a, tile) : HeadUnit{0, 128 * tile, 0, true};
+    touch_rows(static_cast<const uint8_t*>(a.w_uq_qr) + (int64_t)u.col0 * value, stride, rows, pieces, u.gap * value);
 }
 
 // grid (2 x tokens: query, key | TOUCH: touching workgroups from `first` on), 256 lanes.  Without them (above 32 tokens) 40 registers
 // instead of 98, all of a token's chain that a SIMD can hold.
 template <int S, bool TOUCH>
-__global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a, int first, int touch)
+__global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a, int first, int touch, bool heads)
 {
     const int id = blockIdx.x;
     if (id < a.t)
@@ -863,7 +1008,7 @@ __global__ __launch_bounds__(256) void mla_norm_kernel(MlaPrologArgs a, int firs
     else if (id < 2 * a.t)
         mla_norm_key_body<S>(a, id - a.t);
     else if constexpr (TOUCH) {
-        if (id >= first) mla_touch(a, id - first, touch);
+        if (id >= first) mla_touch(a, id - first, touch, heads);
     }
 }
 
@@ -976,7 +1121,7 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb_batch_kernel(MlaPrologArgs
 // grid (3 x tokens: the MLA norms, the indexer's key path and weights (128 lanes) | TOUCH: touching workgroups from `first` on),
 // 256 lanes
 template <int S, bool TOUCH>
-__global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, PrologArgs p, int first, int touch)
+__global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, PrologArgs p, int first, int touch, bool heads)
 {
     const int id = blockIdx.x;
     if (id < m.t)
@@ -989,9 +1134,9 @@ __global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, Prolog
     } else if (TOUCH && id >= first) {
         const int tile = id - first, nqb = m.n * MQH / 128;
         if (tile < nqb)
-            mla_touch(m, tile, touch);
+            mla_touch(m, tile, touch, heads);
         else
-            touch_rows(reinterpret_cast<const uint8_t*>(p.w_qb) + (int64_t)(tile - nqb) * PD, (int64_t)p.n * PD, min(p.r, touch / PD) & ~31, 8);
+            touch_rows(reinterpret_cast<const uint8_t*>(p.w_qb) + (int64_t)(tile - nqb) * PD, (int64_t)p.n * PD, min(p.r, touch / PD) & ~31, 8, 0);
     }
 }
 
@@ -1003,6 +1148,17 @@ __global__ __launch_bounds__(256) void fused_qb_kernel(MlaPrologArgs m, PrologAr
     const int nqb = m.n * MQH / 128;
     if ((int)blockIdx.x < nqb)
         mla_qb_body(m, blockIdx.x, lds);
+    else
+        prolog_q_stream_body(p, blockIdx.x - nqb, lds);
+}
+
+// The same with a head's absorbed product behind it (mla_head_body).
+__global__ __launch_bounds__(256) void fused_head_kernel(MlaPrologArgs m, PrologArgs p)
+{
+    __shared__ __align__(16) uint8_t lds[PROLOG_STREAM_LDS > HEAD_LDS ? PROLOG_STREAM_LDS : HEAD_LDS];
+    const int nqb = m.n * MQH / 128;
+    if ((int)blockIdx.x < nqb)
+        mla_head_body<true>(m, blockIdx.x, lds);
     else
         prolog_q_stream_body(p, blockIdx.x - nqb, lds);
 }
@@ -1298,6 +1454,15 @@ static bool qb_batch(const MlaPrologArgs& a, const PrologArgs* p)
     return p ? a.t <= 128 || (slices > 172 && slices <= 256) : slices <= 256;
 }
 
+// Up to 32 tokens the absorbed product behind the head's query product, while that is a workgroup to a CU (us a call, two kernels / one,
+// warm weights: fused, 1 token 27.1 / 24.7, 8: 28.5 / 26.0, 32: 30.1 / 27.5, of 16 heads 23.1 / 21.6; bf16 form, 24 tokens 29.8 / 27.6, out
+// of HBM 36.0 / 33.9, of 16 heads 23.3 / 22.4; int8 form, 8 tokens 23.8 / 22.3, out of HBM 28.4 / 28.2).  The int8 form of few heads has short
+// streams behind each other: of 16 19.8 / 20.0, 32: 20.0 / 20.5, 64: 20.7 / 20.7.
+static bool head_units(const MlaPrologArgs& a, const PrologArgs* p)
+{
+    return a.t < BIG_T && a.n * MQH / 128 + (p ? p->n : 0) <= 256 && (p || !a.quant || a.n > 64);
+}
+
 // p == nullptr: the MLA prolog on its own; otherwise the fused operator (m and p bound by fused_prolog_bind)
 static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hipStream_t stream)
 {
@@ -1305,6 +1470,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
     const int ttiles = (a.t + MTOK - 1) / MTOK;
     hipError_t e;
     const bool big = a.t >= BIG_T; // the kernels that own an output tile
+    const bool heads = head_units(a, p);
     {
         ScopedKernelTimer tm(KID_MLA_XA, stream);
         if (a.t <= BIG_T2) {
@@ -1332,9 +1498,9 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
             constexpr int S = decltype(splits)::value;
             constexpr bool TOUCH = decltype(touch)::value;
             if (p)
-                hipLaunchKernelGGL((fused_norm_kernel<S, TOUCH>), dim3(grid), dim3(256), 0, stream, a, *p, first, bytes);
+                hipLaunchKernelGGL((fused_norm_kernel<S, TOUCH>), dim3(grid), dim3(256), 0, stream, a, *p, first, bytes, heads);
             else
-                hipLaunchKernelGGL((mla_norm_kernel<S, TOUCH>), dim3(grid), dim3(256), 0, stream, a, first, bytes);
+                hipLaunchKernelGGL((mla_norm_kernel<S, TOUCH>), dim3(grid), dim3(256), 0, stream, a, first, bytes, heads);
         };
         auto launch_with = [&](auto touch) {
             if (in_flight == 2)
@@ -1367,10 +1533,15 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
     if ((e = hipGetLastError()) != hipSuccess) return e;
     {
         ScopedKernelTimer tm(KID_MLA_QB, stream);
-        if (!a.quant && big) {
+        if (heads) {
+            if (p)
+                hipLaunchKernelGGL(fused_head_kernel, dim3(a.n * MQH / 128 + p->n), dim3(256), 0, stream, a, *p);
+            else
+                hipLaunchKernelGGL((a.quant ? mla_head_kernel<true> : mla_head_kernel<false>), dim3(a.n * MQH / 128), dim3(256), 0, stream, a);
+        } else if (!a.quant && big) {
             hipLaunchKernelGGL(mla_qb16_wide_kernel, dim3((a.n * MQH + 255) / 256, (a.t + 127) / 128), dim3(GT_LANES), 0, stream, a);
         } else if (!a.quant) {
-            hipLaunchKernelGGL(mla_qb16_kernel, dim3((a.n * MQH + 127) / 128), dim3(256), 0, stream, a);
+            hipLaunchKernelGGL(mla_qb16_kernel, dim3(a.n * MQH / 128), dim3(256), 0, stream, a);
         } else if (big) {
             if (qb_batch(a, p)) {
                 token_blocks(a.t, [&](auto tt) {
@@ -1400,7 +1571,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
             hipLaunchKernelGGL(mla_qb_kernel, dim3(a.n * MQH / 128), dim3(256), 0, stream, a);
         }
     }
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = hipGetLastError()) != hipSuccess || heads) return e;
     {
         ScopedKernelTimer tm(KID_MLA_WUK, stream);
         const int wtiles = (a.t + WW_TOK - 1) / WW_TOK;

@@ -212,6 +212,15 @@ def test_x_product_in_splits_of_whole_stages(cuda, t, n, h):
     check_against_oracle(mla_case, idx_case, fused)
 
 
+@pytest.mark.parametrize("t,n,r", [(1, 2, 128), (32, 16, 384), (31, 66, 256), (5, 128, 1536), (9, 130, 128)])
+def test_absorbed_product_behind_the_query_product(cuda, t, n, r):
+    # beside the index heads', to 128 heads (130: kernels of their own).  The separate call of up to 64 heads is two kernels: the same bits
+    mla_case, idx_case = op.make_fused_case(t, 1, 300, seed=150 + n, n_idx=64, h=512, q_lora_rank=r, n=n)
+    fused = run_fused(mla_case, idx_case, cuda)
+    same_as_separate(fused, run_separate(mla_case, idx_case, cuda), idx_case)
+    check_against_oracle(mla_case, idx_case, fused)
+
+
 @pytest.mark.parametrize("t,n_idx,r,h", [(257, 128, 1664, 256), (258, 64, 1536, 2304), (259, 64, 384, 1280), (1284, 128, 128, 512)])
 def test_norms_by_wavefronts(cuda, t, n_idx, r, h):
     # above 256 tokens and with at most four splits of x's product, four tokens to a workgroup: one, two and three of them and all in the

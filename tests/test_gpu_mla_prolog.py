@@ -256,6 +256,20 @@ def test_decode_batches_of_many_heads(cuda, n, quant_b):
     (check if quant_b else check_bf16_form)(case, run(case, cuda))
 
 
+@pytest.mark.parametrize("t,n,r,quant_b", [(1, 66, 640, True), (32, 96, 384, True), (31, 170, 128, True), (7, 64, 256, True), (32, 2, 256, False),
+                                           (31, 16, 1280, False), (1, 170, 256, False)])
+def test_absorbed_product_behind_the_query_product(cuda, t, n, r, quant_b):
+    # a head's 128 first dims and its absorbed product to a workgroup, the rotary dims of two heads to another: pairs of heads in whole
+    # rounds of the XCDs (16, 96) and not, the most heads of one workgroup to a CU; int8 of 64 heads is the two kernels behind each other.
+    # One stage of the query product, as many as are ahead, and more
+    case = op.make_case(t, 1, 300, seed=140 + n, h=512, q_lora_rank=r, n=n, quant_b=quant_b)
+    got = run(case, cuda)
+    if quant_b:
+        check(case, got)
+    else:
+        check_bf16_form(case, got, outliers=1e-4)
+
+
 @pytest.mark.parametrize("quant_b", [True, False])
 def test_a_tokens_bits_do_not_depend_on_the_batch(cuda, quant_b):
     """Up to 32 tokens and from 33 on other kernels form the products; up to 256 tokens their fp32 sums are the same (chains of 128
