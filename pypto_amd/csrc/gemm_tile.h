@@ -194,11 +194,11 @@ __device__ __forceinline__ int gt_wave_across()
 }
 
 // acc[nb][tb] += w[k, col0 + ..]^T . q[token, k], int8, by wave 4 wr + wc.  w0, w1: first contraction row of the two halves' columns, ldw bytes a
-// row; q: [t, ldq], column of the first contraction row.  Register e of acc[nb][tb]: output 64 wc + 16 nb + 4 g + e, token
+// row, the second 64 of either half `gap` columns further on; q: [t, ldq], column of the first contraction row.  Register e of acc[nb][tb]: output 64 wc + 16 nb + 4 g + e, token
 // 16 TB wr + 16 tb + l16.
 template <int TB>
 __device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t* w0, const int8_t* w1, int64_t ldw, const int8_t* q,
-                                              int64_t ldq, int tok0, int t, int stages, uint8_t* lds, int wave)
+                                              int64_t ldq, int tok0, int t, int stages, uint8_t* lds, int wave, int gap = 0)
 {
     using T = GtTile<TB>;
     const int lane = threadIdx.x & 63;
@@ -216,7 +216,10 @@ __device__ __forceinline__ void gt_product_i8(i32x4 (&acc)[4][TB], const int8_t*
         qo[i] = (uint32_t)(min(qrow, t - 1 - tok0) * (int)ldq + 16 * (pos ^ ((qrow >> 1) & 7)));
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i) wo[i] = (uint32_t)((row + 64 * i) * (int)ldw + 16 * (pos ^ (((row >> 1) & 3) | ((row >> 2) & 4))));
+    for (int i = 0; i < 2; ++i) {
+        const int piece = pos ^ (((row >> 1) & 3) | ((row >> 2) & 4));
+        wo[i] = (uint32_t)((row + 64 * i) * (int)ldw + 16 * piece + (piece >= 4 ? gap : 0));
+    }
     auto copy_q = [&](int i, int st, int b) { gt_copy(qb + st * GT_KI8, qo[i], lds + b + qd[i]); };
     auto copy_w = [&](int i, int st, int b) {
         gt_copy((i < 2 ? w0 : w1) + (int64_t)st * GT_KI8 * ldw, wo[i & 1], lds + T::WOFF + b + 8192 * i + 1024 * wave);
@@ -334,7 +337,7 @@ __device__ __forceinline__ void gt_stream_i8(i32x4 (&acc)[2][2], const int8_t* w
 // 33 to 160 tokens x 128 outputs, 512 lanes: a stream of weights still, all tokens beside them, two stages in flight (fused prolog of 40
 // tokens, weights out of HBM, 38.1 us; with three 38.6, with five 39.2).  Wave (wr, wc) owns tokens [16 TT wr, +16 TT) x two blocks of
 // 16 outputs 32 apart, gt_batch_block(wc, nb): what a rotary embedding pairs is in one lane.  Register e of acc[nb][tb]: output
-// 16 gt_batch_block + 4 g + e, token 16 TT wr + 16 tb + l16.
+// 16 gt_batch_block + 4 g + e, token 16 TT wr + 16 tb + l16.  The second 64 outputs lie `gap` columns further on.
 template <int TT>
 struct GtBatch {
     static constexpr int TOK = 32 * TT, QBYTES = TOK * 128, STAGE = QBYTES + 128 * 128, FIT = 160 * 1024 / STAGE, RING = FIT < 3 ? FIT : 3, LDS = RING * STAGE;
@@ -342,7 +345,7 @@ struct GtBatch {
 __device__ __forceinline__ int gt_batch_block(int wc, int nb) { return (wc & 1) + 2 * nb + 4 * (wc >> 1); }
 template <int TT>
 __device__ __forceinline__ void gt_batch_i8(i32x4 (&acc)[2][TT], const int8_t* w, int64_t ldw, const int8_t* q, int64_t ldq, int t, int stages,
-                                            uint8_t* lds)
+                                            uint8_t* lds, int gap = 0)
 {
     using T = GtBatch<TT>;
     const int lane = threadIdx.x & 63, wave = gt_wave();
@@ -360,7 +363,8 @@ __device__ __forceinline__ void gt_batch_i8(i32x4 (&acc)[2][TT], const int8_t* w
         qd[i] = 1024 * c;
         qo[i] = (uint32_t)(min(qrow, t - 1) * (int)ldq + 16 * (pos ^ ((qrow >> 1) & 7)));
     }
-    wo = (uint32_t)(lane >> 3) * (uint32_t)ldw + 16 * (pos ^ (((row >> 1) & 3) | ((row >> 2) & 4))); // (the same 64 rows on)
+    const int piece = pos ^ (((row >> 1) & 3) | ((row >> 2) & 4)); // (the same 64 rows on)
+    wo = (uint32_t)(lane >> 3) * (uint32_t)ldw + 16 * piece + (piece >= 4 ? gap : 0);
     const uint8_t* qr = lds + (16 * TT * wr + l16) * 128;
     const int qpos = 16 * (g ^ ((l16 >> 1) & 7));
     const uint8_t* wrow = lds + T::QBYTES + (16 * g + (l16 >> 1)) * 128 + 8 * (l16 & 1);

@@ -23,7 +23,7 @@
 //   mla_qb_kernel    int8 MFMA GEMM q_norm @ w_uq_qr, 128 outputs x 32 tokens per workgroup, weights streamed to LDS
 //                    (gemm_tile.h); dequantisation and the query's rotary embedding on the tile
 //   mla_wuk_kernel   per (head, 128 outputs): q_b[:, head, :128] @ w_uk[head]; for many tokens or heads per head (mla_wuk_wide_kernel)
-// Up to 32 tokens and 170 heads the last two are one kernel, mla_head_kernel: a head's dims and its absorbed product in one workgroup.
+// The last two are one kernel wherever that is faster (head_units): a head's dims and its absorbed product in one workgroup.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1019,7 +1019,7 @@ __global__ __launch_bounds__(256) void mla_qb_kernel(MlaPrologArgs a)
     mla_qb_body(a, blockIdx.x, lds);
 }
 
-// For more tokens than mla_qb_batch_kernel takes (qb_batch): 32 TB tokens x 256 outputs per workgroup (gemm_tile.h), the same exact
+// For more tokens than mla_qb_batch_kernel takes (qb_batch), of few heads: 32 TB tokens x 256 outputs per workgroup (gemm_tile.h), the same exact
 // sums and the same operations behind them.  128 x 128 tiles through registers are bound by the operands' way into LDS: MLA prolog
 // of 200 tokens 66.2 us a call against 57.2.
 constexpr int mla_qb_wide_lds(int tb) // the product's stages, or four blocks of the output tile
@@ -1070,28 +1070,190 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_qb_wide_kernel(MlaPrologArgs 
     mla_qb_wide_body<TB>(a, blockIdx.x, blockIdx.y * 32 * TB, lds);
 }
 
+// q_b[:, head, :128] @ w_uk[head] behind a tile of q_b, by the workgroup of 512 lanes that has it in LDS: wave w owns outputs [64 w, +64),
+// whose weights lie in its registers (64 a lane) and come straight from memory: a lane loads 4 neighbouring outputs of 8 contraction rows at a
+// time and turns them by byte permutes into what the matrix instructions want.  Which 4 of the 64 is chosen so that a lane's
+// results for a token are runs of 8 neighbouring outputs; exchanged between tokens 8 apart, a store is 8 whole lines of 128 bytes.
+//
+// As a kernel of its own (mla_wuk_wide_kernel) the product waits for memory: at 1501 tokens 49 MB of q_b out and in again and 197 MB
+// of outputs, 45 us in which the matrix pipes stand still, behind a query product of 91 that writes little.  Here the outputs of some workgroups
+// leave while others multiply, and q_b's first dims stay in LDS.  Call of 1501 tokens, us: two kernels 203.4; one, with halves of lines to
+// a store, 198.5; whole lines 198.9; and streaming stores (they do not push the operands out of the L2) 183.1, halves of lines 183.0 (int8 form
+// alone 161.8 and 170.4); long workgroups sent out first and short ones kept for the end 174.4 (wide_unit).
+struct AbsorbedWide {
+    static constexpr int ROW = MNOPE * 2 + 16; // bytes of a tile's LDS row, padded: 16 rows in 16 different places
+    u32x2 raw[MNOPE / 4];
+    bf16x8 w[4][MNOPE / 32];
+
+    __device__ __forceinline__ void load(const MlaPrologArgs& a, int head)
+    {
+        const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+        const uint16_t* src = a.w_uk + ((int64_t)head * MNOPE + 8 * g) * MC + 64 * gt_wave() + 4 * (2 * (l16 >> 2) + (l16 & 1) + 4 * (l16 & 2));
+#pragma unroll
+        for (int ks = 0; ks < MNOPE / 32; ++ks)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) raw[8 * ks + k] = *reinterpret_cast<const u32x2*>(src + (32 * ks + k) * MC);
+    }
+    __device__ __forceinline__ void turn()
+    {
+#pragma unroll
+        for (int ks = 0; ks < MNOPE / 32; ++ks)
+#pragma unroll
+            for (int cb = 0; cb < 4; ++cb) {
+                u32x4 v;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    v[k] = __builtin_amdgcn_perm(raw[8 * ks + 2 * k + 1][cb >> 1], raw[8 * ks + 2 * k][cb >> 1], cb & 1 ? 0x07060302u : 0x05040100u);
+                w[cb][ks] = __builtin_bit_cast(bf16x8, v);
+            }
+    }
+    // 16 BLOCKS tokens from tok0 on, their rows at `tile`
+    template <int BLOCKS, bool STREAM>
+    __device__ __forceinline__ void multiply(const MlaPrologArgs& a, int head, int tok0, const uint8_t* tile) const
+    {
+        const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+        uint16_t* dst = a.q_nope + ((int64_t)(tok0 + (l16 & 7)) * a.n + head) * MC + 64 * gt_wave() + 8 * g + 4 * (l16 & 8);
+#pragma unroll
+        for (int tb = 0; tb < BLOCKS; ++tb) {
+            f32x4 acc[4];
+#pragma unroll
+            for (int cb = 0; cb < 4; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < MNOPE / 32; ++ks) {
+                const bf16x8 x = *reinterpret_cast<const bf16x8*>(tile + (16 * tb + l16) * ROW + 64 * ks + 16 * g);
+#pragma unroll
+                for (int cb = 0; cb < 4; ++cb) acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[cb][ks], x, acc[cb], 0, 0, 0);
+            }
+            // register e of acc[cb]: output 8 g + 32 (e / 2) + 4 (e % 2) + cb of token l16
+            const bool up = l16 >= 8;
+            u32x4 o[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                o[h] = u32x4{pack_bf16x2(acc[0][2 * h], acc[1][2 * h]), pack_bf16x2(acc[2][2 * h], acc[3][2 * h]),
+                             pack_bf16x2(acc[0][2 * h + 1], acc[1][2 * h + 1]), pack_bf16x2(acc[2][2 * h + 1], acc[3][2 * h + 1])};
+            u32x4 lo, hi;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t v = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(up ? o[0][i] : o[1][i]), 0x128, 0xf, 0xf, true);
+                lo[i] = up ? v : o[0][i];
+                hi[i] = up ? o[1][i] : v;
+            }
+            auto store = [&](u32x4 v, int tok) {
+                if (tok0 + tok + (l16 & 7) >= a.t) return;
+                u32x4* to = reinterpret_cast<u32x4*>(dst + (int64_t)tok * a.n * MC);
+                if constexpr (STREAM)
+                    __builtin_nontemporal_store(v, to);
+                else
+                    *to = v;
+            };
+            store(lo, 16 * tb);
+            store(hi, 16 * tb + 8);
+        }
+    }
+};
+
+constexpr int mla_heads_wide_lds(int tb) // the product's stages, or two heads' tile
+{
+    const int epi = 2 * 32 * tb * AbsorbedWide::ROW, ring = gt_lds_bytes(tb);
+    return epi > ring ? epi : ring;
+}
+// mla_qb_wide_body's product and arithmetic by other units: two heads' first dims and the absorbed products behind them, or (rope) four heads'
+// rotary dims.  What bounds it at 1501 tokens: without the outputs' stores a call takes 172 us, without the absorbed products 159.
+template <int TB>
+__device__ __forceinline__ void mla_heads_wide_body(const MlaPrologArgs& a, int unit, bool rope, int tok0, uint8_t* lds)
+{
+#pragma clang fp contract(off)
+    using T = GtTile<TB>;
+    static_assert(mla_heads_wide_lds(TB) >= mla_qb_wide_lds(TB), "LDS");
+    const int tid = threadIdx.x, lane = tid & 63, wave = gt_wave(), l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
+    i32x4 acc[4][TB]; // [nb][tb]
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
+    const int nq = a.n * MQH;
+    // first columns of the two halves, and of this wave's 64 (a last unit with two heads takes them twice; the second time is dropped)
+    const int c0 = rope ? 4 * unit * MQH + MNOPE : 2 * unit * MQH, c1 = rope ? min(4 * unit + 2, a.n - 2) * MQH + MNOPE : c0 + MQH;
+    const int gap = rope ? MQH - 64 : 0, cw = (wc >> 1 ? c1 : c0) + (wc & 1) * (64 + gap);
+    const int8_t* w = static_cast<const int8_t*>(a.w_uq_qr);
+    gt_product_i8<TB>(acc, w + c0, w + c1, nq, a.q_norm, a.r, tok0, a.t, a.r / GT_KI8, lds, wave, gap);
+    AbsorbedWide ab;
+    if (!rope) ab.load(a, 2 * unit);
+    // register e of acc[nb][tb]: output 64 wc + 16 nb + 4 g + e, token 16 TB wr + 16 tb + l16
+    f32x4 ws[4];
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + cw + 16 * nb + 4 * g);
+    const int row = rope ? QBS_ROW : AbsorbedWide::ROW;
+    uint8_t* to = lds + (rope ? wc * T::TOK * QBS_ROW : (wc >> 1) * T::TOK * AbsorbedWide::ROW + (wc & 1) * 128) + (16 * TB * wr + l16) * row + 8 * g;
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) {
+        const float qs = a.q_norm_scale[min(tok0 + 16 * TB * wr + 16 * tb + l16, a.t - 1)];
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs) * ws[nb][e];
+            *reinterpret_cast<u32x2*>(to + 16 * tb * row + 32 * nb) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        }
+    }
+    __syncthreads();
+    if (rope) {
+        qb_store_blocks<T::TOK>(a, lds, 3 * 4 * unit + 2, tok0, 3);
+        return;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        ab.turn();
+        if (h == 0) ab.load(a, 2 * unit + 1);
+        ab.multiply<2 * TB, true>(a, 2 * unit + h, tok0, lds + h * T::TOK * AbsorbedWide::ROW);
+    }
+}
+// Workgroup id's unit where n1 long units go out among n2 short ones, eight of a kind at a time (an XCD each), `share` / 256 of the
+// groups long ones while they last.  kind -1: none.  Up to two rounds of workgroups long ones first (fused, 612 tokens: evenly mixed 97.1 us, two
+// thirds 95.8, all first 91.4; int8 form 512 tokens 79.4 / 79.4 / 71.8 in tiles of 128); in more, some short ones among them, so that not all CUs
+// store at the same time (1501 tokens 187.6 evenly mixed, 180.2 with 170, 174.4 with 210, 178.9 with 256; 1200: 176.6, 155.6, 158.0, 162.3).
+struct WideUnit {
+    int kind, at;
+};
+__device__ __forceinline__ WideUnit wide_unit(int id, int n1, int n2, int share)
+{
+    const int g1 = (n1 + 7) / 8, g2 = (n2 + 7) / 8, j = id / 8;
+    auto firsts = [&](int k) { return max(k - g2, min(g1, (k * share + 255) / 256)); };
+    const int before = firsts(j);
+    const bool first = firsts(j + 1) > before;
+    const int at = 8 * (first ? before : j - before) + id % 8;
+    return {at >= (first ? n1 : n2) ? -1 : first ? 0 : 1, at};
+}
+
 // 33 to QB_BATCH_T tokens: 128 outputs per workgroup of 512 lanes, all tokens, the weights streamed (gt_batch_i8); the same exact sums
-// and the same operations behind them.  Its 192 workgroups at model sizes keep twice as many CUs at the weights as tiles of 256
+// and the same operations behind them.  ABSORB (head_units): a head's first dims and the absorbed product behind them, or the rotary dims of two heads.  Its 192 workgroups at model sizes keep twice as many CUs at the weights as tiles of 256
 // outputs.  Call of 40 tokens 33.8 -> 30.6 us, 96: 37.9 -> 35.0, 160: 50.6 -> 46.4.
-template <int TT>
+template <int TT, bool ABSORB>
 __device__ __forceinline__ void mla_qb_batch_body(const MlaPrologArgs& a, int tile, uint8_t* lds)
 {
 #pragma clang fp contract(off)
     using T = GtBatch<TT>;
-    static_assert(2 * T::TOK * QBS_ROW <= T::LDS, "the output tile takes the stages' place");
-    const int lane = threadIdx.x & 63, wave = gt_wave(), l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3, col0 = 128 * tile;
+    static_assert(2 * T::TOK * QBS_ROW <= T::LDS && T::TOK * AbsorbedWide::ROW <= T::LDS, "the output tile takes the stages' place");
+    const int lane = threadIdx.x & 63, wave = gt_wave(), l16 = lane & 15, g = lane >> 4, wr = wave >> 2, wc = wave & 3;
+    const bool nope = ABSORB && tile < a.n; // a head's first dims, then two heads' rotary dims
+    const int pair = tile - a.n, gap = ABSORB && !nope ? MQH - 64 : 0;
+    const int col0 = !ABSORB ? 128 * tile : nope ? tile * MQH : 2 * pair * MQH + MNOPE;
     float qs[TT];
     f32x4 ws[2];
 #pragma unroll
     for (int tb = 0; tb < TT; ++tb) qs[tb] = a.q_norm_scale[min(16 * TT * wr + 16 * tb + l16, a.t - 1)];
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + col0 + 16 * gt_batch_block(wc, nb) + 4 * g);
+    for (int nb = 0; nb < 2; ++nb) ws[nb] = *reinterpret_cast<const f32x4*>(a.w_qb_scale + col0 + (wc >> 1) * gap + 16 * gt_batch_block(wc, nb) + 4 * g);
+    AbsorbedWide ab;
+    if (nope) ab.load(a, tile);
     i32x4 acc[2][TT];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
         for (int tb = 0; tb < TT; ++tb) acc[nb][tb] = i32x4{0, 0, 0, 0};
-    gt_batch_i8<TT>(acc, static_cast<const int8_t*>(a.w_uq_qr) + col0, (int64_t)a.n * MQH, a.q_norm, a.r, a.t, a.r / GT_KI8, lds);
+    gt_batch_i8<TT>(acc, static_cast<const int8_t*>(a.w_uq_qr) + col0, (int64_t)a.n * MQH, a.q_norm, a.r, a.t, a.r / GT_KI8, lds, gap);
+    const int row = nope ? AbsorbedWide::ROW : QBS_ROW;
+    uint8_t* to = lds + (16 * TT * wr + l16) * row + 8 * g;
 #pragma unroll
     for (int tb = 0; tb < TT; ++tb)
 #pragma unroll
@@ -1100,18 +1262,22 @@ __device__ __forceinline__ void mla_qb_batch_body(const MlaPrologArgs& a, int ti
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = ((float)acc[nb][tb][e] * qs[tb]) * ws[nb][e];
             const int cb = gt_batch_block(wc, nb);
-            *reinterpret_cast<u32x2*>(lds + ((cb >> 2) * T::TOK + 16 * TT * wr + 16 * tb + l16) * QBS_ROW + (16 * (cb & 3) + 4 * g) * 2) =
+            *reinterpret_cast<u32x2*>(to + 16 * tb * row + 32 * (cb & 3) + (cb >> 2) * (nope ? 128 : T::TOK * QBS_ROW)) =
                 u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
         }
     __syncthreads();
-    qb_store_blocks<T::TOK, 256>(a, lds, 2 * tile, 0);
+    if (nope) {
+        ab.turn();
+        ab.multiply<2 * TT, false>(a, tile, 0, lds);
+    } else
+        qb_store_blocks<T::TOK, 256>(a, lds, ABSORB ? 6 * pair + 2 : 2 * tile, 0, ABSORB ? 3 : 1);
 }
 // grid (n * 192 / 128), 512 lanes
-template <int TT>
+template <int TT, bool ABSORB>
 __global__ __launch_bounds__(GT_LANES, 2) void mla_qb_batch_kernel(MlaPrologArgs a)
 {
     __shared__ __align__(16) uint8_t lds[GtBatch<TT>::LDS];
-    mla_qb_batch_body<TT>(a, blockIdx.x, lds);
+    mla_qb_batch_body<TT, ABSORB>(a, blockIdx.x, lds);
 }
 
 // ------------------------------------------------------------------------------------------------ fused with the indexer prolog
@@ -1166,17 +1332,17 @@ __global__ __launch_bounds__(256) void fused_head_kernel(MlaPrologArgs m, Prolog
 // The same pair at 33 to QB_BATCH_T tokens.  The kernel at model sizes: 40 tokens 13.8 us, 96: 16.0, 128: 18.4, 160: 22.1; tiles of
 // 128 x 128 through registers, three stages of loads in flight and two barriers a stage, took 20.7 up to 128 tokens, tiles of 256
 // outputs 24.4 at 160.  grid (index heads + n * 192 / 128), 512 lanes
-template <int TT>
+template <int TT, bool ABSORB>
 __global__ __launch_bounds__(GT_LANES, 2) void fused_qb_batch_kernel(MlaPrologArgs m, PrologArgs p)
 {
     __shared__ __align__(16) uint8_t lds[GtBatch<TT>::LDS];
     if ((int)blockIdx.x < p.n) // (the index heads have the longer epilogue)
         prolog_q_batch_body<TT>(p, blockIdx.x, lds);
     else
-        mla_qb_batch_body<TT>(m, blockIdx.x - p.n, lds);
+        mla_qb_batch_body<TT, ABSORB>(m, blockIdx.x - p.n, lds);
 }
 
-// For more tokens than that (qb_batch) the two products in one launch of gemm_tile.h's tiles: the index heads' part alone is half a round of workgroups
+// For more tokens than that (qb_batch), of few heads, the two products in one launch of gemm_tile.h's tiles: the index heads' part alone is half a round of workgroups
 // up to 512 tokens (call of 257 tokens 83.0 us as two launches, 72.2 as one, 512: 104.4 / 96.3, 1024: 163.6 / 160.7, 1344: 211.5 /
 // 194.6, 4096: 604.7 / 591.0).  Tiles of 128 to 256 tokens, by modelled time (with 224 at most: 512 tokens 94.5 us a call, 1024: 159.8,
 // 1501: 215.7; so 91.9, 153.6, 207.0).
@@ -1197,6 +1363,35 @@ __global__ __launch_bounds__(GT_LANES, 2) void fused_qb_wide_kernel(MlaPrologArg
         id -= nqt * rows;
         mla_qb_wide_body<TB>(m, id % nqb, id / nqb * 32 * TB, lds);
     }
+}
+
+// The same with the absorbed products behind the heads' first dims, and alone.  grid (groups of eight units of wide_unit), 512 lanes
+template <int TB>
+__global__ __launch_bounds__(GT_LANES, 2) void fused_heads_wide_kernel(MlaPrologArgs m, PrologArgs p, int share)
+{
+    constexpr int A = mla_heads_wide_lds(TB), B = prolog_q_wide_lds(TB);
+    __shared__ __align__(16) uint8_t lds[A > B ? A : B];
+    const int nqt = (p.n + 1) / 2, nab = m.n / 2, nro = (m.n + 3) / 4, rows = (m.t + 32 * TB - 1) / (32 * TB);
+    const WideUnit u = wide_unit(blockIdx.x, nab * rows, (nqt + nro) * rows, share);
+    if (u.kind < 0) return;
+    if (u.kind == 0)
+        mla_heads_wide_body<TB>(m, u.at % nab, false, u.at / nab * 32 * TB, lds);
+    else if (u.at < nqt * rows)
+        prolog_q_wide_body<TB>(p, 2 * (u.at % nqt), u.at / nqt * 32 * TB, lds);
+    else {
+        const int id = u.at - nqt * rows;
+        mla_heads_wide_body<TB>(m, id % nro, true, id / nro * 32 * TB, lds);
+    }
+}
+template <int TB>
+__global__ __launch_bounds__(GT_LANES, 2) void mla_heads_wide_kernel(MlaPrologArgs a, int share)
+{
+    __shared__ __align__(16) uint8_t lds[mla_heads_wide_lds(TB)];
+    const int nab = a.n / 2, nro = (a.n + 3) / 4, rows = (a.t + 32 * TB - 1) / (32 * TB);
+    const WideUnit u = wide_unit(blockIdx.x, nab * rows, nro * rows, share);
+    if (u.kind < 0) return;
+    const int per = u.kind == 0 ? nab : nro;
+    mla_heads_wide_body<TB>(a, u.at % per, u.kind == 1, u.at / per * 32 * TB, lds);
 }
 
 // ------------------------------------------------------------------------------------------------ q_b[:, head, :128] @ w_uk[head]
@@ -1270,7 +1465,7 @@ __global__ __launch_bounds__(256) void mla_wuk_kernel(MlaPrologArgs a)
     }
 }
 
-// The same product for more tiles than WUK_TILES, with the same sums in the same order.  Bound by the outputs' way to memory (1501 tokens x 128
+// The same product for more tiles than WUK_TILES where it is a kernel of its own (the bf16 form; few heads).  Bound by the outputs' way to memory (1501 tokens x 128
 // heads: 197 MB out, 49 in, 47 us at the rate of a large copy).  By tiles of 64 tokens x 128 outputs, two workgroups to a CU with
 // the weights in LDS, every tile's rows were read four times over and a tile passed two barriers: 65 us.  So a workgroup of 512
 // lanes owns a head's whole 512 outputs and walks the token tiles of 64, z of them side by side (z: one workgroup to a CU); wave w
@@ -1458,9 +1653,51 @@ static bool qb_batch(const MlaPrologArgs& a, const PrologArgs* p)
 // warm weights: fused, 1 token 27.1 / 24.7, 8: 28.5 / 26.0, 32: 30.1 / 27.5, of 16 heads 23.1 / 21.6; bf16 form, 24 tokens 29.8 / 27.6, out
 // of HBM 36.0 / 33.9, of 16 heads 23.3 / 22.4; int8 form, 8 tokens 23.8 / 22.3, out of HBM 28.4 / 28.2).  The int8 form of few heads has short
 // streams behind each other: of 16 19.8 / 20.0, 32: 20.0 / 20.5, 64: 20.7 / 20.7.
+//
+// From 33 to QB_BATCH_T tokens, one workgroup to a CU still, the first weights of the absorbed product are fetched ahead of the stream of the
+// others (three sets of operands in turn, us a call, two kernels / one: fused, 33 tokens 36.0 / 33.7, 64: 39.3 / 36.6, 96: 46.4 / 41.8; one set, 48
+// tokens 31.6 / 31.4, 96: 38.6 / 36.4, 128: 42.7 / 39.1, 160: 50.4 / 44.0, of 16 heads 64: 27.9 / 26.0; int8 form, three sets, 48 tokens 29.8 / 29.7,
+// 96: 37.6 / 36.3, one set 26.8 / 28.0 and 31.7 / 32.6, 160: 41.9 / 39.7, of 64 heads 96: 27.9 / 28.4).  In two rounds (256 heads) 128 tokens take
+// 67.2 / 67.6 fused, 58.5 / 59.8 alone.
+// Above, whole tiles of 256 outputs with it: fused, 200 tokens 55.7 / 51.4, 300: 64.4 / 56.9, 512: 83.6 / 73.3, 800: 121.0 / 111.2, 1024:
+// 142.3 / 126.2, 1501: 203.3 / 174.4; int8 form 200: 46.3 / 45.9, 512: 71.0 / 67.0, 640: 81.3 / 80.5, 1024: 126.7 / 118.1, 1501: 179.1 / 159.9.  Few heads
+// are few long workgroups: fused, 16 heads 512: 54.1 / 54.5, 700: 64.7 / 63.4; 32 heads 250: 46.4 / 47.2, 400: 54.3 / 52.8; int8 form 64 heads
+// 330: 47.1 / 47.6, 400: 50.7 / 49.8; 32 heads 512: 49.4 / 51.2, 1024: 68.0 / 66.1.
 static bool head_units(const MlaPrologArgs& a, const PrologArgs* p)
 {
-    return a.t < BIG_T && a.n * MQH / 128 + (p ? p->n : 0) <= 256 && (p || !a.quant || a.n > 64);
+    const int slices = a.n * MQH / 128 + (p ? p->n : 0);
+    if (a.t < BIG_T) return slices <= 256 && (p || !a.quant || a.n > 64);
+    if (!a.quant) return false;
+    if (qb_batch(a, p)) return slices <= 256 && (p || (a.n >= 96 && a.t > 64));
+    return (int64_t)a.n * a.t >= (p ? 10000 : 24000);
+}
+
+// Token blocks (4 to 8) of the tiles with the absorbed product behind: the end of the last of n1 long and n2 short workgroups on 256
+// CUs, long ones first, with times (in no unit) that rank the tiles as measured (best of 4 .. 8 taken for 257, 300, 410, 512, 612, 800, 958 and 1501 tokens
+// fused, within 1 us of it alone).
+static double heads_end(int64_t n1, int64_t n2, double t1, double t2)
+{
+    const double begin = n1 / 256 * t1;
+    const int64_t rest = n1 % 256;
+    double end = begin + (rest ? t1 : 0);
+    for (int64_t k = 0;; ++k) // k, k + 1, .. rounds of short ones beside the last long ones
+        for (const double e : {begin + k * t2, begin + t1 + k * t2}) {
+            const int64_t behind = rest ? std::max<int64_t>(0, (int64_t)((e - begin - t1) / t2 + 1e-9)) : 0;
+            if ((256 - rest) * (int64_t)((e - begin) / t2 + 1e-9) + rest * behind >= n2) return std::max(end, e);
+        }
+}
+static int heads_token_blocks(const MlaPrologArgs& a, const PrologArgs* p)
+{
+    int best = 4;
+    double best_end = 1e30;
+    for (int tb = 4; tb <= 8; ++tb) {
+        const int64_t rows = (a.t + 32 * tb - 1) / (32 * tb);
+        const double depth = a.r / 1536.0 * tb;
+        const double end = p ? heads_end(a.n / 2 * rows, ((a.n + 3) / 4 + (p->n + 1) / 2) * rows, 8.0 + 1.2 * depth, 3.3 + 1.3 * depth)
+                             : heads_end(a.n / 2 * rows, (a.n + 3) / 4 * rows, 9.9 + 1.17 * depth, 5.3 + 1.16 * depth);
+        if (end < best_end) best = tb, best_end = end;
+    }
+    return best;
 }
 
 // p == nullptr: the MLA prolog on its own; otherwise the fused operator (m and p bound by fused_prolog_bind)
@@ -1533,7 +1770,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
     if ((e = hipGetLastError()) != hipSuccess) return e;
     {
         ScopedKernelTimer tm(KID_MLA_QB, stream);
-        if (heads) {
+        if (heads && !big) {
             if (p)
                 hipLaunchKernelGGL(fused_head_kernel, dim3(a.n * MQH / 128 + p->n), dim3(256), 0, stream, a, *p);
             else
@@ -1546,10 +1783,29 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
             if (qb_batch(a, p)) {
                 token_blocks(a.t, [&](auto tt) {
                     constexpr int TT = std::clamp(decltype(tt)::value, 2, QB_BATCH_T / 32);
-                    if (p)
-                        hipLaunchKernelGGL(fused_qb_batch_kernel<TT>, dim3(a.n * MQH / 128 + p->n), dim3(GT_LANES), 0, stream, a, *p);
+                    auto launch = [&](auto absorb) {
+                        constexpr bool ABSORB = decltype(absorb)::value;
+                        if (p)
+                            hipLaunchKernelGGL((fused_qb_batch_kernel<TT, ABSORB>), dim3(a.n * MQH / 128 + p->n), dim3(GT_LANES), 0, stream, a, *p);
+                        else
+                            hipLaunchKernelGGL((mla_qb_batch_kernel<TT, ABSORB>), dim3(a.n * MQH / 128), dim3(GT_LANES), 0, stream, a);
+                    };
+                    if (heads)
+                        launch(std::true_type{});
                     else
-                        hipLaunchKernelGGL(mla_qb_batch_kernel<TT>, dim3(a.n * MQH / 128), dim3(GT_LANES), 0, stream, a);
+                        launch(std::false_type{});
+                });
+            } else if (heads) {
+                const int qcols = p ? (p->n + 1) / 2 : 0;
+                gt_dispatch(heads_token_blocks(a, p), [&](auto tb) {
+                    constexpr int TB = decltype(tb)::value;
+                    const int rows = (a.t + 32 * TB - 1) / (32 * TB), first = a.n / 2 * rows, second = ((a.n + 3) / 4 + qcols) * rows;
+                    const int share = first + second <= 512 ? 256 : 210;
+                    const dim3 grid(8 * ((first + 7) / 8 + (second + 7) / 8));
+                    if (p)
+                        hipLaunchKernelGGL(fused_heads_wide_kernel<TB>, grid, dim3(GT_LANES), 0, stream, a, *p, share);
+                    else
+                        hipLaunchKernelGGL(mla_heads_wide_kernel<TB>, grid, dim3(GT_LANES), 0, stream, a, share);
                 });
             } else {
                 const int cols = (a.n * MQH + 255) / 256, qcols = p ? (p->n + 1) / 2 : 0, stages = a.r / GT_KI8;

@@ -221,6 +221,18 @@ def test_absorbed_product_behind_the_query_product(cuda, t, n, r):
     check_against_oracle(mla_case, idx_case, fused)
 
 
+@pytest.mark.parametrize("t,n,r", [(33, 4, 128), (64, 128, 256), (97, 66, 128), (129, 80, 384), (160, 128, 256), (160, 66, 256), (257, 60, 384),
+                                   (300, 128, 1536), (330, 130, 128), (410, 128, 128), (512, 128, 256), (1030, 128, 128)])
+def test_absorbed_product_behind_tiles(cuda, t, n, r):
+    # all tokens beside 128 outputs, blocks of 32 tokens with the last ones missing; tiles of 128 to 256 tokens, one and two rounds of
+    # workgroups and more, where the units go out in turn; 66 and 130 heads end with half a unit of rotary dims and begin rounds of the XCDs anew.
+    # Separate calls of few heads are two kernels: the same bits
+    mla_case, idx_case = op.make_fused_case(t, 1, 300, seed=160 + n, n_idx=64, h=512, q_lora_rank=r, n=n)
+    fused = run_fused(mla_case, idx_case, cuda)
+    same_as_separate(fused, run_separate(mla_case, idx_case, cuda), idx_case)
+    check_against_oracle(mla_case, idx_case, fused)
+
+
 @pytest.mark.parametrize("t,n_idx,r,h", [(257, 128, 1664, 256), (258, 64, 1536, 2304), (259, 64, 384, 1280), (1284, 128, 128, 512)])
 def test_norms_by_wavefronts(cuda, t, n_idx, r, h):
     # above 256 tokens and with at most four splits of x's product, four tokens to a workgroup: one, two and three of them and all in the

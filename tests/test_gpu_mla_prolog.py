@@ -270,6 +270,13 @@ def test_absorbed_product_behind_the_query_product(cuda, t, n, r, quant_b):
         check_bf16_form(case, got, outliers=1e-4)
 
 
+@pytest.mark.parametrize("t,n,r", [(65, 96, 128), (96, 170, 384), (160, 98, 128), (161, 150, 128), (192, 300, 128), (300, 128, 1536), (385, 128, 128), (512, 128, 256)])
+def test_absorbed_product_behind_tiles(cuda, t, n, r):
+    # 128 outputs of a head and all tokens to a workgroup; two heads and tiles of 128 to 256 tokens, with and without whole groups of four heads
+    case = op.make_case(t, 1, 300, seed=170 + n, h=512, q_lora_rank=r, n=n)
+    check(case, run(case, cuda))
+
+
 @pytest.mark.parametrize("quant_b", [True, False])
 def test_a_tokens_bits_do_not_depend_on_the_batch(cuda, quant_b):
     """Up to 32 tokens and from 33 on other kernels form the products; up to 256 tokens their fp32 sums are the same (chains of 128
