@@ -506,6 +506,84 @@ __device__ __forceinline__ void gt_product_bf16(f32x16 (&sum)[2][2], const uint1
     finish(stages, true);
 }
 
+// gt_batch_i8's stream in bf16, 33 to 128 tokens: w0, w1 are the two blocks of 64 outputs, ldw values a row.  Wave (wr, wc) owns outputs [32 wc, +32) of
+// the token blocks wr, wr + 2.  Register e of sum[i]: output 32 wc + 8 (e / 4) + 4 hl + e % 4, token 32 (wr + 2 i) + lane % 32.  The sums are
+// gt_product_bf16's, to the bit.
+template <int TT>
+struct GtBatch16 {
+    static constexpr int TOK = 32 * TT, XBYTES = TOK * 128, STAGE = XBYTES + 2 * 64 * 128, FIT = 160 * 1024 / STAGE, RING = FIT < 4 ? FIT : 4, LDS = RING * STAGE;
+    static constexpr int NB = (TT + 1) / 2; // token blocks of a wave
+};
+template <int TT, int CHAIN, int GROUP>
+__device__ __forceinline__ void gt_batch_bf16(f32x16 (&sum)[GtBatch16<TT>::NB], const uint16_t* w0, const uint16_t* w1, int64_t ldw, const uint16_t* x,
+                                              int64_t ldx, int t, int stages, uint8_t* lds)
+{
+#pragma clang fp contract(off)
+    using T = GtBatch16<TT>;
+    constexpr int NB = T::NB, XC = (TT + 1) / 2;
+    const int lane = threadIdx.x & 63, wave = gt_wave();
+    const int l32 = lane & 31, hl = lane >> 5, jj = lane & 15, mh = (lane >> 4) & 1, wr = wave >> 2, wc = wave & 3;
+    // copies of a wave: token rows 64 i + 8 w + lane / 8 (the last rows again where eight waves have more hands than rows), weight rows 8 w + lane / 8
+    // of either block
+    const int row = 8 * wave + (lane >> 3), pos = lane & 7;
+    uint32_t xo[XC];
+    int xd[XC];
+#pragma unroll
+    for (int i = 0; i < XC; ++i) {
+        const int c = min(8 * i + wave, 4 * TT - 1), xrow = 8 * c + (lane >> 3);
+        xd[i] = 1024 * c;
+        xo[i] = (uint32_t)(min(xrow, t - 1) * (int)ldx * 2 + 16 * (pos ^ ((xrow >> 1) & 7)));
+    }
+    const uint32_t wo = (uint32_t)row * (uint32_t)ldw * 2 + 16 * (pos ^ ((row << 1) & 4));
+    const uint8_t* xr = lds + (32 * wr + l32) * 128;
+    const int xf = (l32 >> 1) & 7;
+    const uint8_t* wrow = lds + T::XBYTES + (wc >> 1) * 8192 + (8 * hl + (jj >> 2)) * 128 + 8 * (jj & 1);
+    const int wpos = 16 * ((4 * (wc & 1) + 2 * mh + ((jj >> 1) & 1)) ^ ((jj >> 1) & 4));
+    f32x16 acc[NB], part[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][e] = part[i][e] = sum[i][e] = 0.f;
+    gt_stages<T::RING, T::STAGE, XC + 2>(
+        stages,
+        [&](int st, int b) {
+            gt_copy(w0 + (int64_t)st * GT_KBF * ldw, wo, lds + b + T::XBYTES + 1024 * wave);
+            gt_copy(w1 + (int64_t)st * GT_KBF * ldw, wo, lds + b + T::XBYTES + 8192 + 1024 * wave);
+#pragma unroll
+            for (int i = 0; i < XC; ++i) gt_copy(x + st * GT_KBF, xo[i], lds + b + xd[i]);
+        },
+        [&](int st, int b) {
+            bf16x8 xv[GT_KBF / 16][NB], wv[GT_KBF / 16];
+#pragma unroll
+            for (int ks = 0; ks < GT_KBF / 16; ++ks) {
+                const uint8_t* p = wrow + b + 2048 * ks + wpos;
+                const s16x4 lo = lds_read_tr(p), hi = lds_read_tr(p + 512);
+                wv[ks] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+                for (int i = 0; i < NB; ++i) // (an odd last block: both rows of waves have it, one drops it)
+                    xv[ks][i] = *reinterpret_cast<const bf16x8*>(xr + b + min(2 * i, TT - 1 - wr) * 4096 + 16 * ((2 * ks + hl) ^ xf));
+            }
+#pragma unroll
+            for (int ks = 0; ks < GT_KBF / 16; ++ks)
+#pragma unroll
+                for (int i = 0; i < NB; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[ks], xv[ks][i], acc[i], 0, 0, 0);
+            const int done = st + 1;
+            const bool last = done == stages;
+            if (done % (CHAIN / GT_KBF) == 0 || last) {
+#pragma unroll
+                for (int i = 0; i < NB; ++i)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) part[i][e] += acc[i][e], acc[i][e] = 0.f;
+            }
+            if (done % (GROUP / GT_KBF) == 0 || last) {
+#pragma unroll
+                for (int i = 0; i < NB; ++i)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) sum[i][e] += part[i][e], part[i][e] = 0.f;
+            }
+        });
+}
+
 // Token blocks TB (4 .. most) of an int8 product's tile, by the time it should take in ns: the grid runs in rounds of one
 // workgroup to each of the 256 CUs; a stage costs its matrix instructions, as the token blocks, and the weights' copies, like
 // about two of them; a round has its ends; the copies together have 26 TB/s.

@@ -48,6 +48,7 @@ constexpr int TROW = 128 * 2 + 32; // bytes per LDS row of a [k][128] bf16 weigh
 constexpr int BIG_T = 33;         // token count from which the query kernels that hold more than 32 tokens take over: the others read the
                                   // weights once per 32 tokens (fused prolog, 32 tokens 30.5 us and 40: 31.2; with the weights read
                                   // twice 63.6)
+constexpr int BATCH16_T = 128;    // token count to which the bf16 form's query product streams its weights beside all tokens
 constexpr int BIG_T2 = 256;       // token count above which the x product's tiles are 256 outputs wide, in splits of its own
 
 // Output tile `tile` (64 columns) of x @ [w_dq | w_dkv_kr | w_k | w_proj]: its weight columns and their row stride.
@@ -1094,6 +1095,21 @@ struct AbsorbedWide {
 #pragma unroll
             for (int k = 0; k < 8; ++k) raw[8 * ks + k] = *reinterpret_cast<const u32x2*>(src + (32 * ks + k) * MC);
     }
+    // The weights of HEADS heads from `head` on into the XCD's L2, a line to a lane, four bytes of which land in 256 bytes of LDS at `drop`.
+    // Nothing waits for them but the first stage of the product that follows, whose copies are younger.  The first token tile of a head does it
+    // for all (they are one XCD's).  Three sets of operands in turn, us a call without / with: fused, 200 tokens 61.2 / 57.0, 512: 89.9 / 86.5, 1501:
+    // 193.3 / 189.3; int8 form 300: 64.2 / 59.4; bf16 form 256: 73.0 / 65.0, 1024: 177.6 / 174.0; one set, bf16 form 256: 57.4 / 59.5.
+    template <int HEADS>
+    static __device__ __forceinline__ void touch(const MlaPrologArgs& a, int head, uint8_t* drop)
+    {
+        const uint16_t* src = a.w_uk + (int64_t)head * MNOPE * MC;
+#pragma unroll
+        for (int i = 0; i < HEADS * MNOPE * MC / 64 / 512; ++i)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                         :
+                         : "s"((gt_lds*)drop), "v"((uint32_t)(128 * (threadIdx.x + 512 * i))), "s"(src)
+                         : "memory");
+    }
     __device__ __forceinline__ void turn()
     {
 #pragma unroll
@@ -1176,6 +1192,7 @@ __device__ __forceinline__ void mla_heads_wide_body(const MlaPrologArgs& a, int 
     const int c0 = rope ? 4 * unit * MQH + MNOPE : 2 * unit * MQH, c1 = rope ? min(4 * unit + 2, a.n - 2) * MQH + MNOPE : c0 + MQH;
     const int gap = rope ? MQH - 64 : 0, cw = (wc >> 1 ? c1 : c0) + (wc & 1) * (64 + gap);
     const int8_t* w = static_cast<const int8_t*>(a.w_uq_qr);
+    if (!rope && tok0 == 0) AbsorbedWide::touch<2>(a, 2 * unit, lds + (T::RING - 1) * T::QBYTES);
     gt_product_i8<TB>(acc, w + c0, w + c1, nq, a.q_norm, a.r, tok0, a.t, a.r / GT_KI8, lds, wave, gap);
     AbsorbedWide ab;
     if (!rope) ab.load(a, 2 * unit);
@@ -1223,6 +1240,91 @@ __device__ __forceinline__ WideUnit wide_unit(int id, int n1, int n2, int share)
     const bool first = firsts(j + 1) > before;
     const int at = 8 * (first ? before : j - before) + id % 8;
     return {at >= (first ? n1 : n2) ? -1 : first ? 0 : 1, at};
+}
+
+// The bf16 form by the same units: 33 to 128 tokens beside a head's first dims or two heads' rotary dims, the weights streamed (gt_batch_bf16);
+// sums and operations are mla_qb16_kernel's.  In tiles of 128 x 256 the 75 MB of weights were 96 workgroups' work on 256 CUs, 23 us, and the absorbed
+// product 7 to 9 behind them.  A call of 33, 64 and 128 tokens 38.4 -> 29.6 us, 40.1 -> 31.2, 46.0 -> 39.4 (three sets of operands 45.3 -> 36.1, 48.5 ->
+// 39.8, 57.9 -> 48.5); 16 heads, 64 tokens 36.8 -> 27.6.  A head's w_uk goes to registers ahead of the stages (behind them, from the L2, 1.4 us more).
+// grid (n * 192 / 128), 512 lanes
+template <int TT>
+__global__ __launch_bounds__(GT_LANES, 2) void mla_heads16_batch_kernel(MlaPrologArgs a)
+{
+    using T = GtBatch16<TT>;
+    static_assert(2 * T::TOK * QBS_ROW <= T::LDS && T::TOK * AbsorbedWide::ROW <= T::LDS, "the output tile takes the stages' place");
+    __shared__ __align__(16) uint8_t lds[T::LDS];
+    const int lane = threadIdx.x & 63, wave = gt_wave(), l32 = lane & 31, hl = lane >> 5, wr = wave >> 2, wc = wave & 3;
+    const bool nope = (int)blockIdx.x < a.n;
+    const int pair = blockIdx.x - a.n, col0 = nope ? blockIdx.x * MQH : 2 * pair * MQH + MNOPE;
+    AbsorbedWide ab;
+    if (nope) ab.load(a, blockIdx.x);
+    f32x16 sum[T::NB];
+    const uint16_t* w = static_cast<const uint16_t*>(a.w_uq_qr) + col0;
+    gt_batch_bf16<TT, 128, XA_SPLIT>(sum, w, w + (nope ? 64 : MQH), a.n * MQH, reinterpret_cast<const uint16_t*>(a.q_norm), a.r, a.t, a.r / GT_KBF, lds);
+    const int row = nope ? AbsorbedWide::ROW : QBS_ROW;
+    uint8_t* to = lds + l32 * row + (wc >> 1) * (nope ? 128 : T::TOK * QBS_ROW) + 64 * (wc & 1) + 8 * hl;
+#pragma unroll
+    for (int i = 0; i < T::NB; ++i)
+        if (wr + 2 * i < TT) // (wave-uniform)
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4)
+                *reinterpret_cast<u32x2*>(to + 32 * (wr + 2 * i) * row + 16 * e4) =
+                    u32x2{pack_bf16x2(sum[i][4 * e4], sum[i][4 * e4 + 1]), pack_bf16x2(sum[i][4 * e4 + 2], sum[i][4 * e4 + 3])};
+    __syncthreads();
+    if (nope) {
+        ab.turn();
+        ab.multiply<2 * TT, false>(a, blockIdx.x, 0, lds);
+    } else
+        qb_store_blocks<T::TOK, 256>(a, lds, 6 * pair + 2, 0, 3);
+}
+
+// More tokens: tiles of 128 tokens x two heads' first dims or four heads' rotary dims (mla_qb16_wide_kernel's product).  Three sets of operands in
+// turn: 200 tokens 64.5 -> 61.8 us, 289: 92.0 -> 81.3, 384: 98.7 -> 84.5, 512: 107.9 -> 103.4, 1024: 175.2 -> 174.0 (one set 176.7 -> 168.5).
+// grid (groups of eight units of wide_unit), 512 lanes
+__global__ __launch_bounds__(GT_LANES, 2) void mla_heads16_wide_kernel(MlaPrologArgs a, int share)
+{
+    using T = GtTile<4>;
+    static_assert(4 * T::TOK * QBS_ROW <= T::LDS && 2 * T::TOK * AbsorbedWide::ROW <= T::LDS, "the output tile takes the operand tiles' place");
+    __shared__ __align__(16) uint8_t lds[T::LDS];
+    const int lane = threadIdx.x & 63, wave = gt_wave(), l32 = lane & 31, hl = lane >> 5, wr = wave >> 2, wc = wave & 3;
+    const int nab = a.n / 2, nro = (a.n + 3) / 4, rows = (a.t + T::TOK - 1) / T::TOK;
+    const WideUnit u = wide_unit(blockIdx.x, nab * rows, nro * rows, share);
+    if (u.kind < 0) return;
+    const bool rope = u.kind == 1;
+    const int per = rope ? nro : nab, unit = u.at % per, tok0 = u.at / per * T::TOK;
+    const uint16_t* src[4];
+    int ld[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { // (heads past the last one: that one again, dropped below)
+        src[i] = static_cast<const uint16_t*>(a.w_uq_qr) + (rope ? min(4 * unit + i, a.n - 1) * MQH + MNOPE : (2 * unit + (i >> 1)) * MQH + 64 * (i & 1));
+        ld[i] = a.n * MQH;
+    }
+    f32x16 sum[2][2];
+    if (!rope && tok0 == 0) AbsorbedWide::touch<2>(a, 2 * unit, lds + (T::RING - 1) * T::QBYTES);
+    gt_product_bf16<128, XA_SPLIT>(sum, src, ld, reinterpret_cast<const uint16_t*>(a.q_norm), a.r, tok0, a.t, a.r / GT_KBF, lds);
+    AbsorbedWide ab;
+    __builtin_amdgcn_sched_barrier(0); // (once the sums' registers are free)
+    if (!rope) ab.load(a, 2 * unit);
+    const int row = rope ? QBS_ROW : AbsorbedWide::ROW;
+    uint8_t* to = lds + (rope ? wc * T::TOK * QBS_ROW : (wc >> 1) * T::TOK * AbsorbedWide::ROW + (wc & 1) * 128) + 2 * l32;
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+                *reinterpret_cast<uint16_t*>(to + (64 * wr + 32 * tb + 8 * (e >> 2) + 4 * hl + (e & 3)) * row + 64 * nb) = f32_to_bf16(sum[tb][nb][e]);
+    __syncthreads();
+    if (rope) {
+        qb_store_blocks<T::TOK>(a, lds, 12 * unit + 2, tok0, 3);
+        return;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        ab.turn();
+        if (h == 0) ab.load(a, 2 * unit + 1);
+        ab.multiply<T::TOK / 16, true>(a, 2 * unit + h, tok0, lds + h * T::TOK * AbsorbedWide::ROW);
+    }
 }
 
 // 33 to QB_BATCH_T tokens: 128 outputs per workgroup of 512 lanes, all tokens, the weights streamed (gt_batch_i8); the same exact sums
@@ -1662,12 +1764,13 @@ static bool qb_batch(const MlaPrologArgs& a, const PrologArgs* p)
 // Above, whole tiles of 256 outputs with it: fused, 200 tokens 55.7 / 51.4, 300: 64.4 / 56.9, 512: 83.6 / 73.3, 800: 121.0 / 111.2, 1024:
 // 142.3 / 126.2, 1501: 203.3 / 174.4; int8 form 200: 46.3 / 45.9, 512: 71.0 / 67.0, 640: 81.3 / 80.5, 1024: 126.7 / 118.1, 1501: 179.1 / 159.9.  Few heads
 // are few long workgroups: fused, 16 heads 512: 54.1 / 54.5, 700: 64.7 / 63.4; 32 heads 250: 46.4 / 47.2, 400: 54.3 / 52.8; int8 form 64 heads
-// 330: 47.1 / 47.6, 400: 50.7 / 49.8; 32 heads 512: 49.4 / 51.2, 1024: 68.0 / 66.1.
+// 330: 47.1 / 47.6, 400: 50.7 / 49.8; 32 heads 512: 49.4 / 51.2, 1024: 68.0 / 66.1; bf16 form 128 heads 129: 58.2 / 58.5, 64 heads 200: 49.5 / 52.7, 512:
+// 61.6 / 60.2, 16 heads 1024: 71.9 / 74.1.
 static bool head_units(const MlaPrologArgs& a, const PrologArgs* p)
 {
     const int slices = a.n * MQH / 128 + (p ? p->n : 0);
     if (a.t < BIG_T) return slices <= 256 && (p || !a.quant || a.n > 64);
-    if (!a.quant) return false;
+    if (!a.quant) return a.t <= BATCH16_T && slices <= 256 || (int64_t)a.n * a.t >= 24000;
     if (qb_batch(a, p)) return slices <= 256 && (p || (a.n >= 96 && a.t > 64));
     return (int64_t)a.n * a.t >= (p ? 10000 : 24000);
 }
@@ -1775,6 +1878,14 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
                 hipLaunchKernelGGL(fused_head_kernel, dim3(a.n * MQH / 128 + p->n), dim3(256), 0, stream, a, *p);
             else
                 hipLaunchKernelGGL((a.quant ? mla_head_kernel<true> : mla_head_kernel<false>), dim3(a.n * MQH / 128), dim3(256), 0, stream, a);
+        } else if (!a.quant && heads && a.t <= BATCH16_T && a.n * MQH / 128 <= 256) {
+            token_blocks(a.t, [&](auto tt) {
+                hipLaunchKernelGGL(mla_heads16_batch_kernel<std::clamp(decltype(tt)::value, 2, 4)>, dim3(a.n * MQH / 128), dim3(GT_LANES), 0, stream, a);
+            });
+        } else if (!a.quant && heads) {
+            const int rows = (a.t + 127) / 128, first = a.n / 2 * rows, second = (a.n + 3) / 4 * rows;
+            hipLaunchKernelGGL(mla_heads16_wide_kernel, dim3(8 * ((first + 7) / 8 + (second + 7) / 8)), dim3(GT_LANES), 0, stream, a,
+                               first + second <= 512 ? 256 : 210);
         } else if (!a.quant && big) {
             hipLaunchKernelGGL(mla_qb16_wide_kernel, dim3((a.n * MQH + 255) / 256, (a.t + 127) / 128), dim3(GT_LANES), 0, stream, a);
         } else if (!a.quant) {

@@ -277,6 +277,14 @@ def test_absorbed_product_behind_tiles(cuda, t, n, r):
     check(case, run(case, cuda))
 
 
+@pytest.mark.parametrize("t,n,r", [(33, 4, 256), (64, 128, 256), (65, 66, 1280), (97, 16, 512), (128, 170, 256), (188, 128, 1280), (300, 82, 256), (700, 128, 256)])
+def test_bf16_absorbed_product_behind_the_query_product(cuda, t, n, r):
+    # two, three and four blocks of 32 tokens with the last ones missing, one and several groups of chains; tiles of 128 tokens, one round of
+    # workgroups and more, half a unit of rotary dims at the end (82 heads)
+    case = op.make_case(t, 1, 300, seed=180 + n, h=512, q_lora_rank=r, n=n, quant_b=False)
+    check_bf16_form(case, run(case, cuda), outliers=1e-4)
+
+
 @pytest.mark.parametrize("quant_b", [True, False])
 def test_a_tokens_bits_do_not_depend_on_the_batch(cuda, quant_b):
     """Up to 32 tokens and from 33 on other kernels form the products; up to 256 tokens their fp32 sums are the same (chains of 128
