@@ -13,7 +13,8 @@
 //
 // At decode sizes (8 - 64 tokens) the operator reads 9 MB of int8 weights once (hidden 5120 x 1792 outputs) and is bound by
 // launch latency and that read; three launches:
-//   apq_norm_kernel   one workgroup per token: the row is read once and stays in registers across the sum
+//   apq_norm_kernel   one workgroup per token: the row is read once and stays in registers across the sum (up to 4 tokens part of the next:
+//                     apq_norm_gemm_kernel)
 //   apq_gemm_kernel   one workgroup per (128 outputs, 256 to 1024 contraction rows, 32 tokens): the weight tile (output
 //                     dimension contiguous in memory) is loaded in one go, parked in LDS and read back with 8-bit
 //                     transposing reads as the A operand of the int8 MFMA; int32 partial sums to the workspace (exact,
@@ -193,6 +194,143 @@ __global__ __launch_bounds__(256) void apq_gemm_kernel(AttnPreArgs a)
 #pragma unroll
         for (int db = 0; db < 2; ++db) *reinterpret_cast<i32x4*>(dst + 16 * db) = acc[db][tb];
     }
+}
+
+// A few tokens' norm and projection in one kernel (norm_in_projection): every workgroup adds up the rows' squares for itself, beside the weights'
+// way from memory, and quantises its own columns, so that a launch of one workgroup per token goes.  The operations and their order are
+// apq_norm_kernel's, lane by lane; the first column tile's workgroups write the sums of hidden states and residual and the quantised rows.  T: most tokens,
+// T / G of them to a group of 256 lanes.
+// grid (n_out / 128, splits of the contraction), 256 G lanes.
+template <int PER, int T, int G>
+__global__ __launch_bounds__(256 * G) void apq_norm_gemm_kernel(AttnPreArgs a)
+{
+#pragma clang fp contract(off)
+    constexpr int NP = 3, QROW = PER * AK + 16, PIECES = PER * AK / 8; // pieces of 8 elements: of a row per lane, of a token's columns here
+    static_assert(G <= 2 && T % G == 0, "");
+    constexpr int TG = T / G, LANES = 256 * G, OWN = (T * PIECES + LANES - 1) / LANES, DB = G == 1 ? 2 : 1;
+    __shared__ __align__(16) uint8_t wl[AK * AROW];
+    __shared__ __align__(16) uint8_t ql[T * QROW];
+    __shared__ float red[T][4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int l16 = lane & 15, g = lane >> 4, ltid = tid & 255, t0 = TG * (tid >> 8);
+    const int col0 = blockIdx.x * AD, split = blockIdx.y;
+    const int stages = a.h / AK, npieces = a.h / 8;
+    u32x4 xr[TG][NP], rr[TG][NP];
+#pragma unroll
+    for (int t = 0; t < TG; ++t)
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const int64_t at = (int64_t)min(t0 + t, a.t - 1) * npieces + min(ltid + 256 * i, npieces - 1);
+            xr[t][i] = reinterpret_cast<const u32x4*>(a.x)[at];
+            rr[t][i] = reinterpret_cast<const u32x4*>(a.residual)[at];
+        }
+    // this workgroup's columns: piece tid + LANES i, token by token
+    u32x4 ox[OWN], orr[OWN], gr[OWN], br[OWN], sr[OWN], fr[OWN];
+    int otok[OWN], opc[OWN];
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+        otok[i] = (tid + LANES * i) / PIECES;
+        opc[i] = split * PIECES + (tid + LANES * i) % PIECES;
+        const int pc = min(opc[i], npieces - 1);
+        const int64_t at = (int64_t)min(otok[i], a.t - 1) * npieces + pc;
+        ox[i] = reinterpret_cast<const u32x4*>(a.x)[at];
+        orr[i] = reinterpret_cast<const u32x4*>(a.residual)[at];
+        gr[i] = reinterpret_cast<const u32x4*>(a.gamma)[pc];
+        br[i] = reinterpret_cast<const u32x4*>(a.bias)[pc];
+        sr[i] = reinterpret_cast<const u32x4*>(a.in_scale)[pc];
+        fr[i] = reinterpret_cast<const u32x4*>(a.in_offset)[pc];
+    }
+    const int srow = tid >> 3, spc = tid & 7;
+    u32x4 stg[PER][AK / 32 / G];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int64_t kbase = (int64_t)min(split * PER + j, stages - 1) * AK;
+#pragma unroll
+        for (int i = 0; i < AK / 32 / G; ++i)
+            stg[j][i] = *reinterpret_cast<const u32x4*>(a.w + (kbase + srow + 32 * G * i) * a.n_out + col0 + 16 * spc);
+    }
+    __builtin_amdgcn_sched_barrier(0); // (every load is out)
+    float part[TG];
+#pragma unroll
+    for (int t = 0; t < TG; ++t) {
+        part[t] = 0.f;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const bool live = ltid + 256 * i < npieces;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float lo = bf16_bits_to_f32(rr[t][i][e] & 0xffffu) + bf16_bits_to_f32(xr[t][i][e] & 0xffffu);
+                const float hi = bf16_bits_to_f32(rr[t][i][e] >> 16) + bf16_bits_to_f32(xr[t][i][e] >> 16);
+                if (live) {
+                    part[t] += (lo * lo) * a.mean_coff;
+                    part[t] += (hi * hi) * a.mean_coff;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < TG; ++t) part[t] = wave_sum_descending(part[t]);
+    if (lane == 0)
+#pragma unroll
+        for (int t = 0; t < TG; ++t) red[t0 + t][wave & 3] = part[t];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+        if (otok[i] >= T) continue;
+        const float denom = sqrtf(((red[otok[i]][0] + red[otok[i]][1]) + (red[otok[i]][2] + red[otok[i]][3])) + a.eps);
+        int8_t q[8];
+        u32x4 ro;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            float s2[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int sh = e * 16;
+                s2[e] = bf16_bits_to_f32((orr[i][w] >> sh) & 0xffffu) + bf16_bits_to_f32((ox[i][w] >> sh) & 0xffffu);
+                const float ga = bf16_bits_to_f32((gr[i][w] >> sh) & 0xffffu), b = bf16_bits_to_f32((br[i][w] >> sh) & 0xffffu);
+                const float sc = bf16_bits_to_f32((sr[i][w] >> sh) & 0xffffu), of = bf16_bits_to_f32((fr[i][w] >> sh) & 0xffffu);
+                const float xn = round_bf16((s2[e] / denom) * ga + b);
+                const float v = __builtin_rintf(xn * sc + of);
+                q[2 * w + e] = (int8_t)(int)fminf(fmaxf(v, -128.f), 127.f);
+            }
+            ro[w] = pack_bf16x2(s2[0], s2[1]);
+        }
+        *reinterpret_cast<u32x2*>(ql + otok[i] * QROW + 8 * (opc[i] - split * PIECES)) = __builtin_bit_cast(u32x2, q);
+        if (blockIdx.x == 0 && otok[i] < a.t && opc[i] < npieces) {
+            const int64_t at = (int64_t)otok[i] * npieces + opc[i];
+            reinterpret_cast<u32x4*>(a.residual_out)[at] = ro;
+            reinterpret_cast<u32x2*>(a.x_q)[at] = __builtin_bit_cast(u32x2, q);
+        }
+    }
+    i32x4 acc[DB]; // wave w: outputs [16 DB w, +16 DB)
+#pragma unroll
+    for (int db = 0; db < DB; ++db) acc[db] = i32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        if (j > 0) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < AK / 32 / G; ++i) {
+            u32x2* d = reinterpret_cast<u32x2*>(wl + (srow + 32 * G * i) * AROW + 16 * spc);
+            d[0] = u32x2{stg[j][i][0], stg[j][i][1]};
+            d[1] = u32x2{stg[j][i][2], stg[j][i][3]};
+        }
+        __syncthreads(); // (and ql)
+        if (split * PER + j >= stages) continue; // uniform over the workgroup
+#pragma unroll
+        for (int ks = 0; ks < AK / 64; ++ks) {
+            const i32x4 qf = *reinterpret_cast<const i32x4*>(ql + min(l16, T - 1) * QROW + j * AK + 64 * ks + 16 * g);
+#pragma unroll
+            for (int db = 0; db < DB; ++db) { // (the byte-transposing read: see apq_gemm_kernel)
+                const uint8_t* p = wl + (ks * 64 + 16 * g + (l16 >> 1)) * AROW + 16 * (DB * wave + db) + 8 * (l16 & 1);
+                const v2i lo = lds_read_tr8(p), hi = lds_read_tr8(p + 8 * AROW);
+                acc[db] = __builtin_amdgcn_mfma_i32_16x16x64_i8(i32x4{lo[0], lo[1], hi[0], hi[1]}, qf, acc[db], 0, 0, 0);
+            }
+        }
+    }
+    if (l16 >= a.t) return;
+    int32_t* dst = a.part + ((int64_t)split * a.t + l16) * a.n_out + col0 + 16 * DB * wave + 4 * g;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) *reinterpret_cast<i32x4*>(dst + 16 * db) = acc[db];
 }
 
 // The projection of a rank's few heads at small prefill sizes (attention_pre_kernel): a workgroup owns 128 tokens x 128 outputs
@@ -717,11 +855,46 @@ void attention_pre_bind_workspace(AttnPreArgs& a, void* ws)
     a.part = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(ws) + align256((uint64_t)a.t * a.h));
 }
 
+// f(integral constants: stages per split, most tokens, groups of lanes) for norm_in_projection's kernel
+template <class F>
+static void norm_gemm_dispatch(int per, int t, F&& f)
+{
+    auto tokens = [&](auto p) {
+        if (t == 1)
+            f(p, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
+        else if (t == 2)
+            f(p, std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
+        else
+            f(p, std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
+    };
+    if (per == 4)
+        tokens(std::integral_constant<int, 4>{});
+    else if (per == 2)
+        tokens(std::integral_constant<int, 2>{});
+    else
+        tokens(std::integral_constant<int, 1>{});
+}
+
+// The sums of hidden states and residual may take the place of either: then one workgroup has to read and write a row.
+static bool rows_apart(const AttnPreArgs& a)
+{
+    const uint64_t bytes = (uint64_t)a.t * a.h * 2, to = (uint64_t)a.residual_out, x = (uint64_t)a.x, r = (uint64_t)a.residual;
+    return (to + bytes <= x || x + bytes <= to) && (to + bytes <= r || r + bytes <= to);
+}
+// Up to 4 tokens the norm joins the projection: every workgroup reads all rows, 20 KB a token (us a call, a kernel of its own / joined, three sets of
+// operands: 14 heads, 1 token 10.8 / 8.4, 2: 11.0 / 9.0, 4: 11.7 / 10.8, 8: 12.1 / 14.7; 28 heads 12.9 / 9.7, 13.2 / 10.4, 13.6 / 11.9, 14.1 / 16.6; 112
+// heads 20.9 / 17.4, 21.4 / 18.4, 22.0 / 21.1, 23.1 / 35.6; two tokens by one group of lanes 9.1, 10.7, 19.0, four by four groups 12.0, 12.8, 26.0).
+static bool norm_in_projection(const AttnPreArgs& a)
+{
+    return a.t <= 4 && a.h <= 3 * 2048 && rows_apart(a) && attention_pre_kernel(a.t, a.n_out) == ApqKernel::stream;
+}
+
 hipError_t attention_pre_launch(const AttnPreArgs& a, hipStream_t stream)
 {
     if (a.t == 0) return hipSuccess;
-    const bool whole = attention_pre_whole(a.t, a.n_out, a.ksplits);
+    const bool whole = attention_pre_whole(a.t, a.n_out, a.ksplits), together = norm_in_projection(a);
     hipError_t e;
+    if (!together)
     {
         ScopedKernelTimer tm(KID_APQ_NORM, stream);
         if (a.h <= 3 * 2048)
@@ -743,6 +916,11 @@ hipError_t attention_pre_launch(const AttnPreArgs& a, hipStream_t stream)
                 hipLaunchKernelGGL((whole ? apq_gemm_big_kernel<TB, true> : apq_gemm_big_kernel<TB, false>),
                                    dim3((a.n_out / AD + 1) / 2, a.ksplits, (a.t + 32 * TB - 1) / (32 * TB)), dim3(GT_LANES), 0, stream, a,
                                    big.per);
+            });
+        } else if (together) {
+            norm_gemm_dispatch(per, a.t, [&](auto p, auto t, auto g) {
+                constexpr int PER = decltype(p)::value, T = decltype(t)::value, G = decltype(g)::value;
+                hipLaunchKernelGGL((apq_norm_gemm_kernel<PER, T, G>), grid, dim3(256 * G), 0, stream, a);
             });
         } else if (kernel == ApqKernel::mid)
             hipLaunchKernelGGL(apq_gemm_mid_kernel, dim3(a.n_out / AD, a.ksplits, (a.t + BTOK - 1) / BTOK), dim3(256), 0, stream, a,

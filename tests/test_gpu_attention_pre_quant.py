@@ -226,6 +226,24 @@ def test_several_stages_per_workgroup_with_a_short_last_split(cuda, t, q_heads, 
     check(case, run(case, cuda))
 
 
+@pytest.mark.parametrize("t,h,q_heads,kv_heads", [(1, 256, 2, 1), (1, 5120, 12, 1), (2, 6144, 12, 1), (3, 5120, 24, 2), (4, 512, 3, 1), (4, 5120, 96, 8),
+                                                  (3, 1280, 94, 9), (2, 5888, 176, 2), (1, 6144, 150, 2), (4, 6144, 150, 2), (5, 5120, 12, 1), (4, 6400, 2, 1)])
+def test_norm_in_the_projection(cuda, t, h, q_heads, kv_heads):
+    """Up to 4 tokens and hidden 6144 the norm is the projection's workgroups' own: one, two and four stages to a workgroup with and without
+    a short last one, one to four tokens; in place of the residual (a kernel of its own there), the same bits."""
+    case = op.make_case(t, h=h, q_heads=q_heads, kv_heads=kv_heads, seed=t + h)
+    got = run(case, cuda)
+    check(case, got)
+    from pypto_amd.glm_v4_5 import glm_attention_pre_quant as impl
+    for place in ("hidden_states", "residual"):
+        on = {k: case[k].to(cuda) for k in NAMES}
+        out = outputs(case, cuda)
+        impl.attention_pre_quant(*[on[k] for k in NAMES], out["query"], out["key"], out["value"], on[place])
+        for name in ("query", "key", "value"):
+            assert torch.equal(out[name].cpu(), got[name]), (place, name)
+        assert torch.equal(on[place].cpu(), got["residual_res"]), place
+
+
 def test_saturation_at_both_ends(cuda):
     """A quantisation scale of 1000: nine in ten values of the quantised row are clamped at -128 or 127."""
     case = op.make_case(4, h=4096, q_heads=2, kv_heads=1, seed=14)
