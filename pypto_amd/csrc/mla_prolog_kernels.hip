@@ -548,12 +548,14 @@ __device__ __forceinline__ void mla_norm_key_body(const MlaPrologArgs& a, int to
     }
 }
 
-// The fused operator's norms where the x product has at most four splits (above 640 tokens at model sizes): a wavefront to each of a
+// The fused operator's norms above 256 tokens where the x product has at most eight splits: a wavefront to each of a
 // token's three chains, the sums of the workgroups above bit for bit - what they spread over four wavefronts (lane l of wave w: columns
 // l + 64 w + 256 i) are four sums of a lane here, and no barrier is passed.
 // What bounds it: the partial sums' way from memory (28 MB at 1501 tokens).  A workgroup to a chain went through barriers with
 // eight chains in flight to a CU, and every token's fetched hadamard_k's 32 KB out of the L2 in 128 loads: the kernel at 1501 tokens 15.1 us, so 11.6,
-// a call 210.7 -> 208.1, 900: 140.4 / 138.1.  The MLA prolog's two chains alone are as fast either way (1024 tokens 8.3 / 8.4).
+// a call 210.7 -> 208.1, 900: 140.4 / 138.1; with five to seven splits, 218 registers, three sets of operands in turn, 257: 63.7 / 63.2, 410: 78.6 / 77.2,
+// 600: 100.8 / 99.2; to 256 tokens slower (200: 57.9 / 58.0, 96: 41.2 / 42.0).  The MLA prolog's two chains alone are no faster (1024 tokens 8.3 / 8.4, a
+// call of 300 60.3 / 61.5).
 // request(i, split) asks for what a chain reads of a split, all S of them in flight together (a split past the end is the last one
 // again, dropped), add(i, first, real) adds it up in order.
 template <int S, class Request, class Add>
@@ -1850,7 +1852,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
             else
                 launch(std::integral_constant<int, 8>{}, touch);
         };
-        if (p && a.t > BIG_T2 && a.ksplits <= 4) {
+        if (p && a.t > BIG_T2 && a.ksplits <= 8) {
             auto wide = [&](auto splits, auto pieces) {
                 hipLaunchKernelGGL((fused_norm_wide_kernel<decltype(splits)::value, decltype(pieces)::value>), dim3(3 * ((a.t + 3) / 4)), dim3(256), 0,
                                    stream, a, *p);
@@ -1863,8 +1865,10 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
             };
             if (in_flight == 2)
                 wide_with(std::integral_constant<int, 2>{});
-            else
+            else if (in_flight == 4)
                 wide_with(std::integral_constant<int, 4>{});
+            else
+                wide_with(std::integral_constant<int, 8>{});
         } else if (ahead)
             launch_with(std::true_type{});
         else

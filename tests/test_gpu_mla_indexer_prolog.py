@@ -233,10 +233,10 @@ def test_absorbed_product_behind_tiles(cuda, t, n, r):
     check_against_oracle(mla_case, idx_case, fused)
 
 
-@pytest.mark.parametrize("t,n_idx,r,h", [(257, 128, 1664, 256), (258, 64, 1536, 2304), (259, 64, 384, 1280), (1284, 128, 128, 512)])
+@pytest.mark.parametrize("t,n_idx,r,h", [(257, 128, 1664, 256), (258, 64, 1536, 2304), (259, 64, 384, 1280), (1284, 128, 128, 512), (261, 64, 128, 5120), (300, 128, 1664, 8192), (270, 64, 256, 9216)])
 def test_norms_by_wavefronts(cuda, t, n_idx, r, h):
-    # above 256 tokens and with at most four splits of x's product, four tokens to a workgroup: one, two and three of them and all in the
-    # last; one, two and three splits; latent ranks past 1536 and no multiple of 256; two index heads to a lane.  The MLA outputs are the
+    # above 256 tokens and with at most eight splits of x's product (nine: a workgroup to a chain), four tokens to a workgroup: one, two and three
+    # of them and all in the last; one, two, three, five and eight splits; latent ranks past 1536 and no multiple of 256; two index heads to a lane.  The MLA outputs are the
     # bits of the separate call, whose norms are workgroups of their own
     mla_case, idx_case = op.make_fused_case(t, 1, 64, seed=130 + n_idx, n_idx=n_idx, h=h, q_lora_rank=r, n=2)
     fused = run_fused(mla_case, idx_case, cuda, entry="mla_indexer_prolog_quant_p")
