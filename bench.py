@@ -325,7 +325,7 @@ def bench_indexer_prolog(args, torch, lib, dev):
         "config": {"workload": f"lightning indexer prolog, {t} tokens, h 7168, q_lora_rank 1536, 64 x 128 index heads"
                                + (", batch 4 x 2 tokens over a 64K-token paged cache (the reference's quoted case)" if published else "")
                                + f", weights rotated over {len(sets)} copies"},
-        "roofline": {"kernel": "prolog (4 kernels)", "bound": "hbm", "achieved": round(work / total_us / 1e3, 1),
+        "roofline": {"kernel": f"prolog ({len(kernels)} kernels)", "bound": "hbm", "achieved": round(work / total_us / 1e3, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(work / total_us / 1e3 / HBM_PEAK_GBS, 4),
                      "traffic": None, "work_per_launch": work, "us_per_launch": round(total_us, 2),
                      "note": "15 MB of weights read once: bound by launch and memory latency at decode sizes"},
@@ -376,7 +376,7 @@ def bench_mla_prolog(args, torch, lib, dev):
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "int8+bf16", "data": "synthetic", "launch": "hip graph replay" if args.graph else "eager",
         "config": {"workload": f"MLA prolog (int8 form), {t} tokens, h 7168, q_lora_rank 1536, 128 heads x 192, "
                                f"kv_lora_rank 512, weights rotated over {len(sets)} copies"},
-        "roofline": {"kernel": "mla prolog (4 kernels)", "bound": "hbm", "achieved": round(work / total_us / 1e3, 1),
+        "roofline": {"kernel": f"mla prolog ({len(kernels)} kernels)", "bound": "hbm", "achieved": round(work / total_us / 1e3, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(work / total_us / 1e3 / HBM_PEAK_GBS, 4),
                      "traffic": None, "work_per_launch": work, "us_per_launch": round(total_us, 2),
                      "note": "85 MB of weights read once per call"},
@@ -432,7 +432,7 @@ def bench_mla_indexer_prolog(args, torch, lib, dev):
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "int8+bf16", "data": "synthetic", "launch": "hip graph replay" if args.graph else "eager",
         "config": {"workload": f"fused MLA + lightning-indexer prolog, {t} tokens, h 7168, q_lora_rank 1536, 128 heads x 192, "
                                f"kv_lora_rank 512, 64 x 128 index heads, weights rotated over {len(sets)} copies"},
-        "roofline": {"kernel": "fused prolog (4 kernels)", "bound": "hbm", "achieved": round(work / total_us / 1e3, 1),
+        "roofline": {"kernel": f"fused prolog ({len(kernels)} kernels)", "bound": "hbm", "achieved": round(work / total_us / 1e3, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(work / total_us / 1e3 / HBM_PEAK_GBS, 4),
                      "traffic": None, "work_per_launch": work, "us_per_launch": round(total_us, 2),
                      "note": "100 MB of weights read once per call"},
@@ -484,7 +484,7 @@ def bench_attention_pre_quant(args, torch, lib, dev):
         "dtype": "int8+bf16", "data": "synthetic", "launch": "hip graph replay" if args.graph else "eager",
         "config": {"workload": f"GLM-4.5 attention_pre_quant, {t} tokens, hidden 5120, {qh} + {kvh} + {kvh} heads of 128, "
                                f"rotary 64, weights rotated over {len(sets)} copies"},
-        "roofline": {"kernel": "attention_pre_quant (3 kernels)", "bound": "hbm", "achieved": round(work / total_us / 1e3, 1),
+        "roofline": {"kernel": f"attention_pre_quant ({len(kernels)} kernels)", "bound": "hbm", "achieved": round(work / total_us / 1e3, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(work / total_us / 1e3 / HBM_PEAK_GBS, 4),
                      "traffic": None, "work_per_launch": work, "us_per_launch": round(total_us, 2),
                      "note": f"{h * n_out / 1e6:.1f} MB of weights read once: bound by launch and memory latency at decode sizes"},
