@@ -14,7 +14,7 @@
 // At decode sizes (8 - 64 tokens) the operator reads 9 MB of int8 weights once (hidden 5120 x 1792 outputs) and is bound by
 // launch latency and that read; three launches:
 //   apq_norm_kernel   one workgroup per token: the row is read once and stays in registers across the sum (up to 4 tokens part of the next:
-//                     apq_norm_gemm_kernel)
+//                     apq_norm_gemm_kernel; up to 160 a workgroup per 256 pieces of a row: apq_norm_pieces_kernel)
 //   apq_gemm_kernel   one workgroup per (128 outputs, 256 to 1024 contraction rows, 32 tokens): the weight tile (output
 //                     dimension contiguous in memory) is loaded in one go, parked in LDS and read back with 8-bit
 //                     transposing reads as the A operand of the int8 MFMA; int32 partial sums to the workspace (exact,
@@ -113,6 +113,74 @@ __global__ __launch_bounds__(256) void apq_norm_kernel(AttnPreArgs a)
         }
         *reinterpret_cast<u32x2*>(a.x_q + (int64_t)tok * a.h + 8 * (tid + 256 * i)) = __builtin_bit_cast(u32x2, q);
     }
+}
+
+// Eight columns of the sums (bf16, `sums`) and of the quantised row: what apq_norm_kernel does with a piece, of which these are the operands.
+__device__ __forceinline__ u32x2 norm_piece(u32x4 x, u32x4 r, u32x4 gamma, u32x4 bias, u32x4 scale, u32x4 offset, float denom, u32x4& sums)
+{
+#pragma clang fp contract(off)
+    int8_t q[8];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        float s2[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int sh = e * 16;
+            s2[e] = bf16_bits_to_f32((r[w] >> sh) & 0xffffu) + bf16_bits_to_f32((x[w] >> sh) & 0xffffu);
+            const float ga = bf16_bits_to_f32((gamma[w] >> sh) & 0xffffu), b = bf16_bits_to_f32((bias[w] >> sh) & 0xffffu);
+            const float sc = bf16_bits_to_f32((scale[w] >> sh) & 0xffffu), of = bf16_bits_to_f32((offset[w] >> sh) & 0xffffu);
+            const float xn = round_bf16((s2[e] / denom) * ga + b);
+            const float v = __builtin_rintf(xn * sc + of);
+            q[2 * w + e] = (int8_t)(int)fminf(fmaxf(v, -128.f), 127.f);
+        }
+        sums[w] = pack_bf16x2(s2[0], s2[1]);
+    }
+    return __builtin_bit_cast(u32x2, q);
+}
+
+// The same with a workgroup to every 256 pieces of a token's row (norm_in_pieces): each adds up the whole row for itself, in the order
+// above, and normalises its own piece a lane.  What bounds the kernel above at few tokens is one CU's vector issue: of a
+// wavefront's 750 instructions 600 are the 20 to 24 columns that a lane normalises one piece behind the other.
+// grid (tokens, pieces / 256 rounded up), 256 lanes
+template <int NP>
+__global__ __launch_bounds__(256) void apq_norm_pieces_kernel(AttnPreArgs a)
+{
+#pragma clang fp contract(off)
+    __shared__ float red[4];
+    const int tok = blockIdx.x, tid = threadIdx.x, npieces = a.h / 8, own = tid + 256 * blockIdx.y, oc = min(own, npieces - 1);
+    const u32x4* xrow = reinterpret_cast<const u32x4*>(a.x + (int64_t)tok * a.h);
+    const u32x4* rrow = reinterpret_cast<const u32x4*>(a.residual + (int64_t)tok * a.h);
+    u32x4 xr[NP], rr[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const int pc = min(tid + 256 * i, npieces - 1);
+        xr[i] = xrow[pc];
+        rr[i] = rrow[pc];
+    }
+    const u32x4 ox = xrow[oc], orr = rrow[oc], g = reinterpret_cast<const u32x4*>(a.gamma)[oc], b = reinterpret_cast<const u32x4*>(a.bias)[oc];
+    const u32x4 sc = reinterpret_cast<const u32x4*>(a.in_scale)[oc], of = reinterpret_cast<const u32x4*>(a.in_offset)[oc];
+    __builtin_amdgcn_sched_barrier(0); // (every load is out)
+    float part = 0.f;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const bool live = tid + 256 * i < npieces;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float lo = bf16_bits_to_f32(rr[i][e] & 0xffffu) + bf16_bits_to_f32(xr[i][e] & 0xffffu);
+            const float hi = bf16_bits_to_f32(rr[i][e] >> 16) + bf16_bits_to_f32(xr[i][e] >> 16);
+            if (live) {
+                part += (lo * lo) * a.mean_coff;
+                part += (hi * hi) * a.mean_coff;
+            }
+        }
+    }
+    const float denom = sqrtf(block_sum_256(part, red, tid) + a.eps);
+    if (own >= npieces) return;
+    u32x4 sums;
+    const u32x2 q = norm_piece(ox, orr, g, b, sc, of, denom, sums);
+    const int64_t at = (int64_t)tok * npieces + own;
+    reinterpret_cast<u32x4*>(a.residual_out)[at] = sums;
+    reinterpret_cast<u32x2*>(a.x_q)[at] = q;
 }
 
 // ------------------------------------------------------------------------------------------------ int8 projection
@@ -278,28 +346,13 @@ __global__ __launch_bounds__(256 * G) void apq_norm_gemm_kernel(AttnPreArgs a)
     for (int i = 0; i < OWN; ++i) {
         if (otok[i] >= T) continue;
         const float denom = sqrtf(((red[otok[i]][0] + red[otok[i]][1]) + (red[otok[i]][2] + red[otok[i]][3])) + a.eps);
-        int8_t q[8];
         u32x4 ro;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            float s2[2];
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int sh = e * 16;
-                s2[e] = bf16_bits_to_f32((orr[i][w] >> sh) & 0xffffu) + bf16_bits_to_f32((ox[i][w] >> sh) & 0xffffu);
-                const float ga = bf16_bits_to_f32((gr[i][w] >> sh) & 0xffffu), b = bf16_bits_to_f32((br[i][w] >> sh) & 0xffffu);
-                const float sc = bf16_bits_to_f32((sr[i][w] >> sh) & 0xffffu), of = bf16_bits_to_f32((fr[i][w] >> sh) & 0xffffu);
-                const float xn = round_bf16((s2[e] / denom) * ga + b);
-                const float v = __builtin_rintf(xn * sc + of);
-                q[2 * w + e] = (int8_t)(int)fminf(fmaxf(v, -128.f), 127.f);
-            }
-            ro[w] = pack_bf16x2(s2[0], s2[1]);
-        }
-        *reinterpret_cast<u32x2*>(ql + otok[i] * QROW + 8 * (opc[i] - split * PIECES)) = __builtin_bit_cast(u32x2, q);
+        const u32x2 q = norm_piece(ox[i], orr[i], gr[i], br[i], sr[i], fr[i], denom, ro);
+        *reinterpret_cast<u32x2*>(ql + otok[i] * QROW + 8 * (opc[i] - split * PIECES)) = q;
         if (blockIdx.x == 0 && otok[i] < a.t && opc[i] < npieces) {
             const int64_t at = (int64_t)otok[i] * npieces + opc[i];
             reinterpret_cast<u32x4*>(a.residual_out)[at] = ro;
-            reinterpret_cast<u32x2*>(a.x_q)[at] = __builtin_bit_cast(u32x2, q);
+            reinterpret_cast<u32x2*>(a.x_q)[at] = q;
         }
     }
     i32x4 acc[DB]; // wave w: outputs [16 DB w, +16 DB)
@@ -900,6 +953,14 @@ static bool norm_in_projection(const AttnPreArgs& a)
     return a.t <= 4 && a.h <= 3 * 2048 && rows_apart(a) && attention_pre_kernel(a.t, a.n_out) == ApqKernel::stream;
 }
 
+// A workgroup to a token leaves CUs idle at few tokens: pieces on workgroups of their own up to 160 (us a call, three sets of operands, hidden 5120, a workgroup to
+// a token / to 256 pieces: 14 heads, 16 tokens 14.1 / 13.6, 32: 16.1 / 15.3, 64: 18.7 / 17.9, 160: 21.6 / 21.2, 200: 23.0 / 23.0, 256: 23.6 / 23.6, 777: 37.4 / 38.9;
+// 28 heads, 8: 15.2 / 14.3, 32: 18.1 / 17.4, 128: 23.8 / 22.9; 112 heads, 8: 23.2 / 22.4, 64: 26.5 / 25.3, 160: 37.5 / 36.6, 256: 45.9 / 45.8, 1024: 82.1 / 83.9).
+static bool norm_in_pieces(const AttnPreArgs& a)
+{
+    return a.t <= 160 && a.h > 2048 && a.h <= 3 * 2048 && rows_apart(a);
+}
+
 hipError_t attention_pre_launch(const AttnPreArgs& a, hipStream_t stream)
 {
     if (a.t == 0) return hipSuccess;
@@ -908,7 +969,9 @@ hipError_t attention_pre_launch(const AttnPreArgs& a, hipStream_t stream)
     if (!together)
     {
         ScopedKernelTimer tm(KID_APQ_NORM, stream);
-        if (a.h <= 3 * 2048)
+        if (norm_in_pieces(a))
+            hipLaunchKernelGGL(apq_norm_pieces_kernel<3>, dim3(a.t, (a.h / 8 + 255) / 256), dim3(256), 0, stream, a);
+        else if (a.h <= 3 * 2048)
             hipLaunchKernelGGL(apq_norm_kernel<3>, dim3(a.t), dim3(256), 0, stream, a);
         else
             hipLaunchKernelGGL(apq_norm_kernel<AMAX_H / 2048>, dim3(a.t), dim3(256), 0, stream, a);

@@ -244,6 +244,23 @@ def test_norm_in_the_projection(cuda, t, h, q_heads, kv_heads):
         assert torch.equal(on[place].cpu(), got["residual_res"]), place
 
 
+@pytest.mark.parametrize("t,h,q_heads", [(5, 2304, 2), (6, 2048, 2), (7, 4096, 3), (9, 4352, 12), (160, 6144, 12), (161, 5120, 2), (33, 5888, 24)])
+def test_norm_by_pieces(cuda, t, h, q_heads):
+    """5 to 160 tokens of hidden 2304 to 6144: a row's pieces on two and three workgroups, the last one short and whole; in place of an input
+    a workgroup has the row, the same bits."""
+    case = op.make_case(t, h=h, q_heads=q_heads, kv_heads=1, seed=t + h)
+    got = run(case, cuda)
+    check(case, got)
+    from pypto_amd.glm_v4_5 import glm_attention_pre_quant as impl
+    for place in ("hidden_states", "residual"):
+        on = {k: case[k].to(cuda) for k in NAMES}
+        out = outputs(case, cuda)
+        impl.attention_pre_quant(*[on[k] for k in NAMES], out["query"], out["key"], out["value"], on[place])
+        for name in ("query", "key", "value"):
+            assert torch.equal(out[name].cpu(), got[name]), (place, name)
+        assert torch.equal(on[place].cpu(), got["residual_res"]), place
+
+
 def test_saturation_at_both_ends(cuda):
     """A quantisation scale of 1000: nine in ten values of the quantised row are clamped at -128 or 127."""
     case = op.make_case(4, h=4096, q_heads=2, kv_heads=1, seed=14)
