@@ -46,6 +46,9 @@ SfaSplits sfa_pick_splits(int t, int nq, int topk, uint64_t scratch); // scratch
 uint64_t sfa_workspace_bytes(int t, int nq, const SfaSplits& splits);
 uint64_t sfa_partials_bytes(int t, int nq, const SfaSplits& splits); // the partial results at the front of that workspace; (m, l) follow
 hipError_t sfa_launch(const SfaArgs& a, hipStream_t stream);
+// The merge of n > 8 splits of the tokens from token0 on (sfa_launch).  Heads of a workgroup of the attention kernels, value columns.
+constexpr int SFA_HEADS_PER_WG = 128, SFA_DN = 512;
+hipError_t sfa_combine_many_launch(const SfaArgs& a, int n, int token0, hipStream_t stream);
 // Device address, on the current device, of the library's own scratch array of SFA_STATIC_SCRATCH_BYTES bytes (looked up
 // once per device).  Every call on a GPU shares that GPU's array.
 constexpr uint64_t SFA_STATIC_SCRATCH_BYTES = 40ull << 20;
