@@ -856,7 +856,10 @@ __device__ __forceinline__ void mla_qb_body(const MlaPrologArgs& a, int tile, ui
 
 // Up to 32 tokens and one workgroup to a CU (head_units): a head's 128 first dims of q_b in one workgroup, which goes on to
 // the absorbed product with the head's w_uk, whose 128 KB follow the other weights through the same stages; the rotary dims of two heads
-// in another.  The three workgroups of two heads, which share cache lines of the int8 weights, go to one XCD.
+// in another.  The three workgroups of two heads, which share cache lines of the int8 weights, go to one XCD, in the last of the rounds of eight pairs too,
+// whose other workgroups have nothing to do (int8 form, us a call of 8 tokens with the last pairs' workgroups side by side / so: 100 heads 23.4 / 21.0, 120:
+// 25.3 / 21.8, 170: 28.2 / 26.5; fused, 126 heads 30.3 / 25.0).  The bf16 form's share none: 170 heads 29.5 side by side, 35.5 so, with 33 workgroups
+// to some XCDs' 32 CUs.
 // A kernel of its own for the absorbed product, 512 workgroups behind a launch and a round trip of q_b through memory, took 4.2 to 5 us.
 constexpr int WUK_CHUNKS = MC / 64; // stages of w_uk: 128 rows x 64 columns
 struct HeadUnit {
@@ -865,10 +868,12 @@ struct HeadUnit {
 };
 __device__ __forceinline__ HeadUnit head_unit(const MlaPrologArgs& a, int id)
 {
-    const bool even = a.n % 16 == 0; // (whole rounds of the XCDs)
-    const int pair = even ? id / 24 * 8 + id % 8 : id / 3, k = even ? id / 8 % 3 : id % 3;
+    const bool rounds = a.quant || a.n % 16 == 0; // of the XCDs, a pair to each
+    const int pair = rounds ? id / 24 * 8 + id % 8 : id / 3, k = rounds ? id / 8 % 3 : id % 3;
+    if (2 * pair >= a.n) return HeadUnit{-1, 0, 0, false}; // none
     return k < 2 ? HeadUnit{2 * pair + k, (2 * pair + k) * MQH, 0, true} : HeadUnit{2 * pair, 2 * pair * MQH + MNOPE, MQH - 64, false};
 }
+__host__ __device__ inline int head_grid(const MlaPrologArgs& a) { return a.quant ? 24 * ((a.n + 15) / 16) : a.n * MQH / 128; }
 struct Absorbed { // wave w: columns 32 (w % 2) of the chunks 2 i + w / 2
     static constexpr int TILE = 2 * MTOK * QBS_ROW, OROW = MC * 2 + 16; // bytes of q_b's tile, of an LDS row of the outputs
     f32x16 acc[WUK_CHUNKS / 2];
@@ -933,6 +938,7 @@ __device__ __forceinline__ void mla_head_body(const MlaPrologArgs& a, int id, ui
 {
     using S = GtStream;
     const HeadUnit u = head_unit(a, id);
+    if (u.head < 0) return; // (uniform)
     uint8_t* tile = lds + S::LDS;
     QbScales scales;
     i32x4 acc[2][2] = {};
@@ -966,7 +972,7 @@ __device__ __forceinline__ void mla_head_body(const MlaPrologArgs& a, int id, ui
         qb_store_blocks<MTOK>(a, tile, 3 * u.head + 2, 0, 3);
     }
 }
-// grid (n * 192 / 128), 256 lanes
+// grid (head_grid), 256 lanes
 template <bool QUANT>
 __global__ __launch_bounds__(256) void mla_head_kernel(MlaPrologArgs a)
 {
@@ -997,6 +1003,7 @@ __device__ __forceinline__ void mla_touch(const MlaPrologArgs& a, int tile, int 
     const int64_t stride = (int64_t)a.n * MQH * value;
     const int rows = min(a.r, bytes / (16 * pieces)) & ~31;
     const HeadUnit u = heads ? head_unit(a, tile) : HeadUnit{0, 128 * tile, 0, true};
+    if (u.head < 0) return;
     touch_rows(static_cast<const uint8_t*>(a.w_uq_qr) + (int64_t)u.col0 * value, stride, rows, pieces, u.gap * value);
 }
 
@@ -1402,7 +1409,7 @@ __global__ __launch_bounds__(256) void fused_norm_kernel(MlaPrologArgs m, Prolog
         if (threadIdx.x >= 128) return; // the barriers inside are among the two remaining waves
         prolog_k_body<S>(p, id - 2 * m.t);
     } else if (TOUCH && id >= first) {
-        const int tile = id - first, nqb = m.n * MQH / 128;
+        const int tile = id - first, nqb = heads ? head_grid(m) : m.n * MQH / 128;
         if (tile < nqb)
             mla_touch(m, tile, touch, heads);
         else
@@ -1426,7 +1433,7 @@ __global__ __launch_bounds__(256) void fused_qb_kernel(MlaPrologArgs m, PrologAr
 __global__ __launch_bounds__(256) void fused_head_kernel(MlaPrologArgs m, PrologArgs p)
 {
     __shared__ __align__(16) uint8_t lds[PROLOG_STREAM_LDS > HEAD_LDS ? PROLOG_STREAM_LDS : HEAD_LDS];
-    const int nqb = m.n * MQH / 128;
+    const int nqb = head_grid(m);
     if ((int)blockIdx.x < nqb)
         mla_head_body<true>(m, blockIdx.x, lds);
     else
@@ -1835,7 +1842,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         const int norms = (p ? 3 : 2) * a.t, first = (norms + 7) / 8 * 8;
         const int slices = a.n * MQH / 128 + (p ? p->n : 0), bytes = touch_bytes(slices, p != nullptr);
         const bool ahead = !big && bytes >= 32 * 256; // (32 rows; the kernels above BIG_T tokens do not wait for their weights)
-        const unsigned grid = ahead ? first + slices : norms;
+        const unsigned grid = ahead ? first + (heads ? head_grid(a) + (p ? p->n : 0) : slices) : norms;
         auto launch = [&](auto splits, auto touch) {
             constexpr int S = decltype(splits)::value;
             constexpr bool TOUCH = decltype(touch)::value;
@@ -1879,9 +1886,9 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
         ScopedKernelTimer tm(KID_MLA_QB, stream);
         if (heads && !big) {
             if (p)
-                hipLaunchKernelGGL(fused_head_kernel, dim3(a.n * MQH / 128 + p->n), dim3(256), 0, stream, a, *p);
+                hipLaunchKernelGGL(fused_head_kernel, dim3(head_grid(a) + p->n), dim3(256), 0, stream, a, *p);
             else
-                hipLaunchKernelGGL((a.quant ? mla_head_kernel<true> : mla_head_kernel<false>), dim3(a.n * MQH / 128), dim3(256), 0, stream, a);
+                hipLaunchKernelGGL((a.quant ? mla_head_kernel<true> : mla_head_kernel<false>), dim3(head_grid(a)), dim3(256), 0, stream, a);
         } else if (!a.quant && heads && a.t <= BATCH16_T && a.n * MQH / 128 <= 256) {
             token_blocks(a.t, [&](auto tt) {
                 hipLaunchKernelGGL(mla_heads16_batch_kernel<std::clamp(decltype(tt)::value, 2, 4)>, dim3(a.n * MQH / 128), dim3(GT_LANES), 0, stream, a);

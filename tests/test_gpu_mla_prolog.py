@@ -270,6 +270,45 @@ def test_absorbed_product_behind_the_query_product(cuda, t, n, r, quant_b):
         check_bf16_form(case, got, outliers=1e-4)
 
 
+def us_of_calls(dev, t, counts, quant_b=True):
+    """us of a call with each of these numbers of heads, measured in turn: the shortest of several rows of calls."""
+    from pypto_amd.deepseek_v32_exp import mla_prolog_quant_impl as impl
+    h, r, bf = 1024, 1536, torch.bfloat16
+    g = torch.Generator(device=dev).manual_seed(7)
+    uni = lambda *shape: torch.empty(shape, device=dev).uniform_(-0.1, 0.1, generator=g)  # noqa: E731
+    calls = []
+    for n in counts:
+        w = uni(r, n * 192)
+        z = lambda *shape, dt=bf: torch.zeros(shape, dtype=dt, device=dev)  # noqa: E731
+        narrow = torch.int8 if quant_b else bf
+        kv, kr, ks = z(2 * t, 128, 1, 512, dt=narrow), z(2 * t, 128, 1, 64), z(2 * t, 128, 1, 4, dt=torch.float32)
+        args = [uni(t, h).to(bf), uni(h, r).to(bf), (w * 1270).to(torch.int8) if quant_b else w.to(bf),
+                torch.full((n * 192 if quant_b else 0, 1), 1e-3, device=dev), uni(n, 128, 512).to(bf), uni(h, 576).to(bf), uni(r).to(bf),
+                uni(512).to(bf), uni(t, 64).to(bf), uni(t, 64).to(bf), torch.arange(t, device=dev), kv, kr, ks, z(t, r, dt=narrow),
+                z(t, 1, dt=torch.float32), z(t, n, 512), z(t, n, 64), kv, kr, ks, EPS, EPS, "PA_BSND", impl.MlaTileConfig(),
+                impl.RopeTileShapeConfig(two_dim=[32, 64], three_dim=[32, 32, 128], four_dim=[16, 128, 128, 128])]
+        calls.append(lambda args=args: impl.mla_prolog_quant_d(*args))
+    best = [float("inf")] * len(calls)
+    for _ in range(8):
+        for i, call in enumerate(calls):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            call()
+            start.record()
+            for _ in range(25):
+                call()
+            end.record()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], start.elapsed_time(end) * 40)
+    return best
+
+
+def test_fewer_heads_of_a_decode_batch_take_no_longer(cuda):
+    """120 heads are seven and a half rounds of the eight XCDs: with pairs of heads spread over several XCDs they took 13 % longer than
+    128, whose pairs each have one."""
+    few, many = us_of_calls(cuda, 8, (120, 128))
+    assert few < 1.05 * many, (few, many)
+
+
 @pytest.mark.parametrize("t,n,r", [(65, 96, 128), (96, 170, 384), (160, 98, 128), (161, 150, 128), (192, 300, 128), (300, 128, 1536), (385, 128, 128), (512, 128, 256)])
 def test_absorbed_product_behind_tiles(cuda, t, n, r):
     # 128 outputs of a head and all tokens to a workgroup; two heads and tiles of 128 to 256 tokens, with and without whole groups of four heads
