@@ -1234,21 +1234,40 @@ __device__ __forceinline__ void mla_heads_wide_body(const MlaPrologArgs& a, int 
         ab.multiply<2 * TB, true>(a, 2 * unit + h, tok0, lds + h * T::TOK * AbsorbedWide::ROW);
     }
 }
-// Workgroup id's unit where n1 long units go out among n2 short ones, eight of a kind at a time (an XCD each), `share` / 256 of the
-// groups long ones while they last.  kind -1: none.  Up to two rounds of workgroups long ones first (fused, 612 tokens: evenly mixed 97.1 us, two
-// thirds 95.8, all first 91.4; int8 form 512 tokens 79.4 / 79.4 / 71.8 in tiles of 128); in more, some short ones among them, so that not all CUs
-// store at the same time (1501 tokens 187.6 evenly mixed, 180.2 with 170, 174.4 with 210, 178.9 with 256; 1200: 176.6, 155.6, 158.0, 162.3).
+// Workgroup id's unit where n1 long units go out among n2 short ones: all of them first (share 256; grid n1 + n2, so that every XCD gets as many
+// workgroups), or eight of a kind at a time (an XCD each), `share` / 256 of the groups long ones while they last (grid wide_grid).  kind -1: none.  Up to
+// two rounds of workgroups long ones first (fused, 612 tokens: evenly mixed 97.1 us, two thirds 95.8, all first 91.4; int8 form 512 tokens 79.4 / 79.4 /
+// 71.8 in tiles of 128); in more, some short ones among them, so that not all CUs store at the same time.  How many matters little: of 256, with 170 / 210
+// / 256, three sets of operands in turn, fused, 900 tokens 128.4 / 128.9 / 128.7, 1200: 168.8 / 167.2 / 169.5, 1501: 188.3 / 186.0 / 186.3; int8 form 1501: 174.5 /
+// 169.2 / 169.2; bf16 form 700: 138.5 / 131.6 / 132.1, 900: 164.3 / 162.8 / 154.7, 1200: 212.4 / 204.5 / 201.6 (runs of one differ by 1 %).
 struct WideUnit {
     int kind, at;
 };
 __device__ __forceinline__ WideUnit wide_unit(int id, int n1, int n2, int share)
 {
+    if (share == 256) return id < n1 ? WideUnit{0, id} : WideUnit{1, id - n1};
     const int g1 = (n1 + 7) / 8, g2 = (n2 + 7) / 8, j = id / 8;
     auto firsts = [&](int k) { return max(k - g2, min(g1, (k * share + 255) / 256)); };
     const int before = firsts(j);
     const bool first = firsts(j + 1) > before;
     const int at = 8 * (first ? before : j - before) + id % 8;
     return {at >= (first ? n1 : n2) ? -1 : first ? 0 : 1, at};
+}
+inline int wide_share(int n1, int n2) { return n1 + n2 <= 512 ? 256 : 210; }
+inline unsigned wide_grid(int n1, int n2) { return wide_share(n1, n2) == 256 ? n1 + n2 : 8 * ((n1 + 7) / 8 + (n2 + 7) / 8); }
+
+// Number `at` of units x rows of tiles: whole rounds of the XCDs keep a unit, and its weights, on one of them in all rows; the tiles of the units left over
+// go to all.  (In row order 65 or 85 units are on other XCDs in every row, and rounded up to eights the workgroups of one round are more than some
+// XCDs have CUs: 170 heads, int8 form 256 tokens 68.8 us a call, 57.5 this way, bf16 form 512 tokens 133 / 114; 130 heads, int8 form 700: 118.8 / 100.9,
+// fused 257: 81.2 / 69.3.)
+struct WidePlace {
+    int unit, row;
+};
+__device__ __forceinline__ WidePlace wide_place(int at, int units, int rows)
+{
+    const int most = units & ~7, left = units - most, b = at - most * rows;
+    if (b < 0) return {at % most, at / most};
+    return {most + b % left, b / left};
 }
 
 // The bf16 form by the same units: 33 to 128 tokens beside a head's first dims or two heads' rotary dims, the weights streamed (gt_batch_bf16);
@@ -1289,7 +1308,7 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_heads16_batch_kernel(MlaProlo
 
 // More tokens: tiles of 128 tokens x two heads' first dims or four heads' rotary dims (mla_qb16_wide_kernel's product).  Three sets of operands in
 // turn: 200 tokens 64.5 -> 61.8 us, 289: 92.0 -> 81.3, 384: 98.7 -> 84.5, 512: 107.9 -> 103.4, 1024: 175.2 -> 174.0 (one set 176.7 -> 168.5).
-// grid (groups of eight units of wide_unit), 512 lanes
+// grid (wide_grid), 512 lanes
 __global__ __launch_bounds__(GT_LANES, 2) void mla_heads16_wide_kernel(MlaPrologArgs a, int share)
 {
     using T = GtTile<4>;
@@ -1300,7 +1319,8 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_heads16_wide_kernel(MlaProlog
     const WideUnit u = wide_unit(blockIdx.x, nab * rows, nro * rows, share);
     if (u.kind < 0) return;
     const bool rope = u.kind == 1;
-    const int per = rope ? nro : nab, unit = u.at % per, tok0 = u.at / per * T::TOK;
+    const WidePlace place = wide_place(u.at, rope ? nro : nab, rows);
+    const int unit = place.unit, tok0 = place.row * T::TOK;
     const uint16_t* src[4];
     int ld[4];
 #pragma unroll
@@ -1476,7 +1496,7 @@ __global__ __launch_bounds__(GT_LANES, 2) void fused_qb_wide_kernel(MlaPrologArg
     }
 }
 
-// The same with the absorbed products behind the heads' first dims, and alone.  grid (groups of eight units of wide_unit), 512 lanes
+// The same with the absorbed products behind the heads' first dims, and alone.  grid (wide_grid), 512 lanes
 template <int TB>
 __global__ __launch_bounds__(GT_LANES, 2) void fused_heads_wide_kernel(MlaPrologArgs m, PrologArgs p, int share)
 {
@@ -1485,14 +1505,14 @@ __global__ __launch_bounds__(GT_LANES, 2) void fused_heads_wide_kernel(MlaProlog
     const int nqt = (p.n + 1) / 2, nab = m.n / 2, nro = (m.n + 3) / 4, rows = (m.t + 32 * TB - 1) / (32 * TB);
     const WideUnit u = wide_unit(blockIdx.x, nab * rows, (nqt + nro) * rows, share);
     if (u.kind < 0) return;
+    const bool rope = u.kind == 1 && u.at >= nqt * rows;
+    const WidePlace place = wide_place(rope ? u.at - nqt * rows : u.at, u.kind == 0 ? nab : rope ? nro : nqt, rows);
     if (u.kind == 0)
-        mla_heads_wide_body<TB>(m, u.at % nab, false, u.at / nab * 32 * TB, lds);
-    else if (u.at < nqt * rows)
-        prolog_q_wide_body<TB>(p, 2 * (u.at % nqt), u.at / nqt * 32 * TB, lds);
-    else {
-        const int id = u.at - nqt * rows;
-        mla_heads_wide_body<TB>(m, id % nro, true, id / nro * 32 * TB, lds);
-    }
+        mla_heads_wide_body<TB>(m, place.unit, false, place.row * 32 * TB, lds);
+    else if (!rope)
+        prolog_q_wide_body<TB>(p, 2 * place.unit, place.row * 32 * TB, lds);
+    else
+        mla_heads_wide_body<TB>(m, place.unit, true, place.row * 32 * TB, lds);
 }
 template <int TB>
 __global__ __launch_bounds__(GT_LANES, 2) void mla_heads_wide_kernel(MlaPrologArgs a, int share)
@@ -1501,8 +1521,8 @@ __global__ __launch_bounds__(GT_LANES, 2) void mla_heads_wide_kernel(MlaPrologAr
     const int nab = a.n / 2, nro = (a.n + 3) / 4, rows = (a.t + 32 * TB - 1) / (32 * TB);
     const WideUnit u = wide_unit(blockIdx.x, nab * rows, nro * rows, share);
     if (u.kind < 0) return;
-    const int per = u.kind == 0 ? nab : nro;
-    mla_heads_wide_body<TB>(a, u.at % per, u.kind == 1, u.at / per * 32 * TB, lds);
+    const WidePlace place = wide_place(u.at, u.kind == 0 ? nab : nro, rows);
+    mla_heads_wide_body<TB>(a, place.unit, u.kind == 1, place.row * 32 * TB, lds);
 }
 
 // ------------------------------------------------------------------------------------------------ q_b[:, head, :128] @ w_uk[head]
@@ -1895,8 +1915,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
             });
         } else if (!a.quant && heads) {
             const int rows = (a.t + 127) / 128, first = a.n / 2 * rows, second = (a.n + 3) / 4 * rows;
-            hipLaunchKernelGGL(mla_heads16_wide_kernel, dim3(8 * ((first + 7) / 8 + (second + 7) / 8)), dim3(GT_LANES), 0, stream, a,
-                               first + second <= 512 ? 256 : 210);
+            hipLaunchKernelGGL(mla_heads16_wide_kernel, dim3(wide_grid(first, second)), dim3(GT_LANES), 0, stream, a, wide_share(first, second));
         } else if (!a.quant && big) {
             hipLaunchKernelGGL(mla_qb16_wide_kernel, dim3((a.n * MQH + 255) / 256, (a.t + 127) / 128), dim3(GT_LANES), 0, stream, a);
         } else if (!a.quant) {
@@ -1922,8 +1941,8 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
                 gt_dispatch(heads_token_blocks(a, p), [&](auto tb) {
                     constexpr int TB = decltype(tb)::value;
                     const int rows = (a.t + 32 * TB - 1) / (32 * TB), first = a.n / 2 * rows, second = ((a.n + 3) / 4 + qcols) * rows;
-                    const int share = first + second <= 512 ? 256 : 210;
-                    const dim3 grid(8 * ((first + 7) / 8 + (second + 7) / 8));
+                    const int share = wide_share(first, second);
+                    const dim3 grid(wide_grid(first, second));
                     if (p)
                         hipLaunchKernelGGL(fused_heads_wide_kernel<TB>, grid, dim3(GT_LANES), 0, stream, a, *p, share);
                     else
