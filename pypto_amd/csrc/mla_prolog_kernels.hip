@@ -1780,28 +1780,41 @@ static bool qb_batch(const MlaPrologArgs& a, const PrologArgs* p)
     return p ? a.t <= 128 || (slices > 172 && slices <= 256) : slices <= 256;
 }
 
-// Up to 32 tokens the absorbed product behind the head's query product, while that is a workgroup to a CU (us a call, two kernels / one,
-// warm weights: fused, 1 token 27.1 / 24.7, 8: 28.5 / 26.0, 32: 30.1 / 27.5, of 16 heads 23.1 / 21.6; bf16 form, 24 tokens 29.8 / 27.6, out
-// of HBM 36.0 / 33.9, of 16 heads 23.3 / 22.4; int8 form, 8 tokens 23.8 / 22.3, out of HBM 28.4 / 28.2).  The int8 form of few heads has short
-// streams behind each other: of 16 19.8 / 20.0, 32: 20.0 / 20.5, 64: 20.7 / 20.7.
+// Where the absorbed product goes behind the heads' query product.  All figures us a call, two kernels / one; "warm": the same weights call after call, else three
+// sets of them in turn, as a stack of layers has it.  Where the two disagree the sets in turn decide.
 //
-// From 33 to QB_BATCH_T tokens, one workgroup to a CU still, the first weights of the absorbed product are fetched ahead of the stream of the
-// others (three sets of operands in turn, us a call, two kernels / one: fused, 33 tokens 36.0 / 33.7, 64: 39.3 / 36.6, 96: 46.4 / 41.8; one set, 48
-// tokens 31.6 / 31.4, 96: 38.6 / 36.4, 128: 42.7 / 39.1, 160: 50.4 / 44.0, of 16 heads 64: 27.9 / 26.0; int8 form, three sets, 48 tokens 29.8 / 29.7,
-// 96: 37.6 / 36.3, one set 26.8 / 28.0 and 31.7 / 32.6, 160: 41.9 / 39.7, of 64 heads 96: 27.9 / 28.4).  In two rounds (256 heads) 128 tokens take
-// 67.2 / 67.6 fused, 58.5 / 59.8 alone.
-// Above, whole tiles of 256 outputs with it: fused, 200 tokens 55.7 / 51.4, 300: 64.4 / 56.9, 512: 83.6 / 73.3, 800: 121.0 / 111.2, 1024:
-// 142.3 / 126.2, 1501: 203.3 / 174.4; int8 form 200: 46.3 / 45.9, 512: 71.0 / 67.0, 640: 81.3 / 80.5, 1024: 126.7 / 118.1, 1501: 179.1 / 159.9.  Few heads
-// are few long workgroups: fused, 16 heads 512: 54.1 / 54.5, 700: 64.7 / 63.4; 32 heads 250: 46.4 / 47.2, 400: 54.3 / 52.8; int8 form 64 heads
-// 330: 47.1 / 47.6, 400: 50.7 / 49.8; 32 heads 512: 49.4 / 51.2, 1024: 68.0 / 66.1; bf16 form 128 heads 129: 58.2 / 58.5, 64 heads 200: 49.5 / 52.7, 512:
-// 61.6 / 60.2, 16 heads 1024: 71.9 / 74.1.
+// Up to 32 tokens while that is a workgroup to a CU (warm: fused, 1 token 27.1 / 24.7, 8: 28.5 / 26.0, 32: 30.1 / 27.5, of 16 heads 23.1 / 21.6; bf16
+// form, 24 tokens 29.8 / 27.6, out of HBM 36.0 / 33.9, of 16 heads 23.3 / 22.4; int8 form, 8 tokens 23.8 / 22.3, out of HBM 28.4 / 28.2).  The int8 form of
+// few heads has short streams behind each other: of 16 19.8 / 20.0, 32: 20.0 / 20.5, 64: 20.7 / 20.7.
+//
+// From 33 to QB_BATCH_T tokens (bf16 form BATCH16_T), one workgroup to a CU still, the first weights of the absorbed product are fetched ahead of the stream of the
+// others (fused, 33 tokens 36.0 / 33.7, 64: 39.3 / 36.6, 96: 46.4 / 41.8; warm, 48: 31.6 / 31.4, 96: 38.6 / 36.4, 128: 42.7 / 39.1, 160: 50.4 / 44.0, of
+// 16 heads 64: 27.9 / 26.0).  The int8 form from 65 tokens and 96 heads on, where the warm call gains nothing: 48 tokens 29.8 / 29.7, warm 26.8 / 28.0;
+// 65: 34.2 / 32.4, warm 30.9 / 31.3; 96: 38.0 / 35.5, warm 32.7 / 33.0; 128: 41.5 / 39.3, warm 35.8 / 35.3; 160: 48.0 / 44.8, warm 43.5 / 41.4; of 64 heads 96: 27.9
+// / 28.4.  In two rounds (256 heads) 128 tokens take 67.2 / 67.6 fused, 58.5 / 59.8 alone, bf16 form of 192 heads 64.4 / 67.1.
+//
+// Above, tiles of two heads, by heads x tokens (warm: fused, 200 tokens 55.7 / 51.4, 300: 64.4 / 56.9, 512: 83.6 / 73.3, 800: 121.0 / 111.2, 1024: 142.3 /
+// 126.2, 1501: 203.3 / 174.4; int8 form 512: 71.0 / 67.0, 640: 81.3 / 80.5, 1024: 126.7 / 118.1, 1501: 179.1 / 159.9).  Few heads are few long workgroups (warm:
+// fused, 16 heads 512: 54.1 / 54.5, 700: 64.7 / 63.4; 32 heads 250: 46.4 / 47.2, 400: 54.3 / 52.8; int8 form 64 heads 330: 47.1 / 47.6, 400: 50.7 / 49.8; 32 heads
+// 512: 49.4 / 51.2, 1024: 68.0 / 66.1; bf16 form 128 heads 129: 58.2 / 58.5, 64 heads 200: 49.5 / 52.7, 512: 61.6 / 60.2, 16 heads 1024: 71.9 / 74.1).  Near the line
+// the warm call loses what the other gains: int8 form 200 tokens 53.9 / 50.5, warm 49.0 / 48.9; 384: 69.2 / 63.3, warm 62.6 / 63.5; bf16 form 200: 64.2 / 61.9, warm 58.8
+// / 61.0; 256: 68.4 / 64.9, warm 62.1 / 62.8; 160 heads, int8 form 188: 58.1 / 53.5, warm 51.5 / 53.6; 256 heads, bf16 form 1024: 309.8 / 318.7, warm 311.4 / 305.0.
+// To 256 tokens the int8 form only of up to 160 heads, whose long and short workgroups are one round (170 heads, 188 tokens 57.2 / 57.5, warm 51.9 / 56.9, 200:
+// 61.1 / 58.7, warm 54.8 / 57.0; 192 heads, 128: 53.9 / 53.8, warm 43.8 / 47.0, 256: 71.2 / 71.8, warm 65.2 / 66.6, 257: 82.5 / 71.2; 256 heads, 128: 57.9 / 58.7,
+// warm 48.1 / 52.7, 256: 76.5 / 76.9), and the bf16 form of 161 to 170 heads, a full round of the two kernels' tiles, later (170 heads, 144 tokens 66.2 / 68.0, warm 61.8 /
+// 64.5, 180: 69.5 / 69.8, warm 62.8 / 66.4, 200: 74.0 / 71.0, warm 67.7 / 67.2; 160 heads, 160: 66.5 / 65.8, warm 61.6 / 63.1; 192 heads, 129: 86.0 / 76.3).
 static bool head_units(const MlaPrologArgs& a, const PrologArgs* p)
 {
     const int slices = a.n * MQH / 128 + (p ? p->n : 0);
+    const int64_t size = (int64_t)a.n * a.t;
     if (a.t < BIG_T) return slices <= 256 && (p || !a.quant || a.n > 64);
-    if (!a.quant) return a.t <= BATCH16_T && slices <= 256 || (int64_t)a.n * a.t >= 24000;
+    if (!a.quant) {
+        if (a.t <= BATCH16_T) return slices <= 256;
+        return size >= (a.t <= 256 && a.n > 160 && a.n <= 170 ? 32000 : 24000);
+    }
     if (qb_batch(a, p)) return slices <= 256 && (p || (a.n >= 96 && a.t > 64));
-    return (int64_t)a.n * a.t >= (p ? 10000 : 24000);
+    if (p) return size >= 10000;
+    return size >= 24000 && (a.n <= 160 || a.t > 256);
 }
 
 // Token blocks (4 to 8) of the tiles with the absorbed product behind: the end of the last of n1 long and n2 short workgroups on 256
@@ -1909,7 +1922,7 @@ static hipError_t launch_prologs(const MlaPrologArgs& a, const PrologArgs* p, hi
                 hipLaunchKernelGGL(fused_head_kernel, dim3(head_grid(a) + p->n), dim3(256), 0, stream, a, *p);
             else
                 hipLaunchKernelGGL((a.quant ? mla_head_kernel<true> : mla_head_kernel<false>), dim3(head_grid(a)), dim3(256), 0, stream, a);
-        } else if (!a.quant && heads && a.t <= BATCH16_T && a.n * MQH / 128 <= 256) {
+        } else if (!a.quant && heads && a.t <= BATCH16_T) {
             token_blocks(a.t, [&](auto tt) {
                 hipLaunchKernelGGL(mla_heads16_batch_kernel<std::clamp(decltype(tt)::value, 2, 4)>, dim3(a.n * MQH / 128), dim3(GT_LANES), 0, stream, a);
             });

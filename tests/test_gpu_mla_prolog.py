@@ -318,6 +318,26 @@ def test_absorbed_product_behind_tiles(cuda, t, n, r):
     check(case, run(case, cuda))
 
 
+@pytest.mark.parametrize("t,n,quant_b,kernels", [(128, 192, True, 2), (200, 170, True, 2), (256, 256, True, 2), (257, 192, True, 1), (200, 160, True, 1),
+                                                 (144, 170, False, 2), (200, 170, False, 1), (128, 192, False, 2), (129, 192, False, 1), (96, 170, True, 1)])
+def test_absorbed_product_where_it_is_faster(cuda, t, n, quant_b, kernels):
+    """More than 160 heads: of up to 256 tokens (bf16 form: 128, and 161 to 170 heads of up to some 190) two kernels are the faster."""
+    import ctypes
+    from pypto_amd import _runtime
+    case, lib = op.make_case(t, 1, 64, seed=190, h=256, q_lora_rank=256, n=n, quant_b=quant_b), _runtime.load_library()
+    assert lib.pto_kernel_timing_enable(1) == 0
+    try:
+        run(case, cuda)
+        ran = {}
+        for name, kid in (("query", 14), ("absorbed", 15)):
+            ms, launches = ctypes.c_double(), ctypes.c_uint64()
+            assert lib.pto_kernel_timing_read(kid, ctypes.byref(ms), ctypes.byref(launches)) == 0
+            ran[name] = launches.value
+    finally:
+        lib.pto_kernel_timing_enable(0)
+    assert ran == {"query": 1, "absorbed": kernels - 1}
+
+
 @pytest.mark.parametrize("t,n,r", [(33, 4, 256), (64, 128, 256), (65, 66, 1280), (97, 16, 512), (128, 170, 256), (188, 128, 1280), (300, 82, 256), (700, 128, 256)])
 def test_bf16_absorbed_product_behind_the_query_product(cuda, t, n, r):
     # two, three and four blocks of 32 tokens with the last ones missing, one and several groups of chains; tiles of 128 tokens, one round of
