@@ -1015,9 +1015,11 @@ int num_cus()
 // splits of these few as fill the CUs once more, where the last round takes less so.  By the time that either should take, in ns:
 // a tile (where more CUs work, the chip's clock falls: 150 workgroups 1700, 200: 1780, 256: 2030), the two ends of a workgroup, a
 // partial result's way to memory and back, the merge's launch.
-// 16 splits at most, but 32 of a single token, whose calls are launches and chains: a layer's step 57.9 us with 16, 55.6 with 32 and with
-// 64; four tokens 32.7 / 34.3 / 38.9 (partial results to write and read).  Its distance from 64 bits is less with more of them (rms 2.12e-3 with 1,
-// 2.05 with 16, 1.94 with 32: P~ is rounded relative to each split's own maximum).
+// 16 splits at most, but 32 of a single token, whose calls are launches and chains, where the tiles saved are more than the partial results to write and read
+// cost, by heads x splits: a call of 2048 rows with 16 / 32, 128 heads 18.4 / 14.9 us, 256: 18.7 / 16.7, 384: 18.9 / 18.8, 512: 20.6 / 22.1, 1024: 24.5 / 27.2; of
+// 1024 rows 14.9 / 14.1, 14.7 / 15.7, 15.1 / 17.5, 17.0 / 21.0; four tokens of 128 heads 20.2 / 21.5 (two of 2048 rows would gain, 18.2 / 16.9, not of 1024, 14.4 /
+// 15.6).  Its distance from 64 bits is less with more of them (mean of 24 calls 2.07e-3 with 16, 1.96e-3 with 32; 1024 rows 2.01, 1.72: P~ is rounded relative to
+// each split's own maximum).
 // Prefill calls of 128 heads and 2048 rows a token, one split each and so, int8 cache: 257 tokens 239 -> 159 us, 300: 244 -> 177, 360:
 // 246 -> 208, 384: 247 -> 218, 520: 370 -> 287, 640: 377 -> 348, 800: 500 -> 437; bf16 cache and packed rows within 1 us of these.
 // (With fp16 partial results 300 take 170, and 129 in two splits each 102 instead of 118 - but calls of one split a token have fp32 sums
@@ -1027,8 +1029,9 @@ SfaSplits sfa_pick_splits(int t, int nq, int topk, uint64_t scratch)
 {
     const int hgroups = (nq + HEADS_PER_WG - 1) / HEADS_PER_WG, cus = std::max(1, num_cus() / hgroups); // (of a head group)
     const int tiles = (topk + T - 1) / T;
+    const int most = t == 1 && hgroups <= 2 && 32 * hgroups <= tiles ? 32 : 16;
     auto even = [&](int n) { // no more splits than n, and no more than share the tiles as well
-        n = std::max(1, std::min({n, tiles, t == 1 ? 32 : 16}));
+        n = std::max(1, std::min({n, tiles, most}));
         const int per = (tiles + n - 1) / n;
         return (tiles + per - 1) / per;
     };

@@ -260,6 +260,16 @@ def test_a_single_token_has_up_to_32_splits(cuda):
         assert torch.equal(out, run_with_splits(case, cuda, 32))
 
 
+@pytest.mark.parametrize("nq,topk,splits", [(128, 1024, 32), (256, 1024, 16), (256, 2048, 32), (300, 2048, 16), (512, 2048, 16)])
+def test_splits_of_a_single_token_by_heads_and_rows(cuda, nq, topk, splits):
+    """32 splits where they save more tiles than their partial results cost: not of many heads, nor of one tile each for two groups of heads."""
+    case = osfa.make_case(1, nq, 1, [5000], topk=topk, seed=96, dist="bench", softmax_scale=192 ** -0.5)
+    out = run_sfa(case, cuda)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert torch.equal(out, run_with_splits(case, cuda, splits))
+        assert not torch.equal(out, run_with_splits(case, cuda, 48 - splits))
+
+
 @pytest.mark.parametrize("t,rest", [(18, 8), (17, 16), (35, 5), (16, 1), (15, 1), (9, 1)])
 def test_tokens_with_different_splits(cuda, t, rest):
     """2048 heads are 16 workgroups a token: 16 tokens fill the CUs.  With a few more, the first tokens are whole rounds of one split
