@@ -759,9 +759,10 @@ __global__ __launch_bounds__(GT_LANES, 2) void apq_gemm_big_kernel(AttnPreArgs a
 
 // ------------------------------------------------------------------------------------------------ heads
 // grid (q_heads + 2 kv_heads, tokens / 4 rounded up), 256 lanes: a wave owns a head of a token, a lane its dims l and 64 + l.
-// Latency-bound: one trip for the partial sums (S: splits whose loads are out together; in eights, and what is left over one by one, 20 splits
-// were six trips: a call of 8 tokens x 28 heads 14.2 us, 13.7 this way, GLM layer of 8 sequences 30.7 / 29.8), the rest in registers (the sum over
-// the dims adds in the order of 64-lane halves, 32, 16, .. 1 apart, then the halves).
+// Latency-bound: one or two trips for the partial sums (S: splits whose loads are out together; in eights, and what is left over one by one, 20 splits
+// were six trips: a call of 8 tokens x 28 heads 14.2 us, 13.7 this way, GLM layer of 8 sequences 30.7 / 29.8; 24 and 32 splits by 20 are loads for 40: in
+// eights / by 20 / by 16, 14 heads, 32 tokens, 24 splits 14.8 / 14.6 / 14.3, 32: 17.6 / 17.8 / 17.6, 28 heads, 8 tokens, 24: 13.6 / 12.2 / 12.0, 32: 15.1 / 15.2 /
+// 15.0, 32 tokens, 16: 13.6 / 13.3 / 13.1), the rest in registers (the sum over the dims adds in the order of 64-lane halves, 32, 16, .. 1 apart, then the halves).
 template <int S>
 __global__ __launch_bounds__(256) void apq_head_kernel(AttnPreArgs a)
 {
@@ -1014,6 +1015,8 @@ hipError_t attention_pre_launch(const AttnPreArgs& a, hipStream_t stream)
             hipLaunchKernelGGL(apq_head_kernel<4>, grid, dim3(256), 0, stream, a);
         else if (a.ksplits <= 10)
             hipLaunchKernelGGL(apq_head_kernel<10>, grid, dim3(256), 0, stream, a);
+        else if (a.ksplits <= 16 || a.ksplits > 20)
+            hipLaunchKernelGGL(apq_head_kernel<16>, grid, dim3(256), 0, stream, a);
         else
             hipLaunchKernelGGL(apq_head_kernel<20>, grid, dim3(256), 0, stream, a);
     }

@@ -261,6 +261,13 @@ def test_norm_by_pieces(cuda, t, h, q_heads):
         assert torch.equal(on[place].cpu(), got["residual_res"]), place
 
 
+@pytest.mark.parametrize("h", [256, 1024, 1280, 2560, 2816, 4096, 4352, 5120, 5376, 8192, 8448, 12544])
+def test_partial_sums_of_any_number_of_splits(cuda, h):
+    """1, 4, 5, 10, 11, 16, 17, 20, 21, 32, 33 and 49 splits of the contraction: up to one group of loads and more, whole and with a rest."""
+    case = op.make_case(6, h=h, q_heads=2, kv_heads=1, seed=h)
+    check(case, run(case, cuda))
+
+
 def test_saturation_at_both_ends(cuda):
     """A quantisation scale of 1000: nine in ten values of the quantised row are clamped at -128 or 127."""
     case = op.make_case(4, h=4096, q_heads=2, kv_heads=1, seed=14)
