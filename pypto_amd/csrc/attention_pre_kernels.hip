@@ -13,8 +13,9 @@
 //
 // At decode sizes (8 - 64 tokens) the operator reads 9 MB of int8 weights once (hidden 5120 x 1792 outputs) and is bound by
 // launch latency and that read; three launches:
-//   apq_norm_kernel   one workgroup per token: the row is read once and stays in registers across the sum (up to 4 tokens part of the next:
-//                     apq_norm_gemm_kernel; up to 160 a workgroup per 256 pieces of a row: apq_norm_pieces_kernel)
+//   apq_norm_kernel   one workgroup per token: the row is read once and stays in registers across the sum (up to 4 tokens of up to 6144 columns part of the next:
+//                     apq_norm_gemm_kernel; up to 160 of hidden 2304 to 6144 a workgroup per 256 pieces of a row: apq_norm_pieces_kernel; where
+//                     the sums take the place of an input always this one)
 //   apq_gemm_kernel   one workgroup per (128 outputs, 256 to 1024 contraction rows, 32 tokens): the weight tile (output
 //                     dimension contiguous in memory) is loaded in one go, parked in LDS and read back with 8-bit
 //                     transposing reads as the A operand of the int8 MFMA; int32 partial sums to the workspace (exact,
@@ -142,10 +143,10 @@ __device__ __forceinline__ u32x2 norm_piece(u32x4 x, u32x4 r, u32x4 gamma, u32x4
 // above, and normalises its own piece a lane.  What bounds the kernel above at few tokens is one CU's vector issue: of a
 // wavefront's 750 instructions 600 are the 20 to 24 columns that a lane normalises one piece behind the other.
 // grid (tokens, pieces / 256 rounded up), 256 lanes
-template <int NP>
 __global__ __launch_bounds__(256) void apq_norm_pieces_kernel(AttnPreArgs a)
 {
 #pragma clang fp contract(off)
+    constexpr int NP = 3; // pieces of the row per lane, for the sum
     __shared__ float red[4];
     const int tok = blockIdx.x, tid = threadIdx.x, npieces = a.h / 8, own = tid + 256 * blockIdx.y, oc = min(own, npieces - 1);
     const u32x4* xrow = reinterpret_cast<const u32x4*>(a.x + (int64_t)tok * a.h);
@@ -266,7 +267,8 @@ __global__ __launch_bounds__(256) void apq_gemm_kernel(AttnPreArgs a)
 
 // A few tokens' norm and projection in one kernel (norm_in_projection): every workgroup adds up the rows' squares for itself, beside the weights'
 // way from memory, and quantises its own columns, so that a launch of one workgroup per token goes.  The operations and their order are
-// apq_norm_kernel's, lane by lane; the first column tile's workgroups write the sums of hidden states and residual and the quantised rows.  T: most tokens,
+// apq_norm_kernel's, lane by lane; the first column tile's workgroups write the sums of hidden states and residual, and the quantised rows (no kernel reads
+// them here, but the workspace's head holds them whatever the number of tokens, and the tests compare them).  T: most tokens,
 // T / G of them to a group of 256 lanes.
 // grid (n_out / 128, splits of the contraction), 256 G lanes.
 template <int PER, int T, int G>
@@ -971,7 +973,7 @@ hipError_t attention_pre_launch(const AttnPreArgs& a, hipStream_t stream)
     {
         ScopedKernelTimer tm(KID_APQ_NORM, stream);
         if (norm_in_pieces(a))
-            hipLaunchKernelGGL(apq_norm_pieces_kernel<3>, dim3(a.t, (a.h / 8 + 255) / 256), dim3(256), 0, stream, a);
+            hipLaunchKernelGGL(apq_norm_pieces_kernel, dim3(a.t, (a.h / 8 + 255) / 256), dim3(256), 0, stream, a);
         else if (a.h <= 3 * 2048)
             hipLaunchKernelGGL(apq_norm_kernel<3>, dim3(a.t), dim3(256), 0, stream, a);
         else

@@ -550,7 +550,7 @@ __device__ __forceinline__ void mla_norm_key_body(const MlaPrologArgs& a, int to
 
 // The fused operator's norms above 256 tokens where the x product has at most eight splits: a wavefront to each of a
 // token's three chains, the sums of the workgroups above bit for bit - what they spread over four wavefronts (lane l of wave w: columns
-// l + 64 w + 256 i) are four sums of a lane here, and no barrier is passed.
+// l + 64 w + 256 i) are four sums of a lane here, and no barrier is passed.  The fused operator has the int8 form only.
 // What bounds it: the partial sums' way from memory (28 MB at 1501 tokens).  A workgroup to a chain went through barriers with
 // eight chains in flight to a CU, and every token's fetched hadamard_k's 32 KB out of the L2 in 128 loads: the kernel at 1501 tokens 15.1 us, so 11.6,
 // a call 210.7 -> 208.1, 900: 140.4 / 138.1; with five to seven splits, 218 registers, three sets of operands in turn, 257: 63.7 / 63.2, 410: 78.6 / 77.2,
@@ -619,25 +619,16 @@ __device__ __forceinline__ void mla_norm_query_wave(const MlaPrologArgs& a, int 
             x[j][e] = round_bf16(half_of(gq[j][e >> 1], e & 1) * (x[j][e] * y));
             mx = fmaxf(mx, fabsf(x[j][e]));
         }
-    if (a.quant) {
-        const float sq = quant_scale(wave_max(mx));
+    const float sq = quant_scale(wave_max(mx));
 #pragma unroll
-        for (int j = 0; j < NP; ++j) {
-            const int c = 256 * j + 4 * lane;
-            uint32_t pk = 0;
+    for (int j = 0; j < NP; ++j) {
+        const int c = 256 * j + 4 * lane;
+        uint32_t pk = 0;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(x[j][e] * sq) & 0xffu) << (8 * e);
-            if (c < r) *reinterpret_cast<uint32_t*>(a.q_norm + (int64_t)tok * r + c) = pk;
-        }
-        if (lane == 0) a.q_norm_scale[tok] = 1.0f / sq;
-    } else {
-        uint16_t* qo = reinterpret_cast<uint16_t*>(a.q_norm) + (int64_t)tok * r;
-#pragma unroll
-        for (int j = 0; j < NP; ++j) {
-            const int c = 256 * j + 4 * lane;
-            if (c < r) *reinterpret_cast<u32x2*>(qo + c) = u32x2{pack_bf16x2(x[j][0], x[j][1]), pack_bf16x2(x[j][2], x[j][3])};
-        }
+        for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)__builtin_rintf(x[j][e] * sq) & 0xffu) << (8 * e);
+        if (c < r) *reinterpret_cast<uint32_t*>(a.q_norm + (int64_t)tok * r + c) = pk;
     }
+    if (lane == 0) a.q_norm_scale[tok] = 1.0f / sq;
 }
 
 // lane l: columns l + 64 m of the 512 normalised ones, and (l < 32) the rotary pair 2 l, 2 l + 1
@@ -678,20 +669,14 @@ __device__ __forceinline__ void mla_norm_key_wave(const MlaPrologArgs& a, int to
     const float y = 1.0f / sqrtf(((ss[0] + ss[1]) + (ss[2] + ss[3])) + a.eps_ckv);
 #pragma unroll
     for (int m = 0; m < M; ++m) v[m] = round_bf16(bf16_to_f32(gk[m]) * (x[m] * y));
-    if (a.quant) {
 #pragma unroll
-        for (int g = 0; g < M / 2; ++g) { // groups of 128
-            const float sq = quant_scale(wave_max(fmaxf(fabsf(v[2 * g]), fabsf(v[2 * g + 1]))));
-            if (row_ok) {
-                a.kv_cache[row * MC + 128 * g + lane] = (int8_t)(int)__builtin_rintf(v[2 * g] * sq);
-                a.kv_cache[row * MC + 128 * g + 64 + lane] = (int8_t)(int)__builtin_rintf(v[2 * g + 1] * sq);
-                if (lane == 0) a.k_scale_cache[row * 4 + g] = 1.0f / sq;
-            }
+    for (int g = 0; g < M / 2; ++g) { // groups of 128
+        const float sq = quant_scale(wave_max(fmaxf(fabsf(v[2 * g]), fabsf(v[2 * g + 1]))));
+        if (row_ok) {
+            a.kv_cache[row * MC + 128 * g + lane] = (int8_t)(int)__builtin_rintf(v[2 * g] * sq);
+            a.kv_cache[row * MC + 128 * g + 64 + lane] = (int8_t)(int)__builtin_rintf(v[2 * g + 1] * sq);
+            if (lane == 0) a.k_scale_cache[row * 4 + g] = 1.0f / sq;
         }
-    } else if (row_ok) {
-        uint16_t* kvo = reinterpret_cast<uint16_t*>(a.kv_cache) + row * MC;
-#pragma unroll
-        for (int m = 0; m < M; ++m) kvo[64 * m + lane] = f32_to_bf16(v[m]);
     }
     if (lane < MROPE / 2 && row_ok) {
         const float xe = round_bf16(pair.x), xo = round_bf16(pair.y);

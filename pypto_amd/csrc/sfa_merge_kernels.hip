@@ -124,8 +124,8 @@ hipError_t sfa_combine_many_launch(const SfaArgs& a, int n, int token0, hipStrea
 {
     const int t = a.b * a.s1, hgroups = (a.nq + SFA_HEADS_PER_WG - 1) / SFA_HEADS_PER_WG;
     const dim3 grid((t - token0) * hgroups * 64);
-    auto merge = token0 > 0 ? (n <= 16 ? sfa_combine_many_kernel<4, true> : sfa_combine_many_kernel<8, true>)
-                            : (n <= 16 ? sfa_combine_many_kernel<4, false> : sfa_combine_many_kernel<8, false>);
+    // (a last round's tokens have up to 16 splits; more are a single token's, or asked for)
+    auto merge = token0 > 0 ? sfa_combine_many_kernel<4, true> : n <= 16 ? sfa_combine_many_kernel<4, false> : sfa_combine_many_kernel<8, false>;
     hipLaunchKernelGGL(merge, grid, dim3(256), 0, stream, static_cast<const void*>(a.part_o), a.part_ml, a.out, a.nq, n, token0, hgroups);
     return hipGetLastError();
 }
