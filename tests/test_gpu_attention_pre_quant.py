@@ -261,6 +261,32 @@ def test_norm_by_pieces(cuda, t, h, q_heads):
         assert torch.equal(on[place].cpu(), got["residual_res"]), place
 
 
+@pytest.mark.parametrize("t,h,q_heads", [(1, 5120, 2), (4, 2048, 12), (3, 6144, 96), (6, 5120, 2), (9, 2304, 12)])
+def test_norms_of_infinities_and_nan(cuda, t, h, q_heads):
+    """Rows with an infinity, with infinities that cancel, a NaN, and the largest finite values, whose squares overflow: the norm in the
+    projection and the norm by pieces give the bits of the workgroup per row, which has them where the sums take an input's place."""
+    case = op.make_case(t, h=h, q_heads=q_heads, kv_heads=1, seed=t + h)
+    x, r, inf = case["hidden_states"], case["residual"], float("inf")
+    x[0, 5] = inf
+    if t > 1:
+        x[1, h - 1], r[1, h - 1] = inf, -inf
+        r[1, 70] = torch.finfo(torch.bfloat16).max
+    if t > 2:
+        r[2, 1] = float("nan")
+    if t > 3:
+        x[3, ::7] = torch.finfo(torch.bfloat16).max
+    got = run(case, cuda)
+    from pypto_amd.glm_v4_5 import glm_attention_pre_quant as impl
+    on = {k: case[k].to(cuda) for k in NAMES}
+    out = outputs(case, cuda)
+    impl.attention_pre_quant(*[on[k] for k in NAMES], out["query"], out["key"], out["value"], on["residual"])
+    for name in ("query", "key", "value"):
+        assert torch.equal(out[name].cpu().view(torch.int16), got[name].view(torch.int16)), name
+    a, b = on["residual"].cpu(), got["residual_res"]
+    assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(0.0), b.nan_to_num(0.0))
+    assert not torch.isfinite(b[0]).all()
+
+
 @pytest.mark.parametrize("h", [256, 1024, 1280, 2560, 2816, 4096, 4352, 5120, 5376, 8192, 8448, 12544])
 def test_partial_sums_of_any_number_of_splits(cuda, h):
     """1, 4, 5, 10, 11, 16, 17, 20, 21, 32, 33 and 49 splits of the contraction: up to one group of loads and more, whole and with a rest."""

@@ -244,6 +244,20 @@ def test_norms_by_wavefronts(cuda, t, n_idx, r, h):
     check_against_oracle(mla_case, idx_case, fused)
 
 
+def test_norms_by_wavefronts_of_infinities_and_nan(cuda):
+    # tokens whose sums are infinite, not a number, and overflow when squared: what the workgroups' norms of the separate call make of them
+    mla_case, idx_case = op.make_fused_case(258, 1, 64, seed=135, n_idx=64, h=2304, q_lora_rank=384, n=2)
+    x = mla_case["x"]
+    x[0, 5], x[1, 7], x[2] = float("inf"), float("nan"), torch.finfo(torch.bfloat16).max / 4
+    x[257, 9] = -float("inf")
+    idx_case["x"] = x
+    fused, sep = run_fused(mla_case, idx_case, cuda, entry="mla_indexer_prolog_quant_p"), run_separate(mla_case, idx_case, cuda)
+    for k in ("q_nope", "q_rope", "kv_cache", "kr_cache", "k_scale_cache", "q_int8", "q_scale"):
+        a, b = fused[k].float(), sep[k].float()
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(0.0), b.nan_to_num(0.0)), k
+    assert fused["q_nope"][3:257].isfinite().all() and not fused["kr_cache"].isfinite().all()
+
+
 def test_query_weights_whose_last_rows_lie_beyond_4_gb(cuda):
     # 33 tokens, 128 rows of 33818880 outputs: the last heads' results are the bits of a call of these heads alone
     n, r = 176140, 128

@@ -359,7 +359,8 @@ def test_a_tokens_bits_do_not_depend_on_the_batch(cuda, quant_b):
 
 
 @pytest.mark.parametrize("t,n,quant_b", [(33, 2, True), (65, 4, True), (97, 128, True), (129, 6, True), (160, 170, True), (160, 172, True),
-                                         (161, 6, True), (193, 2, True), (225, 2, True), (256, 4, True), (64, 4, False), (200, 4, False)])
+                                         (161, 6, True), (193, 2, True), (225, 2, True), (256, 4, True), (64, 4, False), (200, 4, False),
+                                         (128, 128, False), (200, 128, False), (256, 98, False), (188, 150, True)])
 def test_streamed_products_have_the_bits_of_the_decode_kernels(cuda, t, n, quant_b):
     """33 to 256 tokens: two to eight blocks of 32 with remainders of one and all rows; the x product over splits of 1024 and 256
     rows, whose sums are the decode kernel's (chains of 128 rows, added up in order), the int8 product's are exact: the last tokens'

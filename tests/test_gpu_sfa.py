@@ -252,6 +252,28 @@ def test_merge_of_more_than_eight_splits(cuda, nq, splits, quant):
     check_rms_vs_fp64(out[:1], first, golds, f"{nq} heads, {splits} splits")
 
 
+@pytest.mark.parametrize("splits", [9, 16, 32, 64])
+def test_merge_of_infinities_and_nan(cuda, splits):
+    """A NaN in one split's keys, an infinity in a query, one in the values alone, a query whose scores are all -inf: the merge of more than eight splits
+    leaves what the merge of eight does, value for value not finite in the same places."""
+    case = osfa.make_case(4, 20, 1, [2300, 2048, 1500, 2300], topk=2048, seed=97, dist="bench", softmax_scale=192 ** -0.5)
+    inf, bs = float("inf"), case["block_size"]
+
+    def row(token, place):
+        pos = int(case["topk_indices"][token, place])
+        return int(case["block_table"][token, pos // bs]) * bs + pos % bs
+
+    case["kn_scales"].view(-1, 4)[row(0, 1000), 2] = float("nan")
+    case["q"].view(4, 20, 576)[1, 3, 7] = inf
+    case["kn_scales"].view(-1, 4)[row(2, 40), 1] = inf
+    case["q"].view(4, 20, 576)[3, 17, 575] = -inf
+    few, many = run_with_splits(case, cuda, 8), run_with_splits(case, cuda, splits)
+    assert torch.equal(few.isnan(), many.isnan()) and torch.equal(few.isinf(), many.isinf())
+    assert few.isnan().any() and few.isfinite().any()
+    ok = few.isfinite()
+    assert count_violations(torch.where(ok, many, 0.0), torch.where(ok, few, 0.0), 2e-3, 2.0 ** -5) == 0
+
+
 def test_a_single_token_has_up_to_32_splits(cuda):
     case = osfa.make_case(1, 128, 1, [5000], topk=2048, seed=95, dist="bench", softmax_scale=192 ** -0.5)
     out = run_sfa(case, cuda)
