@@ -903,8 +903,10 @@ __global__ void sfa_zero_kernel(uint32_t* out, int64_t n_words)
 // workgroup merges, for one token, what the attention workgroups left for column group wv / 2 and pair 2 (wv % 2) + hb: 32 heads x
 // 128 value columns; its wavefront i takes 16 of the heads and 64 columns, a lane owning for its head (16 (i % 2) + l16) the four
 // 4-column runs at 16 j + 4 g of these.  G = 2, 4 or 8, the smallest that covers the split count: every split's loads are requested
-// before any is used (splits past the last are the last again with weight 0).  More than eight splits: sfa_combine_many_launch.  The workgroup then
-// turns its 32 x 128 block through LDS and writes the 256-byte row pieces, 16 lanes a piece.
+// before any is used (splits past the last are the last again with weight 0).  That it is written as a loop over groups, of which there is one, is for the code that
+// comes of it: without the loop the kernel takes longer, whether the loads are left to the compiler (by the profiler, with / without, 48 tokens 8.96 / 9.45 us, 96:
+// 8.14 / 8.38) or kept in front by a fence (26: 7.65 / 7.78, 48: 8.96 / 9.13, 96: 8.14 / 8.38), the pairs (m, l) first or last.  More than eight splits:
+// sfa_combine_many_launch.  The workgroup then turns its 32 x 128 block through LDS and writes the 256-byte row pieces, 16 lanes a piece.
 // grid (tokens with several splits x head groups x 16), 256 lanes; token0: the first of these tokens.
 constexpr int CROW = 128 * 2 + 16; // LDS row of the merge's transposition: 128 bf16 plus one 16-byte chunk of padding
 template <int G, bool FP32>
@@ -932,35 +934,46 @@ __global__ __launch_bounds__(256) void sfa_combine_kernel(const void* __restrict
     const int64_t split_stride = (int64_t)hgroups * 8 * 8192; // elements between two splits of a token
     const P* frag0 = part_o + ((partial * hgroups + hz) * 8 + wv) * 8192 + hb * 4096 + cb * 1024 + b * 512; // (the workgroup's four wavefronts read 8 or 16 KB in a row per split)
     const float2* ml0 = reinterpret_cast<const float2*>(part_ml) + partial * nq + min(head_base + 16 * b + l16, nq - 1);
-    typename std::conditional<FP32, f32x8, f16x8>::type v[G][2];
-    float2 ml[G];
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-        const int s = min(j, nsplit - 1);
-        const P* base = frag0 + s * split_stride;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            if constexpr (FP32) {
-                const f32x4 *lo = reinterpret_cast<const f32x4*>(base + h * 1024) + lane, *hi = lo + 64;
-                v[j][h] = __builtin_shufflevector(*lo, *hi, 0, 1, 2, 3, 4, 5, 6, 7);
-            } else
-                v[j][h] = *reinterpret_cast<const f16x8*>(base + h * 1024 + lane * 8);
-        }
-        ml[j] = ml0[(int64_t)s * nq];
-        if (j >= nsplit) ml[j].y = 0.f;
-    }
-    STEP_FENCE(); // (left alone, fewer of the loads are in flight: fp32, 44 tokens of 5 splits 13.4 us, so 13.0)
-#pragma unroll
-    for (int j = 0; j < G; ++j) M = ml[j].y > 0.f ? fmaxf(M, ml[j].x) : M;
-    if (M != -INFINITY) { // (otherwise nothing attended)
+    for (int s0 = 0; s0 < nsplit; s0 += G) {
+        typename std::conditional<FP32, f32x8, f16x8>::type v[G][2];
+        float2 ml[G];
 #pragma unroll
         for (int j = 0; j < G; ++j) {
-            const float w = ml[j].y > 0.f ? exp2f(ml[j].x - M) * ml[j].y : 0.f;
-            L += w;
+            const int s = min(s0 + j, nsplit - 1);
+            const P* base = frag0 + s * split_stride;
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < 2; ++h) {
+                if constexpr (FP32) {
+                    const f32x4 *lo = reinterpret_cast<const f32x4*>(base + h * 1024) + lane, *hi = lo + 64;
+                    v[j][h] = __builtin_shufflevector(*lo, *hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                } else
+                    v[j][h] = *reinterpret_cast<const f16x8*>(base + h * 1024 + lane * 8);
+            }
+            ml[j] = ml0[(int64_t)s * nq];
+            if (s0 + j >= nsplit) ml[j].y = 0.f;
+        }
+        if constexpr (FP32) STEP_FENCE(); // (left alone, fewer of the loads are in flight: 44 tokens of 5 splits 13.4 us, so 13.0)
+        // the group's maximum joins the running one: what was summed so far is rescaled once per group
+        float Mg = M;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) acc[h][e] += (float)v[j][h][e] * w;
+        for (int j = 0; j < G; ++j) Mg = ml[j].y > 0.f ? fmaxf(Mg, ml[j].x) : Mg;
+        if (Mg != -INFINITY) { // (otherwise nothing attended in these splits)
+            if (s0 > 0) {
+                const float back = exp2f(M - Mg); // 0 while nothing has been summed (M = -inf)
+                L *= back;
+#pragma unroll
+                for (int x = 0; x < 16; ++x) (&acc[0][0])[x] *= back;
+            }
+            M = Mg;
+#pragma unroll
+            for (int j = 0; j < G; ++j) {
+                const float w = ml[j].y > 0.f ? exp2f(ml[j].x - M) * ml[j].y : 0.f;
+                L += w;
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) acc[h][e] += (float)v[j][h][e] * w;
+            }
         }
     }
     const float inv = L > 0.f ? 1.f / L : 0.f;
