@@ -8,10 +8,10 @@
 // their products, 111 K with the copies between the matrix instructions, 107 K with the products half a stage behind the reads
 // besides (a call of 777 tokens x 112 heads 90.8 us, 88.7, 86.4; 1024 tokens 101.0, 98.3, 95.9).  With the reads between the matrix
 // instructions too, instead of in one go behind the barrier, a stage by itself takes 2295 ticks, not 2440 (256 tokens 2490 / 2717, 128:
-// 1488 / 1551; calls of 777 and 1024 tokens 75.6 -> 71.8 us and 79.9 -> 78.7).  Below that the chip's power decides: matrix
-// instructions 78 % of the time hold the clock at 1.85 GHz (four waves with half again the tile each read a quarter less of LDS, and
-// the compiler moves their sums between register files: 57 -> 74 us at 256 tokens).  The waves' priorities make no difference: the
-// second wave of a SIMD is done when it would be anyway, the first waits for it at the barrier.  And
+// 1488 / 1551).  A whole call keeps little of it (777 tokens 73.6 -> 72.6 us, 1024: 87.4 -> 86.1, 300: 53.4 -> 54.2, and 50.3 -> 48.7 with warm weights): the
+// chip's power decides, matrix instructions 78 % of the time hold the clock at 1.85 GHz (four waves with half again the tile each read a
+// quarter less of LDS, and the compiler moves their sums between register files: 57 -> 74 us at 256 tokens).  The waves' priorities make no
+// difference: the second wave of a SIMD is done when it would be anyway, the first waits for it at the barrier.  And
 //  - a stage's operands are copied to LDS by the memory pipe itself (global_load_lds_dwordx4: no registers, no LDS store
 //    instructions), into the buffer that is not being read, so that a stage has one barrier;
 //  - rows of 128 bytes are kept unpadded (a copy writes 64 lanes x 16 bytes in a row) and spread over the banks by
